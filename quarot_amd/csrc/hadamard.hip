@@ -1883,10 +1883,15 @@ int launch_hadamard_mm(const void* x, void* y, int64_t rows, int n, int K, const
 // The hadK factor then runs on the matrix cores as in hadamard_mm_kernel (T^T as first operand, hadK
 // fragments in registers, 8-byte result writes).  All of a row's loads are issued at once and the next
 // row's are requested before the matrix stage.
-template <bool QUANT, int CPL>
+// fp32-precision mode (MODE32, m = 1024; bound by vector and matrix instruction issue like the fp16 form, 38 us at 2048 rows,
+// plus the lo planes: 49 us at 1777 rows): the scaled U is kept as two fp16 planes, hi = fp16(U) and lo = fp16(U - hi), in
+// two copies of the fragment array (2 x 68 KB of LDS; the fp16 result row has no place there, so the results leave from
+// registers in every variant of this mode), and each product of the hadK stage is a hi and a lo matrix instruction.
+template <bool QUANT, int CPL, bool MODE32>
 __global__ __launch_bounds__(1024) void hadamard_bm_kernel(const f16* __restrict__ x, f16* __restrict__ y, int64_t rows,
-                                                           int n, int K, const f16* __restrict__ hadK, float scale,
+                                                           int n, int K, const void* __restrict__ hadK, float scale,
                                                            float clip, u32* __restrict__ q, f16* __restrict__ scales) {
+    static_assert(!MODE32 || CPL == 2, "the fp32-precision mode is built for m = 1024");
     constexpr int BT = 1024, NW = 16;
     constexpr int M_ = 512 * CPL, LOG2M = CPL == 1 ? 9 : 10;
     constexpr int CT = M_ / 16;                  // 16-column tiles
@@ -1897,8 +1902,9 @@ __global__ __launch_bounds__(1024) void hadamard_bm_kernel(const f16* __restrict
     constexpr int YS = M_ + 8;
     extern __shared__ f32x4 smem_raw[];
     __shared__ u32 red[NW];
-    u32x4* Tl = (u32x4*)smem_raw;                // [KS2][4][CT][TS]
-    f16* Yl = (f16*)(Tl + KS2 * 4 * CT * TS);    // [K][YS]
+    constexpr int TN = KS2 * 4 * CT * TS;
+    u32x4* Tl = (u32x4*)smem_raw;                // [KS2][4][CT][TS]; MODE32: a second array with the lo plane behind it
+    f16* Yl = (f16*)(Tl + TN);                   // [K][YS] (not in MODE32)
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int l16 = lane & 15, g = lane >> 4;
     const int nchunks = n >> 3;
@@ -1930,12 +1936,18 @@ __global__ __launch_bounds__(1024) void hadamard_bm_kernel(const f16* __restrict
     };
     int64_t row = blockIdx.x;
     if (row < rows) request(row);           // in flight while the fragments are made and T is cleared
+    // MODE32: the first 32 sums carry a factor 1 / 32 (a power of two: no rounding), so that T never leaves the fp16 range
+    // where x does not, and both lo planes (T's and U's) are stored 2048 times as large (hb's copy for T carries
+    // 1 / 2048, U's sums take it when they are added) so that lo keeps its eleven bits for small activations too (without the factor it would be subnormal
+    // below 0.25)
+    constexpr float SA = MODE32 ? 0.03125f : 1.0f;
+    const float uscale = MODE32 ? scale * 32.0f : scale;
     f16x8 ha[2], hb[2];
     if (CPL == 2) {
 #pragma unroll
         for (int t = 0; t < 8; ++t) {
 #pragma unroll
-            for (int cth = 0; cth < 2; ++cth) ha[cth][t] = (__builtin_popcount((g * 8 + t) & (cth * 16 + l16)) & 1) ? (f16)-1.0f : (f16)1.0f;
+            for (int cth = 0; cth < 2; ++cth) ha[cth][t] = (__builtin_popcount((g * 8 + t) & (cth * 16 + l16)) & 1) ? (f16)-SA : (f16)SA;
             const int b = 16 * (t >> 2) + 4 * g + (t & 3);
 #pragma unroll
             for (int bt = 0; bt < 2; ++bt) hb[bt][t] = (__builtin_popcount(b & (bt * 16 + l16)) & 1) ? (f16)-1.0f : (f16)1.0f;
@@ -1951,12 +1963,19 @@ __global__ __launch_bounds__(1024) void hadamard_bm_kernel(const f16* __restrict
             for (int hh = 0; hh < 2; ++hh) {
                 const int hr = rt * 16 + l16, hc = ks * 32 + g * 8 + hh * 4;
                 f16x4 v = {(f16)0, (f16)0, (f16)0, (f16)0};
-                if (hr < K && hc < K) v = *(const f16x4*)(hadK + hr * K + hc);
+                if (hr < K && hc < K) {
+                    if (MODE32) {
+                        const f32x4 w = *(const f32x4*)((const float*)hadK + hr * K + hc);
+                        v = f16x4{(f16)w[0], (f16)w[1], (f16)w[2], (f16)w[3]};
+                    } else {
+                        v = *(const f16x4*)((const f16*)hadK + hr * K + hc);
+                    }
+                }
 #pragma unroll
                 for (int e = 0; e < 4; ++e) hf[rt][ks][hh * 4 + e] = v[e];
             }
     // slots of T for k >= K are never written afterwards: clear once
-    for (int i = tid; i < KS2 * 4 * CT * TS; i += BT) Tl[i] = u32x4{0, 0, 0, 0};
+    for (int i = tid; i < (MODE32 ? 2 : 1) * TN; i += BT) Tl[i] = u32x4{0, 0, 0, 0};
 
     __syncthreads();
     for (; row < rows; row += gridDim.x) {
@@ -1965,7 +1984,7 @@ __global__ __launch_bounds__(1024) void hadamard_bm_kernel(const f16* __restrict
             if (works) {
 #pragma unroll
                 for (int cth = 0; cth < 2; ++cth) {
-                    u32 o[2][2][2];                      // [segment of the pair][b' tile][pair of e]: fp16 pairs
+                    u32 o[2][2][2], ol[2][2][2];         // [segment of the pair][b' tile][pair of e]: fp16 pairs (hi, lo)
 #pragma unroll
                     for (int sg = 0; sg < 2; ++sg) {
                         // T = hi + lo, both fp16, as packed pairs (the difference is exact in fp32, so one rounding each)
@@ -1978,7 +1997,9 @@ __global__ __launch_bounds__(1024) void hadamard_bm_kernel(const f16* __restrict
 #pragma unroll
                             for (int pr = 0; pr < 2; ++pr) {
                                 const f16x2 hi = __builtin_convertvector(f32x2_t{da[2 * pr], da[2 * pr + 1]}, f16x2);
-                                const f16x2 lo = __builtin_convertvector(f32x2_t{da[2 * pr] - (float)hi[0], da[2 * pr + 1] - (float)hi[1]}, f16x2);
+                                f32x2_t rest = {da[2 * pr] - (float)hi[0], da[2 * pr + 1] - (float)hi[1]};
+                                if (MODE32) rest = f32x2_t{rest[0] * 2048.0f, rest[1] * 2048.0f};
+                                const f16x2 lo = __builtin_convertvector(rest, f16x2);
                                 whi[bt * 2 + pr] = __builtin_bit_cast(u32, hi);
                                 wlo[bt * 2 + pr] = __builtin_bit_cast(u32, lo);
                             }
@@ -1987,9 +2008,18 @@ __global__ __launch_bounds__(1024) void hadamard_bm_kernel(const f16* __restrict
 #pragma unroll
                         for (int bt = 0; bt < 2; ++bt) {
                             f32x4 db = __builtin_amdgcn_mfma_f32_16x16x32_f16(hb[bt], thi, f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-                            db = __builtin_amdgcn_mfma_f32_16x16x32_f16(hb[bt], tlo, db, 0, 0, 0);
-                            o[sg][bt][0] = narrow_f16x2(db[0] * scale, db[1] * scale);
-                            o[sg][bt][1] = narrow_f16x2(db[2] * scale, db[3] * scale);
+                            f16x8 hl = hb[bt];
+                            if (MODE32) hl = hl * (f16)(1.0f / 2048.0f);
+                            db = __builtin_amdgcn_mfma_f32_16x16x32_f16(hl, tlo, db, 0, 0, 0);
+#pragma unroll
+                            for (int pr = 0; pr < 2; ++pr) {
+                                const float u0 = db[2 * pr] * uscale, u1 = db[2 * pr + 1] * uscale;
+                                o[sg][bt][pr] = narrow_f16x2(u0, u1);
+                                if (MODE32) {
+                                    const f16x2 h = as_f16x2(o[sg][bt][pr]);
+                                    ol[sg][bt][pr] = narrow_f16x2((u0 - (float)h[0]) * 2048.0f, (u1 - (float)h[1]) * 2048.0f);
+                                }
+                            }
                         }
                     }
                     // position (b' = 16 bt + 4 g + e, c' = 16 cth + l16) = column tile 2 b' + cth, column l16; the pair's
@@ -2001,6 +2031,8 @@ __global__ __launch_bounds__(1024) void hadamard_bm_kernel(const f16* __restrict
                         for (int e = 0; e < 4; ++e) {
                             const u32 sel = (e & 1) ? 0x07060302u : 0x05040100u;      // high or low halves of two dwords
                             dst[(2 * (16 * bt + 4 * g + e)) * TS * 4] = __builtin_amdgcn_perm(o[1][bt][e >> 1], o[0][bt][e >> 1], sel);
+                            if (MODE32)
+                                dst[(2 * (16 * bt + 4 * g + e)) * TS * 4 + TN * 4] = __builtin_amdgcn_perm(ol[1][bt][e >> 1], ol[0][bt][e >> 1], sel);
                         }
                 }
             }
@@ -2039,8 +2071,8 @@ __global__ __launch_bounds__(1024) void hadamard_bm_kernel(const f16* __restrict
         const int64_t nrow = row + gridDim.x;
         if (nrow < rows) request(nrow);
         __syncthreads();
-        if constexpr (QUANT && CPL == 2) {
-            if (y == nullptr) {
+        if constexpr ((QUANT || MODE32) && CPL == 2) {
+            if (MODE32 || y == nullptr) {
                 // ---- no copy of the transformed row wanted (the decode step, prefill): the results of the hadK stage
                 // stay in registers and become codes there, as in hadamard_m64r_kernel -- same layout: lanes l16 + 16 g
                 // hold, for output row k' = 16 rt + l16, the columns 16 c + 4 g .. + 3 of this wave's four column tiles
@@ -2052,13 +2084,23 @@ __global__ __launch_bounds__(1024) void hadamard_bm_kernel(const f16* __restrict
                 f16x8 th4[4];
 #pragma unroll
                 for (int c = 0; c < 4; ++c) th4[c] = __builtin_bit_cast(f16x8, Tl[(g * CT + wave * 4 + c) * TS + l16]);
+                f16x8 tl4[MODE32 ? 4 : 1];
+                if (MODE32) {
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) tl4[MODE32 ? c : 0] = __builtin_bit_cast(f16x8, Tl[TN + (g * CT + wave * 4 + c) * TS + l16]);
+                }
                 u32x2 yv[RT][4];
                 float mxf = 0.f, probe = 0.f;
 #pragma unroll
                 for (int c = 0; c < 4; ++c)
 #pragma unroll
                     for (int rt = 0; rt < RT; ++rt) {
-                        const f32x4 acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(th4[c], hf[rt][0], f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+                        f32x4 acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(th4[c], hf[rt][0], f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+                        if (MODE32) {
+                            const f32x4 al = __builtin_amdgcn_mfma_f32_16x16x32_f16(tl4[MODE32 ? c : 0], hf[rt][0], f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) acc[e] = __builtin_fmaf(al[e], 1.0f / 2048.0f, acc[e]);
+                        }
                         if (c == 0 && rt == 0) probe = acc[0];
                         yv[rt][c][0] = cvt_f16x2(acc[0], acc[1]);
                         yv[rt][c][1] = cvt_f16x2(acc[2], acc[3]);
@@ -2067,6 +2109,32 @@ __global__ __launch_bounds__(1024) void hadamard_bm_kernel(const f16* __restrict
                         mxf = __builtin_fmaxf(__builtin_fmaxf(mxf, __builtin_fabsf(acc[0])), __builtin_fabsf(acc[1]));
                         mxf = __builtin_fmaxf(__builtin_fmaxf(mxf, __builtin_fabsf(acc[2])), __builtin_fabsf(acc[3]));
                     }
+                if (MODE32 && y) {
+                    // the transformed row: the 8-byte pieces (g, c) -> lane c, piece g (first across the halves of the wave,
+                    // then neighbouring rows of 16 lanes), so that a lane stores 32 consecutive bytes and four lanes a line
+                    f16* const yrow = y + row * (int64_t)n;
+#pragma unroll
+                    for (int rt = 0; rt < RT; ++rt) {
+                        u32x2 p[4];
+#pragma unroll
+                        for (int d = 0; d < 2; ++d) {
+                            const auto a = __builtin_amdgcn_permlane32_swap(yv[rt][0][d], yv[rt][2][d], false, false);
+                            const auto b = __builtin_amdgcn_permlane32_swap(yv[rt][1][d], yv[rt][3][d], false, false);
+                            const auto e = __builtin_amdgcn_permlane16_swap(a[0], b[0], false, false);
+                            const auto o = __builtin_amdgcn_permlane16_swap(a[1], b[1], false, false);
+                            p[0][d] = e[0], p[1][d] = e[1], p[2][d] = o[0], p[3][d] = o[1];
+                        }
+                        if (dval[rt]) {
+                            u32x4* const d4 = (u32x4*)(yrow + (rt * 16 + l16) * M_ + wave * 64 + g * 16);
+                            d4[0] = u32x4{p[0][0], p[0][1], p[1][0], p[1][1]};
+                            d4[1] = u32x4{p[2][0], p[2][1], p[3][0], p[3][1]};
+                        }
+                    }
+                    if (!QUANT) {
+                        __syncthreads();                // (the next row's phase 1 writes T)
+                        continue;
+                    }
+                }
                 // the row's maximum: rounded once (rounding is monotone); an infinity or NaN anywhere in the row reaches
                 // every output, so one output per lane tells, and a wave that sees one takes the exact form (NaN wins)
                 u32 mx = f16_bits((f16)mxf);
@@ -2211,23 +2279,28 @@ bool bm_applies(int n, int K) {
     return (m == 512 && K <= 64) || (m == 1024 && K <= 32);
 }
 
-template <bool QUANT>
+template <bool QUANT, bool MODE32 = false>
 int launch_hadamard_bm(const void* x, void* y, int64_t rows, int n, int K, const void* hadK, float scale, float clip,
                        void* q, void* scales, hipStream_t st) {
     const int m = n / K;
     const int cpl = m / 512;
-    const size_t lds = (size_t)(cpl == 1 ? 2 : 1) * 4 * (m / 16) * 17 * 16 + (size_t)K * (m + 8) * 2;
+    const size_t planes = (size_t)(cpl == 1 || MODE32 ? 2 : 1) * 4 * (m / 16) * 17 * 16;
+    const size_t lds = planes + (MODE32 ? 0 : (size_t)K * (m + 8) * 2);
     const unsigned grid = (unsigned)(rows < 256 ? rows : 256);
 #define QR_BM(CPL)                                                                                                     \
     do {                                                                                                               \
-        auto kern = hadamard_bm_kernel<QUANT, CPL>;                                                                    \
+        auto kern = hadamard_bm_kernel<QUANT, CPL, MODE32>;                                                                   \
         hipError_t e = qr_allow_dynamic_lds((const void*)kern, lds);   \
         if (e != hipSuccess) return (int)e;                                                                            \
-        kern<<<dim3(grid), dim3(1024), lds, st>>>((const f16*)x, (f16*)y, rows, n, K, (const f16*)hadK, scale, clip,   \
-                                                  (u32*)q, (f16*)scales);                                              \
+        kern<<<dim3(grid), dim3(1024), lds, st>>>((const f16*)x, (f16*)y, rows, n, K, hadK, scale, clip, (u32*)q,      \
+                                                  (f16*)scales);                                                       \
     } while (0)
-    if (cpl == 1) QR_BM(1);
-    else QR_BM(2);
+    if constexpr (MODE32) {
+        QR_BM(2);
+    } else {
+        if (cpl == 1) QR_BM(1);
+        else QR_BM(2);
+    }
 #undef QR_BM
     return qr_launch_status();
 }
@@ -2494,6 +2567,11 @@ extern "C" int qr_hadamard_quantize_f16_i4(const void* x, int64_t rows, int n, i
         return launch_hadamard_mm<true, true>(x, y_or_null, rows, n, pow2_split(n), nullptr, scale, clip, q, scales, st);
     if (mode == QR_DTYPE_F16 && bm_applies(n, K))
         return launch_hadamard_bm<true>(x, y_or_null, rows, n, K, hadK, scale, clip, q, scales, st);
+    // fp32 precision behind a 1024-point factor: the matrix-core kernel with hi / lo planes at every row count (the general
+    // kernel's fp32 row fills a CU's LDS and it forms the hadK fragments from scalar LDS reads: 1777 x 28672 393 us against
+    // 49 us here = 2.6 TB/s, 4096 rows 934 against 99, 1 and 64 rows 56 against 14)
+    if (mode == QR_DTYPE_F32 && bm_applies(n, K) && n / K == 1024)
+        return launch_hadamard_bm<true, true>(x, y_or_null, rows, n, K, hadK, scale, clip, q, scales, st);
     if (mm_applies(n, K)) {
         if (mode == QR_DTYPE_F16) return launch_hadamard_mm<false, true>(x, y_or_null, rows, n, K, hadK, scale, clip, q, scales, st);
         return launch_hadamard_mm<true, true>(x, y_or_null, rows, n, K, hadK, scale, clip, q, scales, st);
