@@ -288,8 +288,6 @@ def mfma_ceiling(seconds):
 
 
 def gemm_kernel_name(m, n, k=0):
-    t256 = ((m + 255) // 256) * ((n + 255) // 256)
-    t128 = ((m + 127) // 128) * ((n + 255) // 256)
     groups = (n + 31) // 32                # the library's choice: enough groups of 32 rows to give every CU a workgroup
     xs = any((groups + rg - 1) // rg >= 192 for rg in range(4, 9))
     if m == 1 or (m <= 4 and not xs):
@@ -298,11 +296,19 @@ def gemm_kernel_name(m, n, k=0):
         if not xs and m >= 40 and k >= 16384:   # narrow weight, many tokens, long K: K sliced across workgroups + slab sum
             return "decode_xs_kernel (K sliced) + dequant_slabs_kernel"
         return "decode_xs_kernel" if xs else "decode_i4_kernel"
-    if t128 >= 128:         # the library's choice between its pipelined kernels, by rounds of tiles (256-, 192- or 128-row)
-        t192 = ((m + 191) // 192) * ((n + 255) // 256)
-        r256, r192, r128 = (t256 + 255) // 256, ((t192 + 255) // 256) * 0.80, ((t128 + 255) // 256) * 0.57
-        return "gemm_sp256_kernel" if (r256 <= r128 and r256 <= r192) or r192 <= r128 else "gemm_spk_kernel"
-    return "gemm_ks_kernel<64,256>"
+    # the library's estimate (gemm.hip, mid_plan) for its tile shapes on 256 CUs, in microseconds
+    st = (max(k, 256) + 255) // 256
+    tiles = lambda bm, bn: ((m + bm - 1) // bm) * ((n + bn - 1) // bn)
+    load = lambda t: (t + 255) // 256
+    n64, n128, nsq = load(tiles(64, 64)), load(tiles(64, 128)), load(tiles(128, 128))
+    est = [(4.2 + st * {1: 0.26, 2: 0.44}.get(n64, (0.25 if n64 < 8 else 0.26) * n64), "gemm_mid_kernel<64,64>"),
+           (4.6 + st * (0.41 if n128 == 1 else 0.52 * n128), "gemm_mid_kernel<64,128>"),
+           (5.0 + st * (0.8 if nsq == 1 else 0.92 * nsq), "gemm_mid_kernel<128,128>")]
+    tall = min((2, 1, 0), key=lambda i: load(tiles(128 + 64 * i, 256)) * (0.57, 0.80, 1.0)[i])      # ties: the taller tile
+    t = tiles(128 + 64 * tall, 256)
+    est.append((load(t) * (5.5 + (1.40, 2.19, 2.75)[tall] * st * (1 - (0.5 if tall else 0.3) * (1 - t / (load(t) * 256)))),
+                "gemm_sp256_kernel" if tall else "gemm_spk_kernel"))
+    return min(est, key=lambda e: e[0])[1]
 
 
 FRONT_KERNEL = {"had": "hadamard kernel + quantiser (fused)", "had32": "hadamard kernel in fp32 precision + quantiser (fused)",

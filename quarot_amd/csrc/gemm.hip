@@ -17,10 +17,8 @@
 // Issue budget: a 32x32x32 int8 MFMA occupies the matrix pipe for 32 cycles and a wave's VALU op
 // takes 4; measured on MI355X, up to ~5 VALU ops per MFMA are hidden.  Unpacking costs 3 VALU ops per
 // packed dword, i.e. 6 (IM + JN) / (IM JN) per MFMA for a wave tile of IM x JN MFMA tiles: 64x128 per
-// wave (4.5) is the smallest tile that fits.  To still run two waves per SIMD on a 128x256 workgroup
-// tile (one tile per CU at M = 2048, N = 4096), eight waves are arranged as 2 (M) x 2 (N) x 2 (K): the
-// two K-groups take alternate 64-k sub-steps of every stage and exchange half of their accumulators
-// through LDS at the end.
+// wave (4.5) is the smallest tile that fits where the matrix pipe is to stay busy.  (Outputs of few tiles, bound by
+// the CUs' intake of operands instead, take the 64x64 wave tiles of gemm_mid.hip.)
 #include "qr_common.h"
 #include "qr_epilogue.h"
 #include <type_traits>
@@ -290,361 +288,6 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void gemm_i4_kernel(
             }
         }
     }
-}
-
-// ------------------------------------------------------------------------------------------------
-// Compute-bound shapes (M > 64): 128x256 workgroup tile, eight waves as 2 (M) x 2 (N) x 2 (K).
-//
-// Both K-groups own the same 64x128 wave tiles and split every 128-k stage between them (group g
-// takes the 64-k sub-step g); they exchange half of their accumulators through LDS at the end.
-// The two waves that share a SIMD belong to different K-groups and run half an iteration out of
-// phase: group 0 reads and unpacks its fragments and then multiplies, group 1 first multiplies the
-// operands it unpacked during the previous iteration and then reads and unpacks the next ones.  So
-// on every SIMD one wave's unpacking (VALU) runs under the other wave's MFMAs instead of both
-// unpacking, then both multiplying.  A stage is 256 k (a full 128-byte line per row, so every line
-// fetched from L2 is used whole); three LDS stages rotate (group 1 reads one stage ahead of group
-// 0), global loads run one more stage ahead through registers, one barrier per stage.
-// (A variant in which half the waves only unpacked into int8 planes in LDS for the other half was
-// measured LDS-bound: twice the LDS bytes at ~128 B/clk/CU exceed the MFMA time.)
-template <int BM, int BN, int WAVES_M, int WAVES_N, bool DEQ>
-__global__ __launch_bounds__(128 * WAVES_M * WAVES_N) void gemm_ks_kernel(
-    const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, int M, int N, int Kb, int32_t* __restrict__ C,
-    f16* __restrict__ Y, const f16* __restrict__ sA, const f16* __restrict__ sB, const f16* __restrict__ bias,
-    int tiles_m, int tiles_n, int ksplit, int nxcd) {
-    constexpr int NT = 128 * WAVES_M * WAVES_N;
-    constexpr int TM = BM / WAVES_M, TN = BN / WAVES_N;
-    constexpr int IM = TM / 32, JN = TN / 32;
-    // ksplit > 1 (int32 output only): the stages of K are divided among ksplit workgroups per tile;
-    // slice s writes its partial sums to the s-th [M, N] slab of C, and a second kernel adds the slabs
-    // (atomic adds into one slab were measured 3-4x slower than the whole unsplit product).
-    // A stage is 128 packed bytes (256 k) per row = one full cache line, eight 16-byte chunks,
-    // four 64-k sub-steps; K-group g multiplies sub-steps 2g and 2g+1.
-    constexpr int CH = (BM + BN) * 8;
-    constexpr int NL = CH / NT;
-    constexpr int NBUF = 3;
-    constexpr int JH = JN / 2;
-    static_assert(CH % NT == 0 && JN % 2 == 0, "tile shape");
-    extern __shared__ u32x4 ks_lds[];                       // [NBUF][CH]; later the accumulator exchange
-
-    const int per_xcd = gridDim.x / nxcd;
-    const int unit = (blockIdx.x % nxcd) * per_xcd + blockIdx.x / nxcd;
-    if (unit >= tiles_m * tiles_n * ksplit) return;
-    const int tile = unit / ksplit, split = unit - tile * ksplit;   // the slices of a tile are neighbours in L2
-    constexpr int GROUP_M = 8;
-    const int group_sz = GROUP_M * tiles_n;
-    const int g = tile / group_sz;
-    const int gm0 = g * GROUP_M;
-    const int gh = (tiles_m - gm0) < GROUP_M ? (tiles_m - gm0) : GROUP_M;
-    const int tm = gm0 + (tile - g * group_sz) % gh;
-    const int tn = (tile - g * group_sz) / gh;
-    const int m0 = tm * BM, n0 = tn * BN;
-
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int kg = wave / (WAVES_M * WAVES_N);
-    const int wxy = wave % (WAVES_M * WAVES_N);
-    const int wm = wxy / WAVES_N, wn = wxy % WAVES_N;
-    const int khalf = lane >> 5;
-    const int all_stages = (Kb + 127) / 128;
-    if (ksplit > 1) C += (int64_t)split * M * N;
-    const int s_first = (int)((int64_t)all_stages * split / ksplit);
-    const int stages = (int)((int64_t)all_stages * (split + 1) / ksplit) - s_first;   // >= 1: ksplit <= all_stages
-    // chunk position within a row is XOR-swizzled with (row >> 1) & 7: the 16 rows a quarter-wave
-    // reads at one logical chunk cover all sixteen 16-byte bank groups (row parity picks the half)
-    auto slot8 = [](int row, int chunk) { return row * 8 + (chunk ^ ((row >> 1) & 7)); };
-
-    // ---- staging (all threads): chunk id = tid + i * NT, eight consecutive threads fetch one row's line.
-    // Thread-invariant parts are kept out of registers: the rows of a thread's chunks differ by
-    // multiples of 64 (same swizzle), so LDS slots differ by compile-time constants.
-    static_assert(NT == 512 && BM % 64 == 0 && BN % 64 == 0, "staging layout");
-    const int srow = tid >> 3;
-    const int scoff = (tid & 7) * 16;
-    const int dst0 = slot8(srow, tid & 7);
-    u32 goff[NL];                                           // byte offset of the row from A (i < BM/64) or B
-#pragma unroll
-    for (int i = 0; i < NL; ++i) {
-        const int row = srow + i * 64;
-        int gr = row < BM ? m0 + row : n0 + row - BM;
-        const int lim = row < BM ? M - 1 : N - 1;
-        gr = gr < lim ? gr : lim;
-        goff[i] = (u32)gr * (u32)Kb;
-    }
-    // branch-free loads: a stage past the end repeats the last one; chunks beyond the row end of a
-    // partly filled last stage re-read the stage's first chunk and are zeroed when written to LDS
-    const bool ragged = (Kb & 127) != 0;
-    auto fetch = [&](int st, u32x4(&r)[NL]) {
-        const int kb = (s_first + (st < stages ? st : stages - 1)) * 128;
-        const u32 off = (u32)((kb + scoff < Kb) ? kb + scoff : kb);
-#pragma unroll
-        for (int i = 0; i < NL; ++i) {
-            if (i * 64 < BM) r[i] = *(const u32x4*)(A + (size_t)(goff[i] + off));
-            else r[i] = *(const u32x4*)(B + (size_t)(goff[i] + off));
-        }
-    };
-    auto deposit = [&](int st, int buf, u32x4(&r)[NL]) {
-        if (st < stages) {
-            if (ragged && (s_first + st) * 128 + scoff >= Kb) {
-#pragma unroll
-                for (int i = 0; i < NL; ++i) r[i] = u32x4{0, 0, 0, 0};
-            }
-            u32x4* base = ks_lds + buf * CH + dst0;
-#pragma unroll
-            for (int i = 0; i < NL; ++i) base[i * 64 * 8] = r[i];
-        }
-    };
-    i32x16 acc[IM][JN];
-#pragma unroll
-    for (int i = 0; i < IM; ++i)
-#pragma unroll
-        for (int j = 0; j < JN; ++j)
-#pragma unroll
-            for (int v = 0; v < 16; ++v) acc[i][j][v] = 0;
-
-    // this wave's fragment slots for its two sub-steps (u = 0, 1): logical chunk (2 kg + u) * 2 + khalf;
-    // tile rows differ by multiples of 32 (same swizzle): compile-time offsets
-    int aslot[2], bslot[2];
-#pragma unroll
-    for (int u = 0; u < 2; ++u) {
-        aslot[u] = slot8(wm * TM + (lane & 31), (2 * kg + u) * 2 + khalf);
-        bslot[u] = slot8(BM + wn * TN + (lane & 31), (2 * kg + u) * 2 + khalf);
-    }
-    struct Ops {
-        i32x4 alo[IM], ahi[IM], blo[JN], bhi[JN];
-    };
-    auto load_ops = [&](int buf, int u, Ops& o) {
-        const u32x4* pa = ks_lds + buf * CH + (u ? aslot[1] : aslot[0]);
-        const u32x4* pb = ks_lds + buf * CH + (u ? bslot[1] : bslot[0]);
-#pragma unroll
-        for (int i = 0; i < IM; ++i) {
-            const u32x4 p = pa[i * 32 * 8];
-            o.alo[i] = (i32x4)((p << 4) & 0xF0F0F0F0u);
-            o.ahi[i] = (i32x4)(p & 0xF0F0F0F0u);
-        }
-#pragma unroll
-        for (int j = 0; j < JN; ++j) {
-            const u32x4 p = pb[j * 32 * 8];
-            o.blo[j] = (i32x4)((p << 4) & 0xF0F0F0F0u);
-            o.bhi[j] = (i32x4)(p & 0xF0F0F0F0u);
-        }
-    };
-    auto multiply = [&](const Ops& o) {
-        // all even-k issues first, then all odd-k ones: consecutive MFMAs never share an accumulator
-#pragma unroll
-        for (int i = 0; i < IM; ++i)
-#pragma unroll
-            for (int j = 0; j < JN; ++j)
-                acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(o.blo[j], o.alo[i], acc[i][j], 0, 0, 0);
-#pragma unroll
-        for (int i = 0; i < IM; ++i)
-#pragma unroll
-            for (int j = 0; j < JN; ++j)
-                acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(o.bhi[j], o.ahi[i], acc[i][j], 0, 0, 0);
-    };
-
-    Ops ops;
-    int bcur = 0;
-    // Global loads run one stage ahead of the LDS fill: stage ks+2 is written to LDS during
-    // iteration ks from registers requested at the end of iteration ks-1.  The first three stages
-    // are requested together: the accumulators are not live yet, so two more register sets are
-    // free, and the prologue costs one memory round trip instead of three.
-    u32x4 regs[NL];
-    {
-        u32x4 first[NL], second[NL];
-        fetch(0, first);
-        fetch(1, second);
-        fetch(2, regs);
-        deposit(0, 0, first);
-        deposit(1, 1, second);
-    }
-    __syncthreads();                                    // stages 0 and 1 visible
-    if (kg == 1) load_ops(0, 0, ops);                   // group 1 starts one unpack ahead
-    for (int ks = 0; ks < stages; ++ks) {
-        const int bnext = bcur == NBUF - 1 ? 0 : bcur + 1;
-        const int bfill = bnext == NBUF - 1 ? 0 : bnext + 1;
-        if (kg == 0) {
-            load_ops(bcur, 0, ops);
-            multiply(ops);
-            load_ops(bcur, 1, ops);
-            multiply(ops);
-        } else {
-            multiply(ops);                              // sub-step 2 of this stage (unpacked earlier)
-            load_ops(bcur, 1, ops);
-            multiply(ops);                              // sub-step 3
-            if (ks + 1 < stages) load_ops(bnext, 0, ops);   // next stage's sub-step 2
-        }
-        deposit(ks + 2, bfill, regs);
-        fetch(ks + 3, regs);
-        __syncthreads();
-        bcur = bnext;
-    }
-
-    // K-split: group 0 finalises the lower half of the j tiles and group 1 the upper half; each sends
-    // the other half across, one row of MFMA tiles (i) per round, four 16-byte pieces per lane.
-    const int j_first = kg * JH;
-    {
-        u32x4* xbuf = ks_lds;
-        const int send0 = (1 - kg) * JH;
-        for (int i = 0; i < IM; ++i) {
-            __syncthreads();
-#pragma unroll
-            for (int jj = 0; jj < JH; ++jj)
-#pragma unroll
-                for (int qv = 0; qv < 4; ++qv) {
-                    const int slot = (((wxy * 2 + (1 - kg)) * JH + jj) * 4 + qv) * 64 + lane;
-                    i32x4 piece;
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        int val = 0;
-#pragma unroll
-                        for (int ii = 0; ii < IM; ++ii)
-#pragma unroll
-                            for (int jx = 0; jx < JN; ++jx)
-                                if (ii == i && jx == send0 + jj) val = acc[ii][jx][qv * 4 + e];
-                        piece[e] = val;
-                    }
-                    xbuf[slot] = (u32x4)piece;
-                }
-            __syncthreads();
-#pragma unroll
-            for (int jj = 0; jj < JH; ++jj)
-#pragma unroll
-                for (int qv = 0; qv < 4; ++qv) {
-                    const int slot = (((wxy * 2 + kg) * JH + jj) * 4 + qv) * 64 + lane;
-                    const i32x4 piece = (i32x4)xbuf[slot];
-#pragma unroll
-                    for (int ii = 0; ii < IM; ++ii)
-#pragma unroll
-                        for (int jx = 0; jx < JN; ++jx)
-                            if (ii == i && jx == j_first + jj) {
-#pragma unroll
-                                for (int e = 0; e < 4; ++e) acc[ii][jx][qv * 4 + e] += piece[e];
-                            }
-                }
-        }
-    }
-
-    // Epilogue: lane l, register v -> n = (v/4)*8 + (l/32)*4 + v%4, m = l%32.
-    // column scales (and bias) of this lane's 4-column groups, fetched up front as 8-byte vectors
-    f16x4 sb4[JH][4], bi4[JH][4];                          // only the j tiles this K-group stores
-    if (DEQ) {
-#pragma unroll
-        for (int jj = 0; jj < JH; ++jj)
-#pragma unroll
-            for (int gq = 0; gq < 4; ++gq) {
-                const int col = n0 + wn * TN + (j_first + jj) * 32 + gq * 8 + khalf * 4;
-                if (col + 4 <= N && (N & 3) == 0) {
-                    sb4[jj][gq] = *(const f16x4*)(sB + col);
-                    if (bias) bi4[jj][gq] = *(const f16x4*)(bias + col);
-                } else {
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        const int cc = col + e < N ? col + e : N - 1;
-                        sb4[jj][gq][e] = sB[cc];
-                        if (bias) bi4[jj][gq][e] = bias[cc];
-                    }
-                }
-            }
-    }
-    // tiles of an fp16 output whose columns all exist leave as full rows through LDS (each K-group its 64 columns)
-    const bool by_rows = DEQ && n0 + BN <= N && (N & 7) == 0 && (((uintptr_t)Y) & 15) == 0;
-    if (DEQ && by_rows) __syncthreads();                    // the exchange buffers are no longer read
-#pragma unroll
-    for (int i = 0; i < IM; ++i) {
-        const int row = m0 + wm * TM + i * 32 + (lane & 31);
-        if (DEQ && by_rows) {
-            const int row0 = m0 + wm * TM + i * 32;           // (rows past M: computed on a clamped scale, not stored)
-            if (row0 >= M) continue;
-            const f16 sa = sA[min(row, M - 1)];
-            f16x4 o[JH][4];
-#pragma unroll
-            for (int j = 0; j < JN; ++j) {
-                if (j < j_first || j >= j_first + JH) continue;
-#pragma unroll
-                for (int gq = 0; gq < 4; ++gq)
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        f16 yv = (f16)(sa * sb4[j % JH][gq][e]) * (f16)(float)(acc[i][j][gq * 4 + e] >> 8);
-                        if (bias) yv = yv + bi4[j % JH][gq][e];
-                        o[j % JH][gq][e] = yv;
-                    }
-            }
-            store_slab_rows<JH>((u32x2*)(ks_lds + wave * (32 * JH * 32 * 2 / 16)), o, lane,
-                                Y + (int64_t)row0 * N + n0 + wn * TN + j_first * 32, N, M - row0);
-            continue;
-        }
-        if (row >= M) continue;
-        f16 sa = (f16)0;
-        if (DEQ) sa = sA[row];
-#pragma unroll
-        for (int j = 0; j < JN; ++j) {
-            if (j < j_first || j >= j_first + JH) continue;     // the other K-group stores this tile
-#pragma unroll
-            for (int gq = 0; gq < 4; ++gq) {
-                const int col = n0 + wn * TN + j * 32 + gq * 8 + khalf * 4;
-                if (col >= N) continue;
-                int v4[4];
-#pragma unroll
-                for (int e = 0; e < 4; ++e) v4[e] = acc[i][j][gq * 4 + e] >> 8;
-                const bool whole = (col + 4 <= N) && ((N & 3) == 0);
-                if (DEQ) {
-                    f16 o[4];
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        f16 yv = (f16)(sa * sb4[j % JH][gq][e]) * (f16)(float)v4[e];
-                        if (bias) yv = yv + bi4[j % JH][gq][e];
-                        o[e] = yv;
-                    }
-                    f16* yp = Y + (int64_t)row * N + col;
-                    if (whole) {
-                        *(f16x4*)yp = f16x4{o[0], o[1], o[2], o[3]};
-                    } else {
-#pragma unroll
-                        for (int e = 0; e < 4; ++e)
-                            if (col + e < N) yp[e] = o[e];
-                    }
-                } else {
-                    int32_t* cp = C + (int64_t)row * N + col;
-                    if (whole) {
-                        *(i32x4*)cp = i32x4{v4[0], v4[1], v4[2], v4[3]};
-                    } else {
-#pragma unroll
-                        for (int e = 0; e < 4; ++e)
-                            if (col + e < N) cp[e] = v4[e];
-                    }
-                }
-            }
-        }
-    }
-}
-
-// ------------------------------------------------------------------------------------------------
-template <int BM, int BN, int WAVES_M, int WAVES_N>
-int launch_ks(const void* A, const void* B, int M, int N, int Kb, void* C, void* Y, const void* sA, const void* sB,
-              const void* bias, hipStream_t st, int ksplit = 1) {
-    constexpr int NT = 128 * WAVES_M * WAVES_N;
-    constexpr size_t STAGES = (size_t)3 * (BM + BN) * 8 * 16;
-    constexpr size_t XCH = (size_t)WAVES_M * WAVES_N * 2 * (BN / WAVES_N / 64) * 256 * 16;
-    constexpr size_t LDS = STAGES > XCH ? STAGES : XCH;
-    const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
-    const int64_t tiles = (int64_t)tiles_m * tiles_n * ksplit;
-    if (tiles > 0x3fffffff) return QR_E_SHAPE;
-    if (ksplit > 1 && Y) return QR_E_UNSUPPORTED;           // partial sums exist only as int32
-    const int nxcd = qr_device().xcds;                      // the grid is a whole number of rounds over the XCDs
-    const unsigned grid = (unsigned)((tiles + nxcd - 1) / nxcd * nxcd);
-    hipError_t e;
-    if (Y) {
-        auto kern = gemm_ks_kernel<BM, BN, WAVES_M, WAVES_N, true>;
-        e = qr_allow_dynamic_lds((const void*)kern, LDS);
-        if (e != hipSuccess) return (int)e;
-        kern<<<dim3(grid), dim3(NT), LDS, st>>>((const uint8_t*)A, (const uint8_t*)B, M, N, Kb, nullptr, (f16*)Y,
-                                                (const f16*)sA, (const f16*)sB, (const f16*)bias, tiles_m, tiles_n, 1, nxcd);
-    } else {
-        auto kern = gemm_ks_kernel<BM, BN, WAVES_M, WAVES_N, false>;
-        e = qr_allow_dynamic_lds((const void*)kern, LDS);
-        if (e != hipSuccess) return (int)e;
-        kern<<<dim3(grid), dim3(NT), LDS, st>>>((const uint8_t*)A, (const uint8_t*)B, M, N, Kb, (int32_t*)C, nullptr,
-                                                nullptr, nullptr, nullptr, tiles_m, tiles_n, ksplit, nxcd);
-    }
-    return qr_launch_status();
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -2153,15 +1796,6 @@ __global__ __launch_bounds__(256) void dequant_slabs_kernel(const int32_t* __res
     }
 }
 
-// Number of K slices for the 64x256-tile kernel, 1 when the shape has no use for a split.  Only
-// prompts of a few hundred tokens qualify (64 < M, fewer than 128 tiles of 128x256): decode batches
-// were measured no faster split than with the decode kernel.  A small cost model in microseconds
-// (6 for launch + prologue + epilogue, 2 more for the second launch, 1.0 per 256-k stage and round
-// of 256 workgroups, slabs written and re-read at 4 TB/s) picks the slice count, and the split is
-// used only when it promises a fifth less time.  Against a sweep of forced slice counts on
-// M = 96..768, N = 4096..12288, K = 4096..28672 the model is within 10 % and picks the measured
-// optimum or its neighbour (e.g. 256 x 4096 x 11008: 48 -> 26 us with four slices, 256 x 8192 x
-// 28672: 119 -> 78 us with two; 512 x 4096 x 4096 and 256 x 11008 x 4096 stay unsplit).
 // Decode against a weight with too few rows for the shared-token kernel to fill the CUs (70B down_proj: 8192 rows =
 // 64 blocks of four groups): at 40 and more tokens each CU's intake of the tokens' codes bounds the barrier-free
 // kernel.  With scratch from the caller the shared-token kernel runs with four groups per workgroup and as many K
@@ -2177,6 +1811,9 @@ int decode_split(int64_t M, int64_t N, int64_t Kb) {
     return s >= 2 ? (int)s : 1;
 }
 
+// How many int32 slabs of [M, N] a caller is asked to provide (qr_workspace_bytes): for prompts of a few hundred tokens an
+// upper bound of the slices that mid_plan may use, larger than it needs since its tiles fill the CUs without a split at
+// most of these shapes; callers size their scratch once per shape.
 int ks_split(int64_t M, int64_t N, int64_t Kb) {
     if (M <= 64) return decode_split(M, N, Kb);
     if (N <= 128) return 1;
@@ -2199,6 +1836,62 @@ int ks_split(int64_t M, int64_t N, int64_t Kb) {
     return best;
 }
 
+// Which kernel takes an output of more than 64 tokens, by an estimate in microseconds (st = stages of 256 k, n = tiles on the
+// busiest of the CUs; fitted to sweeps of 65 .. 1500 tokens against 1902 .. 28672 weight rows at K = 4096 .. 28672 with
+// every kernel forced, and within 10 % of them):
+//   64 x 64 tiles   4.2 + st (n = 1: 0.26, 2: 0.44, more: 0.25 n, from 8 on 0.26 n)      three workgroups share a CU
+//   64 x 128        4.6 + st (0.41 n, from the second on 0.52 n)
+//   128 x 128       5.0 + st (n = 1: 0.80, more: 0.92 n)
+//   128 / 192 / 256 x 256 (the pipelined kernels)   rounds (5.5 + {1.40, 2.19, 2.75} st (1 - {0.3, 0.5, 0.5} idle)), idle = share of
+//                   the rounds' places without a tile (the clock is higher then)
+// The small tiles are bound by the CUs' intake of operands, the pipelined ones by the matrix pipe, so the small ones lead
+// while the large ones leave CUs idle: 333 x 4096 x 4096 11.2 us (64 x 256 tiles on 96 CUs before: 21.8), 777 x 4096 x 4096
+// 17.7 (22.5), 512 x 8192 x 8192 32.1 (43.5), 1024 x 4096 x 11008 42 (56); 777 x 8192 x 8192 stays with 192- or 128-row
+// tiles (48 against 56), 200 x 28672 x 8192 too (48 against 57).
+// Very few tiles and a long K: slices of K over several workgroups with int32 slabs in the caller's scratch and a second
+// launch that adds them (+ 3.5 us and the slabs' way out and back at 4 TB/s).
+struct MidPlan {
+    int kernel;         // 0 .. 2: qr_internal_gemm_mid's shapes; 3, 4, 5: pipelined 128-, 192-, 256-row tiles
+    int split;
+};
+MidPlan mid_plan(int64_t M, int64_t N, int64_t Kb, int64_t max_split) {
+    const int64_t cus = qr_device().cus, st = (Kb + 127) / 128;
+    auto tiles = [&](int64_t bm, int64_t bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
+    auto loaded = [&](int64_t t) { return (double)((t + cus - 1) / cus); };
+    auto t64 = [&](int64_t t, int64_t stages) {
+        const double n = loaded(t);
+        return 4.2 + (double)stages * (n == 1 ? 0.26 : n == 2 ? 0.44 : n < 8 ? 0.25 * n : 0.26 * n);
+    };
+    MidPlan best{0, 1};
+    double t_best = t64(tiles(64, 64), st);
+    auto consider = [&](int kernel, int split, double t) {
+        if (t < t_best) {
+            t_best = t;
+            best = MidPlan{kernel, split};
+        }
+    };
+    const double n128 = loaded(tiles(64, 128));
+    consider(1, 1, 4.6 + (double)st * (n128 == 1 ? 0.41 : 0.52 * n128));
+    const double nsq = loaded(tiles(128, 128));
+    consider(2, 1, 5.0 + (double)st * (nsq == 1 ? 0.80 : 0.92 * nsq));
+    // Among the pipelined kernels taller tiles run faster per unit of work (3 unpacking instructions per MFMA at 256 rows,
+    // 3.5 at 192, 4.5 at 128) but quantise worse over the CUs: rounds of tiles are compared, a 128x256 tile costing 0.57
+    // and a 192x256 tile 0.80 of a 256x256 one (measured over 300..4096 tokens against 4096..27648 weight rows: rounds of
+    // 27-29 / 40-41 / 48-51 us at K = 4096; every one of those shapes gets the fastest of the three).  Ties go to the
+    // taller tile.
+    const double share[3] = {0.57, 0.80, 1.0}, slope[3] = {1.40, 2.19, 2.75};
+    int tall = 2;
+    for (int i = 1; i >= 0; --i)
+        if (loaded(tiles(128 + 64 * i, 256)) * share[i] < loaded(tiles(128 + 64 * tall, 256)) * share[tall]) tall = i;
+    const int64_t t = tiles(128 + 64 * tall, 256);
+    const double rounds = loaded(t);
+    const double idle = 1.0 - (double)t / (rounds * (double)cus);
+    consider(3 + tall, 1, rounds * (5.5 + slope[tall] * (double)st * (1.0 - (tall == 0 ? 0.3 : 0.5) * idle)));
+    for (int64_t ks = 2; ks <= max_split && ks <= st / 4; ++ks)
+        consider(0, (int)ks, t64(tiles(64, 64) * ks, (st + ks - 1) / ks) + 3.5 + 2.0 * (double)ks * (double)M * (double)N * 4.0 / 4.0e6);
+    return best;
+}
+
 int gemm_dispatch(const void* A, const void* B, int64_t M, int64_t N, int64_t K, void* C, void* Y, const void* sA,
                   const void* sB, const void* bias, hipStream_t st, void* ws = nullptr, size_t ws_bytes = 0) {
     if (M < 0 || N < 0 || K < 0) return QR_E_SHAPE;
@@ -2214,48 +1907,38 @@ int gemm_dispatch(const void* A, const void* B, int64_t M, int64_t N, int64_t K,
         if (M <= 128) return launch_cfg<128, 128, 2, 2>(A, B, m, n, kb, C, Y, sA, sB, bias, st);
         return launch_cfg<256, 256, 4, 2>(A, B, m, n, kb, C, Y, sA, sB, bias, st);
     }
-    const int64_t t256 = ((M + 255) / 256) * ((N + 255) / 256);
     // one to four tokens: the dot-product kernel -- except two to four tokens against a weight with enough rows for the
     // shared-token kernel, which is ahead there (57344 x 8192: 40.2 against 42.9 us)
     if (M == 1 || (M <= 4 && decode_xs_groups(n) == 0)) return launch_gemv(A, B, m, n, kb, C, Y, sA, sB, bias, st);
-    // too few tiles for the CUs: split K across workgroups when the caller passed scratch for the
-    // slices' partial sums
-    const int split = ks_split(M, N, kb);
-    if (split > 1 && Y && ws && ws_bytes >= (size_t)split * (size_t)M * (size_t)N * 4 && ((uintptr_t)ws & 15) == 0) {
-        int rc = M <= 64 ? launch_decode_xs(A, B, m, n, kb, ws, nullptr, nullptr, nullptr, nullptr, st, 4, split)
-                         : launch_ks<64, 256, 1, 4>(A, B, m, n, kb, ws, nullptr, nullptr, nullptr, nullptr, st, split);
-        if (rc != QR_OK) return rc;
+    // the slabs of a K split go to scratch from the caller; without it (or with too little) the single-launch kernels run
+    const bool scratch = Y && ws && ((uintptr_t)ws & 15) == 0;
+    auto add_slabs = [&](int split) {
         int64_t db = (M * N / 4 + 255) / 256;
         db = db < 1 ? 1 : (db > 4096 ? 4096 : db);
         dequant_slabs_kernel<<<dim3((unsigned)db), dim3(256), 0, st>>>((const int32_t*)ws, split, (const f16*)sA,
                                                                       (const f16*)sB, (const f16*)bias, M, N, (f16*)Y);
         return qr_launch_status();
-    }
+    };
     if (M <= 64) {
+        const int split = decode_split(M, N, kb);
+        if (split > 1 && scratch && ws_bytes >= (size_t)split * (size_t)M * (size_t)N * 4) {
+            const int rc = launch_decode_xs(A, B, m, n, kb, ws, nullptr, nullptr, nullptr, nullptr, st, 4, split);
+            return rc != QR_OK ? rc : add_slabs(split);
+        }
         // weight streaming: with enough groups of 32 rows to fill the CUs the kernel that shares the
         // tokens' codes through LDS (they are read once per workgroup); otherwise the barrier-free
         // kernel in which the waves of a workgroup split K over groups of 32 rows
         if (const int rg = decode_xs_groups(n)) return launch_decode_xs(A, B, m, n, kb, C, Y, sA, sB, bias, st, rg);
         return launch_decode(A, B, m, n, kb, C, Y, sA, sB, bias, st);
     }
-    const int64_t t128x256 = ((M + 127) / 128) * ((N + 255) / 256);
-    const int64_t cus = qr_device().cus;
-    if (t128x256 >= cus / 2) {
-        // Taller tiles run faster per unit of work (3 unpacking instructions per MFMA at 256 rows, 3.5 at 192,
-        // 4.5 at 128) but quantise worse over the 256 CUs: compare rounds of tiles, a 128x256 tile costing 0.57
-        // and a 192x256 tile 0.80 of a 256x256 one (measured over 300..4096 tokens against 4096..27648 weight
-        // rows: rounds of 27-29 / 40-41 / 48-51 us at K = 4096; with these ratios every one of those shapes gets
-        // the fastest kernel).  Ties go to the taller tile.
-        const int64_t t192 = ((M + 191) / 192) * ((N + 255) / 256);
-        const double rounds256 = (double)((t256 + cus - 1) / cus);
-        const double rounds192 = (double)((t192 + cus - 1) / cus) * 0.80;
-        const double rounds128 = (double)((t128x256 + cus - 1) / cus) * 0.57;
-        if (rounds256 <= rounds128 && rounds256 <= rounds192) return launch_sp256(A, B, m, n, kb, C, Y, sA, sB, bias, st);
-        if (rounds192 <= rounds128) return launch_sp256(A, B, m, n, kb, C, Y, sA, sB, bias, st, 192);
-        return launch_spk(A, B, m, n, kb, C, Y, sA, sB, bias, st);
+    const MidPlan plan = mid_plan(M, N, kb, scratch ? (int64_t)(ws_bytes / ((size_t)M * (size_t)N * 4)) : 1);
+    if (plan.split > 1) {
+        const int rc = qr_internal_gemm_mid(plan.kernel, A, B, m, n, kb, ws, nullptr, nullptr, nullptr, nullptr, st, plan.split);
+        return rc != QR_OK ? rc : add_slabs(plan.split);
     }
-    if (N > 128) return launch_ks<64, 256, 1, 4>(A, B, m, n, kb, C, Y, sA, sB, bias, st);
-    return launch_cfg<128, 128, 2, 2>(A, B, m, n, kb, C, Y, sA, sB, bias, st);
+    if (plan.kernel <= 2) return qr_internal_gemm_mid(plan.kernel, A, B, m, n, kb, C, Y, sA, sB, bias, st, 1);
+    if (plan.kernel == 3) return launch_spk(A, B, m, n, kb, C, Y, sA, sB, bias, st);
+    return launch_sp256(A, B, m, n, kb, C, Y, sA, sB, bias, st, plan.kernel == 4 ? 192 : 256);
 }
 
 }  // namespace

@@ -475,6 +475,35 @@ def test_linear_with_workspace_splits_k_and_matches_bit_for_bit(m, n, k):
         assert np.array_equal(bits(y.cpu().numpy()), bits(want))
 
 
+@pytest.mark.parametrize("m,n,k", [(65, 64, 64), (65, 130, 192), (128, 257, 320), (129, 200, 832), (200, 1902, 1088),      # 64 x 64 tiles
+                                   (300, 4096, 3648), (320, 4104, 3584),                                               # 64 x 128
+                                   (777, 4096, 1088), (640, 4100, 2240)])                                              # 128 x 128
+def test_linear_on_small_tiles_bit_exact_at_tile_and_stage_edges(m, n, k):
+    """Outputs of few tiles (gemm_mid_kernel, its three tile shapes): token counts and weight rows that end inside a tile,
+    fewer stages of 256 k than stage buffers, a K that ends after one, two or three of a stage's four sub-steps (only the
+    K-groups inside it multiply).  fp16 and int32 outputs against the oracle, inside a guard band."""
+    rng = np.random.default_rng(m + n + k)
+    a = rng.integers(0, 256, (m, k // 2), dtype=np.uint8)
+    w = rng.integers(0, 256, (n, k // 2), dtype=np.uint8)
+    a[0, :], w[0, :] = 0x88, 0x88                                  # the largest possible sum: 64 k
+    sa = (np.abs(rng.standard_normal(m)) * 0.2 + 0.01).astype(F16)
+    sw = (np.abs(rng.standard_normal(n)) * 0.01 + 0.001).astype(F16)
+    bias = rng.standard_normal(n).astype(F16)
+    ga, gw, gsa, gsw, gb = gpu(a), gpu(w), gpu(sa), gpu(sw), gpu(bias)
+    L, st = _lib.lib(), torch.cuda.current_stream().cuda_stream
+    cols = np.unique(np.concatenate([np.arange(0, n, 37), np.arange(max(0, n - 70), n)]))
+    for b, nb in ((gb, bias), (None, None)):
+        guarded = torch.full((m * n + 64,), 7.0, dtype=torch.float16, device="cuda")
+        y = guarded[32:-32].view(m, n)
+        _lib.check(L.qr_linear_i4_f16(ga.data_ptr(), gsa.data_ptr(), gw.data_ptr(), gsw.data_ptr(),
+                                      0 if b is None else b.data_ptr(), m, n, k, y.data_ptr(), st))
+        want = o.linear4bit(a, sa, w[cols], sw[cols], None if nb is None else nb[cols])
+        assert np.array_equal(bits(y[:, cols].cpu().numpy()), bits(want))
+        assert bool((guarded[:32] == 7).all()) and bool((guarded[-32:] == 7).all())
+    got = quarot_amd.matmul(ga, gw)[:, cols].cpu().numpy()
+    assert np.array_equal(got, o.int4_matmul(a, w[cols]))
+
+
 def test_linear4bit_module_from_float_and_state_dict():
     w = (torch.randn(96, 128, generator=torch.Generator().manual_seed(4)) * 0.02).half()
     s = (w.abs().amax(dim=1, keepdim=True) / 7).half()
