@@ -105,6 +105,14 @@ int qr_hadamard_quantize_f16_i4(const void* x, int64_t rows, int n, int K, const
                                 void* y_or_null, void* stream);
 
 /*
+ * RMSNorm.forward without a gain (quarot/nn/normalization.py:15-21):
+ *   y[r, c] = fp16( float(x[r, c]) * 1/sqrt( sum_c x[r, c]^2 / mean_dim + eps ) ), sums and products in fp32;
+ * the rows that qr_rmsnorm_quantize_f16_i4 quantises, bit for bit.
+ *   x, y fp16 [rows, cols], 16-byte aligned, cols a multiple of 8 and <= 32768 (QR_E_UNSUPPORTED otherwise); y may alias x.
+ */
+int qr_rmsnorm_f16(const void* x, int64_t rows, int64_t cols, int mean_dim, float eps, void* y, void* stream);
+
+/*
  * Fused RMSNorm + Quantizer: the chain in front of q/k/v_proj and gate/up_proj
  * (quarot/nn/normalization.py:15-21 then quarot/nn/quantization.py:9-13; chained in
  * e2e/quantized_llama/modeling_llama.py:40-44,108-110).

@@ -19,7 +19,7 @@ from . import nn
 
 __all__ = [
     "matmul", "sym_quant", "sym_dequant", "PackedQuantizedTensor",      # the reference's names
-    "quantize_rows", "hadamard_quantize", "rmsnorm_quantize", "heads_hadamard_quantize", "linear_i4", "quantized_linear", "convert_i4_f6", "linear_f6",   # fused entry points
+    "quantize_rows", "hadamard_quantize", "rmsnorm", "rmsnorm_quantize", "heads_hadamard_quantize", "linear_i4", "quantized_linear", "convert_i4_f6", "linear_f6",   # fused entry points
 ]
 
 
@@ -215,6 +215,18 @@ def hadamard_quantize(x, hadK, K, clip_ratio=1.0, force_fp32=False, return_trans
     s_shape = tuple(lead[:1]) + (1,) + tuple(lead[1:])
     packed = PackedQuantizedTensor(q.view(*lead, q.shape[-1]), s.view(s_shape))
     return (packed, y.view(x.shape)) if return_transformed else packed
+
+
+def rmsnorm(x, mean_dim, eps=1e-5):
+    """RMSNorm.forward of fp16 rows in one kernel (quarot/nn/normalization.py:15-21)."""
+    assert x.dtype == torch.float16
+    x2, _ = _flat2d(x)
+    dev = _require_gpu_contiguous("rmsnorm", x=x2)
+    y = torch.empty_like(x2)
+    with _lib.on_device(dev):
+        _lib.check(_lib.lib().qr_rmsnorm_f16(_ptr(x2), x2.shape[0], x2.shape[1], int(mean_dim), float(eps), _ptr(y),
+                                             _lib.stream_ptr(dev)))
+    return y.view(x.shape)
 
 
 def rmsnorm_quantize(x, mean_dim, eps=1e-5, clip_ratio=1.0, return_normalized=False):

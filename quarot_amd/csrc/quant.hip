@@ -89,8 +89,11 @@ __device__ __forceinline__ float wave_sum_f32_dpp(float v) {
 // registers between the two reductions.  The normalised value is rounded to fp16 exactly where
 // the unfused chain stores it -- fp16( float(x) * rsqrt(sum(x^2) / mean_dim + eps) ), all in fp32 --
 // and the quantiser runs on those fp16 values.  Only the association order of the fp32 sum of
-// squares is this kernel's own.
-template <int NV>
+// squares is this kernel's own.  QUANT = false: the normalised rows alone (RMSNorm.forward), bound by memory -- 4 bytes
+// per value -- where the eight conversion, elementwise and reduction kernels of the same expression in torch move about
+// 34: 32768 x 4096 91 us = 5.9 TB/s; 333 x 4096 with the quantiser and three 4096-wide layers behind it 99.5 -> 65.9 us
+// (torch's kernels alone 29 us).
+template <int NV, bool QUANT>
 __global__ __launch_bounds__(QT) void rmsnorm_quant_rows_kernel(const u32x4* __restrict__ x, float mean_dim, float eps,
                                                                 float clip, int cols8, u32* __restrict__ q,
                                                                 f16* __restrict__ scale_out, u32x4* __restrict__ y) {
@@ -128,9 +131,18 @@ __global__ __launch_bounds__(QT) void rmsnorm_quant_rows_kernel(const u32x4* __r
             const f16x2 h = as_f16x2(v[i][w]);
             v[i][w] = narrow_f16x2((float)h[0] * r, (float)h[1] * r);
         }
+        if (!QUANT) continue;
         const u32 mi = absmax_bits8(v[i]);
         m = m > mi ? m : mi;
     }
+    if (!QUANT || y) {
+#pragma unroll
+        for (int i = 0; i < NV; ++i) {
+            const int c = threadIdx.x + i * QT;
+            if (c < cols8) y[row * (int64_t)cols8 + c] = v[i];
+        }
+    }
+    if (!QUANT) return;
     m = wave_max_u32_dpp(m);
     if (lane == 0) red[wave] = m;
     __syncthreads();
@@ -140,13 +152,6 @@ __global__ __launch_bounds__(QT) void rmsnorm_quant_rows_kernel(const u32x4* __r
     if (threadIdx.x == 0) scale_out[row] = sh;
     const float s = (float)sh;
     u32* qr = q + row * (int64_t)cols8;
-    if (y) {
-#pragma unroll
-        for (int i = 0; i < NV; ++i) {
-            const int c = threadIdx.x + i * QT;
-            if (c < cols8) y[row * (int64_t)cols8 + c] = v[i];
-        }
-    }
     if (fast_quant_ok(m, s)) {       // workgroup-uniform
         const FastRecip fr = make_fast_recip(s);
 #pragma unroll
@@ -384,21 +389,16 @@ extern "C" int qr_quantize_rows_f16_i4(const void* x, float clip, int64_t rows, 
     return launch_quant<false>(x, nullptr, clip, rows, cols, q, scales, (hipStream_t)stream);
 }
 
-extern "C" int qr_rmsnorm_quantize_f16_i4(const void* x, int64_t rows, int64_t cols, int mean_dim, float eps, float clip,
-                                          void* q, void* scales, void* y_or_null, void* stream) {
-    if (rows < 0 || cols <= 0 || mean_dim <= 0) return QR_E_SHAPE;
-    if (rows == 0) return QR_OK;
-    if (rows > 0x7fffffffLL) return QR_E_SHAPE;
-    if (!x || !q || !scales) return QR_E_NULL;
-    if (cols % 8 != 0 || cols > 32768) return QR_E_UNSUPPORTED;
-    if (((uintptr_t)x & 15) || ((uintptr_t)y_or_null & 15) || ((uintptr_t)q & 3)) return QR_E_ALIGN;
+namespace {
+template <bool QUANT>
+int launch_rmsnorm(const void* x, int64_t rows, int64_t cols, int mean_dim, float eps, float clip, void* q, void* scales,
+                   void* y, hipStream_t st) {
     const int cols8 = (int)(cols / 8);
     const int nv = (cols8 + QT - 1) / QT;
     dim3 grid((unsigned)rows), block(QT);
-    hipStream_t st = (hipStream_t)stream;
-#define QR_LAUNCH(NV)                                                                                                 \
-    rmsnorm_quant_rows_kernel<NV><<<grid, block, 0, st>>>((const u32x4*)x, (float)mean_dim, eps, clip, cols8, (u32*)q, \
-                                                          (f16*)scales, (u32x4*)y_or_null)
+#define QR_LAUNCH(NV)                                                                                                       \
+    rmsnorm_quant_rows_kernel<NV, QUANT><<<grid, block, 0, st>>>((const u32x4*)x, (float)mean_dim, eps, clip, cols8, (u32*)q, \
+                                                                 (f16*)scales, (u32x4*)y)
     if (nv <= 1) QR_LAUNCH(1);
     else if (nv <= 2) QR_LAUNCH(2);
     else if (nv <= 4) QR_LAUNCH(4);
@@ -407,6 +407,28 @@ extern "C" int qr_rmsnorm_quantize_f16_i4(const void* x, int64_t rows, int64_t c
     else QR_LAUNCH(16);
 #undef QR_LAUNCH
     return qr_launch_status();
+}
+}  // namespace
+
+extern "C" int qr_rmsnorm_quantize_f16_i4(const void* x, int64_t rows, int64_t cols, int mean_dim, float eps, float clip,
+                                          void* q, void* scales, void* y_or_null, void* stream) {
+    if (rows < 0 || cols <= 0 || mean_dim <= 0) return QR_E_SHAPE;
+    if (rows == 0) return QR_OK;
+    if (rows > 0x7fffffffLL) return QR_E_SHAPE;
+    if (!x || !q || !scales) return QR_E_NULL;
+    if (cols % 8 != 0 || cols > 32768) return QR_E_UNSUPPORTED;
+    if (((uintptr_t)x & 15) || ((uintptr_t)y_or_null & 15) || ((uintptr_t)q & 3)) return QR_E_ALIGN;
+    return launch_rmsnorm<true>(x, rows, cols, mean_dim, eps, clip, q, scales, y_or_null, (hipStream_t)stream);
+}
+
+extern "C" int qr_rmsnorm_f16(const void* x, int64_t rows, int64_t cols, int mean_dim, float eps, void* y, void* stream) {
+    if (rows < 0 || cols <= 0 || mean_dim <= 0) return QR_E_SHAPE;
+    if (rows == 0) return QR_OK;
+    if (rows > 0x7fffffffLL) return QR_E_SHAPE;
+    if (!x || !y) return QR_E_NULL;
+    if (cols % 8 != 0 || cols > 32768) return QR_E_UNSUPPORTED;
+    if (((uintptr_t)x & 15) || ((uintptr_t)y & 15)) return QR_E_ALIGN;
+    return launch_rmsnorm<false>(x, rows, cols, mean_dim, eps, 1.0f, nullptr, nullptr, y, (hipStream_t)stream);
 }
 
 extern "C" int qr_heads_hadamard_quantize_f16_i4(const void* x, int64_t rows, int heads, int head_dim,

@@ -952,6 +952,22 @@ def test_fused_rmsnorm_quantize(shape, clip):
     assert close(staged_y.cpu().numpy(), want_y)
 
 
+@pytest.mark.parametrize("rows,cols,mean_dim", [(1, 8, 8), (3, 2048, 2048), (2, 2056, 100), (5, 32768, 32768)])
+def test_rmsnorm_kernel_returns_the_rows_that_the_fused_front_quantises(rows, cols, mean_dim):
+    """RMSNorm.forward on fp16 GPU rows is the fused front's arithmetic without the quantiser: the same bits, within
+    tolerance of the oracle; a strided input and one that needs its gradient run through torch, to the same tolerance."""
+    x = gpu(synth_x(rows, cols, seed=cols))
+    y = quarot_amd.nn.RMSNorm(mean_dim)(x)
+    assert torch.equal(y, quarot_amd.rmsnorm_quantize(x, mean_dim, 1e-5, 1.0, return_normalized=True)[1])
+    want = o.rmsnorm(x.cpu().numpy(), mean_dim, 1e-5)
+    assert close(y.cpu().numpy(), want)
+    assert close(quarot_amd.nn.RMSNorm(mean_dim)(torch.cat([x, x], 1)[:, :cols]).cpu().numpy(), want)
+    leaf = x.clone().requires_grad_()
+    out = quarot_amd.nn.RMSNorm(mean_dim)(leaf)
+    out.float().sum().backward()
+    assert close(out.detach().cpu().numpy(), want) and leaf.grad is not None
+
+
 def test_fused_rmsnorm_quantize_full_size_and_errors():
     """Benchmark-size input (2048 x 4096) on strided rows; mean_dim different from the width;
     argument errors of the C entry point."""
