@@ -44,6 +44,9 @@ extern "C" {
  * of the transformed rows), QR_E_UNSUPPORTED with nothing launched otherwise: pass the table then. */
 #define QR_HADK_SIGNS 0x100
 
+/* Flag or-ed into qr_hadamard's `dtype` QR_DTYPE_F16 (see there). */
+#define QR_HAD_FP32 0x200
+
 /* Library version (major*10000 + minor*100 + patch). */
 int qr_version(void);
 
@@ -63,7 +66,8 @@ const char* qr_strerror(int code);
  *   scale   applied in fp32 after the butterflies (the reference passes 1/sqrt(n)).
  * Numerics: butterflies and scale in fp32.  QR_DTYPE_F16: the power-of-two stage is rounded to fp16
  * before the hadK stage, whose fp32 accumulation is rounded to fp16 (the reference's staging).
- * QR_DTYPE_F32: fp32 throughout.
+ * QR_DTYPE_F32: fp32 throughout.  QR_DTYPE_F16 | QR_HAD_FP32: x and y fp16, hadK fp32, no rounding to fp16 between the
+ * two factors (results to fp32 accuracy, rounded to fp16 once); QR_E_UNSUPPORTED for n <= 128.
  */
 int qr_hadamard(const void* x, void* y, int64_t rows, int n, int K, const void* hadK,
                 int dtype, float scale, void* stream);

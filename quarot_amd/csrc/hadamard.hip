@@ -2509,6 +2509,19 @@ extern "C" int qr_hadamard(const void* x, void* y, int64_t rows, int n, int K, c
     if (!x || !y || (K > 1 && !hadK)) return QR_E_NULL;
     if (((uintptr_t)x & 15) || ((uintptr_t)y & 15)) return QR_E_ALIGN;
     hipStream_t st = (hipStream_t)stream;
+    if (dtype == (QR_DTYPE_F16 | QR_HAD_FP32)) {
+        // fp16 rows through fp32-precision arithmetic (a program with force_fp32 that keeps its modules apart): one pass of
+        // 4 bytes per value instead of the 20 of a conversion, the fp32 transform and a conversion back -- 1178 x 13824
+        // 129 -> 39 us, 2048 x 5120 65 -> 17, 122 x 28672 69 -> 11, 1777 x 28672 455 -> 51.  Rows of 128 and shorter keep those three steps.
+        if (n <= 128) return QR_E_UNSUPPORTED;
+        if (K == 1 && pow2_split(n))
+            return launch_hadamard_mm<true, false>(x, y, rows, n, pow2_split(n), nullptr, scale, 1.f, nullptr, nullptr, st);
+        if (bm_applies(n, K) && n / K == 1024)
+            return launch_hadamard_bm<false, true>(x, y, rows, n, K, hadK, scale, 1.f, nullptr, nullptr, st);
+        if (mm_applies(n, K))
+            return launch_hadamard_mm<true, false>(x, y, rows, n, K, hadK, scale, 1.f, nullptr, nullptr, st);
+        return launch_hadamard<f16, true, false>(x, y, rows, n, K, hadK, scale, 1.f, nullptr, nullptr, st);
+    }
     if (tiny_applies(n, K)) {
         if (dtype == QR_DTYPE_F16) return launch_hadamard_tiny<f16>(x, y, rows, n, K, hadK, scale, st);
         if (dtype == QR_DTYPE_F32) return launch_hadamard_tiny<float>(x, y, rows, n, K, hadK, scale, st);

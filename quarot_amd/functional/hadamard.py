@@ -137,6 +137,24 @@ def matmul_hadU_cuda(X, hadK, K):
     return _run(X, hadK if K > 1 else None, K, scale).reshape(X.shape)
 
 
+def matmul_hadU_cuda_fp32(X, hadK, K):
+    """matmul_hadU_cuda(X.float(), hadK, K) rounded to X's fp16, in one pass over fp16 rows on the GPU; the two conversions
+    around the fp32 transform where the library has no such kernel (rows of 128 and shorter, beyond 32768)."""
+    n = X.shape[-1]
+    if 128 < n <= MAX_FUSED_ROW and (K == 1 or hadK is not None):
+        xc = X.contiguous()
+        table = None if K == 1 else hadK.to(device=xc.device, dtype=torch.float32).contiguous()
+        y = torch.empty_like(xc)
+        with _lib.on_device(xc.device):
+            rc = _lib.lib().qr_hadamard(xc.data_ptr(), y.data_ptr(), xc.numel() // n, n, int(K),
+                                        None if table is None else table.data_ptr(), _lib.QR_DTYPE_F16 | _lib.QR_HAD_FP32,
+                                        had_scale(n), _lib.stream_ptr(xc.device))
+        if rc != _lib.QR_E_UNSUPPORTED:
+            _lib.check(rc)
+            return y.view(X.shape)
+    return matmul_hadU_cuda(X.float(), hadK, K).to(X.dtype)
+
+
 def matmul_hadUt_cuda(X, hadK, K):
     return matmul_hadU_cuda(X, hadK.T if hadK is not None else None, K)
 

@@ -21,6 +21,8 @@ class OnlineHadamard(torch.nn.Module):
     def forward(self, x):
         x_dtype = x.dtype
         if self.fp32_had:
+            if x_dtype == torch.float16 and x.is_cuda:
+                return quarot_amd.functional.hadamard.matmul_hadU_cuda_fp32(x, self.had_rem_dim, self.rem_dim)
             x = x.float()
         x = quarot_amd.functional.matmul_hadU_cuda(x, self.had_rem_dim, self.rem_dim)
         return x.to(x_dtype)

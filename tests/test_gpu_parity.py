@@ -968,6 +968,21 @@ def test_rmsnorm_kernel_returns_the_rows_that_the_fused_front_quantises(rows, co
     assert close(out.detach().cpu().numpy(), want) and leaf.grad is not None
 
 
+@pytest.mark.parametrize("n", [256, 4096, 11008, 13824, 17920, 14336, 28672])
+def test_online_hadamard_fp32_on_fp16_rows_is_the_fp32_transform_rounded_once(n):
+    """force_fp32 on fp16 rows in one pass (every kernel family behind it) against the fp32 transform of the same rows in
+    fp32 tensors: both carry fp32 accuracy (2^-20 of the row's root mean square), so a result is the same fp16 value or,
+    where the exact one lies that close to a rounding boundary, its neighbour."""
+    x = gpu(synth_x(33, n, seed=n))
+    had = quarot_amd.nn.OnlineHadamard(n, force_fp32=True).cuda()
+    y = had(x)
+    ref = quarot_amd.functional.matmul_hadU_cuda(x.float(), had.had_rem_dim, had.rem_dim)
+    assert y.dtype == torch.float16 and y.shape == x.shape
+    slack = 2.0 ** -10 * ref.abs() + 2.0 ** -20 * ref.pow(2).mean(1, keepdim=True).sqrt()
+    assert bool(((y.float() - ref).abs() <= slack).all()) and float((y == ref.half()).float().mean()) > 0.99
+    assert torch.equal(had(torch.cat([x, x], 1)[:, :n]), y)                   # strided rows
+
+
 def test_fused_rmsnorm_quantize_full_size_and_errors():
     """Benchmark-size input (2048 x 4096) on strided rows; mean_dim different from the width;
     argument errors of the C entry point."""
