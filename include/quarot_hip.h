@@ -47,6 +47,12 @@ extern "C" {
 /* Flag or-ed into qr_hadamard's `dtype` QR_DTYPE_F16 (see there). */
 #define QR_HAD_FP32 0x200
 
+/* Flag or-ed into q_had_mode of qr_kv_quant_append_batch_decode_f16_i4: the first 4 * batch_size * num_heads bytes of the
+ * workspace (an arrival counter per sequence and head) are zero, and no other launch uses them meanwhile.  A split along
+ * the sequence is then merged in the same launch, by the last workgroup of a pair to arrive, which leaves its counter at
+ * zero: a caller zeroes a new workspace once. */
+#define QR_DECODE_COUNTERS_ZERO 0x100
+
 /* Library version (major*10000 + minor*100 + patch). */
 int qr_version(void);
 
@@ -335,8 +341,8 @@ int qr_kv_quant_append_f16_i4(const void* k, const void* v, int64_t tokens, cons
  *   rtol 1e-3 / atol 1e-3 of the exact softmax over the dequantised cache.
  *   max_seq_len: an upper bound of the sequences' lengths if the caller knows one, else 0.  With it and a
  *   workspace of qr_batch_decode_workspace_bytes(batch_size, num_heads, max_seq_len) bytes (16-byte
- *   aligned) a small batch is split along the sequence over several workgroups per (sequence, head) and
- *   a second launch merges them; without, one workgroup serves each (sequence, head).
+ *   aligned: a counter per sequence and head, then the partial states) a small batch is split along the
+ *   sequence over several workgroups per (sequence, head) and a second launch merges them; without, one workgroup serves each (sequence, head).
  */
 size_t qr_batch_decode_workspace_bytes(int64_t batch_size, int num_heads, int64_t max_seq_len);
 int qr_batch_decode_i4(void* o, const void* q, const void* kv_data, const void* kv_param,
@@ -364,11 +370,12 @@ int qr_batch_decode_qhad_i4(void* o, const void* q, const void* kv_data, const v
  * append_indptr NULL) followed by qr_batch_decode_i4 / qr_batch_decode_qhad_i4 -- what
  * MultiLayerPagedKVCache4Bit.update and the callable it returns do for a decode step
  * (quarot/transformers/kv_cache.py:104-129,224-251).  The page tables already count the new token (it is the
- * LAST position of its sequence, as for qr_kv_quant_append_f16_i4); the first wave of every (sequence, head)
- * quantises the token's key (through H_128 when k_had_mode = 1) and value with the arithmetic of that entry
- * point -- the same codes, scales and zeros, written to the same page slots -- and attends to them from its
- * registers while the other waves walk the cached positions.
- *   k, v fp16 [batch_size, num_heads, 128] (16-byte aligned); q_had_mode 0 / 1 as the two entry points above;
+ * LAST position of its sequence, as for qr_kv_quant_append_f16_i4); the first two waves of every (sequence, head)
+ * quantise the token's key (through H_128 when k_had_mode = 1) and value with the arithmetic of that entry
+ * point -- the same codes, scales and zeros, written to the same page slots -- while the other waves walk the
+ * cached positions.
+ *   k, v fp16 [batch_size, num_heads, 128] (16-byte aligned); q_had_mode 0 / 1 as the two entry points above, optionally
+ *   | QR_DECODE_COUNTERS_ZERO (then also a split along the sequence is one launch);
  *   everything else as qr_batch_decode_i4.  A sequence whose page list is empty is skipped by the append and
  *   gets a NaN output row, as there.
  */

@@ -57,6 +57,7 @@ SIGNATURES = {
 QR_DTYPE_F16, QR_DTYPE_F32 = 0, 1
 QR_HADK_SIGNS = 0x100          # or-ed into a `mode`: hadK is passed as sign words (include/quarot_hip.h)
 QR_HAD_FP32 = 0x200            # or-ed into qr_hadamard's dtype: fp16 rows, fp32-precision arithmetic
+QR_DECODE_COUNTERS_ZERO = 0x100    # or-ed into q_had_mode of the one-launch decode step: the workspace's counters are zero
 QR_E_NULL, QR_E_SHAPE, QR_E_UNSUPPORTED = -1, -2, -3
 
 _lib = None

@@ -88,33 +88,118 @@ __device__ __forceinline__ float row_rotate(float v) {   // DPP row_ror within e
     return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, true));
 }
 
+// value held by lane (id ^ MASK), for the butterflies of the query's transform
+template <int MASK>
+__device__ __forceinline__ float butterfly(float t, int lane) {
+    // upper lane of a pair: partner - own, lower lane: own + partner
+    if constexpr (MASK == 16 || MASK == 32) {
+        const u32 w = __builtin_bit_cast(u32, t);
+        float lo, hi;
+        if constexpr (MASK == 16) {
+            const auto r = __builtin_amdgcn_permlane16_swap(w, w, false, false);
+            lo = __builtin_bit_cast(float, (u32)r[0]), hi = __builtin_bit_cast(float, (u32)r[1]);
+        } else {
+            const auto r = __builtin_amdgcn_permlane32_swap(w, w, false, false);
+            lo = __builtin_bit_cast(float, (u32)r[0]), hi = __builtin_bit_cast(float, (u32)r[1]);
+        }
+        return (lane & MASK) ? lo - hi : lo + hi;
+    } else {
+        const int i = __builtin_bit_cast(int, t);
+        int o;
+        if constexpr (MASK == 1) o = __builtin_amdgcn_mov_dpp(i, 0xB1, 0xF, 0xF, true);
+        else if constexpr (MASK == 2) o = __builtin_amdgcn_mov_dpp(i, 0x4E, 0xF, 0xF, true);
+        else if constexpr (MASK == 4) o = __builtin_amdgcn_ds_swizzle(i, 0x101F);
+        else o = __builtin_amdgcn_mov_dpp(i, 0x128, 0xF, 0xF, true);                    // row_ror:8 == xor 8
+        const float other = __builtin_bit_cast(float, o);
+        return (lane & MASK) ? other - t : t + other;
+    }
+}
+
+// sum over the two lanes 32 (or 16) apart of two registers at once: the lower lane ends with a's sum, the upper with b's
+template <int MASK>
+__device__ __forceinline__ float fold_pair(float a, float b) {
+    const u32 wa = __builtin_bit_cast(u32, a), wb = __builtin_bit_cast(u32, b);
+    if constexpr (MASK == 32) {
+        const auto r = __builtin_amdgcn_permlane32_swap(wa, wb, false, false);
+        return __builtin_bit_cast(float, (u32)r[0]) + __builtin_bit_cast(float, (u32)r[1]);
+    } else {
+        const auto r = __builtin_amdgcn_permlane16_swap(wa, wb, false, false);
+        return __builtin_bit_cast(float, (u32)r[0]) + __builtin_bit_cast(float, (u32)r[1]);
+    }
+}
+__device__ __forceinline__ float wave_total(float v) {      // of a value that the four lanes of a group share: sum over groups
+    v += row_rotate<0x124>(v);
+    v += row_rotate<0x128>(v);
+    v = fold_pair<16>(v, v);
+    return fold_pair<32>(v, v);
+}
+
+// the partial states of one (sequence, head) -> its output; eight states' loads are in flight at a time
+__device__ __forceinline__ void merge_states(const float* src, int splits, int dim, f16* o) {
+    auto get = [](const float* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
+    float M = -5e4f, D = 0.f, O = 0.f;
+    for (int s0 = 0; s0 < splits; s0 += 8) {
+        float m8[8], d8[8], o8[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            const float* p = src + (int64_t)(s0 + k < splits ? s0 + k : splits - 1) * 132;
+            m8[k] = get(p), d8[k] = get(p + 1), o8[k] = get(p + 4 + dim);
+        }
+        float top = M;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) top = __builtin_fmaxf(top, m8[k]);
+        const float keep = __builtin_amdgcn_exp2f(M - top);
+        D *= keep, O *= keep, M = top;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            const float w = s0 + k < splits ? __builtin_amdgcn_exp2f(m8[k] - M) : 0.f;
+            D = __builtin_fmaf(d8[k], w, D);
+            O = __builtin_fmaf(o8[k], w, O);
+        }
+    }
+    o[dim] = (f16)(O / D);
+}
+
 // ALIGNED: page_size is a multiple of 16, so the 16 positions of a wave step lie in one page.
-// NW: waves per workgroup (4 or 16): a (sequence, head) gets NW * splits waves in all.
+// NW: waves per workgroup (4, 8 or 16): a (sequence, head) gets NW * splits waves in all.
 // APPEND: the sequence's LAST position is the token of this step, and its key and value arrive as fp16 vectors
-// (knew, vnew: [batch, heads, 128]) instead of lying in the cache already: the first wave of the (sequence, head)
-// quantises them itself (kv_quant_one_vector: the bits of the quantise-and-append kernel), writes codes and parameters
-// to the position's page slot, and takes the position into its softmax state from its own registers; the walk over
-// the cache stops one position short.  A decode step is then ONE launch instead of append + attention.
+// (knew, vnew: [batch, heads, 128]) instead of lying in the cache already: the first two waves of the (sequence, head)
+// quantise the key and the value (kv_quant_one_vector: the bits of the quantise-and-append kernel), write codes and
+// parameters to the position's page slot, and leave the position's logit and its dequantised value in LDS as one more
+// softmax state for the merge; the walk over the cache stops one position short.  A decode step is then ONE launch
+// instead of append + attention.
+// Short sequences and small batches are bound by the fixed path of a workgroup, so it is kept short: every load that
+// depends on nothing but the workgroup's number (query, new key and value) is requested first, then the first step of the
+// cache; a wave transforms the query once, two values per lane (56 vector instructions instead of ~450 with 32 values in
+// every lane), and hands it to its lane groups through 256 bytes of LDS; at the end a wave folds its 16 lane groups into
+// one state by exchanging halves (64 instructions instead of 190 for four states), so one barrier and a merge of NW
+// states remain.
 template <bool ALIGNED, int NW, bool APPEND = false>
 __global__ __launch_bounds__(64 * NW, (NW == 16 ? 1 : NW == 8 ? 2 : 4)) void paged_decode_i4_kernel(
     const f16* __restrict__ q, PagedKV c, f16* __restrict__ o, float sm_scale_log2, int splits, float* __restrict__ part,
-    int q_had, const u32x4* __restrict__ knew = nullptr, const u32x4* __restrict__ vnew = nullptr, int k_had = 0) {
-    __shared__ float st[NW * 4 * 4 * 36];                  // [wave * 4 + row][quarter][m, d, -, -, acc[32]]
-    __shared__ float st2[(NW / 2) * 128 * 3];              // second merge level: [part][dimension][m, d, o]
-    __shared__ u32x4 fresh[APPEND ? 26 : 1];               // APPEND: staging [16], the new key's codes [4], the value's [4], parameters
+    int q_had, u32* __restrict__ arrived, const u32x4* __restrict__ knew = nullptr, const u32x4* __restrict__ vnew = nullptr,
+    int k_had = 0) {
+    __shared__ f32x4 st4[NW * 33];                         // per wave: [m, d, -, -], 128 outputs; before that the query (256 bytes)
+    __shared__ u32x4 fresh[APPEND ? 2 * 16 : 1];           // APPEND: staging of the quantising waves, then their codes
+    __shared__ float newv[APPEND ? 128 + 2 : 1];           // APPEND: the new position's value and its [m, d]
+    float* const st = (float*)st4;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int slot = lane >> 2, c4 = lane & 3;
     const int bh = blockIdx.x / splits, sp = blockIdx.x - bh * splits;
     const int b = bh / c.num_heads, h = bh - b * c.num_heads;
+    const u32 qword = ((const u32*)q)[(int64_t)bh * 64 + lane];          // dimensions 2 lane, 2 lane + 1
+    const bool appends = APPEND && sp == 0 && wave < 2;     // wave-uniform; wave 0: the key, wave 1: the value
+    u32x4 piece = {0, 0, 0, 0};
+    if (APPEND && appends) piece = (wave == 0 ? knew : vnew)[(int64_t)bh * 16 + (lane & 15)];
     const int p0 = c.indptr[b], npages = c.indptr[b + 1] - p0;
     const int seq_all = npages > 0 ? (npages - 1) * c.page_size + c.last_page_offset[b] : 0;
     const int seq_len = APPEND ? seq_all - 1 : seq_all;     // positions read from the cache
     if (npages <= 0) {
-        // A sequence without pages (uniform over the workgroup): nothing may be read -- its slice of kv_indices is
-        // empty, and so may be the whole list and the page pool.  The result is the empty softmax state, i.e. the
+        // A sequence without pages (uniform over the workgroups of the pair): nothing may be read -- its slice of kv_indices
+        // is empty, and so may be the whole list and the page pool.  The result is the empty softmax state, i.e. the
         // 0 / 0 that the loop below would arrive at (and the reference's kernel does).
         if (threadIdx.x < 128) {
-            if (splits == 1) {
+            if (splits == 1 || arrived) {
                 o[(int64_t)bh * 128 + threadIdx.x] = (f16)__builtin_nanf("");
             } else {
                 float* dst = part + (int64_t)blockIdx.x * 132;
@@ -128,114 +213,6 @@ __global__ __launch_bounds__(64 * NW, (NW == 16 ? 1 : NW == 8 ? 2 : 4)) void pag
         return;
     }
 
-    const bool appends = APPEND && sp == 0 && wave == 0;    // wave-uniform
-    if (APPEND && appends) {
-        const int64_t vec = (int64_t)bh * 16;
-        u32 W[8];
-        f16 sc, zp;
-        const int pos = seq_all - 1, it = pos / c.page_size, entry = pos - it * c.page_size;
-        const int64_t page = c.indices[p0 + it];
-        const bool page_ok = page >= 0 && page < c.num_pages;
-        const float hs = 0.08838834764831845f;                 // 1 / sqrt(128)
-        const u32x4 piece[2] = {knew[vec + (lane & 15)], vnew[vec + (lane & 15)]};      // both in flight at once
-#pragma unroll
-        for (int kv = 0; kv < 2; ++kv) {
-            if (kv == 0 && k_had) kv_quant_one_vector<true>(piece[0], fresh, hs, W, sc, zp);
-            else kv_quant_one_vector<false>(piece[kv], fresh, hs, W, sc, zp);
-            const u32 prm = pack_scale_zero(sc, zp);
-            const int hh = lane >> 5;
-            if (page_ok && (lane & 31) == 0) {
-                const int64_t s = paged_slot(c, page, kv, h, entry);
-                u32x4* dst = (u32x4*)c.data + s * 4 + 2 * hh;
-                dst[0] = u32x4{W[0], W[1], W[2], W[3]};
-                dst[1] = u32x4{W[4], W[5], W[6], W[7]};
-                if (hh == 0) c.param[s] = prm;
-            }
-            // for the position's own turn after the walk: pieces 2 hh, 2 hh + 1 of the 64 code bytes, and the parameters
-            if ((lane & 31) == 0) {
-                fresh[16 + 4 * kv + 2 * hh] = u32x4{W[0], W[1], W[2], W[3]};
-                fresh[16 + 4 * kv + 2 * hh + 1] = u32x4{W[4], W[5], W[6], W[7]};
-                if (hh == 0) ((u32*)(fresh + 24))[kv] = page_ok ? prm : 0u;
-                if (hh == 0 && kv == 0) ((u32*)(fresh + 24))[2] = page_ok ? 1u : 0u;
-            }
-            __builtin_amdgcn_wave_barrier();
-        }
-    }
-
-    // this lane's 32 query values as fp16 pairs in the order the codes are consumed: word j of a 16-byte
-    // piece holds dimensions 8 j .. 8 j + 7, and (word >> 4 i) & 0x000F000F isolates codes i and i + 4
-    f16x2 qp[4][4];
-    float ql = 0.f;                                        // sum of this lane's 32 values
-    {
-        const u32x4* qsrc = (const u32x4*)(q + (int64_t)bh * 128 + c4 * 32);
-        u32x4 qw[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) qw[j] = qsrc[j];
-        if (q_had) {
-            // The query's Hadamard over the head dimension (matmul_had_cuda on q, kv_cache.py:30-33,113) here instead of
-            // in a launch of its own: 128-point transform in fp32 -- five butterfly levels over the lane's 32 values,
-            // two across the four lanes of a position group -- times 1 / sqrt(128), rounded to fp16 like that
-            // function's result.
-            float t[32];
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-#pragma unroll
-                for (int k = 0; k < 4; ++k) {
-                    const f16x2 pr = as_f16x2(qw[j][k]);
-                    t[8 * j + 2 * k] = (float)pr[0];
-                    t[8 * j + 2 * k + 1] = (float)pr[1];
-                }
-#pragma unroll
-            for (int hb = 1; hb < 32; hb <<= 1)
-#pragma unroll
-                for (int i = 0; i < 32; ++i)
-                    if ((i & hb) == 0) {
-                        const float a = t[i], b = t[i + hb];
-                        t[i] = a + b;
-                        t[i + hb] = a - b;
-                    }
-#pragma unroll
-            for (int i = 0; i < 32; ++i) {
-                const float o1 = __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, t[i]), 0xB1, 0xF, 0xF, true));
-                t[i] = (c4 & 1) ? o1 - t[i] : t[i] + o1;                // lanes ^ 1: index bit 5
-                const float o2 = __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, t[i]), 0x4E, 0xF, 0xF, true));
-                t[i] = (c4 & 2) ? o2 - t[i] : t[i] + o2;                // lanes ^ 2: index bit 6
-            }
-            const float hs = 0.08838834764831845f;                       // 1 / sqrt(128)
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-#pragma unroll
-                for (int k = 0; k < 4; ++k) qw[j][k] = narrow_f16x2(t[8 * j + 2 * k] * hs, t[8 * j + 2 * k + 1] * hs);
-        }
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const u32x4 w = qw[j];
-            f16 e[8];
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                const f16x2 pr = as_f16x2(w[k]);
-                e[2 * k] = pr[0];
-                e[2 * k + 1] = pr[1];
-                ql += (float)pr[0] + (float)pr[1];
-            }
-#pragma unroll
-            for (int i = 0; i < 4; ++i) qp[j][i] = f16x2{e[i], e[i + 4]};
-        }
-    }
-    const float qs = quad_sum(ql);                         // sum of all 128 query values
-    float qbias = 0.f;                                     // sum over this lane's values of q * (bias of its code)
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-            qbias = __builtin_fmaf((float)qp[j][i][0] + (float)qp[j][i][1], (i & 1) ? kBiasOdd : kBiasEven, qbias);
-    u32 mask_lo = 0x000F000Fu, bias_lo = 0x64006400u, mask_hi = 0x00F000F0u, bias_hi = 0x54005400u;
-    asm volatile("" : "+v"(mask_lo), "+v"(bias_lo), "+v"(mask_hi), "+v"(bias_hi));     // kept in registers for v_and_or_b32
-
-    float m = -5e4f, d = 0.f, pz = 0.f, psum = 0.f, acc[32];
-#pragma unroll
-    for (int i = 0; i < 32; ++i) acc[i] = 0.f;
-
     const int chunks = (seq_len + 15) >> 4;
     // a vector's place: slot = page * page_slots + head_slots + entry (K), + kv_slots (V); 64 code bytes and
     // one parameter word per slot
@@ -246,10 +223,10 @@ __global__ __launch_bounds__(64 * NW, (NW == 16 ? 1 : NW == 8 ? 2 : 4)) void pag
     // ALIGNED: chunk g lies in page g / cpp at entry 16 (g % cpp); both advance without divisions
     const int cpp = ALIGNED ? c.page_size >> 4 : 1;
     const int it_step = stride / cpp, r_step = stride - it_step * cpp;
-    // APPEND: the wave that quantises the new token leaves its first two chunks (one step's worth) to its two
-    // neighbours, which take one each after their own walk: its extra work would otherwise stand at the launch's end
+    // APPEND: the wave that quantises the key leaves its first two chunks (one step's worth) to waves 2 and 3, which take
+    // one each after their own walk: its extra work would otherwise stand at the launch's end
     const int g_first = sp * NW + wave;
-    int g = g_first + ((APPEND && appends) ? stride * AU : 0);
+    int g = g_first + ((APPEND && appends && wave == 0) ? stride * AU : 0);
     int it_u = g / cpp, r_u = g - it_u * cpp;
     // Two sets of AU positions per lane group: the loads of the next set are issued before the current
     // one is consumed, so their latency hides under the arithmetic.  Loads are unconditional (a position
@@ -263,6 +240,7 @@ __global__ __launch_bounds__(64 * NW, (NW == 16 ? 1 : NW == 8 ? 2 : 4)) void pag
     auto issue = [&](Step& t, int g0) {
         int64_t page[AU];
         int entry[AU];
+        const int32_t* pp[AU];
         // page numbers first (scalar loads when ALIGNED), then every vector load of the step
 #pragma unroll
         for (int u = 0; u < AU; ++u) {
@@ -282,16 +260,18 @@ __global__ __launch_bounds__(64 * NW, (NW == 16 ? 1 : NW == 8 ? 2 : 4)) void pag
                 entry[u] = pos - it * c.page_size;
             }
             t.ok[u] = pos < seq_len && it < npages;
-            const int32_t* pp = c.indices + p0 + (it < npages ? it : 0);
-            if (ALIGNED) {
-                // a scalar load, spelled out: behind the scheduling barriers of the loop the compiler falls back
-                // to a vector load plus a wait for EVERY outstanding vector load, which would drain the pipeline
-                int pg;
-                asm volatile("s_load_dword %0, %1, 0x0\n\ts_waitcnt lgkmcnt(0)" : "=s"(pg) : "s"(pp) : "memory");
-                page[u] = pg;
-            } else {
-                page[u] = *pp;
-            }
+            pp[u] = c.indices + p0 + (it < npages ? it : 0);
+            if (!ALIGNED) page[u] = *pp[u];
+        }
+        if (ALIGNED) {
+            // scalar loads, spelled out and waited for together: behind the scheduling barriers of the loop the compiler
+            // falls back to vector loads plus a wait for EVERY outstanding vector load, which would drain the pipeline
+            static_assert(AU == 2, "two page numbers per step");
+            int pg0, pg1;
+            asm volatile("s_load_dword %0, %2, 0x0\n\ts_load_dword %1, %3, 0x0\n\ts_waitcnt lgkmcnt(0)"
+                         : "=&s"(pg0), "=&s"(pg1) : "s"(pp[0]), "s"(pp[1]) : "memory");
+            page[0] = pg0;
+            page[1] = pg1;
         }
 #pragma unroll
         for (int u = 0; u < AU; ++u) {
@@ -308,23 +288,122 @@ __global__ __launch_bounds__(64 * NW, (NW == 16 ? 1 : NW == 8 ? 2 : 4)) void pag
             t.vp[u] = *(const u32*)((const uint8_t*)(c.param + kbase + kv_slots) + e * 4u);
         }
     };
+    Step sa, sb;
+    if (!appends) issue(sa, g);                             // (the quantising waves: behind their quantiser, which needs the registers)
+    __builtin_amdgcn_sched_barrier(0);
+
+    // The query, with the Hadamard over the head dimension (matmul_had_cuda on q, kv_cache.py:30-33,113) here instead of in
+    // a launch of its own: 128-point transform in fp32 -- index bit 0 inside the lane, bits 1 .. 6 across lanes -- times
+    // 1 / sqrt(128), rounded to fp16 like that function's result.
+    // Then this lane's 32 query values as fp16 pairs in the order the codes are consumed: word j of a 16-byte
+    // piece holds dimensions 8 j .. 8 j + 7, and (word >> 4 i) & 0x000F000F isolates codes i and i + 4.
+    f16x2 qp[4][4];
+    float qs, qbias = 0.f;                                 // sum of all 128 values; sum over this lane's of q * (bias of its code)
+    {
+        u32 w = qword;
+        if (q_had) {
+            const f16x2 pr = as_f16x2(qword);
+            float t0 = (float)pr[0] + (float)pr[1], t1 = (float)pr[0] - (float)pr[1];
+            t0 = butterfly<1>(t0, lane), t1 = butterfly<1>(t1, lane);
+            t0 = butterfly<2>(t0, lane), t1 = butterfly<2>(t1, lane);
+            t0 = butterfly<4>(t0, lane), t1 = butterfly<4>(t1, lane);
+            t0 = butterfly<8>(t0, lane), t1 = butterfly<8>(t1, lane);
+            t0 = butterfly<16>(t0, lane), t1 = butterfly<16>(t1, lane);
+            t0 = butterfly<32>(t0, lane), t1 = butterfly<32>(t1, lane);
+            const float hs = 0.08838834764831845f;         // 1 / sqrt(128)
+            w = narrow_f16x2(t0 * hs, t1 * hs);
+        }
+        u32* const mine = (u32*)(st4 + wave * 33);         // private to the wave (LDS operations of one wave execute in order)
+        mine[lane] = w;
+        __builtin_amdgcn_wave_barrier();
+        float ql = 0.f;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const u32x4 v = ((const u32x4*)mine)[c4 * 4 + j];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) ql = __builtin_amdgcn_fdot2(as_f16x2(v[k]), f16x2{(f16)1.0f, (f16)1.0f}, ql, false);
+            qp[j][0] = as_f16x2(__builtin_amdgcn_perm(v[2], v[0], 0x05040100u));
+            qp[j][1] = as_f16x2(__builtin_amdgcn_perm(v[2], v[0], 0x07060302u));
+            qp[j][2] = as_f16x2(__builtin_amdgcn_perm(v[3], v[1], 0x05040100u));
+            qp[j][3] = as_f16x2(__builtin_amdgcn_perm(v[3], v[1], 0x07060302u));
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const f16 bi = (f16)((i & 1) ? kBiasOdd : kBiasEven);
+                qbias = __builtin_amdgcn_fdot2(qp[j][i], f16x2{bi, bi}, qbias, false);
+            }
+        }
+        qs = quad_sum(ql);
+        __builtin_amdgcn_wave_barrier();
+    }
+    u32 mask_lo = 0x000F000Fu, bias_lo = 0x64006400u, mask_hi = 0x00F000F0u, bias_hi = 0x54005400u;
+    asm volatile("" : "+v"(mask_lo), "+v"(bias_lo), "+v"(mask_hi), "+v"(bias_hi));     // kept in registers for v_and_or_b32
+
+    // logit of a position from its key's quarter: q . (bias + codes) with fp32 accumulation of exact products, minus
+    // sum(q * bias), over the four lanes of the position
+    auto logit = [&](u32x4 kw, u32 kp) {
+        float a0 = 0.f, a1 = 0.f;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const CodePairs cp = code_pairs(kw[j], mask_lo, bias_lo, mask_hi, bias_hi);
+            a0 = __builtin_amdgcn_fdot2(qp[j][0], as_f16x2(cp.p[0]), a0, false);
+            a1 = __builtin_amdgcn_fdot2(qp[j][1], as_f16x2(cp.p[1]), a1, false);
+            a0 = __builtin_amdgcn_fdot2(qp[j][2], as_f16x2(cp.p[2]), a0, false);
+            a1 = __builtin_amdgcn_fdot2(qp[j][3], as_f16x2(cp.p[3]), a1, false);
+        }
+        const float dot = quad_sum((a0 + a1) - qbias);
+        const f16x2 prm = as_f16x2(kp);
+        return (dot * (float)prm[0] - (float)prm[1] * qs) * sm_scale_log2;
+    };
+
+    if (APPEND && appends) {
+        u32 W[8];
+        f16 sc, zp;
+        const int pos = seq_all - 1, it = pos / c.page_size, entry = pos - it * c.page_size;
+        const int64_t page = c.indices[p0 + it];
+        const bool page_ok = page >= 0 && page < c.num_pages;
+        const float hs = 0.08838834764831845f;                 // 1 / sqrt(128)
+        u32x4* const stage = fresh + wave * 16;
+        if (wave == 0 && k_had) kv_quant_one_vector<true>(piece, stage, hs, W, sc, zp);
+        else kv_quant_one_vector<false>(piece, stage, hs, W, sc, zp);
+        const u32 prm = pack_scale_zero(sc, zp);
+        const int hh = lane >> 5;
+        if ((lane & 31) == 0) {
+            const u32x4 c0 = {W[0], W[1], W[2], W[3]}, c1 = {W[4], W[5], W[6], W[7]};
+            stage[2 * hh] = c0;                                // the position's 64 code bytes, for its own turn below
+            stage[2 * hh + 1] = c1;
+            if (page_ok) {
+                const int64_t s = paged_slot(c, page, wave, h, entry);
+                u32x4* dst = (u32x4*)c.data + s * 4 + 2 * hh;
+                dst[0] = c0;
+                dst[1] = c1;
+                if (hh == 0) c.param[s] = prm;
+            }
+        }
+        __builtin_amdgcn_wave_barrier();
+        if (wave == 0) {
+            const float lg = logit(stage[c4], prm);
+            if (lane == 0) {
+                newv[128] = page_ok ? lg : -__builtin_inff();
+                newv[129] = page_ok ? 1.f : 0.f;
+            }
+        } else {
+            const u32 byte = ((const uint8_t*)stage)[lane];
+            const float z = page_ok ? (float)zp : 0.f, s = page_ok ? (float)sc : 0.f;
+            newv[2 * lane] = (float)(byte & 15u) * s - z;
+            newv[2 * lane + 1] = (float)(byte >> 4) * s - z;
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        issue(sa, g);
+    }
+
+    float m = -5e4f, d = 0.f, pz = 0.f, psum = 0.f, acc[32];
+#pragma unroll
+    for (int i = 0; i < 32; ++i) acc[i] = 0.f;
     auto consume = [&](const Step& t) {
         float lg[AU], mx = m;
 #pragma unroll
         for (int u = 0; u < AU; ++u) {
-            // q . (bias + codes) with fp32 accumulation of exact products, minus sum(q * bias)
-            float a0 = 0.f, a1 = 0.f;
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const CodePairs cp = code_pairs(t.kw[u][j], mask_lo, bias_lo, mask_hi, bias_hi);
-                a0 = __builtin_amdgcn_fdot2(qp[j][0], as_f16x2(cp.p[0]), a0, false);
-                a1 = __builtin_amdgcn_fdot2(qp[j][1], as_f16x2(cp.p[1]), a1, false);
-                a0 = __builtin_amdgcn_fdot2(qp[j][2], as_f16x2(cp.p[2]), a0, false);
-                a1 = __builtin_amdgcn_fdot2(qp[j][3], as_f16x2(cp.p[3]), a1, false);
-            }
-            const float dot = quad_sum((a0 + a1) - qbias);
-            const f16x2 prm = as_f16x2(t.kp[u]);
-            const float x = (dot * (float)prm[0] - (float)prm[1] * qs) * sm_scale_log2;
+            const float x = logit(t.kw[u], t.kp[u]);
             lg[u] = t.ok[u] ? x : -__builtin_inff();
             mx = __builtin_fmaxf(mx, lg[u]);
         }
@@ -355,9 +434,7 @@ __global__ __launch_bounds__(64 * NW, (NW == 16 ? 1 : NW == 8 ? 2 : 4)) void pag
             }
         }
     };
-    Step sa, sb;
     const int gs = stride * AU;
-    issue(sa, g);
     for (; g < chunks; g += 2 * gs) {
         issue(sb, g + gs);
         __builtin_amdgcn_sched_barrier(0);                 // the compiler would otherwise sink the loads below the arithmetic
@@ -368,8 +445,8 @@ __global__ __launch_bounds__(64 * NW, (NW == 16 ? 1 : NW == 8 ? 2 : 4)) void pag
         if (g + gs < chunks) consume(sb);                  // (no loads inside: the branch does not disturb the wait counts)
         __builtin_amdgcn_sched_barrier(0);
     }
-    if (APPEND && sp == 0 && (wave == 1 || wave == 2)) {
-        const int extra = sp * NW + (wave == 2 ? stride : 0);           // the quantising wave's first or second chunk
+    if (APPEND && sp == 0 && (wave == 2 || wave == 3)) {
+        const int extra = wave == 3 ? stride : 0;                       // the first wave's first or second chunk
         if (extra < chunks) {
             it_u = extra / cpp;
             r_u = extra - it_u * cpp;
@@ -378,115 +455,96 @@ __global__ __launch_bounds__(64 * NW, (NW == 16 ? 1 : NW == 8 ? 2 : 4)) void pag
             consume(sb);
         }
     }
-    if (APPEND && appends) {
-        // the new position, from the codes this wave made: lane group 0 takes it, the others sit the turn out
-        Step tn;
-        const u32* prm = (const u32*)(fresh + 24);
-        const bool valid = prm[2] != 0u;
-#pragma unroll
-        for (int u = 0; u < AU; ++u) {
-            tn.kw[u] = fresh[16 + c4];
-            tn.vw[u] = fresh[20 + c4];
-            tn.kp[u] = prm[0];
-            tn.vp[u] = prm[1];
-            tn.ok[u] = u == 0 && slot == 0 && valid;
-        }
-        consume(tn);
-    }
-    // ---- merge: first the four lane groups of each row of 16 lanes (two DPP rotations: every lane ends
-    // with its row's state), then the NW * 4 row states of the workgroup through LDS
-#pragma unroll
-    for (int i = 0; i < 32; ++i) acc[i] -= __builtin_fmaf(psum, (i & 1) ? kBiasOdd : kBiasEven, pz);     // sum p (code scale - zero)
-#pragma unroll
-    for (int step = 0; step < 2; ++step) {
-        const float om = step == 0 ? row_rotate<0x124>(m) : row_rotate<0x128>(m);
-        const float od = step == 0 ? row_rotate<0x124>(d) : row_rotate<0x128>(d);
-        const float M = __builtin_fmaxf(m, om);
-        const float ws = __builtin_amdgcn_exp2f(m - M), wo = __builtin_amdgcn_exp2f(om - M);
-        d = __builtin_fmaf(d, ws, od * wo);
-#pragma unroll
-        for (int i = 0; i < 32; ++i) {
-            const float oa = step == 0 ? row_rotate<0x124>(acc[i]) : row_rotate<0x128>(acc[i]);
-            acc[i] = __builtin_fmaf(acc[i], ws, oa * wo);
-        }
-        m = M;
-    }
-    if ((lane & 12) == 0) {                                           // the first lane group of every row writes
-        float* mine = st + ((wave * 4 + (lane >> 4)) * 4 + c4) * 36;
-        mine[0] = m;
-        mine[1] = d;
-#pragma unroll
-        for (int i = 0; i < 32; ++i) mine[4 + i] = acc[i];
-    }
-    __syncthreads();
-    // two levels, so that no thread walks more than eight states: thread (part, dimension) merges the row
-    // states part, part + PARTS, ...; then 128 threads merge the PARTS partial results
-    constexpr int PARTS = NW / 2, PER = NW * 4 / PARTS;              // 8 states per thread
+    // ---- merge.  The wave's 16 lane groups: everything scaled to the wave's maximum, then summed -- the outputs by
+    // exchanging halves between lanes 32 and 16 apart (a lane of row r of 16 keeps outputs 8 (r & 1) + 16 (r >> 1) .. + 7 of
+    // its quarter) and adding up the row's four groups by two rotations.
     {
-        const int dim = threadIdx.x & 127, prt = threadIdx.x >> 7, qd = dim >> 5, r = dim & 31;
-        float sm_[PER], sd_[PER], so_[PER], M = -5e4f;
+        float M = __builtin_fmaxf(m, row_rotate<0x124>(m));
+        M = __builtin_fmaxf(M, row_rotate<0x128>(M));
+        const float r0 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, M), 0));
+        const float r1 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, M), 16));
+        const float r2 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, M), 32));
+        const float r3 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, M), 48));
+        M = __builtin_fmaxf(__builtin_fmaxf(r0, r1), __builtin_fmaxf(r2, r3));
+        const float w = __builtin_amdgcn_exp2f(m - M);
+        d = wave_total(d * w);
+        pz = wave_total(pz * w);
+        psum = wave_total(psum * w);
+        float v16[16], v8[8];
 #pragma unroll
-        for (int k = 0; k < PER; ++k) {
-            const float* src = st + ((prt + k * PARTS) * 4 + qd) * 36;
-            sm_[k] = src[0];
-            sd_[k] = src[1];
-            so_[k] = src[4 + r];
-            M = __builtin_fmaxf(M, sm_[k]);
-        }
-        float D = 0.f, O = 0.f;
+        for (int i = 0; i < 16; ++i) v16[i] = fold_pair<32>(acc[i] * w, acc[i + 16] * w);
 #pragma unroll
-        for (int k = 0; k < PER; ++k) {
-            const float w = __builtin_amdgcn_exp2f(sm_[k] - M);
-            D = __builtin_fmaf(sd_[k], w, D);
-            O = __builtin_fmaf(so_[k], w, O);
+        for (int i = 0; i < 8; ++i) v8[i] = fold_pair<16>(v16[i], v16[i + 8]);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            v8[i] += row_rotate<0x124>(v8[i]);
+            v8[i] += row_rotate<0x128>(v8[i]);
+            v8[i] -= __builtin_fmaf(psum, (i & 1) ? kBiasOdd : kBiasEven, pz);      // sum p (code scale - zero)
         }
-        float* dst = st2 + (prt * 128 + dim) * 3;
-        dst[0] = M;
-        dst[1] = D;
-        dst[2] = O;
+        f32x4* const mine = st4 + wave * 33;
+        if ((lane & 12) == 0) {
+            const int base = 1 + c4 * 8 + ((lane >> 5) & 1) * 4 + ((lane >> 4) & 1) * 2;
+            mine[base] = f32x4{v8[0], v8[1], v8[2], v8[3]};
+            mine[base + 1] = f32x4{v8[4], v8[5], v8[6], v8[7]};
+        }
+        if (lane == 0) mine[0] = f32x4{M, d, 0.f, 0.f};
     }
     __syncthreads();
+    // the workgroup's NW states (and the new position's), one thread per dimension
     if (threadIdx.x < 128) {
         const int dim = threadIdx.x;
-        float M = -5e4f;
+        float sm_[NW], M = -5e4f;
 #pragma unroll
-        for (int k = 0; k < PARTS; ++k) M = __builtin_fmaxf(M, st2[(k * 128 + dim) * 3]);
+        for (int k = 0; k < NW; ++k) {
+            sm_[k] = st[k * 132];
+            M = __builtin_fmaxf(M, sm_[k]);
+        }
+        float nm = -__builtin_inff();
+        if (APPEND && sp == 0) {
+            nm = newv[128];
+            M = __builtin_fmaxf(M, nm);
+        }
         float D = 0.f, O = 0.f;
 #pragma unroll
-        for (int k = 0; k < PARTS; ++k) {
-            const float* src = st2 + (k * 128 + dim) * 3;
-            const float w = __builtin_amdgcn_exp2f(src[0] - M);
-            D = __builtin_fmaf(src[1], w, D);
-            O = __builtin_fmaf(src[2], w, O);
+        for (int k = 0; k < NW; ++k) {
+            const float w = __builtin_amdgcn_exp2f(sm_[k] - M);
+            D = __builtin_fmaf(st[k * 132 + 1], w, D);
+            O = __builtin_fmaf(st[k * 132 + 4 + dim], w, O);
+        }
+        if (APPEND && sp == 0) {
+            const float w = __builtin_amdgcn_exp2f(nm - M) * newv[129];
+            D += w;
+            O = __builtin_fmaf(newv[dim], w, O);
         }
         if (splits == 1) {
             o[(int64_t)bh * 128 + dim] = (f16)(O / D);     // an empty sequence gives 0 / 0, as the reference's kernel does
-        } else {
-            float* dst = part + (int64_t)blockIdx.x * 132;
-            if (dim == 0) {
-                dst[0] = M;
-                dst[1] = D;
-            }
-            dst[4 + dim] = O;
+            return;
         }
+        // (device scope: past the L2 of this XCD, where the workgroup that merges may not run)
+        float* dst = part + (int64_t)blockIdx.x * 132;
+        if (dim == 0) {
+            __hip_atomic_store(dst, M, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(dst + 1, D, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        __hip_atomic_store(dst + 4 + dim, O, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
+    if (splits == 1 || !arrived) return;                    // (not merged here: paged_decode_merge_kernel follows)
+    // The last of the pair's workgroups to arrive merges their states and leaves the counter at zero for the next launch.
+    // Each wave waits until its stores are acknowledged before the barrier, and the count comes behind it.
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    __shared__ u32 before;
+    if (threadIdx.x == 0) before = __hip_atomic_fetch_add(arrived + bh, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    if (before != (u32)splits - 1u) return;
+    if (threadIdx.x == 0) __hip_atomic_store(arrived + bh, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (threadIdx.x < 128) merge_states(part + (int64_t)bh * splits * 132, splits, threadIdx.x, o + (int64_t)bh * 128);
 }
 
 // combines the `splits` partial states of every (sequence, head)
 __global__ __launch_bounds__(128) void paged_decode_merge_kernel(const float* __restrict__ part, int splits,
                                                                  f16* __restrict__ o) {
-    const int64_t bh = blockIdx.x;
-    const int dim = threadIdx.x;
-    const float* src = part + bh * splits * 132;
-    float M = -5e4f;
-    for (int s = 0; s < splits; ++s) M = __builtin_fmaxf(M, src[s * 132]);
-    float D = 0.f, O = 0.f;
-    for (int s = 0; s < splits; ++s) {
-        const float w = __builtin_amdgcn_exp2f(src[s * 132] - M);
-        D = __builtin_fmaf(src[s * 132 + 1], w, D);
-        O = __builtin_fmaf(src[s * 132 + 4 + dim], w, O);
-    }
-    o[bh * 128 + dim] = (f16)(O / D);
+    merge_states(part + (int64_t)blockIdx.x * splits * 132, splits, threadIdx.x, o + (int64_t)blockIdx.x * 128);
 }
 
 int check_cache(const void* kv_data, const void* kv_param, const void* kv_indptr, const void* kv_indices,
@@ -559,9 +617,15 @@ extern "C" int qr_kv_append_i4(void* kv_data, void* kv_param, const void* kv_ind
 }
 
 namespace {
-// Waves per (sequence, head): enough to fill the GPU's wave slots (16 per CU), each with at least four steps of 16
-// positions when the caller says how long the sequences can be.  Up to 16 of them form one workgroup;
-// beyond that the sequence is split over several workgroups, which needs room for their partial states.
+// Waves of a workgroup and workgroups of a (sequence, head), by an estimate in microseconds fitted to a sweep of 1 .. 40
+// sequences x 89 .. 16000 positions x 8 .. 64 heads with every plan forced (within 20 % of them, the chosen plan within
+// 5 % of the best one measured):
+//   3.3 for the launch and its first loads, 2.7 / 3.4 / 5.0 per workgroup of 4 / 8 / 16 waves on the busiest CU (query,
+//   merge), 1.8 when the states of several workgroups are merged (+ 0.3 for every eight of them), and the walk: 0.37 per
+//   chunk of 16 positions for one wave, but no faster than 0.069 per chunk for a CU (its vector units dequantise; 0.093
+//   with a single wave per SIMD).
+// One sequence of 2048 x 32 heads: 32 workgroups of 8 waves leave 224 CUs idle and are bound by the vector units of the
+// others (14.7 us); 256 workgroups of 4 waves, 8 per head: 9.1 us.
 struct DecodePlan {
     int nw, splits;
 };
@@ -569,19 +633,33 @@ DecodePlan decode_plan(int64_t batch_size, int num_heads, int64_t max_seq_len) {
     const int64_t bh = batch_size * num_heads, cus = qr_device().cus;
     if (max_seq_len <= 0) return DecodePlan{bh >= 4 * cus ? 4 : bh >= cus ? 8 : 16, 1};
     const int64_t chunks = (max_seq_len + 15) / 16;
-    int64_t wp = (16 * cus + bh - 1) / bh, cap = chunks / 4;
-    wp = wp > cap ? cap : wp;
-    if (wp <= 4) return DecodePlan{4, 1};
-    if (wp <= 16) return DecodePlan{8, 1};                  // (measured a few percent ahead of 16 waves at 256 (sequence, head) pairs)
-    int64_t s = (wp + 15) / 16;
-    return DecodePlan{16, (int)(s > 16 ? 16 : s)};
+    DecodePlan best{4, 1};
+    double t_best = 1e30;
+    for (int nw = 4; nw <= 16; nw *= 2)
+        for (int s = 1; s <= 32; s *= 2) {
+            if (s > 1 && nw * s > chunks) break;            // (a wave without a chunk of its own)
+            const double load = (double)(bh * s) / (double)cus;
+            const double busiest = load < 4.0 ? (double)((bh * s + cus - 1) / cus) : load;     // (many small workgroups even out)
+            const double wave_chunks = (double)((chunks + nw * s - 1) / (nw * s));
+            const double cu_chunks = busiest * (double)chunks / s;
+            const double walk_wave = 0.37 * wave_chunks, walk_cu = (busiest * nw <= 4.0 ? 0.093 : 0.069) * cu_chunks;
+            const double t = 3.3 + busiest * (nw == 4 ? 2.7 : nw == 8 ? 3.4 : 5.0) + (s > 1 ? 1.8 + 0.3 * (s / 8) : 0.0) +
+                             (walk_wave > walk_cu ? walk_wave : walk_cu);
+            if (t < t_best) {
+                t_best = t;
+                best = DecodePlan{nw, s};
+            }
+        }
+    return best;
 }
+// the workspace: one arrival counter per (sequence, head), then the partial states
+size_t decode_counter_bytes(int64_t bh) { return ((size_t)bh * 4 + 255) & ~(size_t)255; }
 }  // namespace
 
 extern "C" size_t qr_batch_decode_workspace_bytes(int64_t batch_size, int num_heads, int64_t max_seq_len) {
     if (batch_size <= 0 || num_heads <= 0) return 0;
     const int s = decode_plan(batch_size, num_heads, max_seq_len).splits;
-    return s > 1 ? (size_t)batch_size * num_heads * s * 132 * sizeof(float) : 0;
+    return s > 1 ? decode_counter_bytes(batch_size * num_heads) + (size_t)batch_size * num_heads * s * 132 * sizeof(float) : 0;
 }
 
 namespace {
@@ -589,7 +667,7 @@ int batch_decode(void* o, const void* q, const void* kv_data, const void* kv_par
                  const void* kv_indices, const void* last_page_offset, int64_t num_pages, int num_layers, int layer_idx,
                  int num_heads, int page_size, int head_dim, int64_t batch_size, int64_t max_seq_len, void* workspace,
                  size_t workspace_bytes, void* stream, int q_had, const void* knew = nullptr, const void* vnew = nullptr,
-                 int k_had = 0) {
+                 int k_had = 0, bool counters_zero = false) {
     const int rc = check_cache(kv_data, kv_param, kv_indptr, kv_indices, last_page_offset, num_pages, num_layers, layer_idx,
                                num_heads, page_size, head_dim, batch_size);
     if (rc != QR_OK) return rc;
@@ -601,9 +679,12 @@ int batch_decode(void* o, const void* q, const void* kv_data, const void* kv_par
                                            num_layers, layer_idx, num_heads, page_size, batch_size);
     DecodePlan plan = decode_plan(batch_size, num_heads, max_seq_len);
     int splits = plan.splits;
+    const size_t counters = decode_counter_bytes(batch_size * num_heads);
     if (splits > 1 && (!workspace || ((uintptr_t)workspace & 15) ||
-                       workspace_bytes < (size_t)batch_size * num_heads * splits * 132 * sizeof(float)))
+                       workspace_bytes < counters + (size_t)batch_size * num_heads * splits * 132 * sizeof(float)))
         splits = 1;                                        // no room for partial states: one workgroup per (sequence, head)
+    float* const part = splits > 1 ? (float*)((char*)workspace + counters) : nullptr;
+    u32* const arrived = splits > 1 && counters_zero ? (u32*)workspace : nullptr;
     const float sm = (float)(1.4426950408889634 / __builtin_sqrt((double)head_dim));
     const unsigned grid = (unsigned)(batch_size * num_heads * splits);
     hipStream_t st = (hipStream_t)stream;
@@ -611,10 +692,10 @@ int batch_decode(void* o, const void* q, const void* kv_data, const void* kv_par
     do {                                                                                                                \
         if (knew)                                                                                                       \
             paged_decode_i4_kernel<AL, NWV, true><<<dim3(grid), dim3(64 * NWV), 0, st>>>(                               \
-                (const f16*)q, c, (f16*)o, sm, splits, (float*)workspace, q_had, (const u32x4*)knew, (const u32x4*)vnew, k_had); \
+                (const f16*)q, c, (f16*)o, sm, splits, part, q_had, arrived, (const u32x4*)knew, (const u32x4*)vnew, k_had); \
         else                                                                                                            \
             paged_decode_i4_kernel<AL, NWV><<<dim3(grid), dim3(64 * NWV), 0, st>>>((const f16*)q, c, (f16*)o, sm, splits, \
-                                                                                  (float*)workspace, q_had);           \
+                                                                                  part, q_had, arrived);               \
     } while (0)
     if (page_size % 16 == 0) {
         if (plan.nw == 16) QR_DECODE(true, 16);
@@ -627,9 +708,8 @@ int batch_decode(void* o, const void* q, const void* kv_data, const void* kv_par
     }
 #undef QR_DECODE
     int lrc = qr_launch_status();
-    if (lrc != QR_OK || splits == 1) return lrc;
-    paged_decode_merge_kernel<<<dim3((unsigned)(batch_size * num_heads)), dim3(128), 0, st>>>((const float*)workspace, splits,
-                                                                                             (f16*)o);
+    if (lrc != QR_OK || splits == 1 || arrived) return lrc;
+    paged_decode_merge_kernel<<<dim3((unsigned)(batch_size * num_heads)), dim3(128), 0, st>>>(part, splits, (f16*)o);
     return qr_launch_status();
 }
 }  // namespace
@@ -661,10 +741,12 @@ extern "C" int qr_kv_quant_append_batch_decode_f16_i4(void* o, const void* q, in
                                                       int num_layers, int layer_idx, int num_heads, int page_size, int head_dim,
                                                       int64_t batch_size, int64_t max_seq_len, void* workspace,
                                                       size_t workspace_bytes, void* stream) {
+    const bool counters_zero = (q_had_mode & QR_DECODE_COUNTERS_ZERO) != 0;
+    q_had_mode &= ~QR_DECODE_COUNTERS_ZERO;
     if ((q_had_mode != 0 && q_had_mode != 1) || (k_had_mode != 0 && k_had_mode != 1)) return QR_E_DTYPE;
     if (batch_size > 0 && (!k || !v)) return QR_E_NULL;
     if (((uintptr_t)k & 15) || ((uintptr_t)v & 15)) return QR_E_ALIGN;
     return batch_decode(o, q, kv_data, kv_param, kv_indptr, kv_indices, last_page_offset, num_pages, num_layers, layer_idx,
                         num_heads, page_size, head_dim, batch_size, max_seq_len, workspace, workspace_bytes, stream, q_had_mode,
-                        k, v, k_had_mode);
+                        k, v, k_had_mode, counters_zero);
 }

@@ -247,7 +247,7 @@ def _decode_workspace_bytes(batch, heads, max_seq_len, device_index=None):
 
 
 def batch_decode_i4(o, q, kv_data, kv_param, kv_indptr, kv_indices, last_page_offset, layer_idx, max_seq_len=0,
-                    q_hadamard=False, workspace=None, append=None):
+                    q_hadamard=False, workspace=None, append=None, counters_zero=False):
     """o[b, h] = softmax(q[b, h] . K^T / sqrt(128)) . V over the int4 cache of sequence b, dequantised in
     registers as float(code) * scale - zero (kv_cache.py:60-67 -> bindings.cpp:118-153).  Writes into `o`
     and returns None, like the reference's binding.  max_seq_len (optional, an upper bound of the
@@ -257,7 +257,9 @@ def batch_decode_i4(o, q, kv_data, kv_param, kv_indptr, kv_indices, last_page_of
     the sequence; one is allocated per call when it is missing or too small.  append = (k, v, hadamard): the fp16
     key and value [batch_size, heads, 128] of the step's new token, which the page tables already count as every
     sequence's last position: the kernel quantises them as quantize_append_kv_i4 would (same codes, scales and zeros,
-    written to the same page slots) and attends to them along with the cache -- append and attention in one launch."""
+    written to the same page slots) and attends to them along with the cache -- append and attention in one launch.
+    counters_zero (with append): the first 4 * batch_size * heads bytes of `workspace` are zero and nobody else uses
+    them meanwhile; a split along the sequence is then merged in the same launch, which leaves them zero."""
     fn = "batch_decode_i4"
     pages, layers, heads, page_size, head_dim = _cache_args(fn, kv_data, kv_param, kv_indptr, kv_indices, last_page_offset, layer_idx)
     for name, t in (("o", o), ("q", q)):
@@ -288,9 +290,11 @@ def batch_decode_i4(o, q, kv_data, kv_param, kv_indptr, kv_indices, last_page_of
             fits = (workspace is not None and workspace.device == dev and workspace.dtype == torch.uint8
                     and workspace.is_contiguous() and workspace.numel() >= ws_bytes)
             ws = workspace if fits else torch.empty((ws_bytes,), dtype=torch.uint8, device=dev)
+            counters_zero = counters_zero and fits
         if append is not None:
             _lib.check(_lib.lib().qr_kv_quant_append_batch_decode_f16_i4(
-                o.data_ptr(), q.data_ptr(), 1 if q_hadamard else 0, append[0].data_ptr(), append[1].data_ptr(),
+                o.data_ptr(), q.data_ptr(), (1 if q_hadamard else 0) | (_lib.QR_DECODE_COUNTERS_ZERO if counters_zero else 0),
+                append[0].data_ptr(), append[1].data_ptr(),
                 1 if append[2] else 0, kv_data.data_ptr(), kv_param.data_ptr(), kv_indptr.data_ptr(), kv_indices.data_ptr(),
                 last_page_offset.data_ptr(), pages, layers, int(layer_idx), heads, page_size, head_dim, batch, int(max_seq_len),
                 None if ws is None else ws.data_ptr(), ws_bytes, _lib.stream_ptr(dev)))
@@ -329,7 +333,7 @@ class _AttentionStub(object):
         # the step's new token, if the cache still holds it back for this call (see MultiLayerPagedKVCache4Bit.update)
         append = take_pending() if take_pending is not None else None
         batch_decode_i4(attn_output, q, **attention_kwargs, layer_idx=layer_idx, max_seq_len=max_seq_len, q_hadamard=fused,
-                        workspace=workspace, append=append)
+                        workspace=workspace, append=append, counters_zero=workspace is not None)
         return attn_output.unsqueeze(1)
 
 
@@ -397,7 +401,8 @@ class MultiLayerPagedKVCache4Bit:
 
     def _decode_workspace(self, num_heads):
         """Scratch for decode attention split along the sequence, kept with the cache (every layer of every decode
-        step would otherwise allocate its own): sized for the longer of the current and the maximum length."""
+        step would otherwise allocate its own): sized for the longer of the current and the maximum length.  Zeroed when
+        it is made: every launch leaves its arrival counters at zero."""
         key = (self.length, num_heads)
         if getattr(self, "_decode_ws_key", None) == key:
             return self._decode_ws
@@ -407,7 +412,7 @@ class MultiLayerPagedKVCache4Bit:
                         for n in (self.length, self.max_seq_len) if n), default=0)
         ws = getattr(self, "_decode_ws", None)
         if need and (ws is None or ws.numel() < need):
-            ws = torch.empty((need,), dtype=torch.uint8, device=dev)
+            ws = torch.zeros((need,), dtype=torch.uint8, device=dev)
         self._decode_ws, self._decode_ws_key = ws, key
         return ws
 

@@ -179,3 +179,43 @@ def test_one_launch_decode_step_replays_from_a_hip_graph_and_rejects_wrong_shape
             kv.batch_decode_i4(out, q, gd1, gp1, *tabs, 0, q_hadamard=True, append=(bad, good, True))
         with pytest.raises(RuntimeError):
             kv.batch_decode_i4(out, q, gd1, gp1, *tabs, 0, q_hadamard=True, append=(good, bad, True))
+
+
+@pytest.mark.parametrize("page_size,lens,heads", [(16, [2048], 32), (16, [5000, 16], 8), (24, [700, 1], 4), (128, [16000], 2)])
+def test_split_sequences_merged_by_the_last_workgroup_of_the_same_launch(page_size, lens, heads):
+    """A step whose sequences are split over several workgroups, with a zeroed workspace: outputs as the unsplit launch and
+    the one with a separate merge give, on every call (the counters are back at zero after each), also after a shorter
+    bound has used the same workspace with another split, and when the launch is replayed from a graph."""
+    rng = np.random.default_rng(page_size + heads)
+    data, param, indptr, indices, last = paged_case(rng, heads, page_size, lens, layers=1)
+    B, L = len(lens), _lib.lib()
+    tabs = (gpu(indptr), gpu(indices), gpu(last))
+    gd, gp = gpu(data), gpu(param)
+    bound = max(lens)
+    need = max(L.qr_batch_decode_workspace_bytes(B, heads, n) for n in (bound, bound // 3 + 1))
+    assert L.qr_batch_decode_workspace_bytes(B, heads, bound) > 0
+    ws = torch.zeros(need, dtype=torch.uint8, device="cuda:0")
+    k, v = gpu(synth_kv(rng, B, heads)), gpu(synth_kv(rng, B, heads))
+    sq = torch.empty((B, heads, 128), dtype=torch.float16, device="cuda:0")
+    out, ref, two = torch.empty_like(sq), torch.empty_like(sq), torch.empty_like(sq)
+    step = lambda y, hint, **kw: kv.batch_decode_i4(y, sq, gd, gp, *tabs, 0, max_seq_len=hint, q_hadamard=True, append=(k, v, True), **kw)
+    graph = None
+    for i in range(5):
+        sq.copy_(gpu((rng.standard_normal((B, heads, 128)) * 2).astype(F16)))
+        step(ref, 0)
+        step(two, bound)
+        if i == 2:
+            step(out, bound // 3 + 1, workspace=ws, counters_zero=True)       # (a bound only chooses the split)
+            assert close(out.cpu().numpy(), ref.cpu().numpy())
+        out.fill_(float("nan"))
+        if i < 3:
+            step(out, bound, workspace=ws, counters_zero=True)
+        else:
+            if graph is None:
+                graph = torch.cuda.CUDAGraph()
+                with torch.cuda.graph(graph):
+                    step(out, bound, workspace=ws, counters_zero=True)
+            graph.replay()
+        torch.cuda.synchronize()
+        assert close(out.cpu().numpy(), ref.cpu().numpy()) and close(two.cpu().numpy(), ref.cpu().numpy())
+        assert int(ws[:4 * B * heads].sum()) == 0
