@@ -332,6 +332,15 @@ int qr_kv_quant_append_f16_i4(const void* k, const void* v, int64_t tokens, cons
                               int64_t batch_size, void* stream);
 
 /*
+ * The page tables of batch_size sequences of `length` (> 0) tokens each, page i of sequence b being page number
+ * i * batch_size + b (get_cache_specs_for_flash_infer without a mask, quarot/transformers/kv_cache.py:253-275):
+ *   kv_indptr int32 [batch_size + 1], kv_indices int32 [batch_size * ceil(length / page_size)],
+ *   last_page_offset int32 [batch_size].
+ */
+int qr_page_tables(int64_t batch_size, int64_t length, int page_size, void* kv_indptr, void* kv_indices,
+                   void* last_page_offset, void* stream);
+
+/*
  * Single-query attention over the paged int4 cache:
  *   o[b, h, :] = sum_j softmax_j( q[b, h, :] . k_j / sqrt(head_dim) ) v_j,   j over the tokens of sequence b,
  *   k_j[i] = float(code) * scale_j - zero_j in fp32 (quarot/kernels/include/flashinfer/quantization.cuh:59-84).

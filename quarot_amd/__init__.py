@@ -14,6 +14,7 @@ import weakref
 import torch
 
 from . import _lib
+from ._lib import host as _host
 from . import functional
 from . import nn
 
@@ -133,6 +134,9 @@ class PackedQuantizedTensor:
 def quantize_rows(x, clip_ratio=1.0):
     """Quantizer.forward in one kernel (quarot/nn/quantization.py:9-13): returns
     (packed uint8 [..., C/2], scales fp16 with the reference's [R, 1]-after-unsqueeze(1) shape)."""
+    fast = _host.quantize_rows(x, clip_ratio)
+    if fast is not None:
+        return fast
     assert x.dtype == torch.float16
     x2, lead = _flat2d(x)
     dev = _require_gpu_contiguous("quantize_rows", x=x2)
@@ -178,9 +182,24 @@ def _hadamard_sign_words(hadK, n, K):
     return words
 
 
+def _hadamard_operand(hadK, n, K, force_fp32):
+    """(hadK as the native route passes it -- its sign words where the library takes them --, the mode)."""
+    mode = _lib.QR_DTYPE_F32 if force_fp32 else _lib.QR_DTYPE_F16
+    if K > 96:
+        signs = _hadamard_sign_words(hadK, n, K)
+        if signs is not None:
+            return signs, mode | _lib.QR_HADK_SIGNS
+    return hadK, mode
+
+
 def hadamard_quantize(x, hadK, K, clip_ratio=1.0, force_fp32=False, return_transformed=False):
     """OnlineHadamard.forward followed by Quantizer.forward in one kernel
     (quarot/nn/hadamard.py:17-23 + quarot/nn/quantization.py:9-13)."""
+    if not return_transformed:
+        operand, mode = _hadamard_operand(hadK, x.shape[-1], K, force_fp32)
+        fast = _host.hadamard_quantize(x, operand, K, mode, functional.hadamard.had_scale(x.shape[-1]), clip_ratio)
+        if fast is not None:
+            return PackedQuantizedTensor(*fast)
     assert x.dtype == torch.float16
     x2, lead = _flat2d(x)
     dev = _require_gpu_contiguous("hadamard_quantize", x=x2, hadK=hadK)
@@ -219,6 +238,9 @@ def hadamard_quantize(x, hadK, K, clip_ratio=1.0, force_fp32=False, return_trans
 
 def rmsnorm(x, mean_dim, eps=1e-5):
     """RMSNorm.forward of fp16 rows in one kernel (quarot/nn/normalization.py:15-21)."""
+    y = _host.rmsnorm(x, mean_dim, eps)
+    if y is not None:
+        return y
     assert x.dtype == torch.float16
     x2, _ = _flat2d(x)
     dev = _require_gpu_contiguous("rmsnorm", x=x2)
@@ -232,6 +254,10 @@ def rmsnorm(x, mean_dim, eps=1e-5):
 def rmsnorm_quantize(x, mean_dim, eps=1e-5, clip_ratio=1.0, return_normalized=False):
     """RMSNorm.forward followed by Quantizer.forward in one kernel
     (quarot/nn/normalization.py:15-21 + quarot/nn/quantization.py:9-13)."""
+    if not return_normalized:
+        fast = _host.rmsnorm_quantize(x, mean_dim, eps, clip_ratio)
+        if fast is not None:
+            return PackedQuantizedTensor(*fast)
     assert x.dtype == torch.float16
     x2, lead = _flat2d(x)
     dev = _require_gpu_contiguous("rmsnorm_quantize", x=x2)
@@ -255,6 +281,10 @@ def heads_hadamard_quantize(x, num_heads, clip_ratio=1.0, return_transformed=Fal
     it; no transposed copies are made.  head_dim 128 and 16, 32 or 64 heads; or a head count that is
     the order of one of the reference's tables (40 for Llama-2-13B, 52 for Llama-30B, ...) with hadK =
     that table (OnlineHadamard's had_rem_dim buffer)."""
+    if not return_transformed and x.dim() >= 2 and x.shape[-2] == num_heads:
+        fast = _host.heads_hadamard_quantize(x, clip_ratio, hadK)
+        if fast is not None:
+            return PackedQuantizedTensor(*fast)
     assert x.dtype == torch.float16
     if x.dim() < 2 or x.shape[-2] != num_heads:
         raise RuntimeError("heads_hadamard_quantize: x must be [..., num_heads, head_dim]")
@@ -287,6 +317,9 @@ def _workspace_bytes(M, N, K, device_index=None):
 
 def linear_i4(x_q, scales_x, weight, weight_scales, bias=None):
     """Linear4bit.forward in one kernel (quarot/nn/linear.py:42-56): matmul + sym_dequant (+ bias)."""
+    y = _host.linear(x_q, scales_x, weight, weight_scales, bias)
+    if y is not None:
+        return y
     assert x_q.shape[-1] % 32 == 0, "A.shape[-1]: {} must be multiplication of 32".format(x_q.shape[-1])
     assert scales_x.dtype == weight_scales.dtype == torch.float16
     a2, lead = _flat2d(x_q)
@@ -359,6 +392,10 @@ def quantized_linear(x, weight, weight_scales, bias=None, hadK=None, K=0, clip_r
     the same two launches as hadamard_quantize / quantize_rows followed by linear_i4 (one or two tokens, plain or behind a
     1024-point Hadamard factor: one kernel that does both), same results bit for bit, half the host-side
     cost.  x fp16 [..., in_features] -> fp16 [..., out_features]."""
+    operand, mode = _hadamard_operand(hadK, x.shape[-1], K, force_fp32) if K else (None, _lib.QR_DTYPE_F16)
+    y = _host.quantized_linear(x, operand, K, mode, functional.hadamard.had_scale(x.shape[-1]), clip_ratio, weight, weight_scales, bias)
+    if y is not None:
+        return y
     assert x.dtype == torch.float16
     assert x.shape[-1] % 64 == 0, "in_features: {} must be a multiple of 64".format(x.shape[-1])
     x2, lead = _flat2d(x)

@@ -1,9 +1,12 @@
-"""ctypes binding of libquarot_hip.so (the C ABI declared in include/quarot_hip.h).
+"""ctypes binding of libquarot_hip.so (the C ABI declared in include/quarot_hip.h), and `host`: the native host side of the
+hot entry points (csrc/host.cpp), whose functions return None where the general route of the wrappers has to decide.
 
 There is no fallback: if the library is missing or a call fails, an exception is raised.
 """
 import ctypes
 import pathlib
+
+import torch            # (before _host.so, which is linked against its libraries)
 
 _PKG = pathlib.Path(__file__).resolve().parent
 LIB_PATH = _PKG / "libquarot_hip.so"
@@ -40,6 +43,7 @@ SIGNATURES = {
                                _i64, _ptr)),
     "qr_kv_quant_append_f16_i4": (_int, (_ptr, _ptr, _i64, _ptr, _int, _ptr, _ptr, _ptr, _ptr, _ptr, _i64, _int, _int, _int, _int,
                                          _int, _i64, _ptr)),
+    "qr_page_tables": (_int, (_i64, _i64, _int, _ptr, _ptr, _ptr, _ptr)),
     "qr_batch_decode_workspace_bytes": (_c.c_size_t, (_i64, _int, _i64)),
     "qr_batch_decode_i4": (_int, (_ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _i64, _int, _int, _int, _int, _int, _i64, _i64, _ptr,
                                   _c.c_size_t, _ptr)),
@@ -59,6 +63,25 @@ QR_HADK_SIGNS = 0x100          # or-ed into a `mode`: hadK is passed as sign wor
 QR_HAD_FP32 = 0x200            # or-ed into qr_hadamard's dtype: fp16 rows, fp32-precision arithmetic
 QR_DECODE_COUNTERS_ZERO = 0x100    # or-ed into q_had_mode of the one-launch decode step: the workspace's counters are zero
 QR_E_NULL, QR_E_SHAPE, QR_E_UNSUPPORTED = -1, -2, -3
+
+class _HostOnUse:
+    """Stands in for _host.so when the package is imported before it is built: tries again when it is used."""
+
+    def __getattr__(self, name):
+        import importlib
+        try:
+            fn = getattr(importlib.import_module("._host", __package__), name)
+        except ImportError as e:
+            raise RuntimeError(f"{_PKG / '_host.so'} cannot be loaded ({e}): build it with `python -m quarot_amd.build` "
+                               "(this package has no CPU or PyTorch fallback)") from e
+        setattr(self, name, fn)
+        return fn
+
+
+try:
+    from . import _host as host
+except ImportError:
+    host = _HostOnUse()
 
 _lib = None
 
@@ -87,7 +110,6 @@ def check(code):
 
 def stream_ptr(device):
     """Raw handle of torch's current stream on `device` (the library launches there)."""
-    import torch
     raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
     if raw is not None and device.index is not None:
         return raw(device.index)                 # same value, without building a Stream object
@@ -108,7 +130,6 @@ _NO_GUARD = _NoGuard()
 def on_device(device):
     """Context that makes `device` current for the launch; nothing to do (and nothing to pay) when
     it already is."""
-    import torch
     if device.index is None or device.index == torch.cuda.current_device():
         return _NO_GUARD
     return torch.cuda.device(device)

@@ -1,4 +1,5 @@
-"""Build recipe for libquarot_hip.so: plain hipcc, gfx950 only, no torch headers.
+"""Build recipe: libquarot_hip.so by plain hipcc, gfx950 only, no torch headers; and _host.so, the CPython module of the
+hot entry points' host side (csrc/host.cpp), by g++ against torch's headers.
 
     python -m quarot_amd.build                # compile every source, link in-tree (quarot_amd/libquarot_hip.so)
     python -m quarot_amd.build --incremental  # recompile only sources newer than their objects
@@ -12,6 +13,7 @@ import sys
 PKG = pathlib.Path(__file__).resolve().parent
 CSRC = PKG / "csrc"
 LIB = PKG / "libquarot_hip.so"
+HOST = PKG / "_host.so"
 OBJ = PKG.parent / "build" / "obj"
 SOURCES = ("api.hip", "quant.hip", "gemm.hip", "gemm_mid.hip", "gemm_f6.hip", "hadamard.hip", "kv.hip", "attn.hip", "calib.hip", "decode_fused.hip",
            "paged_f16.hip")
@@ -24,6 +26,21 @@ FLAGS = ("--offload-arch=gfx950", "-O3", "-fPIC", "-std=c++17", "-fno-gpu-rdc",
          "-Wno-unused-command-line-argument")
 
 
+def _host_commands():
+    """(compile, link) of _host.so: one object, then the link against libquarot_hip.so beside it."""
+    import sysconfig
+    import torch
+    from torch.utils import cpp_extension
+    src, obj = CSRC / "host.cpp", OBJ / "host.o"
+    include = [f"-I{d}" for d in (*cpp_extension.include_paths(), "/opt/rocm/include", sysconfig.get_paths()["include"])]
+    compile_ = ["g++", "-O2", "-fPIC", "-std=c++17", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+                f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *include, "-c", str(src), "-o", str(obj)]
+    torch_lib = pathlib.Path(torch.__file__).resolve().parent / "lib"
+    link = ["g++", "-shared", str(obj), "-o", str(HOST), f"-L{torch_lib}", "-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip",
+            f"-L{PKG}", f"-l:{LIB.name}", "-Wl,-rpath,$ORIGIN"]
+    return src, obj, compile_, link
+
+
 def _run(cmd, verbose):
     if verbose:
         print(" ".join(cmd), flush=True)
@@ -31,7 +48,7 @@ def _run(cmd, verbose):
     # hipcc's host pass warns that it does not know the packed-fp32 feature: harmless, filtered.
     err = "\n".join(l for l in res.stderr.splitlines() if "packed-fp32-ops" not in l)
     if res.returncode != 0:
-        raise RuntimeError(f"hipcc failed ({res.returncode}):\n{err}")
+        raise RuntimeError(f"{cmd[0]} failed ({res.returncode}):\n{err}")
     if verbose and err.strip():
         print(err, file=sys.stderr)
 
@@ -48,10 +65,15 @@ def build(verbose=True, incremental=False):
         fresh = incremental and obj.exists() and obj.stat().st_mtime > max(src.stat().st_mtime, headers_mtime)
         if not fresh:
             jobs.append(["hipcc", *FLAGS, "-c", str(src), "-o", str(obj)])
+    host_src, host_obj, host_compile, host_link = _host_commands()
+    header = PKG.parent / "include" / "quarot_hip.h"
+    if not (incremental and host_obj.exists() and host_obj.stat().st_mtime > max(host_src.stat().st_mtime, header.stat().st_mtime)):
+        jobs.append(host_compile)
     workers = max(1, min(len(jobs), (os.cpu_count() or 2)))
     with concurrent.futures.ThreadPoolExecutor(max_workers=workers) as pool:
         list(pool.map(lambda c: _run(c, verbose), jobs))
     _run(["hipcc", "--offload-arch=gfx950", "-shared", "-fPIC", "-fno-gpu-rdc", *objs, "-o", str(LIB)], verbose)
+    _run(host_link, verbose)
     return LIB
 
 

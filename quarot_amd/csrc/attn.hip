@@ -547,6 +547,21 @@ __global__ __launch_bounds__(128) void paged_decode_merge_kernel(const float* __
     merge_states(part + (int64_t)blockIdx.x * splits * 132, splits, threadIdx.x, o + (int64_t)blockIdx.x * 128);
 }
 
+// page tables of `batch` sequences of `length` tokens each: page i of sequence b is page number i * batch + b
+// (quarot/transformers/kv_cache.py:253-275 builds them with nine torch kernels per decode step)
+__global__ __launch_bounds__(256) void page_tables_kernel(int batch, int pages, int last, int32_t* __restrict__ indptr,
+                                                          int32_t* __restrict__ indices, int32_t* __restrict__ last_page_offset) {
+    const int step = gridDim.x * 256, first = blockIdx.x * 256 + threadIdx.x;
+    for (int i = first; i < batch * pages; i += step) {
+        const int b = i / pages;
+        indices[i] = (i - b * pages) * batch + b;
+    }
+    for (int b = first; b <= batch; b += step) {
+        indptr[b] = b * pages;
+        if (b < batch) last_page_offset[b] = last;
+    }
+}
+
 int check_cache(const void* kv_data, const void* kv_param, const void* kv_indptr, const void* kv_indices,
                 const void* last_page_offset, int64_t num_pages, int num_layers, int layer_idx, int num_heads,
                 int page_size, int head_dim, int64_t batch_size) {
@@ -590,6 +605,20 @@ __attribute__((visibility("hidden"))) PagedKV qr_internal_paged_kv(void* kv_data
     c.page_size = page_size;
     c.batch_size = (int)batch_size;
     return c;
+}
+
+extern "C" int qr_page_tables(int64_t batch_size, int64_t length, int page_size, void* kv_indptr, void* kv_indices,
+                              void* last_page_offset, void* stream) {
+    if (batch_size < 0 || length <= 0 || page_size <= 0) return QR_E_SHAPE;
+    if (batch_size == 0) return QR_OK;
+    const int64_t pages = (length + page_size - 1) / page_size;
+    if (batch_size * pages > 0x3fffffff) return QR_E_SHAPE;
+    if (!kv_indptr || !kv_indices || !last_page_offset) return QR_E_NULL;
+    const int64_t blocks = (batch_size * pages + 255) / 256;
+    page_tables_kernel<<<dim3((unsigned)(blocks > 256 ? 256 : blocks)), dim3(256), 0, (hipStream_t)stream>>>(
+        (int)batch_size, (int)pages, (int)(length - (pages - 1) * page_size), (int32_t*)kv_indptr, (int32_t*)kv_indices,
+        (int32_t*)last_page_offset);
+    return qr_launch_status();
 }
 
 extern "C" int qr_kv_append_i4(void* kv_data, void* kv_param, const void* kv_indptr, const void* kv_indices,

@@ -1,0 +1,423 @@
+// Host side of the package's hot entry points: argument checks, output allocation and the call into libquarot_hip.so as
+// one CPython function each, where the Python wrappers take 10 - 25 us per call -- longer than most decode kernels run.
+//
+// Every function returns None instead of raising when the arguments are not the plain case it serves (a tensor subclass, a
+// tensor that is not contiguous or not on the current device, a wrong dtype or size, an empty input, a refusal by the
+// library): the Python wrapper then takes its general route, which handles the case or raises the documented error.
+// Launches go to torch's current stream, outputs and scratch come from torch's allocator.
+#define PY_SSIZE_T_CLEAN
+#include <Python.h>
+
+#include <ATen/ops/empty.h>
+#include <c10/hip/HIPFunctions.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include "../../include/quarot_hip.h"
+
+namespace {
+
+const at::Tensor* tensor(PyObject* o) { return THPVariable_CheckExact(o) ? &THPVariable_Unpack(o) : nullptr; }
+
+bool plain(const at::Tensor* t, at::ScalarType dtype, int device) {
+    return t && t->is_cuda() && t->scalar_type() == dtype && t->device().index() == device && t->is_contiguous();
+}
+// an optional operand: None is fine and has no address
+bool plain_or_none(PyObject* o, at::ScalarType dtype, int device, const at::Tensor** out) {
+    *out = nullptr;
+    if (o == Py_None) return true;
+    *out = tensor(o);
+    return plain(*out, dtype, device);
+}
+
+constexpr auto kHalf = at::kHalf;
+constexpr auto kByte = at::kByte;
+
+// the tensor's device if it is the current one, else -1 (which no tensor on a GPU has)
+int device_of(const at::Tensor* t) {
+    if (!t || !t->is_cuda()) return -1;
+    const int d = (int)t->device().index();
+    return d == (int)c10::hip::current_device() ? d : -1;
+}
+void* stream(int device) { return (void*)c10::hip::getCurrentHIPStream((c10::DeviceIndex)device).stream(); }
+at::Tensor fresh(at::IntArrayRef sizes, at::ScalarType dtype, int device) {
+    return at::empty(sizes, at::TensorOptions().dtype(dtype).device(at::Device(at::kCUDA, (c10::DeviceIndex)device)));
+}
+void* ptr(const at::Tensor* t) { return t ? t->data_ptr() : nullptr; }
+
+PyObject* none() { Py_RETURN_NONE; }
+PyObject* wrap(at::Tensor&& t) { return THPVariable_Wrap(std::move(t)); }
+PyObject* wrap2(at::Tensor&& a, at::Tensor&& b) {
+    PyObject* pa = wrap(std::move(a));
+    PyObject* pb = pa ? wrap(std::move(b)) : nullptr;
+    if (!pb) {
+        Py_XDECREF(pa);
+        return nullptr;
+    }
+    PyObject* t = PyTuple_New(2);
+    if (!t) {
+        Py_DECREF(pa);
+        Py_DECREF(pb);
+        return nullptr;
+    }
+    PyTuple_SET_ITEM(t, 0, pa);
+    PyTuple_SET_ITEM(t, 1, pb);
+    return t;
+}
+
+// rows of a quantiser's input: fp16 [..., n], contiguous, on the current device
+struct Rows {
+    const at::Tensor* x;
+    int device;
+    int64_t rows, n;
+    bool ok;
+};
+Rows rows_of(PyObject* o) {
+    Rows r{tensor(o), -1, 0, 0, false};
+    r.device = device_of(r.x);
+    if (!plain(r.x, kHalf, r.device) || r.x->dim() < 1) return r;
+    r.n = r.x->size(-1);
+    r.ok = r.n > 0 && r.x->numel() > 0;
+    if (r.ok) r.rows = r.x->numel() / r.n;
+    return r;
+}
+// codes [..., n / 2] and scales with the shape torch.max(dim=-1)[0].unsqueeze(1) has
+struct Packed {
+    at::Tensor codes, scales;
+};
+Packed packed_for(const Rows& r, int lead) {                // lead: how many leading dimensions of x stay
+    c10::SmallVector<int64_t, 6> qs(r.x->sizes().begin(), r.x->sizes().begin() + lead), ss;
+    qs.push_back((r.n + 1) / 2);
+    for (int i = 0; i < lead; ++i) {
+        if (i == 1) ss.push_back(1);
+        ss.push_back(r.x->size(i));
+    }
+    if (lead <= 1) ss.push_back(1);
+    return Packed{fresh(qs, kByte, r.device), fresh(ss, kHalf, r.device)};
+}
+
+bool arg_int(PyObject* o, long long* v) {
+    *v = PyLong_AsLongLong(o);
+    if (*v == -1 && PyErr_Occurred()) {
+        PyErr_Clear();
+        return false;
+    }
+    return true;
+}
+bool arg_float(PyObject* o, double* v) {
+    *v = PyFloat_AsDouble(o);
+    if (*v == -1.0 && PyErr_Occurred()) {
+        PyErr_Clear();
+        return false;
+    }
+    return true;
+}
+
+#define QR_ARGS(COUNT)                                                     \
+    if (nargs != (COUNT)) {                                                \
+        PyErr_SetString(PyExc_TypeError, "expected " #COUNT " arguments"); \
+        return nullptr;                                                    \
+    }                                                                      \
+    try {
+#define QR_END                                                             \
+    }                                                                      \
+    catch (const std::exception& e) {                                      \
+        PyErr_SetString(PyExc_RuntimeError, e.what());                     \
+        return nullptr;                                                    \
+    }
+
+// quantize_rows(x, clip) -> (codes, scales)
+PyObject* quantize_rows(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
+    QR_ARGS(2)
+    const Rows r = rows_of(a[0]);
+    double clip;
+    if (!r.ok || !arg_float(a[1], &clip)) return none();
+    Packed p = packed_for(r, (int)r.x->dim() - 1);
+    if (qr_quantize_rows_f16_i4(r.x->data_ptr(), (float)clip, r.rows, r.n, p.codes.data_ptr(), p.scales.data_ptr(),
+                                stream(r.device)) != QR_OK)
+        return none();
+    return wrap2(std::move(p.codes), std::move(p.scales));
+    QR_END
+}
+
+// rmsnorm(x, mean_dim, eps) -> y
+PyObject* rmsnorm(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
+    QR_ARGS(3)
+    const Rows r = rows_of(a[0]);
+    long long mean_dim;
+    double eps;
+    if (!r.ok || !arg_int(a[1], &mean_dim) || !arg_float(a[2], &eps) || mean_dim > 0x7fffffff) return none();
+    at::Tensor y = fresh(r.x->sizes(), kHalf, r.device);
+    if (qr_rmsnorm_f16(r.x->data_ptr(), r.rows, r.n, (int)mean_dim, (float)eps, y.data_ptr(), stream(r.device)) != QR_OK)
+        return none();
+    return wrap(std::move(y));
+    QR_END
+}
+
+// rmsnorm_quantize(x, mean_dim, eps, clip) -> (codes, scales)
+PyObject* rmsnorm_quantize(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
+    QR_ARGS(4)
+    const Rows r = rows_of(a[0]);
+    long long mean_dim;
+    double eps, clip;
+    if (!r.ok || r.n % 8 || !arg_int(a[1], &mean_dim) || !arg_float(a[2], &eps) || !arg_float(a[3], &clip) || mean_dim > 0x7fffffff)
+        return none();
+    Packed p = packed_for(r, (int)r.x->dim() - 1);
+    if (qr_rmsnorm_quantize_f16_i4(r.x->data_ptr(), r.rows, r.n, (int)mean_dim, (float)eps, (float)clip, p.codes.data_ptr(),
+                                   p.scales.data_ptr(), nullptr, stream(r.device)) != QR_OK)
+        return none();
+    return wrap2(std::move(p.codes), std::move(p.scales));
+    QR_END
+}
+
+// heads_hadamard_quantize(x [..., heads, 128], clip, hadK or None) -> (codes, scales) of the rows reshaped to [..., heads * 128]
+PyObject* heads_hadamard_quantize(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
+    QR_ARGS(3)
+    Rows r = rows_of(a[0]);
+    double clip;
+    if (!r.ok || r.x->dim() < 2 || r.n != 128 || !arg_float(a[1], &clip)) return none();
+    const int64_t heads = r.x->size(-2);
+    const at::Tensor* hadK;
+    if (!plain_or_none(a[2], kHalf, r.device, &hadK) || heads > 64 || (hadK && hadK->numel() != heads * heads)) return none();
+    r.n = heads * 128;
+    r.rows = r.x->numel() / r.n;
+    Packed p = packed_for(r, (int)r.x->dim() - 2);
+    if (qr_heads_hadamard_quantize_f16_i4(r.x->data_ptr(), r.rows, (int)heads, 128, ptr(hadK), (float)clip, p.codes.data_ptr(),
+                                          p.scales.data_ptr(), nullptr, stream(r.device)) != QR_OK)
+        return none();
+    return wrap2(std::move(p.codes), std::move(p.scales));
+    QR_END
+}
+
+// A Hadamard factor as the library takes it: None (K = 1), the table of the mode's dtype, or its sign words.
+bool table_arg(PyObject* o, long long mode, int64_t K, int device, const at::Tensor** out) {
+    *out = nullptr;
+    if (K <= 1) return true;
+    const bool signs = (mode & QR_HADK_SIGNS) != 0;
+    *out = tensor(o);
+    const auto dtype = signs ? kByte : (mode & ~(QR_HADK_SIGNS | QR_HAD_FP32)) == QR_DTYPE_F32 || (mode & QR_HAD_FP32) ? at::kFloat : kHalf;
+    return plain(*out, dtype, device) && (*out)->numel() == (signs ? K * ((K + 31) / 32) * 4 : K * K);
+}
+
+// hadamard(x, hadK or None, K, mode, scale) -> y: qr_hadamard on fp16 rows (mode QR_DTYPE_F16, optionally | QR_HAD_FP32)
+PyObject* hadamard(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
+    QR_ARGS(5)
+    const Rows r = rows_of(a[0]);
+    long long K, mode;
+    double scale;
+    const at::Tensor* table;
+    if (!r.ok || !arg_int(a[2], &K) || !arg_int(a[3], &mode) || !arg_float(a[4], &scale) || r.n > 0x7fffffff ||
+        (mode & ~QR_HAD_FP32) != QR_DTYPE_F16 || !table_arg(a[1], mode, K, r.device, &table))
+        return none();
+    at::Tensor y = fresh(r.x->sizes(), kHalf, r.device);
+    if (qr_hadamard(r.x->data_ptr(), y.data_ptr(), r.rows, (int)r.n, (int)K, ptr(table), (int)mode, (float)scale,
+                    stream(r.device)) != QR_OK)
+        return none();
+    return wrap(std::move(y));
+    QR_END
+}
+
+// hadamard_quantize(x, table, K, mode, scale, clip) -> (codes, scales)
+PyObject* hadamard_quantize(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
+    QR_ARGS(6)
+    const Rows r = rows_of(a[0]);
+    long long K, mode;
+    double scale, clip;
+    const at::Tensor* table;
+    if (!r.ok || r.n % 2 || r.n > 0x7fffffff || !arg_int(a[2], &K) || !arg_int(a[3], &mode) || !arg_float(a[4], &scale) ||
+        !arg_float(a[5], &clip) || !table_arg(a[1], mode, K, r.device, &table))
+        return none();
+    Packed p = packed_for(r, (int)r.x->dim() - 1);
+    if (qr_hadamard_quantize_f16_i4(r.x->data_ptr(), r.rows, (int)r.n, (int)K, ptr(table), (int)mode, (float)scale, (float)clip,
+                                    p.codes.data_ptr(), p.scales.data_ptr(), nullptr, stream(r.device)) != QR_OK)
+        return none();
+    return wrap2(std::move(p.codes), std::move(p.scales));
+    QR_END
+}
+
+// weight [N, K / 2], its scales and an optional bias
+struct Weight {
+    const at::Tensor *w, *s, *b;
+    int64_t N;
+};
+bool weight_args(PyObject* w, PyObject* s, PyObject* b, int64_t half_k, int device, Weight* out) {
+    out->w = tensor(w);
+    out->s = tensor(s);
+    if (!plain(out->w, kByte, device) || !plain(out->s, kHalf, device) || !plain_or_none(b, kHalf, device, &out->b)) return false;
+    if (out->w->dim() != 2 || out->w->size(1) != half_k) return false;
+    out->N = out->w->size(0);
+    return out->N > 0 && out->s->numel() == out->N && (!out->b || out->b->numel() == out->N);
+}
+
+// linear(codes, scales, weight, weight_scales, bias or None) -> y
+PyObject* linear(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
+    QR_ARGS(5)
+    const at::Tensor *q = tensor(a[0]), *sx = tensor(a[1]);
+    const int device = device_of(q);
+    Weight w;
+    if (!plain(q, kByte, device) || !plain(sx, kHalf, device) || q->dim() < 1 || q->numel() == 0) return none();
+    const int64_t half_k = q->size(-1), M = q->numel() / half_k;
+    if (sx->numel() != M || !weight_args(a[2], a[3], a[4], half_k, device, &w)) return none();
+    c10::SmallVector<int64_t, 6> sizes(q->sizes().begin(), q->sizes().end());
+    sizes.back() = w.N;
+    at::Tensor y = fresh(sizes, kHalf, device);
+    const size_t need = qr_workspace_bytes(M, w.N, half_k * 2);
+    at::Tensor ws;                                          // (few output tiles: room for the slabs of a K split)
+    if (need) ws = fresh({(int64_t)need}, kByte, device);
+    if (qr_linear_i4_f16_ws(q->data_ptr(), sx->data_ptr(), w.w->data_ptr(), w.s->data_ptr(), ptr(w.b), M, w.N, half_k * 2,
+                            y.data_ptr(), need ? ws.data_ptr() : nullptr, need, stream(device)) != QR_OK)
+        return none();
+    return wrap(std::move(y));
+    QR_END
+}
+
+// quantized_linear(x, table or None, K, mode, scale, clip, weight, weight_scales, bias or None) -> y (K = 0: no Hadamard)
+PyObject* quantized_linear(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
+    QR_ARGS(9)
+    const Rows r = rows_of(a[0]);
+    long long K, mode;
+    double scale, clip;
+    const at::Tensor* table;
+    Weight w;
+    if (!r.ok || r.n % 64 || r.n > 0x7fffffff || !arg_int(a[2], &K) || !arg_int(a[3], &mode) || !arg_float(a[4], &scale) ||
+        !arg_float(a[5], &clip) || !table_arg(a[1], mode, K, r.device, &table) ||
+        !weight_args(a[6], a[7], a[8], r.n / 2, r.device, &w))
+        return none();
+    c10::SmallVector<int64_t, 6> sizes(r.x->sizes().begin(), r.x->sizes().end());
+    sizes.back() = w.N;
+    at::Tensor y = fresh(sizes, kHalf, r.device);
+    const size_t need = qr_quantized_linear_workspace_bytes(r.rows, w.N, r.n);
+    at::Tensor ws = fresh({(int64_t)(need < 16 ? 16 : need)}, kByte, r.device);
+    if (qr_quantized_linear_f16(r.x->data_ptr(), r.rows, r.n, (int)K, ptr(table), (int)mode, (float)scale, (float)clip,
+                                w.w->data_ptr(), w.s->data_ptr(), ptr(w.b), w.N, y.data_ptr(), ws.data_ptr(), need,
+                                stream(r.device)) != QR_OK)
+        return none();
+    return wrap(std::move(y));
+    QR_END
+}
+
+// ---- the paged cache -------------------------------------------------------------------------------------------------
+struct Cache {
+    const at::Tensor *data, *param, *indptr, *indices, *last;
+    int64_t pages, batch;
+    int layers, heads, page_size;
+};
+bool cache_args(PyObject* const* a, int device, long long layer, Cache* c) {
+    c->data = tensor(a[0]);
+    c->param = tensor(a[1]);
+    c->indptr = tensor(a[2]);
+    c->indices = tensor(a[3]);
+    c->last = tensor(a[4]);
+    if (!plain(c->data, kByte, device) || !plain(c->param, kHalf, device) || !plain(c->indptr, at::kInt, device) ||
+        !plain(c->indices, at::kInt, device) || !plain(c->last, at::kInt, device))
+        return false;
+    const auto d = c->data->sizes(), p = c->param->sizes();
+    if (d.size() != 6 || p.size() != 6 || d[2] != 2 || d[5] != 64 || p[5] != 2) return false;
+    for (int i = 0; i < 5; ++i)
+        if (d[i] != p[i] || d[i] > 0x7fffffff) return false;
+    c->pages = d[0];
+    c->layers = (int)d[1];
+    c->heads = (int)d[3];
+    c->page_size = (int)d[4];
+    c->batch = c->last->numel();
+    return c->indptr->dim() == 1 && c->indices->dim() == 1 && c->last->dim() == 1 && c->batch > 0 &&
+           c->indptr->numel() == c->batch + 1 && layer >= 0 && layer < c->layers;
+}
+
+// page_tables(batch, length, page_size, reference tensor on the device) -> (indptr, indices, last_page_offset)
+PyObject* page_tables(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
+    QR_ARGS(4)
+    long long batch, length, page;
+    const int device = device_of(tensor(a[3]));
+    if (device < 0 || !arg_int(a[0], &batch) || !arg_int(a[1], &length) || !arg_int(a[2], &page) || batch <= 0 || page <= 0 ||
+        length <= 0 || page > 0x7fffffff)
+        return none();
+    at::Tensor indptr = fresh({batch + 1}, at::kInt, device);
+    at::Tensor indices = fresh({batch * ((length + page - 1) / page)}, at::kInt, device);
+    at::Tensor last = fresh({batch}, at::kInt, device);
+    if (qr_page_tables(batch, length, (int)page, indptr.data_ptr(), indices.data_ptr(), last.data_ptr(), stream(device)) != QR_OK)
+        return none();
+    PyObject* t = PyTuple_New(3);
+    if (!t) return nullptr;
+    at::Tensor* const all[3] = {&indptr, &indices, &last};
+    for (int i = 0; i < 3; ++i) {
+        PyObject* o = wrap(std::move(*all[i]));
+        if (!o) {
+            Py_DECREF(t);
+            return nullptr;
+        }
+        PyTuple_SET_ITEM(t, i, o);
+    }
+    return t;
+    QR_END
+}
+
+// quantize_append(kv_data, kv_param, indptr, indices, last, k, v, seqlen_indptr or None, layer, hadamard) -> True
+PyObject* quantize_append(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
+    QR_ARGS(10)
+    const int device = device_of(tensor(a[0]));
+    long long layer;
+    Cache c;
+    if (!arg_int(a[8], &layer) || !cache_args(a, device, layer, &c)) return none();
+    const at::Tensor *k = tensor(a[5]), *v = tensor(a[6]), *seq;
+    if (!plain(k, kHalf, device) || !plain(v, kHalf, device) || !plain_or_none(a[7], at::kInt, device, &seq)) return none();
+    if (k->dim() != 3 || k->sizes() != v->sizes() || k->size(1) != c.heads || k->size(2) != 128 || k->numel() == 0) return none();
+    const int64_t tokens = k->size(0);
+    if (seq ? (seq->dim() != 1 || seq->numel() != c.batch + 1) : tokens != c.batch) return none();
+    const int had = PyObject_IsTrue(a[9]);
+    if (qr_kv_quant_append_f16_i4(k->data_ptr(), v->data_ptr(), tokens, ptr(seq), had ? 1 : 0, c.data->data_ptr(), c.param->data_ptr(),
+                                  c.indptr->data_ptr(), c.indices->data_ptr(), c.last->data_ptr(), c.pages, c.layers, (int)layer, c.heads,
+                                  c.page_size, 128, c.batch, stream(device)) != QR_OK)
+        return none();
+    Py_RETURN_TRUE;
+    QR_END
+}
+
+// decode_step(kv_data, kv_param, indptr, indices, last, q, k, v, layer, q_hadamard, k_hadamard, max_seq_len, workspace or None)
+// -> o.  The step's new token is quantised, stored and attended to in the same launch; a workspace has zeroed counters.
+PyObject* decode_step(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
+    QR_ARGS(13)
+    const int device = device_of(tensor(a[0]));
+    long long layer, bound;
+    Cache c;
+    if (!arg_int(a[8], &layer) || !arg_int(a[11], &bound) || !cache_args(a, device, layer, &c)) return none();
+    const at::Tensor *q = tensor(a[5]), *k = tensor(a[6]), *v = tensor(a[7]), *ws;
+    if (!plain(q, kHalf, device) || !plain(k, kHalf, device) || !plain(v, kHalf, device) || !plain_or_none(a[12], kByte, device, &ws))
+        return none();
+    const int64_t vec = c.batch * c.heads * 128;
+    if (q->numel() != vec || k->numel() != vec || v->numel() != vec || q->size(-1) != 128 || k->size(-1) != 128 || v->size(-1) != 128 ||
+        q->dim() < 2 || q->size(-2) != c.heads || k->size(-2) != c.heads || v->size(-2) != c.heads)
+        return none();
+    const size_t need = bound > 0 ? qr_batch_decode_workspace_bytes(c.batch, c.heads, bound) : 0;
+    const bool kept = need && ws && (size_t)ws->numel() >= need;
+    at::Tensor own;
+    if (need && !kept) own = fresh({(int64_t)need}, kByte, device);
+    const int qh = (PyObject_IsTrue(a[9]) ? 1 : 0) | (kept ? QR_DECODE_COUNTERS_ZERO : 0), kh = PyObject_IsTrue(a[10]) ? 1 : 0;
+    at::Tensor o = fresh(q->sizes(), kHalf, device);
+    if (qr_kv_quant_append_batch_decode_f16_i4(o.data_ptr(), q->data_ptr(), qh, k->data_ptr(), v->data_ptr(), kh, c.data->data_ptr(),
+                                               c.param->data_ptr(), c.indptr->data_ptr(), c.indices->data_ptr(), c.last->data_ptr(),
+                                               c.pages, c.layers, (int)layer, c.heads, c.page_size, 128, c.batch, bound,
+                                               kept ? ws->data_ptr() : need ? own.data_ptr() : nullptr, need, stream(device)) != QR_OK)
+        return none();
+    return wrap(std::move(o));
+    QR_END
+}
+
+#define QR_METHOD(NAME) {#NAME, (PyCFunction)(void (*)(void))NAME, METH_FASTCALL, nullptr}
+PyMethodDef methods[] = {QR_METHOD(quantize_rows),
+                         QR_METHOD(rmsnorm),
+                         QR_METHOD(rmsnorm_quantize),
+                         QR_METHOD(heads_hadamard_quantize),
+                         QR_METHOD(hadamard),
+                         QR_METHOD(hadamard_quantize),
+                         QR_METHOD(linear),
+                         QR_METHOD(quantized_linear),
+                         QR_METHOD(page_tables),
+                         QR_METHOD(quantize_append),
+                         QR_METHOD(decode_step),
+                         {nullptr, nullptr, 0, nullptr}};
+PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__host() { return PyModule_Create(&module); }

@@ -100,6 +100,9 @@ def hadamard_transform(x, scale=1.0):
 
 
 def _run(x, hadK, K, scale):
+    y = _lib.host.hadamard(x, hadK, K, _lib.QR_DTYPE_F16, scale)
+    if y is not None:
+        return y
     if x.dtype not in (torch.float16, torch.float32):
         raise RuntimeError(f"hadamard: unsupported dtype {x.dtype}")
     if not x.is_cuda:
@@ -141,6 +144,9 @@ def matmul_hadU_cuda_fp32(X, hadK, K):
     """matmul_hadU_cuda(X.float(), hadK, K) rounded to X's fp16, in one pass over fp16 rows on the GPU; the two conversions
     around the fp32 transform where the library has no such kernel (rows of 128 and shorter, beyond 32768)."""
     n = X.shape[-1]
+    y = _lib.host.hadamard(X, hadK, K, _lib.QR_DTYPE_F16 | _lib.QR_HAD_FP32, had_scale(n))
+    if y is not None:
+        return y
     if 128 < n <= MAX_FUSED_ROW and (K == 1 or hadK is not None):
         xc = X.contiguous()
         table = None if K == 1 else hadK.to(device=xc.device, dtype=torch.float32).contiguous()

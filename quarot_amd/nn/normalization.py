@@ -36,6 +36,9 @@ class RMSNormQuantizer(torch.nn.Module):
         self.input_clip_ratio = input_clip_ratio
 
     def forward(self, x: torch.Tensor):
+        fast = quarot_amd._host.rmsnorm_quantize(x, self.mean_dim, self.eps, self.input_clip_ratio)
+        if fast is not None:
+            return quarot_amd.PackedQuantizedTensor(*fast)
         if x.dtype != torch.float16 or x.shape[-1] % 8 != 0 or x.shape[-1] > 32768:
             y = RMSNorm(self.mean_dim, self.eps)(x)
             return quarot_amd.PackedQuantizedTensor(*quarot_amd.quantize_rows(y, self.input_clip_ratio))

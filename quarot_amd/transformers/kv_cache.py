@@ -4,7 +4,6 @@ the cache) and the cache class the model code drives; and the same cache with fp
 disable_quant mode: init_kv_f16 / append_kv_f16 / batch_decode_f16)."""
 import functools
 import math
-import weakref
 
 import torch
 
@@ -70,24 +69,9 @@ def matmul_had_cuda(X, dtype):
 # paged int4 cache: kv_data uint8 [pages, layers, 2, heads, page_size, head_dim / 2],
 # kv_param fp16 [pages, layers, 2, heads, page_size, 2] = {scale, zero}
 
-_CHECKED = None     # the five cache tensors validated last (weak references), their element counts, their dimensions
-
-
 def _cache_args(fn, kv_data, kv_param, kv_indptr, kv_indices, last_page_offset, layer_idx, f16=False):
     """The checks of quarot/kernels/bindings.cpp:118-374 (CHECK_INPUT / CHECK_DIM / CHECK_EQ) as RuntimeError; f16: the
-    cache with fp16 pages (the *_f16 bindings).
-    A decode step passes the same five tensor objects to the append and to the attention of every layer: the
-    objects validated last (same identity, same element counts) are not walked through again."""
-    global _CHECKED
-    seen = _CHECKED
-    if seen is not None:
-        refs, counts, dims = seen
-        if (refs[0]() is kv_data and refs[1]() is kv_param and refs[2]() is kv_indptr and refs[3]() is kv_indices
-                and refs[4]() is last_page_offset and kv_data.dtype == (torch.float16 if f16 else torch.uint8)
-                and counts == (kv_data.numel(), kv_param.numel(), kv_indptr.numel(), kv_indices.numel(), last_page_offset.numel())):
-            if not (0 <= int(layer_idx) < dims[1]):
-                raise RuntimeError(f"{fn}: layer_idx out of range")
-            return dims
+    cache with fp16 pages (the *_f16 bindings)."""
     for name, t in (("kv_data", kv_data), ("kv_param", kv_param), ("kv_indptr", kv_indptr), ("kv_indicies", kv_indices),
                     ("last_page_offset", last_page_offset)):
         if not (t.is_cuda):
@@ -115,10 +99,7 @@ def _cache_args(fn, kv_data, kv_param, kv_indptr, kv_indices, last_page_offset, 
         raise RuntimeError(f"{fn}: CHECK_EQ(head_dim, 128) failed. {head_dim} vs 128")
     if not (0 <= int(layer_idx) < layers):
         raise RuntimeError(f"{fn}: layer_idx out of range")
-    dims = (pages, layers, heads, page_size, head_dim)
-    five = (kv_data, kv_param, kv_indptr, kv_indices, last_page_offset)
-    _CHECKED = (tuple(weakref.ref(t) for t in five), tuple(t.numel() for t in five), dims)
-    return dims
+    return pages, layers, heads, page_size, head_dim
 
 
 def _append(fn, kv_data, kv_param, kv_indptr, kv_indices, last_page_offset, k, v, k_param, v_param, seqlen_indptr, layer_idx,
@@ -214,6 +195,8 @@ def quantize_append_kv_i4(kv_data, kv_param, kv_indptr, kv_indices, last_page_of
     straight into the pages: matmul_had_cuda + asym_quantize_and_pack_i4 (twice) + the two torch.cat +
     init_kv_i4 / append_kv_i4 of MultiLayerPagedKVCache4Bit.update (kv_cache.py:174-251) as one launch,
     with the same codes, scales and zeros.  seqlen_indptr None: one token per sequence."""
+    if _lib.host.quantize_append(kv_data, kv_param, kv_indptr, kv_indices, last_page_offset, k, v, seqlen_indptr, layer_idx, hadamard):
+        return
     fn = "quantize_append_kv_i4"
     pages, layers, heads, page_size, head_dim = _cache_args(fn, kv_data, kv_param, kv_indptr, kv_indices, last_page_offset, layer_idx)
     batch = last_page_offset.shape[0]
@@ -319,6 +302,16 @@ class _AttentionStub(object):
     def forward(self, q, num_kv_heads, attention_kwargs, layer_idx, max_seq_len=0, workspace=None, take_pending=None):
         batch_size, q_len, num_qo_heads, head_dim = q.shape
         assert q_len == 1
+        # the step's new token, if the cache still holds it back for this call (see MultiLayerPagedKVCache4Bit.update)
+        append = take_pending() if take_pending is not None else None
+        if append is not None and self.hadamard_dtype in (None, torch.float16):
+            s = attention_kwargs
+            o = _lib.host.decode_step(s["kv_data"], s["kv_param"], s["kv_indptr"], s["kv_indices"], s["last_page_offset"], q,
+                                      append[0], append[1], layer_idx, self.hadamard_dtype is not None, append[2], max_seq_len, workspace)
+            if o is not None:
+                return o
+        if append is not None:
+            append = (append[0].view(batch_size, -1, head_dim), append[1].view(batch_size, -1, head_dim), append[2])
         q = q.view(batch_size, num_qo_heads, head_dim)
         if self.disable_quant:                   # fp16 pages (kv_cache.py:116-119)
             if self.hadamard_dtype is not None:
@@ -330,8 +323,6 @@ class _AttentionStub(object):
         if self.hadamard_dtype is not None and not fused:
             q = matmul_had_cuda(q, dtype=self.hadamard_dtype)
         attn_output = torch.empty_like(q)
-        # the step's new token, if the cache still holds it back for this call (see MultiLayerPagedKVCache4Bit.update)
-        append = take_pending() if take_pending is not None else None
         batch_decode_i4(attn_output, q, **attention_kwargs, layer_idx=layer_idx, max_seq_len=max_seq_len, q_hadamard=fused,
                         workspace=workspace, append=append, counters_zero=workspace is not None)
         return attn_output.unsqueeze(1)
@@ -390,7 +381,8 @@ class MultiLayerPagedKVCache4Bit:
             held = self._pending.pop(layer, None)
             if held is not None:
                 _, k, v, specs, hadamard = held
-                quantize_append_kv_i4(**specs, k=k, v=v, seqlen_indptr=None, layer_idx=layer, hadamard=hadamard)
+                quantize_append_kv_i4(**specs, k=k.view(k.shape[0], *k.shape[-2:]), v=v.view(v.shape[0], *v.shape[-2:]),
+                                      seqlen_indptr=None, layer_idx=layer, hadamard=hadamard)
 
     def _take_pending(self, layer_idx, token):
         held = self._pending.get(layer_idx)
@@ -428,14 +420,13 @@ class MultiLayerPagedKVCache4Bit:
     def update(self, key_states, value_states, layer_idx, cache_kwargs=None):
         b_sz, added_length, num_heads, head_dim = key_states.shape
         assert b_sz == self.batch_size
-        cache_kwargs = cache_kwargs or {}
         if self._pending:
             self._flush()
         if layer_idx == 0:
             new_length = self.length + added_length
             self._ensure_page_cnt_per_batch(self.page_cnt_from_length(new_length))
             self.length = new_length
-        attention_mask = cache_kwargs.get("attention_mask")
+        attention_mask = cache_kwargs.get("attention_mask") if cache_kwargs else None
         first = self._needs_init[layer_idx]
         specs = self.get_cache_specs_for_flash_infer(attention_mask)
         if self.disable_quant:
@@ -464,15 +455,15 @@ class MultiLayerPagedKVCache4Bit:
                                       layer_idx=layer_idx, hadamard=fused_had)
             return key_states, value_states
         assert added_length == 1
-        k3 = k_in.reshape(self.batch_size, num_heads, head_dim).contiguous()
-        v3 = value_states.reshape(self.batch_size, num_heads, head_dim).contiguous()
-        if k3.dtype == torch.float16 and v3.dtype == torch.float16 and head_dim == 128:
+        k1, v1 = k_in.contiguous(), value_states.contiguous()
+        if k1.dtype == torch.float16 and v1.dtype == torch.float16 and head_dim == 128:
             # held for the attention call, which quantises and stores the token itself
             token = object()
-            self._pending[layer_idx] = (token, k3, v3, specs, fused_had)
+            self._pending[layer_idx] = (token, k1, v1, specs, fused_had)
             take = functools.partial(self._take_pending, layer_idx, token)
         else:
-            quantize_append_kv_i4(**specs, k=k3, v=v3, seqlen_indptr=None, layer_idx=layer_idx, hadamard=fused_had)
+            quantize_append_kv_i4(**specs, k=k1.view(b_sz, num_heads, head_dim), v=v1.view(b_sz, num_heads, head_dim),
+                                  seqlen_indptr=None, layer_idx=layer_idx, hadamard=fused_had)
             take = None
         return functools.partial(self._stub.forward, num_kv_heads=num_heads, attention_kwargs=specs, layer_idx=layer_idx,
                                  max_seq_len=self.length, workspace=self._decode_workspace(num_heads), take_pending=take)
@@ -509,21 +500,21 @@ class MultiLayerPagedKVCache4Bit:
             self._flush()
         if attention_mask is None:
             # every sequence holds self.length tokens: the tables depend on that number alone and are built
-            # once per length (every layer of a decode step asks for them), with host arithmetic
+            # once per length (every layer of a decode step asks for them), by one launch
             cached = getattr(self, "_specs", None)
             if cached is not None and cached[0] == self.length:
                 return cached[1]
-            page_cnt = self.page_cnt_from_length(self.length)
-            ptr = self.length % self.page_size
-            ptr = self.page_size if (self.length != 0 and ptr == 0) else ptr
-            arange = functools.partial(torch.arange, device=self.device, dtype=torch.int32)
-            specs = {
-                "kv_data": self._pages,
-                "kv_indptr": arange(0, self.batch_size + 1) * page_cnt,
-                "kv_indices": (arange(page_cnt).unsqueeze(0) * self.batch_size + arange(self.batch_size).unsqueeze(1)).reshape(-1),
-                "last_page_offset": torch.full((self.batch_size,), ptr, dtype=torch.int32, device=self.device),
-                "kv_param": self._scales,
-            }
+            tables = _lib.host.page_tables(self.batch_size, self.length, self.page_size, self._pages)
+            if tables is None:                   # an empty cache, or one on another than the current device
+                page_cnt = self.page_cnt_from_length(self.length)
+                ptr = self.length % self.page_size
+                ptr = self.page_size if (self.length != 0 and ptr == 0) else ptr
+                arange = functools.partial(torch.arange, device=self.device, dtype=torch.int32)
+                tables = (arange(0, self.batch_size + 1) * page_cnt,
+                          (arange(page_cnt).unsqueeze(0) * self.batch_size + arange(self.batch_size).unsqueeze(1)).reshape(-1),
+                          torch.full((self.batch_size,), ptr, dtype=torch.int32, device=self.device))
+            specs = {"kv_data": self._pages, "kv_indptr": tables[0], "kv_indices": tables[1], "last_page_offset": tables[2],
+                     "kv_param": self._scales}
             self._specs = (self.length, specs)
             return specs
         seqlens_in_batch = attention_mask.sum(dim=-1, dtype=torch.int32)

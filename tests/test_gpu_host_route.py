@@ -1,0 +1,80 @@
+"""The native host side of the entry points (csrc/host.cpp): same results and shapes as the general route of the Python
+wrappers, and None -- which sends a call down that route -- for whatever is not its plain case."""
+import pytest
+import torch
+
+import quarot_amd
+from quarot_amd import _lib
+from quarot_amd.transformers import kv_cache as kv
+
+pytestmark = pytest.mark.gpu
+host = quarot_amd._host
+
+
+class _Refuses:
+    """A host module that refuses every call: the wrappers take their general route."""
+
+    def __getattr__(self, name):
+        return lambda *args: None
+
+
+@pytest.fixture
+def general_route(monkeypatch):
+    def switch():
+        monkeypatch.setattr(quarot_amd, "_host", _Refuses())
+        monkeypatch.setattr(_lib, "host", _Refuses())
+    return switch
+
+
+@pytest.mark.parametrize("lead", [(1,), (7,), (2, 3), (1, 70), (2, 1, 3)])
+def test_same_results_and_shapes_as_the_general_route(lead, general_route):
+    torch.manual_seed(len(lead))
+    x = torch.randn(*lead, 11008, device="cuda").half()
+    nn = quarot_amd.nn
+    with torch.device("cuda"):
+        lin = nn.Linear4bit(11008, 320, bias=True).half()
+        plain = nn.Linear4bit(11008, 320).half()
+    lin.weight_scales.uniform_(1e-3, 2e-3), plain.weight_scales.uniform_(1e-3, 2e-3), lin.bias.normal_()
+    xh = torch.randn(*lead, 40, 128, device="cuda").half()
+    modules = [nn.Quantizer(0.9), nn.RMSNorm(11008), nn.RMSNormQuantizer(11008, input_clip_ratio=0.95), nn.OnlineHadamard(11008).cuda(),
+               nn.OnlineHadamard(11008, force_fp32=True).cuda(), nn.OnlineHadamardQuantizer(11008).cuda(),
+               nn.OnlineHadamardQuantizer(11008, force_fp32=True).cuda(), nn.HeadsHadamardQuantizer(40).cuda(),
+               nn.Linear4bitSequential(nn.Quantizer(), lin), nn.Linear4bitSequential(nn.OnlineHadamard(11008).cuda(), nn.Quantizer(), plain),
+               torch.nn.Sequential(nn.Quantizer(), lin)]
+    run = lambda: [m(xh if isinstance(m, nn.HeadsHadamardQuantizer) else x) for m in modules]
+    got = run()
+    general_route()
+    for a, b in zip(got, run()):
+        if isinstance(a, quarot_amd.PackedQuantizedTensor):
+            assert a.scales_x.shape == b.scales_x.shape and torch.equal(a.scales_x.view(torch.int16), b.scales_x.view(torch.int16))
+            a, b = a.quantized_x, b.quantized_x
+        assert a.shape == b.shape and a.dtype == b.dtype
+        assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
+
+
+def test_refuses_what_is_not_its_plain_case():
+    x = torch.randn(4, 128, device="cuda").half()
+    for bad in (x.cpu(), x.float(), x.t(), x[:, ::2], x[:0], x[0, 0], torch.nn.Module(), None, 3):
+        assert host.quantize_rows(bad, 1.0) is None
+    assert host.quantize_rows(x, "1.0") is None
+    assert isinstance(host.quantize_rows(torch.nn.Parameter(x, requires_grad=False), 1.0), tuple)
+    q, s = host.quantize_rows(x, 1.0)
+    w, sw = torch.zeros(8, 64, dtype=torch.uint8, device="cuda"), torch.ones(8, 1, device="cuda").half()
+    assert host.linear(q, s, w, sw, None).shape == (4, 8)
+    for args in ((q, s[:2], w, sw, None), (q, s, w[:, :32], sw, None), (q, s, w, sw[:4], None), (q, s, w, sw, sw[:4].view(-1)),
+                 (q, s, w, sw.float(), None), (q.cpu(), s, w, sw, None), (q, s, None, sw, None)):
+        assert host.linear(*args) is None
+    with pytest.raises(TypeError):
+        host.linear(q, s)
+
+
+@pytest.mark.parametrize("batch,length,page", [(1, 1, 16), (3, 16, 16), (5, 17, 16), (2, 4001, 128), (40, 300, 5)])
+def test_page_tables_in_one_launch(batch, length, page, general_route):
+    c = kv.MultiLayerPagedKVCache4Bit(batch, page, length, "cuda", 1, 1, 128)
+    c.length = length
+    got = c.get_cache_specs_for_flash_infer(None)
+    general_route()
+    c._specs = None
+    want = c.get_cache_specs_for_flash_infer(None)
+    for name in ("kv_indptr", "kv_indices", "last_page_offset"):
+        assert got[name].dtype == torch.int32 and torch.equal(got[name], want[name]), name
