@@ -61,11 +61,10 @@ __device__ __forceinline__ bool paged_locate(const PagedKV& c, const int32_t* __
     return page >= 0 && page < c.num_pages;
 }
 
-// destination of a quantise-and-append kernel: the cache, which tokens the vectors belong to, K or V
+// destination of a quantise-and-append kernel: the cache, which tokens the vectors belong to
 struct PagedDst {
     PagedKV c;
     const int32_t* append_indptr;     // nullptr: one new token per sequence
-    int kv;                           // 0: K, 1: V
 };
 
 __device__ __forceinline__ u32 pack_scale_zero(f16 scale, f16 zero) {

@@ -109,6 +109,31 @@ def test_quantise_and_append_places_the_oracle_quantisers_codes(page_size, lens,
     assert torch.equal(gd2, gd3) and torch.equal(gp2, gp3)
 
 
+@pytest.mark.parametrize("heads,page_size,lens,add", [
+    (1, 16, [70, 1], [70, 1]),               # one head: blocks of 32 tokens, the last one short
+    (2, 16, [16], [16]), (3, 5, [17, 40], [17, 33]), (5, 64, [90], [31]),      # 16 tokens x 2 heads: whole, odd heads, remainders
+    (7, 16, [9, 9], [5, 0]), (33, 16, [3], [3]), (64, 16, [2, 40], [1, 1]), (40, 1, [1], [1]),   # fewer tokens than a block holds
+    (2, 16, [3] * 1024, [2] * 1024), (2, 16, [3] * 1025, [2] * 1025),          # the table of sequences: full, and one too many
+    (8, 16, [9, 30], [12, 30]), (8, 128, [20000], [20000]),                    # tokens without a place; several rounds of workgroups
+])
+def test_quantise_and_append_at_the_edges_of_its_blocks(heads, page_size, lens, add):
+    """Every byte of the cache equals the oracle quantiser's codes at the oracle append's places; tokens of an append longer than
+    its sequence have no place and are written nowhere."""
+    rng = np.random.default_rng(heads * 1000 + page_size)
+    data, param, indptr, indices, last = paged_case(rng, heads, page_size, lens, layers=1)
+    app = np.concatenate([[0], np.cumsum(add)]).astype(np.int32)
+    k, v = synth_kv(rng, int(app[-1]), heads), synth_kv(rng, int(app[-1]), heads)
+    gd, gp = gpu(data), gpu(param)
+    kv.quantize_append_kv_i4(gd, gp, gpu(indptr), gpu(indices), gpu(last), gpu(k), gpu(v), gpu(app), 0, hadamard=True)
+    kq, ks, kz = o.kv_asym_quant(kv.matmul_had_cuda(gpu(k), torch.float16).cpu().numpy())
+    vq, vs, vz = o.kv_asym_quant(v)
+    kp, vp = np.concatenate([ks, kz], -1), np.concatenate([vs, vz], -1)
+    placed = np.concatenate([np.arange(app[b] + max(0, add[b] - lens[b]), app[b + 1]) for b in range(len(lens))])
+    fits = np.concatenate([[0], np.cumsum(np.minimum(add, lens))]).astype(np.int32)
+    o.paged_append(data, param, indptr, indices, last, kq[placed], vq[placed], kp[placed], vp[placed], 0, fits)
+    assert np.array_equal(gd.cpu().numpy(), data) and np.array_equal(bits(gp.cpu().numpy()), bits(param))
+
+
 @pytest.mark.parametrize("hadamard", [True, False])
 def test_quantise_and_append_with_infinities_and_nans_equals_the_separate_quantisers(hadamard):
     """A vector that holds an infinity or a NaN: the one-launch quantise-and-append must store what the separate
