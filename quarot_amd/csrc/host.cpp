@@ -3,21 +3,37 @@
 //
 // Every function returns None instead of raising when the arguments are not the plain case it serves (a tensor subclass, a
 // tensor that is not contiguous or not on the current device, a wrong dtype or size, an empty input, a refusal by the
-// library): the Python wrapper then takes its general route, which handles the case or raises the documented error.
+// library, a call under a transform or a tracer): the Python wrapper then takes its general route, which handles the case or
+// raises the documented error.
 // Launches go to torch's current stream, outputs and scratch come from torch's allocator.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
 #include <ATen/ops/empty.h>
 #include <c10/hip/HIPFunctions.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/hip/HIPStream.h>
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include "../../include/quarot_hip.h"
 
 namespace {
 
-const at::Tensor* tensor(PyObject* o) { return THPVariable_CheckExact(o) ? &THPVariable_Unpack(o) : nullptr; }
+// A tensor with memory of its own and nothing that watches what is done to it: no subclass, no wrapper of a function
+// transform (vmap, jvp, functionalisation), no tangent of forward-mode differentiation, no active tracer or dispatch mode.
+const at::Tensor* tensor(PyObject* o) {
+    using c10::DispatchKey;
+    constexpr c10::DispatchKeySet wrapped{DispatchKey::Python, DispatchKey::Functionalize, DispatchKey::FuncTorchBatched,
+                                          DispatchKey::FuncTorchGradWrapper};
+    constexpr c10::DispatchKeySet modes{DispatchKey::Python, DispatchKey::Functionalize, DispatchKey::Tracer,
+                                        DispatchKey::FuncTorchDynamicLayerFrontMode};
+    if (!THPVariable_CheckExact(o)) return nullptr;
+    const at::Tensor* t = &THPVariable_Unpack(o);
+    if (t->key_set().has_any(wrapped) || c10::impl::tls_local_dispatch_key_set().included_.has_any(modes) || t->_fw_grad(0).defined())
+        return nullptr;
+    return t;
+}
 
 bool plain(const at::Tensor* t, at::ScalarType dtype, int device) {
     return t && t->is_cuda() && t->scalar_type() == dtype && t->device().index() == device && t->is_contiguous();
@@ -118,13 +134,8 @@ bool arg_float(PyObject* o, double* v) {
         PyErr_SetString(PyExc_TypeError, "expected " #COUNT " arguments"); \
         return nullptr;                                                    \
     }                                                                      \
-    try {
-#define QR_END                                                             \
-    }                                                                      \
-    catch (const std::exception& e) {                                      \
-        PyErr_SetString(PyExc_RuntimeError, e.what());                     \
-        return nullptr;                                                    \
-    }
+    HANDLE_TH_ERRORS
+#define QR_END END_HANDLE_TH_ERRORS
 
 // quantize_rows(x, clip) -> (codes, scales)
 PyObject* quantize_rows(PyObject*, PyObject* const* a, Py_ssize_t nargs) {

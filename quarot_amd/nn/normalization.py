@@ -6,7 +6,8 @@ import quarot_amd
 class RMSNorm(torch.nn.Module):
     """Weight-less RMS normalisation in fp32 (quarot/nn/normalization.py:3-21); the learned gain
     has been folded into the following linear layer offline.  fp16 rows on the GPU go through one kernel (qr_rmsnorm_f16);
-    other dtypes and devices, strided rows, widths it does not take and inputs that need a gradient through torch."""
+    other dtypes and devices, strided rows, widths it does not take, inputs that need a gradient and calls under a tracer
+    or a function transform through torch."""
 
     def __init__(self, mean_dim: int, eps=1e-5):
         super().__init__()
@@ -15,9 +16,11 @@ class RMSNorm(torch.nn.Module):
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         dt = x.dtype
-        if (dt == torch.float16 and x.is_cuda and x.is_contiguous() and x.shape[-1] % 8 == 0 and 0 < x.shape[-1] <= 32768
-                and x.data_ptr() % 16 == 0 and not (x.requires_grad and torch.is_grad_enabled())):
-            return quarot_amd.rmsnorm(x, self.mean_dim, self.eps)
+        if not torch.jit.is_scripting():
+            if not torch.compiler.is_compiling() and not (x.requires_grad and torch.is_grad_enabled()):
+                y = quarot_amd._host.rmsnorm(x, self.mean_dim, self.eps)
+                if y is not None:
+                    return y
         xf = x.to(torch.float32) if dt == torch.float16 else x
         var = xf.pow(2).sum(-1, keepdim=True) / self.mean_dim
         return (xf * torch.rsqrt(var + self.eps)).to(dt)

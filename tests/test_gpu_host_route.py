@@ -36,7 +36,7 @@ def test_same_results_and_shapes_as_the_general_route(lead, general_route):
         plain = nn.Linear4bit(11008, 320).half()
     lin.weight_scales.uniform_(1e-3, 2e-3), plain.weight_scales.uniform_(1e-3, 2e-3), lin.bias.normal_()
     xh = torch.randn(*lead, 40, 128, device="cuda").half()
-    modules = [nn.Quantizer(0.9), nn.RMSNorm(11008), nn.RMSNormQuantizer(11008, input_clip_ratio=0.95), nn.OnlineHadamard(11008).cuda(),
+    modules = [nn.Quantizer(0.9), lambda y: quarot_amd.rmsnorm(y, 11008), nn.RMSNormQuantizer(11008, input_clip_ratio=0.95), nn.OnlineHadamard(11008).cuda(),
                nn.OnlineHadamard(11008, force_fp32=True).cuda(), nn.OnlineHadamardQuantizer(11008).cuda(),
                nn.OnlineHadamardQuantizer(11008, force_fp32=True).cuda(), nn.HeadsHadamardQuantizer(40).cuda(),
                nn.Linear4bitSequential(nn.Quantizer(), lin), nn.Linear4bitSequential(nn.OnlineHadamard(11008).cuda(), nn.Quantizer(), plain),
@@ -78,3 +78,37 @@ def test_page_tables_in_one_launch(batch, length, page, general_route):
     want = c.get_cache_specs_for_flash_infer(None)
     for name in ("kv_indptr", "kv_indices", "last_page_offset"):
         assert got[name].dtype == torch.int32 and torch.equal(got[name], want[name]), name
+
+
+def test_rmsnorm_under_transforms_tracers_and_forward_mode():
+    """What torch's operations took before there was a kernel, RMSNorm still takes."""
+    import torch.autograd.forward_ad as fwad
+    from torch.fx.experimental.proxy_tensor import make_fx
+    norm = quarot_amd.nn.RMSNorm(64)
+    x, t = torch.randn(2, 5, 3, 64, device="cuda").half().unbind(0)
+    plain = norm(x)
+    want = torch.func.jvp(lambda y: norm(y.float()), (x,), (t,))[1]           # (fp32 rows: always torch)
+    assert torch.equal(torch.func.vmap(norm)(x), norm(x.clone()))
+    near = lambda a: torch.testing.assert_close(a.float(), want, rtol=1e-3, atol=2e-3)      # fp16 results of values up to ~4
+    near(torch.func.jvp(norm, (x,), (t,))[1])
+    with fwad.dual_level():
+        near(fwad.unpack_dual(norm(fwad.make_dual(x, t))).tangent)
+    more = torch.cat([x, x])
+    for traced in (make_fx(norm)(x), torch.jit.trace(norm, x)):
+        torch.testing.assert_close(traced(x * 2), plain, rtol=1e-3, atol=1e-3)
+    assert torch.jit.trace(norm, x)(more).shape == more.shape and torch.jit.script(norm)(x).shape == x.shape
+    leaf = x.clone().requires_grad_()
+    assert norm(leaf).requires_grad and not norm(x).requires_grad
+
+
+def test_out_of_memory_keeps_its_type():
+    n = 1 << 15
+    q, s = torch.zeros(n, 32, dtype=torch.uint8, device="cuda"), torch.ones(n, 1, device="cuda").half()
+    torch.cuda.empty_cache()
+    allowed = torch.cuda.memory_reserved() + 2 ** 30
+    torch.cuda.set_per_process_memory_fraction(allowed / torch.cuda.mem_get_info()[1])
+    try:
+        with pytest.raises(torch.OutOfMemoryError):                           # 2 GiB of output
+            host.linear(q, s, q, s, None)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
