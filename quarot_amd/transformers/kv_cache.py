@@ -394,7 +394,8 @@ class MultiLayerPagedKVCache4Bit:
     def _decode_workspace(self, num_heads):
         """Scratch for decode attention split along the sequence, kept with the cache (every layer of every decode
         step would otherwise allocate its own): sized for the longer of the current and the maximum length.  Zeroed when
-        it is made: every launch leaves its arrival counters at zero."""
+        it is made: every launch leaves its arrival counters at zero.  One made while a graph is captured is zeroed by that
+        graph's replays only, so it is not kept."""
         key = (self.length, num_heads)
         if getattr(self, "_decode_ws_key", None) == key:
             return self._decode_ws
@@ -405,6 +406,8 @@ class MultiLayerPagedKVCache4Bit:
         ws = getattr(self, "_decode_ws", None)
         if need and (ws is None or ws.numel() < need):
             ws = torch.zeros((need,), dtype=torch.uint8, device=dev)
+            if torch.cuda.is_current_stream_capturing():
+                return ws
         self._decode_ws, self._decode_ws_key = ws, key
         return ws
 

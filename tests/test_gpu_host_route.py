@@ -112,3 +112,27 @@ def test_out_of_memory_keeps_its_type():
             host.linear(q, s, q, s, None)
     finally:
         torch.cuda.set_per_process_memory_fraction(1.0)
+
+
+def test_decode_workspace_made_under_capture_is_not_kept():
+    """The arrival counters of such a workspace are zeroed by replays of that graph only: an eager step without a replay
+    makes its own."""
+    g = torch.Generator(device="cuda").manual_seed(3)
+    rnd = lambda n: torch.randn(1, n, 4, 128, generator=g, device="cuda").half()
+    k0, v0, step = rnd(2048), rnd(2048), [rnd(1) for _ in range(3)]
+    caches = [kv.MultiLayerPagedKVCache4Bit(1, 16, 2100, "cuda", 1, 4, 128) for _ in range(2)]
+    for c in caches:
+        c.pages.zero_(), c.scales.zero_()
+        c.update(k0, v0, 0)
+        c._decode_ws = c._decode_ws_key = None
+    run = lambda c: c.update(step[0], step[1], 0)(step[2])
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        captured = run(caches[0])
+    assert caches[0]._decode_ws is None
+    for _ in range(3):
+        graph.replay()
+        caches[1].length = 2048
+        want = run(caches[1])
+        assert torch.equal(captured, want)
+    assert torch.equal(run(caches[0]), run(caches[1])) and caches[0]._decode_ws is not None
