@@ -41,6 +41,20 @@ __device__ __forceinline__ void lane_stage(float (&v)[8], int lane) {
     }
 }
 
+__device__ __forceinline__ u32 as_u32(float v) { return __builtin_bit_cast(u32, v); }
+__device__ __forceinline__ float as_f32(u32 w) { return __builtin_bit_cast(float, w); }
+
+// A butterfly level between the lanes of a row of 16: v + s * (the value of the lane that DPP names), one instruction.  s = -1
+// in the lower lane of a pair and +1 in the upper one, whose values are held negated: (a, -b) -> (a - (-b), -b + a).
+template <int DPP>
+__device__ __forceinline__ void row_stage(float (&v)[8], float s) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        const int i = __builtin_bit_cast(int, v[e]);
+        v[e] = __builtin_fmaf(__builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(i, DPP, 0xF, 0xF, true)), s, v[e]);
+    }
+}
+
 __device__ __forceinline__ void reg_fwht8(float (&v)[8]) {
 #pragma unroll
     for (int h = 1; h < 8; h <<= 1)
@@ -1883,10 +1897,14 @@ int launch_hadamard_mm(const void* x, void* y, int64_t rows, int n, int K, const
 // The hadK factor then runs on the matrix cores as in hadamard_mm_kernel (T^T as first operand, hadK
 // fragments in registers, 8-byte result writes).  All of a row's loads are issued at once and the next
 // row's are requested before the matrix stage.
-// fp32-precision mode (MODE32, m = 1024; bound by vector and matrix instruction issue like the fp16 form, 38 us at 2048 rows,
-// plus the lo planes: 49 us at 1777 rows): the scaled U is kept as two fp16 planes, hi = fp16(U) and lo = fp16(U - hi), in
-// two copies of the fragment array (2 x 68 KB of LDS; the fp16 result row has no place there, so the results leave from
-// registers in every variant of this mode), and each product of the hadK stage is a hi and a lo matrix instruction.
+// fp32-precision mode (MODE32, m = 1024): the same bits as the general kernel above gives.  A row's scale is the rounding of
+// ONE value, its largest: a transform whose sums merely are as accurate rounds it the other way in one row of ten thousand,
+// and then every code of that row moves.  So phase 1 is the general kernel's butterflies, index bits 0 .. 9 in turn in
+// fp32, organised so that a level costs one instruction per value (FWHT below) instead of two and a trip through LDS; the scaled U
+// is kept as its two fp16 planes, hi = fp16(U) and lo = fp16(U - hi), in two copies of the fragment array (2 x 68 KB of LDS;
+// the fp16 result row has no place there, so the results leave from registers in every variant of this mode), and each
+// product of the hadK stage is a hi and a lo matrix instruction into one accumulator, in that order.  Bound by vector
+// instruction issue: 1777 x 28672 393 us in the general kernel, 58 us here.
 template <bool QUANT, int CPL, bool MODE32>
 __global__ __launch_bounds__(1024) void hadamard_bm_kernel(const f16* __restrict__ x, f16* __restrict__ y, int64_t rows,
                                                            int n, int K, const void* __restrict__ hadK, float scale,
@@ -1915,6 +1933,8 @@ __global__ __launch_bounds__(1024) void hadamard_bm_kernel(const f16* __restrict
     // both stages
     constexpr int XL = CPL == 2 ? 4 : SPW * CPL;
     const bool works = CPL == 2 && wave * 2 < K;
+    // MODE32: the chunk (of 64) of a lane, see the butterflies: lanes L and L ^ 1, ^ 2, ^ 7, ^ 8 hold chunks that differ in bit 0, 1, 2, 3
+    const int chunk = MODE32 ? lane ^ ((lane >> 2 & 1) * 3) : l16 * 4 + g;
     u32x4 raw[XL];
     auto request = [&](int64_t row) {
         if (CPL == 2) {
@@ -1922,7 +1942,7 @@ __global__ __launch_bounds__(1024) void hadamard_bm_kernel(const f16* __restrict
             for (int sg = 0; sg < 2; ++sg)          // (waves beyond the last pair repeat wave 0's loads and drop them: no branch)
 #pragma unroll
                 for (int bt = 0; bt < 2; ++bt)
-                    raw[sg * 2 + bt] = *((const u32x4*)(x + row * (int64_t)n) + ((works ? wave : 0) * 2 + sg) * 128 + bt * 64 + l16 * 4 + g);
+                    raw[sg * 2 + bt] = *((const u32x4*)(x + row * (int64_t)n) + ((works ? wave : 0) * 2 + sg) * 128 + bt * 64 + chunk);
             return;
         }
 #pragma unroll
@@ -1936,18 +1956,12 @@ __global__ __launch_bounds__(1024) void hadamard_bm_kernel(const f16* __restrict
     };
     int64_t row = blockIdx.x;
     if (row < rows) request(row);           // in flight while the fragments are made and T is cleared
-    // MODE32: the first 32 sums carry a factor 1 / 32 (a power of two: no rounding), so that T never leaves the fp16 range
-    // where x does not, and both lo planes (T's and U's) are stored 2048 times as large (hb's copy for T carries
-    // 1 / 2048, U's sums take it when they are added) so that lo keeps its eleven bits for small activations too (without the factor it would be subnormal
-    // below 0.25)
-    constexpr float SA = MODE32 ? 0.03125f : 1.0f;
-    const float uscale = MODE32 ? scale * 32.0f : scale;
     f16x8 ha[2], hb[2];
-    if (CPL == 2) {
+    if (CPL == 2 && !MODE32) {
 #pragma unroll
         for (int t = 0; t < 8; ++t) {
 #pragma unroll
-            for (int cth = 0; cth < 2; ++cth) ha[cth][t] = (__builtin_popcount((g * 8 + t) & (cth * 16 + l16)) & 1) ? (f16)-SA : (f16)SA;
+            for (int cth = 0; cth < 2; ++cth) ha[cth][t] = (__builtin_popcount((g * 8 + t) & (cth * 16 + l16)) & 1) ? (f16)-1.0f : (f16)1.0f;
             const int b = 16 * (t >> 2) + 4 * g + (t & 3);
 #pragma unroll
             for (int bt = 0; bt < 2; ++bt) hb[bt][t] = (__builtin_popcount(b & (bt * 16 + l16)) & 1) ? (f16)-1.0f : (f16)1.0f;
@@ -1980,11 +1994,71 @@ __global__ __launch_bounds__(1024) void hadamard_bm_kernel(const f16* __restrict
     __syncthreads();
     for (; row < rows; row += gridDim.x) {
         // ---- phase 1: the power-of-two factor of every segment, results in fragment order in LDS
-        if (CPL == 2) {
+        if constexpr (MODE32) {
+            // Index bits 0 .. 2 lie in a lane's chunk, bits 3 .. 6 on the lanes of a row of 16, bits 7 and 8 on its rows, bit 9
+            // is the lane's second chunk.  Bits 3 .. 6: the partner is fetched by the addition itself (DPP), which adds s times
+            // the partner: v + s p with s = -1 below and +1 above is the butterfly when the values above are held negated, and
+            // the sign for all four levels is applied to the fp16 pairs at the start (negation passes through the other
+            // levels).  DPP has no exchange of lanes L and L ^ 4, but the mirror image of eight lanes is L ^ 7: hence the chunk
+            // numbers.  Bits 7 and 8: two registers trade the halves that the other needs, after which the register's number
+            // is the bit's and the lane's row that of the register, so bits 0 and 1 end on the rows of lanes.
+            if (works) {
+                const u32 flip = (__builtin_popcount(chunk & 15) & 1) ? 0x80008000u : 0u;
+                float v[2][2][8];
+#pragma unroll
+                for (int sg = 0; sg < 2; ++sg) {
+#pragma unroll
+                    for (int bt = 0; bt < 2; ++bt) {
+#pragma unroll
+                        for (int w = 0; w < 4; ++w) {
+                            const f16x2 pair = as_f16x2(raw[sg * 2 + bt][w] ^ flip);
+                            v[sg][bt][2 * w] = (float)pair[0], v[sg][bt][2 * w + 1] = (float)pair[1];
+                        }
+                        reg_fwht8(v[sg][bt]);
+                        row_stage<0xB1>(v[sg][bt], (chunk & 1) ? 1.0f : -1.0f);         // quad_perm [1, 0, 3, 2]: L ^ 1
+                        row_stage<0x4E>(v[sg][bt], (chunk & 2) ? 1.0f : -1.0f);         // quad_perm [2, 3, 0, 1]: L ^ 2
+                        row_stage<0x141>(v[sg][bt], (chunk & 4) ? 1.0f : -1.0f);        // row_half_mirror: L ^ 7
+                        row_stage<0x128>(v[sg][bt], (chunk & 8) ? 1.0f : -1.0f);        // row_ror:8: L ^ 8
+#pragma unroll
+                        for (int e = 0; e < 8; e += 2) {                                // bit 7, against bit 0
+                            const auto t = __builtin_amdgcn_permlane16_swap(as_u32(v[sg][bt][e]), as_u32(v[sg][bt][e + 1]), false, false);
+                            v[sg][bt][e] = as_f32(t[0]) + as_f32(t[1]), v[sg][bt][e + 1] = as_f32(t[0]) - as_f32(t[1]);
+                        }
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {                                   // bit 8, against bit 1
+                            const int e = (i >> 1) * 4 + (i & 1);
+                            const auto t = __builtin_amdgcn_permlane32_swap(as_u32(v[sg][bt][e]), as_u32(v[sg][bt][e + 2]), false, false);
+                            v[sg][bt][e] = as_f32(t[0]) + as_f32(t[1]), v[sg][bt][e + 2] = as_f32(t[0]) - as_f32(t[1]);
+                        }
+                    }
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) {                                       // bit 9
+                        const float a = v[sg][0][e], b = v[sg][1][e];
+                        v[sg][0][e] = a + b, v[sg][1][e] = a - b;
+                    }
+                }
+                // register (bt, e) of a lane = position 512 bt + 256 e1 + 128 e0 + 8 (chunk % 16) + 4 e2 + (row of lanes, bits
+                // 0 and 1); the pair's two k are one 32-bit word of that position's fragment (k-group wave / 4): a write
+                // instruction's 64 words fall on the sixteen banks of this wave's word evenly
+                const int pos = (chunk & 15) * 8 + (lane >> 4);
+                u32* const dst = (u32*)(Tl + ((wave >> 2) * CT + (pos >> 4)) * TS + (pos & 15)) + (wave & 3);
+#pragma unroll
+                for (int bt = 0; bt < 2; ++bt)
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) {
+                        const float u0 = v[0][bt][e] * scale, u1 = v[1][bt][e] * scale;
+                        const u32 hi = narrow_f16x2(u0, u1);
+                        const f16x2 h = as_f16x2(hi);
+                        const int at = ((32 * bt + 16 * (e >> 1 & 1) + 8 * (e & 1)) * TS + 4 * (e >> 2)) * 4;
+                        dst[at] = hi;
+                        dst[at + TN * 4] = narrow_f16x2(u0 - (float)h[0], u1 - (float)h[1]);
+                    }
+            }
+        } else if (CPL == 2) {
             if (works) {
 #pragma unroll
                 for (int cth = 0; cth < 2; ++cth) {
-                    u32 o[2][2][2], ol[2][2][2];         // [segment of the pair][b' tile][pair of e]: fp16 pairs (hi, lo)
+                    u32 o[2][2][2];                      // [segment of the pair][b' tile][pair of e]: fp16 pairs
 #pragma unroll
                     for (int sg = 0; sg < 2; ++sg) {
                         // T = hi + lo, both fp16, as packed pairs (the difference is exact in fp32, so one rounding each)
@@ -1997,9 +2071,7 @@ __global__ __launch_bounds__(1024) void hadamard_bm_kernel(const f16* __restrict
 #pragma unroll
                             for (int pr = 0; pr < 2; ++pr) {
                                 const f16x2 hi = __builtin_convertvector(f32x2_t{da[2 * pr], da[2 * pr + 1]}, f16x2);
-                                f32x2_t rest = {da[2 * pr] - (float)hi[0], da[2 * pr + 1] - (float)hi[1]};
-                                if (MODE32) rest = f32x2_t{rest[0] * 2048.0f, rest[1] * 2048.0f};
-                                const f16x2 lo = __builtin_convertvector(rest, f16x2);
+                                const f16x2 lo = __builtin_convertvector(f32x2_t{da[2 * pr] - (float)hi[0], da[2 * pr + 1] - (float)hi[1]}, f16x2);
                                 whi[bt * 2 + pr] = __builtin_bit_cast(u32, hi);
                                 wlo[bt * 2 + pr] = __builtin_bit_cast(u32, lo);
                             }
@@ -2008,18 +2080,9 @@ __global__ __launch_bounds__(1024) void hadamard_bm_kernel(const f16* __restrict
 #pragma unroll
                         for (int bt = 0; bt < 2; ++bt) {
                             f32x4 db = __builtin_amdgcn_mfma_f32_16x16x32_f16(hb[bt], thi, f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-                            f16x8 hl = hb[bt];
-                            if (MODE32) hl = hl * (f16)(1.0f / 2048.0f);
-                            db = __builtin_amdgcn_mfma_f32_16x16x32_f16(hl, tlo, db, 0, 0, 0);
-#pragma unroll
-                            for (int pr = 0; pr < 2; ++pr) {
-                                const float u0 = db[2 * pr] * uscale, u1 = db[2 * pr + 1] * uscale;
-                                o[sg][bt][pr] = narrow_f16x2(u0, u1);
-                                if (MODE32) {
-                                    const f16x2 h = as_f16x2(o[sg][bt][pr]);
-                                    ol[sg][bt][pr] = narrow_f16x2((u0 - (float)h[0]) * 2048.0f, (u1 - (float)h[1]) * 2048.0f);
-                                }
-                            }
+                            db = __builtin_amdgcn_mfma_f32_16x16x32_f16(hb[bt], tlo, db, 0, 0, 0);
+                            o[sg][bt][0] = narrow_f16x2(db[0] * scale, db[1] * scale);
+                            o[sg][bt][1] = narrow_f16x2(db[2] * scale, db[3] * scale);
                         }
                     }
                     // position (b' = 16 bt + 4 g + e, c' = 16 cth + l16) = column tile 2 b' + cth, column l16; the pair's
@@ -2031,8 +2094,6 @@ __global__ __launch_bounds__(1024) void hadamard_bm_kernel(const f16* __restrict
                         for (int e = 0; e < 4; ++e) {
                             const u32 sel = (e & 1) ? 0x07060302u : 0x05040100u;      // high or low halves of two dwords
                             dst[(2 * (16 * bt + 4 * g + e)) * TS * 4] = __builtin_amdgcn_perm(o[1][bt][e >> 1], o[0][bt][e >> 1], sel);
-                            if (MODE32)
-                                dst[(2 * (16 * bt + 4 * g + e)) * TS * 4 + TN * 4] = __builtin_amdgcn_perm(ol[1][bt][e >> 1], ol[0][bt][e >> 1], sel);
                         }
                 }
             }
@@ -2096,11 +2157,7 @@ __global__ __launch_bounds__(1024) void hadamard_bm_kernel(const f16* __restrict
 #pragma unroll
                     for (int rt = 0; rt < RT; ++rt) {
                         f32x4 acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(th4[c], hf[rt][0], f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-                        if (MODE32) {
-                            const f32x4 al = __builtin_amdgcn_mfma_f32_16x16x32_f16(tl4[MODE32 ? c : 0], hf[rt][0], f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-#pragma unroll
-                            for (int e = 0; e < 4; ++e) acc[e] = __builtin_fmaf(al[e], 1.0f / 2048.0f, acc[e]);
-                        }
+                        if (MODE32) acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(tl4[MODE32 ? c : 0], hf[rt][0], acc, 0, 0, 0);
                         if (c == 0 && rt == 0) probe = acc[0];
                         yv[rt][c][0] = cvt_f16x2(acc[0], acc[1]);
                         yv[rt][c][1] = cvt_f16x2(acc[2], acc[3]);
@@ -2512,7 +2569,7 @@ extern "C" int qr_hadamard(const void* x, void* y, int64_t rows, int n, int K, c
     if (dtype == (QR_DTYPE_F16 | QR_HAD_FP32)) {
         // fp16 rows through fp32-precision arithmetic (a program with force_fp32 that keeps its modules apart): one pass of
         // 4 bytes per value instead of the 20 of a conversion, the fp32 transform and a conversion back -- 1178 x 13824
-        // 129 -> 39 us, 2048 x 5120 65 -> 17, 122 x 28672 69 -> 11, 1777 x 28672 455 -> 51.  Rows of 128 and shorter keep those three steps.
+        // 129 -> 39 us, 2048 x 5120 65 -> 17, 122 x 28672 69 -> 11, 1777 x 28672 455 -> 60.  Rows of 128 and shorter keep those three steps.
         if (n <= 128) return QR_E_UNSUPPORTED;
         if (K == 1 && pow2_split(n))
             return launch_hadamard_mm<true, false>(x, y, rows, n, pow2_split(n), nullptr, scale, 1.f, nullptr, nullptr, st);
@@ -2582,7 +2639,7 @@ extern "C" int qr_hadamard_quantize_f16_i4(const void* x, int64_t rows, int n, i
         return launch_hadamard_bm<true>(x, y_or_null, rows, n, K, hadK, scale, clip, q, scales, st);
     // fp32 precision behind a 1024-point factor: the matrix-core kernel with hi / lo planes at every row count (the general
     // kernel's fp32 row fills a CU's LDS and it forms the hadK fragments from scalar LDS reads: 1777 x 28672 393 us against
-    // 49 us here = 2.6 TB/s, 4096 rows 934 against 99, 1 and 64 rows 56 against 14)
+    // 58 us here = 2.2 TB/s)
     if (mode == QR_DTYPE_F32 && bm_applies(n, K) && n / K == 1024)
         return launch_hadamard_bm<true, true>(x, y_or_null, rows, n, K, hadK, scale, clip, q, scales, st);
     if (mm_applies(n, K)) {
