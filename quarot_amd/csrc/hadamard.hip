@@ -508,8 +508,7 @@ bool km_applies(int n, int K, bool mode32) {
 template <bool MODE32, bool QUANT, int LOG2M, int KS2, bool XLDS>
 __global__ __launch_bounds__(HT) void hadamard_mm_kernel(const f16* __restrict__ x, f16* __restrict__ y, int64_t rows,
                                                          int n, int K, const void* __restrict__ hadK, float scale,
-                                                         float clip, u32* __restrict__ q, f16* __restrict__ scales,
-                                                         int ident) {
+                                                         float clip, u32* __restrict__ q, f16* __restrict__ scales) {
     constexpr int M_ = 1 << LOG2M;
     constexpr int KS1 = M_ / 32;                 // contraction steps of stage 1
     constexpr int CT = M_ / 16;                  // 16-column tiles of T / Y
@@ -588,11 +587,7 @@ __global__ __launch_bounds__(HT) void hadamard_mm_kernel(const f16* __restrict__
                 for (int e = 0; e < 4; ++e) hf[t][ks][hh * 4 + e] = v[e];
             }
     }
-    // Sylvester fragments: H_m[r][r'] = (-1)^popcount(r & r').  With `ident` the inner factor is the
-    // identity instead, y = x . (hadK (x) I_m)^T * scale: the transform ACROSS m-wide groups, which is what
-    // OnlineHadamard(num_heads) on the transposed attention output computes (e2e/quantized_llama/
-    // modeling_llama.py:108-110), with the same staging as the reference (x * scale rounded to fp16, then
-    // hadK @ .: quarot/functional/hadamard.py:94-101 with n / K = 1).
+    // Sylvester fragments: H_m[r][r'] = (-1)^popcount(r & r')
     f16x8 b1[NCT][KS1];
 #pragma unroll
     for (int c = 0; c < NCT; ++c)
@@ -602,8 +597,7 @@ __global__ __launch_bounds__(HT) void hadamard_mm_kernel(const f16* __restrict__
             for (int j = 0; j < 8; ++j) {
                 const int rp = (wave + 4 * c) * 16 + l16;
                 const int r = ks * 32 + g * 8 + j;
-                const f16 sylv = (__builtin_popcount(r & rp) & 1) ? (f16)-1.0f : (f16)1.0f;
-                b1[c][ks][j] = ident ? (r == rp ? (f16)1.0f : (f16)0.0f) : sylv;
+                b1[c][ks][j] = (__builtin_popcount(r & rp) & 1) ? (f16)-1.0f : (f16)1.0f;
             }
 
     // stage-1 A-fragments for the tile pair s2 of a row: [2 tiles][KS1] 16-byte loads
@@ -1758,10 +1752,10 @@ bool mm_applies(int n, int K) {
 
 template <bool MODE32, bool QUANT>
 int launch_hadamard_mm(const void* x, void* y, int64_t rows, int n, int K, const void* hadK, float scale, float clip,
-                       void* q, void* scales, hipStream_t st, int ident = 0, int signs = 0) {
+                       void* q, void* scales, hipStream_t st, int signs = 0) {
     const int m = n / K;
     const int KS2 = ((K + 31) & ~31) >> 5;
-    if (m == 128 && KS2 >= 2 && KS2 != 3 && !ident && !MODE32 && QUANT && y == nullptr && hadK != nullptr && ((uintptr_t)x & 15) == 0) {
+    if (m == 128 && KS2 >= 2 && KS2 != 3 && !MODE32 && QUANT && y == nullptr && hadK != nullptr && ((uintptr_t)x & 15) == 0) {
         // m = 128 behind one of the reference's tables of order 36 and more (Llama-2-13B: 5120 = 40 x 128, 13824 =
         // 108 x 128): the lean fused kernel with eight column tiles.  Orders 140 .. 172 need more registers than two
         // workgroups per CU leave a wave (231 .. 260 spilled) and run one workgroup per CU.
@@ -1783,7 +1777,7 @@ int launch_hadamard_mm(const void* x, void* y, int64_t rows, int n, int K, const
 #undef QR_M128Q
         return qr_launch_status();
     }
-    if (m == 64 && K >= 64 && !ident) {
+    if (m == 64 && K >= 64) {
         // the latency-organised kernel (it relies on every wave's first tile lying inside hadK), while
         // two workgroups still fit on a CU
         const int tpw = (2 * KS2 + 3) / 4;
@@ -1857,7 +1851,7 @@ int launch_hadamard_mm(const void* x, void* y, int64_t rows, int n, int K, const
         const int64_t cap = (int64_t)qr_device().cus * qr_blocks_per_cu((const void*)kern, HT, lds);                                      \
         const unsigned grid = (unsigned)(rows < cap ? rows : cap);                                                     \
         kern<<<dim3(grid), dim3(HT), lds, st>>>((const f16*)x, (f16*)y, rows, n, K, hadK, scale, clip, (u32*)q,        \
-                                                (f16*)scales, ident);                                                  \
+                                                (f16*)scales);                                                         \
     } while (0)
 #define QR_MM_X(L2M, KS)                 \
     if (xlds) QR_MM(L2M, KS, true);      \
@@ -2619,8 +2613,8 @@ extern "C" int qr_hadamard_quantize_f16_i4(const void* x, int64_t rows, int n, i
         // hadK as sign words: the lean kernel of the m = 64 widths behind a table of order 97 .. 192 only (nothing is
         // launched otherwise: the caller passes the table itself)
         if (K <= 96 || y_or_null || !mm_applies(n, K) || n / K != 64 || ((uintptr_t)hadK & 3)) return QR_E_UNSUPPORTED;
-        if (mode == QR_DTYPE_F16) return launch_hadamard_mm<false, true>(x, nullptr, rows, n, K, hadK, scale, clip, q, scales, st, 0, 1);
-        return launch_hadamard_mm<true, true>(x, nullptr, rows, n, K, hadK, scale, clip, q, scales, st, 0, 1);
+        if (mode == QR_DTYPE_F16) return launch_hadamard_mm<false, true>(x, nullptr, rows, n, K, hadK, scale, clip, q, scales, st, 1);
+        return launch_hadamard_mm<true, true>(x, nullptr, rows, n, K, hadK, scale, clip, q, scales, st, 1);
     }
     if (tiny_applies(n, K)) return QR_E_UNSUPPORTED;       // rows this short: qr_hadamard, then qr_quantize_rows_f16_i4
     if (mode == QR_DTYPE_F16 && K == 1 && n == 128) {
@@ -2657,13 +2651,180 @@ extern "C" int qr_hadamard_quantize_f16_i4(const void* x, int64_t rows, int n, i
     return QR_E_DTYPE;
 }
 
-// quant.hip: Hadamard across `heads` groups of 128 + quantiser for head counts that are orders of the
-// reference's tables: the fused two-stage kernel with the identity as inner factor
+namespace {
+
+// ---- Hadamard across H heads of 128 values for a table's order H = K <= 60, + quantiser ----------
+// OnlineHadamard(num_heads) on the transposed attention output, transpose back, Quantizer
+// (e2e/quantized_llama/modeling_llama.py:108-110): T = fp16(x * scale), Y = hadK . T over the head index for each of the 128
+// positions (quarot/functional/hadamard.py:94-101 with n / K = 1), rounded to fp16, quantised along the token.
+// One WAVE per token, no LDS and no barrier.  The contraction runs over the heads, 256 bytes apart in memory, and a matrix
+// fragment wants eight of them for one position: a lane loads 16-byte chunks (positions 8 l16 .. + 7) of the heads of its
+// group, and the conversion that packs two scaled values into a dword takes them from two heads instead of from two
+// positions, so the transposition costs nothing.  With hadK as first operand a lane's results are, for RT x 4 heads, the
+// SAME eight positions 8 l16 .. + 7: one dword of codes (or 16 bytes of y) per head without an exchange, and hadK's rows are
+// dealt to the operand so that the four groups of lanes hold neighbouring heads: 256 bytes of codes per store.
+// 8191 x 40 heads 44.1 us (the two-stage kernel with the identity as inner factor, which this one replaces) -> 19.4 =
+// 5.4 TB/s, 2048 x 40 14.7 -> 6.4, 333 x 40 7.3 -> 4.2, 333 x 52 7.6 -> 5.1, one token 6.1 -> 3.5; same bits.
+template <int RT>
+__global__ __launch_bounds__(HT, (RT == 1 ? 4 : RT == 2 ? 4 : RT == 3 ? 3 : 2)) void heads_matrix_quant_kernel(const f16* __restrict__ x, f16* __restrict__ y, int64_t rows, int K,
+                                                                const f16* __restrict__ hadK, float scale, float clip,
+                                                                u32* __restrict__ q, f16* __restrict__ scales) {
+    constexpr int KS2 = (RT + 1) / 2;                   // contraction steps of 32 heads, each two halves of 16
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int l16 = lane & 15, g = lane >> 4;
+    const int64_t step = (int64_t)gridDim.x * (HT / QR_WAVE);
+    int64_t row = (int64_t)blockIdx.x * (HT / QR_WAVE) + wave;
+    if (row >= rows) return;                            // a whole wave: nothing below synchronises waves
+    // chunk (h, i): head 16 h + 4 g + i, positions 8 l16 .. + 7; heads beyond K lie outside the token's buffer: loads give 0,
+    // stores are dropped, so neither needs a branch
+    auto token = [&](const void* base, int64_t r, int bytes) {
+        return __builtin_amdgcn_make_buffer_rsrc((void*)((const char*)base + r * (int64_t)(K * bytes)), 0, K * bytes, 0x00020000);
+    };
+    u32x4 raw[RT][4];
+    auto request = [&](int64_t r) {
+        const __amdgpu_buffer_rsrc_t src = token(x, r, 256);
+        int l = g * 1024 + l16 * 16;
+        asm volatile("" : "+v"(l));                     // (here and below: opaque, so that the constants stay in the instructions'
+#pragma unroll                                          // offset fields; hoisted out of the loop they would be a register each)
+        for (int h = 0; h < RT; ++h)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) raw[h][i] = __builtin_amdgcn_raw_buffer_load_b128(src, l + h * 4096 + i * 256, 0, 0);
+    };
+    request(row);
+    // hadK: row l16 of tile rt is head kout(rt, l16), contraction index 32 ks + 16 (j / 4) + 4 g + j % 4 (K is a multiple of 4)
+    f16x8 hf[RT][KS2];
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+        for (int ks = 0; ks < KS2; ++ks)
+#pragma unroll
+            for (int hh = 0; hh < 2; ++hh) {
+                const int hr = rt * 16 + (l16 & 3) * 4 + (l16 >> 2), hc = ks * 32 + hh * 16 + g * 4;
+                f16x4 v = {(f16)0, (f16)0, (f16)0, (f16)0};
+                if (hr < K && hc < K) v = *(const f16x4*)(hadK + hr * K + hc);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) hf[rt][ks][hh * 4 + e] = v[e];
+            }
+    float zero = -0.0f;
+    asm volatile("" : "+v"(zero));                      // opaque, or the compiler splits the fma (exact with -0) into convert + multiply
+    for (; row < rows; row += step) {
+        // result (rt, e) of a lane: head 16 rt + 4 e + g, positions 8 l16 + 2 w, + 1 in word w
+        u32 yv[RT][4][4];
+        float mxf = 0.f, probe = 0.f;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+            u32x4 th[2][KS2];                           // [position 2 w, 2 w + 1][step]
+#pragma unroll
+            for (int h = 0; h < 2 * KS2; ++h)
+#pragma unroll
+                for (int p = 0; p < 2; ++p)
+#pragma unroll
+                    for (int i = 0; i < 4; i += 2) {
+                        u32 packed = 0;
+                        if (h < RT) {
+                            const float a = __builtin_fmaf((float)as_f16x2(raw[h < RT ? h : 0][i][w])[p], scale, zero);
+                            const float b = __builtin_fmaf((float)as_f16x2(raw[h < RT ? h : 0][i + 1][w])[p], scale, zero);
+                            packed = narrow_f16x2(a, b);
+                        }
+                        th[p][h >> 1][2 * (h & 1) + (i >> 1)] = packed;
+                    }
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt) {
+                f32x4 acc[2];
+#pragma unroll
+                for (int p = 0; p < 2; ++p) {
+                    acc[p] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                    for (int ks = 0; ks < KS2; ++ks)
+                        acc[p] = __builtin_amdgcn_mfma_f32_16x16x32_f16(hf[rt][ks], __builtin_bit_cast(f16x8, th[p][ks]), acc[p], 0, 0, 0);
+                }
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    yv[rt][e][w] = cvt_f16x2(acc[0][e], acc[1][e]);
+                    // (heads beyond K are zero rows of the operand: their results are 0, or NaN from 0 . inf, which the
+                    // maximum instruction drops)
+                    mxf = __builtin_fmaxf(__builtin_fmaxf(mxf, __builtin_fabsf(acc[0][e])), __builtin_fabsf(acc[1][e]));
+                }
+                // an infinity or NaN at a position reaches every head of that position: one result per position tells
+                if (rt == 0) probe += (acc[0][0] - acc[0][0]) + (acc[1][0] - acc[1][0]);
+            }
+            __builtin_amdgcn_sched_barrier(0);          // (word by word: all four at once would need twice the registers)
+        }
+        const int64_t at = row;
+        u32 mx = f16_bits((f16)mxf);                    // (rounding is monotone: the largest of the rounded values)
+        if (__builtin_amdgcn_ballot_w64(mx >= 0x7c00u || probe != probe) != 0) {
+            u16x2 m2 = {0, 0};                          // the exact form: packed maxima of the magnitudes, NaN wins
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+#pragma unroll
+                    for (int w = 0; w < 4; ++w)
+                        m2 = __builtin_elementwise_max(
+                            m2, __builtin_bit_cast(u16x2, 16 * rt + 4 * e + g < K ? yv[rt][e][w] & 0x7fff7fffu : 0u));
+            mx = m2[0] > m2[1] ? m2[0] : m2[1];
+        }
+        mx = wave_max_u32_dpp(mx);
+        const f16 sh = quantizer_scale(f16_from_bits((unsigned short)mx), clip);
+        if (lane == 0) scales[at] = sh;
+        const float s = (float)sh;
+        const __amdgpu_buffer_rsrc_t qrow = token(q, at, 64);
+        int lane4 = lane * 4;
+        asm volatile("" : "+v"(lane4));
+        auto codes_from = [&](auto form) {
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const u32 codes = form(u32x4{yv[rt][e][0], yv[rt][e][1], yv[rt][e][2], yv[rt][e][3]});
+                    __builtin_amdgcn_raw_buffer_store_b32(codes, qrow, lane4 + rt * 1024 + e * 256, 0, 0);
+                    if (e & 1) __builtin_amdgcn_sched_barrier(0);
+                }
+        };
+        if (fast_quant_ok(mx, s)) {
+            const FastRecip fq = make_fast_recip(s);
+            if (clamp_cannot_act(clip, s)) codes_from([&](u32x4 h) { return sym_codes8_fast<false>(h, fq); });
+            else codes_from([&](u32x4 h) { return sym_codes8_fast<true>(h, fq); });
+        } else {
+            const bool fast = scale_fast_ok(s);
+            const float rs = fast ? 1.0f / s : 0.0f;
+            codes_from([&](u32x4 h) { return sym_codes8(h, s, rs, fast); });
+        }
+        // (not earlier: requested before the codes are formed they cost a wave per SIMD: 8191 x 40 heads 21.3 against 19.4 us)
+        if (row + step < rows) request(row + step);
+        if (y) {
+            const __amdgpu_buffer_rsrc_t yrow = token(y, at, 256);
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    __builtin_amdgcn_raw_buffer_store_b128(u32x4{yv[rt][e][0], yv[rt][e][1], yv[rt][e][2], yv[rt][e][3]}, yrow,
+                                                           lane4 * 4 + rt * 4096 + e * 1024, 0, 0);
+        }
+    }
+}
+
+}  // namespace
+
+// quant.hip: Hadamard across `heads` groups of 128 + quantiser for head counts that are orders of the reference's tables
+// (multiples of 4 up to 60)
 __attribute__((visibility("hidden"))) int qr_internal_heads_matrix_quantize(const void* x, int64_t rows, int heads,
                                                                             const void* hadK, float clip, void* q,
                                                                             void* scales, void* y_or_null, hipStream_t st) {
-    const int n = heads * 128;
-    if (!mm_applies(n, heads)) return QR_E_UNSUPPORTED;
-    return launch_hadamard_mm<false, true>(x, y_or_null, rows, n, heads, hadK, 1.0f / __builtin_sqrtf((float)heads), clip, q,
-                                           scales, st, 1);
+    if (heads < 4 || heads > 64 || heads % 4 != 0) return QR_E_UNSUPPORTED;
+#define QR_HEADS(RT)                                                                                                   \
+    do {                                                                                                               \
+        auto kern = heads_matrix_quant_kernel<RT>;                                                                     \
+        const int64_t cap = (int64_t)qr_device().cus * qr_blocks_per_cu((const void*)kern, HT, 0);                     \
+        const int64_t blocks = (rows + HT / QR_WAVE - 1) / (HT / QR_WAVE);                                             \
+        kern<<<dim3((unsigned)(blocks < cap ? blocks : cap)), dim3(HT), 0, st>>>(                                      \
+            (const f16*)x, (f16*)y_or_null, rows, heads, (const f16*)hadK, 1.0f / __builtin_sqrtf((float)heads), clip, \
+            (u32*)q, (f16*)scales);                                                                                    \
+    } while (0)
+    if (heads <= 16) QR_HEADS(1);
+    else if (heads <= 32) QR_HEADS(2);
+    else if (heads <= 48) QR_HEADS(3);
+    else QR_HEADS(4);
+#undef QR_HEADS
+    return qr_launch_status();
 }

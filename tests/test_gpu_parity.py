@@ -1030,6 +1030,29 @@ def test_fused_heads_hadamard_quantize(heads, rows, clip):
     assert float((p.quantized_x == staged.quantized_x).float().mean()) > 0.99
 
 
+@pytest.mark.parametrize("heads", [12, 20, 28, 36, 40, 52, 60])
+@pytest.mark.parametrize("rows,clip", [(1, 1.0), (4, 0.9), (5, 1.0), (3089, 1.0)])
+def test_fused_heads_hadamard_quantize_behind_a_table(heads, rows, clip):
+    """Every order of the tables up to 60 (one to four tiles of sixteen heads, whole and partial), token counts below, at and
+    above a workgroup's four and above one round of the grid, against float64: T = fp16(x * scale), hadK . T, rounded to fp16
+    once; the fp32 sums of at most 60 products stay within 60 * 2^-24 of the sum of magnitudes.  Codes and scales are
+    the Quantizer's on the returned rows, bit for bit, with and without the copy of the rows."""
+    x = gpu(synth_x(rows, heads * 128, seed=heads + rows)).view(rows, heads, 128)
+    mod = quarot_amd.nn.HeadsHadamardQuantizer(heads, input_clip_ratio=clip).cuda()
+    assert mod.had.rem_dim == heads
+    p = mod(x)
+    p2, y = quarot_amd.heads_hadamard_quantize(x, heads, clip, return_transformed=True, hadK=mod.had.had_rem_dim)
+    pq = quarot_amd.nn.Quantizer(clip)(y.reshape(rows, heads * 128))
+    for got in (p, p2):
+        assert torch.equal(got.quantized_x.reshape(rows, -1), pq.quantized_x.reshape(rows, -1))
+        assert torch.equal(got.scales_x.reshape(-1).view(torch.int16), pq.scales_x.reshape(-1).view(torch.int16))
+    t = (x.float() * (1.0 / np.sqrt(np.float32(heads)))).half().cpu().double()
+    h = mod.had.had_rem_dim.cpu().double()
+    ref = torch.matmul(h, t)
+    slack = 2.0 ** -11 * ref.abs() + 60 * 2.0 ** -24 * torch.matmul(h.abs(), t.abs()) + 2.0 ** -24
+    assert bool(((y.cpu().double().view(rows, heads, 128) - ref).abs() <= slack).all())
+
+
 @pytest.mark.parametrize("heads", [32, 64, 40])
 def test_fused_heads_hadamard_quantize_infinite_nan_zero_huge_and_tiny_rows(heads):
     """Rows holding an infinity, a NaN, only zeros, a value near the fp16 maximum, and values near the
