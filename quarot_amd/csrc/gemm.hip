@@ -309,11 +309,25 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void gemm_i4_kernel(
 //   gemm_spk_kernel    128x256 tile (one per CU at M = 2048, N = 4096), waves 2 (N) x 2 (K): the two
 //                      K-groups take alternate pairs of sub-steps and exchange half of their
 //                      accumulators through LDS at the end.
-template <bool DEQ, bool RAGGED, int BM = 256>
-__global__ __launch_bounds__(256) void gemm_sp256_kernel(
+// Row and column of tile `unit` of a grid of tiles: columns of eight row tiles in turn, so that tiles in flight together
+// share rows of both operands in an XCD's L2.
+struct TilePlace {
+    int tm, tn;
+};
+__device__ __forceinline__ TilePlace tile_place(int unit, int tiles_m, int tiles_n) {
+    constexpr int GROUP_M = 8;
+    const int group_sz = GROUP_M * tiles_n;
+    const int g = unit / group_sz;
+    const int gm0 = g * GROUP_M;
+    const int gh = (tiles_m - gm0) < GROUP_M ? (tiles_m - gm0) : GROUP_M;
+    return TilePlace{gm0 + (unit - g * group_sz) % gh, (unit - g * group_sz) / gh};
+}
+
+template <bool DEQ, bool RAGGED, int BM>
+__device__ __forceinline__ void sp256_tile(
     const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, int M, int N, int Kb, int32_t* __restrict__ C,
     f16* __restrict__ Y, const f16* __restrict__ sA, const f16* __restrict__ sB, const f16* __restrict__ bias,
-    int tiles_m, int tiles_n, int nxcd) {
+    int m0, int n0) {
     static_assert(BM == 256 || BM == 192, "wave tiles of 4 or 3 accumulator tiles along M");
     constexpr int BN = 256, NT = 256;
     constexpr int TM = BM / 2, TN = 128, IM = TM / 32, JN = 4;
@@ -325,18 +339,6 @@ __global__ __launch_bounds__(256) void gemm_sp256_kernel(
     constexpr int S0 = 4;                                   // first slot that unpacks (LDS reads are issued in slots 0..7, in fragment order)
     constexpr bool DIRECT = !RAGGED;                        // whole stages go straight into LDS (see gemm_spk_kernel)
     extern __shared__ u32x4 sp2_lds[];                       // [2][CH]; later the output slabs
-
-    const int per_xcd = gridDim.x / nxcd;
-    int tile = (blockIdx.x % nxcd) * per_xcd + blockIdx.x / nxcd;
-    if (tile >= tiles_m * tiles_n) return;
-    constexpr int GROUP_M = 8;
-    const int group_sz = GROUP_M * tiles_n;
-    const int g = tile / group_sz;
-    const int gm0 = g * GROUP_M;
-    const int gh = (tiles_m - gm0) < GROUP_M ? (tiles_m - gm0) : GROUP_M;
-    const int tm = gm0 + (tile - g * group_sz) % gh;
-    const int tn = (tile - g * group_sz) / gh;
-    const int m0 = tm * BM, n0 = tn * BN;
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wm = wave >> 1, wn = wave & 1;
@@ -581,10 +583,10 @@ __global__ __launch_bounds__(256) void gemm_sp256_kernel(
 }
 
 template <bool DEQ, bool RAGGED>
-__global__ __launch_bounds__(256) void gemm_spk_kernel(
+__device__ __forceinline__ void spk_tile(
     const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, int M, int N, int Kb, int32_t* __restrict__ C,
     f16* __restrict__ Y, const f16* __restrict__ sA, const f16* __restrict__ sB, const f16* __restrict__ bias,
-    int tiles_m, int tiles_n, int nxcd) {
+    int m0, int n0) {
     constexpr int BM = 128, BN = 256, NT = 256;
     constexpr int TM = 128, TN = 128, IM = 4, JN = 4;
     constexpr int CH = (BM + BN) * 8;                       // 16-byte chunks per stage
@@ -599,18 +601,6 @@ __global__ __launch_bounds__(256) void gemm_spk_kernel(
     // be written as zeros) at M = 2048, N = 4096, K = 11008 and K = 4096.
     constexpr bool DIRECT = !RAGGED;
     extern __shared__ u32x4 spk_lds[];                       // [DIRECT ? 3 : 2][CH]; later the output slabs
-
-    const int per_xcd = gridDim.x / nxcd;
-    int tile = (blockIdx.x % nxcd) * per_xcd + blockIdx.x / nxcd;
-    if (tile >= tiles_m * tiles_n) return;
-    constexpr int GROUP_M = 8;
-    const int group_sz = GROUP_M * tiles_n;
-    const int g = tile / group_sz;
-    const int gm0 = g * GROUP_M;
-    const int gh = (tiles_m - gm0) < GROUP_M ? (tiles_m - gm0) : GROUP_M;
-    const int tm = gm0 + (tile - g * group_sz) % gh;
-    const int tn = (tile - g * group_sz) / gh;
-    const int m0 = tm * BM, n0 = tn * BN;
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wm = 0, wn = wave & 1, kg = wave >> 1;        // K-group kg multiplies sub-steps 2 kg and 2 kg + 1 of every stage
@@ -924,6 +914,53 @@ __global__ __launch_bounds__(256) void gemm_spk_kernel(
     }
 }
 
+template <bool DEQ, bool RAGGED, int BM = 256>
+__global__ __launch_bounds__(256) void gemm_sp256_kernel(
+    const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, int M, int N, int Kb, int32_t* __restrict__ C,
+    f16* __restrict__ Y, const f16* __restrict__ sA, const f16* __restrict__ sB, const f16* __restrict__ bias,
+    int tiles_m, int tiles_n, int nxcd) {
+    const int per_xcd = gridDim.x / nxcd;
+    const int tile = (blockIdx.x % nxcd) * per_xcd + blockIdx.x / nxcd;
+    if (tile >= tiles_m * tiles_n) return;
+    const TilePlace p = tile_place(tile, tiles_m, tiles_n);
+    sp256_tile<DEQ, RAGGED, BM>(A, B, M, N, Kb, C, Y, sA, sB, bias, p.tm * BM, p.tn * 256);
+}
+
+template <bool DEQ, bool RAGGED>
+__global__ __launch_bounds__(256) void gemm_spk_kernel(
+    const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, int M, int N, int Kb, int32_t* __restrict__ C,
+    f16* __restrict__ Y, const f16* __restrict__ sA, const f16* __restrict__ sB, const f16* __restrict__ bias,
+    int tiles_m, int tiles_n, int nxcd) {
+    const int per_xcd = gridDim.x / nxcd;
+    const int tile = (blockIdx.x % nxcd) * per_xcd + blockIdx.x / nxcd;
+    if (tile >= tiles_m * tiles_n) return;
+    const TilePlace p = tile_place(tile, tiles_m, tiles_n);
+    spk_tile<DEQ, RAGGED>(A, B, M, N, Kb, C, Y, sA, sB, bias, p.tm * 128, p.tn * 256);
+}
+
+// Whole rounds of 256x256 tiles over the CUs, then the tiles of the last round, where they are at most half as many as
+// there are CUs, as two 128x256 tiles each: a last round of R tiles keeps cus - R CUs idle for a whole tile's time, its halves
+// fill 2 R CUs for 0.57 of it.  `whole` (a multiple of the CU count) workgroups take the whole tiles, those after them the halves; both kinds
+// need a CU to themselves (LDS), so a half starts where a whole tile has ended.
+template <bool DEQ>
+__global__ __launch_bounds__(256) void gemm_sp256_tail_kernel(
+    const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, int M, int N, int Kb, int32_t* __restrict__ C,
+    f16* __restrict__ Y, const f16* __restrict__ sA, const f16* __restrict__ sB, const f16* __restrict__ bias,
+    int tiles_m, int tiles_n, int nxcd, int whole) {
+    if ((int)blockIdx.x < whole) {
+        const TilePlace p = tile_place((blockIdx.x % nxcd) * (whole / nxcd) + blockIdx.x / nxcd, tiles_m, tiles_n);
+        sp256_tile<DEQ, false, 256>(A, B, M, N, Kb, C, Y, sA, sB, bias, p.tm * 256, p.tn * 256);
+        return;
+    }
+    const int b = blockIdx.x - whole;
+    const int unit = (b % nxcd) * (((int)gridDim.x - whole) / nxcd) + b / nxcd;
+    if (whole + unit / 2 >= tiles_m * tiles_n) return;
+    const TilePlace p = tile_place(whole + unit / 2, tiles_m, tiles_n);
+    const int m0 = p.tm * 256 + (unit & 1) * 128;
+    if (m0 >= M) return;
+    spk_tile<DEQ, false>(A, B, M, N, Kb, C, Y, sA, sB, bias, m0, p.tn * 256);
+}
+
 int launch_spk(const void* A, const void* B, int M, int N, int Kb, void* C, void* Y, const void* sA, const void* sB,
                const void* bias, hipStream_t st) {
     const int tiles_m = (M + 127) / 128, tiles_n = (N + 255) / 256;
@@ -985,6 +1022,25 @@ int launch_sp256(const void* A, const void* B, int M, int N, int Kb, void* C, vo
     else
         kern<<<dim3(grid), dim3(256), LDS, st>>>((const uint8_t*)A, (const uint8_t*)B, M, N, Kb, (int32_t*)C, nullptr,
                                                  nullptr, nullptr, nullptr, tiles_m, tiles_n, nxcd);
+    return qr_launch_status();
+}
+
+// gemm_sp256_tail_kernel (K a multiple of 256, more than one round of tiles, CUs a multiple of the XCDs: mid_plan's rule)
+int launch_sp256_tail(const void* A, const void* B, int M, int N, int Kb, void* C, void* Y, const void* sA, const void* sB,
+                      const void* bias, hipStream_t st) {
+    const size_t LDS = (size_t)3 * (128 + 256) * 8 * 16;    // the larger of the two tiles' stage buffers
+    const int tiles_m = (M + 255) / 256, tiles_n = (N + 255) / 256;
+    const int nxcd = qr_device().xcds, cus = qr_device().cus;
+    const int64_t tiles = (int64_t)tiles_m * tiles_n, whole = tiles / cus * cus;
+    const int64_t halves = ((tiles - whole) * 2 + nxcd - 1) / nxcd * nxcd;
+    if (whole + halves > 0x3fffffff) return QR_E_SHAPE;
+    if ((int64_t)M * Kb >= (1LL << 32) || (int64_t)N * Kb >= (1LL << 32)) return QR_E_UNSUPPORTED;
+    auto kern = Y ? gemm_sp256_tail_kernel<true> : gemm_sp256_tail_kernel<false>;
+    const hipError_t e = qr_allow_dynamic_lds((const void*)kern, LDS);
+    if (e != hipSuccess) return (int)e;
+    kern<<<dim3((unsigned)(whole + halves)), dim3(256), LDS, st>>>((const uint8_t*)A, (const uint8_t*)B, M, N, Kb, (int32_t*)C,
+                                                                   (f16*)Y, (const f16*)sA, (const f16*)sB, (const f16*)bias,
+                                                                   tiles_m, tiles_n, nxcd, (int)whole);
     return qr_launch_status();
 }
 
@@ -1851,7 +1907,8 @@ int ks_split(int64_t M, int64_t N, int64_t Kb) {
 // Very few tiles and a long K: slices of K over several workgroups with int32 slabs in the caller's scratch and a second
 // launch that adds them (+ 3.5 us and the slabs' way out and back at 4 TB/s).
 struct MidPlan {
-    int kernel;         // 0 .. 2: qr_internal_gemm_mid's shapes; 3, 4, 5: pipelined 128-, 192-, 256-row tiles
+    int kernel;         // 0 .. 2: qr_internal_gemm_mid's shapes; 3, 4, 5: pipelined 128-, 192-, 256-row tiles; 6: 256-row
+                        // tiles and a last round of 128-row ones
     int split;
 };
 MidPlan mid_plan(int64_t M, int64_t N, int64_t Kb, int64_t max_split) {
@@ -1887,6 +1944,13 @@ MidPlan mid_plan(int64_t M, int64_t N, int64_t Kb, int64_t max_split) {
     const double rounds = loaded(t);
     const double idle = 1.0 - (double)t / (rounds * (double)cus);
     consider(3 + tall, 1, rounds * (5.5 + slope[tall] * (double)st * (1.0 - (tall == 0 ? 0.3 : 0.5) * idle)));
+    // Whole rounds of 256-row tiles and the rest as 128-row ones in the same launch, where that rest is at most half a round:
+    // 8191 x 5120 x 5120 175 -> 166 us, 6684 x 8192 x 8192 333 -> 307, 10435 x 5120 x 5120 226 -> 209, 32768 x 4096 x 11008
+    // 1099 -> 1078.  The estimate for 192-row tiles is 6 % high beside it (4583 x 5120 x 15360: 265 us against 268).
+    const int64_t whole = tiles(256, 256) / cus, left = tiles(256, 256) % cus;
+    if (Kb % 128 == 0 && cus % qr_device().xcds == 0 && whole > 0 && left > 0 && 2 * left <= cus)
+        consider(6, 1, (tall == 1 ? 1.06 : 1.0) * ((double)whole * (5.5 + slope[2] * (double)st) + 5.5 +
+                                                   slope[0] * (double)st * (1.0 - 0.3 * (1.0 - 2.0 * (double)left / (double)cus))));
     for (int64_t ks = 2; ks <= max_split && ks <= st / 4; ++ks)
         consider(0, (int)ks, t64(tiles(64, 64) * ks, (st + ks - 1) / ks) + 3.5 + 2.0 * (double)ks * (double)M * (double)N * 4.0 / 4.0e6);
     return best;
@@ -1938,6 +2002,7 @@ int gemm_dispatch(const void* A, const void* B, int64_t M, int64_t N, int64_t K,
     }
     if (plan.kernel <= 2) return qr_internal_gemm_mid(plan.kernel, A, B, m, n, kb, C, Y, sA, sB, bias, st, 1);
     if (plan.kernel == 3) return launch_spk(A, B, m, n, kb, C, Y, sA, sB, bias, st);
+    if (plan.kernel == 6) return launch_sp256_tail(A, B, m, n, kb, C, Y, sA, sB, bias, st);
     return launch_sp256(A, B, m, n, kb, C, Y, sA, sB, bias, st, plan.kernel == 4 ? 192 : 256);
 }
 

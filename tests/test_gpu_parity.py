@@ -1030,6 +1030,28 @@ def test_fused_heads_hadamard_quantize(heads, rows, clip):
     assert float((p.quantized_x == staged.quantized_x).float().mean()) > 0.99
 
 
+@pytest.mark.parametrize("M,N,K", [(7934, 5120, 512), (8191, 5120, 768), (4554, 12289, 256), (6657, 8203, 512), (13308, 4100, 1280)])
+def test_gemm_whole_rounds_and_a_last_round_of_half_tiles(M, N, K):
+    """Outputs whose 256x256 tiles are some rounds over 256 CUs and at most half a round more: the last ones run as two
+    128-row tiles each.  Row counts that leave the second half of the last row tile partial or empty, column counts that
+    are no multiple of 4 or 8.  The integer product is exact in fp32 (K * 64 < 2^24); the fp16 output is one formula of it."""
+    g = torch.Generator(device="cuda").manual_seed(M)
+    a, w = (torch.randint(-8, 8, (r, K), generator=g, device="cuda", dtype=torch.int8) for r in (M, N))
+    packed = lambda t: ((t[:, 0::2] & 15) | (t[:, 1::2] << 4)).view(torch.uint8).contiguous()
+    sa = (torch.rand(M, 1, generator=g, device="cuda") * 0.1 + 0.01).half()
+    sw = (torch.rand(N, 1, generator=g, device="cuda") * 0.01 + 0.001).half()
+    bias = torch.randn(N, generator=g, device="cuda").half()
+    want = a.float() @ w.float().T
+    got = quarot_amd.matmul(packed(a), packed(w))
+    assert torch.equal(got, want.int())
+    with torch.device("cuda"):
+        lin = quarot_amd.nn.Linear4bit(K, N, bias=True).half()
+    lin.weight, lin.weight_scales, lin.bias = packed(w), sw, bias
+    y = lin(quarot_amd.PackedQuantizedTensor(packed(a), sa))
+    ref = quarot_amd.sym_dequant(got, sa, sw.T.contiguous().view(-1, 1)) + bias
+    assert torch.equal(y, ref)
+
+
 @pytest.mark.parametrize("heads", [12, 20, 28, 36, 40, 52, 60])
 @pytest.mark.parametrize("rows,clip", [(1, 1.0), (4, 0.9), (5, 1.0), (3089, 1.0)])
 def test_fused_heads_hadamard_quantize_behind_a_table(heads, rows, clip):
