@@ -1238,16 +1238,11 @@ __global__ __launch_bounds__(512) void decode_i4_kernel(const uint8_t* __restric
 //   on the order): with a row pitch that is a power of two, workgroups marching through K in step
 //   would all be reading the same few memory channels at any one time (measured 49 -> 41 us at
 //   57344 x 8192).
-// * ksplit > 1 (int32 output only; weights with few rows, 32..64 tokens): `ksplit` workgroups share a block of R
-//   groups and each walks its own slice of K, writing its partial sums to its own [M, N] slab of C -- a workgroup then
-//   pulls 1 / ksplit of the tokens' codes through its CU's vector memory path, which is what bounds this shape (every
-//   CU reading ALL the tokens' codes next to its share of the weights: 0.92 MB beside 0.46 MB at 64 tokens).
 template <int MT, int R, int RD, bool DEQ>
 __global__ __launch_bounds__(768) void decode_xs_kernel(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B,
                                                         int M, int N, int Kb, int32_t* __restrict__ C,
                                                         f16* __restrict__ Y, const f16* __restrict__ sA,
-                                                        const f16* __restrict__ sB, const f16* __restrict__ bias,
-                                                        int ksplit) {
+                                                        const f16* __restrict__ sB, const f16* __restrict__ bias) {
     constexpr int XR = MT * 32;                             // staged rows of X
     constexpr int NL = MT + R;                              // 16-byte chunks per loader thread and stage: 32 rows each
     constexpr int XPLANES = XR * 16;                        // slots of the tokens' planes (32 bytes per packed chunk)
@@ -1257,12 +1252,8 @@ __global__ __launch_bounds__(768) void decode_xs_kernel(const uint8_t* __restric
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int r = lane & 31, h = lane >> 5;
     const bool loader = wave >= 8;                          // waves 8..11 fetch, waves 0..R-1 multiply
-    const int rblock = blockIdx.x / ksplit, slice = blockIdx.x - rblock * ksplit;
-    const int n0 = rblock * (R * 32);
-    const int all_stages = (Kb + 127) / 128;
-    const int sfirst = (int)((int64_t)all_stages * slice / ksplit);
-    const int stages = (int)((int64_t)all_stages * (slice + 1) / ksplit) - sfirst;      // >= 1: ksplit <= all_stages
-    if (ksplit > 1) C += (int64_t)slice * M * N;
+    const int n0 = blockIdx.x * (R * 32);
+    const int stages = (Kb + 127) / 128;
     const bool ragged = (Kb & 127) != 0;
     auto slot8 = [](int row, int chunk) { return row * 8 + (chunk ^ ((row >> 1) & 7)); };
     auto slot16 = [](int row, int chunk, int plane) {
@@ -1284,10 +1275,10 @@ __global__ __launch_bounds__(768) void decode_xs_kernel(const uint8_t* __restric
     }
     const int wdst0 = XPLANES + slot8(srow, piece);         // rows differ by multiples of 32: same swizzle
     const int xdst0 = slot16(srow, piece, 0);
-    const int s0 = rblock % stages;
+    const int s0 = blockIdx.x % stages;
     auto stage_of = [&](int st) {                           // absolute stage of this workgroup's st-th step
-        int a = (st < stages ? st : stages - 1) + s0;
-        return sfirst + (a >= stages ? a - stages : a);
+        const int a = (st < stages ? st : stages - 1) + s0;
+        return a >= stages ? a - stages : a;
     };
     auto fetch = [&](int st, u32x4(&v)[NL]) {
         const int kb = stage_of(st) * 128;
@@ -1757,9 +1748,8 @@ int decode_xs_groups(int N) {
 }
 
 int launch_decode_xs(const void* A, const void* B, int M, int N, int Kb, void* C, void* Y, const void* sA,
-                     const void* sB, const void* bias, hipStream_t st, int rg, int ksplit = 1) {
-    if (ksplit > 1 && Y) return QR_E_UNSUPPORTED;           // partial sums exist only as int32
-    const unsigned grid = (unsigned)((((N + 31) / 32 + rg - 1) / rg) * ksplit);
+                     const void* sB, const void* bias, hipStream_t st, int rg) {
+    const unsigned grid = (unsigned)(((N + 31) / 32 + rg - 1) / rg);
 #define QR_XS(MT, R)                                                                                                  \
     do {                                                                                                              \
         constexpr int RD = 3;   /* deeper rings were measured slower (4: +3 %, 5: +6 %) */                            \
@@ -1770,13 +1760,13 @@ int launch_decode_xs(const void* A, const void* B, int M, int N, int Kb, void* C
             e = qr_allow_dynamic_lds((const void*)kern, LDS);                                                         \
             if (e != hipSuccess) return (int)e;                                                                       \
             kern<<<dim3(grid), dim3(768), LDS, st>>>((const uint8_t*)A, (const uint8_t*)B, M, N, Kb, nullptr, (f16*)Y, \
-                                                     (const f16*)sA, (const f16*)sB, (const f16*)bias, 1);            \
+                                                     (const f16*)sA, (const f16*)sB, (const f16*)bias);               \
         } else {                                                                                                      \
             auto kern = decode_xs_kernel<MT, R, RD, false>;                                                           \
             e = qr_allow_dynamic_lds((const void*)kern, LDS);                                                         \
             if (e != hipSuccess) return (int)e;                                                                       \
             kern<<<dim3(grid), dim3(768), LDS, st>>>((const uint8_t*)A, (const uint8_t*)B, M, N, Kb, (int32_t*)C,     \
-                                                     nullptr, nullptr, nullptr, nullptr, ksplit);                     \
+                                                     nullptr, nullptr, nullptr, nullptr);                             \
         }                                                                                                             \
     } while (0)
 #define QR_XS_R(MT)                                                                                                   \
@@ -1852,26 +1842,54 @@ __global__ __launch_bounds__(256) void dequant_slabs_kernel(const int32_t* __res
     }
 }
 
-// Decode against a weight with too few rows for the shared-token kernel to fill the CUs (70B down_proj: 8192 rows =
-// 64 blocks of four groups): at 40 and more tokens each CU's intake of the tokens' codes bounds the barrier-free
-// kernel.  With scratch from the caller the shared-token kernel runs with four groups per workgroup and as many K
-// slices per block as fill the CUs, and dequant_slabs_kernel adds the slabs.  Measured (8192 x 28672, both launches):
-// 64 tokens 35.5 -> 30.6 us, 48 tokens 31.3 -> 29.8; level at 32 and behind below that, and behind at every token count
-// when K is 8192 (the slices get too short for their fixed costs): those shapes keep the barrier-free kernel.
-int decode_split(int64_t M, int64_t N, int64_t Kb) {
-    if (M < 40 || M > 64 || Kb < 8192 || decode_xs_groups((int)N) != 0) return 1;
-    const int64_t blocks = ((N + 31) / 32 + 3) / 4, cus = qr_device().cus, all_stages = (Kb + 127) / 128;
-    int64_t s = cus / blocks;
-    if (s > all_stages / 16) s = all_stages / 16;
-    if (s > 8) s = 8;
-    return s >= 2 ? (int)s : 1;
+// 8 .. 64 tokens against a weight with too few rows for the shared-token kernel: the barrier-free kernel, or 64 x 64 tiles in
+// the STREAM form of gemm_mid_kernel, with K in slices over several workgroups (int32 slabs in the caller's scratch and a
+// second launch that adds them) where that fills CUs.  In the barrier-free kernel every group of 32 weight rows pulls all the tokens'
+// codes through its CU, which takes in some 60 GB/s, and a 64-row tile halves that; but its fixed path is shorter (one barrier).
+// Estimates in microseconds, st = stages of 256 k, fitted to both kernels at 5 .. 64 tokens x 1041 .. 22016 weight rows x K = 1024
+// .. 28672, with weights in the last-level cache and from memory (which differ by less than the kernels do):
+//   barrier-free   3 + st (0.12 + 0.0028 M), 1.2 more for a second tile of tokens; up to 3.5 more between 4096 and 8192 rows where K is longer
+//                  than the waves' rings; the whole times 0.8 + rows / 12500 beyond 8192 rows (less where K is short)
+//   STREAM tiles   4.4 + st / slices x (0.235 + 0.0009 M up to 128 workgroups, 0.28 + 0.002 M up to a workgroup per CU,
+//                  0.25 + 0.0012 M for each of several), at least the weights at 6.2 TB/s; slices: + 2.5, 0.3 for each beyond
+//                  three, the slabs' way out and back at 4 TB/s, 4 where rows are no whole number of 16-byte pieces
+// From memory, before / after: 48 x 12288 x 4096 14.2 / 9.1 us, 48 x 13824 x 5120 19.8 / 11.1, 48 x 22016 x 4096 20.6 / 13.5, 48 x 5120 x
+// 13824 17.6 / 13.3, 48 x 4096 x 11008 14.9 / 12.0, 25 x 12288 x 8192 17.0 / 14.3; 32 x 4096 x 4096 stays (6.1 against 8.3).  Below eight tokens
+// the two are within 5 % of each other where the tiles lead at all.  Slices only where three or more fit, or where two save 4 us
+// (40 tokens and K = 16384 on): the scratch that callers are asked for grows with them.
+struct DecodePlan {
+    bool tiles;
+    int split;
+};
+DecodePlan decode_plan(int64_t M, int64_t N, int64_t Kb, int64_t max_split) {
+    DecodePlan best{false, 1};
+    if (M < 8 || M > 64 || decode_xs_groups((int)N) != 0) return best;
+    const int64_t cus = qr_device().cus, st = (Kb + 127) / 128, tiles = (N + 63) / 64;
+    const double m = (double)M, s = (double)st;
+    double t_best = 3.0 + s * (0.12 + 0.0028 * m) + (M > 32 ? 1.2 : 0.0);
+    if (N > 8192) t_best = 3.0 + (t_best * (0.8 + (double)N / 12500.0) - 3.0) * (s < 16.0 ? s / 16.0 : 1.0);
+    else if (N > 4096 && st > 24) t_best += 3.5 * (double)(N - 4096) / 4096.0;
+    const int64_t most = tiles * 3 <= cus || (M >= 40 && Kb >= 8192) ? (max_split < 8 ? max_split : 8) : 1;
+    for (int64_t ks = 1; ks <= most && (ks == 1 || (ks <= st / 4 && tiles * ks <= cus)); ++ks) {
+        const int64_t wgs = tiles * ks;
+        const double slope = wgs * 2 <= cus ? 0.235 + 0.0009 * m
+                             : wgs <= cus   ? 0.28 + 0.002 * m : (0.25 + 0.0012 * m) * (double)((wgs + cus - 1) / cus);
+        const double walk = (double)((st + ks - 1) / ks) * slope, stream = (double)N * (double)Kb / 6.2e6;
+        double t = 4.4 + (walk > stream ? walk : stream);
+        if (ks > 1) t += 2.5 + (ks > 3 ? 0.3 * (double)(ks - 3) : 0.0) + 2.0 * (double)ks * m * (double)N * 4.0 / 4.0e6 + (N % 4 ? 4.0 : 0.0);
+        if (t < t_best) {
+            t_best = t;
+            best = DecodePlan{true, (int)ks};
+        }
+    }
+    return best;
 }
 
 // How many int32 slabs of [M, N] a caller is asked to provide (qr_workspace_bytes): for prompts of a few hundred tokens an
 // upper bound of the slices that mid_plan may use, larger than it needs since its tiles fill the CUs without a split at
 // most of these shapes; callers size their scratch once per shape.
 int ks_split(int64_t M, int64_t N, int64_t Kb) {
-    if (M <= 64) return decode_split(M, N, Kb);
+    if (M <= 64) return decode_plan(M, N, Kb, 8).split;
     if (N <= 128) return 1;
     const int64_t tn = (N + 255) / 256;
     const int64_t cus = qr_device().cus;
@@ -1984,11 +2002,12 @@ int gemm_dispatch(const void* A, const void* B, int64_t M, int64_t N, int64_t K,
         return qr_launch_status();
     };
     if (M <= 64) {
-        const int split = decode_split(M, N, kb);
-        if (split > 1 && scratch && ws_bytes >= (size_t)split * (size_t)M * (size_t)N * 4) {
-            const int rc = launch_decode_xs(A, B, m, n, kb, ws, nullptr, nullptr, nullptr, nullptr, st, 4, split);
-            return rc != QR_OK ? rc : add_slabs(split);
+        const DecodePlan plan = decode_plan(M, N, kb, scratch ? (int64_t)(ws_bytes / ((size_t)M * (size_t)N * 4)) : 1);
+        if (plan.tiles && plan.split > 1) {
+            const int rc = qr_internal_gemm_mid(3, A, B, m, n, kb, ws, nullptr, nullptr, nullptr, nullptr, st, plan.split);
+            return rc != QR_OK ? rc : add_slabs(plan.split);
         }
+        if (plan.tiles) return qr_internal_gemm_mid(3, A, B, m, n, kb, C, Y, sA, sB, bias, st, 1);
         // weight streaming: with enough groups of 32 rows to fill the CUs the kernel that shares the
         // tokens' codes through LDS (they are read once per workgroup); otherwise the barrier-free
         // kernel in which the waves of a workgroup split K over groups of 32 rows

@@ -11,12 +11,17 @@
 // Stages go straight from global memory into LDS (buffer_load ... lds), NBUF - 1 stages ahead, one barrier per stage;
 // while a stage's MFMAs run, the wave's fragments of the next sub-step are read and unpacked.
 // K need not be a multiple of 256: a sub-step beyond K is skipped (its loads repeat the stage's first piece).
+// STREAM (up to 64 tokens: one row of tiles, every weight used once): the weights' loads are nontemporal, so that they do not
+// push the tokens' codes out of the caches, and tile t starts its walk over K at stage t (integer sums do not depend on the order),
+// so that the workgroups do not all ask the same memory channels at a time where the row pitch is a power of two.  With
+// weights that come from memory (more of them in turn than the last-level cache holds), 48 tokens against 12288 x 4096: 11.2 -> 9.1 us, 8192 x 8192
+// 17.2 -> 13.1, 28672 x 8192 30.9 -> 26.4.
 #include "qr_common.h"
 #include "qr_epilogue.h"
 
 namespace {
 
-template <int BM, int BN, int WK, int NBUF, bool DEQ>
+template <int BM, int BN, int WK, int NBUF, bool DEQ, bool STREAM>
 __global__ __launch_bounds__(64 * (BM / 64) * (BN / 64) * WK) void gemm_mid_kernel(
     const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, int M, int N, int Kb, int32_t* __restrict__ C,
     f16* __restrict__ Y, const f16* __restrict__ sA, const f16* __restrict__ sB, const f16* __restrict__ bias,
@@ -48,6 +53,7 @@ __global__ __launch_bounds__(64 * (BM / 64) * (BN / 64) * WK) void gemm_mid_kern
     if (ksplit > 1) C += (int64_t)split * M * N;
     const int s0 = (int)((int64_t)all_stages * split / ksplit);
     const int stages = (int)((int64_t)all_stages * (split + 1) / ksplit) - s0;      // >= 1: ksplit <= all_stages
+    const int rot = STREAM && (Kb & 127) == 0 ? tile % stages : 0;     // (a last stage that ends inside K stays the last)
     auto slot8 = [](int row, int chunk) { return row * 8 + (chunk ^ ((row >> 1) & 7)); };
 
     // ---- staging: a thread fetches, for its rows srow + i RPL, the piece that the XOR-keyed layout keeps at its place
@@ -65,12 +71,13 @@ __global__ __launch_bounds__(64 * (BM / 64) * (BN / 64) * WK) void gemm_mid_kern
     const __amdgpu_buffer_rsrc_t rsrc_a = __builtin_amdgcn_make_buffer_rsrc((void*)A, 0, (int)((u32)M * (u32)Kb), 0x00020000);
     const __amdgpu_buffer_rsrc_t rsrc_b = __builtin_amdgcn_make_buffer_rsrc((void*)B, 0, (int)((u32)N * (u32)Kb), 0x00020000);
     auto request1 = [&](int st, int buf, int i) {           // load i of stage st into stage buffer buf
-        const int kb = (s0 + st) * 128;
+        const int at = st + rot;
+        const int kb = (s0 + (STREAM && at >= stages ? at - stages : at)) * 128;
         __attribute__((address_space(3))) void* dst =
             (__attribute__((address_space(3))) void*)(mid_lds + buf * CH + i * NT + wave * 64);
         const u32 o = goff[i] + (u32)(kb + piece < Kb ? piece : 0);
         if (i * RPL < BM) __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_a, dst, 16, o, kb, 0, 0);
-        else __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_b, dst, 16, o, kb, 0, 0);
+        else __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_b, dst, 16, o, kb, 0, STREAM ? 2 : 0);
     };
 
     // ---- fragments.  A K-group holds its accumulator tiles permuted so that the ones it finalises are always the first:
@@ -303,7 +310,7 @@ __global__ __launch_bounds__(64 * (BM / 64) * (BN / 64) * WK) void gemm_mid_kern
         }
 }
 
-template <int BM, int BN, int WK, int NBUF>
+template <int BM, int BN, int WK, int NBUF, bool STREAM = false>
 int launch_mid(const void* A, const void* B, int M, int N, int Kb, void* C, void* Y, const void* sA, const void* sB,
                const void* bias, hipStream_t st, int ksplit) {
     constexpr int NT = 64 * (BM / 64) * (BN / 64) * WK;
@@ -316,7 +323,7 @@ int launch_mid(const void* A, const void* B, int M, int N, int Kb, void* C, void
     if ((int64_t)M * Kb >= (1LL << 32) || (int64_t)N * Kb >= (1LL << 32)) return QR_E_UNSUPPORTED;   // (32-bit buffer offsets)
     const int nxcd = qr_device().xcds;                      // the grid is a whole number of rounds over the XCDs
     const unsigned grid = (unsigned)((tiles + nxcd - 1) / nxcd * nxcd);
-    auto kern = Y ? gemm_mid_kernel<BM, BN, WK, NBUF, true> : gemm_mid_kernel<BM, BN, WK, NBUF, false>;
+    auto kern = Y ? gemm_mid_kernel<BM, BN, WK, NBUF, true, STREAM> : gemm_mid_kernel<BM, BN, WK, NBUF, false, STREAM>;
     const hipError_t e = qr_allow_dynamic_lds((const void*)kern, LDS);
     if (e != hipSuccess) return (int)e;
     kern<<<dim3(grid), dim3(NT), LDS, st>>>((const uint8_t*)A, (const uint8_t*)B, M, N, Kb, (int32_t*)C, (f16*)Y, (const f16*)sA,
@@ -326,14 +333,22 @@ int launch_mid(const void* A, const void* B, int M, int N, int Kb, void* C, void
 
 }  // namespace
 
-// shape: 0 = 64 x 64, 1 = 64 x 128, 2 = 128 x 128 tiles.  Three stage buffers of 16 or 24 KB let three or two workgroups
-// share a CU; 64 x 128 with five and 64 x 64 with four buffers were no faster (11.8 against 11.2 us, 8.3 against 8.2 at
-// 128 and 333 tokens x 4096 x 4096): the loads are bound by rate, not by how many are in flight.
+// shape: 0 = 64 x 64, 1 = 64 x 128, 2 = 128 x 128 tiles; 3 = 64 x 64 in the STREAM form (M <= 64).  Three stage buffers of 16
+// or 24 KB let three or two workgroups share a CU; 64 x 128 with five and 64 x 64 with four buffers were no faster (11.8
+// against 11.2 us, 8.3 against 8.2 at 128 and 333 tokens x 4096 x 4096): the loads are bound by rate, not by how many are
+// in flight.  The STREAM form's come from memory: with at most a workgroup per CU it takes five buffers, 64 KB in flight (48 x
+// 5120 x 13824 in two slices of K 17.8 -> 15.7 us), with more workgroups three (48 x 22016 x 4096 14.3 -> 13.5).
 __attribute__((visibility("hidden"))) int qr_internal_gemm_mid(int shape, const void* A, const void* B, int M, int N, int Kb,
                                                                void* C, void* Y, const void* sA, const void* sB,
                                                                const void* bias, hipStream_t st, int ksplit) {
     if (ksplit > 1 && Y) return QR_E_UNSUPPORTED;           // partial sums exist only as int32
     if (shape == 0) return launch_mid<64, 64, 4, 3>(A, B, M, N, Kb, C, Y, sA, sB, bias, st, ksplit);
     if (shape == 1) return launch_mid<64, 128, 4, 3>(A, B, M, N, Kb, C, Y, sA, sB, bias, st, ksplit);
+    if (shape == 3) {
+        if (M > 64) return QR_E_UNSUPPORTED;
+        if ((int64_t)((N + 63) / 64) * ksplit <= qr_device().cus)
+            return launch_mid<64, 64, 4, 5, true>(A, B, M, N, Kb, C, Y, sA, sB, bias, st, ksplit);
+        return launch_mid<64, 64, 4, 3, true>(A, B, M, N, Kb, C, Y, sA, sB, bias, st, ksplit);
+    }
     return launch_mid<128, 128, 2, 4>(A, B, M, N, Kb, C, Y, sA, sB, bias, st, ksplit);
 }

@@ -1030,6 +1030,32 @@ def test_fused_heads_hadamard_quantize(heads, rows, clip):
     assert float((p.quantized_x == staged.quantized_x).float().mean()) > 0.99
 
 
+@pytest.mark.parametrize("N,K", [(4104, 11008), (5121, 13824), (8192, 8256), (8200, 28672), (12289, 4096), (22016, 1088), (17000, 64), (520, 8192)])
+@pytest.mark.parametrize("M", [7, 8, 31, 33, 64])
+def test_decode_batches_on_streamed_tiles(M, N, K):
+    """7 to 64 tokens against weights of 520 to 22016 rows: 64 x 64 tiles with one workgroup per CU and with two, K whole and
+    in slices, K that ends inside a stage of 256, column counts that leave the last tile partial or are no multiple of 4.
+    The integer product is exact in fp32 (K * 64 < 2^24); the fp16 output is one formula of it, with and without scratch."""
+    g = torch.Generator(device="cuda").manual_seed(M + N)
+    a, w = (torch.randint(-8, 8, (r, K), generator=g, device="cuda", dtype=torch.int8) for r in (M, N))
+    packed = lambda t: ((t[:, 0::2] & 15) | (t[:, 1::2] << 4)).view(torch.uint8).contiguous()
+    sa = (torch.rand(M, 1, generator=g, device="cuda") * 0.1 + 0.01).half()
+    sw = (torch.rand(N, 1, generator=g, device="cuda") * 0.01 + 0.001).half()
+    bias = torch.randn(N, generator=g, device="cuda").half()
+    got = quarot_amd.matmul(packed(a), packed(w))
+    assert torch.equal(got, (a.float() @ w.float().T).int())
+    with torch.device("cuda"):
+        lin = quarot_amd.nn.Linear4bit(K, N, bias=True).half()
+    lin.weight, lin.weight_scales, lin.bias = packed(w), sw, bias
+    ref = quarot_amd.sym_dequant(got, sa, sw) + bias
+    assert torch.equal(lin(quarot_amd.PackedQuantizedTensor(packed(a), sa)), ref)
+    y = torch.empty(M, N, dtype=torch.float16, device="cuda")
+    pa, pw = packed(a), lin.weight
+    assert _lib.lib().qr_linear_i4_f16(pa.data_ptr(), sa.data_ptr(), pw.data_ptr(), sw.data_ptr(), bias.data_ptr(), M, N, K,
+                                       y.data_ptr(), torch.cuda.current_stream().cuda_stream) == 0
+    assert torch.equal(y, ref)
+
+
 @pytest.mark.parametrize("M,N,K", [(7934, 5120, 512), (8191, 5120, 768), (4554, 12289, 256), (6657, 8203, 512), (13308, 4100, 1280)])
 def test_gemm_whole_rounds_and_a_last_round_of_half_tiles(M, N, K):
     """Outputs whose 256x256 tiles are some rounds over 256 CUs and at most half a round more: the last ones run as two
