@@ -95,7 +95,7 @@ PROFILE_OF = {
     "c4g8": "decode_xs_c4g8_decode_8_tokens_70b_gate_up.txt", "c4g32": "decode_xs_c4g32_decode_32_tokens_70b_gate_up.txt",
     "c4g64": "decode_xs_c4g64_decode_64_tokens_70b_gate_up.txt", "c4m1": "bm_gemv_c4m1_decode_70b_down_proj.txt",
     "c4m8": "decode_i4_c4m8_decode_8_tokens_70b_down_proj.txt", "c4m32": "decode_i4_c4m32_decode_32_tokens_70b_down_proj.txt",
-    "c4m64": "decode_xs_sliced_c4m64_decode_64_tokens_70b_down_proj.txt", "c5": "kv_quant_c5_kv_cache_32x4096x8x128.txt",
+    "c4m64": "gemm_mid_sliced_c4m64_decode_64_tokens_70b_down_proj.txt", "c5": "kv_quant_c5_kv_cache_32x4096x8x128.txt",
     "c6": "paged_decode_i4_c6_decode_attention_32x4096x8x128.txt",
     "b13v": "gemm_sp256_b13v_2048x5120x5120.txt", "b70v": "gemm_sp256_b70v_2048x8192x8192.txt",
     "b13d": "gemm_sp256_b13d_2048x13824x5120.txt", "b70d": "gemm_sp256_b70d_2048x28672x8192.txt",
@@ -317,7 +317,7 @@ def gemm_kernel_name(m, n, k=0):
     tiles = lambda bm, bn: ((m + bm - 1) // bm) * ((n + bn - 1) // bn)
     load = lambda t: (t + 255) // 256
     n64, n128, nsq = load(tiles(64, 64)), load(tiles(64, 128)), load(tiles(128, 128))
-    est = [(4.2 + st * {1: 0.26, 2: 0.44}.get(n64, (0.25 if n64 < 8 else 0.26) * n64), "gemm_mid_kernel<64,64>"),
+    est = [(4.2 + st * {1: 0.26, 2: 0.44}.get(n64, (0.27 if n64 >= 5 and st > 32 else 0.25 if n64 < 8 else 0.26) * n64), "gemm_mid_kernel<64,64>"),
            (4.6 + st * (0.41 if n128 == 1 else 0.52 * n128), "gemm_mid_kernel<64,128>"),
            (5.0 + st * (0.8 if nsq == 1 else 0.92 * nsq), "gemm_mid_kernel<128,128>")]
     tall = min((2, 1, 0), key=lambda i: load(tiles(128 + 64 * i, 256)) * (0.57, 0.80, 1.0)[i])      # ties: the taller tile
