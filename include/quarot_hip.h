@@ -73,7 +73,9 @@ const char* qr_strerror(int code);
  * Numerics: butterflies and scale in fp32.  QR_DTYPE_F16: the power-of-two stage is rounded to fp16
  * before the hadK stage, whose fp32 accumulation is rounded to fp16 (the reference's staging).
  * QR_DTYPE_F32: fp32 throughout.  QR_DTYPE_F16 | QR_HAD_FP32: x and y fp16, hadK fp32, no rounding to fp16 between the
- * two factors (results to fp32 accuracy, rounded to fp16 once); QR_E_UNSUPPORTED for n <= 128.
+ * two factors, results rounded to fp16 once; QR_E_UNSUPPORTED for n <= 128.  K = 1: fp32 throughout, the bits of QR_DTYPE_F32
+ * on the same rows.  K > 1: as QR_DTYPE_F32, whose hadK stage takes the scaled value as the sum of two fp16 values (22 bits, of
+ * magnitude 2^-24 and more).
  */
 int qr_hadamard(const void* x, void* y, int64_t rows, int n, int K, const void* hadK,
                 int dtype, float scale, void* stream);

@@ -2565,8 +2565,10 @@ extern "C" int qr_hadamard(const void* x, void* y, int64_t rows, int n, int K, c
         // 4 bytes per value instead of the 20 of a conversion, the fp32 transform and a conversion back -- 1178 x 13824
         // 129 -> 39 us, 2048 x 5120 65 -> 17, 122 x 28672 69 -> 11, 1777 x 28672 455 -> 60.  Rows of 128 and shorter keep those three steps.
         if (n <= 128) return QR_E_UNSUPPORTED;
-        if (K == 1 && pow2_split(n))
-            return launch_hadamard_mm<true, false>(x, y, rows, n, pow2_split(n), nullptr, scale, 1.f, nullptr, nullptr, st);
+        // Power-of-two rows: the general kernel's fp32 butterflies from end to end, the fp32 transform's bits.  (The two-factor
+        // kernel holds the value between its factors as two fp16 planes, and the low one has no bits left for small rows: of
+        // 4096-wide rows of 1e-2 6 % and of 1e-3 33 % of the results were not the transform's nearest fp16 value.)
+        if (K == 1) return launch_hadamard<f16, true, false>(x, y, rows, n, K, hadK, scale, 1.f, nullptr, nullptr, st);
         if (bm_applies(n, K) && n / K == 1024)
             return launch_hadamard_bm<false, true>(x, y, rows, n, K, hadK, scale, 1.f, nullptr, nullptr, st);
         if (mm_applies(n, K))

@@ -978,6 +978,28 @@ def test_online_hadamard_fp32_on_fp16_rows_is_the_fp32_transform_rounded_once(n)
     assert torch.equal(had(torch.cat([x, x], 1)[:, :n]), y)                   # strided rows
 
 
+@pytest.mark.parametrize("n", [256, 1024, 2048, 4096, 8192, 16384, 32768])
+@pytest.mark.parametrize("size", [300.0, 1.0, 0.1, 1e-2, 1e-3, 1e-4])
+def test_online_hadamard_fp32_on_power_of_two_fp16_rows_keeps_small_activations(n, size):
+    """force_fp32 without a table is fp32 butterflies from end to end, whatever the rows' magnitude: the bits of the fp32
+    transform of the same rows rounded once.  That one is within log2(n) roundings of float64, 2^-24 of the row's root mean
+    square each, next to the fp16 rounding itself (2^-11, or 2^-25 below the normal range)."""
+    g = torch.Generator().manual_seed(n)
+    x = torch.randn(17, n, generator=g) * size
+    x[:, ::97] *= 20
+    x = x.clamp(-6e4, 6e4).half().cuda()
+    y = quarot_amd.nn.OnlineHadamard(n, force_fp32=True).cuda()(x)
+    assert torch.equal(y, quarot_amd.functional.matmul_hadU_cuda(x.float(), None, 1).half())
+    t, s = x.double(), 1
+    while s < n:
+        t = t.view(17, n // (2 * s), 2, s)
+        t = torch.stack([t[:, :, 0] + t[:, :, 1], t[:, :, 0] - t[:, :, 1]], 2)
+        s *= 2
+    ref = t.view(17, n) / n ** 0.5
+    slack = 2.0 ** -11 * ref.abs() + 2.0 ** -25 + np.log2(n) * 2.0 ** -24 * ref.pow(2).mean(1, keepdim=True).sqrt()
+    assert bool(((y.double() - ref).abs() <= slack).all())
+
+
 def test_fused_rmsnorm_quantize_full_size_and_errors():
     """Benchmark-size input (2048 x 4096) on strided rows; mean_dim different from the width;
     argument errors of the C entry point."""
