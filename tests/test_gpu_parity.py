@@ -1646,7 +1646,7 @@ def test_runs_on_the_current_stream():
 
 
 @pytest.mark.parametrize("M", [1, 2])
-@pytest.mark.parametrize("n", [12288, 28672])
+@pytest.mark.parametrize("n", [12288, 20480, 28672])
 def test_one_token_hadamard_linear_in_one_launch(n, M):
     """One or two tokens behind a 1024-point factor and a table of order 12, 20 or 28: qr_quantized_linear_f16 runs the front
     and the dot products in ONE kernel in which every workgroup transforms the rows itself.  Its output must carry the
