@@ -136,3 +136,16 @@ def test_rmsnorm_matches_formula():
 def test_packed_tensor_carrier():
     p = quarot_amd.PackedQuantizedTensor(torch.zeros(3, 4, dtype=torch.uint8), torch.ones(3, 1, dtype=torch.float16))
     assert p.size() == (3, 4) and p.dtype == torch.uint8 and p.device.type == "cpu"
+
+
+def test_native_host_route_raises_hip_errors_and_leaves_refusals_to_the_general_route():
+    """A refusal of the library (negative) sends a call to the Python wrapper's general route.  A HIP error (positive) must be
+    raised at once: the library has cleared it, so the general route's second attempt would report success."""
+    from quarot_amd import _lib, _host
+    assert _host.outcome(0) is True
+    for code in (-1, -2, -3, -4, -7):
+        assert _host.outcome(code) is False
+    for code in (1, 2, 719):
+        with pytest.raises(RuntimeError, match=rf"libquarot_hip: .*\(code {code}\)") as raised:
+            _host.outcome(code)
+        assert _lib.lib().qr_strerror(code).decode() in str(raised.value)
