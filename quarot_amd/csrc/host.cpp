@@ -59,7 +59,14 @@ int device_of(const at::Tensor* t) {
     return d == (int)c10::hip::current_device() ? d : -1;
 }
 void* stream(int device) { return (void*)c10::hip::getCurrentHIPStream((c10::DeviceIndex)device).stream(); }
+// Allocations and launches run without the interpreter's lock: an allocation may have to give memory back first, a launch waits
+// while the queue is full, and other Python threads go on meanwhile.
+struct Unlocked {
+    PyThreadState* const state = PyEval_SaveThread();
+    ~Unlocked() { PyEval_RestoreThread(state); }
+};
 at::Tensor fresh(at::IntArrayRef sizes, at::ScalarType dtype, int device) {
+    const Unlocked unlocked;
     return at::empty(sizes, at::TensorOptions().dtype(dtype).device(at::Device(at::kCUDA, (c10::DeviceIndex)device)));
 }
 void* ptr(const at::Tensor* t) { return t ? t->data_ptr() : nullptr; }
@@ -67,9 +74,18 @@ void* ptr(const at::Tensor* t) { return t ? t->data_ptr() : nullptr; }
 // What a call of the library came to.  Its own refusals are negative codes and leave the case to the general route.  A positive
 // code is a HIP error, which the library has taken off the runtime's record: a second attempt by the general route would
 // report success over it.
-bool done(int rc) {
+bool success(int rc) {
     if (rc > 0) throw std::runtime_error("libquarot_hip: " + std::string(qr_strerror(rc)) + " (code " + std::to_string(rc) + ")");
     return rc == QR_OK;
+}
+template <typename Call>
+bool done(Call&& call) {
+    int rc;
+    {
+        const Unlocked unlocked;
+        rc = call();
+    }
+    return success(rc);
 }
 
 PyObject* none() { Py_RETURN_NONE; }
@@ -155,8 +171,8 @@ PyObject* quantize_rows(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
     double clip;
     if (!r.ok || !arg_float(a[1], &clip)) return none();
     Packed p = packed_for(r, (int)r.x->dim() - 1);
-    if (!done(qr_quantize_rows_f16_i4(r.x->data_ptr(), (float)clip, r.rows, r.n, p.codes.data_ptr(), p.scales.data_ptr(),
-                                      stream(r.device))))
+    if (!done([&] { return qr_quantize_rows_f16_i4(r.x->data_ptr(), (float)clip, r.rows, r.n, p.codes.data_ptr(), p.scales.data_ptr(),
+                                                      stream(r.device)); }))
         return none();
     return wrap2(std::move(p.codes), std::move(p.scales));
     QR_END
@@ -170,7 +186,7 @@ PyObject* rmsnorm(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
     double eps;
     if (!r.ok || !arg_int(a[1], &mean_dim) || !arg_float(a[2], &eps) || mean_dim > 0x7fffffff) return none();
     at::Tensor y = fresh(r.x->sizes(), kHalf, r.device);
-    if (!done(qr_rmsnorm_f16(r.x->data_ptr(), r.rows, r.n, (int)mean_dim, (float)eps, y.data_ptr(), stream(r.device))))
+    if (!done([&] { return qr_rmsnorm_f16(r.x->data_ptr(), r.rows, r.n, (int)mean_dim, (float)eps, y.data_ptr(), stream(r.device)); }))
         return none();
     return wrap(std::move(y));
     QR_END
@@ -185,8 +201,8 @@ PyObject* rmsnorm_quantize(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
     if (!r.ok || r.n % 8 || !arg_int(a[1], &mean_dim) || !arg_float(a[2], &eps) || !arg_float(a[3], &clip) || mean_dim > 0x7fffffff)
         return none();
     Packed p = packed_for(r, (int)r.x->dim() - 1);
-    if (!done(qr_rmsnorm_quantize_f16_i4(r.x->data_ptr(), r.rows, r.n, (int)mean_dim, (float)eps, (float)clip, p.codes.data_ptr(),
-                                         p.scales.data_ptr(), nullptr, stream(r.device))))
+    if (!done([&] { return qr_rmsnorm_quantize_f16_i4(r.x->data_ptr(), r.rows, r.n, (int)mean_dim, (float)eps, (float)clip, p.codes.data_ptr(),
+                                                         p.scales.data_ptr(), nullptr, stream(r.device)); }))
         return none();
     return wrap2(std::move(p.codes), std::move(p.scales));
     QR_END
@@ -204,8 +220,8 @@ PyObject* heads_hadamard_quantize(PyObject*, PyObject* const* a, Py_ssize_t narg
     r.n = heads * 128;
     r.rows = r.x->numel() / r.n;
     Packed p = packed_for(r, (int)r.x->dim() - 2);
-    if (!done(qr_heads_hadamard_quantize_f16_i4(r.x->data_ptr(), r.rows, (int)heads, 128, ptr(hadK), (float)clip, p.codes.data_ptr(),
-                                                p.scales.data_ptr(), nullptr, stream(r.device))))
+    if (!done([&] { return qr_heads_hadamard_quantize_f16_i4(r.x->data_ptr(), r.rows, (int)heads, 128, ptr(hadK), (float)clip, p.codes.data_ptr(),
+                                                                p.scales.data_ptr(), nullptr, stream(r.device)); }))
         return none();
     return wrap2(std::move(p.codes), std::move(p.scales));
     QR_END
@@ -232,8 +248,8 @@ PyObject* hadamard(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
         (mode & ~QR_HAD_FP32) != QR_DTYPE_F16 || !table_arg(a[1], mode, K, r.device, &table))
         return none();
     at::Tensor y = fresh(r.x->sizes(), kHalf, r.device);
-    if (!done(qr_hadamard(r.x->data_ptr(), y.data_ptr(), r.rows, (int)r.n, (int)K, ptr(table), (int)mode, (float)scale,
-                          stream(r.device))))
+    if (!done([&] { return qr_hadamard(r.x->data_ptr(), y.data_ptr(), r.rows, (int)r.n, (int)K, ptr(table), (int)mode, (float)scale,
+                                          stream(r.device)); }))
         return none();
     return wrap(std::move(y));
     QR_END
@@ -250,8 +266,8 @@ PyObject* hadamard_quantize(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
         !arg_float(a[5], &clip) || !table_arg(a[1], mode, K, r.device, &table))
         return none();
     Packed p = packed_for(r, (int)r.x->dim() - 1);
-    if (!done(qr_hadamard_quantize_f16_i4(r.x->data_ptr(), r.rows, (int)r.n, (int)K, ptr(table), (int)mode, (float)scale, (float)clip,
-                                          p.codes.data_ptr(), p.scales.data_ptr(), nullptr, stream(r.device))))
+    if (!done([&] { return qr_hadamard_quantize_f16_i4(r.x->data_ptr(), r.rows, (int)r.n, (int)K, ptr(table), (int)mode, (float)scale, (float)clip,
+                                                          p.codes.data_ptr(), p.scales.data_ptr(), nullptr, stream(r.device)); }))
         return none();
     return wrap2(std::move(p.codes), std::move(p.scales));
     QR_END
@@ -286,8 +302,8 @@ PyObject* linear(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
     const size_t need = qr_workspace_bytes(M, w.N, half_k * 2);
     at::Tensor ws;                                          // (few output tiles: room for the slabs of a K split)
     if (need) ws = fresh({(int64_t)need}, kByte, device);
-    if (!done(qr_linear_i4_f16_ws(q->data_ptr(), sx->data_ptr(), w.w->data_ptr(), w.s->data_ptr(), ptr(w.b), M, w.N, half_k * 2,
-                                  y.data_ptr(), need ? ws.data_ptr() : nullptr, need, stream(device))))
+    if (!done([&] { return qr_linear_i4_f16_ws(q->data_ptr(), sx->data_ptr(), w.w->data_ptr(), w.s->data_ptr(), ptr(w.b), M, w.N, half_k * 2,
+                                                  y.data_ptr(), need ? ws.data_ptr() : nullptr, need, stream(device)); }))
         return none();
     return wrap(std::move(y));
     QR_END
@@ -310,9 +326,9 @@ PyObject* quantized_linear(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
     at::Tensor y = fresh(sizes, kHalf, r.device);
     const size_t need = qr_quantized_linear_workspace_bytes(r.rows, w.N, r.n);
     at::Tensor ws = fresh({(int64_t)(need < 16 ? 16 : need)}, kByte, r.device);
-    if (!done(qr_quantized_linear_f16(r.x->data_ptr(), r.rows, r.n, (int)K, ptr(table), (int)mode, (float)scale, (float)clip,
-                                      w.w->data_ptr(), w.s->data_ptr(), ptr(w.b), w.N, y.data_ptr(), ws.data_ptr(), need,
-                                      stream(r.device))))
+    if (!done([&] { return qr_quantized_linear_f16(r.x->data_ptr(), r.rows, r.n, (int)K, ptr(table), (int)mode, (float)scale, (float)clip,
+                                                      w.w->data_ptr(), w.s->data_ptr(), ptr(w.b), w.N, y.data_ptr(), ws.data_ptr(), need,
+                                                      stream(r.device)); }))
         return none();
     return wrap(std::move(y));
     QR_END
@@ -357,7 +373,7 @@ PyObject* page_tables(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
     at::Tensor indptr = fresh({batch + 1}, at::kInt, device);
     at::Tensor indices = fresh({batch * ((length + page - 1) / page)}, at::kInt, device);
     at::Tensor last = fresh({batch}, at::kInt, device);
-    if (!done(qr_page_tables(batch, length, (int)page, indptr.data_ptr(), indices.data_ptr(), last.data_ptr(), stream(device))))
+    if (!done([&] { return qr_page_tables(batch, length, (int)page, indptr.data_ptr(), indices.data_ptr(), last.data_ptr(), stream(device)); }))
         return none();
     PyObject* t = PyTuple_New(3);
     if (!t) return nullptr;
@@ -387,9 +403,9 @@ PyObject* quantize_append(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
     const int64_t tokens = k->size(0);
     if (seq ? (seq->dim() != 1 || seq->numel() != c.batch + 1) : tokens != c.batch) return none();
     const int had = PyObject_IsTrue(a[9]);
-    if (!done(qr_kv_quant_append_f16_i4(k->data_ptr(), v->data_ptr(), tokens, ptr(seq), had ? 1 : 0, c.data->data_ptr(), c.param->data_ptr(),
-                                        c.indptr->data_ptr(), c.indices->data_ptr(), c.last->data_ptr(), c.pages, c.layers, (int)layer, c.heads,
-                                        c.page_size, 128, c.batch, stream(device))))
+    if (!done([&] { return qr_kv_quant_append_f16_i4(k->data_ptr(), v->data_ptr(), tokens, ptr(seq), had ? 1 : 0, c.data->data_ptr(), c.param->data_ptr(),
+                                                        c.indptr->data_ptr(), c.indices->data_ptr(), c.last->data_ptr(), c.pages, c.layers, (int)layer, c.heads,
+                                                        c.page_size, 128, c.batch, stream(device)); }))
         return none();
     Py_RETURN_TRUE;
     QR_END
@@ -416,10 +432,10 @@ PyObject* decode_step(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
     if (need && !kept) own = fresh({(int64_t)need}, kByte, device);
     const int qh = (PyObject_IsTrue(a[9]) ? 1 : 0) | (kept ? QR_DECODE_COUNTERS_ZERO : 0), kh = PyObject_IsTrue(a[10]) ? 1 : 0;
     at::Tensor o = fresh(q->sizes(), kHalf, device);
-    if (!done(qr_kv_quant_append_batch_decode_f16_i4(o.data_ptr(), q->data_ptr(), qh, k->data_ptr(), v->data_ptr(), kh, c.data->data_ptr(),
-                                                     c.param->data_ptr(), c.indptr->data_ptr(), c.indices->data_ptr(), c.last->data_ptr(),
-                                                     c.pages, c.layers, (int)layer, c.heads, c.page_size, 128, c.batch, bound,
-                                                     kept ? ws->data_ptr() : need ? own.data_ptr() : nullptr, need, stream(device))))
+    if (!done([&] { return qr_kv_quant_append_batch_decode_f16_i4(o.data_ptr(), q->data_ptr(), qh, k->data_ptr(), v->data_ptr(), kh, c.data->data_ptr(),
+                                                                     c.param->data_ptr(), c.indptr->data_ptr(), c.indices->data_ptr(), c.last->data_ptr(),
+                                                                     c.pages, c.layers, (int)layer, c.heads, c.page_size, 128, c.batch, bound,
+                                                                     kept ? ws->data_ptr() : need ? own.data_ptr() : nullptr, need, stream(device)); }))
         return none();
     return wrap(std::move(o));
     QR_END
@@ -430,7 +446,7 @@ PyObject* outcome(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
     QR_ARGS(1)
     long long rc;
     if (!arg_int(a[0], &rc)) return none();
-    return PyBool_FromLong(done((int)rc));
+    return PyBool_FromLong(success((int)rc));
     QR_END
 }
 

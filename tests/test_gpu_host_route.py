@@ -136,3 +136,33 @@ def test_decode_workspace_made_under_capture_is_not_kept():
         want = run(caches[1])
         assert torch.equal(captured, want)
     assert torch.equal(run(caches[0]), run(caches[1])) and caches[0]._decode_ws is not None
+
+
+def test_other_threads_run_while_the_host_route_launches():
+    """With a switch interval that never ends, another Python thread gets on only when this one gives the interpreter's lock away:
+    at each allocation and launch, as around ctypes' calls."""
+    import sys
+    import threading
+    import time
+    x = torch.randn(4, 128, device="cuda").half()
+    host.quantize_rows(x, 1.0)
+    turns, stop, started, interval = [0], threading.Event(), threading.Event(), sys.getswitchinterval()
+
+    def other():
+        started.set()
+        while not stop.is_set():
+            turns[0] += 1
+            time.sleep(0)
+
+    thread = threading.Thread(target=other, daemon=True)
+    sys.setswitchinterval(1e4)
+    try:
+        thread.start()
+        assert started.wait(30)
+        before = turns[0]
+        kept = [host.quantize_rows(x, 1.0) for _ in range(200)]               # (freeing a tensor may give the lock away too)
+        assert turns[0] - before >= len(kept)
+    finally:
+        stop.set()
+        sys.setswitchinterval(interval)
+        thread.join(30)
