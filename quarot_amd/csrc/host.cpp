@@ -156,6 +156,13 @@ bool arg_float(PyObject* o, double* v) {
     return true;
 }
 
+bool arg_bool(PyObject* o, bool* v) {
+    const int truth = PyObject_IsTrue(o);
+    if (truth < 0) PyErr_Clear();
+    *v = truth > 0;
+    return truth >= 0;
+}
+
 #define QR_ARGS(COUNT)                                                     \
     if (nargs != (COUNT)) {                                                \
         PyErr_SetString(PyExc_TypeError, "expected " #COUNT " arguments"); \
@@ -395,14 +402,14 @@ PyObject* quantize_append(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
     QR_ARGS(10)
     const int device = device_of(tensor(a[0]));
     long long layer;
+    bool had;
     Cache c;
-    if (!arg_int(a[8], &layer) || !cache_args(a, device, layer, &c)) return none();
+    if (!arg_int(a[8], &layer) || !arg_bool(a[9], &had) || !cache_args(a, device, layer, &c)) return none();
     const at::Tensor *k = tensor(a[5]), *v = tensor(a[6]), *seq;
     if (!plain(k, kHalf, device) || !plain(v, kHalf, device) || !plain_or_none(a[7], at::kInt, device, &seq)) return none();
     if (k->dim() != 3 || k->sizes() != v->sizes() || k->size(1) != c.heads || k->size(2) != 128 || k->numel() == 0) return none();
     const int64_t tokens = k->size(0);
     if (seq ? (seq->dim() != 1 || seq->numel() != c.batch + 1) : tokens != c.batch) return none();
-    const int had = PyObject_IsTrue(a[9]);
     if (!done([&] { return qr_kv_quant_append_f16_i4(k->data_ptr(), v->data_ptr(), tokens, ptr(seq), had ? 1 : 0, c.data->data_ptr(), c.param->data_ptr(),
                                                         c.indptr->data_ptr(), c.indices->data_ptr(), c.last->data_ptr(), c.pages, c.layers, (int)layer, c.heads,
                                                         c.page_size, 128, c.batch, stream(device)); }))
@@ -417,8 +424,11 @@ PyObject* decode_step(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
     QR_ARGS(13)
     const int device = device_of(tensor(a[0]));
     long long layer, bound;
+    bool q_had, k_had;
     Cache c;
-    if (!arg_int(a[8], &layer) || !arg_int(a[11], &bound) || !cache_args(a, device, layer, &c)) return none();
+    if (!arg_int(a[8], &layer) || !arg_bool(a[9], &q_had) || !arg_bool(a[10], &k_had) || !arg_int(a[11], &bound) ||
+        !cache_args(a, device, layer, &c))
+        return none();
     const at::Tensor *q = tensor(a[5]), *k = tensor(a[6]), *v = tensor(a[7]), *ws;
     if (!plain(q, kHalf, device) || !plain(k, kHalf, device) || !plain(v, kHalf, device) || !plain_or_none(a[12], kByte, device, &ws))
         return none();
@@ -430,7 +440,7 @@ PyObject* decode_step(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
     const bool kept = need && ws && (size_t)ws->numel() >= need;
     at::Tensor own;
     if (need && !kept) own = fresh({(int64_t)need}, kByte, device);
-    const int qh = (PyObject_IsTrue(a[9]) ? 1 : 0) | (kept ? QR_DECODE_COUNTERS_ZERO : 0), kh = PyObject_IsTrue(a[10]) ? 1 : 0;
+    const int qh = (q_had ? 1 : 0) | (kept ? QR_DECODE_COUNTERS_ZERO : 0), kh = k_had ? 1 : 0;
     at::Tensor o = fresh(q->sizes(), kHalf, device);
     if (!done([&] { return qr_kv_quant_append_batch_decode_f16_i4(o.data_ptr(), q->data_ptr(), qh, k->data_ptr(), v->data_ptr(), kh, c.data->data_ptr(),
                                                                      c.param->data_ptr(), c.indptr->data_ptr(), c.indices->data_ptr(), c.last->data_ptr(),

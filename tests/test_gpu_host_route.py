@@ -166,3 +166,15 @@ def test_other_threads_run_while_the_host_route_launches():
         stop.set()
         sys.setswitchinterval(interval)
         thread.join(30)
+
+
+def test_a_flag_without_a_truth_value_raises_its_own_error():
+    """As the general route does, with nothing stored: not a launch followed by a SystemError."""
+    c = kv.MultiLayerPagedKVCache4Bit(1, 16, 16, "cuda", 1, 2, 128)
+    c.length = 1
+    c.pages.zero_()
+    tables = c.get_cache_specs_for_flash_infer(None)
+    x = torch.randn(1, 2, 128, device="cuda").half()
+    with pytest.raises(RuntimeError, match="[Bb]oolean value"):
+        kv.quantize_append_kv_i4(**tables, k=x, v=x, seqlen_indptr=None, layer_idx=0, hadamard=torch.ones(2))
+    assert int(c.pages.max()) == 0
