@@ -300,10 +300,17 @@ class _AttentionStub(object):
         self.hadamard_dtype = hadamard_dtype
 
     def forward(self, q, num_kv_heads, attention_kwargs, layer_idx, max_seq_len=0, workspace=None, take_pending=None):
-        batch_size, q_len, num_qo_heads, head_dim = q.shape
-        assert q_len == 1
-        # the step's new token, if the cache still holds it back for this call (see MultiLayerPagedKVCache4Bit.update)
+        assert q.shape[1] == 1
+        # the step's new token, if the cache still holds it back for this call (see MultiLayerPagedKVCache4Bit.update); a call
+        # that raises leaves it there
         append = take_pending() if take_pending is not None else None
+        o = self._attend(q, attention_kwargs, layer_idx, max_seq_len, workspace, append)
+        if append is not None:
+            take_pending(stored=True)
+        return o
+
+    def _attend(self, q, attention_kwargs, layer_idx, max_seq_len, workspace, append):
+        batch_size, _, num_qo_heads, head_dim = q.shape
         if append is not None and self.hadamard_dtype in (None, torch.float16):
             s = attention_kwargs
             o = _lib.host.decode_step(s["kv_data"], s["kv_param"], s["kv_indptr"], s["kv_indices"], s["last_page_offset"], q,
@@ -384,11 +391,12 @@ class MultiLayerPagedKVCache4Bit:
                 quantize_append_kv_i4(**specs, k=k.view(k.shape[0], *k.shape[-2:]), v=v.view(v.shape[0], *v.shape[-2:]),
                                       seqlen_indptr=None, layer_idx=layer, hadamard=hadamard)
 
-    def _take_pending(self, layer_idx, token):
+    def _take_pending(self, layer_idx, token, stored=False):
         held = self._pending.get(layer_idx)
         if held is None or held[0] is not token:
             return None                          # stored meanwhile (or this callable was used before): plain attention
-        del self._pending[layer_idx]
+        if stored:
+            del self._pending[layer_idx]
         return held[1], held[2], held[4]
 
     def _decode_workspace(self, num_heads):

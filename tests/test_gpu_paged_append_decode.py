@@ -246,3 +246,24 @@ def test_decode_attention_is_as_exact_in_every_dimension(B, S, heads):
     even, odd = float(off[..., 0::2].double().mean()), float(off[..., 1::2].double().mean())
     assert odd < 0.2 and even <= 1.2 * odd + 4 * (2 * odd / (B * heads * 64)) ** 0.5, (even, odd)
     assert float((out - want).norm() / want.norm()) < 3e-4              # fp16 rounding alone: 2.1e-4
+
+
+@pytest.mark.parametrize("hadamard_dtype", [torch.float16, None])
+def test_a_step_whose_attention_call_raises_keeps_its_token(hadamard_dtype):
+    """update() has accepted the step's key and value; a query that the attention call refuses must not lose them: the pages hold
+    the token afterwards, and the call can be made again."""
+    rng = np.random.default_rng(4)
+    k0, v0, k, v, q = (gpu(synth_kv(rng, n, 3)).view(1, n, 3, 128) for n in (5, 5, 1, 1, 1))
+    caches = [kv.MultiLayerPagedKVCache4Bit(1, 4, 8, "cuda:0", 1, 3, 128, hadamard_dtype=hadamard_dtype) for _ in range(3)]
+    calls = []
+    for c in caches:
+        c.pages.zero_(), c.scales.zero_()
+        c.update(k0, v0, 0)
+        calls.append(c.update(k, v, 0))
+    for bad in (q[:, :, :2].contiguous(), q[..., :64].contiguous(), q.double()):
+        for call in calls[:2]:
+            with pytest.raises(Exception):
+                call(bad)
+    assert torch.equal(calls[0](q), calls[2](q))
+    for c in caches[:2]:                                                # after the repeated call, and without one
+        assert torch.equal(c.pages, caches[2].pages) and torch.equal(c.scales, caches[2].scales)
