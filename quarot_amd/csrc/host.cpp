@@ -13,6 +13,7 @@
 #include <c10/hip/HIPFunctions.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/hip/HIPStream.h>
+#include <hip/hip_runtime_api.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
@@ -397,6 +398,21 @@ PyObject* page_tables(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
     QR_END
 }
 
+// capture_id(reference tensor on the device) -> the number of the graph capture that the device's current stream is part of; None
+// outside a capture
+PyObject* capture_id(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
+    QR_ARGS(1)
+    const int device = device_of(tensor(a[0]));
+    if (device < 0) return none();
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    unsigned long long id = 0;
+    const hipError_t e = hipStreamGetCaptureInfo((hipStream_t)stream(device), &status, &id);
+    success((int)e);
+    if (status != hipStreamCaptureStatusActive) return none();
+    return PyLong_FromUnsignedLongLong(id);
+    QR_END
+}
+
 // quantize_append(kv_data, kv_param, indptr, indices, last, k, v, seqlen_indptr or None, layer, hadamard) -> True
 PyObject* quantize_append(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
     QR_ARGS(10)
@@ -470,6 +486,7 @@ PyMethodDef methods[] = {QR_METHOD(quantize_rows),
                          QR_METHOD(linear),
                          QR_METHOD(quantized_linear),
                          QR_METHOD(page_tables),
+                         QR_METHOD(capture_id),
                          QR_METHOD(quantize_append),
                          QR_METHOD(decode_step),
                          QR_METHOD(outcome),

@@ -304,6 +304,7 @@ class _AttentionStub(object):
         # the step's new token, if the cache still holds it back for this call (see MultiLayerPagedKVCache4Bit.update); a call
         # that raises leaves it there
         append = take_pending() if take_pending is not None else None
+        workspace = workspace() if workspace is not None else None
         o = self._attend(q, attention_kwargs, layer_idx, max_seq_len, workspace, append)
         if append is not None:
             take_pending(stored=True)
@@ -335,6 +336,9 @@ class _AttentionStub(object):
         return attn_output.unsqueeze(1)
 
 
+_MAX_WORKSPACES = 8      # streams whose decode workspace a cache keeps
+
+
 class MultiLayerPagedKVCache4Bit:
     """Paged int4 KV cache of all layers with the interface of kv_cache.py:132-289: `update` quantises
     and stores the new keys and values (the first call per layer takes the whole prompt and returns the
@@ -357,6 +361,9 @@ class MultiLayerPagedKVCache4Bit:
         self._scales = torch.empty((max_page_cnt * batch_size, n_layers, 2, num_heads, page_size, 2), dtype=torch.float16,
                                    device=device)
         self._pending = {}      # layer -> (token, k, v, specs, hadamard): a decode step's new token, held for the attention call
+        self._workspaces = {}           # stream -> (key, workspace), see _decode_workspace
+        self._captured_ws = {}          # the same for the capture under way
+        self._decode_ws = None          # the workspace of the last eager step
         self.max_seq_len = max_seq_len
         self._needs_init = [True] * n_layers
         self.length = 0
@@ -399,24 +406,38 @@ class MultiLayerPagedKVCache4Bit:
             del self._pending[layer_idx]
         return held[1], held[2], held[4]
 
-    def _decode_workspace(self, num_heads):
-        """Scratch for decode attention split along the sequence, kept with the cache (every layer of every decode
-        step would otherwise allocate its own): sized for the longer of the current and the maximum length.  Zeroed when
-        it is made: every launch leaves its arrival counters at zero.  One made while a graph is captured is zeroed by that
-        graph's replays only, so it is not kept."""
-        key = (self.length, num_heads)
-        if getattr(self, "_decode_ws_key", None) == key:
-            return self._decode_ws
+    def _decode_workspace(self, num_heads, length):
+        """Scratch for decode attention split along the sequence, for a launch on the current stream.  It is kept with the cache
+        (every layer of every decode step would otherwise allocate its own), one per stream, since it holds partial states
+        and arrival counters: launches of one stream follow each other and leave the counters at zero, launches of two may
+        overlap.  Sized for the longer of the given and the maximum length, zeroed when it is made.  One made while a graph is
+        captured is zeroed by that graph's replays only, and only they may use it: it is kept for the rest of that capture."""
         dev = self._pages.device
         with _lib.on_device(dev):
+            stream, capturing = _lib.stream_ptr(dev), torch.cuda.is_current_stream_capturing()
+            # (a refused capture_id: a number of its own, so nothing is found again)
+            key = (num_heads, length, (_lib.host.capture_id(self._pages) or object()) if capturing else None)
+            kept = self._captured_ws if capturing else self._workspaces
+            found = kept.get(stream)
+            if found is not None and found[0] == key:
+                if not capturing:
+                    self._decode_ws = found[1]
+                return found[1]
             need = max((_decode_workspace_bytes(self.batch_size, num_heads, int(n), dev.index)
-                        for n in (self.length, self.max_seq_len) if n), default=0)
-        ws = getattr(self, "_decode_ws", None)
-        if need and (ws is None or ws.numel() < need):
-            ws = torch.zeros((need,), dtype=torch.uint8, device=dev)
-            if torch.cuda.is_current_stream_capturing():
-                return ws
-        self._decode_ws, self._decode_ws_key = ws, key
+                        for n in (length, self.max_seq_len) if n), default=0)
+            ws = found[1] if found is not None and found[0][2] == key[2] and found[0][0] == num_heads else None
+            if need and (ws is None or ws.numel() < need):
+                ws = torch.empty((need,), dtype=torch.uint8, device=dev)
+                ws[:4 * self.batch_size * num_heads].zero_()           # the counters
+        if capturing:
+            self._captured_ws = {stream: (key, ws)}
+            return ws
+        self._captured_ws = {}
+        kept = {s: w for s, w in kept.items() if s != stream}
+        while len(kept) >= _MAX_WORKSPACES:                            # (allocated and used on its own stream: freed behind its launches)
+            kept.pop(next(iter(kept)))
+        kept[stream] = (key, ws)
+        self._workspaces, self._decode_ws = kept, ws
         return ws
 
     def _ensure_page_cnt_per_batch(self, expected_page_cnt_per_batch):
@@ -477,7 +498,8 @@ class MultiLayerPagedKVCache4Bit:
                                   seqlen_indptr=None, layer_idx=layer_idx, hadamard=fused_had)
             take = None
         return functools.partial(self._stub.forward, num_kv_heads=num_heads, attention_kwargs=specs, layer_idx=layer_idx,
-                                 max_seq_len=self.length, workspace=self._decode_workspace(num_heads), take_pending=take)
+                                 max_seq_len=self.length, workspace=functools.partial(self._decode_workspace, num_heads, self.length),
+                                 take_pending=take)
 
     def _update_f16(self, key_states, value_states, layer_idx, attention_mask, first, specs):
         """update() with fp16 pages (kv_cache.py:187-251 with disable_quant): the transformed keys and the values are

@@ -178,3 +178,93 @@ def test_a_flag_without_a_truth_value_raises_its_own_error():
     with pytest.raises(RuntimeError, match="[Bb]oolean value"):
         kv.quantize_append_kv_i4(**tables, k=x, v=x, seqlen_indptr=None, layer_idx=0, hadamard=torch.ones(2))
     assert int(c.pages.max()) == 0
+
+
+def _decode_caches(n, length=2048, heads=4):
+    """Caches that hold the same prompt, and tensors of some decode steps; steps of this length are split over workgroups."""
+    g = torch.Generator(device="cuda").manual_seed(5)
+    rnd = lambda t: torch.randn(1, t, heads, 128, generator=g, device="cuda").half()
+    k0, v0, steps = rnd(length), rnd(length), [[rnd(1) for _ in range(3)] for _ in range(4)]
+    caches = [kv.MultiLayerPagedKVCache4Bit(1, 16, length + 52, "cuda", 1, heads, 128) for _ in range(n)]
+    for c in caches:
+        c.pages.zero_(), c.scales.zero_()
+        c.update(k0, v0, 0)
+    assert kv._decode_workspace_bytes(1, heads, length + 1, 0) > 0
+    return caches, steps
+
+
+class _Spy:
+    """The host module, with a record of the workspaces that decode steps were launched with."""
+
+    def __init__(self):
+        self.workspaces = []
+
+    def __getattr__(self, name):
+        return getattr(host, name)
+
+    def decode_step(self, *args):
+        self.workspaces.append(args[12])
+        return host.decode_step(*args)
+
+
+@pytest.fixture
+def spy(monkeypatch):
+    monkeypatch.setattr(_lib, "host", _Spy())
+    return _lib.host
+
+
+def test_decode_workspaces_of_two_streams_are_two(spy):
+    """A workspace holds partial states and arrival counters; launches of different streams may overlap, so they share none, and
+    what an overlap would leave in one stream's counters does not reach another stream's steps."""
+    (a, b), steps = _decode_caches(2)
+    streams, got = [torch.cuda.Stream() for _ in range(2)], []
+    torch.cuda.synchronize()
+    for i, s in enumerate(steps):
+        with torch.cuda.stream(streams[1 - i % 2]):
+            call = a.update(s[0], s[1], 0)
+        torch.cuda.synchronize()
+        with torch.cuda.stream(streams[i % 2]):                        # (the stream of the call counts, not update's)
+            got.append(call(s[2]))
+        torch.cuda.synchronize()
+        if i == 1:
+            spy.workspaces[1][:16] = 1                                 # (the fourth step, on that stream, is not looked at)
+    ws = list(spy.workspaces)
+    want = [b.update(s[0], s[1], 0)(s[2]) for s in steps[:3]]
+    assert all(torch.equal(x, y) for x, y in zip(got, want))
+    assert ws[0] is ws[2] and ws[1] is ws[3] and ws[0].data_ptr() != ws[1].data_ptr()
+    for _ in range(2 * kv._MAX_WORKSPACES):
+        with torch.cuda.stream(torch.cuda.Stream()):
+            a.length -= 1
+            a.update(steps[0][0], steps[0][1], 0)(steps[0][2])
+    torch.cuda.synchronize()
+    assert len(a._workspaces) <= kv._MAX_WORKSPACES
+
+
+def test_a_captured_decode_step_has_its_own_workspace(spy):
+    """Replays may overlap eager steps of any stream: a graph uses no workspace of an eager step or of another graph, one for all
+    the layers of a capture, and zeroes its counters itself."""
+    (a, b), steps = _decode_caches(2)
+    run = lambda c, s: c.update(s[0], s[1], 0)(s[2])
+
+    def captured(s):
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            a.length -= 1
+            out = [run(a, s)]
+            a.length -= 1                                              # (a second layer, as far as the workspace goes)
+            out.append(run(a, s))
+        return graph, out
+
+    assert torch.equal(run(a, steps[0]), run(b, steps[0]))
+    one, out = captured(steps[1])
+    two, _ = captured(steps[1])
+    eager, _, ws, same, other = spy.workspaces[:5]
+    assert ws is same and len({t.data_ptr() for t in (eager, ws, other)}) == 3
+    eager[:16] = 1                                                     # a step of another stream in flight
+    b.length -= 1
+    want = run(b, steps[1])
+    for _ in range(3):
+        ws[:16] = 1                                                    # whatever its memory held
+        one.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out[0], want) and torch.equal(out[1], want)
