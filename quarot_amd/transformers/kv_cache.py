@@ -364,6 +364,7 @@ class MultiLayerPagedKVCache4Bit:
         self._workspaces = {}           # stream -> (key, workspace), see _decode_workspace
         self._captured_ws = {}          # the same for the capture under way
         self._decode_ws = None          # the workspace of the last eager step
+        self._captured_specs = None     # page tables of the capture under way
         self.max_seq_len = max_seq_len
         self._needs_init = [True] * n_layers
         self.length = 0
@@ -406,6 +407,13 @@ class MultiLayerPagedKVCache4Bit:
             del self._pending[layer_idx]
         return held[1], held[2], held[4]
 
+    def _capture(self):
+        """The graph capture that the current stream is part of: its number (one that no other capture equals where the native
+        host side cannot tell), None outside one."""
+        if not (self._pages.is_cuda and torch.cuda.is_current_stream_capturing()):
+            return None
+        return _lib.host.capture_id(self._pages) or object()
+
     def _decode_workspace(self, num_heads, length):
         """Scratch for decode attention split along the sequence, for a launch on the current stream.  It is kept with the cache
         (every layer of every decode step would otherwise allocate its own), one per stream, since it holds partial states
@@ -414,13 +422,12 @@ class MultiLayerPagedKVCache4Bit:
         captured is zeroed by that graph's replays only, and only they may use it: it is kept for the rest of that capture."""
         dev = self._pages.device
         with _lib.on_device(dev):
-            stream, capturing = _lib.stream_ptr(dev), torch.cuda.is_current_stream_capturing()
-            # (a refused capture_id: a number of its own, so nothing is found again)
-            key = (num_heads, length, (_lib.host.capture_id(self._pages) or object()) if capturing else None)
-            kept = self._captured_ws if capturing else self._workspaces
+            stream, capture = _lib.stream_ptr(dev), self._capture()
+            key = (num_heads, length, capture)
+            kept = self._workspaces if capture is None else self._captured_ws
             found = kept.get(stream)
             if found is not None and found[0] == key:
-                if not capturing:
+                if capture is None:
                     self._decode_ws = found[1]
                 return found[1]
             need = max((_decode_workspace_bytes(self.batch_size, num_heads, int(n), dev.index)
@@ -429,7 +436,7 @@ class MultiLayerPagedKVCache4Bit:
             if need and (ws is None or ws.numel() < need):
                 ws = torch.empty((need,), dtype=torch.uint8, device=dev)
                 ws[:4 * self.batch_size * num_heads].zero_()           # the counters
-        if capturing:
+        if capture is not None:
             self._captured_ws = {stream: (key, ws)}
             return ws
         self._captured_ws = {}
@@ -533,9 +540,11 @@ class MultiLayerPagedKVCache4Bit:
             self._flush()
         if attention_mask is None:
             # every sequence holds self.length tokens: the tables depend on that number alone and are built
-            # once per length (every layer of a decode step asks for them), by one launch
-            cached = getattr(self, "_specs", None)
-            if cached is not None and cached[0] == self.length:
+            # once per length (every layer of a decode step asks for them), by one launch.  Those of a capture are filled by
+            # its replays only, and it reads no others, which an eager step of another length would free.
+            capture = self._capture()
+            cached = self._captured_specs if capture is not None else getattr(self, "_specs", None)
+            if cached is not None and cached[0] == self.length and (capture is None or cached[2] == capture):
                 return cached[1]
             tables = _lib.host.page_tables(self.batch_size, self.length, self.page_size, self._pages)
             if tables is None:                   # an empty cache, or one on another than the current device
@@ -548,7 +557,10 @@ class MultiLayerPagedKVCache4Bit:
                           torch.full((self.batch_size,), ptr, dtype=torch.int32, device=self.device))
             specs = {"kv_data": self._pages, "kv_indptr": tables[0], "kv_indices": tables[1], "last_page_offset": tables[2],
                      "kv_param": self._scales}
-            self._specs = (self.length, specs)
+            if capture is None:
+                self._specs, self._captured_specs = (self.length, specs), None
+            else:
+                self._captured_specs = (self.length, specs, capture)
             return specs
         seqlens_in_batch = attention_mask.sum(dim=-1, dtype=torch.int32)
         page_cnt = self.page_cnt_from_length(seqlens_in_batch)

@@ -268,3 +268,29 @@ def test_a_captured_decode_step_has_its_own_workspace(spy):
         one.replay()
         torch.cuda.synchronize()
         assert torch.equal(out[0], want) and torch.equal(out[1], want)
+
+
+def test_page_tables_made_under_capture_are_that_graphs_own():
+    """They are filled by replays only: an eager step at that length that comes first makes its own, and the graph reads none of an
+    eager step, whose memory goes back when the cache grows."""
+    (a, b), steps = _decode_caches(2)
+    tables = lambda c: [c.get_cache_specs_for_flash_infer(None)[n] for n in ("kv_indptr", "kv_indices", "last_page_offset")]
+    eager = tables(a)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        inside, again = tables(a), tables(a)
+        a.length += 1
+        longer = tables(a)
+        out = a._stub.forward(steps[0][2], 4, a.get_cache_specs_for_flash_infer(None), 0, a.length)
+        a.length -= 1
+    assert all(x is y for x, y in zip(inside, again)) and not any(x is y for x, y in zip(inside, eager))
+    a.length += 1
+    for x, y in zip(tables(a), longer):                                # no replay yet
+        assert x is not y
+    b.length += 1
+    assert all(torch.equal(x, y) for x, y in zip(tables(a), tables(b)))
+    want = b._stub.forward(steps[0][2], 4, b.get_cache_specs_for_flash_infer(None), 0, b.length)
+    for _ in range(3):
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want) and all(torch.equal(x, y) for x, y in zip(longer, tables(b)))
