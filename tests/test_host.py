@@ -149,3 +149,22 @@ def test_native_host_route_raises_hip_errors_and_leaves_refusals_to_the_general_
         with pytest.raises(RuntimeError, match=rf"libquarot_hip: .*\(code {code}\)") as raised:
             _host.outcome(code)
         assert _lib.lib().qr_strerror(code).decode() in str(raised.value)
+
+
+def test_package_works_without_the_native_host_route(monkeypatch):
+    """A _host.so that is missing or does not fit the installed torch costs host time, not function: its functions refuse, with a
+    warning, and the wrappers' general route decides; torch-only modules run."""
+    import sys
+    from quarot_amd import _lib
+    monkeypatch.setitem(sys.modules, "quarot_amd._host", None)             # `import` raises ImportError
+    host = _lib._HostOnUse()
+    with pytest.warns(UserWarning, match="_host.so"):
+        assert host.linear(1, 2, 3) is None
+    monkeypatch.setattr(quarot_amd, "_host", host)
+    monkeypatch.setattr(_lib, "host", host)
+    x = torch.randn(3, 16, dtype=torch.float16)
+    with pytest.warns(UserWarning, match="_host.so"):
+        y = quarot_amd.nn.RMSNorm(16)(x)
+    np.testing.assert_allclose(y.numpy(), o.rmsnorm(x.numpy(), 16, 1e-5), rtol=1e-3, atol=1e-3)
+    with pytest.warns(UserWarning, match="_host.so"), pytest.raises(RuntimeError, match="GPU|CUDA|cuda"):
+        quarot_amd.nn.Quantizer()(x)                                       # the general route's own error
