@@ -287,48 +287,11 @@ def mfma_ceiling(seconds):
     return res
 
 
-def gemm_kernel_name(m, n, k=0):
-    groups = (n + 31) // 32                # the library's choice: enough groups of 32 rows to give every CU a workgroup
-    xs = any((groups + rg - 1) // rg >= 192 for rg in range(4, 9))
-    if m == 1 or (m <= 4 and not xs):
-        return "gemv_i4_kernel"
-    if m <= 64:
-        if xs or m < 8:
-            return "decode_xs_kernel" if xs else "decode_i4_kernel"
-        # the library's estimate (gemm.hip, decode_plan) on 256 CUs: the barrier-free kernel against 64 x 64 tiles, K whole or sliced
-        st, t64 = (max(k, 256) + 255) // 256, (n + 63) // 64
-        best, slices = 3.0 + st * (0.12 + 0.0028 * m) + (1.2 if m > 32 else 0.0), 0
-        if n > 8192:
-            best = 3.0 + (best * (0.8 + n / 12500) - 3.0) * min(1.0, st / 16)
-        elif n > 4096 and st > 24:
-            best += 3.5 * (n - 4096) / 4096
-        for ks in range(1, 9):
-            wgs = t64 * ks
-            if ks > 1 and (ks > st // 4 or wgs > 256 or not (t64 * 3 <= 256 or (m >= 40 and k >= 16384))):
-                break
-            slope = 0.235 + 0.0009 * m if wgs <= 128 else 0.28 + 0.002 * m if wgs <= 256 else (0.25 + 0.0012 * m) * ((wgs + 255) // 256)
-            t = 4.4 + max((st + ks - 1) // ks * slope, n * (k / 2) / 6.2e6)
-            t += 2.5 + 0.3 * max(0, ks - 3) + 2.0 * ks * m * n / 1e6 + (4.0 if n % 4 else 0.0) if ks > 1 else 0.0
-            if t < best:
-                best, slices = t, ks
-        return ("decode_i4_kernel", "gemm_mid_kernel<64,64>")[slices > 0] + (" (K sliced) + dequant_slabs_kernel" if slices > 1 else "")
-    # the library's estimate (gemm.hip, mid_plan) for its tile shapes on 256 CUs, in microseconds
-    st = (max(k, 256) + 255) // 256
-    tiles = lambda bm, bn: ((m + bm - 1) // bm) * ((n + bn - 1) // bn)
-    load = lambda t: (t + 255) // 256
-    n64, n128, nsq = load(tiles(64, 64)), load(tiles(64, 128)), load(tiles(128, 128))
-    est = [(4.2 + st * {1: 0.26, 2: 0.44}.get(n64, (0.27 if n64 >= 5 and st > 32 else 0.25 if n64 < 8 else 0.26) * n64), "gemm_mid_kernel<64,64>"),
-           (4.6 + st * (0.41 if n128 == 1 else 0.52 * n128), "gemm_mid_kernel<64,128>"),
-           (5.0 + st * (0.8 if nsq == 1 else 0.92 * nsq), "gemm_mid_kernel<128,128>")]
-    tall = min((2, 1, 0), key=lambda i: load(tiles(128 + 64 * i, 256)) * (0.57, 0.80, 1.0)[i])      # ties: the taller tile
-    t = tiles(128 + 64 * tall, 256)
-    est.append((load(t) * (5.5 + (1.40, 2.19, 2.75)[tall] * st * (1 - (0.5 if tall else 0.3) * (1 - t / (load(t) * 256)))),
-                "gemm_sp256_kernel" if tall else "gemm_spk_kernel"))
-    whole, left = divmod(tiles(256, 256), 256)
-    if k % 256 == 0 and whole and 0 < left <= 128:
-        est.append(((1.06 if tall == 1 else 1.0) * (whole * (5.5 + 2.75 * st) + 5.5 + 1.4 * st * (1 - 0.3 * (1 - left / 128))),
-                    "gemm_sp256_tail_kernel"))
-    return min(est, key=lambda e: e[0])[1]
+def gemm_kernel_name(m, n, k):
+    """The library's own choice for a linear layer of this shape."""
+    from quarot_amd import _lib
+    L = _lib.lib()
+    return L.qr_linear_plan(m, n, k, L.qr_workspace_bytes(m, n, k), None).decode()
 
 
 FRONT_KERNEL = {"had": "hadamard kernel + quantiser (fused)", "had32": "hadamard kernel in fp32 precision + quantiser (fused)",

@@ -199,6 +199,10 @@ int qr_linear_i4_f16(const void* A, const void* sA, const void* W, const void* s
  *   bit either way (integer partial sums).  Calls that share a workspace must not overlap.
  */
 size_t qr_workspace_bytes(int64_t M, int64_t N, int64_t K);
+/* The kernel (and a second one that adds slices of K, if any) that qr_linear_i4_f16_ws launches for a shape with that much
+ * workspace on the current device, as text for reports; NULL for a shape that it refuses.  *scratch_bytes (optional): how much
+ * of the workspace they use; a workspace of that size selects the same kernels. */
+const char* qr_linear_plan(int64_t M, int64_t N, int64_t K, size_t workspace_bytes, size_t* scratch_bytes);
 int qr_linear_i4_f16_ws(const void* A, const void* sA, const void* W, const void* sW,
                         const void* bias_or_null, int64_t M, int64_t N, int64_t K, void* y,
                         void* workspace, size_t workspace_bytes, void* stream);

@@ -1977,6 +1977,33 @@ MidPlan mid_plan(int64_t M, int64_t N, int64_t Kb, int64_t max_split) {
     return best;
 }
 
+// The kernel that takes a shape, with room for max_split slabs of the output, and the slices of K that it runs in.
+enum class Gemm { large, gemv, shared_tokens, decode, stream64, mid64, mid64x128, mid128, spk, sp192, sp256, sp256_tail };
+struct GemmPlan {
+    Gemm kernel;
+    int split;
+};
+GemmPlan gemm_plan(int64_t M, int64_t N, int64_t Kb, int64_t max_split) {
+    // An operand of 4 GiB or more: every specialised kernel below addresses its operands through 32-bit offsets;
+    // the plain tiled kernel computes 64-bit row addresses and takes any shape (rows beyond M or N are clamped).
+    if (M * Kb >= (1LL << 32) || N * Kb >= (1LL << 32)) return GemmPlan{Gemm::large, 1};
+    if (M > 64) {
+        const MidPlan plan = mid_plan(M, N, Kb, max_split);
+        constexpr Gemm kernels[] = {Gemm::mid64, Gemm::mid64x128, Gemm::mid128, Gemm::spk, Gemm::sp192, Gemm::sp256, Gemm::sp256_tail};
+        return GemmPlan{kernels[plan.kernel], plan.split};
+    }
+    // one to four tokens: the dot-product kernel -- except two to four tokens against a weight with enough rows for the
+    // shared-token kernel, which is ahead there (57344 x 8192: 40.2 against 42.9 us)
+    const bool xs = decode_xs_groups((int)N) != 0;
+    if (M == 1 || (M <= 4 && !xs)) return GemmPlan{Gemm::gemv, 1};
+    const DecodePlan plan = decode_plan(M, N, Kb, max_split);
+    if (plan.tiles) return GemmPlan{Gemm::stream64, plan.split};
+    // weight streaming: with enough groups of 32 rows to fill the CUs the kernel that shares the
+    // tokens' codes through LDS (they are read once per workgroup); otherwise the barrier-free
+    // kernel in which the waves of a workgroup split K over groups of 32 rows
+    return GemmPlan{xs ? Gemm::shared_tokens : Gemm::decode, 1};
+}
+
 int gemm_dispatch(const void* A, const void* B, int64_t M, int64_t N, int64_t K, void* C, void* Y, const void* sA,
                   const void* sB, const void* bias, hipStream_t st, void* ws = nullptr, size_t ws_bytes = 0) {
     if (M < 0 || N < 0 || K < 0) return QR_E_SHAPE;
@@ -1986,46 +2013,32 @@ int gemm_dispatch(const void* A, const void* B, int64_t M, int64_t N, int64_t K,
     if (((uintptr_t)A & 15) || ((uintptr_t)B & 15)) return QR_E_ALIGN;
     if (Y ? ((uintptr_t)Y & 7) : ((uintptr_t)C & 15)) return QR_E_ALIGN;
     const int m = (int)M, n = (int)N, kb = (int)(K / 2);
-    // An operand of 4 GiB or more: every specialised kernel below addresses its operands through 32-bit offsets;
-    // the plain tiled kernel computes 64-bit row addresses and takes any shape (rows beyond M or N are clamped).
-    if (M * (int64_t)kb >= (1LL << 32) || N * (int64_t)kb >= (1LL << 32)) {
-        if (M <= 128) return launch_cfg<128, 128, 2, 2>(A, B, m, n, kb, C, Y, sA, sB, bias, st);
-        return launch_cfg<256, 256, 4, 2>(A, B, m, n, kb, C, Y, sA, sB, bias, st);
-    }
-    // one to four tokens: the dot-product kernel -- except two to four tokens against a weight with enough rows for the
-    // shared-token kernel, which is ahead there (57344 x 8192: 40.2 against 42.9 us)
-    if (M == 1 || (M <= 4 && decode_xs_groups(n) == 0)) return launch_gemv(A, B, m, n, kb, C, Y, sA, sB, bias, st);
     // the slabs of a K split go to scratch from the caller; without it (or with too little) the single-launch kernels run
     const bool scratch = Y && ws && ((uintptr_t)ws & 15) == 0;
-    auto add_slabs = [&](int split) {
+    const GemmPlan plan = gemm_plan(M, N, kb, scratch ? (int64_t)(ws_bytes / ((size_t)M * (size_t)N * 4)) : 1);
+    const int mid = plan.kernel == Gemm::stream64 ? 3 : (int)plan.kernel - (int)Gemm::mid64;      // qr_internal_gemm_mid's shape
+    if (plan.split > 1) {
+        const int rc = qr_internal_gemm_mid(mid, A, B, m, n, kb, ws, nullptr, nullptr, nullptr, nullptr, st, plan.split);
+        if (rc != QR_OK) return rc;
         int64_t db = (M * N / 4 + 255) / 256;
         db = db < 1 ? 1 : (db > 4096 ? 4096 : db);
-        dequant_slabs_kernel<<<dim3((unsigned)db), dim3(256), 0, st>>>((const int32_t*)ws, split, (const f16*)sA,
+        dequant_slabs_kernel<<<dim3((unsigned)db), dim3(256), 0, st>>>((const int32_t*)ws, plan.split, (const f16*)sA,
                                                                       (const f16*)sB, (const f16*)bias, M, N, (f16*)Y);
         return qr_launch_status();
-    };
-    if (M <= 64) {
-        const DecodePlan plan = decode_plan(M, N, kb, scratch ? (int64_t)(ws_bytes / ((size_t)M * (size_t)N * 4)) : 1);
-        if (plan.tiles && plan.split > 1) {
-            const int rc = qr_internal_gemm_mid(3, A, B, m, n, kb, ws, nullptr, nullptr, nullptr, nullptr, st, plan.split);
-            return rc != QR_OK ? rc : add_slabs(plan.split);
-        }
-        if (plan.tiles) return qr_internal_gemm_mid(3, A, B, m, n, kb, C, Y, sA, sB, bias, st, 1);
-        // weight streaming: with enough groups of 32 rows to fill the CUs the kernel that shares the
-        // tokens' codes through LDS (they are read once per workgroup); otherwise the barrier-free
-        // kernel in which the waves of a workgroup split K over groups of 32 rows
-        if (const int rg = decode_xs_groups(n)) return launch_decode_xs(A, B, m, n, kb, C, Y, sA, sB, bias, st, rg);
-        return launch_decode(A, B, m, n, kb, C, Y, sA, sB, bias, st);
     }
-    const MidPlan plan = mid_plan(M, N, kb, scratch ? (int64_t)(ws_bytes / ((size_t)M * (size_t)N * 4)) : 1);
-    if (plan.split > 1) {
-        const int rc = qr_internal_gemm_mid(plan.kernel, A, B, m, n, kb, ws, nullptr, nullptr, nullptr, nullptr, st, plan.split);
-        return rc != QR_OK ? rc : add_slabs(plan.split);
+    switch (plan.kernel) {
+        case Gemm::large:
+            if (M <= 128) return launch_cfg<128, 128, 2, 2>(A, B, m, n, kb, C, Y, sA, sB, bias, st);
+            return launch_cfg<256, 256, 4, 2>(A, B, m, n, kb, C, Y, sA, sB, bias, st);
+        case Gemm::gemv: return launch_gemv(A, B, m, n, kb, C, Y, sA, sB, bias, st);
+        case Gemm::shared_tokens: return launch_decode_xs(A, B, m, n, kb, C, Y, sA, sB, bias, st, decode_xs_groups(n));
+        case Gemm::decode: return launch_decode(A, B, m, n, kb, C, Y, sA, sB, bias, st);
+        case Gemm::spk: return launch_spk(A, B, m, n, kb, C, Y, sA, sB, bias, st);
+        case Gemm::sp192: return launch_sp256(A, B, m, n, kb, C, Y, sA, sB, bias, st, 192);
+        case Gemm::sp256: return launch_sp256(A, B, m, n, kb, C, Y, sA, sB, bias, st, 256);
+        case Gemm::sp256_tail: return launch_sp256_tail(A, B, m, n, kb, C, Y, sA, sB, bias, st);
+        default: return qr_internal_gemm_mid(mid, A, B, m, n, kb, C, Y, sA, sB, bias, st, 1);
     }
-    if (plan.kernel <= 2) return qr_internal_gemm_mid(plan.kernel, A, B, m, n, kb, C, Y, sA, sB, bias, st, 1);
-    if (plan.kernel == 3) return launch_spk(A, B, m, n, kb, C, Y, sA, sB, bias, st);
-    if (plan.kernel == 6) return launch_sp256_tail(A, B, m, n, kb, C, Y, sA, sB, bias, st);
-    return launch_sp256(A, B, m, n, kb, C, Y, sA, sB, bias, st, plan.kernel == 4 ? 192 : 256);
 }
 
 }  // namespace
@@ -2045,6 +2058,30 @@ extern "C" size_t qr_workspace_bytes(int64_t M, int64_t N, int64_t K) {
     if (M <= 0 || N <= 0 || K <= 0 || K % 64 != 0) return 0;
     const int split = ks_split(M, N, K / 2);
     return split > 1 ? (size_t)split * (size_t)M * (size_t)N * 4 : 0;
+}
+
+extern "C" const char* qr_linear_plan(int64_t M, int64_t N, int64_t K, size_t workspace_bytes, size_t* scratch_bytes) {
+    if (scratch_bytes) *scratch_bytes = 0;
+    if (M <= 0 || N <= 0 || K <= 0 || K % 64 != 0 || K > 131008 || M > 0x7fffffff || N > 0x7fffffff) return nullptr;
+    const size_t slab = (size_t)M * (size_t)N * 4;
+    const GemmPlan plan = gemm_plan(M, N, K / 2, workspace_bytes ? (int64_t)(workspace_bytes / slab) : 1);
+    const bool slices = plan.split > 1;
+    if (slices && scratch_bytes) *scratch_bytes = slab * (size_t)plan.split;
+    switch (plan.kernel) {
+        case Gemm::large: return "gemm_i4_kernel";
+        case Gemm::gemv: return "gemv_i4_kernel";
+        case Gemm::shared_tokens: return "decode_xs_kernel";
+        case Gemm::decode: return "decode_i4_kernel";
+        case Gemm::stream64:
+        case Gemm::mid64: return slices ? "gemm_mid_kernel<64,64> (K sliced) + dequant_slabs_kernel" : "gemm_mid_kernel<64,64>";
+        case Gemm::mid64x128: return "gemm_mid_kernel<64,128>";
+        case Gemm::mid128: return "gemm_mid_kernel<128,128>";
+        case Gemm::spk: return "gemm_spk_kernel";
+        case Gemm::sp192:
+        case Gemm::sp256: return "gemm_sp256_kernel";
+        case Gemm::sp256_tail: return "gemm_sp256_tail_kernel";
+    }
+    return nullptr;
 }
 
 // ---- the entry point that allocates nothing ---------------------------------------------------------

@@ -135,3 +135,23 @@ def test_missing_library_fails_loudly(monkeypatch, tmp_path):
     monkeypatch.setattr(_lib, "LIB_PATH", tmp_path / "nope.so")
     with pytest.raises(RuntimeError, match="no CPU or PyTorch fallback"):
         _lib.lib()
+
+
+def test_plan_names_a_kernel_for_every_shape_and_stays_within_the_workspace(lib):
+    """qr_linear_plan: a name for every shape that the product takes, scratch that is a whole number of [M, N] int32 slabs, no more
+    than offered, and the same plan again when only that much is offered; NULL for shapes that are refused."""
+    seen = set()
+    used = ctypes.c_size_t()
+    for m in (1, 2, 4, 5, 7, 8, 24, 40, 48, 64, 65, 128, 300, 333, 777, 1260, 2048, 8191, 32768):
+        for n in (1, 100, 128, 520, 4096, 5120, 8192, 12288, 28672, 57344):
+            for k in (64, 1088, 4096, 11008, 28672, 131008):
+                offered = lib.qr_workspace_bytes(m, n, k)
+                name = lib.qr_linear_plan(m, n, k, offered, ctypes.byref(used))
+                assert name and used.value <= offered and used.value % (m * n * 4) == 0, (m, n, k)
+                assert (b"sliced" in name) == (used.value > 0)
+                assert lib.qr_linear_plan(m, n, k, used.value, None) == name
+                assert b"sliced" not in lib.qr_linear_plan(m, n, k, 0, None)
+                seen.add(name)
+    assert len(seen) == 10 and lib.qr_linear_plan(1 << 17, 128, 131008, 0, None) == b"gemm_i4_kernel", seen
+    for bad in ((0, 1, 64), (1, 0, 64), (1, 1, 0), (1, 1, 100), (1, 1, 131072), (1 << 31, 1, 64)):
+        assert lib.qr_linear_plan(*bad, 0, None) is None
