@@ -7,6 +7,7 @@ its C ABI.  Extras that fuse adjacent steps are listed after the reference's nam
 
     import quarot_amd as quarot
 """
+import ctypes
 import functools
 
 import weakref
@@ -310,9 +311,11 @@ def heads_hadamard_quantize(x, num_heads, clip_ratio=1.0, return_transformed=Fal
 
 @functools.lru_cache(maxsize=4096)
 def _workspace_bytes(M, N, K, device_index=None):
-    # (the library's split plan depends on the CURRENT device's compute-unit count: callers make the
-    # device current first, and the device index is part of the cache key)
-    return _lib.lib().qr_workspace_bytes(M, N, K)
+    # what the library's plan uses of the scratch that it asks for.  (The plan depends on the CURRENT device's compute-unit
+    # count: callers make the device current first, and the device index is part of the cache key)
+    used, L = ctypes.c_size_t(), _lib.lib()
+    L.qr_linear_plan(M, N, K, L.qr_workspace_bytes(M, N, K), ctypes.byref(used))
+    return used.value
 
 
 def linear_i4(x_q, scales_x, weight, weight_scales, bias=None):
@@ -383,7 +386,8 @@ def linear_f6(x6, scales_x, weight6, weight_scales, bias=None):
 
 @functools.lru_cache(maxsize=4096)
 def _quantized_linear_workspace_bytes(M, N, K, device_index=None):
-    return _lib.lib().qr_quantized_linear_workspace_bytes(M, N, K)       # (per device, like _workspace_bytes)
+    L = _lib.lib()                                                       # (per device, like _workspace_bytes)
+    return L.qr_quantized_linear_workspace_bytes(M, N, K) - L.qr_workspace_bytes(M, N, K) + _workspace_bytes(M, N, K, device_index)
 
 
 def quantized_linear(x, weight, weight_scales, bias=None, hadK=None, K=0, clip_ratio=1.0, force_fp32=False):

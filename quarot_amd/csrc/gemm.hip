@@ -1885,9 +1885,11 @@ DecodePlan decode_plan(int64_t M, int64_t N, int64_t Kb, int64_t max_split) {
     return best;
 }
 
-// How many int32 slabs of [M, N] a caller is asked to provide (qr_workspace_bytes): for prompts of a few hundred tokens an
-// upper bound of the slices that mid_plan may use, larger than it needs since its tiles fill the CUs without a split at
-// most of these shapes; callers size their scratch once per shape.
+// How many int32 slabs of [M, N] a caller is asked to provide (qr_workspace_bytes).  Up to 64 tokens: what decode_plan uses.  For
+// prompts of a few hundred tokens it is a contract, not a plan: these are the shapes and slices that the first kernel of this
+// path could use (64 x 256 tiles: 6 us, 1.0 per stage and round of tiles, the slabs), and what earlier versions asked for, also of
+// the callers of qr_linear_i4_f16_static.  mid_plan takes at most so many slices and, with tiles that fill the CUs by
+// themselves, none at most of these shapes; qr_linear_plan says how many, which is what the Python package allocates.
 int ks_split(int64_t M, int64_t N, int64_t Kb) {
     if (M <= 64) return decode_plan(M, N, Kb, 8).split;
     if (N <= 128) return 1;

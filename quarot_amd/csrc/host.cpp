@@ -295,6 +295,16 @@ bool weight_args(PyObject* w, PyObject* s, PyObject* b, int64_t half_k, int devi
     return out->N > 0 && out->s->numel() == out->N && (!out->b || out->b->numel() == out->N);
 }
 
+// What the library asks for as scratch of the product of a shape, and what its plan uses of it.
+struct Slabs {
+    size_t asked, used;
+};
+Slabs slab_bytes(int64_t M, int64_t N, int64_t K) {
+    Slabs s{qr_workspace_bytes(M, N, K), 0};
+    if (s.asked) qr_linear_plan(M, N, K, s.asked, &s.used);
+    return s;
+}
+
 // linear(codes, scales, weight, weight_scales, bias or None) -> y
 PyObject* linear(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
     QR_ARGS(5)
@@ -307,7 +317,7 @@ PyObject* linear(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
     c10::SmallVector<int64_t, 6> sizes(q->sizes().begin(), q->sizes().end());
     sizes.back() = w.N;
     at::Tensor y = fresh(sizes, kHalf, device);
-    const size_t need = qr_workspace_bytes(M, w.N, half_k * 2);
+    const size_t need = slab_bytes(M, w.N, half_k * 2).used;
     at::Tensor ws;                                          // (few output tiles: room for the slabs of a K split)
     if (need) ws = fresh({(int64_t)need}, kByte, device);
     if (!done([&] { return qr_linear_i4_f16_ws(q->data_ptr(), sx->data_ptr(), w.w->data_ptr(), w.s->data_ptr(), ptr(w.b), M, w.N, half_k * 2,
@@ -332,7 +342,8 @@ PyObject* quantized_linear(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
     c10::SmallVector<int64_t, 6> sizes(r.x->sizes().begin(), r.x->sizes().end());
     sizes.back() = w.N;
     at::Tensor y = fresh(sizes, kHalf, r.device);
-    const size_t need = qr_quantized_linear_workspace_bytes(r.rows, w.N, r.n);
+    const Slabs slabs = slab_bytes(r.rows, w.N, r.n);
+    const size_t need = qr_quantized_linear_workspace_bytes(r.rows, w.N, r.n) - slabs.asked + slabs.used;
     at::Tensor ws = fresh({(int64_t)(need < 16 ? 16 : need)}, kByte, r.device);
     if (!done([&] { return qr_quantized_linear_f16(r.x->data_ptr(), r.rows, r.n, (int)K, ptr(table), (int)mode, (float)scale, (float)clip,
                                                       w.w->data_ptr(), w.s->data_ptr(), ptr(w.b), w.N, y.data_ptr(), ws.data_ptr(), need,

@@ -294,3 +294,30 @@ def test_page_tables_made_under_capture_are_that_graphs_own():
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, want) and all(torch.equal(x, y) for x, y in zip(longer, tables(b)))
+
+
+@pytest.mark.parametrize("m,n,k", [(128, 4096, 11008), (256, 4096, 11008), (48, 5120, 13824), (96, 512, 8192)])
+def test_linear_allocates_the_scratch_that_its_plan_uses(m, n, k, general_route):
+    """The slabs of a K split are allocated where K is split, and not where the library would take room for them but has no use for
+    it (128 x 11008 -> 4096: 10 MiB); on both routes, alone and behind the quantiser."""
+    import ctypes
+    L, used = _lib.lib(), ctypes.c_size_t()
+    L.qr_linear_plan(m, n, k, L.qr_workspace_bytes(m, n, k), ctypes.byref(used))
+    x, w, sw = torch.randn(m, k, device="cuda").half(), torch.zeros(n, k // 2, dtype=torch.uint8, device="cuda"), torch.ones(n, 1, device="cuda").half()
+    q, s = quarot_amd.quantize_rows(x)
+
+    def taken(call):
+        torch.cuda.synchronize()
+        before = torch.cuda.memory_allocated()
+        torch.cuda.reset_peak_memory_stats()
+        call()
+        return torch.cuda.max_memory_allocated() - before
+
+    def both():
+        yield taken(lambda: quarot_amd.linear_i4(q, s, w, sw)), 0
+        yield taken(lambda: quarot_amd.quantized_linear(x, w, sw)), m * k // 2 + 2 * m
+    for route in ("native", "general"):
+        for got, codes in both():
+            least = 2 * m * n + used.value + codes
+            assert least <= got < least + 2 ** 21, (route, got, least)         # (the allocator leaves up to 1 MiB of a block unused)
+        general_route()
