@@ -188,7 +188,7 @@ int qr_linear_i4_f16(const void* A, const void* sA, const void* W, const void* s
 
 /*
  * The same with a caller-provided scratch buffer, for shapes whose output tiles would occupy only a
- * fraction of the CUs (decode batches of 40..64 tokens against a narrow weight with K >= 16384,
+ * fraction of the CUs (decode batches of 8..64 tokens against a narrow weight,
  * prompts of a few hundred tokens): K is then split across workgroups, each slice leaves its int32 partial sums in
  * `workspace` and a second kernel adds and dequantises them (two launches on `stream`).  The library never
  * allocates (the reference's bindings allocate their outputs with torch::empty,
@@ -217,8 +217,8 @@ int qr_linear_i4_f16_ws(const void* A, const void* sA, const void* W, const void
  *   Same operands and bit-identical results as qr_linear_i4_f16_ws with a sufficient workspace.
  *   A shape whose qr_workspace_bytes(M, N, K) exceeds QR_STATIC_SCRATCH_BYTES returns
  *   QR_E_SCRATCH_LIMIT and launches nothing (use qr_linear_i4_f16 or the _ws form); shapes that need
- *   no scratch run the single-launch kernels.
- *   All calls on one GPU share that GPU's buffer: calls that overlap in time on one GPU (different
+ *   no scratch run the single-launch kernels, and so do 64 tokens and fewer unless M >= 40 and K >= 16384.
+ *   All other calls on one GPU share that GPU's buffer: of those, calls that overlap in time on one GPU (different
  *   streams or host threads) race.  The first call on a device looks the buffer's address up
  *   (hipGetSymbolAddress); make that call outside graph capture.  The buffer is the CURRENT device's
  *   (hipGetDevice at the time of the call): `stream` must belong to the current device.  A failure

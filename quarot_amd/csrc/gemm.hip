@@ -2120,7 +2120,9 @@ int static_scratch(void** out) {
 extern "C" int qr_linear_i4_f16_static(const void* A, const void* sA, const void* W, const void* sW,
                                        const void* bias_or_null, int64_t M, int64_t N, int64_t K, void* y, void* stream) {
     if (M > 0 && N > 0 && (!y || !sA || !sW)) return QR_E_NULL;
-    const size_t need = qr_workspace_bytes(M, N, K);
+    // Decode batches use the buffer from 40 tokens and K = 16384 on only, as the header promises, though decode_plan would slice K
+    // from 8 tokens on: calls of the other sizes share nothing and may overlap.
+    const size_t need = M > 64 || (M >= 40 && K >= 16384) ? qr_workspace_bytes(M, N, K) : 0;
     if (need > (size_t)QR_STATIC_SCRATCH_BYTES) return QR_E_SCRATCH_LIMIT;
     void* ws = nullptr;
     if (need) {                                  // every slab cell is written before it is read: nothing to clear

@@ -18,6 +18,17 @@ def gpu(a):
     return torch.from_numpy(np.ascontiguousarray(a)).to("cuda:0")
 
 
+@pytest.fixture(scope="module", autouse=True)
+def first_call_on_the_device():
+    """The documented first call, which looks the buffer up: it loads the code object that holds the buffer where no other kernel of that
+    object has run yet (this file alone), and with it the buffer's memory."""
+    a, w, sa, sw, _ = [gpu(t) for t in operands(64, 256, 16384, 0)]
+    y = torch.empty(64, 256, dtype=torch.float16, device="cuda:0")
+    assert _lib.lib().qr_linear_i4_f16_static(a.data_ptr(), sa.data_ptr(), w.data_ptr(), sw.data_ptr(), None, 64, 256, 16384, y.data_ptr(),
+                                              torch.cuda.current_stream().cuda_stream) == 0
+    torch.cuda.synchronize()
+
+
 def operands(m, n, k, seed):
     rng = np.random.default_rng(seed)
     a = o.pack_i4(rng.integers(-8, 8, (m, k)))
@@ -79,3 +90,29 @@ def test_static_scratch_limit_and_argument_errors():
     assert L.qr_linear_i4_f16_static(one, one, one, one, None, 128, 4096, 100, one, None) == -2
     assert L.qr_linear_i4_f16_static(one, None, one, one, None, 128, 4096, 4096, one, None) == -1
     assert L.qr_linear_i4_f16_static(one, one, one, one, None, 0, 4096, 4096, None, None) == 0
+
+
+@pytest.mark.parametrize("m,n,k,launches", [(8, 4096, 28672, 1), (16, 4096, 28672, 1), (24, 5120, 13824, 1), (39, 4096, 28672, 1),
+                                            (48, 5120, 13824, 1), (64, 4096, 16320, 1), (40, 4096, 16384, 2), (64, 8192, 28672, 2)])
+def test_static_scratch_is_left_alone_by_decode_batches_below_40_tokens_or_16384_columns(m, n, k, launches):
+    """Calls of those sizes may overlap: they must not share the library's buffer.  A call that uses it is two launches (slices, then
+    their sum), one that does not is one; the launches are counted in a captured graph.  Results are the oracle's either way."""
+    L, used = _lib.lib(), ctypes.c_size_t()
+    L.qr_linear_plan(m, n, k, L.qr_workspace_bytes(m, n, k), ctypes.byref(used))
+    assert used.value > 0                                              # (with a workspace of its own it would be sliced)
+    a, w, sa, sw, _ = operands(m, n, k, m + n)
+    ga, gw, gsa, gsw = gpu(a), gpu(w), gpu(sa), gpu(sw)
+    y = torch.empty(m, n, dtype=torch.float16, device="cuda:0")
+    call = lambda: L.qr_linear_i4_f16_static(ga.data_ptr(), gsa.data_ptr(), gw.data_ptr(), gsw.data_ptr(), None, m, n, k, y.data_ptr(),
+                                             torch.cuda.current_stream().cuda_stream)
+    assert call() == 0
+    cols = np.arange(0, n, 61)
+    want = o.linear4bit(a, sa, w[cols], sw[cols], None)
+    assert np.array_equal(y[:, cols].cpu().numpy().view(np.uint16), want.view(np.uint16))
+    graph = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(graph):
+        assert call() == 0
+    path = next(line.split()[-1] for line in open("/proc/self/maps") if "libamdhip64" in line)
+    count = ctypes.c_size_t()
+    assert ctypes.CDLL(path).hipGraphGetNodes(ctypes.c_void_p(graph.raw_cuda_graph()), None, ctypes.byref(count)) == 0
+    assert count.value == launches
