@@ -1916,9 +1916,13 @@ int ks_split(int64_t M, int64_t N, int64_t Kb) {
 // busiest of the CUs; fitted to sweeps of 65 .. 1500 tokens against 1902 .. 28672 weight rows at K = 4096 .. 28672 with
 // every kernel forced, and within 10 % of them):
 //   64 x 64 tiles   4.2 + st (n = 1: 0.26, 2: 0.44, more: 0.25 n, from 8 on 0.26 n)      three workgroups share a CU
-//                   0.27 n from 5 on where K > 8192: in loops of this product alone they lead 128-row tiles there (1260 x 4096 x 11008
-//                   55 us against 64), but behind its Hadamard the pipelined kernel's clock is higher (69.9 against 66.8 for both
-//                   launches), and 542 x 8192 x 28672 is level even alone (141 against 139)
+//                   0.27 n from 5 on where K > 8192 and the weights are over 36 MB: they are read once per 64 tokens there and once per
+//                   128 by the pipelined kernel (the only other candidate in that corner), from memory.  5 tiles per CU, weights and
+//                   inputs cold, 64 x 64 / pipelined, alone and behind a quantiser or a Hadamard: 300 x 13824 x 13824 58.1 / 60.1,
+//                   62.3 / 59.0, 67.0 / 63.9 us; 600 x 8192 x 20480 89 / 87, 96 / 92, 106 / 96; 600 x 8192 x 28672 119 / 113, 125 / 120,
+//                   133 / 127.  Below the line: 1260 x 4096 x 11008 46.5 / 50.8, 55.9 / 54.2, 59.4 / 59.5; 1000 x 5120 x 13824 57.7 / 61.1,
+//                   64.2 / 65.8, 70.3 / 71.3; 2560 x 2048 x 28672 111 / 114, 135 / 138, 150 / 152.  (A layer alone, without a front, is up to
+//                   8 % better off on the small tiles above the line as well: 600 x 8192 x 11008 48 / 52; such widths follow a front.)
 //   64 x 128        4.6 + st (0.41 n, from the second on 0.52 n)
 //   128 x 128       5.0 + st (n = 1: 0.80, more: 0.92 n)
 //   128 / 192 / 256 x 256 (the pipelined kernels)   rounds (5.5 + {1.40, 2.19, 2.75} st (1 - {0.3, 0.5, 0.5} idle)), idle = share of
@@ -1938,9 +1942,10 @@ MidPlan mid_plan(int64_t M, int64_t N, int64_t Kb, int64_t max_split) {
     const int64_t cus = qr_device().cus, st = (Kb + 127) / 128;
     auto tiles = [&](int64_t bm, int64_t bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
     auto loaded = [&](int64_t t) { return (double)((t + cus - 1) / cus); };
+    const bool heavy = st > 32 && N * Kb > 36000000;
     auto t64 = [&](int64_t t, int64_t stages) {
         const double n = loaded(t);
-        return 4.2 + (double)stages * (n == 1 ? 0.26 : n == 2 ? 0.44 : n >= 5 && stages > 32 ? 0.27 * n : n < 8 ? 0.25 * n : 0.26 * n);
+        return 4.2 + (double)stages * (n == 1 ? 0.26 : n == 2 ? 0.44 : n >= 5 && heavy ? 0.27 * n : n < 8 ? 0.25 * n : 0.26 * n);
     };
     MidPlan best{0, 1};
     double t_best = t64(tiles(64, 64), st);

@@ -155,3 +155,13 @@ def test_plan_names_a_kernel_for_every_shape_and_stays_within_the_workspace(lib)
     assert len(seen) == 10 and lib.qr_linear_plan(1 << 17, 128, 131008, 0, None) == b"gemm_i4_kernel", seen
     for bad in ((0, 1, 64), (1, 0, 64), (1, 1, 0), (1, 1, 100), (1, 1, 131072), (1 << 31, 1, 64)):
         assert lib.qr_linear_plan(*bad, 0, None) is None
+
+
+def test_plan_of_five_small_tiles_per_cu_depends_on_the_weights(lib):
+    """64 x 64 tiles, five on the busiest CU, against a long K: they keep light weights (up to 36 MB) and leave heavier ones, read from
+    memory once per row of tiles, to the pipelined kernel; up to K = 8192 the weights do not matter."""
+    for m, n, k, small in ((1260, 4096, 11008, True), (1000, 5120, 13824, True), (2560, 2048, 28672, True), (4901, 879, 13824, True),
+                           (1280, 4096, 17920, False), (600, 8192, 28672, False), (300, 13824, 13824, False),
+                           (640, 8192, 8192, True), (300, 13824, 8192, True)):
+        name = lib.qr_linear_plan(m, n, k, 0, None)
+        assert name == (b"gemm_mid_kernel<64,64>" if small else b"gemm_spk_kernel"), (m, n, k, name)
