@@ -67,7 +67,6 @@ struct Unlocked {
     ~Unlocked() { PyEval_RestoreThread(state); }
 };
 at::Tensor fresh(at::IntArrayRef sizes, at::ScalarType dtype, int device) {
-    const Unlocked unlocked;
     return at::empty(sizes, at::TensorOptions().dtype(dtype).device(at::Device(at::kCUDA, (c10::DeviceIndex)device)));
 }
 void* ptr(const at::Tensor* t) { return t ? t->data_ptr() : nullptr; }
@@ -178,10 +177,13 @@ PyObject* quantize_rows(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
     const Rows r = rows_of(a[0]);
     double clip;
     if (!r.ok || !arg_float(a[1], &clip)) return none();
-    Packed p = packed_for(r, (int)r.x->dim() - 1);
-    if (!done([&] { return qr_quantize_rows_f16_i4(r.x->data_ptr(), (float)clip, r.rows, r.n, p.codes.data_ptr(), p.scales.data_ptr(),
-                                                      stream(r.device)); }))
-        return none();
+    Packed p;
+    const auto call = [&] {
+        p = packed_for(r, (int)r.x->dim() - 1);
+        return qr_quantize_rows_f16_i4(r.x->data_ptr(), (float)clip, r.rows, r.n, p.codes.data_ptr(), p.scales.data_ptr(),
+                                       stream(r.device));
+    };
+    if (!done(call)) return none();
     return wrap2(std::move(p.codes), std::move(p.scales));
     QR_END
 }
@@ -193,9 +195,12 @@ PyObject* rmsnorm(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
     long long mean_dim;
     double eps;
     if (!r.ok || !arg_int(a[1], &mean_dim) || !arg_float(a[2], &eps) || mean_dim > 0x7fffffff) return none();
-    at::Tensor y = fresh(r.x->sizes(), kHalf, r.device);
-    if (!done([&] { return qr_rmsnorm_f16(r.x->data_ptr(), r.rows, r.n, (int)mean_dim, (float)eps, y.data_ptr(), stream(r.device)); }))
-        return none();
+    at::Tensor y;
+    const auto call = [&] {
+        y = fresh(r.x->sizes(), kHalf, r.device);
+        return qr_rmsnorm_f16(r.x->data_ptr(), r.rows, r.n, (int)mean_dim, (float)eps, y.data_ptr(), stream(r.device));
+    };
+    if (!done(call)) return none();
     return wrap(std::move(y));
     QR_END
 }
@@ -208,10 +213,13 @@ PyObject* rmsnorm_quantize(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
     double eps, clip;
     if (!r.ok || r.n % 8 || !arg_int(a[1], &mean_dim) || !arg_float(a[2], &eps) || !arg_float(a[3], &clip) || mean_dim > 0x7fffffff)
         return none();
-    Packed p = packed_for(r, (int)r.x->dim() - 1);
-    if (!done([&] { return qr_rmsnorm_quantize_f16_i4(r.x->data_ptr(), r.rows, r.n, (int)mean_dim, (float)eps, (float)clip, p.codes.data_ptr(),
-                                                         p.scales.data_ptr(), nullptr, stream(r.device)); }))
-        return none();
+    Packed p;
+    const auto call = [&] {
+        p = packed_for(r, (int)r.x->dim() - 1);
+        return qr_rmsnorm_quantize_f16_i4(r.x->data_ptr(), r.rows, r.n, (int)mean_dim, (float)eps, (float)clip, p.codes.data_ptr(),
+                                          p.scales.data_ptr(), nullptr, stream(r.device));
+    };
+    if (!done(call)) return none();
     return wrap2(std::move(p.codes), std::move(p.scales));
     QR_END
 }
@@ -227,10 +235,13 @@ PyObject* heads_hadamard_quantize(PyObject*, PyObject* const* a, Py_ssize_t narg
     if (!plain_or_none(a[2], kHalf, r.device, &hadK) || heads > 64 || (hadK && hadK->numel() != heads * heads)) return none();
     r.n = heads * 128;
     r.rows = r.x->numel() / r.n;
-    Packed p = packed_for(r, (int)r.x->dim() - 2);
-    if (!done([&] { return qr_heads_hadamard_quantize_f16_i4(r.x->data_ptr(), r.rows, (int)heads, 128, ptr(hadK), (float)clip, p.codes.data_ptr(),
-                                                                p.scales.data_ptr(), nullptr, stream(r.device)); }))
-        return none();
+    Packed p;
+    const auto call = [&] {
+        p = packed_for(r, (int)r.x->dim() - 2);
+        return qr_heads_hadamard_quantize_f16_i4(r.x->data_ptr(), r.rows, (int)heads, 128, ptr(hadK), (float)clip, p.codes.data_ptr(),
+                                                 p.scales.data_ptr(), nullptr, stream(r.device));
+    };
+    if (!done(call)) return none();
     return wrap2(std::move(p.codes), std::move(p.scales));
     QR_END
 }
@@ -255,10 +266,13 @@ PyObject* hadamard(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
     if (!r.ok || !arg_int(a[2], &K) || !arg_int(a[3], &mode) || !arg_float(a[4], &scale) || r.n > 0x7fffffff ||
         (mode & ~QR_HAD_FP32) != QR_DTYPE_F16 || !table_arg(a[1], mode, K, r.device, &table))
         return none();
-    at::Tensor y = fresh(r.x->sizes(), kHalf, r.device);
-    if (!done([&] { return qr_hadamard(r.x->data_ptr(), y.data_ptr(), r.rows, (int)r.n, (int)K, ptr(table), (int)mode, (float)scale,
-                                          stream(r.device)); }))
-        return none();
+    at::Tensor y;
+    const auto call = [&] {
+        y = fresh(r.x->sizes(), kHalf, r.device);
+        return qr_hadamard(r.x->data_ptr(), y.data_ptr(), r.rows, (int)r.n, (int)K, ptr(table), (int)mode, (float)scale,
+                           stream(r.device));
+    };
+    if (!done(call)) return none();
     return wrap(std::move(y));
     QR_END
 }
@@ -273,10 +287,13 @@ PyObject* hadamard_quantize(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
     if (!r.ok || r.n % 2 || r.n > 0x7fffffff || !arg_int(a[2], &K) || !arg_int(a[3], &mode) || !arg_float(a[4], &scale) ||
         !arg_float(a[5], &clip) || !table_arg(a[1], mode, K, r.device, &table))
         return none();
-    Packed p = packed_for(r, (int)r.x->dim() - 1);
-    if (!done([&] { return qr_hadamard_quantize_f16_i4(r.x->data_ptr(), r.rows, (int)r.n, (int)K, ptr(table), (int)mode, (float)scale, (float)clip,
-                                                          p.codes.data_ptr(), p.scales.data_ptr(), nullptr, stream(r.device)); }))
-        return none();
+    Packed p;
+    const auto call = [&] {
+        p = packed_for(r, (int)r.x->dim() - 1);
+        return qr_hadamard_quantize_f16_i4(r.x->data_ptr(), r.rows, (int)r.n, (int)K, ptr(table), (int)mode, (float)scale, (float)clip,
+                                           p.codes.data_ptr(), p.scales.data_ptr(), nullptr, stream(r.device));
+    };
+    if (!done(call)) return none();
     return wrap2(std::move(p.codes), std::move(p.scales));
     QR_END
 }
@@ -316,13 +333,15 @@ PyObject* linear(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
     if (sx->numel() != M || !weight_args(a[2], a[3], a[4], half_k, device, &w)) return none();
     c10::SmallVector<int64_t, 6> sizes(q->sizes().begin(), q->sizes().end());
     sizes.back() = w.N;
-    at::Tensor y = fresh(sizes, kHalf, device);
     const size_t need = slab_bytes(M, w.N, half_k * 2).used;
-    at::Tensor ws;                                          // (few output tiles: room for the slabs of a K split)
-    if (need) ws = fresh({(int64_t)need}, kByte, device);
-    if (!done([&] { return qr_linear_i4_f16_ws(q->data_ptr(), sx->data_ptr(), w.w->data_ptr(), w.s->data_ptr(), ptr(w.b), M, w.N, half_k * 2,
-                                                  y.data_ptr(), need ? ws.data_ptr() : nullptr, need, stream(device)); }))
-        return none();
+    at::Tensor y, ws;                                       // (ws: few output tiles, room for the slabs of a K split)
+    const auto call = [&] {
+        y = fresh(sizes, kHalf, device);
+        if (need) ws = fresh({(int64_t)need}, kByte, device);
+        return qr_linear_i4_f16_ws(q->data_ptr(), sx->data_ptr(), w.w->data_ptr(), w.s->data_ptr(), ptr(w.b), M, w.N, half_k * 2,
+                                   y.data_ptr(), need ? ws.data_ptr() : nullptr, need, stream(device));
+    };
+    if (!done(call)) return none();
     return wrap(std::move(y));
     QR_END
 }
@@ -341,14 +360,17 @@ PyObject* quantized_linear(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
         return none();
     c10::SmallVector<int64_t, 6> sizes(r.x->sizes().begin(), r.x->sizes().end());
     sizes.back() = w.N;
-    at::Tensor y = fresh(sizes, kHalf, r.device);
     const Slabs slabs = slab_bytes(r.rows, w.N, r.n);
     const size_t need = qr_quantized_linear_workspace_bytes(r.rows, w.N, r.n) - slabs.asked + slabs.used;
-    at::Tensor ws = fresh({(int64_t)(need < 16 ? 16 : need)}, kByte, r.device);
-    if (!done([&] { return qr_quantized_linear_f16(r.x->data_ptr(), r.rows, r.n, (int)K, ptr(table), (int)mode, (float)scale, (float)clip,
-                                                      w.w->data_ptr(), w.s->data_ptr(), ptr(w.b), w.N, y.data_ptr(), ws.data_ptr(), need,
-                                                      stream(r.device)); }))
-        return none();
+    at::Tensor y, ws;
+    const auto call = [&] {
+        y = fresh(sizes, kHalf, r.device);
+        ws = fresh({(int64_t)(need < 16 ? 16 : need)}, kByte, r.device);
+        return qr_quantized_linear_f16(r.x->data_ptr(), r.rows, r.n, (int)K, ptr(table), (int)mode, (float)scale, (float)clip,
+                                       w.w->data_ptr(), w.s->data_ptr(), ptr(w.b), w.N, y.data_ptr(), ws.data_ptr(), need,
+                                       stream(r.device));
+    };
+    if (!done(call)) return none();
     return wrap(std::move(y));
     QR_END
 }
@@ -389,11 +411,14 @@ PyObject* page_tables(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
     if (device < 0 || !arg_int(a[0], &batch) || !arg_int(a[1], &length) || !arg_int(a[2], &page) || batch <= 0 || page <= 0 ||
         length <= 0 || page > 0x7fffffff)
         return none();
-    at::Tensor indptr = fresh({batch + 1}, at::kInt, device);
-    at::Tensor indices = fresh({batch * ((length + page - 1) / page)}, at::kInt, device);
-    at::Tensor last = fresh({batch}, at::kInt, device);
-    if (!done([&] { return qr_page_tables(batch, length, (int)page, indptr.data_ptr(), indices.data_ptr(), last.data_ptr(), stream(device)); }))
-        return none();
+    at::Tensor indptr, indices, last;
+    const auto call = [&] {
+        indptr = fresh({batch + 1}, at::kInt, device);
+        indices = fresh({batch * ((length + page - 1) / page)}, at::kInt, device);
+        last = fresh({batch}, at::kInt, device);
+        return qr_page_tables(batch, length, (int)page, indptr.data_ptr(), indices.data_ptr(), last.data_ptr(), stream(device));
+    };
+    if (!done(call)) return none();
     PyObject* t = PyTuple_New(3);
     if (!t) return nullptr;
     at::Tensor* const all[3] = {&indptr, &indices, &last};
@@ -409,18 +434,18 @@ PyObject* page_tables(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
     QR_END
 }
 
-// capture_id(reference tensor on the device) -> the number of the graph capture that the device's current stream is part of; None
-// outside a capture
-PyObject* capture_id(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
+// where(reference tensor) -> what its device's current stream is: the stream's handle, or (handle, number of the capture) while a
+// graph is captured from it
+PyObject* where(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
     QR_ARGS(1)
     const int device = device_of(tensor(a[0]));
     if (device < 0) return none();
+    void* const st = stream(device);
     hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
     unsigned long long id = 0;
-    const hipError_t e = hipStreamGetCaptureInfo((hipStream_t)stream(device), &status, &id);
-    success((int)e);
-    if (status != hipStreamCaptureStatusActive) return none();
-    return PyLong_FromUnsignedLongLong(id);
+    if (hipStreamGetCaptureInfo((hipStream_t)st, &status, &id) != hipSuccess) (void)hipGetLastError();     // (the default stream beside a capture)
+    if (status != hipStreamCaptureStatusActive) return PyLong_FromVoidPtr(st);
+    return Py_BuildValue("(NK)", PyLong_FromVoidPtr(st), id);
     QR_END
 }
 
@@ -437,10 +462,12 @@ PyObject* quantize_append(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
     if (k->dim() != 3 || k->sizes() != v->sizes() || k->size(1) != c.heads || k->size(2) != 128 || k->numel() == 0) return none();
     const int64_t tokens = k->size(0);
     if (seq ? (seq->dim() != 1 || seq->numel() != c.batch + 1) : tokens != c.batch) return none();
-    if (!done([&] { return qr_kv_quant_append_f16_i4(k->data_ptr(), v->data_ptr(), tokens, ptr(seq), had ? 1 : 0, c.data->data_ptr(), c.param->data_ptr(),
-                                                        c.indptr->data_ptr(), c.indices->data_ptr(), c.last->data_ptr(), c.pages, c.layers, (int)layer, c.heads,
-                                                        c.page_size, 128, c.batch, stream(device)); }))
-        return none();
+    const auto call = [&] {
+        return qr_kv_quant_append_f16_i4(k->data_ptr(), v->data_ptr(), tokens, ptr(seq), had ? 1 : 0, c.data->data_ptr(), c.param->data_ptr(),
+                                         c.indptr->data_ptr(), c.indices->data_ptr(), c.last->data_ptr(), c.pages, c.layers, (int)layer, c.heads,
+                                         c.page_size, 128, c.batch, stream(device));
+    };
+    if (!done(call)) return none();
     Py_RETURN_TRUE;
     QR_END
 }
@@ -465,15 +492,17 @@ PyObject* decode_step(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
         return none();
     const size_t need = bound > 0 ? qr_batch_decode_workspace_bytes(c.batch, c.heads, bound) : 0;
     const bool kept = need && ws && (size_t)ws->numel() >= need;
-    at::Tensor own;
-    if (need && !kept) own = fresh({(int64_t)need}, kByte, device);
     const int qh = (q_had ? 1 : 0) | (kept ? QR_DECODE_COUNTERS_ZERO : 0), kh = k_had ? 1 : 0;
-    at::Tensor o = fresh(q->sizes(), kHalf, device);
-    if (!done([&] { return qr_kv_quant_append_batch_decode_f16_i4(o.data_ptr(), q->data_ptr(), qh, k->data_ptr(), v->data_ptr(), kh, c.data->data_ptr(),
-                                                                     c.param->data_ptr(), c.indptr->data_ptr(), c.indices->data_ptr(), c.last->data_ptr(),
-                                                                     c.pages, c.layers, (int)layer, c.heads, c.page_size, 128, c.batch, bound,
-                                                                     kept ? ws->data_ptr() : need ? own.data_ptr() : nullptr, need, stream(device)); }))
-        return none();
+    at::Tensor o, own;
+    const auto call = [&] {
+        if (need && !kept) own = fresh({(int64_t)need}, kByte, device);
+        o = fresh(q->sizes(), kHalf, device);
+        return qr_kv_quant_append_batch_decode_f16_i4(o.data_ptr(), q->data_ptr(), qh, k->data_ptr(), v->data_ptr(), kh, c.data->data_ptr(),
+                                                      c.param->data_ptr(), c.indptr->data_ptr(), c.indices->data_ptr(), c.last->data_ptr(),
+                                                      c.pages, c.layers, (int)layer, c.heads, c.page_size, 128, c.batch, bound,
+                                                      kept ? ws->data_ptr() : need ? own.data_ptr() : nullptr, need, stream(device));
+    };
+    if (!done(call)) return none();
     return wrap(std::move(o));
     QR_END
 }
@@ -497,7 +526,7 @@ PyMethodDef methods[] = {QR_METHOD(quantize_rows),
                          QR_METHOD(linear),
                          QR_METHOD(quantized_linear),
                          QR_METHOD(page_tables),
-                         QR_METHOD(capture_id),
+                         QR_METHOD(where),
                          QR_METHOD(quantize_append),
                          QR_METHOD(decode_step),
                          QR_METHOD(outcome),

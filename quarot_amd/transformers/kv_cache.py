@@ -299,27 +299,32 @@ class _AttentionStub(object):
         self.disable_quant = disable_quant
         self.hadamard_dtype = hadamard_dtype
 
-    def forward(self, q, num_kv_heads, attention_kwargs, layer_idx, max_seq_len=0, workspace=None, take_pending=None):
+    def forward(self, q, num_kv_heads, attention_kwargs, layer_idx, max_seq_len=0, cache=None, token=None):
         assert q.shape[1] == 1
-        # the step's new token, if the cache still holds it back for this call (see MultiLayerPagedKVCache4Bit.update); a call
-        # that raises leaves it there
-        append = take_pending() if take_pending is not None else None
-        workspace = workspace() if workspace is not None else None
-        o = self._attend(q, attention_kwargs, layer_idx, max_seq_len, workspace, append)
-        if append is not None:
-            take_pending(stored=True)
+        if cache is None:
+            return self._attend(q, attention_kwargs, layer_idx, max_seq_len, None, None)
+        # the step's new token, if the cache still holds it back for this call (see MultiLayerPagedKVCache4Bit.update; otherwise it
+        # has been stored meanwhile, or this callable was used before); a call that raises leaves it there
+        held = cache._pending.get(layer_idx)
+        if held is None or held[0] is not token:
+            held = None
+        o = self._attend(q, attention_kwargs, layer_idx, max_seq_len, cache._decode_workspace(num_kv_heads, max_seq_len), held)
+        if held is not None:
+            cache._pending.pop(layer_idx, None)
         return o
 
-    def _attend(self, q, attention_kwargs, layer_idx, max_seq_len, workspace, append):
+    def _attend(self, q, attention_kwargs, layer_idx, max_seq_len, workspace, held):
+        append = None
+        if held is not None:
+            _, k, v, _, k_hadamard = held
+            if self.hadamard_dtype in (None, torch.float16):
+                s = attention_kwargs
+                o = _lib.host.decode_step(s["kv_data"], s["kv_param"], s["kv_indptr"], s["kv_indices"], s["last_page_offset"], q, k, v,
+                                          layer_idx, self.hadamard_dtype is not None, k_hadamard, max_seq_len, workspace)
+                if o is not None:
+                    return o
+            append = (k.view(k.shape[0], -1, k.shape[-1]), v.view(v.shape[0], -1, v.shape[-1]), k_hadamard)
         batch_size, _, num_qo_heads, head_dim = q.shape
-        if append is not None and self.hadamard_dtype in (None, torch.float16):
-            s = attention_kwargs
-            o = _lib.host.decode_step(s["kv_data"], s["kv_param"], s["kv_indptr"], s["kv_indices"], s["last_page_offset"], q,
-                                      append[0], append[1], layer_idx, self.hadamard_dtype is not None, append[2], max_seq_len, workspace)
-            if o is not None:
-                return o
-        if append is not None:
-            append = (append[0].view(batch_size, -1, head_dim), append[1].view(batch_size, -1, head_dim), append[2])
         q = q.view(batch_size, num_qo_heads, head_dim)
         if self.disable_quant:                   # fp16 pages (kv_cache.py:116-119)
             if self.hadamard_dtype is not None:
@@ -361,10 +366,10 @@ class MultiLayerPagedKVCache4Bit:
         self._scales = torch.empty((max_page_cnt * batch_size, n_layers, 2, num_heads, page_size, 2), dtype=torch.float16,
                                    device=device)
         self._pending = {}      # layer -> (token, k, v, specs, hadamard): a decode step's new token, held for the attention call
-        self._workspaces = {}           # stream -> (key, workspace), see _decode_workspace
-        self._captured_ws = {}          # the same for the capture under way
-        self._decode_ws = None          # the workspace of the last eager step
-        self._captured_specs = None     # page tables of the capture under way
+        self._workspaces = {}           # _where() -> (heads, length, workspace), see _decode_workspace
+        self._decode_ws = None          # the one made last, captures aside
+        self._specs = None              # (length, page tables)
+        self._captured_specs = None     # (length, page tables, _where()) of the capture under way
         self.max_seq_len = max_seq_len
         self._needs_init = [True] * n_layers
         self.length = 0
@@ -399,20 +404,16 @@ class MultiLayerPagedKVCache4Bit:
                 quantize_append_kv_i4(**specs, k=k.view(k.shape[0], *k.shape[-2:]), v=v.view(v.shape[0], *v.shape[-2:]),
                                       seqlen_indptr=None, layer_idx=layer, hadamard=hadamard)
 
-    def _take_pending(self, layer_idx, token, stored=False):
-        held = self._pending.get(layer_idx)
-        if held is None or held[0] is not token:
-            return None                          # stored meanwhile (or this callable was used before): plain attention
-        if stored:
-            del self._pending[layer_idx]
-        return held[1], held[2], held[4]
-
-    def _capture(self):
-        """The graph capture that the current stream is part of: its number (one that no other capture equals where the native
-        host side cannot tell), None outside one."""
-        if not (self._pages.is_cuda and torch.cuda.is_current_stream_capturing()):
-            return None
-        return _lib.host.capture_id(self._pages) or object()
+    def _where(self):
+        """The stream that work on the cache is launched on now: its handle, or while a graph is captured from it (handle, number
+        of the capture) -- one that no other capture equals where the native host side cannot tell."""
+        where = _lib.host.where(self._pages)
+        if where is None and self._pages.is_cuda:
+            with _lib.on_device(self._pages.device):
+                where = _lib.stream_ptr(self._pages.device)
+                if torch.cuda.is_current_stream_capturing():
+                    where = (where, object())
+        return where
 
     def _decode_workspace(self, num_heads, length):
         """Scratch for decode attention split along the sequence, for a launch on the current stream.  It is kept with the cache
@@ -420,31 +421,26 @@ class MultiLayerPagedKVCache4Bit:
         and arrival counters: launches of one stream follow each other and leave the counters at zero, launches of two may
         overlap.  Sized for the longer of the given and the maximum length, zeroed when it is made.  One made while a graph is
         captured is zeroed by that graph's replays only, and only they may use it: it is kept for the rest of that capture."""
+        where = self._where()
+        found = self._workspaces.get(where)
+        if found is not None and found[0] == num_heads and found[1] == length:
+            return found[2]
         dev = self._pages.device
         with _lib.on_device(dev):
-            stream, capture = _lib.stream_ptr(dev), self._capture()
-            key = (num_heads, length, capture)
-            kept = self._workspaces if capture is None else self._captured_ws
-            found = kept.get(stream)
-            if found is not None and found[0] == key:
-                if capture is None:
-                    self._decode_ws = found[1]
-                return found[1]
             need = max((_decode_workspace_bytes(self.batch_size, num_heads, int(n), dev.index)
                         for n in (length, self.max_seq_len) if n), default=0)
-            ws = found[1] if found is not None and found[0][2] == key[2] and found[0][0] == num_heads else None
+            ws = found[2] if found is not None and found[0] == num_heads else None
             if need and (ws is None or ws.numel() < need):
                 ws = torch.empty((need,), dtype=torch.uint8, device=dev)
                 ws[:4 * self.batch_size * num_heads].zero_()           # the counters
-        if capture is not None:
-            self._captured_ws = {stream: (key, ws)}
-            return ws
-        self._captured_ws = {}
-        kept = {s: w for s, w in kept.items() if s != stream}
-        while len(kept) >= _MAX_WORKSPACES:                            # (allocated and used on its own stream: freed behind its launches)
+        # (other captures are over, or fill theirs anew; a stream's own is freed behind its launches)
+        kept = {w: found for w, found in self._workspaces.items() if w != where and not isinstance(w, tuple)}
+        while len(kept) >= _MAX_WORKSPACES:
             kept.pop(next(iter(kept)))
-        kept[stream] = (key, ws)
-        self._workspaces, self._decode_ws = kept, ws
+        kept[where] = (num_heads, length, ws)
+        self._workspaces = kept
+        if not isinstance(where, tuple):
+            self._decode_ws = ws
         return ws
 
     def _ensure_page_cnt_per_batch(self, expected_page_cnt_per_batch):
@@ -499,14 +495,12 @@ class MultiLayerPagedKVCache4Bit:
             # held for the attention call, which quantises and stores the token itself
             token = object()
             self._pending[layer_idx] = (token, k1, v1, specs, fused_had)
-            take = functools.partial(self._take_pending, layer_idx, token)
         else:
             quantize_append_kv_i4(**specs, k=k1.view(b_sz, num_heads, head_dim), v=v1.view(b_sz, num_heads, head_dim),
                                   seqlen_indptr=None, layer_idx=layer_idx, hadamard=fused_had)
-            take = None
+            token = None
         return functools.partial(self._stub.forward, num_kv_heads=num_heads, attention_kwargs=specs, layer_idx=layer_idx,
-                                 max_seq_len=self.length, workspace=functools.partial(self._decode_workspace, num_heads, self.length),
-                                 take_pending=take)
+                                 max_seq_len=self.length, cache=self, token=token)
 
     def _update_f16(self, key_states, value_states, layer_idx, attention_mask, first, specs):
         """update() with fp16 pages (kv_cache.py:187-251 with disable_quant): the transformed keys and the values are
@@ -542,9 +536,10 @@ class MultiLayerPagedKVCache4Bit:
             # every sequence holds self.length tokens: the tables depend on that number alone and are built
             # once per length (every layer of a decode step asks for them), by one launch.  Those of a capture are filled by
             # its replays only, and it reads no others, which an eager step of another length would free.
-            capture = self._capture()
-            cached = self._captured_specs if capture is not None else getattr(self, "_specs", None)
-            if cached is not None and cached[0] == self.length and (capture is None or cached[2] == capture):
+            where = self._where()
+            captured = isinstance(where, tuple)
+            cached = self._captured_specs if captured else self._specs
+            if cached is not None and cached[0] == self.length and (not captured or cached[2] == where):
                 return cached[1]
             tables = _lib.host.page_tables(self.batch_size, self.length, self.page_size, self._pages)
             if tables is None:                   # an empty cache, or one on another than the current device
@@ -557,10 +552,10 @@ class MultiLayerPagedKVCache4Bit:
                           torch.full((self.batch_size,), ptr, dtype=torch.int32, device=self.device))
             specs = {"kv_data": self._pages, "kv_indptr": tables[0], "kv_indices": tables[1], "last_page_offset": tables[2],
                      "kv_param": self._scales}
-            if capture is None:
-                self._specs, self._captured_specs = (self.length, specs), None
+            if captured:
+                self._captured_specs = (self.length, specs, where)
             else:
-                self._captured_specs = (self.length, specs, capture)
+                self._specs, self._captured_specs = (self.length, specs), None
             return specs
         seqlens_in_batch = attention_mask.sum(dim=-1, dtype=torch.int32)
         page_cnt = self.page_cnt_from_length(seqlens_in_batch)
