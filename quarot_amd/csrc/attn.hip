@@ -417,7 +417,9 @@ __global__ __launch_bounds__(64 * NW, (NW == 16 ? 1 : NW == 8 ? 2 : 4)) void pag
 #pragma unroll
         for (int u = 0; u < AU; ++u) {
             const float p = __builtin_amdgcn_exp2f(lg[u] - m);
-            const f16x2 prm = as_f16x2(t.vp[u]);
+            // (a lane without a position may have fetched the first slot of the page that the new token opens: whatever its
+            // memory held, and 0 times a NaN is a NaN.  The codes are finite as they are.)
+            const f16x2 prm = as_f16x2(t.ok[u] ? t.vp[u] : 0u);
             const float ps = p * (float)prm[0];
             d += p;
             pz = __builtin_fmaf(p, (float)prm[1], pz);

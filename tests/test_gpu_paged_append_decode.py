@@ -267,3 +267,26 @@ def test_a_step_whose_attention_call_raises_keeps_its_token(hadamard_dtype):
     assert torch.equal(calls[0](q), calls[2](q))
     for c in caches[:2]:                                                # after the repeated call, and without one
         assert torch.equal(c.pages, caches[2].pages) and torch.equal(c.scales, caches[2].scales)
+
+
+@pytest.mark.parametrize("page_size,heads,B", [(16, 4, 2), (32, 8, 1), (5, 3, 2)])
+def test_a_step_that_opens_a_page_reads_none_of_what_its_memory_held(page_size, heads, B):
+    """The pool is uninitialised memory.  Where the new token is the first of its page, that page holds nothing valid while the
+    other waves walk over the cache; what they fetch from it -- parameters that are NaNs or infinities here -- must not meet
+    the sums, not even with a probability of zero."""
+    rng = np.random.default_rng(page_size)
+    most = 64 * page_size
+    prompt = [gpu(synth_kv(rng, B * most, heads)).view(B, most, heads, 128) for _ in range(2)]
+    q, k, v = (gpu(synth_kv(rng, B, heads)).view(B, 1, heads, 128) for _ in range(3))
+    cache = kv.MultiLayerPagedKVCache4Bit(B, page_size, most + page_size, "cuda:0", 1, heads, 128)
+    cache.update(*prompt, 0)
+    pages, scales = cache.pages.clone(), cache.scales.clone()
+    for length in range(page_size, most + 1, page_size):
+        outs = []
+        for left in (0.0, float("nan"), float("inf"), -float("inf")):
+            cache.pages.copy_(pages), cache.scales.copy_(scales)
+            cache.length = length
+            cache.scales[length // page_size * B:] = left
+            outs.append(cache.update(k, v, 0)(q))
+        assert bool(torch.isfinite(outs[0]).all())
+        assert all(torch.equal(y, outs[0]) for y in outs[1:]), length
