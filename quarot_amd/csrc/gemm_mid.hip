@@ -333,10 +333,12 @@ int launch_mid(const void* A, const void* B, int M, int N, int Kb, void* C, void
 
 }  // namespace
 
-// shape: 0 = 64 x 64, 1 = 64 x 128, 2 = 128 x 128 tiles; 3 = 64 x 64 in the STREAM form (M <= 64).  Three stage buffers of 16
-// or 24 KB let three or two workgroups share a CU; 64 x 128 with five and 64 x 64 with four buffers were no faster (11.8
-// against 11.2 us, 8.3 against 8.2 at 128 and 333 tokens x 4096 x 4096): the loads are bound by rate, not by how many are
-// in flight.  The STREAM form's come from memory: with at most a workgroup per CU it takes five buffers, 64 KB in flight (48 x
+// shape: 0 = 64 x 64, 1 = 64 x 128, 2 = 128 x 128 tiles; 3 = 64 x 64 in the STREAM form (M <= 64).  Three stage buffers of 16 KB
+// let three 64 x 64 workgroups share a CU.  A 64 x 128 or 128 x 128 one has a CU to itself: eight waves exchange 96 KB of
+// accumulators through LDS at the end, more than the 72 KB of its three stage buffers, and four buffers are 128 KB.
+// 64 x 128 with five and 64 x 64 with four buffers were no faster (11.8 against 11.2 us, 8.3 against 8.2 at 128 and 333
+// tokens x 4096 x 4096): the loads are bound by rate, not by how many are in flight.  The STREAM form's come from memory:
+// with at most a workgroup per CU it takes five buffers, 64 KB in flight (48 x
 // 5120 x 13824 in two slices of K 17.8 -> 15.7 us), with more workgroups three (48 x 22016 x 4096 14.3 -> 13.5).
 __attribute__((visibility("hidden"))) int qr_internal_gemm_mid(int shape, const void* A, const void* B, int M, int N, int Kb,
                                                                void* C, void* Y, const void* sA, const void* sB,
