@@ -269,6 +269,7 @@ int qr_linear_f6_f16(const void* A6, const void* sA, const void* W6, const void*
  *   sW fp16 [N], bias fp16 [N] or NULL -> y fp16 [M, N].
  *   workspace: device memory, 16-byte aligned, at least qr_quantized_linear_workspace_bytes(M, N, K)
  *   bytes (never 0 for M > 0), else QR_E_WORKSPACE.  Calls that share a workspace must not overlap.
+ *   Of the qr_workspace_bytes(M, N, K) that it holds for slices of K, only what qr_linear_plan reports as used has to be there.
  */
 size_t qr_quantized_linear_workspace_bytes(int64_t M, int64_t N, int64_t K);
 int qr_quantized_linear_f16(const void* x, int64_t M, int64_t K, int had_K, const void* hadK, int mode,
