@@ -142,7 +142,7 @@ def matmul_hadU_cuda(X, hadK, K):
 
 def matmul_hadU_cuda_fp32(X, hadK, K):
     """matmul_hadU_cuda(X.float(), hadK, K) rounded to X's fp16, in one pass over fp16 rows on the GPU; the two conversions
-    around the fp32 transform where the library has no such kernel (rows of 128 and shorter, beyond 32768)."""
+    around the fp32 transform where the library refuses that (rows of 128 and shorter, beyond 32768, not 16-byte aligned)."""
     n = X.shape[-1]
     y = _lib.host.hadamard(X, hadK, K, _lib.QR_DTYPE_F16 | _lib.QR_HAD_FP32, had_scale(n))
     if y is not None:
@@ -155,7 +155,7 @@ def matmul_hadU_cuda_fp32(X, hadK, K):
             rc = _lib.lib().qr_hadamard(xc.data_ptr(), y.data_ptr(), xc.numel() // n, n, int(K),
                                         None if table is None else table.data_ptr(), _lib.QR_DTYPE_F16 | _lib.QR_HAD_FP32,
                                         had_scale(n), _lib.stream_ptr(xc.device))
-        if rc != _lib.QR_E_UNSUPPORTED:
+        if rc >= 0:
             _lib.check(rc)
             return y.view(X.shape)
     return matmul_hadU_cuda(X.float(), hadK, K).to(X.dtype)

@@ -978,6 +978,17 @@ def test_online_hadamard_fp32_on_fp16_rows_is_the_fp32_transform_rounded_once(n)
     assert torch.equal(had(torch.cat([x, x], 1)[:, :n]), y)                   # strided rows
 
 
+@pytest.mark.parametrize("n", [64, 256, 4096, 5120, 28672])
+def test_online_hadamard_fp32_on_unaligned_fp16_rows(n):
+    """Contiguous rows at an odd storage offset (a slice of a flat buffer): the one-pass kernels refuse them, the conversion to fp32
+    does not mind."""
+    flat = torch.randn(5 * n + 3, device="cuda").half()
+    x = flat[3:].view(5, n)
+    had = quarot_amd.nn.OnlineHadamard(n, force_fp32=True).cuda()
+    want = quarot_amd.functional.matmul_hadU_cuda(x.float(), had.had_rem_dim, had.rem_dim).half()
+    assert x.is_contiguous() and torch.equal(had(x), want)
+
+
 @pytest.mark.parametrize("n", [256, 1024, 2048, 4096, 8192, 16384, 32768])
 @pytest.mark.parametrize("size", [300.0, 1.0, 0.1, 1e-2, 1e-3, 1e-4])
 def test_online_hadamard_fp32_on_power_of_two_fp16_rows_keeps_small_activations(n, size):
