@@ -300,7 +300,8 @@ class _AttentionStub(object):
         self.hadamard_dtype = hadamard_dtype
 
     def forward(self, q, num_kv_heads, attention_kwargs, layer_idx, max_seq_len=0, cache=None, token=None):
-        assert q.shape[1] == 1
+        _, q_len, _, _ = q.shape
+        assert q_len == 1
         if cache is None:
             return self._attend(q, attention_kwargs, layer_idx, max_seq_len, None, None)
         # the step's new token, if the cache still holds it back for this call (see MultiLayerPagedKVCache4Bit.update; otherwise it

@@ -290,3 +290,14 @@ def test_a_step_that_opens_a_page_reads_none_of_what_its_memory_held(page_size, 
             outs.append(cache.update(k, v, 0)(q))
         assert bool(torch.isfinite(outs[0]).all())
         assert all(torch.equal(y, outs[0]) for y in outs[1:]), length
+
+
+def test_a_query_without_its_head_axis_is_refused():
+    """[batch, 1, 128] where [batch, 1, heads, 128] is due: also where the cache has one head and the elements would fit."""
+    cache = kv.MultiLayerPagedKVCache4Bit(2, 16, 16, "cuda:0", 1, 1, 128)
+    k, v, q = (torch.randn(2, 1, 1, 128, device="cuda:0").half() for _ in range(3))
+    cache.update(k, v, 0)
+    call = cache.update(k, v, 0)
+    with pytest.raises(ValueError):
+        call(q[:, :, 0])
+    assert call(q).shape == q.shape
