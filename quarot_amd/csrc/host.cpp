@@ -438,12 +438,13 @@ PyObject* page_tables(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
 // graph is captured from it
 PyObject* where(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
     QR_ARGS(1)
-    const int device = device_of(tensor(a[0]));
-    if (device < 0) return none();
-    void* const st = stream(device);
+    if (!THPVariable_Check(a[0])) return none();
+    const at::Tensor& t = THPVariable_Unpack(a[0]);
+    if (!t.is_cuda()) return none();
+    void* const st = stream((int)t.device().index());
     hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
     unsigned long long id = 0;
-    if (hipStreamGetCaptureInfo((hipStream_t)st, &status, &id) != hipSuccess) (void)hipGetLastError();     // (the default stream beside a capture)
+    if (st && hipStreamGetCaptureInfo((hipStream_t)st, &status, &id) != hipSuccess) (void)hipGetLastError();     // (no capture starts on the default stream)
     if (status != hipStreamCaptureStatusActive) return PyLong_FromVoidPtr(st);
     return Py_BuildValue("(NK)", PyLong_FromVoidPtr(st), id);
     QR_END

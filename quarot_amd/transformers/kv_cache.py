@@ -302,14 +302,24 @@ class _AttentionStub(object):
     def forward(self, q, num_kv_heads, attention_kwargs, layer_idx, max_seq_len=0, cache=None, token=None):
         _, q_len, _, _ = q.shape
         assert q_len == 1
-        if cache is None:
-            return self._attend(q, attention_kwargs, layer_idx, max_seq_len, None, None)
-        # the step's new token, if the cache still holds it back for this call (see MultiLayerPagedKVCache4Bit.update; otherwise it
-        # has been stored meanwhile, or this callable was used before); a call that raises leaves it there
-        held = cache._pending.get(layer_idx)
-        if held is None or held[0] is not token:
-            held = None
-        o = self._attend(q, attention_kwargs, layer_idx, max_seq_len, cache._decode_workspace(num_kv_heads, max_seq_len), held)
+        o = workspace = held = None
+        if cache is not None:
+            # the step's new token, if the cache still holds it back for this call (see MultiLayerPagedKVCache4Bit.update; otherwise it
+            # has been stored meanwhile, or this callable was used before); a call that raises leaves it there
+            held = cache._pending.get(layer_idx)
+            if held is not None and held[0] is not token:
+                held = None
+            kept = cache._workspaces.get(_lib.host.where(cache._pages))          # (_decode_workspace's own first look, a call less)
+            if kept is not None and kept[0] == num_kv_heads and kept[1] == max_seq_len:
+                workspace = kept[2]
+            else:
+                workspace = cache._decode_workspace(num_kv_heads, max_seq_len)
+        if held is not None and self.hadamard_dtype in (None, torch.float16):
+            s = attention_kwargs
+            o = _lib.host.decode_step(s["kv_data"], s["kv_param"], s["kv_indptr"], s["kv_indices"], s["last_page_offset"], q, held[1],
+                                      held[2], layer_idx, self.hadamard_dtype is not None, held[4], max_seq_len, workspace)
+        if o is None:
+            o = self._attend(q, attention_kwargs, layer_idx, max_seq_len, workspace, held)
         if held is not None:
             cache._pending.pop(layer_idx, None)
         return o
@@ -318,12 +328,6 @@ class _AttentionStub(object):
         append = None
         if held is not None:
             _, k, v, _, k_hadamard = held
-            if self.hadamard_dtype in (None, torch.float16):
-                s = attention_kwargs
-                o = _lib.host.decode_step(s["kv_data"], s["kv_param"], s["kv_indptr"], s["kv_indices"], s["last_page_offset"], q, k, v,
-                                          layer_idx, self.hadamard_dtype is not None, k_hadamard, max_seq_len, workspace)
-                if o is not None:
-                    return o
             append = (k.view(k.shape[0], -1, k.shape[-1]), v.view(v.shape[0], -1, v.shape[-1]), k_hadamard)
         batch_size, _, num_qo_heads, head_dim = q.shape
         q = q.view(batch_size, num_qo_heads, head_dim)
@@ -464,7 +468,11 @@ class MultiLayerPagedKVCache4Bit:
             self.length = new_length
         attention_mask = cache_kwargs.get("attention_mask") if cache_kwargs else None
         first = self._needs_init[layer_idx]
-        specs = self.get_cache_specs_for_flash_infer(attention_mask)
+        made = self._specs
+        if made is not None and made[0] == self.length and attention_mask is None and type(_lib.host.where(self._pages)) is int:
+            specs = made[1]                      # (what the call below finds for a later layer, outside a capture)
+        else:
+            specs = self.get_cache_specs_for_flash_infer(attention_mask)
         if self.disable_quant:
             return self._update_f16(key_states, value_states, layer_idx, attention_mask, first, specs)
         k_in, fused_had = key_states, self.hadamard_dtype is not None
