@@ -61,10 +61,17 @@ int device_of(const at::Tensor* t) {
 }
 void* stream(int device) { return (void*)c10::hip::getCurrentHIPStream((c10::DeviceIndex)device).stream(); }
 // Allocations and launches run without the interpreter's lock: an allocation may have to give memory back first, a launch waits
-// while the queue is full, and other Python threads go on meanwhile.
+// while the queue is full, and other Python threads go on meanwhile.  Where this one is the interpreter's only thread the lock stays:
+// giving it away and taking it back costs about 0.2 us of a call's 4.5.
+bool only_thread() {
+    PyThreadState* const own = PyThreadState_Get();
+    return PyInterpreterState_ThreadHead(PyThreadState_GetInterpreter(own)) == own && !PyThreadState_Next(own);
+}
 struct Unlocked {
-    PyThreadState* const state = PyEval_SaveThread();
-    ~Unlocked() { PyEval_RestoreThread(state); }
+    PyThreadState* const state = only_thread() ? nullptr : PyEval_SaveThread();
+    ~Unlocked() {
+        if (state) PyEval_RestoreThread(state);
+    }
 };
 at::Tensor fresh(at::IntArrayRef sizes, at::ScalarType dtype, int device) {
     return at::empty(sizes, at::TensorOptions().dtype(dtype).device(at::Device(at::kCUDA, (c10::DeviceIndex)device)));
