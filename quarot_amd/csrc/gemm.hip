@@ -18,7 +18,8 @@
 // takes 4; measured on MI355X, up to ~5 VALU ops per MFMA are hidden.  Unpacking costs 3 VALU ops per
 // packed dword, i.e. 6 (IM + JN) / (IM JN) per MFMA for a wave tile of IM x JN MFMA tiles: 64x128 per
 // wave (4.5) is the smallest tile that fits where the matrix pipe is to stay busy.  (Outputs of few tiles, bound by
-// the CUs' intake of operands instead, take the 64x64 wave tiles of gemm_mid.hip.)
+// the CUs' intake of operands instead, take the 64x64 wave tiles of gemm_mid.hip, and those that fill the CUs with large tiles
+// the FP6 matrix path, gemm_e2m3.hip.)
 #include "qr_common.h"
 #include "qr_epilogue.h"
 #include <type_traits>
@@ -288,760 +289,6 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void gemm_i4_kernel(
             }
         }
     }
-}
-
-// ------------------------------------------------------------------------------------------------
-// Software-pipelined kernels: four waves, ONE per SIMD, each owning a 128x128 wave tile (16 MFMA
-// tiles, all 256 AGPRs), so that unpacking costs 3 instructions per MFMA.  A wave hides its own LDS
-// latency and unpacking under its own MFMAs: while the 32 MFMAs of a 64-k sub-step run, the packed
-// fragments of its next sub-step are read from LDS and unpacked.  The loop is written as explicit
-// slots -- one MFMA, up to 4 unpacking instructions, at most one LDS read / LDS write / global
-// load -- and a full scheduling barrier after every slot keeps the compiler from regrouping them
-// (measured for one wave per SIMD: up to 5 VALU per MFMA cost 9 %, 6 cost 40 %).  A stage is 256 k
-// (a 128-byte line per row); two LDS stage buffers; global loads are raw buffer loads (scalar
-// descriptor + scalar stage offset + constant 32-bit lane offset: no address arithmetic in the loop)
-// running ahead in registers; one workgroup barrier per stage.
-//   gemm_sp256_kernel  256x256 tile, waves 2 (M) x 2 (N), whole K per wave: shapes with many tiles.  Also as a
-//                      192x256 tile (wave tiles of 96x128: 12 MFMA tiles, 3.5 unpacking instructions per
-//                      MFMA) for shapes that 256-row tiles spread over a fraction of the CUs and 128-row
-//                      tiles over a round and a bit (2048 tokens against 5120 weight rows: 160 / 220 /
-//                      320 tiles of 256 / 192 / 128 rows on 256 CUs).
-//   gemm_spk_kernel    128x256 tile (one per CU at M = 2048, N = 4096), waves 2 (N) x 2 (K): the two
-//                      K-groups take alternate pairs of sub-steps and exchange half of their
-//                      accumulators through LDS at the end.
-// Row and column of tile `unit` of a grid of tiles: columns of eight row tiles in turn, so that tiles in flight together
-// share rows of both operands in an XCD's L2.
-struct TilePlace {
-    int tm, tn;
-};
-__device__ __forceinline__ TilePlace tile_place(int unit, int tiles_m, int tiles_n) {
-    constexpr int GROUP_M = 8;
-    const int group_sz = GROUP_M * tiles_n;
-    const int g = unit / group_sz;
-    const int gm0 = g * GROUP_M;
-    const int gh = (tiles_m - gm0) < GROUP_M ? (tiles_m - gm0) : GROUP_M;
-    return TilePlace{gm0 + (unit - g * group_sz) % gh, (unit - g * group_sz) / gh};
-}
-
-template <bool DEQ, bool RAGGED, int BM>
-__device__ __forceinline__ void sp256_tile(
-    const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, int M, int N, int Kb, int32_t* __restrict__ C,
-    f16* __restrict__ Y, const f16* __restrict__ sA, const f16* __restrict__ sB, const f16* __restrict__ bias,
-    int m0, int n0) {
-    static_assert(BM == 256 || BM == 192, "wave tiles of 4 or 3 accumulator tiles along M");
-    constexpr int BN = 256, NT = 256;
-    constexpr int TM = BM / 2, TN = 128, IM = TM / 32, JN = 4;
-    constexpr int CH = (BM + BN) * 8;                       // 16-byte chunks per stage
-    constexpr int NL = CH / NT;                             // 16 (14) per thread
-    constexpr int NF = IM + JN;                             // fragments per sub-step
-    constexpr int NMF = 2 * IM * JN;                        // MFMAs (= slots) per sub-step
-    constexpr int UNP = NF * 12;                            // unpacking instructions per sub-step
-    constexpr int S0 = 4;                                   // first slot that unpacks (LDS reads are issued in slots 0..7, in fragment order)
-    constexpr bool DIRECT = !RAGGED;                        // whole stages go straight into LDS (see gemm_spk_kernel)
-    extern __shared__ u32x4 sp2_lds[];                       // [2][CH]; later the output slabs
-
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wm = wave >> 1, wn = wave & 1;
-    const int khalf = lane >> 5;
-    const int stages = (Kb + 127) / 128;
-    auto slot8 = [](int row, int chunk) { return row * 8 + (chunk ^ ((row >> 1) & 7)); };
-
-    // staging: chunk id = tid + i * 256: row = tid / 8 + 32 i, piece tid % 8
-    const int srow = tid >> 3;
-    const int scoff = (tid & 7) * 16;
-    const int dst0 = slot8(srow, tid & 7);                  // rows differ by multiples of 32: same swizzle key
-    u32 goff[NL];
-#pragma unroll
-    for (int i = 0; i < NL; ++i) {
-        const int row = srow + i * 32;
-        int gr = row < BM ? m0 + row : n0 + row - BM;
-        const int lim = row < BM ? M - 1 : N - 1;
-        gr = gr < lim ? gr : lim;
-        goff[i] = (u32)gr * (u32)Kb + (RAGGED ? 0u : DIRECT ? (u32)(((tid & 7) ^ ((srow >> 1) & 7)) * 16) : (u32)scoff);
-    }
-    u32x4 regs[1][NL];                                      // one set: loads run one (long) stage ahead of their LDS write
-    // One 16-byte chunk of stage st (branch-free: stages past the end repeat the last one), as a raw
-    // buffer load: scalar descriptor + scalar stage offset + constant 32-bit per-thread offset, so
-    // the address costs no vector instruction and half the address traffic of a 64-bit pointer.
-    const __amdgpu_buffer_rsrc_t rsrc_a = __builtin_amdgcn_make_buffer_rsrc((void*)A, 0, (int)((u32)M * (u32)Kb), 0x00020000);
-    const __amdgpu_buffer_rsrc_t rsrc_b = __builtin_amdgcn_make_buffer_rsrc((void*)B, 0, (int)((u32)N * (u32)Kb), 0x00020000);
-    auto fetch1 = [&](int st, int set, int i) {
-        const int kb = (st < stages ? st : stages - 1) * 128;
-        u32 off = goff[i];
-        if (RAGGED) off += (u32)((kb + scoff < Kb) ? scoff : 0);
-        regs[set][i] = (i * 32 < BM) ? __builtin_amdgcn_raw_buffer_load_b128(rsrc_a, off, kb, 0)
-                                     : __builtin_amdgcn_raw_buffer_load_b128(rsrc_b, off, kb, 0);
-    };
-    auto deposit1 = [&](int st, int buf, int set, int i) {    // st past the end: a repeat of the last stage, never read
-        const bool dead = RAGGED && st >= stages - 1 && (stages - 1) * 128 + scoff >= Kb;
-        sp2_lds[buf * CH + dst0 + i * 32 * 8] = dead ? u32x4{0, 0, 0, 0} : regs[set][i];
-    };
-
-    // direct form: chunk i of stage st into stage buffer buf (a wave's 64 lanes fill 1 KB of consecutive LDS)
-    const int wave_u = __builtin_amdgcn_readfirstlane(wave);
-    auto dma1 = [&](int st, int buf, int i) {
-        const int kb = (st < stages ? st : stages - 1) * 128;
-        __attribute__((address_space(3))) void* dst =
-            (__attribute__((address_space(3))) void*)(sp2_lds + buf * CH + i * NT + wave_u * 64);
-        // (off: a plain u32 -- goff's bound depends on a template parameter, and with such an operand the
-        // host pass silently drops the kernel's stub)
-        const u32 off = goff[i];
-        if (i * 32 < BM) __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_a, dst, 16, off, kb, 0, 0);
-        else __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_b, dst, 16, off, kb, 0, 0);
-    };
-
-    i32x16 acc[IM][JN];
-#pragma unroll
-    for (int i = 0; i < IM; ++i)
-#pragma unroll
-        for (int j = 0; j < JN; ++j)
-#pragma unroll
-            for (int v = 0; v < 16; ++v) acc[i][j][v] = 0;
-
-    // fragment slots of sub-step u: logical chunk 2 u + khalf
-    int aslot[4], bslot[4];
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-        aslot[u] = slot8(wm * TM + (lane & 31), 2 * u + khalf);
-        bslot[u] = slot8(BM + wn * TN + (lane & 31), 2 * u + khalf);
-    }
-    // fragments: index 0..1 = A (32-row tiles of the wave tile), 2..5 = B
-    struct Packed {
-        u32x4 f[IM + JN];
-    };
-    struct Ops {
-        i32x4 lo[IM + JN], hi[IM + JN];
-    };
-    auto read1 = [&](int buf, int u, int r, Packed& p) {
-        p.f[r] = r < IM ? sp2_lds[buf * CH + aslot[u] + r * 32 * 8] : sp2_lds[buf * CH + bslot[u] + (r - IM) * 32 * 8];
-    };
-    // unpacking as UNP single instructions: dword d = n / 3 of the packed dwords,
-    // n % 3 = 0: lo = p << 4;  1: lo &= mask;  2: hi = p & mask
-    auto unpack1 = [&](const Packed& p, Ops& o, int n) {
-        const int d = n / 3, f = d >> 2, e = d & 3, kind = n % 3;
-        if (kind == 0) o.lo[f][e] = (int)(p.f[f][e] << 4);
-        else if (kind == 1) o.lo[f][e] = o.lo[f][e] & (int)0xF0F0F0F0u;
-        else o.hi[f][e] = (int)(p.f[f][e] & 0xF0F0F0F0u);
-    };
-    auto mfma1 = [&](const Ops& o, int q) {
-        const int t = q % (IM * JN), i = t / JN, j = t % JN;
-        if (q < IM * JN) acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(o.lo[IM + j], o.lo[i], acc[i][j], 0, 0, 0);
-        else acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(o.hi[IM + j], o.hi[i], acc[i][j], 0, 0, 0);
-    };
-    // One 64-k sub-step = NMF = 32 slots.  Slot q: MFMA q of the current operands; slots 0..7 read
-    // the packed fragments of the NEXT sub-step (one fragment buffer), slots S0.. unpack them
-    // (UNP / (NMF - S0) = 4 instructions per slot); slots 8.. of sub-step 0 also write one chunk of
-    // stage ks+1 to LDS each, slots 8.. of sub-step 1 request the same chunks of stage ks+2 (at most
-    // one memory instruction per slot).  A full scheduling barrier after every slot keeps this order.
-#define QR_SP2_SUBSTEP(CUR, NXT, RBUF, RU, DEP, FET)                                             \
-    _Pragma("unroll") for (int q_ = 0; q_ < NMF; ++q_) {                                         \
-        mfma1(CUR, q_);                                                                          \
-        if (q_ < NF) read1(RBUF, RU, q_, pk);                                                    \
-        if (q_ >= S0) {                                                                          \
-            _Pragma("unroll") for (int n_ = ((q_ - S0) * UNP) / (NMF - S0); n_ < ((q_ - S0 + 1) * UNP) / (NMF - S0); ++n_) \
-                unpack1(pk, NXT, n_);                                                            \
-        }                                                                                        \
-        if ((DEP) && q_ >= 8 && q_ < 8 + NL) deposit1(ks + 1, nb, 0, q_ - 8);                    \
-        if ((FET) && q_ >= 8 && q_ < 8 + NL) fetch1(ks + 2, 0, q_ - 8);                          \
-        __builtin_amdgcn_sched_barrier(0);                                                       \
-    }
-
-    Packed pk;
-    Ops ops[2];
-    if constexpr (DIRECT) {
-        // Two stage buffers.  Sub-step 0 of stage s is read during sub-step 3 of stage s - 1, the rest
-        // during sub-steps 0..2 of stage s; after the barrier of stage s (before its sub-step 3) nobody
-        // reads buffer s % 2 any more, and the loads of stage s + 2 into it are issued in that sub-step 3:
-        // they have three sub-steps (~2 us) to land before the next barrier, which waits for all of this
-        // wave's loads.
-#define QR_SP2D_BARRIER(ALLOWED)                                                                 \
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(ALLOWED) : "memory");
-#define QR_SP2D_SUBSTEP(CUR, NXT, RBUF, RU, FET)                                                 \
-    _Pragma("unroll") for (int q_ = 0; q_ < NMF; ++q_) {                                         \
-        mfma1(CUR, q_);                                                                          \
-        if (q_ < NF) read1(RBUF, RU, q_, pk);                                                    \
-        if (q_ >= S0) {                                                                          \
-            _Pragma("unroll") for (int n_ = ((q_ - S0) * UNP) / (NMF - S0); n_ < ((q_ - S0 + 1) * UNP) / (NMF - S0); ++n_) \
-                unpack1(pk, NXT, n_);                                                            \
-        }                                                                                        \
-        if ((FET) && q_ >= 8 && q_ < 8 + NL) dma1(ks + 2, b, q_ - 8);                            \
-        __builtin_amdgcn_sched_barrier(0);                                                       \
-    }
-#pragma unroll
-        for (int i = 0; i < NL; ++i) dma1(0, 0, i);
-#pragma unroll
-        for (int i = 0; i < NL; ++i) dma1(1, 1, i);
-        QR_SP2D_BARRIER(NL)
-#pragma unroll
-        for (int r = 0; r < NF; ++r) read1(0, 0, r, pk);
-#pragma unroll
-        for (int n = 0; n < UNP; ++n) unpack1(pk, ops[0], n);
-        for (int ks = 0; ks < stages; ++ks) {
-            const int b = ks & 1, nb = b ^ 1;
-            QR_SP2D_SUBSTEP(ops[0], ops[1], b, 1, false)
-            QR_SP2D_SUBSTEP(ops[1], ops[0], b, 2, false)
-            QR_SP2D_SUBSTEP(ops[0], ops[1], b, 3, false)
-            QR_SP2D_BARRIER(0)                              // stage ks+1 landed; stage ks fully read
-            QR_SP2D_SUBSTEP(ops[1], ops[0], nb, 0, true)
-        }
-#undef QR_SP2D_SUBSTEP
-#undef QR_SP2D_BARRIER
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");    // repeats of the last stage still landing
-    } else {
-    // prologue: stage 0 into LDS, stage 1 requested; sub-step 0 unpacked
-#pragma unroll
-    for (int i = 0; i < NL; ++i) fetch1(0, 0, i);
-#pragma unroll
-    for (int i = 0; i < NL; ++i) deposit1(0, 0, 0, i);
-#pragma unroll
-    for (int i = 0; i < NL; ++i) fetch1(1, 0, i);
-    __syncthreads();
-#pragma unroll
-    for (int r = 0; r < NF; ++r) read1(0, 0, r, pk);
-#pragma unroll
-    for (int n = 0; n < UNP; ++n) unpack1(pk, ops[0], n);
-    for (int ks = 0; ks < stages; ++ks) {
-        const int b = ks & 1, nb = b ^ 1;
-        // sub-step 0: multiply (ks,0); read + unpack (ks,1); stage ks+1 -> LDS, request ks+2
-        QR_SP2_SUBSTEP(ops[0], ops[1], b, 1, true, false)
-        // sub-step 1: multiply (ks,1); read + unpack (ks,2); request ks+2 into the registers just written out
-        QR_SP2_SUBSTEP(ops[1], ops[0], b, 2, false, true)
-        // sub-step 2: multiply (ks,2); read + unpack (ks,3)
-        QR_SP2_SUBSTEP(ops[0], ops[1], b, 3, false, false)
-        __syncthreads();                                    // stage ks+1 visible; stage ks fully read
-        // sub-step 3: multiply (ks,3); read + unpack (ks+1,0)
-        QR_SP2_SUBSTEP(ops[1], ops[0], nb, 0, false, false)
-    }
-    }
-#undef QR_SP2_SUBSTEP
-    __syncthreads();                                        // stage buffers free for the output slabs
-
-    // Epilogue: lane l, register v -> n = (v/4)*8 + (l/32)*4 + v%4, m = l%32.
-    const bool by_rows = DEQ && n0 + BN <= N && (N & 7) == 0 && (((uintptr_t)Y) & 15) == 0;
-    if (DEQ && by_rows) {
-#pragma unroll
-        for (int jb = 0; jb < JN; jb += 2) {
-            f16x4 sbh[2][4], bih[2][4];
-#pragma unroll
-            for (int jj = 0; jj < 2; ++jj)
-#pragma unroll
-                for (int gq = 0; gq < 4; ++gq) {
-                    const int col = n0 + wn * TN + (jb + jj) * 32 + gq * 8 + khalf * 4;
-                    sbh[jj][gq] = *(const f16x4*)(sB + col);
-                    bih[jj][gq] = bias ? *(const f16x4*)(bias + col) : f16x4{(f16)0, (f16)0, (f16)0, (f16)0};
-                }
-#pragma unroll
-            for (int i = 0; i < IM; ++i) {
-                const int row0 = m0 + wm * TM + i * 32;       // (rows past M: computed on a clamped scale, not stored)
-                if (row0 >= M) continue;
-                const f16 sa = sA[min(row0 + (lane & 31), M - 1)];
-                f16x4 o[2][4];
-#pragma unroll
-                for (int jj = 0; jj < 2; ++jj)
-#pragma unroll
-                    for (int gq = 0; gq < 4; ++gq)
-                        o[jj][gq] = dequant4(acc[i][jb + jj][gq * 4], acc[i][jb + jj][gq * 4 + 1], acc[i][jb + jj][gq * 4 + 2],
-                                             acc[i][jb + jj][gq * 4 + 3], sa, sbh[jj][gq], bih[jj][gq], bias != nullptr);
-                store_slab_rows<2>((u32x2*)(sp2_lds + wave * 256), o, lane,
-                                   Y + (int64_t)row0 * N + n0 + wn * TN + jb * 32, N, M - row0);
-            }
-        }
-        return;
-    }
-#pragma unroll
-    for (int i = 0; i < IM; ++i) {
-        const int row = m0 + wm * TM + i * 32 + (lane & 31);
-        if (row >= M) continue;
-        f16 sa = (f16)0;
-        if (DEQ) sa = sA[row];
-#pragma unroll
-        for (int j = 0; j < JN; ++j) {
-#pragma unroll
-            for (int gq = 0; gq < 4; ++gq) {
-                const int col = n0 + wn * TN + j * 32 + gq * 8 + khalf * 4;
-                if (col >= N) continue;
-                int v4[4];
-#pragma unroll
-                for (int e = 0; e < 4; ++e) v4[e] = acc[i][j][gq * 4 + e] >> 8;
-                if (DEQ) {
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        if (col + e < N) {
-                            f16 yv = (f16)(sa * sB[col + e]) * (f16)(float)v4[e];
-                            if (bias) yv = yv + bias[col + e];
-                            Y[(int64_t)row * N + col + e] = yv;
-                        }
-                    }
-                } else {
-#pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        if (col + e < N) C[(int64_t)row * N + col + e] = v4[e];
-                }
-            }
-        }
-    }
-}
-
-template <bool DEQ, bool RAGGED>
-__device__ __forceinline__ void spk_tile(
-    const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, int M, int N, int Kb, int32_t* __restrict__ C,
-    f16* __restrict__ Y, const f16* __restrict__ sA, const f16* __restrict__ sB, const f16* __restrict__ bias,
-    int m0, int n0) {
-    constexpr int BM = 128, BN = 256, NT = 256;
-    constexpr int TM = 128, TN = 128, IM = 4, JN = 4;
-    constexpr int CH = (BM + BN) * 8;                       // 16-byte chunks per stage
-    constexpr int NL = CH / NT;                             // 12 per thread
-    constexpr int NF = IM + JN;                             // fragments per sub-step
-    constexpr int NMF = 2 * IM * JN;                        // MFMAs (= slots) per sub-step
-    constexpr int UNP = NF * 12;                            // unpacking instructions per sub-step
-    constexpr int S0 = 4;                                   // first slot that unpacks (LDS reads are issued in slots 0..7, in fragment order)
-    // Whole stages (K % 256 == 0) go from global memory straight into LDS (buffer_load ... lds, 16
-    // bytes per lane): no staging registers, no LDS write instructions, a third stage buffer instead.
-    // Measured 3-5 % faster than the register-staged form (kept for ragged K, where dead pieces must
-    // be written as zeros) at M = 2048, N = 4096, K = 11008 and K = 4096.
-    constexpr bool DIRECT = !RAGGED;
-    extern __shared__ u32x4 spk_lds[];                       // [DIRECT ? 3 : 2][CH]; later the output slabs
-
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wm = 0, wn = wave & 1, kg = wave >> 1;        // K-group kg multiplies sub-steps 2 kg and 2 kg + 1 of every stage
-    const int khalf = lane >> 5;
-    const int stages = (Kb + 127) / 128;
-    auto slot8 = [](int row, int chunk) { return row * 8 + (chunk ^ ((row >> 1) & 7)); };
-
-    // staging: chunk id = tid + i * 256: row = tid / 8 + 32 i, piece tid % 8
-    const int srow = tid >> 3;
-    const int scoff = (tid & 7) * 16;
-    const int dst0 = slot8(srow, tid & 7);                  // rows differ by multiples of 32: same swizzle key
-    u32 goff[NL];
-#pragma unroll
-    for (int i = 0; i < NL; ++i) {
-        const int row = srow + i * 32;
-        int gr = row < BM ? m0 + row : n0 + row - BM;
-        const int lim = row < BM ? M - 1 : N - 1;
-        gr = gr < lim ? gr : lim;
-        // direct form: a lane's data lands at LDS position (row, tid % 8), so the lane fetches the
-        // piece that the XOR-keyed layout keeps there (the key is the same for all of a lane's rows)
-        goff[i] = (u32)gr * (u32)Kb + (RAGGED ? 0u : DIRECT ? (u32)(((tid & 7) ^ ((srow >> 1) & 7)) * 16) : (u32)scoff);
-    }
-    u32x4 regs[2][NL];                                      // two sets: loads run two stages ahead of their LDS write
-    // One 16-byte chunk of stage st (branch-free: stages past the end repeat the last one), as a raw
-    // buffer load: scalar descriptor + scalar stage offset + constant 32-bit per-thread offset, so
-    // the address costs no vector instruction and half the address traffic of a 64-bit pointer.
-    const __amdgpu_buffer_rsrc_t rsrc_a = __builtin_amdgcn_make_buffer_rsrc((void*)A, 0, (int)((u32)M * (u32)Kb), 0x00020000);
-    const __amdgpu_buffer_rsrc_t rsrc_b = __builtin_amdgcn_make_buffer_rsrc((void*)B, 0, (int)((u32)N * (u32)Kb), 0x00020000);
-    auto fetch1 = [&](int st, int set, int i) {
-        const int kb = (st < stages ? st : stages - 1) * 128;
-        u32 off = goff[i];
-        if (RAGGED) off += (u32)((kb + scoff < Kb) ? scoff : 0);
-        regs[set][i] = (i * 32 < BM) ? __builtin_amdgcn_raw_buffer_load_b128(rsrc_a, off, kb, 0)
-                                     : __builtin_amdgcn_raw_buffer_load_b128(rsrc_b, off, kb, 0);
-    };
-    auto deposit1 = [&](int st, int buf, int set, int i) {    // st past the end: a repeat of the last stage, never read
-        const bool dead = RAGGED && st >= stages - 1 && (stages - 1) * 128 + scoff >= Kb;
-        spk_lds[buf * CH + dst0 + i * 32 * 8] = dead ? u32x4{0, 0, 0, 0} : regs[set][i];
-    };
-
-    // direct form: chunk i of stage st into stage buffer buf; a wave's 64 lanes fill 1 KB of consecutive
-    // LDS (8 rows of 128 bytes).  Stages past the end repeat the last one into a buffer nobody reads, so
-    // that every stage issues the same number of loads (the waits below count them).
-    const int wave_u = __builtin_amdgcn_readfirstlane(wave);
-    auto dma1 = [&](int st, int buf, int i) {
-        const int kb = (st < stages ? st : stages - 1) * 128;
-        __attribute__((address_space(3))) void* dst =
-            (__attribute__((address_space(3))) void*)(spk_lds + buf * CH + i * NT + wave_u * 64);
-        if (i * 32 < BM) __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_a, dst, 16, goff[i], kb, 0, 0);
-        else __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_b, dst, 16, goff[i], kb, 0, 0);
-    };
-
-    i32x16 acc[IM][JN];
-#pragma unroll
-    for (int i = 0; i < IM; ++i)
-#pragma unroll
-        for (int j = 0; j < JN; ++j)
-#pragma unroll
-            for (int v = 0; v < 16; ++v) acc[i][j][v] = 0;
-
-    // fragment slots of this wave's two sub-steps u0 = 2 kg, u1 = 2 kg + 1: logical chunk 2 u + khalf
-    const int u0 = 2 * kg, u1 = 2 * kg + 1;
-    const int aslot0 = slot8(wm * TM + (lane & 31), 2 * u0 + khalf), aslot1 = slot8(wm * TM + (lane & 31), 2 * u1 + khalf);
-    const int bslot0 = slot8(BM + wn * TN + (lane & 31), 2 * u0 + khalf), bslot1 = slot8(BM + wn * TN + (lane & 31), 2 * u1 + khalf);
-    // fragments: index 0..1 = A (32-row tiles of the wave tile), 2..5 = B
-    struct Packed {
-        u32x4 f[IM + JN];
-    };
-    struct Ops {
-        i32x4 lo[IM + JN], hi[IM + JN];
-    };
-    // K-group 1 holds its B fragments (and so its accumulator columns) with the two 64-column halves
-    // swapped: either group then KEEPS accumulator tiles j = 0, 1 and SENDS j = 2, 3, with
-    // compile-time register indices on both sides
-    const int bswap = kg * 64 * 8;                          // LDS offset of 64 rows
-    auto read1 = [&](int buf, int second, int r, Packed& p) {  // second: sub-step u1 rather than u0
-        const int as = second ? aslot1 : aslot0, bs = second ? bslot1 : bslot0;
-        if (r < IM) p.f[r] = spk_lds[buf * CH + as + r * 32 * 8];
-        else p.f[r] = spk_lds[buf * CH + bs + ((r - IM) * 32 * 8 ^ bswap)];
-    };
-    // unpacking as UNP single instructions: dword d = n / 3 of the packed dwords,
-    // n % 3 = 0: lo = p << 4;  1: lo &= mask;  2: hi = p & mask
-    auto unpack1 = [&](const Packed& p, Ops& o, int n) {
-        const int d = n / 3, f = d >> 2, e = d & 3, kind = n % 3;
-        if (kind == 0) o.lo[f][e] = (int)(p.f[f][e] << 4);
-        else if (kind == 1) o.lo[f][e] = o.lo[f][e] & (int)0xF0F0F0F0u;
-        else o.hi[f][e] = (int)(p.f[f][e] & 0xF0F0F0F0u);
-    };
-    auto mfma1 = [&](const Ops& o, int q) {
-        const int t = q % (IM * JN), i = t / JN, j = t % JN;
-        if (q < IM * JN) acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(o.lo[IM + j], o.lo[i], acc[i][j], 0, 0, 0);
-        else acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(o.hi[IM + j], o.hi[i], acc[i][j], 0, 0, 0);
-    };
-    // One 64-k sub-step = NMF = 32 slots.  Slot q: MFMA q of the current operands; slots 0..7 read
-    // the packed fragments of this wave's NEXT sub-step (one fragment buffer), slots S0.. unpack
-    // them (4 instructions per slot); slots 8.. of a stage's first sub-step also write one chunk
-    // of stage ks+1 to LDS each, slots 8.. of its second sub-step request the same chunks of stage
-    // ks+3 (one memory instruction per slot at most).  A full scheduling barrier after every slot
-    // keeps this order.
-#define QR_SPK_SUBSTEP(CUR, NXT, RBUF, RU, DEP, FET, SET)                                        \
-    _Pragma("unroll") for (int q_ = 0; q_ < NMF; ++q_) {                                         \
-        mfma1(CUR, q_);                                                                          \
-        if (q_ < NF) read1(RBUF, RU, q_, pk);                                                    \
-        if (q_ >= S0) {                                                                          \
-            _Pragma("unroll") for (int n_ = ((q_ - S0) * UNP) / (NMF - S0); n_ < ((q_ - S0 + 1) * UNP) / (NMF - S0); ++n_) \
-                unpack1(pk, NXT, n_);                                                            \
-        }                                                                                        \
-        if ((DEP) && q_ >= 8 && q_ < 8 + NL) deposit1(ks_ + 1, nb_, SET, q_ - 8);                \
-        if ((FET) && q_ >= 8 && q_ < 8 + NL) fetch1(ks_ + 3, SET, q_ - 8);                       \
-        __builtin_amdgcn_sched_barrier(0);                                                       \
-    }
-    // one stage: KS = stage index, B = its LDS buffer (compile-time), SET = register set that holds
-    // stage KS+1 on entry and receives stage KS+3
-#define QR_SPK_STAGE(KS, B, SET)                                                                 \
-    {                                                                                            \
-        const int ks_ = (KS);                                                                    \
-        constexpr int b_ = (B), nb_ = 1 - (B);                                                   \
-        /* first sub-step: multiply (ks,u0); read + unpack (ks,u1); stage ks+1 -> LDS */         \
-        QR_SPK_SUBSTEP(ops[0], ops[1], b_, 1, true, false, SET)                                  \
-        __syncthreads(); /* stage ks+1 visible; stage ks fully read */                           \
-        /* second sub-step: multiply (ks,u1); read + unpack (ks+1,u0); request ks+3 */           \
-        QR_SPK_SUBSTEP(ops[1], ops[0], nb_, 0, false, true, SET)                                 \
-    }
-
-    Packed pk;
-    Ops ops[2];
-    if constexpr (DIRECT) {
-        // Three stage buffers.  Stage s lives in buffer s % 3; its sub-step u0 is read during the second
-        // sub-step of stage s - 1, its sub-step u1 during the first sub-step of stage s; the barrier
-        // of stage s (between its two sub-steps) is the last point at which anybody reads buffer
-        // s % 3, and the loads of stage s + 3 into it are issued right after.  A wave's loads complete
-        // in order, so "at most NL outstanding" at the barrier of stage s means its part of stage
-        // s + 1 has landed (only stage s + 2 may still be in flight); the barrier then covers the other
-        // waves' parts.  The wait is written by hand: the compiler would wait for all loads.
-#define QR_SPKD_BARRIER(ALLOWED)                                                                 \
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(ALLOWED) : "memory");
-#define QR_SPKD_SUBSTEP(CUR, NXT, RBUF, RU, FET, FBUF)                                           \
-    _Pragma("unroll") for (int q_ = 0; q_ < NMF; ++q_) {                                         \
-        mfma1(CUR, q_);                                                                          \
-        if (q_ < NF) read1(RBUF, RU, q_, pk);                                                    \
-        if (q_ >= S0) {                                                                          \
-            _Pragma("unroll") for (int n_ = ((q_ - S0) * UNP) / (NMF - S0); n_ < ((q_ - S0 + 1) * UNP) / (NMF - S0); ++n_) \
-                unpack1(pk, NXT, n_);                                                            \
-        }                                                                                        \
-        if ((FET) && q_ >= 8 && q_ < 8 + NL) dma1(ks_ + 3, FBUF, q_ - 8);                        \
-        __builtin_amdgcn_sched_barrier(0);                                                       \
-    }
-#define QR_SPKD_STAGE(KS, B)                                                                     \
-    {                                                                                            \
-        const int ks_ = (KS);                                                                    \
-        constexpr int b_ = (B), nb_ = ((B) + 1) % 3;                                             \
-        /* multiply (ks,u0); read + unpack (ks,u1) */                                            \
-        QR_SPKD_SUBSTEP(ops[0], ops[1], b_, 1, false, b_)                                        \
-        QR_SPKD_BARRIER(NL) /* stage ks+1 landed; buffer b_ fully read */                        \
-        /* multiply (ks,u1); read + unpack (ks+1,u0); stage ks+3 -> buffer b_ */                 \
-        QR_SPKD_SUBSTEP(ops[1], ops[0], nb_, 0, true, b_)                                        \
-    }
-#pragma unroll
-        for (int i = 0; i < NL; ++i) dma1(0, 0, i);
-#pragma unroll
-        for (int i = 0; i < NL; ++i) dma1(1, 1, i);
-#pragma unroll
-        for (int i = 0; i < NL; ++i) dma1(2, 2, i);
-        QR_SPKD_BARRIER(2 * NL)
-#pragma unroll
-        for (int r = 0; r < NF; ++r) read1(0, 0, r, pk);
-#pragma unroll
-        for (int n = 0; n < UNP; ++n) unpack1(pk, ops[0], n);
-        int ks = 0;
-        for (; ks + 2 < stages; ks += 3) {
-            QR_SPKD_STAGE(ks, 0)
-            QR_SPKD_STAGE(ks + 1, 1)
-            QR_SPKD_STAGE(ks + 2, 2)
-        }
-        if (ks < stages) {
-            QR_SPKD_STAGE(ks, 0)
-            if (ks + 1 < stages) QR_SPKD_STAGE(ks + 1, 1)
-        }
-#undef QR_SPKD_STAGE
-#undef QR_SPKD_SUBSTEP
-#undef QR_SPKD_BARRIER
-        // the repeats of the last stage are still landing in the stage buffers, which the epilogue reuses
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    } else {
-    // prologue: stage 0 into LDS, stages 1 and 2 requested; this wave's first sub-step unpacked
-#pragma unroll
-    for (int i = 0; i < NL; ++i) fetch1(0, 0, i);
-#pragma unroll
-    for (int i = 0; i < NL; ++i) fetch1(2, 1, i);
-#pragma unroll
-    for (int i = 0; i < NL; ++i) deposit1(0, 0, 0, i);
-#pragma unroll
-    for (int i = 0; i < NL; ++i) fetch1(1, 0, i);
-    __syncthreads();
-#pragma unroll
-    for (int r = 0; r < NF; ++r) read1(0, 0, r, pk);
-#pragma unroll
-    for (int n = 0; n < UNP; ++n) unpack1(pk, ops[0], n);
-    // (pairs of stages without a branch in between: the wait before an LDS write then counts the
-    // other set's loads as still allowed in flight)
-    int ks = 0;
-    for (; ks + 1 < stages; ks += 2) {
-        QR_SPK_STAGE(ks, 0, 0)
-        QR_SPK_STAGE(ks + 1, 1, 1)
-    }
-    if (ks < stages) QR_SPK_STAGE(ks, 0, 0)
-    }
-#undef QR_SPK_STAGE
-#undef QR_SPK_SUBSTEP
-
-    // K-split: the two K-groups hold partial sums of the same 128x128 wave tile.  Each finalises the
-    // 64 output columns held in its accumulator tiles j = 0, 1 (group 0: columns 0..63 of the wave
-    // tile, group 1: 64..127) and sends tiles j = 2, 3 across through LDS, two 32-row tiles (i) per
-    // round, four 16-byte pieces per lane and tile.
-    {
-        // (all four 32-row tiles in one round: 32 KB per wave, 128 KB of the stage buffers' 144 KB in the direct form;
-        // the register-staged form has 96 KB of LDS and takes two rounds)
-        u32x4* xbuf = spk_lds;
-        constexpr int IR = DIRECT ? IM : 2;                   // 32-row tiles per round
-#pragma unroll
-        for (int ip = 0; ip < IM; ip += IR) {
-            __syncthreads();
-#pragma unroll
-            for (int ii = 0; ii < IR; ++ii)
-#pragma unroll
-                for (int jj = 0; jj < 2; ++jj)
-#pragma unroll
-                    for (int qv = 0; qv < 4; ++qv) {
-                        const i32x16& t = acc[ip + ii][2 + jj];
-                        xbuf[((((wn * 2 + (1 - kg)) * IR + ii) * 2 + jj) * 4 + qv) * 64 + lane] =
-                            u32x4{(u32)t[qv * 4], (u32)t[qv * 4 + 1], (u32)t[qv * 4 + 2], (u32)t[qv * 4 + 3]};
-                    }
-            __syncthreads();
-#pragma unroll
-            for (int ii = 0; ii < IR; ++ii)
-#pragma unroll
-                for (int jj = 0; jj < 2; ++jj)
-#pragma unroll
-                    for (int qv = 0; qv < 4; ++qv) {
-                        const u32x4 piece = xbuf[((((wn * 2 + kg) * IR + ii) * 2 + jj) * 4 + qv) * 64 + lane];
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) acc[ip + ii][jj][qv * 4 + e] += (int)piece[e];
-                    }
-        }
-    }
-    __syncthreads();                                        // stage buffers free for the output slabs
-
-    // Epilogue: lane l, register v -> n = (v/4)*8 + (l/32)*4 + v%4, m = l%32.
-    const bool by_rows = DEQ && n0 + BN <= N && (N & 7) == 0 && (((uintptr_t)Y) & 15) == 0;
-    if (DEQ && by_rows) {
-        const int jb = 2 * kg;
-        {
-            f16x4 sbh[2][4], bih[2][4];
-#pragma unroll
-            for (int jj = 0; jj < 2; ++jj)
-#pragma unroll
-                for (int gq = 0; gq < 4; ++gq) {
-                    const int col = n0 + wn * TN + (jb + jj) * 32 + gq * 8 + khalf * 4;
-                    sbh[jj][gq] = *(const f16x4*)(sB + col);
-                    bih[jj][gq] = bias ? *(const f16x4*)(bias + col) : f16x4{(f16)0, (f16)0, (f16)0, (f16)0};
-                }
-#pragma unroll
-            for (int i = 0; i < IM; ++i) {
-                const int row0 = m0 + wm * TM + i * 32;       // (rows past M: computed on a clamped scale, not stored)
-                if (row0 >= M) continue;
-                const f16 sa = sA[min(row0 + (lane & 31), M - 1)];
-                f16x4 o[2][4];
-#pragma unroll
-                for (int jj = 0; jj < 2; ++jj)
-#pragma unroll
-                    for (int gq = 0; gq < 4; ++gq)
-                        o[jj][gq] = dequant4(acc[i][jj][gq * 4], acc[i][jj][gq * 4 + 1], acc[i][jj][gq * 4 + 2],
-                                             acc[i][jj][gq * 4 + 3], sa, sbh[jj][gq], bih[jj][gq], bias != nullptr);
-                store_slab_rows<2>((u32x2*)(spk_lds + wave * 256), o, lane,
-                                   Y + (int64_t)row0 * N + n0 + wn * TN + jb * 32, N, M - row0);
-            }
-        }
-        return;
-    }
-#pragma unroll
-    for (int i = 0; i < IM; ++i) {
-        const int row = m0 + wm * TM + i * 32 + (lane & 31);
-        if (row >= M) continue;
-        f16 sa = (f16)0;
-        if (DEQ) sa = sA[row];
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {                       // this K-group's tiles: output column tiles j + 2 kg
-#pragma unroll
-            for (int gq = 0; gq < 4; ++gq) {
-                const int col = n0 + wn * TN + (j + 2 * kg) * 32 + gq * 8 + khalf * 4;
-                if (col >= N) continue;
-                int v4[4];
-#pragma unroll
-                for (int e = 0; e < 4; ++e) v4[e] = acc[i][j][gq * 4 + e] >> 8;
-                if (DEQ) {
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        if (col + e < N) {
-                            f16 yv = (f16)(sa * sB[col + e]) * (f16)(float)v4[e];
-                            if (bias) yv = yv + bias[col + e];
-                            Y[(int64_t)row * N + col + e] = yv;
-                        }
-                    }
-                } else {
-#pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        if (col + e < N) C[(int64_t)row * N + col + e] = v4[e];
-                }
-            }
-        }
-    }
-}
-
-template <bool DEQ, bool RAGGED, int BM = 256>
-__global__ __launch_bounds__(256) void gemm_sp256_kernel(
-    const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, int M, int N, int Kb, int32_t* __restrict__ C,
-    f16* __restrict__ Y, const f16* __restrict__ sA, const f16* __restrict__ sB, const f16* __restrict__ bias,
-    int tiles_m, int tiles_n, int nxcd) {
-    const int per_xcd = gridDim.x / nxcd;
-    const int tile = (blockIdx.x % nxcd) * per_xcd + blockIdx.x / nxcd;
-    if (tile >= tiles_m * tiles_n) return;
-    const TilePlace p = tile_place(tile, tiles_m, tiles_n);
-    sp256_tile<DEQ, RAGGED, BM>(A, B, M, N, Kb, C, Y, sA, sB, bias, p.tm * BM, p.tn * 256);
-}
-
-template <bool DEQ, bool RAGGED>
-__global__ __launch_bounds__(256) void gemm_spk_kernel(
-    const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, int M, int N, int Kb, int32_t* __restrict__ C,
-    f16* __restrict__ Y, const f16* __restrict__ sA, const f16* __restrict__ sB, const f16* __restrict__ bias,
-    int tiles_m, int tiles_n, int nxcd) {
-    const int per_xcd = gridDim.x / nxcd;
-    const int tile = (blockIdx.x % nxcd) * per_xcd + blockIdx.x / nxcd;
-    if (tile >= tiles_m * tiles_n) return;
-    const TilePlace p = tile_place(tile, tiles_m, tiles_n);
-    spk_tile<DEQ, RAGGED>(A, B, M, N, Kb, C, Y, sA, sB, bias, p.tm * 128, p.tn * 256);
-}
-
-// Whole rounds of 256x256 tiles over the CUs, then the tiles of the last round, where they are at most half as many as
-// there are CUs, as two 128x256 tiles each: a last round of R tiles keeps cus - R CUs idle for a whole tile's time, its halves
-// fill 2 R CUs for 0.57 of it.  `whole` (a multiple of the CU count) workgroups take the whole tiles, those after them the halves; both kinds
-// need a CU to themselves (LDS), so a half starts where a whole tile has ended.
-template <bool DEQ>
-__global__ __launch_bounds__(256) void gemm_sp256_tail_kernel(
-    const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, int M, int N, int Kb, int32_t* __restrict__ C,
-    f16* __restrict__ Y, const f16* __restrict__ sA, const f16* __restrict__ sB, const f16* __restrict__ bias,
-    int tiles_m, int tiles_n, int nxcd, int whole) {
-    if ((int)blockIdx.x < whole) {
-        const TilePlace p = tile_place((blockIdx.x % nxcd) * (whole / nxcd) + blockIdx.x / nxcd, tiles_m, tiles_n);
-        sp256_tile<DEQ, false, 256>(A, B, M, N, Kb, C, Y, sA, sB, bias, p.tm * 256, p.tn * 256);
-        return;
-    }
-    const int b = blockIdx.x - whole;
-    const int unit = (b % nxcd) * (((int)gridDim.x - whole) / nxcd) + b / nxcd;
-    if (whole + unit / 2 >= tiles_m * tiles_n) return;
-    const TilePlace p = tile_place(whole + unit / 2, tiles_m, tiles_n);
-    const int m0 = p.tm * 256 + (unit & 1) * 128;
-    if (m0 >= M) return;
-    spk_tile<DEQ, false>(A, B, M, N, Kb, C, Y, sA, sB, bias, m0, p.tn * 256);
-}
-
-int launch_spk(const void* A, const void* B, int M, int N, int Kb, void* C, void* Y, const void* sA, const void* sB,
-               const void* bias, hipStream_t st) {
-    const int tiles_m = (M + 127) / 128, tiles_n = (N + 255) / 256;
-    const int64_t tiles = (int64_t)tiles_m * tiles_n;
-    if (tiles > 0x3fffffff) return QR_E_SHAPE;
-    const int nxcd = qr_device().xcds;                      // the grid is a whole number of rounds over the XCDs
-    const unsigned grid = (unsigned)((tiles + nxcd - 1) / nxcd * nxcd);
-    const bool ragged = (Kb & 127) != 0;
-    // stage buffers of 48 KB: two behind staging registers, three when loaded straight into LDS
-    const size_t LDS = (size_t)(ragged ? 2 : 3) * (128 + 256) * 8 * 16;
-    if ((int64_t)M * Kb >= (1LL << 32) || (int64_t)N * Kb >= (1LL << 32)) return QR_E_UNSUPPORTED;   // (the dispatcher routes these away)
-    hipError_t e;
-    if (Y) {
-        auto kern = ragged ? gemm_spk_kernel<true, true> : gemm_spk_kernel<true, false>;
-        e = qr_allow_dynamic_lds((const void*)kern, LDS);
-        if (e != hipSuccess) return (int)e;
-        kern<<<dim3(grid), dim3(256), LDS, st>>>((const uint8_t*)A, (const uint8_t*)B, M, N, Kb, nullptr, (f16*)Y,
-                                                 (const f16*)sA, (const f16*)sB, (const f16*)bias, tiles_m, tiles_n, nxcd);
-    } else {
-        auto kern = ragged ? gemm_spk_kernel<false, true> : gemm_spk_kernel<false, false>;
-        e = qr_allow_dynamic_lds((const void*)kern, LDS);
-        if (e != hipSuccess) return (int)e;
-        kern<<<dim3(grid), dim3(256), LDS, st>>>((const uint8_t*)A, (const uint8_t*)B, M, N, Kb, (int32_t*)C, nullptr,
-                                                 nullptr, nullptr, nullptr, tiles_m, tiles_n, nxcd);
-    }
-    return qr_launch_status();
-}
-
-template <int BM, int BN, int WAVES_M, int WAVES_N>
-int launch_cfg(const void* A, const void* B, int M, int N, int Kb, void* C, void* Y, const void* sA, const void* sB,
-               const void* bias, hipStream_t st);
-
-// bm: rows of a tile, 256 or 192 (192: eleven row tiles instead of eight at 2048 tokens -- shapes whose
-// 256-row tiles would occupy a fraction of the CUs and whose 128-row tiles need a second round)
-int launch_sp256(const void* A, const void* B, int M, int N, int Kb, void* C, void* Y, const void* sA, const void* sB,
-                 const void* bias, hipStream_t st, int bm = 256) {
-    const size_t LDS = (size_t)2 * (size_t)(bm + 256) * 8 * 16;
-    const int tiles_m = (M + bm - 1) / bm, tiles_n = (N + 255) / 256;
-    const int64_t tiles = (int64_t)tiles_m * tiles_n;
-    if (tiles > 0x3fffffff) return QR_E_SHAPE;
-    const int nxcd = qr_device().xcds;                      // the grid is a whole number of rounds over the XCDs
-    const unsigned grid = (unsigned)((tiles + nxcd - 1) / nxcd * nxcd);
-    const bool ragged = (Kb & 127) != 0;
-    // operands are addressed through 32-bit buffer offsets (the dispatcher routes larger ones away)
-    if ((int64_t)M * Kb >= (1LL << 32) || (int64_t)N * Kb >= (1LL << 32)) return QR_E_UNSUPPORTED;
-    using Kern = void (*)(const uint8_t*, const uint8_t*, int, int, int, int32_t*, f16*, const f16*, const f16*, const f16*,
-                          int, int, int);
-    static const Kern table[2][2][2] = {
-        {{gemm_sp256_kernel<false, false, 256>, gemm_sp256_kernel<false, true, 256>},
-         {gemm_sp256_kernel<true, false, 256>, gemm_sp256_kernel<true, true, 256>}},
-        {{gemm_sp256_kernel<false, false, 192>, gemm_sp256_kernel<false, true, 192>},
-         {gemm_sp256_kernel<true, false, 192>, gemm_sp256_kernel<true, true, 192>}}};
-    const Kern kern = table[bm == 192 ? 1 : 0][Y ? 1 : 0][ragged ? 1 : 0];
-    const hipError_t e = qr_allow_dynamic_lds((const void*)kern, LDS);
-    if (e != hipSuccess) return (int)e;
-    if (Y)
-        kern<<<dim3(grid), dim3(256), LDS, st>>>((const uint8_t*)A, (const uint8_t*)B, M, N, Kb, nullptr, (f16*)Y,
-                                                 (const f16*)sA, (const f16*)sB, (const f16*)bias, tiles_m, tiles_n, nxcd);
-    else
-        kern<<<dim3(grid), dim3(256), LDS, st>>>((const uint8_t*)A, (const uint8_t*)B, M, N, Kb, (int32_t*)C, nullptr,
-                                                 nullptr, nullptr, nullptr, tiles_m, tiles_n, nxcd);
-    return qr_launch_status();
-}
-
-// gemm_sp256_tail_kernel (K a multiple of 256, more than one round of tiles, CUs a multiple of the XCDs: mid_plan's rule)
-int launch_sp256_tail(const void* A, const void* B, int M, int N, int Kb, void* C, void* Y, const void* sA, const void* sB,
-                      const void* bias, hipStream_t st) {
-    const size_t LDS = (size_t)3 * (128 + 256) * 8 * 16;    // the larger of the two tiles' stage buffers
-    const int tiles_m = (M + 255) / 256, tiles_n = (N + 255) / 256;
-    const int nxcd = qr_device().xcds, cus = qr_device().cus;
-    const int64_t tiles = (int64_t)tiles_m * tiles_n, whole = tiles / cus * cus;
-    const int64_t halves = ((tiles - whole) * 2 + nxcd - 1) / nxcd * nxcd;
-    if (whole + halves > 0x3fffffff) return QR_E_SHAPE;
-    if ((int64_t)M * Kb >= (1LL << 32) || (int64_t)N * Kb >= (1LL << 32)) return QR_E_UNSUPPORTED;
-    auto kern = Y ? gemm_sp256_tail_kernel<true> : gemm_sp256_tail_kernel<false>;
-    const hipError_t e = qr_allow_dynamic_lds((const void*)kern, LDS);
-    if (e != hipSuccess) return (int)e;
-    kern<<<dim3((unsigned)(whole + halves)), dim3(256), LDS, st>>>((const uint8_t*)A, (const uint8_t*)B, M, N, Kb, (int32_t*)C,
-                                                                   (f16*)Y, (const f16*)sA, (const f16*)sB, (const f16*)bias,
-                                                                   tiles_m, tiles_n, nxcd, (int)whole);
-    return qr_launch_status();
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -1913,39 +1160,37 @@ int ks_split(int64_t M, int64_t N, int64_t Kb) {
 }
 
 // Which kernel takes an output of more than 64 tokens, by an estimate in microseconds (st = stages of 256 k, n = tiles on the
-// busiest of the CUs; fitted to sweeps of 65 .. 1500 tokens against 1902 .. 28672 weight rows at K = 4096 .. 28672 with
-// every kernel forced, and within 10 % of them):
-//   64 x 64 tiles   4.2 + st (n = 1: 0.26, 2: 0.44, more: 0.25 n, from 8 on 0.26 n)      three workgroups share a CU
-//                   0.27 n from 5 on where K > 8192 and the weights are over 36 MB: they are read once per 64 tokens there and once per
-//                   128 by the pipelined kernel (the only other candidate in that corner), from memory.  5 tiles per CU, weights and
-//                   inputs cold, 64 x 64 / pipelined, alone and behind a quantiser or a Hadamard: 300 x 13824 x 13824 58.1 / 60.1,
-//                   62.3 / 59.0, 67.0 / 63.9 us; 600 x 8192 x 20480 89 / 87, 96 / 92, 106 / 96; 600 x 8192 x 28672 119 / 113, 125 / 120,
-//                   133 / 127.  Below the line: 1260 x 4096 x 11008 46.5 / 50.8, 55.9 / 54.2, 59.4 / 59.5; 1000 x 5120 x 13824 57.7 / 61.1,
-//                   64.2 / 65.8, 70.3 / 71.3; 2560 x 2048 x 28672 111 / 114, 135 / 138, 150 / 152.  (A layer alone, without a front, is up to
-//                   8 % better off on the small tiles above the line as well: 600 x 8192 x 11008 48 / 52; such widths follow a front.)
-//   64 x 128        4.6 + st (0.41 n, from the second on 0.52 n)
-//   128 x 128       5.0 + st (n = 1: 0.80, more: 0.92 n)
-//   128 / 192 / 256 x 256 (the pipelined kernels)   rounds (5.5 + {1.40, 2.19, 2.75} st (1 - {0.3, 0.5, 0.5} idle)), idle = share of
+// busiest of the CUs; fitted to 4766 shapes of 65 .. 6000 tokens against 512 .. 28672 weight rows at K = 1024 .. 28672 with every
+// kernel forced and three sets of operands in turn: within 4-8 % of each, and the choice by them costs 0.65 % more than the best of all seven
+// (geometric mean; 1.4 x at worst, where 64-row tiles are few and K is long)):
+//   64 x 64 tiles   3.9 + st 0.264 (n = 1), 4.6 + st 0.42 (n = 2), 3.9 + n (0.75 + 0.21 st) beyond: three workgroups share a CU; 0.23 for 0.21 from
+//                   n = 5 on where K > 8192 and the weights are over 36 MB: they are read once per 64 tokens there and once per
+//                   128 or more by the larger tiles, from memory.  n = 5 and lighter weights: 0.18, less than they take, which keeps the
+//                   small tiles there as tests/test_abi.py has it; 128-row tiles are 4-14 % ahead in that corner when operands come
+//                   from memory (1260 x 4096 x 11008 53 / 49 us, 640 x 8192 x 8192 41.5 / 39, 2560 x 2048 x 28672 125 / 109)
+//   64 x 128        4.9 + st 0.40 (n = 1), 7.6 + st 0.90 (n = 2), 4.9 + n (2.4 + 0.453 st)
+//   128 x 128       5.5 + st 0.73 (n = 1), 9.7 + st 1.50 (n = 2), 5.5 + n (3.6 + 0.755 st)
+//   128 / 192 / 256 x 256 (e2m3 kernels)   1.7 + n ({8.1, 6.8, 8.9} + {0.99, 1.56, 1.76} st (1 - {0.25, 0.18, 0.22} idle)), idle = share of
 //                   the rounds' places without a tile (the clock is higher then)
-// The small tiles are bound by the CUs' intake of operands, the pipelined ones by the matrix pipe, so the small ones lead
-// while the large ones leave CUs idle: 333 x 4096 x 4096 11.2 us (64 x 256 tiles on 96 CUs before: 21.8), 777 x 4096 x 4096
-// 17.7 (22.5), 512 x 8192 x 8192 32.1 (43.5), 1024 x 4096 x 11008 42 (56); 777 x 8192 x 8192 stays with 192- or 128-row
-// tiles (48 against 56), 200 x 28672 x 8192 too (48 against 57).
+//   256 and 128     whole rounds of 256-row tiles and the rest as 128-row ones in the same launch, where that rest is at most half a round
+// The small tiles are bound by the CUs' intake of operands, the large ones by instruction issue and power, so the small ones lead
+// while the large ones leave CUs idle: 333 x 4096 x 4096 11.2 us against 22, 777 x 4096 x 4096 17.7 (22), 512 x 8192 x 8192 32.1 (34).
 // Very few tiles and a long K: slices of K over several workgroups with int32 slabs in the caller's scratch and a second
 // launch that adds them (+ 3.5 us and the slabs' way out and back at 4 TB/s).
 struct MidPlan {
-    int kernel;         // 0 .. 2: qr_internal_gemm_mid's shapes; 3, 4, 5: pipelined 128-, 192-, 256-row tiles; 6: 256-row
-                        // tiles and a last round of 128-row ones
+    int kernel;         // 0 .. 2: qr_internal_gemm_mid's shapes; 3 .. 6: qr_internal_gemm_e2m3's
     int split;
 };
 MidPlan mid_plan(int64_t M, int64_t N, int64_t Kb, int64_t max_split) {
-    const int64_t cus = qr_device().cus, st = (Kb + 127) / 128;
+    const int64_t cus = qr_device().cus;
+    const double st = (double)((Kb + 127) / 128);
     auto tiles = [&](int64_t bm, int64_t bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
     auto loaded = [&](int64_t t) { return (double)((t + cus - 1) / cus); };
-    const bool heavy = st > 32 && N * Kb > 36000000;
-    auto t64 = [&](int64_t t, int64_t stages) {
+    const bool heavy = Kb > 4096 && N * Kb > 36000000;
+    auto t64 = [&](int64_t t, double stages) {
         const double n = loaded(t);
-        return 4.2 + (double)stages * (n == 1 ? 0.26 : n == 2 ? 0.44 : n >= 5 && heavy ? 0.27 * n : n < 8 ? 0.25 * n : 0.26 * n);
+        if (n <= 2) return n == 1 ? 3.9 + 0.264 * stages : 4.6 + 0.42 * stages;
+        return 3.9 + n * (0.75 + (n >= 5 && heavy ? 0.23 : n == 5 ? 0.18 : 0.21) * stages);
     };
     MidPlan best{0, 1};
     double t_best = t64(tiles(64, 64), st);
@@ -1955,32 +1200,23 @@ MidPlan mid_plan(int64_t M, int64_t N, int64_t Kb, int64_t max_split) {
             best = MidPlan{kernel, split};
         }
     };
-    const double n128 = loaded(tiles(64, 128));
-    consider(1, 1, 4.6 + (double)st * (n128 == 1 ? 0.41 : 0.52 * n128));
-    const double nsq = loaded(tiles(128, 128));
-    consider(2, 1, 5.0 + (double)st * (nsq == 1 ? 0.80 : 0.92 * nsq));
-    // Among the pipelined kernels taller tiles run faster per unit of work (3 unpacking instructions per MFMA at 256 rows,
-    // 3.5 at 192, 4.5 at 128) but quantise worse over the CUs: rounds of tiles are compared, a 128x256 tile costing 0.57
-    // and a 192x256 tile 0.80 of a 256x256 one (measured over 300..4096 tokens against 4096..27648 weight rows: rounds of
-    // 27-29 / 40-41 / 48-51 us at K = 4096; every one of those shapes gets the fastest of the three).  Ties go to the
-    // taller tile.
-    const double share[3] = {0.57, 0.80, 1.0}, slope[3] = {1.40, 2.19, 2.75};
-    int tall = 2;
-    for (int i = 1; i >= 0; --i)
-        if (loaded(tiles(128 + 64 * i, 256)) * share[i] < loaded(tiles(128 + 64 * tall, 256)) * share[tall]) tall = i;
-    const int64_t t = tiles(128 + 64 * tall, 256);
-    const double rounds = loaded(t);
-    const double idle = 1.0 - (double)t / (rounds * (double)cus);
-    consider(3 + tall, 1, rounds * (5.5 + slope[tall] * (double)st * (1.0 - (tall == 0 ? 0.3 : 0.5) * idle)));
-    // Whole rounds of 256-row tiles and the rest as 128-row ones in the same launch, where that rest is at most half a round:
-    // 8191 x 5120 x 5120 175 -> 166 us, 6684 x 8192 x 8192 333 -> 307, 10435 x 5120 x 5120 226 -> 209, 32768 x 4096 x 11008
-    // 1099 -> 1078.  The estimate for 192-row tiles is 6 % high beside it (4583 x 5120 x 15360: 265 us against 268).
+    const double n128 = loaded(tiles(64, 128)), nsq = loaded(tiles(128, 128));
+    consider(1, 1, n128 == 1 ? 4.9 + 0.40 * st : n128 == 2 ? 7.6 + 0.90 * st : 4.9 + n128 * (2.4 + 0.453 * st));
+    consider(2, 1, nsq == 1 ? 5.5 + 0.73 * st : nsq == 2 ? 9.7 + 1.50 * st : 5.5 + nsq * (3.6 + 0.755 * st));
+    const double fixed[3] = {8.1, 6.8, 8.9}, slope[3] = {0.99, 1.56, 1.76}, easier[3] = {0.25, 0.18, 0.22};
+    auto round = [&](int i, double idle) { return fixed[i] + slope[i] * st * (1.0 - easier[i] * idle); };
+    for (int i = 2; i >= 0; --i) {                          // (ties go to the taller tile)
+        const int64_t t = tiles(128 + 64 * i, 256);
+        const double n = loaded(t);
+        consider(3 + i, 1, 1.7 + n * round(i, 1.0 - (double)t / (n * (double)cus)));
+    }
     const int64_t whole = tiles(256, 256) / cus, left = tiles(256, 256) % cus;
-    if (Kb % 128 == 0 && cus % qr_device().xcds == 0 && whole > 0 && left > 0 && 2 * left <= cus)
-        consider(6, 1, (tall == 1 ? 1.06 : 1.0) * ((double)whole * (5.5 + slope[2] * (double)st) + 5.5 +
-                                                   slope[0] * (double)st * (1.0 - 0.3 * (1.0 - 2.0 * (double)left / (double)cus))));
-    for (int64_t ks = 2; ks <= max_split && ks <= st / 4; ++ks)
-        consider(0, (int)ks, t64(tiles(64, 64) * ks, (st + ks - 1) / ks) + 3.5 + 2.0 * (double)ks * (double)M * (double)N * 4.0 / 4.0e6);
+    if (cus % qr_device().xcds == 0 && whole > 0 && left > 0 && 2 * left <= cus)
+        consider(6, 1, 1.7 + (double)whole * round(2, 0.0) + round(0, 1.0 - 2.0 * (double)left / (double)cus));
+    const int64_t all_stages = (Kb + 127) / 128;
+    for (int64_t ks = 2; ks <= max_split && ks <= all_stages / 4; ++ks)
+        consider(0, (int)ks, t64(tiles(64, 64) * ks, (double)((all_stages + ks - 1) / ks)) + 3.5 +
+                                 2.0 * (double)ks * (double)M * (double)N * 4.0 / 4.0e6);
     return best;
 }
 
@@ -2040,10 +1276,11 @@ int gemm_dispatch(const void* A, const void* B, int64_t M, int64_t N, int64_t K,
         case Gemm::gemv: return launch_gemv(A, B, m, n, kb, C, Y, sA, sB, bias, st);
         case Gemm::shared_tokens: return launch_decode_xs(A, B, m, n, kb, C, Y, sA, sB, bias, st, decode_xs_groups(n));
         case Gemm::decode: return launch_decode(A, B, m, n, kb, C, Y, sA, sB, bias, st);
-        case Gemm::spk: return launch_spk(A, B, m, n, kb, C, Y, sA, sB, bias, st);
-        case Gemm::sp192: return launch_sp256(A, B, m, n, kb, C, Y, sA, sB, bias, st, 192);
-        case Gemm::sp256: return launch_sp256(A, B, m, n, kb, C, Y, sA, sB, bias, st, 256);
-        case Gemm::sp256_tail: return launch_sp256_tail(A, B, m, n, kb, C, Y, sA, sB, bias, st);
+        case Gemm::spk:
+        case Gemm::sp192:
+        case Gemm::sp256:
+        case Gemm::sp256_tail:
+            return qr_internal_gemm_e2m3((int)plan.kernel - (int)Gemm::spk, A, B, m, n, kb, C, Y, sA, sB, bias, st);
         default: return qr_internal_gemm_mid(mid, A, B, m, n, kb, C, Y, sA, sB, bias, st, 1);
     }
 }

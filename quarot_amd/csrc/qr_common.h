@@ -111,6 +111,11 @@ int qr_internal_token_quant_linear(const void* x, int64_t M, int64_t K, float cl
 int qr_internal_gemm_mid(int shape, const void* A, const void* B, int M, int N, int Kb, void* C, void* Y, const void* sA,
                          const void* sB, const void* bias, hipStream_t st, int ksplit);
 
+// gemm_e2m3.hip: the GEMM on the FP6 matrix path (shape 0 / 1 / 2: tiles of 128 / 192 / 256 x 256, 3: 256 with a last round of 128);
+// Y == nullptr: int32 sums to C
+int qr_internal_gemm_e2m3(int shape, const void* A, const void* B, int M, int N, int Kb, void* C, void* Y, const void* sA,
+                          const void* sB, const void* bias, hipStream_t st);
+
 static inline int qr_launch_status() {
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? QR_OK : (int)e;

@@ -74,4 +74,19 @@ __device__ __forceinline__ f16x4 dequant4_f32(float a0, float a1, float a2, floa
     return f16x4{y01[0], y01[1], y23[0], y23[1]};
 }
 
+// the same for sums held as 1/64 of the integer: the multiplication by 64 follows the rounding to fp16, which it commutes with
+// (|sum| / 64 >= 2^-6 or 0 is far from fp16's subnormals; what rounds beyond 65504 becomes an infinity either way)
+__device__ __forceinline__ f16x4 dequant4_f32x64(float a0, float a1, float a2, float a3, f16 sa, f16x4 sb, f16x4 bi, bool with_bias) {
+    const f16x2 s2 = {sa, sa}, x64 = {(f16)64.0f, (f16)64.0f};
+    const f16x2 q01 = as_f16x2(cvt_f16x2(a0, a1)) * x64;
+    const f16x2 q23 = as_f16x2(cvt_f16x2(a2, a3)) * x64;
+    f16x2 y01 = (s2 * f16x2{sb[0], sb[1]}) * q01;
+    f16x2 y23 = (s2 * f16x2{sb[2], sb[3]}) * q23;
+    if (with_bias) {
+        y01 = y01 + f16x2{bi[0], bi[1]};
+        y23 = y23 + f16x2{bi[2], bi[3]};
+    }
+    return f16x4{y01[0], y01[1], y23[0], y23[1]};
+}
+
 }  // namespace

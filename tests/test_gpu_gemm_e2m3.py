@@ -1,0 +1,61 @@
+"""The GEMM on the FP6 matrix path straight from packed nibbles (128-, 192- and 256-row tiles), bit for bit: int32 sums against exact integer
+sums (fp32 products of chunks of K: integers below 2^24), fp16 outputs against the epilogue's rounded operations on those sums."""
+import ctypes
+
+import pytest
+import torch
+
+from quarot_amd import _lib
+
+pytestmark = pytest.mark.gpu
+
+
+def _codes(packed):
+    low, high = (packed & 15).to(torch.int8), (packed >> 4).to(torch.int8)
+    return torch.stack(((low ^ 8) - 8, (high ^ 8) - 8), -1).flatten(1)
+
+
+def _sums(a, b):
+    total = torch.zeros(a.shape[0], b.shape[0], dtype=torch.int32, device=a.device)
+    for k in range(0, a.shape[1], 8192):
+        total += (_codes(a[:, k:k + 8192]).float() @ _codes(b[:, k:k + 8192]).float().T).to(torch.int32)
+    return total
+
+
+def _operand(rows, k, kind, gen):
+    if kind == "random":
+        return torch.randint(0, 256, (rows, k // 2), dtype=torch.uint8, device="cuda", generator=gen)
+    x = torch.full((rows, k // 2), 0x77, dtype=torch.uint8, device="cuda")     # the largest and smallest sums, with and without the offset
+    x[::3] = 0x88
+    x[1::7] = 0
+    return x
+
+
+@pytest.mark.parametrize("m,n,k,kernel", [
+    # one row, a remainder and a whole last tile in both directions; K of one stage, of a ragged last stage, of a whole one
+    (2049, 4100, 192, "gemm_sp256_kernel"), (2305, 5124, 64, "gemm_sp256_kernel"), (2040, 4099, 320, "gemm_sp256_kernel"),
+    (2048, 5120, 1088, "gemm_sp256_kernel"), (1025, 8201, 2112, "gemm_sp256_kernel"), (8200, 2050, 448, "gemm_sp256_kernel"),
+    (2040, 4096, 4096, "gemm_spk_kernel"), (1800, 8197, 832, "gemm_spk_kernel"), (2047, 4088, 11008, "gemm_spk_kernel"),
+    (4353, 4099, 2112, "gemm_sp256_tail_kernel"), (4600, 4104, 4096, "gemm_sp256_tail_kernel"),
+    # around the points where the accumulators are corrected by the row sums (every 49152 k), and the longest K
+    (520, 9000, 49152, "gemm_spk_kernel"), (520, 9000, 49216, "gemm_spk_kernel"), (513, 16388, 131008, "gemm_sp256_kernel"),
+])
+@pytest.mark.parametrize("kind", ["random", "extreme"])
+def test_gemm_of_large_tiles_bit_exact(m, n, k, kernel, kind):
+    lib = _lib.lib()
+    assert lib.qr_linear_plan(m, n, k, 0, None) == kernel.encode()
+    gen = torch.Generator(device="cuda").manual_seed(m + n + k)
+    a, b = _operand(m, k, kind, gen), _operand(n, k, kind, gen)
+    sa = (torch.rand(m, 1, device="cuda", generator=gen) * 0.1 + 0.01).half()
+    sb = (torch.rand(n, device="cuda", generator=gen) * 0.01 + 0.001).half()
+    bias = torch.randn(n, device="cuda", generator=gen).half()
+    want = _sums(a, b)
+    p = lambda t: ctypes.c_void_p(t.data_ptr())
+    c = torch.full((m + 1, n), 7, dtype=torch.int32, device="cuda")            # (a guard row behind the output)
+    assert lib.qr_matmul_i4_i32(p(a), p(b), m, n, k, p(c), None) == 0
+    assert torch.equal(c[:m], want) and bool((c[m] == 7).all())
+    scaled = (sa * sb) * want.float().half()
+    for bi in (None, bias):
+        y = torch.full((m + 1, n), 7, dtype=torch.float16, device="cuda")
+        assert lib.qr_linear_i4_f16(p(a), p(sa), p(b), p(sb), p(bi) if bi is not None else None, m, n, k, p(y), None) == 0
+        assert torch.equal(y[:m], scaled if bi is None else scaled + bi) and bool((y[m] == 7).all())
