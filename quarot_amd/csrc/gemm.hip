@@ -1205,13 +1205,14 @@ MidPlan mid_plan(int64_t M, int64_t N, int64_t Kb, int64_t max_split) {
     consider(2, 1, nsq == 1 ? 5.5 + 0.73 * st : nsq == 2 ? 9.7 + 1.50 * st : 5.5 + nsq * (3.6 + 0.755 * st));
     const double fixed[3] = {8.1, 6.8, 8.9}, slope[3] = {0.99, 1.56, 1.76}, easier[3] = {0.25, 0.18, 0.22};
     auto round = [&](int i, double idle) { return fixed[i] + slope[i] * st * (1.0 - easier[i] * idle); };
-    for (int i = 2; i >= 0; --i) {                          // (ties go to the taller tile)
+    const bool reach = N < (1LL << 22);                     // 256 rows of the output within the 32-bit offsets of the stores
+    for (int i = 2; reach && i >= 0; --i) {                 // (ties go to the taller tile)
         const int64_t t = tiles(128 + 64 * i, 256);
         const double n = loaded(t);
         consider(3 + i, 1, 1.7 + n * round(i, 1.0 - (double)t / (n * (double)cus)));
     }
     const int64_t whole = tiles(256, 256) / cus, left = tiles(256, 256) % cus;
-    if (cus % qr_device().xcds == 0 && whole > 0 && left > 0 && 2 * left <= cus)
+    if (reach && cus % qr_device().xcds == 0 && whole > 0 && left > 0 && 2 * left <= cus)
         consider(6, 1, 1.7 + (double)whole * round(2, 0.0) + round(0, 1.0 - 2.0 * (double)left / (double)cus));
     const int64_t all_stages = (Kb + 127) / 128;
     for (int64_t ks = 2; ks <= max_split && ks <= all_stages / 4; ++ks)

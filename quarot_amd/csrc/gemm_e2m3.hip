@@ -67,9 +67,11 @@ constexpr int e2m3_lds(int BM, int KG) { return (KG == 1 ? 2 : 3) * (BM + 256) *
 // What bounds it (256 rows, 32768 x 4096 x 11008): a wave issues an instruction in about 5 cycles, and a sub-step has 20 matrix and 112
 // vector instructions, 8 LDS reads, 4 loads and some 20 others: 55 cycles of 2.05 GHz per accumulator tile and sub-step, where the
 // matrix unit alone would need 36; the clock is the power limit's (2.4 GHz without load).  Inside the loop that is 5.0e15 operations
-// per second (the int8 instruction with nothing else going on sustains 3.9-4.2e15); the whole launch, with 1.9 us before and 7.7 us after the
-// loop of every tile (the compute units write 33 MB at a time), 4.2e15: 700 us against 870-890 of the int8 kernel with the same tiles;
-// 32768 x 11008 x 4096 840 us (1010), 8192 x 5120 x 5120 129 (146), 1777 x 8192 x 28672 194 (244), 2048 x 4096 x 11008 53 (58-66).
+// per second (the int8 instruction with nothing else going on sustains 3.9-4.2e15); the whole launch, with 1.9 us before and about 6 us after
+// the loop of every tile (3 us of arithmetic with one wave per SIMD, then the compute units write 33 MB at a time), 4.2e15: 690 us against
+// 870-890 of the int8 kernel with the same tiles; 32768 x 11008 x 4096 818 us (1010; 850 with a branch around every store),
+// 8192 x 5120 x 5120 127 (146), 1777 x 8192 x 28672 194 (244), 2048 x 4096 x 11008 53 (58-66).  Delaying the first workgroups by 0 .. 8 us, so
+// that compute units do not write at once, changed nothing.
 template <bool RAGGED, int BM, int KG>
 __device__ __forceinline__ void e2m3_tile(
     const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, int M, int N, int Kb, int32_t* __restrict__ C,
@@ -253,7 +255,7 @@ __device__ __forceinline__ void e2m3_tile(
 
     // The epilogue's scales and bias are fetched first and parked in LDS: a load in the epilogue would wait for the stores before it.
     // (Indices clamped to the matrix: what belongs to rows and columns beyond it is never stored.)
-    f16 pre_sb = (f16)0, pre_bi = (f16)0, pre_sa = (f16)0;
+    f16 pre_sb = (f16)0, pre_bi = (f16)-0.0f, pre_sa = (f16)0;
     if (Y) {
         const int col = n0 + tid < N ? n0 + tid : N - 1, row = m0 + tid < M ? m0 + tid : M - 1;
         pre_sb = sB[col], pre_sa = sA[row];
@@ -365,7 +367,11 @@ __device__ __forceinline__ void e2m3_tile(
 
     // Epilogue: lane l, register v -> column (v / 4) * 8 + (l / 32) * 4 + v % 4 of the B tile, token l % 32
     constexpr int JO = KG == 2 ? 2 : 4;                     // column groups that this wave puts out
-    if (Y && n0 + 256 <= N && (N & 7) == 0 && (((uintptr_t)Y) & 15) == 0) {
+    if (Y) {
+        // one slab of 32 x 64 behind the other, the stores of each behind the next one's arithmetic
+        char* const region = lds + wave * 4096;
+        const SlabOut out = slab_out(Y, m0, M - m0 < BM ? M - m0 : BM, N, lane);
+        Slab slab;
 #pragma unroll
         for (int jb = 0; jb < JO; jb += 2) {
             f16x4 sbh[2][4], bih[2][4];
@@ -379,56 +385,46 @@ __device__ __forceinline__ void e2m3_tile(
                 }
 #pragma unroll
             for (int i = 0; i < IM; ++i) {
-                const int row0 = m0 + wm * TM + ga(i) * 32;
-                if (row0 >= M) continue;
                 const f16 sa = scales[512 + wm * TM + ga(i) * 32 + (lane & 31)];
                 f16x4 o[2][4];
 #pragma unroll
-                for (int jj = 0; jj < 2; ++jj) asm volatile("" : "+a"(acc[i][jb + jj]));     // (moved out of its registers here, not before)
-#pragma unroll
-                for (int jj = 0; jj < 2; ++jj)
+                for (int jj = 0; jj < 2; ++jj) {
+                    asm volatile("" : "+a"(acc[i][jb + jj]));                   // (moved out of its registers here, not before)
 #pragma unroll
                     for (int gq = 0; gq < 4; ++gq)
                         o[jj][gq] = dequant4_f32x64(acc[i][jb + jj][gq * 4], acc[i][jb + jj][gq * 4 + 1], acc[i][jb + jj][gq * 4 + 2],
-                                                    acc[i][jb + jj][gq * 4 + 3], sa, sbh[jj][gq], bih[jj][gq], bias != nullptr);
-                store_slab_rows<2>((u32x2*)(e2m3_smem + wave * 256), o, lane,
-                                   Y + (int64_t)row0 * N + n0 + wn * 128 + gb(jb) * 32, N, M - row0);
+                                                    acc[i][jb + jj][gq * 4 + 3], sa, sbh[jj][gq], bih[jj][gq]);
+                }
+                if (jb + i > 0)
+                    slab_store(out, slab, wm * TM + ga(i > 0 ? i - 1 : IM - 1) * 32, n0 + wn * 128 + gb(i > 0 ? jb : jb - 2) * 32, lane);
+                slab = slab_turn(region, o, lane);
             }
         }
+        slab_store(out, slab, wm * TM + ga(IM - 1) * 32, n0 + wn * 128 + gb(JO - 2) * 32, lane);
         return;
     }
-    // tiles that overhang the rows of B, rows of no whole number of 16-byte pieces, int32 output: four columns of a row per lane at a time
+    // int32 sums: four columns of a row per lane and store
+    const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)(C + (int64_t)m0 * N), 0, (int)((u32)(M - m0 < BM ? M - m0 : BM) * (u32)N * 4u), 0x00020000);
 #pragma unroll
     for (int i = 0; i < IM; ++i) {
-        const int row = m0 + wm * TM + ga(i) * 32 + (lane & 31);
-        if (row >= M) continue;
-        const f16 sa = scales[512 + wm * TM + ga(i) * 32 + (lane & 31)];
+        const u32 row = (u32)(wm * TM + ga(i) * 32 + (lane & 31)) * (u32)N;
 #pragma unroll
         for (int j = 0; j < JO; ++j) {
             asm volatile("" : "+a"(acc[i][j]));
 #pragma unroll
             for (int gq = 0; gq < 4; ++gq) {
-                const int c = wn * 128 + gb(j) * 32 + gq * 8 + khalf * 4, col = n0 + c;
-                if (col >= N) continue;
-                const bool whole = (N & 3) == 0;            // (then the four columns exist, and are aligned)
-                const float v0 = acc[i][j][gq * 4], v1 = acc[i][j][gq * 4 + 1], v2 = acc[i][j][gq * 4 + 2], v3 = acc[i][j][gq * 4 + 3];
-                if (Y) {
-                    const f16x4 o = dequant4_f32x64(v0, v1, v2, v3, sa, *(const f16x4*)(scales + c), *(const f16x4*)(scales + 256 + c),
-                                                    bias != nullptr);
-                    f16* const yp = Y + (int64_t)row * N + col;
-                    if (whole) *(f16x4*)yp = o;
-                    else
+                const int col = n0 + wn * 128 + gb(j) * 32 + gq * 8 + khalf * 4;
+                const u32 off = (row + (u32)col) * 4u;
+                u32x4 o;
 #pragma unroll
-                        for (int e = 0; e < 4; ++e)
-                            if (col + e < N) yp[e] = o[e];
+                for (int e = 0; e < 4; ++e) o[e] = (u32)(int)(64.f * acc[i][j][gq * 4 + e]);
+                if ((N & 3) == 0) {                         // (then the four columns exist, and are aligned)
+                    __builtin_amdgcn_raw_buffer_store_b128(o, rsrc, col < N ? off : 0xFFFFFF00u, 0, 0);
                 } else {
-                    const i32x4 o = {(int)(64.f * v0), (int)(64.f * v1), (int)(64.f * v2), (int)(64.f * v3)};
-                    int32_t* const cp = C + (int64_t)row * N + col;
-                    if (whole) *(i32x4*)cp = o;
-                    else
 #pragma unroll
-                        for (int e = 0; e < 4; ++e)
-                            if (col + e < N) cp[e] = o[e];
+                    for (int e = 0; e < 4; ++e)
+                        __builtin_amdgcn_raw_buffer_store_b32(o[e], rsrc, col + e < N ? off + 4u * e : 0xFFFFFF00u, 0, 0);
                 }
             }
         }
@@ -489,7 +485,7 @@ __global__ __launch_bounds__(256) void gemm_sp256_tail_kernel(
 // multiple of the XCDs).  Y == nullptr: int32 sums to C.  K up to 131008; operands below 4 GiB (32-bit buffer offsets).
 int qr_internal_gemm_e2m3(int shape, const void* A, const void* B, int M, int N, int Kb, void* C, void* Y, const void* sA,
                           const void* sB, const void* bias, hipStream_t st) {
-    if ((int64_t)M * Kb >= (1LL << 32) || (int64_t)N * Kb >= (1LL << 32)) return QR_E_UNSUPPORTED;   // (the dispatcher routes these away)
+    if ((int64_t)M * Kb >= (1LL << 32) || (int64_t)N * Kb >= (1LL << 32) || N >= (1 << 22)) return QR_E_UNSUPPORTED;   // (the dispatcher routes these away)
     const int bm = shape == 0 ? 128 : shape == 1 ? 192 : 256;
     const int tiles_m = (M + bm - 1) / bm, tiles_n = (N + 255) / 256;
     const int nxcd = qr_device().xcds, cus = qr_device().cus;
