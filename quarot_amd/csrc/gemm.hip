@@ -1168,6 +1168,9 @@ int ks_split(int64_t M, int64_t N, int64_t Kb) {
 //                   128 or more by the larger tiles, from memory.  n = 5 and lighter weights: 0.18, less than they take, which keeps the
 //                   small tiles there as tests/test_abi.py has it; 128-row tiles are 4-14 % ahead in that corner when operands come
 //                   from memory (1260 x 4096 x 11008 53 / 49 us, 640 x 8192 x 8192 41.5 / 39, 2560 x 2048 x 28672 125 / 109)
+//   96 x 64         5.1 + st 0.325 (n = 1; 0.37 where K > 8192 and the weights are over 36 MB), 8.0 + st 0.69 (n = 2), 5.1 + n (2.0 + 0.335 st)
+//                   (5094 more shapes of 65 .. 1500 tokens: ahead by 11 % on the tenth of them where it is the best, mostly n = 1, and
+//                   the choice among all kernels costs 0.9 % more than the best of them, 2.1 % without it)
 //   64 x 128        4.9 + st 0.40 (n = 1), 7.6 + st 0.90 (n = 2), 4.9 + n (2.4 + 0.453 st)
 //   128 x 128       5.5 + st 0.73 (n = 1), 9.7 + st 1.50 (n = 2), 5.5 + n (3.6 + 0.755 st)
 //   128 / 192 / 256 x 256 (e2m3 kernels)   1.7 + n ({8.1, 6.8, 8.9} + {0.99, 1.56, 1.76} st (1 - {0.25, 0.18, 0.22} idle)), idle = share of
@@ -1178,7 +1181,7 @@ int ks_split(int64_t M, int64_t N, int64_t Kb) {
 // Very few tiles and a long K: slices of K over several workgroups with int32 slabs in the caller's scratch and a second
 // launch that adds them (+ 3.5 us and the slabs' way out and back at 4 TB/s).
 struct MidPlan {
-    int kernel;         // 0 .. 2: qr_internal_gemm_mid's shapes; 3 .. 6: qr_internal_gemm_e2m3's
+    int kernel;         // 0 .. 2: qr_internal_gemm_mid's shapes; 3 .. 6: qr_internal_gemm_e2m3's; 7: 96 x 64 tiles
     int split;
 };
 MidPlan mid_plan(int64_t M, int64_t N, int64_t Kb, int64_t max_split) {
@@ -1200,6 +1203,8 @@ MidPlan mid_plan(int64_t M, int64_t N, int64_t Kb, int64_t max_split) {
             best = MidPlan{kernel, split};
         }
     };
+    const double n96 = loaded(tiles(96, 64));
+    consider(7, 1, n96 == 1 ? 5.1 + (heavy ? 0.37 : 0.325) * st : n96 == 2 ? 8.0 + 0.69 * st : 5.1 + n96 * (2.0 + 0.335 * st));
     const double n128 = loaded(tiles(64, 128)), nsq = loaded(tiles(128, 128));
     consider(1, 1, n128 == 1 ? 4.9 + 0.40 * st : n128 == 2 ? 7.6 + 0.90 * st : 4.9 + n128 * (2.4 + 0.453 * st));
     consider(2, 1, nsq == 1 ? 5.5 + 0.73 * st : nsq == 2 ? 9.7 + 1.50 * st : 5.5 + nsq * (3.6 + 0.755 * st));
@@ -1222,7 +1227,7 @@ MidPlan mid_plan(int64_t M, int64_t N, int64_t Kb, int64_t max_split) {
 }
 
 // The kernel that takes a shape, with room for max_split slabs of the output, and the slices of K that it runs in.
-enum class Gemm { large, gemv, shared_tokens, decode, stream64, mid64, mid64x128, mid128, spk, sp192, sp256, sp256_tail };
+enum class Gemm { large, gemv, shared_tokens, decode, stream64, mid64, mid64x128, mid128, spk, sp192, sp256, sp256_tail, mid96 };
 struct GemmPlan {
     Gemm kernel;
     int split;
@@ -1233,7 +1238,7 @@ GemmPlan gemm_plan(int64_t M, int64_t N, int64_t Kb, int64_t max_split) {
     if (M * Kb >= (1LL << 32) || N * Kb >= (1LL << 32)) return GemmPlan{Gemm::large, 1};
     if (M > 64) {
         const MidPlan plan = mid_plan(M, N, Kb, max_split);
-        constexpr Gemm kernels[] = {Gemm::mid64, Gemm::mid64x128, Gemm::mid128, Gemm::spk, Gemm::sp192, Gemm::sp256, Gemm::sp256_tail};
+        constexpr Gemm kernels[] = {Gemm::mid64, Gemm::mid64x128, Gemm::mid128, Gemm::spk, Gemm::sp192, Gemm::sp256, Gemm::sp256_tail, Gemm::mid96};
         return GemmPlan{kernels[plan.kernel], plan.split};
     }
     // one to four tokens: the dot-product kernel -- except two to four tokens against a weight with enough rows for the
@@ -1260,7 +1265,7 @@ int gemm_dispatch(const void* A, const void* B, int64_t M, int64_t N, int64_t K,
     // the slabs of a K split go to scratch from the caller; without it (or with too little) the single-launch kernels run
     const bool scratch = Y && ws && ((uintptr_t)ws & 15) == 0;
     const GemmPlan plan = gemm_plan(M, N, kb, scratch ? (int64_t)(ws_bytes / ((size_t)M * (size_t)N * 4)) : 1);
-    const int mid = plan.kernel == Gemm::stream64 ? 3 : (int)plan.kernel - (int)Gemm::mid64;      // qr_internal_gemm_mid's shape
+    const int mid = plan.kernel == Gemm::stream64 ? 3 : plan.kernel == Gemm::mid96 ? 4 : (int)plan.kernel - (int)Gemm::mid64;      // qr_internal_gemm_mid's shape
     if (plan.split > 1) {
         const int rc = qr_internal_gemm_mid(mid, A, B, m, n, kb, ws, nullptr, nullptr, nullptr, nullptr, st, plan.split);
         if (rc != QR_OK) return rc;
@@ -1318,6 +1323,7 @@ extern "C" const char* qr_linear_plan(int64_t M, int64_t N, int64_t K, size_t wo
         case Gemm::shared_tokens: return "decode_xs_kernel";
         case Gemm::decode: return "decode_i4_kernel";
         case Gemm::stream64:
+        case Gemm::mid96:                                   // (its form with three row tiles per wave)
         case Gemm::mid64: return slices ? "gemm_mid_kernel<64,64> (K sliced) + dequant_slabs_kernel" : "gemm_mid_kernel<64,64>";
         case Gemm::mid64x128: return "gemm_mid_kernel<64,128>";
         case Gemm::mid128: return "gemm_mid_kernel<128,128>";

@@ -8,6 +8,8 @@
 // 64 x 64 spread the same bytes over all CUs.  Every wave owns a 64 x 64 wave tile (6 unpacking instructions per MFMA,
 // affordable where the pipe idles anyway); WK groups of waves take the 64-k sub-steps of a 256-k stage (a 128-byte line
 // per row) in turn, so a small tile still keeps eight waves busy, and add their accumulators through LDS at the end.
+// One tile of 96 x 64 per CU takes in 160 rows per stage where one of 64 x 128 takes 192 and two of 64 x 64 take 256: 333 x 4096 x 4096
+// 11.3 -> 10.2 us, 192 x 8192 x 8192 16.8 -> 15.3, 333 x 4096 x 11008 20.7 -> 18.5, 180 x 8192 x 28672 58 -> 47.
 // Stages go straight from global memory into LDS (buffer_load ... lds), NBUF - 1 stages ahead, one barrier per stage;
 // while a stage's MFMAs run, the wave's fragments of the next sub-step are read and unpacked.
 // K need not be a multiple of 256: a sub-step beyond K is skipped (its loads repeat the stage's first piece).
@@ -21,16 +23,19 @@
 
 namespace {
 
-template <int BM, int BN, int WK, int NBUF, bool DEQ, bool STREAM>
-__global__ __launch_bounds__(64 * (BM / 64) * (BN / 64) * WK) void gemm_mid_kernel(
+template <int TM, int BN, int WK, int NBUF, bool DEQ, bool STREAM, int IM = 2>
+__global__ __launch_bounds__(64 * (TM / 64) * (BN / 64) * WK) void gemm_mid_kernel(
     const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, int M, int N, int Kb, int32_t* __restrict__ C,
     f16* __restrict__ Y, const f16* __restrict__ sA, const f16* __restrict__ sB, const f16* __restrict__ bias,
     int tiles_m, int tiles_n, int ksplit, int nxcd) {
-    constexpr int WM = BM / 64, WN = BN / 64, NT = 64 * WM * WN * WK;
+    constexpr int WM = TM / 64, WN = BN / 64, NT = 64 * WM * WN * WK;
+    constexpr int BM = 32 * IM * WM;                        // rows of the tile: TM, or half as many again (IM = 3)
+    constexpr int NF = IM + 2, NMF = 4 * IM, UNP = 12 * NF; // fragments, matrix and unpacking instructions of a sub-step
     constexpr int CH = (BM + BN) * 8;                       // 16-byte pieces per stage
     constexpr int NL = CH / NT;                             // ... per thread
     constexpr int RPL = NT / 8;                             // rows per load instruction of the workgroup
     constexpr int SUB = 4 / WK;                             // sub-steps per wave and stage
+    static_assert(IM == 2 || (IM == 3 && TM == 64 && BN == 64 && WK == 4 && !STREAM), "wave tiles of 64 x 64 or 96 x 64");
     static_assert((WK == 2 || WK == 4) && CH % NT == 0 && BM % RPL == 0 && RPL % 16 == 0, "tile shape");
     extern __shared__ u32x4 mid_lds[];                      // [NBUF][CH]; later the accumulator exchange, then the output slabs
 
@@ -82,33 +87,32 @@ __global__ __launch_bounds__(64 * (BM / 64) * (BN / 64) * WK) void gemm_mid_kern
 
     // ---- fragments.  A K-group holds its accumulator tiles permuted so that the ones it finalises are always the first:
     // WK = 4: register r is tile r ^ kg of the 2 x 2 (row tile (r ^ kg) >> 1, column tile (r ^ kg) & 1), tile kg is its own;
-    // WK = 2: the row tiles swapped in group 1, row tile kg is its own.
-    const int fi = WK == 4 ? kg >> 1 : kg, fj = WK == 4 ? kg & 1 : 0;
-    i32x16 acc[2][2];
+    // WK = 2: the row tiles swapped in group 1, row tile kg is its own.  96-row tiles: six tiles for four groups, summed row by row instead.
+    const int fi = IM == 3 ? 0 : WK == 4 ? kg >> 1 : kg, fj = IM == 2 && WK == 4 ? kg & 1 : 0;
+    i32x16 acc[IM][2];
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < IM; ++i)
 #pragma unroll
         for (int j = 0; j < 2; ++j)
 #pragma unroll
             for (int v = 0; v < 16; ++v) acc[i][j][v] = 0;
-    int fslot[SUB][4];                                      // LDS slots of the wave's four fragments (two of A, two of B)
+    int fslot[SUB][NF];                                     // LDS slots of the wave's fragments (IM of A, two of B)
 #pragma unroll
     for (int u = 0; u < SUB; ++u) {
         const int chunk = 2 * (kg * SUB + u) + khalf;
 #pragma unroll
-        for (int t = 0; t < 2; ++t) {
-            fslot[u][t] = slot8(wm * 64 + (t ^ fi) * 32 + (lane & 31), chunk);
-            fslot[u][2 + t] = slot8(BM + wn * 64 + (t ^ fj) * 32 + (lane & 31), chunk);
-        }
+        for (int t = 0; t < IM; ++t) fslot[u][t] = slot8(wm * 64 + (t ^ fi) * 32 + (lane & 31), chunk);
+#pragma unroll
+        for (int t = 0; t < 2; ++t) fslot[u][IM + t] = slot8(BM + wn * 64 + (t ^ fj) * 32 + (lane & 31), chunk);
     }
     struct Packed {
-        u32x4 f[4];
+        u32x4 f[NF];
     };
     struct Ops {
-        i32x4 lo[4], hi[4];
+        i32x4 lo[NF], hi[NF];
     };
     auto read1 = [&](int buf, int u, int t, Packed& p) { p.f[t] = mid_lds[buf * CH + fslot[u][t]]; };
-    // unpacking as 48 single instructions: dword d = n / 3 of the packed dwords, n % 3 = 0: lo = p << 4; 1: lo &= mask;
+    // unpacking as 12 NF single instructions: dword d = n / 3 of the packed dwords, n % 3 = 0: lo = p << 4; 1: lo &= mask;
     // 2: hi = p & mask
     auto unpack1 = [&](const Packed& p, Ops& o, int n) {
         const int d = n / 3, f = d >> 2, e = d & 3, kind = n % 3;
@@ -117,27 +121,27 @@ __global__ __launch_bounds__(64 * (BM / 64) * (BN / 64) * WK) void gemm_mid_kern
         else o.hi[f][e] = (int)(p.f[f][e] & 0xF0F0F0F0u);
     };
     auto mfma1 = [&](const Ops& o, int q) {
-        const int i = (q >> 1) & 1, j = q & 1;
-        if (q < 4) acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(o.lo[2 + j], o.lo[i], acc[i][j], 0, 0, 0);
-        else acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(o.hi[2 + j], o.hi[i], acc[i][j], 0, 0, 0);
+        const int i = (q >> 1) % IM, j = q & 1;
+        if (q < 2 * IM) acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(o.lo[IM + j], o.lo[i], acc[i][j], 0, 0, 0);
+        else acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(o.hi[IM + j], o.hi[i], acc[i][j], 0, 0, 0);
     };
-    // One 64-k sub-step = 8 slots, each an MFMA of the current operands, a share of the next sub-step's unpacking (its four
-    // fragments are read in slot 0; 48 instructions in slots S0 .. 7) and at most one load request; a full scheduling
+    // One 64-k sub-step = NMF slots, each an MFMA of the current operands, a share of the next sub-step's unpacking (its
+    // fragments are read in slot 0; UNP instructions from slot S0 on) and at most one load request; a full scheduling
     // barrier after every slot keeps the two waves of a SIMD from unpacking and multiplying in step.
     constexpr int S0 = 3;
     auto substep = [&](const Ops& cur, Ops& nxt, int rbuf, int ru, auto&& req) {
         Packed pk;
 #pragma unroll
-        for (int q = 0; q < 8; ++q) {
+        for (int q = 0; q < NMF; ++q) {
             mfma1(cur, q);
             if (q == 0) {
 #pragma unroll
-                for (int t = 0; t < 4; ++t) read1(rbuf, ru, t, pk);
+                for (int t = 0; t < NF; ++t) read1(rbuf, ru, t, pk);
             }
             if (q >= 1 && q <= NL) req(q - 1);
             if (q >= S0) {
 #pragma unroll
-                for (int n = (q - S0) * 48 / (8 - S0); n < (q - S0 + 1) * 48 / (8 - S0); ++n) unpack1(pk, nxt, n);
+                for (int n = (q - S0) * UNP / (NMF - S0); n < (q - S0 + 1) * UNP / (NMF - S0); ++n) unpack1(pk, nxt, n);
             }
             __builtin_amdgcn_sched_barrier(0);
         }
@@ -145,16 +149,16 @@ __global__ __launch_bounds__(64 * (BM / 64) * (BN / 64) * WK) void gemm_mid_kern
     auto fill = [&](int rbuf, int ru, Ops& o) {             // the same without a multiplication under it
         Packed pk;
 #pragma unroll
-        for (int t = 0; t < 4; ++t) read1(rbuf, ru, t, pk);
+        for (int t = 0; t < NF; ++t) read1(rbuf, ru, t, pk);
 #pragma unroll
-        for (int n = 0; n < 48; ++n) unpack1(pk, o, n);
+        for (int n = 0; n < UNP; ++n) unpack1(pk, o, n);
     };
     // sub-step (st, u) lies inside K (K is a multiple of 64; uniform over the wave)
     auto inside = [&](int st, int u) { return (s0 + st) * 128 + (kg * SUB + u) * 32 < Kb; };
     auto multiply = [&](int st, int u, const Ops& o) {
         if (inside(st, u)) {
 #pragma unroll
-            for (int q = 0; q < 8; ++q) mfma1(o, q);
+            for (int q = 0; q < NMF; ++q) mfma1(o, q);
         }
     };
 
@@ -170,6 +174,20 @@ __global__ __launch_bounds__(64 * (BM / 64) * (BN / 64) * WK) void gemm_mid_kern
         else QR_MID_WAIT(4 * NL);
     };
     static_assert(NBUF >= 3 && NBUF <= 5, "waits are spelled for at most four stages behind the needed one");
+    // (IM = 3) the epilogue's scales and bias: rows tid / 8 + 32 p, columns (tid % 8) * 8 .. + 7; -0 where there is no bias, which leaves every
+    // value as it is
+    const bool lines = DEQ && n0 + BN <= N && (N & 7) == 0 && (((uintptr_t)Y) & 15) == 0;
+    f16 sa3[3];
+    f16x8 sb8, bi8;
+    if (IM == 3 && lines) {
+#pragma unroll
+        for (int p = 0; p < 3; ++p) sa3[p] = sA[min(m0 + (tid >> 3) + 32 * p, M - 1)];
+        sb8 = *(const f16x8*)(sB + n0 + (tid & 7) * 8);
+        if (bias) bi8 = *(const f16x8*)(bias + n0 + (tid & 7) * 8);
+        else
+#pragma unroll
+            for (int e = 0; e < 8; ++e) bi8[e] = (f16)-0.0f;
+    }
     for (int st = 0; st < NBUF && st < stages; ++st)
 #pragma unroll
         for (int i = 0; i < NL; ++i) request1(st, st, i);
@@ -222,6 +240,64 @@ __global__ __launch_bounds__(64 * (BM / 64) * (BN / 64) * WK) void gemm_mid_kern
 
     // ---- the K-groups' sums: every group sends the tiles it does not finalise through LDS and adds what it receives
     __syncthreads();                                        // stage buffers free
+    if constexpr (IM == 3) {
+        // Every group puts all its sums out, [group][96 rows][16 pieces of four columns], pieces XORed with the row; a thread adds up the four
+        // groups' eight columns (tid % 8) * 8 .. of rows tid / 8 + 32 p and stores them, eight threads a line.
+        const int key = lane & 15;
+#pragma unroll
+        for (int i = 0; i < IM; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+                for (int qv = 0; qv < 4; ++qv)
+                    mid_lds[(kg * 96 + i * 32 + (lane & 31)) * 16 + ((j * 8 + qv * 2 + khalf) ^ key)] =
+                        u32x4{(u32)acc[i][j][qv * 4], (u32)acc[i][j][qv * 4 + 1], (u32)acc[i][j][qv * 4 + 2], (u32)acc[i][j][qv * 4 + 3]};
+        __syncthreads();
+#pragma unroll
+        for (int p = 0; p < 3; ++p) {
+            const int r = (tid >> 3) + 32 * p, row = m0 + r, col = n0 + (tid & 7) * 8;
+            i32x4 v[2] = {i32x4{0, 0, 0, 0}, i32x4{0, 0, 0, 0}};
+#pragma unroll
+            for (int g = 0; g < 4; ++g)
+#pragma unroll
+                for (int h = 0; h < 2; ++h)
+                    v[h] += __builtin_bit_cast(i32x4, mid_lds[(g * 96 + r) * 16 + (((tid & 7) * 2 + h) ^ (r & 15))]);
+            if (row >= M) continue;
+            if (lines) {
+                u32x4 o;
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const f16x4 y = dequant4(v[h][0], v[h][1], v[h][2], v[h][3], sa3[p], f16x4{sb8[4 * h], sb8[4 * h + 1], sb8[4 * h + 2], sb8[4 * h + 3]},
+                                             f16x4{bi8[4 * h], bi8[4 * h + 1], bi8[4 * h + 2], bi8[4 * h + 3]}, true);
+                    const u32x2 w = __builtin_bit_cast(u32x2, y);
+                    o[2 * h] = w[0], o[2 * h + 1] = w[1];
+                }
+                __builtin_nontemporal_store(o, (u32x4*)(Y + (int64_t)row * N + col));
+                continue;
+            }
+            const f16 s = DEQ ? sA[row] : (f16)0;
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                if (!DEQ && col + 4 * h + 4 <= N && (N & 3) == 0) {
+                    *(i32x4*)(C + (int64_t)row * N + col + 4 * h) = i32x4{v[h][0] >> 8, v[h][1] >> 8, v[h][2] >> 8, v[h][3] >> 8};
+                    continue;
+                }
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int c = col + 4 * h + e;
+                    if (c >= N) continue;
+                    if (DEQ) {
+                        f16 yv = (f16)(s * sB[c]) * (f16)(float)(v[h][e] >> 8);
+                        if (bias) yv = yv + bias[c];
+                        Y[(int64_t)row * N + c] = yv;
+                    } else {
+                        C[(int64_t)row * N + c] = v[h][e] >> 8;
+                    }
+                }
+            }
+        }
+        return;
+    }
     if (WK == 4) {
 #pragma unroll
         for (int r = 1; r < 4; ++r)
@@ -266,7 +342,7 @@ __global__ __launch_bounds__(64 * (BM / 64) * (BN / 64) * WK) void gemm_mid_kern
     const int row0 = m0 + wm * 64 + fi * 32, col0 = n0 + wn * 64 + fj * 32;
     if (row0 >= M) return;
     const int row = row0 + (lane & 31);
-    if (DEQ && n0 + BN <= N && (N & 7) == 0 && (((uintptr_t)Y) & 15) == 0) {
+    if (lines) {
         const f16 sa = sA[min(row, M - 1)];                 // (rows past M: computed on a clamped scale, not stored)
         f16x4 o[NJ][4];
 #pragma unroll
@@ -310,12 +386,12 @@ __global__ __launch_bounds__(64 * (BM / 64) * (BN / 64) * WK) void gemm_mid_kern
         }
 }
 
-template <int BM, int BN, int WK, int NBUF, bool STREAM = false>
+template <int TM, int BN, int WK, int NBUF, bool STREAM = false, int IM = 2>
 int launch_mid(const void* A, const void* B, int M, int N, int Kb, void* C, void* Y, const void* sA, const void* sB,
                const void* bias, hipStream_t st, int ksplit) {
-    constexpr int NT = 64 * (BM / 64) * (BN / 64) * WK;
+    constexpr int NT = 64 * (TM / 64) * (BN / 64) * WK, BM = TM / 2 * IM;
     constexpr size_t STAGES = (size_t)NBUF * (BM + BN) * 128;
-    constexpr size_t XCH = (size_t)(BM / 64) * (BN / 64) * WK * (WK == 4 ? 3 : 2) * 4096;
+    constexpr size_t XCH = IM == 3 ? (size_t)WK * BM * BN * 4 : (size_t)(TM / 64) * (BN / 64) * WK * (WK == 4 ? 3 : 2) * 4096;
     constexpr size_t LDS = STAGES > XCH ? STAGES : XCH;
     const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
     const int64_t tiles = (int64_t)tiles_m * tiles_n * ksplit;
@@ -323,7 +399,7 @@ int launch_mid(const void* A, const void* B, int M, int N, int Kb, void* C, void
     if ((int64_t)M * Kb >= (1LL << 32) || (int64_t)N * Kb >= (1LL << 32)) return QR_E_UNSUPPORTED;   // (32-bit buffer offsets)
     const int nxcd = qr_device().xcds;                      // the grid is a whole number of rounds over the XCDs
     const unsigned grid = (unsigned)((tiles + nxcd - 1) / nxcd * nxcd);
-    auto kern = Y ? gemm_mid_kernel<BM, BN, WK, NBUF, true, STREAM> : gemm_mid_kernel<BM, BN, WK, NBUF, false, STREAM>;
+    auto kern = Y ? gemm_mid_kernel<TM, BN, WK, NBUF, true, STREAM, IM> : gemm_mid_kernel<TM, BN, WK, NBUF, false, STREAM, IM>;
     const hipError_t e = qr_allow_dynamic_lds((const void*)kern, LDS);
     if (e != hipSuccess) return (int)e;
     kern<<<dim3(grid), dim3(NT), LDS, st>>>((const uint8_t*)A, (const uint8_t*)B, M, N, Kb, (int32_t*)C, (f16*)Y, (const f16*)sA,
@@ -333,11 +409,12 @@ int launch_mid(const void* A, const void* B, int M, int N, int Kb, void* C, void
 
 }  // namespace
 
-// shape: 0 = 64 x 64, 1 = 64 x 128, 2 = 128 x 128 tiles; 3 = 64 x 64 in the STREAM form (M <= 64).  Three stage buffers of 16 KB
+// shape: 0 = 64 x 64, 1 = 64 x 128, 2 = 128 x 128 tiles; 3 = 64 x 64 in the STREAM form (M <= 64); 4 = 96 x 64.  Three stage buffers of 16 KB
 // let three 64 x 64 workgroups share a CU.  A 64 x 128 or 128 x 128 one has a CU to itself: eight waves exchange 96 KB of
 // accumulators through LDS at the end, more than the 72 KB of its three stage buffers, and four buffers are 128 KB.
 // 64 x 128 with five and 64 x 64 with four buffers were no faster (11.8 against 11.2 us, 8.3 against 8.2 at 128 and 333
-// tokens x 4096 x 4096): the loads are bound by rate, not by how many are in flight.  The STREAM form's come from memory:
+// tokens x 4096 x 4096): the loads are bound by rate, not by how many are in flight.  96 x 64 has a CU to itself as well (the
+// exchange is 96 KB) and four waves: four buffers 10.2, five 10.8 us at 333 x 4096 x 4096.  The STREAM form's come from memory:
 // with at most a workgroup per CU it takes five buffers, 64 KB in flight (48 x
 // 5120 x 13824 in two slices of K 17.8 -> 15.7 us), with more workgroups three (48 x 22016 x 4096 14.3 -> 13.5).
 __attribute__((visibility("hidden"))) int qr_internal_gemm_mid(int shape, const void* A, const void* B, int M, int N, int Kb,
@@ -346,6 +423,7 @@ __attribute__((visibility("hidden"))) int qr_internal_gemm_mid(int shape, const 
     if (ksplit > 1 && Y) return QR_E_UNSUPPORTED;           // partial sums exist only as int32
     if (shape == 0) return launch_mid<64, 64, 4, 3>(A, B, M, N, Kb, C, Y, sA, sB, bias, st, ksplit);
     if (shape == 1) return launch_mid<64, 128, 4, 3>(A, B, M, N, Kb, C, Y, sA, sB, bias, st, ksplit);
+    if (shape == 4) return launch_mid<64, 64, 4, 4, false, 3>(A, B, M, N, Kb, C, Y, sA, sB, bias, st, ksplit);
     if (shape == 3) {
         if (M > 64) return QR_E_UNSUPPORTED;
         if ((int64_t)((N + 63) / 64) * ksplit <= qr_device().cus)

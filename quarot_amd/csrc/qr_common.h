@@ -107,7 +107,7 @@ int qr_internal_token_hadamard_linear(const void* x, int64_t M, int n, int K, co
 int qr_internal_token_quant_linear(const void* x, int64_t M, int64_t K, float clip, const void* W, const void* sW,
                                    const void* bias, int64_t N, void* y, hipStream_t st);
 
-// gemm_mid.hip: the GEMM on small tiles (shape 0: 64 x 64, 1: 64 x 128, 2: 128 x 128); ksplit > 1 writes int32 slabs to C
+// gemm_mid.hip: the GEMM on small tiles (shape 0: 64 x 64, 1: 64 x 128, 2: 128 x 128, 3: 64 x 64 for one row of tiles, 4: 96 x 64); ksplit > 1 writes int32 slabs to C
 int qr_internal_gemm_mid(int shape, const void* A, const void* B, int M, int N, int Kb, void* C, void* Y, const void* sA,
                          const void* sB, const void* bias, hipStream_t st, int ksplit);
 

@@ -1,4 +1,4 @@
-"""The GEMM on the FP6 matrix path straight from packed nibbles (128-, 192- and 256-row tiles), bit for bit: int32 sums against exact integer
+"""The GEMM on the FP6 matrix path straight from packed nibbles (128-, 192- and 256-row tiles) and on 96 x 64 tiles, bit for bit: int32 sums against exact integer
 sums (fp32 products of chunks of K: integers below 2^24), fp16 outputs against the epilogue's rounded operations on those sums."""
 import ctypes
 
@@ -31,19 +31,8 @@ def _operand(rows, k, kind, gen):
     return x
 
 
-@pytest.mark.parametrize("m,n,k,kernel", [
-    # one row, a remainder and a whole last tile in both directions; K of one stage, of a ragged last stage, of a whole one
-    (2049, 4100, 192, "gemm_sp256_kernel"), (2305, 5124, 64, "gemm_sp256_kernel"), (2040, 4099, 320, "gemm_sp256_kernel"),
-    (2048, 5120, 1088, "gemm_sp256_kernel"), (1025, 8201, 2112, "gemm_sp256_kernel"), (8200, 2050, 448, "gemm_sp256_kernel"),
-    (2040, 4096, 4096, "gemm_spk_kernel"), (1800, 8197, 832, "gemm_spk_kernel"), (2047, 4088, 11008, "gemm_spk_kernel"),
-    (4353, 4099, 2112, "gemm_sp256_tail_kernel"), (4600, 4104, 4096, "gemm_sp256_tail_kernel"),
-    # around the points where the accumulators are corrected by the row sums (every 49152 k), and the longest K
-    (520, 9000, 49152, "gemm_spk_kernel"), (520, 9000, 49216, "gemm_spk_kernel"), (513, 16388, 131008, "gemm_sp256_kernel"),
-])
-@pytest.mark.parametrize("kind", ["random", "extreme"])
-def test_gemm_of_large_tiles_bit_exact(m, n, k, kernel, kind):
+def _compare(m, n, k, kind):
     lib = _lib.lib()
-    assert lib.qr_linear_plan(m, n, k, 0, None) == kernel.encode()
     gen = torch.Generator(device="cuda").manual_seed(m + n + k)
     a, b = _operand(m, k, kind, gen), _operand(n, k, kind, gen)
     sa = (torch.rand(m, 1, device="cuda", generator=gen) * 0.1 + 0.01).half()
@@ -59,3 +48,27 @@ def test_gemm_of_large_tiles_bit_exact(m, n, k, kernel, kind):
         y = torch.full((m + 1, n), 7, dtype=torch.float16, device="cuda")
         assert lib.qr_linear_i4_f16(p(a), p(sa), p(b), p(sb), p(bi) if bi is not None else None, m, n, k, p(y), None) == 0
         assert torch.equal(y[:m], scaled if bi is None else scaled + bi) and bool((y[m] == 7).all())
+
+
+@pytest.mark.parametrize("m,n,k,kernel", [
+    # one row, a remainder and a whole last tile in both directions; K of one stage, of a ragged last stage, of a whole one
+    (2049, 4100, 192, "gemm_sp256_kernel"), (2305, 5124, 64, "gemm_sp256_kernel"), (2040, 4099, 320, "gemm_sp256_kernel"),
+    (2048, 5120, 1088, "gemm_sp256_kernel"), (1025, 8201, 2112, "gemm_sp256_kernel"), (8200, 2050, 448, "gemm_sp256_kernel"),
+    (2040, 4096, 4096, "gemm_spk_kernel"), (1800, 8197, 832, "gemm_spk_kernel"), (2047, 4088, 11008, "gemm_spk_kernel"),
+    (4353, 4099, 2112, "gemm_sp256_tail_kernel"), (4600, 4104, 4096, "gemm_sp256_tail_kernel"),
+    # around the points where the accumulators are corrected by the row sums (every 49152 k), and the longest K
+    (520, 9000, 49152, "gemm_spk_kernel"), (520, 9000, 49216, "gemm_spk_kernel"), (513, 16388, 131008, "gemm_sp256_kernel"),
+])
+@pytest.mark.parametrize("kind", ["random", "extreme"])
+def test_gemm_of_large_tiles_bit_exact(m, n, k, kernel, kind):
+    assert _lib.lib().qr_linear_plan(m, n, k, 0, None) == kernel.encode()
+    _compare(m, n, k, kind)
+
+
+@pytest.mark.parametrize("m,n,k", [
+    # 96 x 64 tiles (the plan's choice for one tile on each CU): whole tiles, one row or column into the last one, K that ends inside a stage,
+    # rows of no whole 16-byte pieces
+    (333, 4096, 4096), (192, 8192, 11008), (193, 5377, 4160), (385, 3200, 4160), (190, 8131, 2112), (275, 5437, 1600), (260, 5440, 2048)])
+@pytest.mark.parametrize("kind", ["random", "extreme"])
+def test_gemm_of_96_row_tiles_bit_exact(m, n, k, kind):
+    _compare(m, n, k, kind)
