@@ -20,16 +20,16 @@ namespace {
 // rings are slower ({1,2,2,1} 21.0, {1,2,2,2} 22.2: more requests queue ahead of what the front waits for).
 constexpr int F0 = 1, F1 = 2, F2 = 2, F3 = 0, RING = F0 + F1 + F2 + F3;
 
-// The dot products that all kernels of this file end in: a wave takes `ng` consecutive pairs of weight rows as one
+// The dot products that all kernels of this file end in: a wave takes `ng` consecutive pairs of weight rows (or single rows, dealt in turn) as one
 // flattened sequence of 1 KB segments (lane l: bytes [16 l, 16 l + 16) of each row's segment), a ring of segments in
 // flight, against the MB tokens' codes in LDS (v_dot8_i32_i4: eight signed 4-bit products per lane and instruction).
 // The kernels place the first requests between the phases of their fronts (fetch) and consume the ring once the codes
 // are in LDS (run).  A row's last segment may be short: the lanes past its end re-read the row's start against zero
 // codes.  The 64 partial sums of each (row, token) pair are added across the wave by a halving exchange, and the lane
 // that ends up with a pair's sum applies Linear4bit's epilogue: y = fp16(fp16(sA sW) fp16(sum)) (+ bias).
-template <int MB>
+template <int MB, int R = 2>
 struct RowPairStream {
-    static constexpr int R = 2, NS = R * MB, LV = NS == 2 ? 1 : NS == 4 ? 2 : NS == 8 ? 3 : 4;
+    static constexpr int NS = R * MB, LV = NS == 1 ? 0 : NS == 2 ? 1 : NS == 4 ? 2 : NS == 8 ? 3 : 4;
     struct Seg {
         u32x4 w[R];
         f16 sb, bi;                              // scale and bias of the output this lane will store
@@ -37,15 +37,28 @@ struct RowPairStream {
     const uint8_t* B;
     const f16* sB;
     const f16* bias;
-    int N, Kb, nseg, g0, gcount, lane, my_m, my_r, fg, fs;
+    int N, Kb, nseg, g0, gstep, gcount, lane, my_m, my_r, fg, fs;
 
     __device__ __forceinline__ void init(const uint8_t* B_, const f16* sB_, const f16* bias_, int N_, int Kb_, int ng, int wave,
                                          int lane_) {
-        B = B_, sB = sB_, bias = bias_, N = N_, Kb = Kb_, lane = lane_;
-        nseg = (Kb + 1023) >> 10;
+        begin(B_, sB_, bias_, N_, Kb_, lane_);
         const int groups = (N + R - 1) / R;
         g0 = ((int)blockIdx.x * 16 + wave) * ng;
+        gstep = 1;
         gcount = g0 >= groups ? 0 : (groups - g0 < ng ? groups - g0 : ng);
+    }
+    // the steps dealt to the waves in turn, the same wave of every workgroup first: few steps spread over all CUs
+    __device__ __forceinline__ void init_dealt(const uint8_t* B_, const f16* sB_, const f16* bias_, int N_, int Kb_, int wave,
+                                               int lane_) {
+        begin(B_, sB_, bias_, N_, Kb_, lane_);
+        const int groups = (N + R - 1) / R;
+        g0 = wave * (int)gridDim.x + (int)blockIdx.x;
+        gstep = 16 * (int)gridDim.x;
+        gcount = g0 >= groups ? 0 : (groups - g0 + gstep - 1) / gstep;
+    }
+    __device__ __forceinline__ void begin(const uint8_t* B_, const f16* sB_, const f16* bias_, int N_, int Kb_, int lane_) {
+        B = B_, sB = sB_, bias = bias_, N = N_, Kb = Kb_, lane = lane_;
+        nseg = (Kb + 1023) >> 10;
         const int vidx = lane >> (6 - LV);       // which of a pair's NS sums this lane stores at the end of the exchange
         my_m = vidx / R, my_r = vidx % R;
         fg = fs = 0;
@@ -54,13 +67,13 @@ struct RowPairStream {
         const int off = (fs * 1024 + lane * 16 < Kb) ? fs * 1024 + lane * 16 : 0;
 #pragma unroll
         for (int r = 0; r < R; ++r) {
-            int nr = (g0 + fg) * R + r;
+            int nr = (g0 + fg * gstep) * R + r;
             nr = nr < N ? nr : N - 1;
             s.w[r] = __builtin_nontemporal_load((const u32x4*)(B + (int64_t)nr * Kb + off));
         }
         // every segment carries its pair's scale along: loading it at the pair's end would make the wave wait for
         // everything it has in flight
-        int col = (g0 + fg) * R + my_r;
+        int col = (g0 + fg * gstep) * R + my_r;
         col = col < N ? col : N - 1;
         s.sb = sB[col];
         s.bi = (bias ? bias : sB)[col];          // (no bias: a harmless second read of the scale)
@@ -108,7 +121,7 @@ struct RowPairStream {
             int sum = vals[0];
             for (; off > 0; off >>= 1) sum += __shfl_xor(sum, off, QR_WAVE);
             if ((lane & ((1 << (6 - LV)) - 1)) == 0) {
-                const int col = (g0 + cg) * R + my_r;
+                const int col = (g0 + cg * gstep) * R + my_r;
                 if (my_m < M && col < N) {
                     f16 yo = (f16)(my_sa * sg.sb) * (f16)(float)sum;
                     if (bias) yo = yo + sg.bi;
@@ -357,6 +370,205 @@ __global__ __launch_bounds__(1024) void bm_gemv_kernel(const f16* __restrict__ x
     ws.run(ring, xq, MB == 1 ? sh_one : sc[ws.my_m], MB, Y);
 }
 
+// ---- OnlineHadamard (m = 64 or 128 behind a table) -> Quantizer -> Linear4bit for one or two tokens ------------
+// The same construction for rows of K m values, m = 64 with K = 97 .. 192 (7B: 11008 = 172 x 64) or m = 128 with K = 33 .. 64 and 97 .. 128
+// (13B: 13824 = 108 x 128, 5120 = 40 x 128): the two matrix stages of hadamard_m64r_kernel / hadamard_m64q_kernel (same
+// fragments, same order of sums: codes and scale are the same bits), with one wave per 16 rows of hadK and 64 columns.  The
+// weight rows of these widths are few (4096 at 7B), so they are dealt to the waves singly: in pairs half of the CUs would have none.
+// What bounds it: latency -- the row through a CU's memory path, two stages, three barriers -- under which the first 80 KB per CU
+// of the weights arrive.  As two launches (front in ONE workgroup, then dot products) 1 x 11008 -> 4096 took 11.9 us a pass.
+template <int LOG2M, int KS2, int MB>
+__global__ __launch_bounds__(1024) void mm_gemv_kernel(const f16* __restrict__ x, int K, const void* __restrict__ hadK, int signs,
+                                                       float scale, float clip, const uint8_t* __restrict__ B,
+                                                       const f16* __restrict__ sB, const f16* __restrict__ bias, int N,
+                                                       f16* __restrict__ Y) {
+    constexpr int M_ = 1 << LOG2M, CT = M_ / 16, S1K = M_ / 32, NT = 2 * KS2, CTW = 4, HV = CT / CTW, NW = 16, RD = RING;
+    extern __shared__ f32x4 smem_raw[];
+    __shared__ u32 red[NW];
+    __shared__ f16 sc[MB];
+    u32x2* Tl = (u32x2*)smem_raw;                // [CT][NT][64 lanes]
+    u32x2* xq = Tl + CT * NT * 64;               // codes of the rows, nseg * 1024 bytes each
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int l16 = lane & 15, g = lane >> 4;
+    const int tile = HV == 2 ? wave >> 1 : wave, half = HV == 2 ? wave & 1 : 0;      // 16 rows of hadK; its 64 columns
+    const int r = tile * 16 + l16, Kb = K * (M_ / 2), nseg = (Kb + 1023) >> 10;
+    const bool works = tile * 16 < K, dval = r < K;
+
+    // ---- requests: the row, the table's rows of this wave, then weights
+    u32x4 xr[S1K];
+    auto request = [&](int row) {
+#pragma unroll
+        for (int c = 0; c < S1K; ++c) xr[c] = *((const u32x4*)x + (int64_t)row * (K * (M_ / 8)) + (dval ? r * (M_ / 8) + 4 * c + g : 0));
+    };
+    request(0);
+    u32x2 hk[KS2][2];                            // hadK[r][32 ks + 16 hh + 4 g ..+ 3], or sign words (see hadamard_m64r_kernel)
+    if (signs) {
+#pragma unroll
+        for (int ks = 0; ks < KS2; ++ks) hk[ks][0][0] = ((const u32*)hadK)[dval ? r * KS2 + ks : 0];
+    } else {
+#pragma unroll
+        for (int ks = 0; ks < KS2; ++ks)
+#pragma unroll
+            for (int hh = 0; hh < 2; ++hh) {
+                const int hc = ks * 32 + hh * 16 + g * 4;
+                hk[ks][hh] = ((const u32x2*)hadK)[dval && hc < K ? (r * K + hc) >> 2 : 0];
+            }
+    }
+    RowPairStream<MB, 1> ws;
+    ws.init_dealt(B, sB, bias, N, Kb, wave, lane);
+    using Seg = typename RowPairStream<MB, 1>::Seg;
+    Seg ring[RD];
+
+    // Sylvester fragments: base tile of the parity of the column tile, and its negative
+    f16x8 sb[2][2];
+#pragma unroll
+    for (int o = 0; o < 2; ++o)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const bool neg = ((__builtin_popcount(((g & 1) * 8 + j) & l16) + ((g >> 1) & o)) & 1) != 0;
+            sb[o][0][j] = neg ? (f16)-1.0f : (f16)1.0f;
+            sb[o][1][j] = neg ? (f16)1.0f : (f16)-1.0f;
+        }
+    // T of tiles beyond K and the codes past the rows' ends: zeros
+    for (int i = tid; i < CT * NT * 32; i += 1024) ((u32x4*)Tl)[i] = u32x4{0, 0, 0, 0};
+    for (int i = tid; i < MB * nseg * 128; i += 1024) xq[i] = u32x2{0, 0};
+    __syncthreads();
+    ws.fetch(ring[0]);                           // (behind every wave's requests for the row)
+    f16 sh_one = (f16)0;
+    f16x8 hf[KS2];
+#pragma unroll
+    for (int row = 0; row < MB; ++row) {
+        // ---- stage 1: T = X . H_m for this wave's 16 rows and four column tiles, rounded to fp16 with the scale
+        if (works) {
+            u32x4 af[S1K];
+#pragma unroll
+            for (int c = 0; c < S1K; ++c) af[c] = dval ? xr[c] : u32x4{0, 0, 0, 0};
+#pragma unroll
+            for (int cc = 0; cc < CTW; ++cc) {
+                // the column tile is half * 4 + cc: its bits above the lowest decide the signs of the contraction's steps
+                f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int c = 0; c < S1K; ++c) {
+                    const f16x8 a = __builtin_bit_cast(f16x8, af[c]);
+                    if (HV == 2 && (c & 2)) {    // (popcount(c & (ct >> 1)) with ct >> 1 = 2 half + cc / 2)
+                        const bool odd = ((__builtin_popcount(c & (cc >> 1)) + half) & 1) != 0;
+                        acc = odd ? __builtin_amdgcn_mfma_f32_16x16x32_f16(a, sb[cc & 1][1], acc, 0, 0, 0)
+                                  : __builtin_amdgcn_mfma_f32_16x16x32_f16(a, sb[cc & 1][0], acc, 0, 0, 0);
+                    } else {
+                        acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, sb[cc & 1][__builtin_popcount(c & (cc >> 1)) & 1], acc, 0, 0, 0);
+                    }
+                }
+                Tl[((half * CTW + cc) * NT + tile) * 64 + lane] = u32x2{narrow_f16x2(acc[0] * scale, acc[1] * scale),
+                                                                        narrow_f16x2(acc[2] * scale, acc[3] * scale)};
+            }
+        }
+        if (row == 0) {                          // the table's fragments, under the other waves' stage 1
+#pragma unroll
+            for (int ks = 0; ks < KS2; ++ks) {
+                u32x4 fr;
+#pragma unroll
+                for (int hh = 0; hh < 2; ++hh) {
+                    const bool ok = dval && ks * 32 + hh * 16 + g * 4 < K;
+                    u32 p0 = hk[ks][hh][0], p1 = hk[ks][hh][1];
+                    if (signs) {
+                        const u32 nib = (hk[ks][0][0] >> (hh * 16 + g * 4)) & 15u;
+                        p0 = 0x3C003C00u | ((nib & 1u) << 15) | ((nib & 2u) << 30);
+                        p1 = 0x3C003C00u | ((nib & 4u) << 13) | ((nib & 8u) << 28);
+                    }
+                    fr[hh * 2] = ok ? p0 : 0u;
+                    fr[hh * 2 + 1] = ok ? p1 : 0u;
+                }
+                hf[ks] = __builtin_bit_cast(f16x8, fr);
+            }
+        }
+        if (row + 1 < MB) request(row + 1);
+        if constexpr (MB == 1) {
+            ws.fetch(ring[1]);
+            ws.fetch(ring[2]);
+        } else {
+            ws.fetch(ring[1 + 2 * row]);
+        }
+        __syncthreads();
+        // ---- stage 2: Y^T = T^T . hadK^T; the row's maximum; the codes
+        u32x2 yv[CTW];
+        float mxf = 0.f, probe = 0.f;
+#pragma unroll
+        for (int cc = 0; cc < CTW; ++cc) {
+            f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+            if (works) {
+#pragma unroll
+                for (int ks = 0; ks < KS2; ++ks) {
+                    const u32x2* const t = Tl + ((half * CTW + cc) * NT + 2 * ks) * 64 + lane;
+                    const u32x2 p0 = t[0], p1 = t[64];
+                    acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, u32x4{p0[0], p0[1], p1[0], p1[1]}), hf[ks], acc,
+                                                                 0, 0, 0);
+                }
+            }
+            if (cc == 0) probe = acc[0];
+            yv[cc] = u32x2{cvt_f16x2(acc[0], acc[1]), cvt_f16x2(acc[2], acc[3])};
+            mxf = __builtin_fmaxf(__builtin_fmaxf(mxf, __builtin_fabsf(acc[0])), __builtin_fabsf(acc[1]));
+            mxf = __builtin_fmaxf(__builtin_fmaxf(mxf, __builtin_fabsf(acc[2])), __builtin_fabsf(acc[3]));
+        }
+        u32 mx = f16_bits((f16)mxf);
+        if (__builtin_amdgcn_ballot_w64(mx >= 0x7c00u || probe != probe) != 0) {         // something non-finite: the exact form
+            u16x2 m2 = {0, 0};
+#pragma unroll
+            for (int cc = 0; cc < CTW; ++cc) {
+                m2 = __builtin_elementwise_max(m2, __builtin_bit_cast(u16x2, dval ? yv[cc][0] & 0x7fff7fffu : 0u));
+                m2 = __builtin_elementwise_max(m2, __builtin_bit_cast(u16x2, dval ? yv[cc][1] & 0x7fff7fffu : 0u));
+            }
+            mx = m2[0] > m2[1] ? m2[0] : m2[1];
+        }
+        mx = wave_max_u32_dpp(mx);
+        if (lane == 0) red[wave] = mx;
+        if constexpr (MB == 1) {
+            ws.fetch(ring[3]);
+            ws.fetch(ring[4]);
+        } else {
+            ws.fetch(ring[2 + 2 * row]);
+        }
+        __syncthreads();
+#pragma unroll
+        for (int w = 0; w < NW; ++w) mx = mx > red[w] ? mx : red[w];
+        const f16 sh = quantizer_scale(f16_from_bits((unsigned short)mx), clip);
+        const float sp = (float)sh;
+        if (MB > 1 && tid == 0) sc[row] = sh;
+        sh_one = sh;
+        u32 c01, c23;
+        auto codes_from = [&](auto pair) {
+            u32 b0[4], b1[4];
+#pragma unroll
+            for (int w = 0; w < 4; ++w) {
+                b0[w] = pair(yv[w >> 1][w & 1]);
+                b1[w] = pair(yv[2 + (w >> 1)][w & 1]);
+            }
+            c01 = pack_nibbles8(b0);
+            c23 = pack_nibbles8(b1);
+        };
+        if (fast_quant_ok(mx, sp)) {
+            const FastRecip fq = make_fast_recip(sp);
+            if (clamp_cannot_act(clip, sp)) codes_from([&](u32 w) { return sym_pair_fast<false>(w, fq); });
+            else codes_from([&](u32 w) { return sym_pair_fast<true>(w, fq); });
+        } else {
+            const bool fs_ok = scale_fast_ok(sp);
+            const float rs = fs_ok ? 1.0f / sp : 0.0f;
+            c01 = sym_codes8(u32x4{yv[0][0], yv[0][1], yv[1][0], yv[1][1]}, sp, rs, fs_ok);
+            c23 = sym_codes8(u32x4{yv[2][0], yv[2][1], yv[3][0], yv[3][1]}, sp, rs, fs_ok);
+        }
+        const auto s1 = __builtin_amdgcn_permlane32_swap(c01, c23, false, false);
+        const u32 ev = __builtin_amdgcn_perm(s1[1], s1[0], 0x05040100u);
+        const u32 od = __builtin_amdgcn_perm(s1[1], s1[0], 0x07060302u);
+        const auto s2 = __builtin_amdgcn_permlane16_swap(ev, od, false, false);
+        if (dval)
+            xq[row * (nseg * 128) + r * CT + half * CTW + g] =
+                u32x2{__builtin_amdgcn_perm(s2[1], s2[0], 0x05040100u), __builtin_amdgcn_perm(s2[1], s2[0], 0x07060302u)};
+        // (the next row's first stage writes T behind every wave's reads of it, the barrier above; the maxima are next written
+        // behind the next row's first barrier)
+    }
+    __syncthreads();
+    ws.run(ring, xq, MB == 1 ? sh_one : sc[ws.my_m], MB, Y);
+}
+
 // ---- Quantizer -> Linear4bit for one token (no Hadamard in front) ---------------------------------------------
 // The same construction with quant_rows_kernel's arithmetic as the front: every workgroup takes the row's largest
 // magnitude, the scale and the codes itself (element-wise work on the row out of L2: the scale and every code are the
@@ -520,6 +732,34 @@ __attribute__((visibility("hidden"))) int qr_internal_token_hadamard_linear(cons
     if (M == 1) QR_BG(1);
     else QR_BG(2);
 #undef QR_BG
+    return qr_launch_status();
+}
+
+// api.hip: the whole layer for one or two tokens whose rows are 64 or 128 K halves behind a table (fp16, or its sign words).
+// QR_E_UNSUPPORTED (nothing launched) for every other shape.
+__attribute__((visibility("hidden"))) int qr_internal_token_mm_linear(const void* x, int64_t M, int n, int K, const void* hadK,
+                                                                      int signs, float scale, float clip, const void* W,
+                                                                      const void* sW, const void* bias, int64_t N, void* y,
+                                                                      hipStream_t st) {
+    if (M < 1 || M > 2 || K <= 32 || (K & 3) != 0 || N <= 0 || N > (1 << 30)) return QR_E_UNSUPPORTED;
+    const int ks2 = (K + 31) / 32;
+    const bool m64 = n == 64 * K && ks2 >= 4 && ks2 <= 6, m128 = n == 128 * K && (ks2 == 2 || ks2 == 4) && !signs;
+    if (!m64 && !m128) return QR_E_UNSUPPORTED;
+    if (((uintptr_t)x & 15) || ((uintptr_t)W & 15) || ((uintptr_t)hadK & (signs ? 3 : 7))) return QR_E_UNSUPPORTED;
+    const int cus = qr_device().cus;
+    const unsigned grid = (unsigned)((N + 15) / 16 < cus ? (N + 15) / 16 : cus);
+    const size_t lds = (size_t)(m64 ? 4 : 8) * (2 * ks2) * 64 * 8 + (size_t)M * (((size_t)n / 2 + 1023) / 1024) * 1024;
+    using Kern = void (*)(const f16*, int, const void*, int, float, float, const uint8_t*, const f16*, const f16*, int, f16*);
+    static const Kern table[5][2] = {{mm_gemv_kernel<6, 4, 1>, mm_gemv_kernel<6, 4, 2>},
+                                     {mm_gemv_kernel<6, 5, 1>, mm_gemv_kernel<6, 5, 2>},
+                                     {mm_gemv_kernel<6, 6, 1>, mm_gemv_kernel<6, 6, 2>},
+                                     {mm_gemv_kernel<7, 2, 1>, mm_gemv_kernel<7, 2, 2>},
+                                     {mm_gemv_kernel<7, 4, 1>, mm_gemv_kernel<7, 4, 2>}};
+    const Kern kern = table[m64 ? ks2 - 4 : ks2 == 2 ? 3 : 4][M - 1];
+    const hipError_t e = qr_allow_dynamic_lds((const void*)kern, lds);
+    if (e != hipSuccess) return (int)e;
+    kern<<<dim3(grid), dim3(1024), lds, st>>>((const f16*)x, K, hadK, signs, scale, clip, (const uint8_t*)W, (const f16*)sW,
+                                              (const f16*)bias, (int)N, (f16*)y);
     return qr_launch_status();
 }
 

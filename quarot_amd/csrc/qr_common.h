@@ -102,6 +102,10 @@ int qr_internal_heads_matrix_quantize(const void* x, int64_t rows, int heads, co
 int qr_internal_token_hadamard_linear(const void* x, int64_t M, int n, int K, const void* hadK, float scale, float clip,
                                       const void* W, const void* sW, const void* bias, int64_t N, void* y, hipStream_t st);
 
+// decode_fused.hip: the same for rows of 64 or 128 values behind a table of order 33 and more, given in fp16 or as its sign words
+int qr_internal_token_mm_linear(const void* x, int64_t M, int n, int K, const void* hadK, int signs, float scale, float clip,
+                                const void* W, const void* sW, const void* bias, int64_t N, void* y, hipStream_t st);
+
 // decode_fused.hip: quantiser + linear layer of one or two tokens in one launch; QR_E_UNSUPPORTED, with nothing
 // launched, for anything else
 int qr_internal_token_quant_linear(const void* x, int64_t M, int64_t K, float clip, const void* W, const void* sW,
