@@ -1217,7 +1217,7 @@ MidPlan mid_plan(int64_t M, int64_t N, int64_t Kb, int64_t max_split) {
         consider(3 + i, 1, 1.7 + n * round(i, 1.0 - (double)t / (n * (double)cus)));
     }
     const int64_t whole = tiles(256, 256) / cus, left = tiles(256, 256) % cus;
-    if (reach && cus % qr_device().xcds == 0 && whole > 0 && left > 0 && 2 * left <= cus)
+    if (reach && Kb > 128 && cus % qr_device().xcds == 0 && whole > 0 && left > 0 && 2 * left <= cus)
         consider(6, 1, 1.7 + (double)whole * round(2, 0.0) + round(0, 1.0 - 2.0 * (double)left / (double)cus));
     const int64_t all_stages = (Kb + 127) / 128;
     for (int64_t ks = 2; ks <= max_split && ks <= all_stages / 4; ++ks)

@@ -50,8 +50,16 @@ __device__ __forceinline__ TilePlace tile_place(int unit, int tiles_m, int tiles
 // on top of the corrected sum of everything before, 64 per k: (225 * 192 + 64 * (512 - 192)) * 256 = 16.3e6 < 2^24 for K up to 131072.
 constexpr int kSegment = 192;
 
-// LDS bytes of a tile: stage buffers, then scales ([256] sB, [256] bias, [BM] sA in fp16), then row sums of both operands
-constexpr int e2m3_lds(int BM, int KG) { return (KG == 1 ? 2 : 3) * (BM + 256) * 128 + (512 + BM) * 2 + KG * (BM + 256) * 4; }
+// LDS bytes: stage buffers, then scales ([256] sB, [256] bias, [BM] sA in fp16; KG = 1: of two tiles), row sums of both operands, and
+// (KG = 1, whose stage buffers hold the next tile's first stages by then) the output slabs
+constexpr int e2m3_lds(int BM, int KG) {
+    return KG == 1 ? 2 * (BM + 256) * 128 + 2 * (512 + BM) * 2 + (BM + 256) * 4 + 16384
+                   : 3 * (BM + 256) * 128 + (512 + BM) * 2 + 2 * (BM + 256) * 4;
+}
+// First row of A and of B of a tile
+struct Origin {
+    int m0, n0;
+};
 
 // Four waves, ONE per SIMD, each with a wave tile of 128 (96) x 128: 16 (12) accumulator tiles, up to all 256 accumulation registers.
 //   KG = 1   waves 2 (M) x 2 (N), BM = 256 or 192, whole K per wave
@@ -61,22 +69,28 @@ constexpr int e2m3_lds(int BM, int KG) { return (KG == 1 ? 2 : 3) * (BM + 256) *
 // which 16 bytes of a line a lane fetches), and a sub-step is 64 k: 16 bytes per lane and fragment of 32 rows.  A wave hides everything
 // under its own matrix instructions, in explicit slots: one matrix instruction and an even share of the 14 vector instructions per
 // fragment that spread the NEXT sub-step's nibbles; behind a fragment's last one the read of the sub-step AFTER that into the same
-// registers; loads of the stage after next, one in three slots (one in every slot, they back up behind one another: 59 instead of 55
-// cycles per slot).  A scheduling barrier after every slot keeps this order.
+// registers; loads of the stage after next, one in two (KG = 2: three) slots (one in every slot, they back up behind one another: 59
+// instead of 55 cycles per slot).  A scheduling barrier after every slot keeps this order.
+//
+// KG = 1: a workgroup takes `count` tiles, place(0), place(1) .., without a gap in this pipeline: where the loop over a tile's K would
+// load stages past its end, it loads the next tile's first ones, and the next tile's first sub-step is spread before the epilogue.
+// With a workgroup per tile every tile paid some 2-3 us for launch, first loads and first sub-step: 32768 x 4096 x 1024 138 -> 122 us,
+// 32768 x 11008 x 4096 835 -> 812, 32768 x 4096 x 11008 710 -> 690.  (The turn is prepared between two runs of the stage loop: a branch
+// for it inside the loop, or one that lets the epilogue's stores pass the first barrier, costs 6 % of every stage.)
 //
 // What bounds it (256 rows, 32768 x 4096 x 11008): a wave issues an instruction in about 5 cycles, and a sub-step has 20 matrix and 112
 // vector instructions, 8 LDS reads, 4 loads and some 20 others: 55 cycles of 2.05 GHz per accumulator tile and sub-step, where the
 // matrix unit alone would need 36; the clock is the power limit's (2.4 GHz without load).  Inside the loop that is 5.0e15 operations
-// per second (the int8 instruction with nothing else going on sustains 3.9-4.2e15); the whole launch, with 1.9 us before and about 6 us after
-// the loop of every tile (3 us of arithmetic with one wave per SIMD, then the compute units write 33 MB at a time), 4.2e15: 690 us against
-// 870-890 of the int8 kernel with the same tiles; 32768 x 11008 x 4096 818 us (1010; 850 with a branch around every store),
-// 8192 x 5120 x 5120 127 (146), 1777 x 8192 x 28672 194 (244), 2048 x 4096 x 11008 53 (58-66).  Delaying the first workgroups by 0 .. 8 us, so
+// per second (the int8 instruction with nothing else going on sustains 3.9-4.2e15); the whole launch, with about 6 us behind the loop of
+// every tile (3 us of arithmetic with one wave per SIMD, then the compute units write 33 MB at a time), 4.3e15: 690 us against
+// 870-890 of the int8 kernel with the same tiles; 32768 x 11008 x 4096 812 us (1010; 850 with a branch around every store),
+// 8192 x 5120 x 5120 124 (146), 1777 x 8192 x 28672 194 (244), 2048 x 4096 x 11008 53 (58-66).  Delaying the first workgroups by 0 .. 8 us, so
 // that compute units do not write at once, changed nothing.
-template <bool RAGGED, int BM, int KG>
-__device__ __forceinline__ void e2m3_tile(
+template <bool DEQ, bool RAGGED, int BM, int KG, class Place>
+__device__ __forceinline__ void e2m3_tiles(
     const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, int M, int N, int Kb, int32_t* __restrict__ C,
     f16* __restrict__ Y, const f16* __restrict__ sA, const f16* __restrict__ sB, const f16* __restrict__ bias,
-    int m0, int n0) {
+    int count, Place place) {
     static_assert(KG == 1 ? (BM == 256 || BM == 192) : BM == 128, "wave tiles of 128 x 128 or 96 x 128");
     constexpr int NT = 256;
     constexpr int TM = KG == 1 ? BM / 2 : BM, IM = TM / 32, JN = 4;
@@ -91,8 +105,8 @@ __device__ __forceinline__ void e2m3_tile(
     constexpr int UNP = 14 * NF;                            // vector instructions that spread a sub-step's fragments
     extern __shared__ u32x4 e2m3_smem[];
     char* const lds = (char*)e2m3_smem;
-    f16* const scales = (f16*)(lds + NBUF * STAGE);
-    float* const rowsum = (float*)(scales + 512 + BM);      // [KG][BM] of A
+    f16* scales = (f16*)(lds + NBUF * STAGE);               // (of the tile at hand)
+    float* const rowsum = (float*)(scales + (KG == 1 ? 2 : 1) * (512 + BM));     // [KG][BM] of A
     float* const colsum = rowsum + KG * BM;                 // [KG][256] of B
 
     const int tid = threadIdx.x, lane = tid & 63;
@@ -105,20 +119,28 @@ __device__ __forceinline__ void e2m3_tile(
     // loads: chunk tid + i * 256 of a stage is 16 bytes of row tid / 8 + 32 i, at LDS position (row, tid % 8): the lane fetches the piece
     // that the layout keeps there (the key is the same for all of a lane's rows)
     const int srow = tid >> 3, piece = ((tid & 7) ^ ((srow >> 1) & 7)) * 16;
+    Origin at = place(0);
     u32 goff[NL];
+    auto aim = [&](Origin o) {
+        int row0 = srow;
+        asm volatile("" : "+v"(row0));                      // (computed here, not kept over the tiles: registers are full)
 #pragma unroll
-    for (int i = 0; i < NL; ++i) {
-        const int row = srow + i * 32;
-        int gr = row < BM ? m0 + row : n0 + row - BM;
-        const int lim = row < BM ? M - 1 : N - 1;
-        gr = gr < lim ? gr : lim;
-        goff[i] = (u32)gr * (u32)Kb + (u32)piece;
-    }
+        for (int i = 0; i < NL; ++i) {
+            const int row = row0 + i * 32;
+            int gr = row < BM ? o.m0 + row : o.n0 + row - BM;
+            const int lim = row < BM ? M - 1 : N - 1;
+            gr = gr < lim ? gr : lim;
+            goff[i] = (u32)gr * (u32)Kb + (u32)piece;
+        }
+    };
+    aim(at);
+    bool more = false;                                      // stages past the end are the next tile's
     const __amdgpu_buffer_rsrc_t rsrc_a = __builtin_amdgcn_make_buffer_rsrc((void*)A, 0, (int)((u32)M * (u32)Kb), 0x00020000);
     const __amdgpu_buffer_rsrc_t rsrc_b = __builtin_amdgcn_make_buffer_rsrc((void*)B, 0, (int)((u32)N * (u32)Kb), 0x00020000);
-    // (stages past the end repeat the last one into a buffer that nobody reads: every stage issues the same number of loads)
+    // (where there is no next tile, stages past the end repeat the last one into a buffer that nobody reads: every stage issues the
+    // same number of loads)
     auto load1 = [&](int st, int buf, int i) __attribute__((always_inline)) {
-        const int kb = (st < stages ? st : stages - 1) * 128;
+        const int kb = (st < stages ? st : more ? st - stages : stages - 1) * 128;
         __attribute__((address_space(3))) void* dst =
             (__attribute__((address_space(3))) void*)(lds + buf * STAGE + (i * NT + wave * 64) * 16);
         // pieces past the end of a row lie beyond the buffer's range and arrive as zeros: codes 0
@@ -128,12 +150,6 @@ __device__ __forceinline__ void e2m3_tile(
     };
 
     f32x16 acc[IM][JN];
-#pragma unroll
-    for (int i = 0; i < IM; ++i)
-#pragma unroll
-        for (int j = 0; j < JN; ++j)
-#pragma unroll
-            for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
 
     // Group of 32 rows that fragment i of A / j of B holds.  Waves that share rows of an operand hold its fragments in different orders, so that
     // fragments 0 and 1, whose rows a wave adds up, are different rows in each; K-group 1 holds the halves of B swapped, so that
@@ -226,9 +242,10 @@ __device__ __forceinline__ void e2m3_tile(
     };
 
     // One sub-step: multiply `cur`, spread `p` into `nxt`, read sub-step RU of the stage buffer at buf_off into `p` behind it, and load chunks
-    // LOAD0 .. LOAD1 of stage load_st into buffer load_buf from slot LSLOT on.  BSLOT >= 0: the stage's barrier stands in this slot (at
-    // most ALLOWED of the wave's loads still in flight), and no read is issued before it.
-    constexpr int EVERY = 3;                                // slots from one load to the next
+    // LOAD0 .. LOAD1 of stage load_st into buffer load_buf from slot LSLOT on. 
+    // BSLOT >= 0: the stage's barrier stands in this slot (at most ALLOWED of the wave's memory operations still in flight), and no read is
+    // issued before it.
+    constexpr int EVERY = KG == 1 ? 2 : 3;                  // slots from one load to the next
 #define QR_E2M3_BARRIER(ALLOWED) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(ALLOWED) : "memory");
     auto substep = [&](const Ops& cur, Ops& nxt, Packed& p, auto ru, int buf_off, auto bslot, auto allowed, int load_st, int load_buf,
                        auto load0, auto load1_, auto lslot) __attribute__((always_inline)) {
@@ -256,26 +273,28 @@ __device__ __forceinline__ void e2m3_tile(
     // The epilogue's scales and bias are fetched first and parked in LDS: a load in the epilogue would wait for the stores before it.
     // (Indices clamped to the matrix: what belongs to rows and columns beyond it is never stored.)
     f16 pre_sb = (f16)0, pre_bi = (f16)-0.0f, pre_sa = (f16)0;
-    if (Y) {
-        const int col = n0 + tid < N ? n0 + tid : N - 1, row = m0 + tid < M ? m0 + tid : M - 1;
+    auto fetch_scales = [&](Origin o) {
+        if (!DEQ) return;
+        const int col = o.n0 + tid < N ? o.n0 + tid : N - 1, row = o.m0 + tid < M ? o.m0 + tid : M - 1;
         pre_sb = sB[col], pre_sa = sA[row];
         if (bias) pre_bi = bias[col];
-    }
-    // Loads of a stage: KG = 1 in sub-steps 2 and 3 of the stage two before it (once its buffer is free) and in sub-step 0 of the one before
-    // it, KG = 2 in the two sub-steps of the stage three before it
-    constexpr int L2 = (NU - 4 + EVERY - 1) / EVERY < NL ? (NU - 4 + EVERY - 1) / EVERY : NL;
-    constexpr int L3 = KG == 2 ? NL : L2 + (NU + EVERY - 1) / EVERY < NL ? L2 + (NU + EVERY - 1) / EVERY : NL;
-    constexpr int AHEAD = KG == 1 ? L3 : 2 * NL;            // loads of later stages that are out when stage 0 is waited for
-#pragma unroll
-    for (int s = 0; s < NBUF; ++s)
-#pragma unroll
-        for (int i = 0; i < (s == 1 ? L3 : NL); ++i) load1(s, s, i);
-    QR_E2M3_BARRIER(AHEAD)
-    if (Y) {
+    };
+    auto park_scales = [&] {
+        if (!DEQ) return;
         scales[tid] = pre_sb;
         scales[256 + tid] = pre_bi;
         if (tid < BM) scales[512 + tid] = pre_sa;
-    }
+    };
+    fetch_scales(at);
+    // Loads of a stage: KG = 1 in sub-steps 2 and 3 of the stage two before it (once its buffer is free), KG = 2 in the two sub-steps of the
+    // stage three before it
+    constexpr int L2 = (NU - 4 + EVERY - 1) / EVERY < NL ? (NU - 4 + EVERY - 1) / EVERY : NL;
+#pragma unroll
+    for (int s = 0; s < NBUF; ++s)
+#pragma unroll
+        for (int i = 0; i < NL; ++i) load1(s, s, i);
+    QR_E2M3_BARRIER((NBUF - 1) * NL)
+    park_scales();
     Packed pk;
     Ops ops[2];
 #pragma unroll
@@ -285,16 +304,36 @@ __device__ __forceinline__ void e2m3_tile(
     for (int t = 0; t < NF; ++t) read1(1, frag_at(t), 0, pk);   // in the order of the loop, whose waits count reads
 
     int off = 0, nxt = STAGE, buf = 0;                          // stage ks is in buffer `buf` at `off`, the next one at `nxt`
-    for (int seg = 0; seg < stages; seg += kSegment) {
-        const int end = seg + kSegment < stages ? seg + kSegment : stages;
+    for (int t = 0;;) {
+    Origin then{0, 0};                                          // the tile after this one
+    // (zeros by matrix instructions: one each, and no vector of zeros that has to live somewhere)
+#pragma unroll
+    for (int i = 0; i < IM; ++i)
+#pragma unroll
+        for (int j = 0; j < JN; ++j) {
+            f32x16 none;
+#pragma unroll
+            for (int v = 0; v < 16; ++v) none[v] = 0.f;
+            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(0.f, 0.f, none, 0, 0, 0);
+        }
+    for (int ks = 0, seg = 0; ks < stages;) {
+        const int end = seg + kSegment < stages ? seg + kSegment : stages;      // the accumulators are corrected here
         if constexpr (KG == 1) {
             // Stage ks is read during sub-steps 2, 3 of stage ks - 1 and 0, 1 of stage ks.  The barrier early in sub-step 2: stage ks + 1 has
             // landed, everybody is done with stage ks.
-            for (int ks = seg; ks < end; ++ks) {
-                substep(ops[0], ops[1], pk, IC<2>(), off, IC<-1>(), IC<0>(), ks + 1, buf ^ 1, IC<L3>(), IC<NL>(), IC<0>());
+            const int turn = stages - 2;                        // from this stage on the loads are the next tile's
+            if (ks == turn && t + 1 < count) {
+                then = place(t + 1);
+                aim(then);
+                fetch_scales(then);
+                more = true;
+            }
+            const int stop = ks < turn && turn < end ? turn : end;
+            for (; ks < stop; ++ks) {
+                substep(ops[0], ops[1], pk, IC<2>(), off, IC<-1>(), IC<0>(), 0, 0, IC<0>(), IC<0>(), IC<0>());
                 substep(ops[1], ops[0], pk, IC<3>(), off, IC<-1>(), IC<0>(), 0, 0, IC<0>(), IC<0>(), IC<0>());
                 substep(ops[0], ops[1], pk, IC<0>(), nxt, IC<3>(), IC<0>(), ks + 2, buf, IC<0>(), IC<L2>(), IC<4>());
-                substep(ops[1], ops[0], pk, IC<1>(), nxt, IC<-1>(), IC<0>(), ks + 2, buf, IC<L2>(), IC<L3>(), IC<0>());
+                substep(ops[1], ops[0], pk, IC<1>(), nxt, IC<-1>(), IC<0>(), ks + 2, buf, IC<L2>(), IC<NL>(), IC<0>());
                 off = STAGE - off;
                 nxt = STAGE - nxt;
                 buf ^= 1;
@@ -302,19 +341,22 @@ __device__ __forceinline__ void e2m3_tile(
         } else {
             // Sub-step v of stage ks is read during sub-step v of stage ks - 1.  The barrier early in the first sub-step: stage ks + 1 has landed
             // (at most stage ks + 2 is out), everybody is done with stage ks.
-            for (int ks = seg; ks < end; ++ks) {
+            for (; ks < end; ++ks) {
                 substep(ops[0], ops[1], pk, IC<0>(), nxt, IC<3>(), IC<NL>(), ks + 3, buf, IC<0>(), IC<L2>(), IC<4>());
                 substep(ops[1], ops[0], pk, IC<1>(), nxt, IC<-1>(), IC<0>(), ks + 3, buf, IC<L2>(), IC<NL>(), IC<0>());
                 nxt = nxt == 2 * STAGE ? 0 : nxt + STAGE;
                 buf = buf == 2 ? 0 : buf + 1;
             }
         }
+        if (ks < end) continue;
         // sum a b / 64 = acc - (sum of the row's u) / 8 - (sum of the column's u) / 8 + number of k: a matrix instruction with k = 2 per tile
         // (each K-group corrects its own part by its own sums).  The compiler does not see that `sums` comes from a matrix instruction: its
         // last result is waited for by hand.
         asm volatile("s_nop 15\n\ts_nop 15" : "+v"(sums)::"memory");
-        if (lane < 8 * NS) {
-            const int g = lane >> 4, r = lane & 15;         // fragments 2 g, 2 g + 1: two of A, then those of B
+        int ls = lane;
+        asm volatile("" : "+v"(ls));
+        if (ls < 8 * NS) {
+            const int g = ls >> 4, r = ls & 15;         // fragments 2 g, 2 g + 1: two of A, then those of B
             float* const s = g == 0 ? rowsum + kg * BM + wm * TM : colsum + kg * 256 + wn * 128;
             const int f0 = g == 0 ? ga(0) : g == 1 ? gb(0) : gb(2), f1 = g == 0 ? ga(1) : g == 1 ? gb(1) : gb(3);
             s[f0 * 32 + r] = sums[0];
@@ -323,21 +365,24 @@ __device__ __forceinline__ void e2m3_tile(
             s[f1 * 32 + 16 + r] = sums[3];
         }
         __syncthreads();
-        const float count = (float)((end - seg) * (256 / KG));
+        const float terms = (float)((end - seg) * (256 / KG));
 #pragma unroll
         for (int i = 0; i < IM; ++i) {
-            const float rs = count - rowsum[kg * BM + wm * TM + ga(i) * 32 + (lane & 31)];
+            const float rs = terms - rowsum[kg * BM + wm * TM + ga(i) * 32 + (ls & 31)];
 #pragma unroll
             for (int j = 0; j < JN; ++j) {
-                const float cs = colsum[kg * 256 + wn * 128 + gb(j) * 32 + (lane & 31)];
-                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(khalf ? 1.f : -cs, khalf ? rs : 1.f, acc[i][j], 0, 0, 0);
+                const float cs = colsum[kg * 256 + wn * 128 + gb(j) * 32 + (ls & 31)];
+                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32((ls >> 5) ? 1.f : -cs, (ls >> 5) ? rs : 1.f, acc[i][j], 0, 0, 0);
             }
         }
         sums = f32x4{0.f, 0.f, 0.f, 0.f};
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");     // (the sums are read before the next ones are written)
+        seg = end;
     }
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");        // repeats of the last stage still landing in the stage buffers
-    __syncthreads();                                        // ... which the exchange and the output slabs reuse
+    // repeats of the last stage are still landing in the stage buffers, which the K-groups' exchange and the next user of this LDS take
+    const bool last = t + 1 == count;
+    if (KG == 2 || last) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if (KG == 2) __syncthreads();
     if constexpr (KG == 2) {
         // the K-groups hold partial sums of the same 128 x 128 wave tile: each keeps the columns j = 0, 1 and sends 2, 3 through LDS
         u32x4* xbuf = e2m3_smem;
@@ -366,11 +411,14 @@ __device__ __forceinline__ void e2m3_tile(
     }
 
     // Epilogue: lane l, register v -> column (v / 4) * 8 + (l / 32) * 4 + v % 4 of the B tile, token l % 32
+    int ln = lane;
+    asm volatile("" : "+v"(ln));                           // (addresses are computed here, not kept over the tiles: registers are full)
+    const int kh = ln >> 5;
     constexpr int JO = KG == 2 ? 2 : 4;                     // column groups that this wave puts out
-    if (Y) {
+    if constexpr (DEQ) {
         // one slab of 32 x 64 behind the other, the stores of each behind the next one's arithmetic
-        char* const region = lds + wave * 4096;
-        const SlabOut out = slab_out(Y, m0, M - m0 < BM ? M - m0 : BM, N, lane);
+        char* const region = (KG == 1 ? (char*)(colsum + 256) : lds) + wave * 4096;
+        const SlabOut out = slab_out(Y, at.m0, M - at.m0 < BM ? M - at.m0 : BM, N, ln);
         Slab slab;
 #pragma unroll
         for (int jb = 0; jb < JO; jb += 2) {
@@ -379,13 +427,13 @@ __device__ __forceinline__ void e2m3_tile(
             for (int jj = 0; jj < 2; ++jj)
 #pragma unroll
                 for (int gq = 0; gq < 4; ++gq) {
-                    const int col = wn * 128 + gb(jb + jj) * 32 + gq * 8 + khalf * 4;
+                    const int col = wn * 128 + gb(jb + jj) * 32 + gq * 8 + kh * 4;
                     sbh[jj][gq] = *(const f16x4*)(scales + col);
                     bih[jj][gq] = *(const f16x4*)(scales + 256 + col);
                 }
 #pragma unroll
             for (int i = 0; i < IM; ++i) {
-                const f16 sa = scales[512 + wm * TM + ga(i) * 32 + (lane & 31)];
+                const f16 sa = scales[512 + wm * TM + ga(i) * 32 + (ln & 31)];
                 f16x4 o[2][4];
 #pragma unroll
                 for (int jj = 0; jj < 2; ++jj) {
@@ -396,25 +444,24 @@ __device__ __forceinline__ void e2m3_tile(
                                                     acc[i][jb + jj][gq * 4 + 3], sa, sbh[jj][gq], bih[jj][gq]);
                 }
                 if (jb + i > 0)
-                    slab_store(out, slab, wm * TM + ga(i > 0 ? i - 1 : IM - 1) * 32, n0 + wn * 128 + gb(i > 0 ? jb : jb - 2) * 32, lane);
-                slab = slab_turn(region, o, lane);
+                    slab_store(out, slab, wm * TM + ga(i > 0 ? i - 1 : IM - 1) * 32, at.n0 + wn * 128 + gb(i > 0 ? jb : jb - 2) * 32, ln);
+                slab = slab_turn(region, o, ln);
             }
         }
-        slab_store(out, slab, wm * TM + ga(IM - 1) * 32, n0 + wn * 128 + gb(JO - 2) * 32, lane);
-        return;
-    }
+        slab_store(out, slab, wm * TM + ga(IM - 1) * 32, at.n0 + wn * 128 + gb(JO - 2) * 32, ln);
+    } else {
     // int32 sums: four columns of a row per lane and store
     const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
-        (void*)(C + (int64_t)m0 * N), 0, (int)((u32)(M - m0 < BM ? M - m0 : BM) * (u32)N * 4u), 0x00020000);
+        (void*)(C + (int64_t)at.m0 * N), 0, (int)((u32)(M - at.m0 < BM ? M - at.m0 : BM) * (u32)N * 4u), 0x00020000);
 #pragma unroll
     for (int i = 0; i < IM; ++i) {
-        const u32 row = (u32)(wm * TM + ga(i) * 32 + (lane & 31)) * (u32)N;
+        const u32 row = (u32)(wm * TM + ga(i) * 32 + (ln & 31)) * (u32)N;
 #pragma unroll
         for (int j = 0; j < JO; ++j) {
             asm volatile("" : "+a"(acc[i][j]));
 #pragma unroll
             for (int gq = 0; gq < 4; ++gq) {
-                const int col = n0 + wn * 128 + gb(j) * 32 + gq * 8 + khalf * 4;
+                const int col = at.n0 + wn * 128 + gb(j) * 32 + gq * 8 + kh * 4;
                 const u32 off = (row + (u32)col) * 4u;
                 u32x4 o;
 #pragma unroll
@@ -429,22 +476,35 @@ __device__ __forceinline__ void e2m3_tile(
             }
         }
     }
+    }
+    if (KG == 2 || last) return;
+    // the next tile's scales into the other half of their place (a slower wave may still read this tile's)
+    scales = scales == (f16*)(lds + NBUF * STAGE) ? scales + 512 + BM : (f16*)(lds + NBUF * STAGE);
+    park_scales();
+    more = false;
+    at = then;
+    ++t;
+    }
 #undef QR_E2M3_BARRIER
 }
 
-template <bool RAGGED, int BM>
+// Tiles are dealt to the XCDs in runs of `per_xcd`, and workgroup b takes every (gridDim / nxcd)-th of its XCD's run
+template <bool DEQ, bool RAGGED, int BM>
 __global__ __launch_bounds__(256) void gemm_sp256_kernel(
     const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, int M, int N, int Kb, int32_t* __restrict__ C,
     f16* __restrict__ Y, const f16* __restrict__ sA, const f16* __restrict__ sB, const f16* __restrict__ bias,
     int tiles_m, int tiles_n, int nxcd, int) {
-    const int per_xcd = gridDim.x / nxcd;
-    const int tile = (blockIdx.x % nxcd) * per_xcd + blockIdx.x / nxcd;
-    if (tile >= tiles_m * tiles_n) return;
-    const TilePlace p = tile_place(tile, tiles_m, tiles_n);
-    e2m3_tile<RAGGED, BM, 1>(A, B, M, N, Kb, C, Y, sA, sB, bias, p.tm * BM, p.tn * 256);
+    const int tiles = tiles_m * tiles_n, per_xcd = (tiles + nxcd - 1) / nxcd, xcd = blockIdx.x % nxcd;
+    const int run = tiles - xcd * per_xcd < per_xcd ? tiles - xcd * per_xcd : per_xcd;
+    const int first = blockIdx.x / nxcd, step = gridDim.x / nxcd;
+    if (first >= run) return;
+    e2m3_tiles<DEQ, RAGGED, BM, 1>(A, B, M, N, Kb, C, Y, sA, sB, bias, (run - first + step - 1) / step, [=](int t) {
+        const TilePlace p = tile_place(xcd * per_xcd + first + t * step, tiles_m, tiles_n);
+        return Origin{p.tm * BM, p.tn * 256};
+    });
 }
 
-template <bool RAGGED>
+template <bool DEQ, bool RAGGED>
 __global__ __launch_bounds__(256) void gemm_spk_kernel(
     const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, int M, int N, int Kb, int32_t* __restrict__ C,
     f16* __restrict__ Y, const f16* __restrict__ sA, const f16* __restrict__ sB, const f16* __restrict__ bias,
@@ -453,30 +513,32 @@ __global__ __launch_bounds__(256) void gemm_spk_kernel(
     const int tile = (blockIdx.x % nxcd) * per_xcd + blockIdx.x / nxcd;
     if (tile >= tiles_m * tiles_n) return;
     const TilePlace p = tile_place(tile, tiles_m, tiles_n);
-    e2m3_tile<RAGGED, 128, 2>(A, B, M, N, Kb, C, Y, sA, sB, bias, p.tm * 128, p.tn * 256);
+    e2m3_tiles<DEQ, RAGGED, 128, 2>(A, B, M, N, Kb, C, Y, sA, sB, bias, 1, [=](int) { return Origin{p.tm * 128, p.tn * 256}; });
 }
 
 // Whole rounds of 256x256 tiles over the CUs, then the tiles of the last round, where they are at most half as many as
 // there are CUs, as two 128x256 tiles each: a last round of R tiles keeps cus - R CUs idle for a whole tile's time, its halves
-// fill 2 R CUs for a part of it.  `whole` (a multiple of the CU count) workgroups take the whole tiles, those after them the halves; both kinds
-// need a CU to themselves (LDS), so a half starts where a whole tile has ended.
-template <bool RAGGED>
+// fill 2 R CUs for a part of it.  A workgroup per CU (both kinds need a CU to themselves: LDS): `whole` tiles among them all, a multiple of
+// their number, then at most one half each.
+template <bool DEQ, bool RAGGED>
 __global__ __launch_bounds__(256) void gemm_sp256_tail_kernel(
     const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, int M, int N, int Kb, int32_t* __restrict__ C,
     f16* __restrict__ Y, const f16* __restrict__ sA, const f16* __restrict__ sB, const f16* __restrict__ bias,
     int tiles_m, int tiles_n, int nxcd, int whole) {
-    if ((int)blockIdx.x < whole) {
-        const TilePlace p = tile_place((blockIdx.x % nxcd) * (whole / nxcd) + blockIdx.x / nxcd, tiles_m, tiles_n);
-        e2m3_tile<RAGGED, 256, 1>(A, B, M, N, Kb, C, Y, sA, sB, bias, p.tm * 256, p.tn * 256);
-        return;
-    }
-    const int b = blockIdx.x - whole;
-    const int unit = (b % nxcd) * (((int)gridDim.x - whole) / nxcd) + b / nxcd;
-    if (whole + unit / 2 >= tiles_m * tiles_n) return;
+    const int grid = gridDim.x, b = blockIdx.x;
+    e2m3_tiles<DEQ, RAGGED, 256, 1>(A, B, M, N, Kb, C, Y, sA, sB, bias, whole / grid, [=](int t) {
+        const int v = b + t * grid;
+        const TilePlace p = tile_place((v % nxcd) * (whole / nxcd) + v / nxcd, tiles_m, tiles_n);
+        return Origin{p.tm * 256, p.tn * 256};
+    });
+    const int halves = ((tiles_m * tiles_n - whole) * 2 + nxcd - 1) / nxcd * nxcd;
+    const int unit = (b % nxcd) * (halves / nxcd) + b / nxcd;
+    if (b >= halves || whole + unit / 2 >= tiles_m * tiles_n) return;
     const TilePlace p = tile_place(whole + unit / 2, tiles_m, tiles_n);
     const int m0 = p.tm * 256 + (unit & 1) * 128;
     if (m0 >= M) return;
-    e2m3_tile<RAGGED, 128, 2>(A, B, M, N, Kb, C, Y, sA, sB, bias, m0, p.tn * 256);
+    __syncthreads();                                        // the LDS changes hands
+    e2m3_tiles<DEQ, RAGGED, 128, 2>(A, B, M, N, Kb, C, Y, sA, sB, bias, 1, [=](int) { return Origin{m0, p.tn * 256}; });
 }
 
 }  // namespace
@@ -490,18 +552,23 @@ int qr_internal_gemm_e2m3(int shape, const void* A, const void* B, int M, int N,
     const int tiles_m = (M + bm - 1) / bm, tiles_n = (N + 255) / 256;
     const int nxcd = qr_device().xcds, cus = qr_device().cus;
     const int64_t tiles = (int64_t)tiles_m * tiles_n, whole = shape == 3 ? tiles / cus * cus : 0;
-    // the grid is a whole number of rounds over the XCDs
-    const int64_t grid = shape == 3 ? whole + ((tiles - whole) * 2 + nxcd - 1) / nxcd * nxcd : (tiles + nxcd - 1) / nxcd * nxcd;
+    // the grid is a whole number of rounds over the XCDs; 192- and 256-row tiles: a workgroup per CU, which takes several (where K is more
+    // than the one stage in which a turn cannot be prepared)
+    const bool turns = shape != 0 && Kb > 128 && cus % nxcd == 0;
+    if (shape == 3 && (!turns || whole == 0 || 2 * (tiles - whole) > cus)) return QR_E_UNSUPPORTED;      // (mid_plan's rule)
+    const int64_t all = (tiles + nxcd - 1) / nxcd * nxcd, grid = turns && all > cus ? cus : all;
     if (grid > 0x3fffffff) return QR_E_SHAPE;
     using Kern = void (*)(const uint8_t*, const uint8_t*, int, int, int, int32_t*, f16*, const f16*, const f16*, const f16*, int, int,
                           int, int);
-    static const Kern table[4][2] = {{gemm_spk_kernel<false>, gemm_spk_kernel<true>},
-                                     {gemm_sp256_kernel<false, 192>, gemm_sp256_kernel<true, 192>},
-                                     {gemm_sp256_kernel<false, 256>, gemm_sp256_kernel<true, 256>},
-                                     {gemm_sp256_tail_kernel<false>, gemm_sp256_tail_kernel<true>}};
+    // (int32 sums take the kernels for any K)
+    static const Kern table[4][3] = {
+        {gemm_spk_kernel<true, false>, gemm_spk_kernel<true, true>, gemm_spk_kernel<false, true>},
+        {gemm_sp256_kernel<true, false, 192>, gemm_sp256_kernel<true, true, 192>, gemm_sp256_kernel<false, true, 192>},
+        {gemm_sp256_kernel<true, false, 256>, gemm_sp256_kernel<true, true, 256>, gemm_sp256_kernel<false, true, 256>},
+        {gemm_sp256_tail_kernel<true, false>, gemm_sp256_tail_kernel<true, true>, gemm_sp256_tail_kernel<false, true>}};
     constexpr int lds256 = e2m3_lds(256, 1), lds128 = e2m3_lds(128, 2);
     const size_t lds = shape == 0 ? lds128 : shape == 1 ? e2m3_lds(192, 1) : shape == 2 ? lds256 : lds128 > lds256 ? lds128 : lds256;
-    const Kern kern = table[shape][(Kb & 127) != 0 ? 1 : 0];
+    const Kern kern = table[shape][!Y ? 2 : (Kb & 127) != 0 ? 1 : 0];
     const hipError_t e = qr_allow_dynamic_lds((const void*)kern, lds);
     if (e != hipSuccess) return (int)e;
     kern<<<dim3((unsigned)grid), dim3(256), lds, st>>>((const uint8_t*)A, (const uint8_t*)B, M, N, Kb, (int32_t*)C, (f16*)Y,
