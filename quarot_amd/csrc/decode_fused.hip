@@ -8,6 +8,7 @@
 // requested, keeps the codes in LDS and goes on as the dot-product kernel does (v_dot8_i32_i4 over 1 KB segments of
 // the weight rows, gemv_i4_kernel's arithmetic and epilogue).  Nothing is exchanged between workgroups.
 #include "qr_common.h"
+#include "qr_mm_row.h"
 
 namespace {
 
@@ -376,112 +377,43 @@ __global__ __launch_bounds__(1024) void bm_gemv_kernel(const f16* __restrict__ x
 // fragments, same order of sums: codes and scale are the same bits), with one wave per 16 rows of hadK and 64 columns.  The
 // weight rows of these widths are few (4096 at 7B), so they are dealt to the waves singly: in pairs half of the CUs would have none.
 // What bounds it: latency -- the row through a CU's memory path, two stages, three barriers -- under which the first 80 KB per CU
-// of the weights arrive.  As two launches (front in ONE workgroup, then dot products) 1 x 11008 -> 4096 took 11.9 us a pass.
+// of the weights arrive.  As two launches (front in ONE workgroup, then dot products) 1 x 11008 -> 4096 took 11.9 us a pass; now 8.1.
 template <int LOG2M, int KS2, int MB>
 __global__ __launch_bounds__(1024) void mm_gemv_kernel(const f16* __restrict__ x, int K, const void* __restrict__ hadK, int signs,
                                                        float scale, float clip, const uint8_t* __restrict__ B,
                                                        const f16* __restrict__ sB, const f16* __restrict__ bias, int N,
                                                        f16* __restrict__ Y) {
-    constexpr int M_ = 1 << LOG2M, CT = M_ / 16, S1K = M_ / 32, NT = 2 * KS2, CTW = 4, HV = CT / CTW, NW = 16, RD = RING;
+    using Front = MmRow<LOG2M, KS2, 1024>;
+    constexpr int NW = 16, RD = RING;
     extern __shared__ f32x4 smem_raw[];
     __shared__ u32 red[NW];
     __shared__ f16 sc[MB];
-    u32x2* Tl = (u32x2*)smem_raw;                // [CT][NT][64 lanes]
-    u32x2* xq = Tl + CT * NT * 64;               // codes of the rows, nseg * 1024 bytes each
+    u32x2* Tl = (u32x2*)smem_raw;
+    u32x2* xq = Tl + Front::T_BYTES / 8;         // codes of the rows, nseg * 1024 bytes each
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int l16 = lane & 15, g = lane >> 4;
-    const int tile = HV == 2 ? wave >> 1 : wave, half = HV == 2 ? wave & 1 : 0;      // 16 rows of hadK; its 64 columns
-    const int r = tile * 16 + l16, Kb = K * (M_ / 2), nseg = (Kb + 1023) >> 10;
-    const bool works = tile * 16 < K, dval = r < K;
+    if constexpr (LOG2M == 7) signs = 0;
+    const int Kb = K * (Front::M_ / 2), nseg = (Kb + 1023) >> 10;
+    u32x2* Hl = xq + MB * nseg * 128;            // the table
 
     // ---- requests: the row, the table's rows of this wave, then weights
-    u32x4 xr[S1K];
-    auto request = [&](int row) {
-#pragma unroll
-        for (int c = 0; c < S1K; ++c) xr[c] = *((const u32x4*)x + (int64_t)row * (K * (M_ / 8)) + (dval ? r * (M_ / 8) + 4 * c + g : 0));
-    };
-    request(0);
-    u32x2 hk[KS2][2];                            // hadK[r][32 ks + 16 hh + 4 g ..+ 3], or sign words (see hadamard_m64r_kernel)
-    if (signs) {
-#pragma unroll
-        for (int ks = 0; ks < KS2; ++ks) hk[ks][0][0] = ((const u32*)hadK)[dval ? r * KS2 + ks : 0];
-    } else {
-#pragma unroll
-        for (int ks = 0; ks < KS2; ++ks)
-#pragma unroll
-            for (int hh = 0; hh < 2; ++hh) {
-                const int hc = ks * 32 + hh * 16 + g * 4;
-                hk[ks][hh] = ((const u32x2*)hadK)[dval && hc < K ? (r * K + hc) >> 2 : 0];
-            }
-    }
+    Front front;
+    front.begin(K, wave, lane);
+    front.request(x, 0);
+    front.request_table(hadK, signs);
     RowPairStream<MB, 1> ws;
     ws.init_dealt(B, sB, bias, N, Kb, wave, lane);
     using Seg = typename RowPairStream<MB, 1>::Seg;
     Seg ring[RD];
-
-    // Sylvester fragments: base tile of the parity of the column tile, and its negative
-    f16x8 sb[2][2];
-#pragma unroll
-    for (int o = 0; o < 2; ++o)
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const bool neg = ((__builtin_popcount(((g & 1) * 8 + j) & l16) + ((g >> 1) & o)) & 1) != 0;
-            sb[o][0][j] = neg ? (f16)-1.0f : (f16)1.0f;
-            sb[o][1][j] = neg ? (f16)1.0f : (f16)-1.0f;
-        }
-    // T of tiles beyond K and the codes past the rows' ends: zeros
-    for (int i = tid; i < CT * NT * 32; i += 1024) ((u32x4*)Tl)[i] = u32x4{0, 0, 0, 0};
-    for (int i = tid; i < MB * nseg * 128; i += 1024) xq[i] = u32x2{0, 0};
+    front.sylvester();
+    for (int i = tid; i < MB * nseg * 128; i += 1024) xq[i] = u32x2{0, 0};       // the codes past the rows' ends stay zeros
     __syncthreads();
     ws.fetch(ring[0]);                           // (behind every wave's requests for the row)
     f16 sh_one = (f16)0;
-    f16x8 hf[KS2];
 #pragma unroll
     for (int row = 0; row < MB; ++row) {
-        // ---- stage 1: T = X . H_m for this wave's 16 rows and four column tiles, rounded to fp16 with the scale
-        if (works) {
-            u32x4 af[S1K];
-#pragma unroll
-            for (int c = 0; c < S1K; ++c) af[c] = dval ? xr[c] : u32x4{0, 0, 0, 0};
-#pragma unroll
-            for (int cc = 0; cc < CTW; ++cc) {
-                // the column tile is half * 4 + cc: its bits above the lowest decide the signs of the contraction's steps
-                f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                for (int c = 0; c < S1K; ++c) {
-                    const f16x8 a = __builtin_bit_cast(f16x8, af[c]);
-                    if (HV == 2 && (c & 2)) {    // (popcount(c & (ct >> 1)) with ct >> 1 = 2 half + cc / 2)
-                        const bool odd = ((__builtin_popcount(c & (cc >> 1)) + half) & 1) != 0;
-                        acc = odd ? __builtin_amdgcn_mfma_f32_16x16x32_f16(a, sb[cc & 1][1], acc, 0, 0, 0)
-                                  : __builtin_amdgcn_mfma_f32_16x16x32_f16(a, sb[cc & 1][0], acc, 0, 0, 0);
-                    } else {
-                        acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, sb[cc & 1][__builtin_popcount(c & (cc >> 1)) & 1], acc, 0, 0, 0);
-                    }
-                }
-                Tl[((half * CTW + cc) * NT + tile) * 64 + lane] = u32x2{narrow_f16x2(acc[0] * scale, acc[1] * scale),
-                                                                        narrow_f16x2(acc[2] * scale, acc[3] * scale)};
-            }
-        }
-        if (row == 0) {                          // the table's fragments, under the other waves' stage 1
-#pragma unroll
-            for (int ks = 0; ks < KS2; ++ks) {
-                u32x4 fr;
-#pragma unroll
-                for (int hh = 0; hh < 2; ++hh) {
-                    const bool ok = dval && ks * 32 + hh * 16 + g * 4 < K;
-                    u32 p0 = hk[ks][hh][0], p1 = hk[ks][hh][1];
-                    if (signs) {
-                        const u32 nib = (hk[ks][0][0] >> (hh * 16 + g * 4)) & 15u;
-                        p0 = 0x3C003C00u | ((nib & 1u) << 15) | ((nib & 2u) << 30);
-                        p1 = 0x3C003C00u | ((nib & 4u) << 13) | ((nib & 8u) << 28);
-                    }
-                    fr[hh * 2] = ok ? p0 : 0u;
-                    fr[hh * 2 + 1] = ok ? p1 : 0u;
-                }
-                hf[ks] = __builtin_bit_cast(f16x8, fr);
-            }
-        }
-        if (row + 1 < MB) request(row + 1);
+        front.stage1(Tl, scale);
+        if (row == 0) front.table(Hl, signs);
+        if (row + 1 < MB) front.request(x, row + 1);
         if constexpr (MB == 1) {
             ws.fetch(ring[1]);
             ws.fetch(ring[2]);
@@ -489,37 +421,8 @@ __global__ __launch_bounds__(1024) void mm_gemv_kernel(const f16* __restrict__ x
             ws.fetch(ring[1 + 2 * row]);
         }
         __syncthreads();
-        // ---- stage 2: Y^T = T^T . hadK^T; the row's maximum; the codes
-        u32x2 yv[CTW];
-        float mxf = 0.f, probe = 0.f;
-#pragma unroll
-        for (int cc = 0; cc < CTW; ++cc) {
-            f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-            if (works) {
-#pragma unroll
-                for (int ks = 0; ks < KS2; ++ks) {
-                    const u32x2* const t = Tl + ((half * CTW + cc) * NT + 2 * ks) * 64 + lane;
-                    const u32x2 p0 = t[0], p1 = t[64];
-                    acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, u32x4{p0[0], p0[1], p1[0], p1[1]}), hf[ks], acc,
-                                                                 0, 0, 0);
-                }
-            }
-            if (cc == 0) probe = acc[0];
-            yv[cc] = u32x2{cvt_f16x2(acc[0], acc[1]), cvt_f16x2(acc[2], acc[3])};
-            mxf = __builtin_fmaxf(__builtin_fmaxf(mxf, __builtin_fabsf(acc[0])), __builtin_fabsf(acc[1]));
-            mxf = __builtin_fmaxf(__builtin_fmaxf(mxf, __builtin_fabsf(acc[2])), __builtin_fabsf(acc[3]));
-        }
-        u32 mx = f16_bits((f16)mxf);
-        if (__builtin_amdgcn_ballot_w64(mx >= 0x7c00u || probe != probe) != 0) {         // something non-finite: the exact form
-            u16x2 m2 = {0, 0};
-#pragma unroll
-            for (int cc = 0; cc < CTW; ++cc) {
-                m2 = __builtin_elementwise_max(m2, __builtin_bit_cast(u16x2, dval ? yv[cc][0] & 0x7fff7fffu : 0u));
-                m2 = __builtin_elementwise_max(m2, __builtin_bit_cast(u16x2, dval ? yv[cc][1] & 0x7fff7fffu : 0u));
-            }
-            mx = m2[0] > m2[1] ? m2[0] : m2[1];
-        }
-        mx = wave_max_u32_dpp(mx);
+        if (row == 0) front.table_read(Hl, signs);
+        u32 mx = front.stage2(Tl);
         if (lane == 0) red[wave] = mx;
         if constexpr (MB == 1) {
             ws.fetch(ring[3]);
@@ -531,37 +434,10 @@ __global__ __launch_bounds__(1024) void mm_gemv_kernel(const f16* __restrict__ x
 #pragma unroll
         for (int w = 0; w < NW; ++w) mx = mx > red[w] ? mx : red[w];
         const f16 sh = quantizer_scale(f16_from_bits((unsigned short)mx), clip);
-        const float sp = (float)sh;
         if (MB > 1 && tid == 0) sc[row] = sh;
         sh_one = sh;
-        u32 c01, c23;
-        auto codes_from = [&](auto pair) {
-            u32 b0[4], b1[4];
-#pragma unroll
-            for (int w = 0; w < 4; ++w) {
-                b0[w] = pair(yv[w >> 1][w & 1]);
-                b1[w] = pair(yv[2 + (w >> 1)][w & 1]);
-            }
-            c01 = pack_nibbles8(b0);
-            c23 = pack_nibbles8(b1);
-        };
-        if (fast_quant_ok(mx, sp)) {
-            const FastRecip fq = make_fast_recip(sp);
-            if (clamp_cannot_act(clip, sp)) codes_from([&](u32 w) { return sym_pair_fast<false>(w, fq); });
-            else codes_from([&](u32 w) { return sym_pair_fast<true>(w, fq); });
-        } else {
-            const bool fs_ok = scale_fast_ok(sp);
-            const float rs = fs_ok ? 1.0f / sp : 0.0f;
-            c01 = sym_codes8(u32x4{yv[0][0], yv[0][1], yv[1][0], yv[1][1]}, sp, rs, fs_ok);
-            c23 = sym_codes8(u32x4{yv[2][0], yv[2][1], yv[3][0], yv[3][1]}, sp, rs, fs_ok);
-        }
-        const auto s1 = __builtin_amdgcn_permlane32_swap(c01, c23, false, false);
-        const u32 ev = __builtin_amdgcn_perm(s1[1], s1[0], 0x05040100u);
-        const u32 od = __builtin_amdgcn_perm(s1[1], s1[0], 0x07060302u);
-        const auto s2 = __builtin_amdgcn_permlane16_swap(ev, od, false, false);
-        if (dval)
-            xq[row * (nseg * 128) + r * CT + half * CTW + g] =
-                u32x2{__builtin_amdgcn_perm(s2[1], s2[0], 0x05040100u), __builtin_amdgcn_perm(s2[1], s2[0], 0x07060302u)};
+        const u32x2 c = front.codes(mx, (float)sh, clip);
+        if (front.dval) xq[row * (nseg * 128) + front.place()] = c;
         // (the next row's first stage writes T behind every wave's reads of it, the barrier above; the maxima are next written
         // behind the next row's first barrier)
     }
@@ -748,7 +624,8 @@ __attribute__((visibility("hidden"))) int qr_internal_token_mm_linear(const void
     if (((uintptr_t)x & 15) || ((uintptr_t)W & 15) || ((uintptr_t)hadK & (signs ? 3 : 7))) return QR_E_UNSUPPORTED;
     const int cus = qr_device().cus;
     const unsigned grid = (unsigned)((N + 15) / 16 < cus ? (N + 15) / 16 : cus);
-    const size_t lds = (size_t)(m64 ? 4 : 8) * (2 * ks2) * 64 * 8 + (size_t)M * (((size_t)n / 2 + 1023) / 1024) * 1024;
+    const size_t lds = (size_t)(m64 ? 4 : 8) * (2 * ks2) * 64 * 8 + (size_t)M * (((size_t)n / 2 + 1023) / 1024) * 1024 +
+                       (signs ? 0 : (size_t)K * K * 2);
     using Kern = void (*)(const f16*, int, const void*, int, float, float, const uint8_t*, const f16*, const f16*, int, f16*);
     static const Kern table[5][2] = {{mm_gemv_kernel<6, 4, 1>, mm_gemv_kernel<6, 4, 2>},
                                      {mm_gemv_kernel<6, 5, 1>, mm_gemv_kernel<6, 5, 2>},

@@ -11,6 +11,7 @@
 //            written back in place.
 //   phase 4  LDS -> global: round to the I/O type; when fused, row abs-max -> scale -> int4 codes.
 #include "qr_common.h"
+#include "qr_mm_row.h"
 
 namespace {
 
@@ -1750,11 +1751,75 @@ bool mm_applies(int n, int K) {
     return m == 64 || m == 128;
 }
 
+// ---- m = 64 or 128 behind a table, quantiser fused, few rows: one row per workgroup, all its waves on that row ----
+// hadamard_m64r_kernel and hadamard_m64q_kernel keep four waves per row, each with the table's fragments of three 16-row tiles, and walk
+// many rows; of a few rows a CU has one or two, and its launch is the chain of those tiles.  Here each wave has one tile and 64 columns.
+// What bounds it: launch, the row's way into one CU, two short stages.  Launches back to back (four-wave kernels -> here): 48 rows of
+// 11008 values 5.9 -> 4.8 us, 8960 5.4 -> 4.5, 6912 4.7 -> 4.0, 13824 7.1 -> 5.9, 5120 4.4 -> 3.8.
+template <int LOG2M, int KS2>
+__global__ __launch_bounds__(128 * KS2 * (LOG2M - 5)) void hadamard_row_quant_kernel(
+    const f16* __restrict__ x, int K, const void* __restrict__ hadK, int signs, float scale, float clip, u32x2* __restrict__ q,
+    f16* __restrict__ scales) {
+    constexpr int THREADS = 128 * KS2 * (LOG2M - 5);
+    using Front = MmRow<LOG2M, KS2, THREADS>;
+    static_assert(THREADS == 64 * Front::WAVES, "a wave per tile and 64 columns");
+    extern __shared__ f32x4 smem_raw[];
+    u32x2* Tl = (u32x2*)smem_raw;
+    u32x2* Hl = Tl + Front::T_BYTES / 8;         // the table, unless it comes as sign words
+    __shared__ u32 red[Front::WAVES];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t row = blockIdx.x;
+    if constexpr (LOG2M == 7) signs = 0;
+    Front front;
+    front.begin(K, wave, lane);
+    front.request(x, row);
+    front.request_table(hadK, signs);
+    front.sylvester();
+    front.stage1(Tl, scale);
+    front.table(Hl, signs);
+    __syncthreads();
+    front.table_read(Hl, signs);
+    u32 mx = front.stage2(Tl);
+    if (lane == 0) red[wave] = mx;
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < Front::WAVES; ++w) mx = mx > red[w] ? mx : red[w];
+    const f16 sh = quantizer_scale(f16_from_bits((unsigned short)mx), clip);
+    if (threadIdx.x == 0) scales[row] = sh;
+    const u32x2 c = front.codes(mx, (float)sh, clip);
+    if (front.dval) q[row * (K * (Front::M_ / 16)) + front.place()] = c;
+}
+
+template <int LOG2M, int KS2>
+int launch_row_quant(const void* x, int64_t rows, int K, const void* hadK, int signs, float scale, float clip, void* q, void* scales,
+                     hipStream_t st) {
+    using Front = MmRow<LOG2M, KS2, 128 * KS2 * (LOG2M - 5)>;
+    const size_t lds = (size_t)Front::T_BYTES + (signs ? 0 : (size_t)K * K * 2);
+    const auto kern = hadamard_row_quant_kernel<LOG2M, KS2>;
+    if (lds > 48 * 1024) {
+        const hipError_t e = qr_allow_dynamic_lds((const void*)kern, lds);
+        if (e != hipSuccess) return (int)e;
+    }
+    kern<<<dim3((unsigned)rows), dim3(64 * Front::WAVES), lds, st>>>((const f16*)x, K, hadK, signs, scale, clip, (u32x2*)q, (f16*)scales);
+    return qr_launch_status();
+}
+
 template <bool MODE32, bool QUANT>
 int launch_hadamard_mm(const void* x, void* y, int64_t rows, int n, int K, const void* hadK, float scale, float clip,
                        void* q, void* scales, hipStream_t st, int signs = 0) {
     const int m = n / K;
     const int KS2 = ((K + 31) & ~31) >> 5;
+    // Up to two rows per CU: one workgroup per row, as many waves as it has tiles.  At 512 rows on 256 CUs it is still ahead (11008 values
+    // 8.4 -> 7.6 us, 13824 10.2 -> 9.3, 5120 5.6 -> 5.3); with a third row the kernels that keep the table's fragments win
+    // (700 rows of 11008: 9.1 us against 9.8, 13824: 11.8 against 12.7).
+    if (!MODE32 && QUANT && y == nullptr && hadK != nullptr && rows <= 2 * (int64_t)qr_device().cus && ((uintptr_t)x & 15) == 0 &&
+        ((uintptr_t)hadK & (signs ? 3 : 7)) == 0) {
+        if (m == 64 && KS2 == 4) return launch_row_quant<6, 4>(x, rows, K, hadK, signs, scale, clip, q, scales, st);
+        if (m == 64 && KS2 == 5) return launch_row_quant<6, 5>(x, rows, K, hadK, signs, scale, clip, q, scales, st);
+        if (m == 64 && KS2 == 6) return launch_row_quant<6, 6>(x, rows, K, hadK, signs, scale, clip, q, scales, st);
+        if (m == 128 && KS2 == 2) return launch_row_quant<7, 2>(x, rows, K, hadK, signs, scale, clip, q, scales, st);
+        if (m == 128 && KS2 == 4) return launch_row_quant<7, 4>(x, rows, K, hadK, signs, scale, clip, q, scales, st);
+    }
     if (m == 128 && KS2 >= 2 && KS2 != 3 && !MODE32 && QUANT && y == nullptr && hadK != nullptr && ((uintptr_t)x & 15) == 0) {
         // m = 128 behind one of the reference's tables of order 36 and more (Llama-2-13B: 5120 = 40 x 128, 13824 =
         // 108 x 128): the lean fused kernel with eight column tiles.  Orders 140 .. 172 need more registers than two
