@@ -196,12 +196,12 @@ __global__ __launch_bounds__(1024) void bm_gemv_kernel(const f16* __restrict__ x
     // ---- fragments: Sylvester factors of both stages -----------------------------------------------------------
     f16x8 ha[2], hb[2];
 #pragma unroll
-    for (int t = 0; t < 8; ++t) {
-#pragma unroll
-        for (int cth = 0; cth < 2; ++cth) ha[cth][t] = (__builtin_popcount((g * 8 + t) & (cth * 16 + l16)) & 1) ? (f16)-1.0f : (f16)1.0f;
-        const int b = 16 * (t >> 2) + 4 * g + (t & 3);
-#pragma unroll
-        for (int bt = 0; bt < 2; ++bt) hb[bt][t] = (__builtin_popcount(b & (bt * 16 + l16)) & 1) ? (f16)-1.0f : (f16)1.0f;
+    for (int t = 0; t < 2; ++t) {
+        // ha[t][j]: row 16 t + l16, contraction 8 g + j; hb[t][j]: row 16 t + l16, contraction 16 (j / 4) + 4 g + j % 4
+        ha[t] = sylvester8(l16, (g & (l16 >> 3)) ^ ((g >> 1) & t));
+        const u32x2 w = __builtin_bit_cast(u32x2, sylvester4(l16, (g & (l16 >> 2)) ^ ((g >> 1) & (l16 >> 3))));
+        const u32 flip = t ? 0x80008000u : 0u;
+        hb[t] = __builtin_bit_cast(f16x8, u32x4{w[0], w[1], w[0] ^ flip, w[1] ^ flip});
     }
     for (int i = tid; i < 4 * CT * TS; i += 1024) Tl[i] = u32x4{0, 0, 0, 0};
     __syncthreads();

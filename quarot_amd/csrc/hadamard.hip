@@ -575,8 +575,7 @@ __global__ __launch_bounds__(HT) void hadamard_mm_kernel(const f16* __restrict__
                 if (hr < K && hc < K) {
                     if (hadK == nullptr) {
                         // power-of-two row: the outer factor is the Sylvester matrix of order K itself
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) v[e] = (__builtin_popcount(hr & (hc + e)) & 1) ? (f16)-1.0f : (f16)1.0f;
+                        v = sylvester4(hr, __builtin_popcount(hr & hc));
                     } else if (MODE32) {
                         const f32x4 w = *(const f32x4*)((const float*)hadK + hr * K + hc);
                         v = f16x4{(f16)w[0], (f16)w[1], (f16)w[2], (f16)w[3]};
@@ -593,13 +592,10 @@ __global__ __launch_bounds__(HT) void hadamard_mm_kernel(const f16* __restrict__
 #pragma unroll
     for (int c = 0; c < NCT; ++c)
 #pragma unroll
-        for (int ks = 0; ks < KS1; ++ks)
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const int rp = (wave + 4 * c) * 16 + l16;
-                const int r = ks * 32 + g * 8 + j;
-                b1[c][ks][j] = (__builtin_popcount(r & rp) & 1) ? (f16)-1.0f : (f16)1.0f;
-            }
+        for (int ks = 0; ks < KS1; ++ks) {
+            const int rp = (wave + 4 * c) * 16 + l16, r = ks * 32 + g * 8;
+            b1[c][ks] = sylvester8(rp, __builtin_popcount(r & rp));
+        }
 
     // stage-1 A-fragments for the tile pair s2 of a row: [2 tiles][KS1] 16-byte loads
     auto load_pair = [&](const f16* xr, int s2, u32x4(&dst)[2][KS1]) {
@@ -831,8 +827,7 @@ __global__ __launch_bounds__(HT, (KS2 <= 2 ? 4 : 2)) void hadamard_m64_kernel(
                 f16x4 v = {(f16)0, (f16)0, (f16)0, (f16)0};
                 if (hr < K && hc < K) {
                     if (hadK == nullptr) {
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) v[e] = (__builtin_popcount(hr & (hc + e)) & 1) ? (f16)-1.0f : (f16)1.0f;
+                        v = sylvester4(hr, __builtin_popcount(hr & hc));
                     } else if (MODE32) {
                         const f32x4 w = *(const f32x4*)((const float*)hadK + hr * K + hc);
                         v = f16x4{(f16)w[0], (f16)w[1], (f16)w[2], (f16)w[3]};
@@ -851,13 +846,10 @@ __global__ __launch_bounds__(HT, (KS2 <= 2 ? 4 : 2)) void hadamard_m64_kernel(
     // (16 registers) stand for all eight fragments; which one an MFMA takes is known at compile time.
     f16x8 sb[2][2];                                          // [ct & 1][negated]
 #pragma unroll
-    for (int o = 0; o < 2; ++o)
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const bool neg = ((__builtin_popcount(((g & 1) * 8 + j) & l16) + ((g >> 1) & o)) & 1) != 0;
-            sb[o][0][j] = neg ? (f16)-1.0f : (f16)1.0f;
-            sb[o][1][j] = neg ? (f16)1.0f : (f16)-1.0f;
-        }
+    for (int o = 0; o < 2; ++o) {
+        sb[o][0] = sylvester8(l16, (g & (l16 >> 3)) ^ ((g >> 1) & o));
+        sb[o][1] = negated(sb[o][0]);
+    }
 
     // staging: load c of a tile covers its rows 8 c .. 8 c + 7, lane -> (row 8 c + lane / 8, piece
     // lane % 8): 1 KB of consecutive addresses per instruction.  Pieces are XOR-keyed by the row so
@@ -1100,13 +1092,10 @@ __global__ __launch_bounds__(HT, (LOG2M == 7 && KS2 >= 5 ? 1 : 2)) void hadamard
     }
     f16x8 sb[2][2];                                          // Sylvester fragments, as in hadamard_m64_kernel
 #pragma unroll
-    for (int o = 0; o < 2; ++o)
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const bool neg = ((__builtin_popcount(((g & 1) * 8 + j) & l16) + ((g >> 1) & o)) & 1) != 0;
-            sb[o][0][j] = neg ? (f16)-1.0f : (f16)1.0f;
-            sb[o][1][j] = neg ? (f16)1.0f : (f16)-1.0f;
-        }
+    for (int o = 0; o < 2; ++o) {
+        sb[o][0] = sylvester8(l16, (g & (l16 >> 3)) ^ ((g >> 1) & o));
+        sb[o][1] = negated(sb[o][0]);
+    }
     // fragment (tile i, k step c) of a row: 16-byte piece 4 c + g of row (wave + 4 i) 16 + l16 of X[K][M_]
     int goff[TPW][S1K];
     bool dval[TPW];
@@ -1385,12 +1374,7 @@ __device__ __forceinline__ void hadamard_m64r_rows(const f16* __restrict__ x, in
     // (sign bits of its fp16 pairs flipped: the products are the same numbers), which saves eight registers
     f16x8 sb[2];
 #pragma unroll
-    for (int o = 0; o < 2; ++o)
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const bool neg = ((__builtin_popcount(((g & 1) * 8 + j) & l16) + ((g >> 1) & o)) & 1) != 0;
-            sb[o][j] = neg ? (f16)-1.0f : (f16)1.0f;
-        }
+    for (int o = 0; o < 2; ++o) sb[o] = sylvester8(l16, (g & (l16 >> 3)) ^ ((g >> 1) & o));
     // dval: this lane's row of tile i exists
     bool dval[TPW];
     int goff[TPW];
@@ -1428,16 +1412,10 @@ __device__ __forceinline__ void hadamard_m64r_rows(const f16* __restrict__ x, in
 #pragma unroll
             for (int ks = 0; ks < KS2; ++ks) {
                 const u32 w = sw[rok ? hr * KS2 + ks : 0];
-                u32x4 fr;
-#pragma unroll
-                for (int hh = 0; hh < 2; ++hh) {
-                    const u32 nib = (w >> (hh * 16 + g * 4)) & 15u;
-                    const bool ok = rok && ks * 32 + hh * 16 + g * 4 < K;
-                    const u32 p0 = 0x3C003C00u | ((nib & 1u) << 15) | ((nib & 2u) << 30);
-                    const u32 p1 = 0x3C003C00u | ((nib & 4u) << 13) | ((nib & 8u) << 28);
-                    fr[hh * 2] = ok ? p0 : 0u;
-                    fr[hh * 2 + 1] = ok ? p1 : 0u;
-                }
+                // (columns beyond K meet zeros of T; rows beyond K, in the last tile only, are zero fragments)
+                const u32x2 f0 = sign_halves(w >> (4 * g)), f1 = sign_halves(w >> (16 + 4 * g));
+                u32x4 fr = {f0[0], f0[1], f1[0], f1[1]};
+                if (i == TPW - 1) fr = rok ? fr : u32x4{0, 0, 0, 0};
                 hf[i][ks] = __builtin_bit_cast(f16x8, fr);
             }
         }
@@ -1453,9 +1431,9 @@ __device__ __forceinline__ void hadamard_m64r_rows(const f16* __restrict__ x, in
 #pragma unroll
                 for (int hh = 0; hh < 2; ++hh) {
                     const int hc = ks * 32 + hh * 16 + g * 4;
+                    const f16x4 v = sylvester4(hr, __builtin_popcount(hr & hc));
 #pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        hf[i][ks][hh * 4 + e] = (hr < K && hc < K) ? ((__builtin_popcount(hr & (hc + e)) & 1) ? (f16)-1.0f : (f16)1.0f) : (f16)0.0f;
+                    for (int e = 0; e < 4; ++e) hf[i][ks][hh * 4 + e] = (hr < K && hc < K) ? v[e] : (f16)0.0f;
                 }
         }
         u32x4* stage = (u32x4*)smem_raw;
@@ -2018,12 +1996,12 @@ __global__ __launch_bounds__(1024) void hadamard_bm_kernel(const f16* __restrict
     f16x8 ha[2], hb[2];
     if (CPL == 2 && !MODE32) {
 #pragma unroll
-        for (int t = 0; t < 8; ++t) {
-#pragma unroll
-            for (int cth = 0; cth < 2; ++cth) ha[cth][t] = (__builtin_popcount((g * 8 + t) & (cth * 16 + l16)) & 1) ? (f16)-1.0f : (f16)1.0f;
-            const int b = 16 * (t >> 2) + 4 * g + (t & 3);
-#pragma unroll
-            for (int bt = 0; bt < 2; ++bt) hb[bt][t] = (__builtin_popcount(b & (bt * 16 + l16)) & 1) ? (f16)-1.0f : (f16)1.0f;
+        for (int t = 0; t < 2; ++t) {
+            // ha[t][j]: row 16 t + l16, contraction 8 g + j; hb[t][j]: row 16 t + l16, contraction 16 (j / 4) + 4 g + j % 4
+            ha[t] = sylvester8(l16, (g & (l16 >> 3)) ^ ((g >> 1) & t));
+            const u32x2 w = __builtin_bit_cast(u32x2, sylvester4(l16, (g & (l16 >> 2)) ^ ((g >> 1) & (l16 >> 3))));
+            const u32 flip = t ? 0x80008000u : 0u;
+            hb[t] = __builtin_bit_cast(f16x8, u32x4{w[0], w[1], w[0] ^ flip, w[1] ^ flip});
         }
     }
     // hadK fragments (second MFMA operand): column k' = rt*16 + l16, contraction k = ks*32 + g*8 + j

@@ -265,13 +265,10 @@ __global__ __launch_bounds__(64 * KM_WAVES, 2) void kv_had128_kernel(const u32x4
     // base tiles of H_128 for ks even / odd: row j = v (jt = 0), inputs k = 16 (ks & 1) + 8 h + e
     f16x8 hb[2], hn[2];
 #pragma unroll
-    for (int o = 0; o < 2; ++o)
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            const bool neg = (__builtin_popcount(v & (16 * o + 8 * h + e)) & 1) != 0;
-            hb[o][e] = neg ? (f16)-1.0f : (f16)1.0f;
-            hn[o][e] = neg ? (f16)1.0f : (f16)-1.0f;
-        }
+    for (int o = 0; o < 2; ++o) {
+        hb[o] = sylvester8(v, __builtin_popcount(v & (16 * o + 8 * h)));
+        hn[o] = negated(hb[o]);
+    }
 
     // PAGED: keys and values of an append in ONE launch.  A part that is quantised WITHOUT the transform -- the values,
     // or keys when the caller wants none -- skips the matrix stage (its bit in plain_mask).

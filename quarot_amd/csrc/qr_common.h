@@ -157,6 +157,24 @@ __device__ __forceinline__ u32 cvt_f16x2(float a, float b) {
     return __builtin_bit_cast(u32, __builtin_convertvector(v, f16x2));
 }
 
+// Pieces of a Sylvester matrix as fp16 +-1: element j is (-1)^(parity(j & l) + odd), j = 0 .. 7 (0 .. 3): bit 0 of l decides the halves
+// of a dword, bits 1 and 2 which dwords are negated, and `odd` (its lowest bit) is the parity of the index bits above.  Every kernel makes its
+// fragments on the way to its first row; a bit count, a compare and a select per element took longer than that row's loads.
+__device__ __forceinline__ f16x4 sylvester4(u32 l, u32 odd) {
+    const u32 w = (0x3C003C00u | (l << 31)) ^ ((odd & 1u) ? 0x80008000u : 0u);
+    return __builtin_bit_cast(f16x4, u32x2{w, w ^ ((l & 2u) ? 0x80008000u : 0u)});
+}
+__device__ __forceinline__ f16x8 sylvester8(u32 l, u32 odd) {
+    const u32x2 w = __builtin_bit_cast(u32x2, sylvester4(l, odd));
+    const u32 m = (l & 4u) ? 0x80008000u : 0u;
+    return __builtin_bit_cast(f16x8, u32x4{w[0], w[1], w[0] ^ m, w[1] ^ m});
+}
+__device__ __forceinline__ f16x8 negated(f16x8 v) { return __builtin_bit_cast(f16x8, __builtin_bit_cast(u32x4, v) ^ 0x80008000u); }
+// four entries of +-1 from four bits (1: -1)
+__device__ __forceinline__ u32x2 sign_halves(u32 bits) {
+    return u32x2{0x3C003C00u | ((bits & 1u) << 15) | ((bits & 2u) << 30), 0x3C003C00u | ((bits & 4u) << 13) | ((bits & 8u) << 28)};
+}
+
 // An 8-byte store that is written through the L2 to memory at once (device scope) instead of staying dirty in the
 // L2 until the kernel ends; the line remains in the L2 for readers on the same XCD.
 __device__ __forceinline__ void store_through(u32x2* dst, u32x2 v) {

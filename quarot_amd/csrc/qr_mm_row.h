@@ -46,19 +46,11 @@ struct MmRow {
             }
         }
     }
-    // sb[o][.][j] = (-1)^parity((8 (g & 1) + j) & l16) (-1)^(o (g >> 1)): bit 0 of j decides the halves of a dword, bits 1 and 2 which
-    // dwords are negated (instead of counting bits for every element: with the sign words spread straight
-    // from shifts and T read 16 bytes at a time, 48 rows of 11008 values 5.6 -> 4.8 us)
     __device__ __forceinline__ void sylvester() {
-        constexpr u32 both = 0x80008000u;
-        const u32 first = (0x3C003C00u | ((u32)(l16 & 1) << 31)) ^ ((g & (l16 >> 3) & 1) ? both : 0u);
-        const u32 m1 = (l16 & 2) ? both : 0u, m2 = (l16 & 4) ? both : 0u, mo = (g & 2) ? both : 0u;
-        const u32x4 w = {first, first ^ m1, first ^ m2, first ^ m1 ^ m2};
 #pragma unroll
         for (int o = 0; o < 2; ++o) {
-            const u32x4 v = o ? u32x4{w[0] ^ mo, w[1] ^ mo, w[2] ^ mo, w[3] ^ mo} : w;
-            sb[o][0] = __builtin_bit_cast(f16x8, v);
-            sb[o][1] = __builtin_bit_cast(f16x8, u32x4{v[0] ^ both, v[1] ^ both, v[2] ^ both, v[3] ^ both});
+            sb[o][0] = sylvester8(l16, (g & (l16 >> 3)) ^ ((g >> 1) & o));
+            sb[o][1] = negated(sb[o][0]);
         }
     }
     // T = X . H_m for this wave's 16 rows and four column tiles, rounded to fp16 with the scale; tiles beyond K: zeros.
@@ -98,13 +90,8 @@ struct MmRow {
 #pragma unroll
             for (int ks = 0; ks < KS2; ++ks) {
                 const u32 w = sw[ks] >> (4 * g);                          // bits 0 .. 3 and 16 .. 19 are this lane's
-                u32x4 fr;
-#pragma unroll
-                for (int d = 0; d < 4; ++d) {
-                    const u32 v = w >> ((d >> 1) * 16 + (d & 1) * 2);
-                    fr[d] = 0x3C003C00u | ((v & 1u) << 15) | ((v & 2u) << 30);
-                }
-                hf[ks] = __builtin_bit_cast(f16x8, fr);
+                const u32x2 f0 = sign_halves(w), f1 = sign_halves(w >> 16);
+                hf[ks] = __builtin_bit_cast(f16x8, u32x4{f0[0], f0[1], f1[0], f1[1]});
             }
         } else {
 #pragma unroll
