@@ -1366,7 +1366,10 @@ __device__ __forceinline__ void hadamard_m64r_rows(const f16* __restrict__ x, in
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l16 = lane & 15, g = lane >> 4;
     const int nchunks = n >> 3;
-    u32x2* Tl = (u32x2*)smem_raw;                                      // [CT][NT][64 lanes]
+    // T: [CT][NT][64 lanes]; with two planes [CT][KS2][64 lanes][2 tiles], a contraction step's fragment read as 16 bytes (2048 rows of
+    // 8192 values 15.0 -> 14.2 us; with one plane the halves of the stores that then share banks cost more: 11008 17.3 -> 17.6)
+    u32x2* Tl = (u32x2*)smem_raw;
+    auto t_at = [&](int ct, int t) { return MODE32 ? ((ct * KS2 + (t >> 1)) * 64 + lane) * 2 + (t & 1) : (ct * NT + t) * 64 + lane; };
     u32x2* Tlo = Tl + CT * NT * 64;                                    // lo plane (fp32-precision mode)
 
     // Sylvester fragments of hadamard_m64_kernel: one base per parity of the column tile; where that kernel takes a
@@ -1560,12 +1563,12 @@ __device__ __forceinline__ void hadamard_m64r_rows(const f16* __restrict__ x, in
                             const f16x2 h = as_f16x2(hi[e]);
                             lo[e] = narrow_f16x2(tv[2 * e] - (float)h[0], tv[2 * e + 1] - (float)h[1]);
                         }
-                        Tlo[(ct * NT + t) * 64 + lane] = lo;
+                        Tlo[t_at(ct, t)] = lo;
                     } else {
                         hi[0] = narrow_f16x2(acc[0] * scale, acc[1] * scale);
                         hi[1] = narrow_f16x2(acc[2] * scale, acc[3] * scale);
                     }
-                    Tl[(ct * NT + t) * 64 + lane] = hi;
+                    Tl[t_at(ct, t)] = hi;
                 }
             }
         }
@@ -1583,8 +1586,12 @@ __device__ __forceinline__ void hadamard_m64r_rows(const f16* __restrict__ x, in
             // fragments of T one contraction step ahead of their use (8 registers; a whole column tile's set ahead
             // was no faster, and three workgroups per CU, which these registers would allow, spilled and lost 15 %)
             auto frag = [&](const u32x2* plane, int ks) {
-                const u32x2 p0 = plane[(ct * NT + 2 * ks) * 64 + lane], p1 = plane[(ct * NT + 2 * ks + 1) * 64 + lane];
-                return u32x4{p0[0], p0[1], p1[0], p1[1]};
+                if constexpr (MODE32) {
+                    return ((const u32x4*)plane)[(ct * KS2 + ks) * 64 + lane];
+                } else {
+                    const u32x2 p0 = plane[(ct * NT + 2 * ks) * 64 + lane], p1 = plane[(ct * NT + 2 * ks + 1) * 64 + lane];
+                    return u32x4{p0[0], p0[1], p1[0], p1[1]};
+                }
             };
             f32x4 acc[TPW];
 #pragma unroll
