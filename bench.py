@@ -80,7 +80,7 @@ for _t in (1, 8, 32, 64):
 PER_CONFIG = ["c1", "c2_fp32had", "c3", "c4g1", "c4g8", "c4g32", "c4g64", "c4m1", "c4m8", "c4m32", "c4m64", "c5", "c6", "b13v", "b70v", "b13d", "b70d",
               "c2_fp6", "c3_fp6"]
 INT8_MFMA_PEAK_TOPS = 5000.0     # MI355X dense int8, published
-FP6_MFMA_PEAK_TOPS = 10100.0     # MI355X dense fp6, published (the opt-in exact int4 GEMM on 6-bit operands)
+FP6_MFMA_PEAK_TOPS = 10100.0     # MI355X dense fp6, published (exact int4 GEMMs of the prefill tiles, and on 6-bit operands)
 HBM_PEAK_GBS = 8000.0
 
 # Profile summaries that hold the FETCH_SIZE / WRITE_SIZE readings of a workload's dominant kernel
@@ -299,6 +299,12 @@ FRONT_KERNEL = {"had": "hadamard kernel + quantiser (fused)", "had32": "hadamard
                 "rmsnorm": "rmsnorm_quant_rows_kernel", "heads": "heads_hadamard_quant_rows_kernel"}
 
 
+def mfma_peak(kernel):
+    """Published rate of the matrix instruction that a GEMM kernel issues: the tiles of 128 and more rows x 256 columns multiply FP6
+    operands, the smaller ones int8."""
+    return FP6_MFMA_PEAK_TOPS if kernel.startswith(("gemm_sp", "gemm_f6")) else INT8_MFMA_PEAK_TOPS
+
+
 class LinearWorkload:
     """One quantised linear layer: front (quantiser, optionally behind a Hadamard / RMSNorm / heads
     Hadamard) + Linear4bit, operands resident in HBM."""
@@ -425,7 +431,7 @@ class LinearWorkload:
         elif self.decode:
             g = {"bound": "hbm", "achieved": round(self.gemm_bytes() / (gemm_ms * 1e-3) / 1e9, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s"}
         else:
-            g = {"bound": "mfma", "achieved": round(self.ops / (gemm_ms * 1e-3) / 1e12, 1), "peak": INT8_MFMA_PEAK_TOPS, "unit": "TOP/s"}
+            g = {"bound": "mfma", "achieved": round(self.ops / (gemm_ms * 1e-3) / 1e12, 1), "peak": mfma_peak(kern), "unit": "TOP/s"}
         g["frac"] = round(g["achieved"] / g["peak"], 4)
         g["kernel"] = kern + (" (exact int4 GEMM on FP6 operands + dequant epilogue)" if self.fp6 else
                               (" (Hadamard + quantiser" if self.front_kind == "had" else " (quantiser")
@@ -478,7 +484,7 @@ def run_linear(name, dev, steps, warmup, repeats, kernel_reps, on_gpu_data, grap
         extra["fp16_linear_ms"] = round(wl.fp16_linear_ms(max(5, steps // 10)), 5)
     # the whole step against the same roofline as its dominant kernel (algorithmic bytes of the GEMM for decode)
     extra["step_frac"] = round((wl.gemm_bytes() / (ms * 1e-3) / 1e9 / HBM_PEAK_GBS) if wl.decode
-                               else wl.ops / (ms * 1e-3) / 1e12 / (FP6_MFMA_PEAK_TOPS if wl.fp6 else INT8_MFMA_PEAK_TOPS), 4)
+                               else wl.ops / (ms * 1e-3) / 1e12 / groof["peak"], 4)
     res = {"ms": ms, "value": round(wl.ops / (ms * 1e-3) / 1e12, 2), "unit": "TOPS", "timing": sp, "roofline": groof,
            "front": froof, "kernels_ms_sum": round((0.0 if wl.single_launch else front_ms) + gemm_ms + (wl.convert_ms if wl.fp6 else 0.0), 5),
            "staged_reference_api_ms": round(float(np.median(staged)), 5), "workload": wl.describe(), **extra}
@@ -515,7 +521,7 @@ def run_layer(dev, steps, warmup, repeats, kernel_reps, fp6=False):
     sp = spread(timed_loops(step, steps, warmup, repeats))
     ms = sp["median_ms"]
     per, gemm_total, front_total = {}, 0.0, 0.0
-    peak = FP6_MFMA_PEAK_TOPS if fp6 else INT8_MFMA_PEAK_TOPS
+    peak = FP6_MFMA_PEAK_TOPS
     for (name, k, n, kind, _), (x, front, lin) in zip(parts, mods):
         p = front(x)
         f_ms = kernel_ms(lambda: front(x), kernel_reps)
@@ -784,7 +790,7 @@ def main():
         traffic *= 4                                       # the step is four launches; the summary holds their average
     roof["traffic"] = traffic
     roof["traffic_source"] = source
-    if roof.get("bound") == "mfma" and not args.fp6:
+    if roof.get("bound") == "mfma" and roof["peak"] == INT8_MFMA_PEAK_TOPS:
         # what the int8 matrix instruction alone sustains on this box right now (register-only loop, operands with the
         # GEMM's bit statistics, ~60 ms of launches): the part's own ceiling for ANY int8 kernel; `frac` stays against `peak`
         roof["attainable"] = round(mfma_i8_rate(1, launches=12), 1)
@@ -799,7 +805,7 @@ def main():
         "ms_per_step": res["ms"], "ms_per_step_mean": res["timing"]["mean_ms"], "ms_per_step_ci95": res["timing"]["ci95_ms"],
         "higher_is_better": True, "scaling": "weak", "vs_baseline": None,
         "dtype": ("f16 -> u4 (fp32 Hadamard, fp16 quantiser)" if kv_line
-                  else "int4 x int4 -> exact integers in fp32 (FP6 MFMA), fp16 scales" if args.fp6
+                  else "int4 x int4 -> exact integers in fp32 (FP6 MFMA), fp16 scales" if roof.get("peak") == FP6_MFMA_PEAK_TOPS
                   else "int4 x int4 -> int32 (int8 MFMA), fp16 scales"),
         "data": "synthetic",
         "config": {"workload": res["workload"], "launch": res.get("launch", "eager"),
