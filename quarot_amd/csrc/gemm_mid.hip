@@ -182,8 +182,9 @@ __global__ __launch_bounds__(64 * (TM / 64) * (BN / 64) * WK) void gemm_mid_kern
     if (IM == 3 && lines) {
 #pragma unroll
         for (int p = 0; p < 3; ++p) sa3[p] = sA[min(m0 + (tid >> 3) + 32 * p, M - 1)];
-        sb8 = *(const f16x8*)(sB + n0 + (tid & 7) * 8);
-        if (bias) bi8 = *(const f16x8*)(bias + n0 + (tid & 7) * 8);
+        typedef f16x8 any_f16x8 __attribute__((aligned(2)));           // (weight scales and bias may start anywhere: views of larger tensors)
+        sb8 = *(const any_f16x8*)(sB + n0 + (tid & 7) * 8);
+        if (bias) bi8 = *(const any_f16x8*)(bias + n0 + (tid & 7) * 8);
         else
 #pragma unroll
             for (int e = 0; e < 8; ++e) bi8[e] = (f16)-0.0f;

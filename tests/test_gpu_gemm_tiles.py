@@ -72,3 +72,18 @@ def test_gemm_of_large_tiles_bit_exact(m, n, k, kernel, kind):
 @pytest.mark.parametrize("kind", ["random", "extreme"])
 def test_gemm_of_96_row_tiles_bit_exact(m, n, k, kind):
     _compare(m, n, k, kind)
+
+
+@pytest.mark.parametrize("m,n,k", [(333, 4096, 4096), (2048, 4096, 1088)])      # 96 x 64 tiles, 128 or more rows
+@pytest.mark.parametrize("shift", [1, 4])
+def test_scales_and_bias_may_start_anywhere(m, n, k, shift):
+    lib = _lib.lib()
+    gen = torch.Generator(device="cuda").manual_seed(m)
+    a, b = _operand(m, k, "random", gen), _operand(n, k, "random", gen)
+    sa = (torch.rand(m + shift, 1, device="cuda", generator=gen) * 0.1 + 0.01).half()[shift:]
+    sb = (torch.rand(n + shift, device="cuda", generator=gen) * 0.01 + 0.001).half()[shift:]
+    bias = torch.randn(n + shift, device="cuda", generator=gen).half()[shift:]
+    p = lambda t: ctypes.c_void_p(t.data_ptr())
+    y = torch.empty(m, n, dtype=torch.float16, device="cuda")
+    assert lib.qr_linear_i4_f16(p(a), p(sa), p(b), p(sb), p(bias), m, n, k, p(y), None) == 0
+    assert torch.equal(y, (sa * sb) * _sums(a, b).float().half() + bias)
