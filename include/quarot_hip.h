@@ -262,8 +262,9 @@ int qr_linear_f6_f16(const void* A6, const void* sA, const void* W6, const void*
  * the 70B down_proj, 28672 = 1024 x 28), mode QR_DTYPE_F16: a single kernel in which every workgroup
  * transforms and quantises the rows itself and goes straight on to its dot products -- the same codes,
  * scales, sums and epilogue, so y carries the same bits, and the weight stream starts while the rows are
- * still being transformed.  ONE or TWO tokens with had_K == 0 (K up to 32768): likewise one kernel, every
- * workgroup quantising the rows itself.  The workspace is checked as always; what it holds afterwards
+ * still being transformed.  Likewise behind a 64-point factor (had_K 100 to 192, table or sign words: 11008 = 64 x 172) or a
+ * 128-point one (had_K 36 to 64 and 100 to 128: 13824 = 128 x 108).  ONE or TWO tokens with had_K == 0 (K up to 32768):
+ * likewise one kernel, every workgroup quantising the rows itself.  The workspace is checked as always; what it holds afterwards
  * is unspecified.
  *   x fp16 [M, K]; had_K, hadK, mode, scale as in qr_hadamard_quantize_f16_i4; W uint8 [N, K/2],
  *   sW fp16 [N], bias fp16 [N] or NULL -> y fp16 [M, N].

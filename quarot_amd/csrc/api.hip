@@ -57,7 +57,8 @@ extern "C" int qr_quantized_linear_f16(const void* x, int64_t M, int64_t K, int 
                                                           (hipStream_t)stream);
         if (rc1 != QR_E_UNSUPPORTED) return rc1;
     }
-    if (M <= 2 && had_K > 1 && (mode & ~QR_HADK_SIGNS) == QR_DTYPE_F16 && hadK && ((uintptr_t)y & 1) == 0) {
+    // the same behind a factor of 64 or 128; an output that the GEMM refuses (8-byte alignment) is left to it
+    if (M <= 2 && had_K > 1 && (mode & ~QR_HADK_SIGNS) == QR_DTYPE_F16 && hadK && ((uintptr_t)y & 7) == 0) {
         const int rc1 = qr_internal_token_mm_linear(x, M, (int)K, had_K, hadK, (mode & QR_HADK_SIGNS) ? 1 : 0, scale, clip, W, sW,
                                                     bias_or_null, N, y, (hipStream_t)stream);
         if (rc1 != QR_E_UNSUPPORTED) return rc1;

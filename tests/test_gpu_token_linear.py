@@ -1,11 +1,15 @@
 """One or two tokens behind a Hadamard of 64 or 128 values and a table of order 33 and more: qr_quantized_linear_f16 runs the front
 and the dot products in one kernel in which every workgroup transforms the rows itself.  Its output must carry the bits of
 the two-launch chain (same codes, same scale, same sums, same epilogue)."""
+import ctypes
+import math
+
 import numpy as np
 import pytest
 import torch
 
 import quarot_amd
+from quarot_amd import _lib
 from oracle import quarot_oracle as o
 
 pytestmark = pytest.mark.gpu
@@ -49,3 +53,19 @@ def test_one_token_behind_a_short_factor_in_one_launch(n, M):
         x[M - 1, 5] = value if value != 1.0 else x[M - 1, 5]
         got, want = quarot_amd.quantized_linear(x, w, sw, None, hadK, K), _chain(x, w, sw, None, hadK, K, 1.0)
         assert torch.equal(got.view(torch.int16), want.view(torch.int16)), (value, scale)
+
+
+def test_output_that_is_not_8_byte_aligned_is_refused():
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    n, N = 11008, 40
+    table, K = quarot_amd.functional.hadamard.get_hadK(n)
+    hadK = table.to("cuda").half()
+    w, sw, _ = _weights(n, N, False, gen)
+    x = torch.randn(1, n, device="cuda", generator=gen).half()
+    lib, size = _lib.lib(), _lib.lib().qr_quantized_linear_workspace_bytes(1, N, n)
+    work, y = torch.empty(size, dtype=torch.uint8, device="cuda"), torch.full((N + 8,), 7, dtype=torch.float16, device="cuda")
+    p = lambda t: ctypes.c_void_p(t.data_ptr())
+    call = lambda out: lib.qr_quantized_linear_f16(p(x), 1, n, K, p(hadK), 0, 1 / math.sqrt(n), 1.0, p(w), p(sw), None, N, p(out), p(work), size, None)
+    assert call(y[1:]) == call(y[2:]) == -4                 # QR_E_ALIGN
+    assert bool((y == 7).all())
+    assert call(y[4:]) == 0 and bool((y[:4] == 7).all()) and bool((y[4 + N:] == 7).all())
