@@ -143,8 +143,9 @@ __device__ __forceinline__ void e2m3_tiles(
         const int kb = (st < stages ? st : more ? st - stages : stages - 1) * 128;
         __attribute__((address_space(3))) void* dst =
             (__attribute__((address_space(3))) void*)(lds + buf * STAGE + (i * NT + wave * 64) * 16);
-        // pieces past the end of a row lie beyond the buffer's range and arrive as zeros: codes 0
-        const u32 off = RAGGED && kb + piece >= Kb ? 0xFFFFFF00u : goff[i];
+        // pieces past the end of a row are sent beyond the buffer's range and arrive as zeros: codes 0 (an operand is a multiple of 32
+        // bytes below 4 GiB: at most 0xFFFFFFE0)
+        const u32 off = RAGGED && kb + piece >= Kb ? 0xFFFFFFE0u : goff[i];
         if (i * 32 < BM) __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_a, dst, 16, off, kb, 0, 0);
         else __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_b, dst, 16, off, kb, 0, 0);
     };

@@ -87,3 +87,20 @@ def test_scales_and_bias_may_start_anywhere(m, n, k, shift):
     y = torch.empty(m, n, dtype=torch.float16, device="cuda")
     assert lib.qr_linear_i4_f16(p(a), p(sa), p(b), p(sb), p(bias), m, n, k, p(y), None) == 0
     assert torch.equal(y, (sa * sb) * _sums(a, b).float().half() + bias)
+
+
+def test_ragged_rows_of_an_operand_that_ends_below_4_gib():
+    """262657 x 16352 bytes = 2^32 - 32: pieces past the end of a row must lie beyond even this operand's last byte."""
+    m, n, k = 262657, 256, 32704
+    assert m * k // 2 == 2**32 - 32 and _lib.lib().qr_linear_plan(m, n, k, 0, None).startswith(b"gemm_sp")
+    gen = torch.Generator(device="cuda").manual_seed(k)
+    a = torch.empty(m, k // 2, dtype=torch.uint8, device="cuda")
+    for rows in a.split(1 << 15):
+        rows.copy_(_operand(rows.shape[0], k, "random", gen))
+    b = _operand(n, k, "random", gen)
+    sa, sb = torch.ones(m, 1, device="cuda").half(), torch.full((n,), 0.001, device="cuda").half()
+    p = lambda t: ctypes.c_void_p(t.data_ptr())
+    y = torch.empty(m, n, dtype=torch.float16, device="cuda")
+    assert _lib.lib().qr_linear_i4_f16(p(a), p(sa), p(b), p(sb), None, m, n, k, p(y), None) == 0
+    for rows in (slice(0, 300), slice(m // 2, m // 2 + 300), slice(m - 300, m)):
+        assert torch.equal(y[rows], (sa[rows] * sb) * _sums(a[rows], b).float().half())
