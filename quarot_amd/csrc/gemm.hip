@@ -1184,7 +1184,7 @@ struct MidPlan {
     int kernel;         // 0 .. 2: qr_internal_gemm_mid's shapes; 3 .. 6: qr_internal_gemm_e2m3's; 7: 96 x 64 tiles
     int split;
 };
-MidPlan mid_plan(int64_t M, int64_t N, int64_t Kb, int64_t max_split) {
+MidPlan mid_plan(int64_t M, int64_t N, int64_t Kb, int64_t max_split, bool fp16) {
     const int64_t cus = qr_device().cus;
     const double st = (double)((Kb + 127) / 128);
     auto tiles = [&](int64_t bm, int64_t bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
@@ -1210,14 +1210,15 @@ MidPlan mid_plan(int64_t M, int64_t N, int64_t Kb, int64_t max_split) {
     consider(2, 1, nsq == 1 ? 5.5 + 0.73 * st : nsq == 2 ? 9.7 + 1.50 * st : 5.5 + nsq * (3.6 + 0.755 * st));
     const double fixed[3] = {8.1, 6.8, 8.9}, slope[3] = {0.99, 1.56, 1.76}, easier[3] = {0.25, 0.18, 0.22};
     auto round = [&](int i, double idle) { return fixed[i] + slope[i] * st * (1.0 - easier[i] * idle); };
-    const bool reach = N < (1LL << 22);                     // 256 rows of the output within the 32-bit offsets of the stores
-    for (int i = 2; reach && i >= 0; --i) {                 // (ties go to the taller tile)
+    auto reach = [&](int64_t rows) { return qr_e2m3_reach(rows, N, fp16); };
+    for (int i = 2; i >= 0; --i) {                          // (ties go to the taller tile)
+        if (!reach(128 + 64 * i)) continue;
         const int64_t t = tiles(128 + 64 * i, 256);
         const double n = loaded(t);
         consider(3 + i, 1, 1.7 + n * round(i, 1.0 - (double)t / (n * (double)cus)));
     }
     const int64_t whole = tiles(256, 256) / cus, left = tiles(256, 256) % cus;
-    if (reach && Kb > 128 && cus % qr_device().xcds == 0 && whole > 0 && left > 0 && 2 * left <= cus)
+    if (reach(256) && Kb > 128 && cus % qr_device().xcds == 0 && whole > 0 && left > 0 && 2 * left <= cus)
         consider(6, 1, 1.7 + (double)whole * round(2, 0.0) + round(0, 1.0 - 2.0 * (double)left / (double)cus));
     const int64_t all_stages = (Kb + 127) / 128;
     for (int64_t ks = 2; ks <= max_split && ks <= all_stages / 4; ++ks)
@@ -1232,12 +1233,12 @@ struct GemmPlan {
     Gemm kernel;
     int split;
 };
-GemmPlan gemm_plan(int64_t M, int64_t N, int64_t Kb, int64_t max_split) {
+GemmPlan gemm_plan(int64_t M, int64_t N, int64_t Kb, int64_t max_split, bool fp16) {
     // An operand of 4 GiB or more: every specialised kernel below addresses its operands through 32-bit offsets;
     // the plain tiled kernel computes 64-bit row addresses and takes any shape (rows beyond M or N are clamped).
     if (M * Kb >= (1LL << 32) || N * Kb >= (1LL << 32)) return GemmPlan{Gemm::large, 1};
     if (M > 64) {
-        const MidPlan plan = mid_plan(M, N, Kb, max_split);
+        const MidPlan plan = mid_plan(M, N, Kb, max_split, fp16);
         constexpr Gemm kernels[] = {Gemm::mid64, Gemm::mid64x128, Gemm::mid128, Gemm::spk, Gemm::sp192, Gemm::sp256, Gemm::sp256_tail, Gemm::mid96};
         return GemmPlan{kernels[plan.kernel], plan.split};
     }
@@ -1264,7 +1265,7 @@ int gemm_dispatch(const void* A, const void* B, int64_t M, int64_t N, int64_t K,
     const int m = (int)M, n = (int)N, kb = (int)(K / 2);
     // the slabs of a K split go to scratch from the caller; without it (or with too little) the single-launch kernels run
     const bool scratch = Y && ws && ((uintptr_t)ws & 15) == 0;
-    const GemmPlan plan = gemm_plan(M, N, kb, scratch ? (int64_t)(ws_bytes / ((size_t)M * (size_t)N * 4)) : 1);
+    const GemmPlan plan = gemm_plan(M, N, kb, scratch ? (int64_t)(ws_bytes / ((size_t)M * (size_t)N * 4)) : 1, Y != nullptr);
     const int mid = plan.kernel == Gemm::stream64 ? 3 : plan.kernel == Gemm::mid96 ? 4 : (int)plan.kernel - (int)Gemm::mid64;      // qr_internal_gemm_mid's shape
     if (plan.split > 1) {
         const int rc = qr_internal_gemm_mid(mid, A, B, m, n, kb, ws, nullptr, nullptr, nullptr, nullptr, st, plan.split);
@@ -1314,7 +1315,7 @@ extern "C" const char* qr_linear_plan(int64_t M, int64_t N, int64_t K, size_t wo
     if (scratch_bytes) *scratch_bytes = 0;
     if (M <= 0 || N <= 0 || K <= 0 || K % 64 != 0 || K > 131008 || M > 0x7fffffff || N > 0x7fffffff) return nullptr;
     const size_t slab = (size_t)M * (size_t)N * 4;
-    const GemmPlan plan = gemm_plan(M, N, K / 2, workspace_bytes ? (int64_t)(workspace_bytes / slab) : 1);
+    const GemmPlan plan = gemm_plan(M, N, K / 2, workspace_bytes ? (int64_t)(workspace_bytes / slab) : 1, true);
     const bool slices = plan.split > 1;
     if (slices && scratch_bytes) *scratch_bytes = slab * (size_t)plan.split;
     switch (plan.kernel) {

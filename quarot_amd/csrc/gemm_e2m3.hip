@@ -545,11 +545,13 @@ __global__ __launch_bounds__(256) void gemm_sp256_tail_kernel(
 }  // namespace
 
 // shape 0 / 1 / 2: tiles of 128 / 192 / 256 rows; 3: 256-row tiles and a last round of 128-row ones (more than one round of tiles, CUs a
-// multiple of the XCDs).  Y == nullptr: int32 sums to C.  K up to 131008; operands below 4 GiB (32-bit buffer offsets).
+// multiple of the XCDs).  Y == nullptr: int32 sums to C.  K up to 131008; operands below 4 GiB (32-bit buffer offsets),
+// outputs within qr_e2m3_reach.
 int qr_internal_gemm_e2m3(int shape, const void* A, const void* B, int M, int N, int Kb, void* C, void* Y, const void* sA,
                           const void* sB, const void* bias, hipStream_t st) {
-    if ((int64_t)M * Kb >= (1LL << 32) || (int64_t)N * Kb >= (1LL << 32) || N >= (1 << 22)) return QR_E_UNSUPPORTED;   // (the dispatcher routes these away)
     const int bm = shape == 0 ? 128 : shape == 1 ? 192 : 256;
+    if ((int64_t)M * Kb >= (1LL << 32) || (int64_t)N * Kb >= (1LL << 32) || !qr_e2m3_reach(bm, N, Y != nullptr))
+        return QR_E_UNSUPPORTED;                            // (the dispatcher routes these away)
     const int tiles_m = (M + bm - 1) / bm, tiles_n = (N + 255) / 256;
     const int nxcd = qr_device().xcds, cus = qr_device().cus;
     const int64_t tiles = (int64_t)tiles_m * tiles_n, whole = shape == 3 ? tiles / cus * cus : 0;

@@ -117,6 +117,8 @@ int qr_internal_gemm_mid(int shape, const void* A, const void* B, int M, int N, 
 
 // gemm_e2m3.hip: the GEMM on the FP6 matrix path (shape 0 / 1 / 2: tiles of 128 / 192 / 256 x 256, 3: 256 with a last round of 128);
 // Y == nullptr: int32 sums to C
+// qr_e2m3_reach: whether its stores, offsets of 32 bits from a tile's first row, reach `rows` rows of an output of N columns
+static inline bool qr_e2m3_reach(int64_t rows, int64_t N, bool fp16) { return rows * N * (fp16 ? 2 : 4) <= 0xFFFFFF00LL; }
 int qr_internal_gemm_e2m3(int shape, const void* A, const void* B, int M, int N, int Kb, void* C, void* Y, const void* sA,
                           const void* sB, const void* bias, hipStream_t st);
 

@@ -71,7 +71,7 @@ __device__ __forceinline__ Slab slab_turn(char* region, const f16x4 (&o)[2][4], 
     for (int p = 0; p < 4; ++p) s.v[p] = *(const u32x4*)(get + p * 1024);
     return s;
 }
-// The rows of an output tile that exist, `rows` of at most 256 from m0 on; N < 2^23 (offsets of 32 bits)
+// The rows of an output tile that exist, `rows` from m0 on: at most 0xFFFFFF00 bytes of them (offsets of 32 bits)
 struct SlabOut {
     __amdgpu_buffer_rsrc_t rsrc;
     u32 lane_at;                                // byte offset of this lane's first piece in a slab

@@ -165,3 +165,11 @@ def test_plan_of_five_small_tiles_per_cu_depends_on_the_weights(lib):
                            (640, 8192, 8192, True), (300, 13824, 8192, True)):
         name = lib.qr_linear_plan(m, n, k, 0, None)
         assert name == (b"gemm_mid_kernel<64,64>" if small else b"gemm_spk_kernel"), (m, n, k, name)
+
+
+def test_plan_of_very_wide_outputs(lib):
+    """The large tiles store through 32-bit offsets from a tile's first row: 256 rows of fp16 up to 2^23 columns, 128 up to 2^24."""
+    for n in ((1 << 22) - 8, 1 << 22, 4500000):
+        assert lib.qr_linear_plan(256, n, 1856, 0, None) == b"gemm_sp256_kernel", n
+    for n in (1 << 24, (1 << 25) + 64):
+        assert lib.qr_linear_plan(256, n, 192, 0, None).startswith(b"gemm_mid_kernel"), n

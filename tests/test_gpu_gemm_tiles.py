@@ -104,3 +104,27 @@ def test_ragged_rows_of_an_operand_that_ends_below_4_gib():
     assert _lib.lib().qr_linear_i4_f16(p(a), p(sa), p(b), p(sb), None, m, n, k, p(y), None) == 0
     for rows in (slice(0, 300), slice(m // 2, m // 2 + 300), slice(m - 300, m)):
         assert torch.equal(y[rows], (sa[rows] * sb) * _sums(a[rows], b).float().half())
+
+
+@pytest.mark.parametrize("m,n,k,int32", [
+    (257, (1 << 22) + 8, 192, False), (130, (1 << 23) - 8, 128, False), (129, 5592403, 192, True), (140, (1 << 23) + 3, 64, False)])
+def test_outputs_of_millions_of_columns(m, n, k, int32):
+    """Either side of what 256, 192 and 128 rows of an output reach through 32-bit offsets; the output inside guard bands."""
+    lib = _lib.lib()
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    a = _operand(m, k, "random", gen)
+    b = torch.randint(0, 256, (n, k // 2), dtype=torch.uint8, device="cuda", generator=gen)
+    p = lambda t: ctypes.c_void_p(t.data_ptr())
+    out = torch.full((m + 2, n), 7, dtype=torch.int32 if int32 else torch.float16, device="cuda")
+    y = out.view(-1)[8:8 + m * n].view(m, n)
+    if int32:
+        assert lib.qr_matmul_i4_i32(p(a), p(b), m, n, k, p(y), None) == 0
+    else:
+        sa = (torch.rand(m, 1, device="cuda", generator=gen) * 0.1 + 0.01).half()
+        sb = (torch.rand(n, device="cuda", generator=gen) * 0.01 + 0.001).half()
+        assert lib.qr_linear_i4_f16(p(a), p(sa), p(b), p(sb), None, m, n, k, p(y), None) == 0
+    assert bool((out.view(-1)[:8] == 7).all()) and bool((out.view(-1)[8 + m * n:] == 7).all())
+    step = 1 << 19
+    for at in range(0, n, step):
+        want = _sums(a, b[at:at + step])
+        assert torch.equal(y[:, at:at + step], want if int32 else (sa * sb[at:at + step]) * want.float().half()), at
