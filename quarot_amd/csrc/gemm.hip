@@ -1165,9 +1165,7 @@ int ks_split(int64_t M, int64_t N, int64_t Kb) {
 // (geometric mean; 1.4 x at worst, where 64-row tiles are few and K is long)):
 //   64 x 64 tiles   3.9 + st 0.264 (n = 1), 4.6 + st 0.42 (n = 2), 3.9 + n (0.75 + 0.21 st) beyond: three workgroups share a CU; 0.23 for 0.21 from
 //                   n = 5 on where K > 8192 and the weights are over 36 MB: they are read once per 64 tokens there and once per
-//                   128 or more by the larger tiles, from memory.  n = 5 and lighter weights: 0.18, less than they take, which keeps the
-//                   small tiles there as tests/test_abi.py has it; 128-row tiles are 4-14 % ahead in that corner when operands come
-//                   from memory (1260 x 4096 x 11008 53 / 49 us, 640 x 8192 x 8192 41.5 / 39, 2560 x 2048 x 28672 125 / 109)
+//                   128 or more by the larger tiles, from memory.
 //   96 x 64         5.1 + st 0.325 (n = 1; 0.37 where K > 8192 and the weights are over 36 MB), 8.0 + st 0.69 (n = 2), 5.1 + n (2.0 + 0.335 st)
 //                   (5094 more shapes of 65 .. 1500 tokens: ahead by 11 % on the tenth of them where it is the best, mostly n = 1, and
 //                   the choice among all kernels costs 0.9 % more than the best of them, 2.1 % without it)
@@ -1193,7 +1191,7 @@ MidPlan mid_plan(int64_t M, int64_t N, int64_t Kb, int64_t max_split, bool fp16)
     auto t64 = [&](int64_t t, double stages) {
         const double n = loaded(t);
         if (n <= 2) return n == 1 ? 3.9 + 0.264 * stages : 4.6 + 0.42 * stages;
-        return 3.9 + n * (0.75 + (n >= 5 && heavy ? 0.23 : n == 5 ? 0.18 : 0.21) * stages);
+        return 3.9 + n * (0.75 + (n >= 5 && heavy ? 0.23 : 0.21) * stages);
     };
     MidPlan best{0, 1};
     double t_best = t64(tiles(64, 64), st);
