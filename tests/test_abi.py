@@ -173,3 +173,12 @@ def test_plan_of_very_wide_outputs(lib):
         assert lib.qr_linear_plan(256, n, 1856, 0, None) == b"gemm_sp256_kernel", n
     for n in (1 << 24, (1 << 25) + 64):
         assert lib.qr_linear_plan(256, n, 192, 0, None).startswith(b"gemm_mid_kernel"), n
+
+
+def test_plan_counts_the_cost_of_an_output_that_ends_inside_a_tile(lib):
+    """A last column of tiles that the output's edge cuts, and rows of no whole 16-byte pieces, leave the small tiles element by element,
+    the 128 x 128 ones slowest (measured: 9 us on 64 x 64 tiles, 14 on 128 x 128, for the first shape)."""
+    for m, n, k in ((133, 11112, 1024), (5568, 448, 448), (440, 5568, 128), (3000, 704, 704), (1001, 2649, 768), (106, 18581, 256)):
+        assert lib.qr_linear_plan(m, n, k, 0, None) == b"gemm_mid_kernel<64,64>", (m, n, k)
+    offered = lib.qr_workspace_bytes(83, 5120, 13824)           # (18 us in slices of K, 22 in one launch)
+    assert b"sliced" in lib.qr_linear_plan(83, 5120, 13824, offered, None)
