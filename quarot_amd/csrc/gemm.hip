@@ -1336,8 +1336,8 @@ extern "C" const char* qr_linear_plan(int64_t M, int64_t N, int64_t K, size_t wo
         case Gemm::shared_tokens: return "decode_xs_kernel";
         case Gemm::decode: return "decode_i4_kernel";
         case Gemm::stream64:
-        case Gemm::mid96:                                   // (its form with three row tiles per wave)
         case Gemm::mid64: return slices ? "gemm_mid_kernel<64,64> (K sliced) + dequant_slabs_kernel" : "gemm_mid_kernel<64,64>";
+        case Gemm::mid96: return "gemm_mid_kernel<96,64>";
         case Gemm::mid64x128: return "gemm_mid_kernel<64,128>";
         case Gemm::mid128: return "gemm_mid_kernel<128,128>";
         case Gemm::spk: return "gemm_spk_kernel";

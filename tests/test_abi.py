@@ -152,7 +152,7 @@ def test_plan_names_a_kernel_for_every_shape_and_stays_within_the_workspace(lib)
                 assert lib.qr_linear_plan(m, n, k, used.value, None) == name
                 assert b"sliced" not in lib.qr_linear_plan(m, n, k, 0, None)
                 seen.add(name)
-    assert len(seen) == 10 and lib.qr_linear_plan(1 << 17, 128, 131008, 0, None) == b"gemm_i4_kernel", seen
+    assert len(seen) == 11 and lib.qr_linear_plan(1 << 17, 128, 131008, 0, None) == b"gemm_i4_kernel", seen
     for bad in ((0, 1, 64), (1, 0, 64), (1, 1, 0), (1, 1, 100), (1, 1, 131072), (1 << 31, 1, 64)):
         assert lib.qr_linear_plan(*bad, 0, None) is None
 

@@ -66,11 +66,19 @@ def test_gemm_of_large_tiles_bit_exact(m, n, k, kernel, kind):
 
 
 @pytest.mark.parametrize("m,n,k", [
-    # 96 x 64 tiles (the plan's choice for one tile on each CU): whole tiles, one row or column into the last one, K that ends inside a stage,
-    # rows of no whole 16-byte pieces
-    (333, 4096, 4096), (192, 8192, 11008), (193, 5377, 4160), (385, 3200, 4160), (190, 8131, 2112), (275, 5437, 1600), (260, 5440, 2048)])
+    # one 96 x 64 tile on each CU: whole tiles, one row or column into the last one, K that ends inside a stage, rows of no whole
+    # 16-byte pieces; the last two: two tiles on a CU
+    (333, 4096, 4096), (192, 8192, 11008), (193, 5377, 4160), (385, 3200, 4160), (260, 5440, 2048), (96, 10241, 4160), (95, 8200, 8256),
+    (257, 10241, 4160), (257, 10241, 11008)])
 @pytest.mark.parametrize("kind", ["random", "extreme"])
 def test_gemm_of_96_row_tiles_bit_exact(m, n, k, kind):
+    assert _lib.lib().qr_linear_plan(m, n, k, 0, None) == b"gemm_mid_kernel<96,64>"
+    _compare(m, n, k, kind)
+
+
+@pytest.mark.parametrize("m,n,k", [(190, 8131, 2112), (275, 5437, 1600)])       # (three 64 x 64 tiles on a CU)
+@pytest.mark.parametrize("kind", ["random", "extreme"])
+def test_gemm_of_64_row_tiles_bit_exact(m, n, k, kind):
     _compare(m, n, k, kind)
 
 
