@@ -25,6 +25,15 @@ def _sums(a, b):
 def _operand(rows, k, kind, gen):
     if kind == "random":
         return torch.randint(0, 256, (rows, k // 2), dtype=torch.uint8, device="cuda", generator=gen)
+    if kind in ("high", "turn", "signs"):
+        r = torch.randint(0, 256, (rows, k // 2), dtype=torch.uint8, device="cuda", generator=gen)
+        x = (r & 0x11) | 0x66                                # codes 6 and 7
+        if kind == "turn":                                   # codes -8 and -7 up to where the accumulators are first corrected
+            x[:, :24576] = (r[:, :24576] & 0x11) | 0x88
+        if kind == "signs":                                  # 6, 7, -7 and -6 (a nibble and its complement)
+            x ^= (r & 0x02) // 0x02 * 0x0F
+            x ^= (r & 0x20) // 0x20 * 0xF0
+        return x
     x = torch.full((rows, k // 2), 0x77, dtype=torch.uint8, device="cuda")     # the largest and smallest sums, with and without the offset
     x[::3] = 0x88
     x[1::7] = 0
@@ -34,7 +43,7 @@ def _operand(rows, k, kind, gen):
 def _compare(m, n, k, kind):
     lib = _lib.lib()
     gen = torch.Generator(device="cuda").manual_seed(m + n + k)
-    a, b = _operand(m, k, kind, gen), _operand(n, k, kind, gen)
+    a, b = _operand(m, k, "high" if kind == "cancel" else kind, gen), _operand(n, k, "signs" if kind == "cancel" else kind, gen)
     sa = (torch.rand(m, 1, device="cuda", generator=gen) * 0.1 + 0.01).half()
     sb = (torch.rand(n, device="cuda", generator=gen) * 0.01 + 0.001).half()
     bias = torch.randn(n, device="cuda", generator=gen).half()
@@ -61,6 +70,32 @@ def _compare(m, n, k, kind):
 ])
 @pytest.mark.parametrize("kind", ["random", "extreme"])
 def test_gemm_of_large_tiles_bit_exact(m, n, k, kernel, kind):
+    assert _lib.lib().qr_linear_plan(m, n, k, 0, None) == kernel.encode()
+    _compare(m, n, k, kind)
+
+
+# Three and more tiles per workgroup, whose pipeline runs on from one tile into the next: 192- and 256-row tiles and whole rounds before a
+# last one of 128-row tiles, K that ends inside a stage, an odd and an even number of stages.
+@pytest.mark.parametrize("m,n,k,kernel", [
+    (9000, 9003, 704, "gemm_sp256_kernel"), (12500, 5124, 448, "gemm_sp256_kernel"),           # 192 rows
+    (24900, 4100, 576, "gemm_sp256_kernel"), (9216, 5120, 1344, "gemm_sp256_kernel"),          # 256 rows
+    (11700, 4100, 576, "gemm_sp256_tail_kernel"), (16640, 4104, 832, "gemm_sp256_tail_kernel"), (6145, 16388, 320, "gemm_sp256_tail_kernel"),
+    (20000, 5121, 1088, "gemm_sp256_tail_kernel")])
+def test_gemm_of_many_large_tiles_bit_exact(m, n, k, kernel):
+    assert _lib.lib().qr_linear_plan(m, n, k, 0, None) == kernel.encode()
+    _compare(m, n, k, "random")
+
+
+# Sums of products of codes + 8, of either parity, up to 14.2 million of the 16.8 million that fp32 holds exactly: "high" 10.3 million
+# before a correction, "turn" 3 million of small products corrected and 11 million of large ones on top, "cancel" 5.7 million that come to
+# a few thousand in the end, so that fp16 outputs are finite.  Walks of three tiles whose turn (two stages before the end) meets the
+# correction every 192 stages: 192, 193 and 194 stages.
+@pytest.mark.parametrize("m,n,k,kernel", [
+    (520, 9000, 49152, "gemm_spk_kernel"), (520, 9000, 98304, "gemm_spk_kernel"), (513, 16388, 131008, "gemm_sp256_kernel"),
+    (11776, 4096, 49152, "gemm_sp256_kernel"), (11700, 4090, 49408, "gemm_sp256_kernel"), (11776, 4096, 49664, "gemm_sp256_kernel"),
+    (8450, 4100, 49408, "gemm_sp256_tail_kernel")])
+@pytest.mark.parametrize("kind", ["high", "turn", "cancel"])
+def test_large_sums_of_either_parity_bit_exact(m, n, k, kernel, kind):
     assert _lib.lib().qr_linear_plan(m, n, k, 0, None) == kernel.encode()
     _compare(m, n, k, kind)
 
