@@ -1780,6 +1780,7 @@ int launch_row_quant(const void* x, int64_t rows, int K, const void* hadK, int s
                      hipStream_t st) {
     using Front = MmRow<LOG2M, KS2, 128 * KS2 * (LOG2M - 5)>;
     const size_t lds = (size_t)Front::T_BYTES + (signs ? 0 : (size_t)K * K * 2);
+    if (rows > (2 * lds <= 160 * 1024 ? 2 : 1) * (int64_t)qr_device().cus) return QR_E_UNSUPPORTED;     // (see the call)
     const auto kern = hadamard_row_quant_kernel<LOG2M, KS2>;
     if (lds > 48 * 1024) {
         const hipError_t e = qr_allow_dynamic_lds((const void*)kern, lds);
@@ -1796,14 +1797,17 @@ int launch_hadamard_mm(const void* x, void* y, int64_t rows, int n, int K, const
     const int KS2 = ((K + 31) & ~31) >> 5;
     // Up to two rows per CU: one workgroup per row, as many waves as it has tiles.  At 512 rows on 256 CUs it is still ahead (11008 values
     // 8.4 -> 7.6 us, 13824 10.2 -> 9.3, 5120 5.6 -> 5.3); with a third row the kernels that keep the table's fragments win
-    // (700 rows of 11008: 9.1 us against 9.8, 13824: 11.8 against 12.7).
+    // (700 rows of 11008: 9.1 us against 9.8, 13824: 11.8 against 12.7).  A table of fp16 lies in LDS: where two workgroups with it do not
+    // fit on a CU (order 172: 2 x 84 KB), only up to one row per CU (512 rows of 11008 10.3 us, with the four-wave kernel 9.0; 256 rows 6.1 / 7.1).
     if (!MODE32 && QUANT && y == nullptr && hadK != nullptr && rows <= 2 * (int64_t)qr_device().cus && ((uintptr_t)x & 15) == 0 &&
         ((uintptr_t)hadK & (signs ? 3 : 7)) == 0) {
-        if (m == 64 && KS2 == 4) return launch_row_quant<6, 4>(x, rows, K, hadK, signs, scale, clip, q, scales, st);
-        if (m == 64 && KS2 == 5) return launch_row_quant<6, 5>(x, rows, K, hadK, signs, scale, clip, q, scales, st);
-        if (m == 64 && KS2 == 6) return launch_row_quant<6, 6>(x, rows, K, hadK, signs, scale, clip, q, scales, st);
-        if (m == 128 && KS2 == 2) return launch_row_quant<7, 2>(x, rows, K, hadK, signs, scale, clip, q, scales, st);
-        if (m == 128 && KS2 == 4) return launch_row_quant<7, 4>(x, rows, K, hadK, signs, scale, clip, q, scales, st);
+        int rc = QR_E_UNSUPPORTED;
+        if (m == 64 && KS2 == 4) rc = launch_row_quant<6, 4>(x, rows, K, hadK, signs, scale, clip, q, scales, st);
+        if (m == 64 && KS2 == 5) rc = launch_row_quant<6, 5>(x, rows, K, hadK, signs, scale, clip, q, scales, st);
+        if (m == 64 && KS2 == 6) rc = launch_row_quant<6, 6>(x, rows, K, hadK, signs, scale, clip, q, scales, st);
+        if (m == 128 && KS2 == 2) rc = launch_row_quant<7, 2>(x, rows, K, hadK, signs, scale, clip, q, scales, st);
+        if (m == 128 && KS2 == 4) rc = launch_row_quant<7, 4>(x, rows, K, hadK, signs, scale, clip, q, scales, st);
+        if (rc != QR_E_UNSUPPORTED) return rc;
     }
     if (m == 128 && KS2 >= 2 && KS2 != 3 && !MODE32 && QUANT && y == nullptr && hadK != nullptr && ((uintptr_t)x & 15) == 0) {
         // m = 128 behind one of the reference's tables of order 36 and more (Llama-2-13B: 5120 = 40 x 128, 13824 =

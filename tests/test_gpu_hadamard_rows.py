@@ -32,7 +32,7 @@ def test_few_rows_have_the_bits_of_many(n, signs):
     assert MANY > 2 * cus
     for clip in (1.0, 0.83):
         many = _bits(quarot_amd.hadamard_quantize(x, hadK, K, clip_ratio=clip))
-        for rows in (1, 2, 7, 48, cus, 2 * cus, 2 * cus + 1):
+        for rows in (1, 2, 7, 48, cus, cus + 1, 2 * cus, 2 * cus + 1):
             few = _bits(quarot_amd.hadamard_quantize(x[:rows].contiguous(), hadK, K, clip_ratio=clip))
             assert torch.equal(few[0], many[0][:rows]) and torch.equal(few[1].view(-1), many[1][:rows].view(-1)), (rows, clip)
         end = _bits(quarot_amd.hadamard_quantize(x[MANY - 33:].contiguous(), hadK, K, clip_ratio=clip))
