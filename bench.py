@@ -41,6 +41,7 @@ Prints ONE JSON line on stdout.  The default run measures the headline workload 
 `per_config`, every other benchmark configuration with fewer repeats.
 """
 import argparse
+import hashlib
 import json
 import os
 import re
@@ -85,7 +86,8 @@ HBM_PEAK_GBS = 8000.0
 
 # Profile summaries that hold the FETCH_SIZE / WRITE_SIZE readings of a workload's dominant kernel
 # ("traffic_kib: kernel=<substring> fetch=<KiB per dispatch> write=<KiB per dispatch>") and the copy
-# calibration ("traffic_scale: fetch=<factor> write=<factor>").
+# calibration ("traffic_scale: fetch=<factor> write=<factor>").  "traffic_code: file=<source> sha256=<digits>" says which code was
+# read (code_digest of the kernel's source): a kernel can be rewritten under its name.
 PROFILE_OF = {
     "c1": "gemm_spk_c1_q_proj_7b.txt", "c1n": "rmsnorm_quant_rows_c1n_q_proj_7b.txt",
     "c1o": "heads_hadamard_quant_c1o_o_proj_7b.txt", "c2": "gemm_spk_and_hadamard_m64r_c2_down_proj_7b.txt",
@@ -104,27 +106,35 @@ PROFILE_OF = {
 }
 
 
+def code_digest(source):
+    """The first 16 digits of the SHA-256 of a source file under quarot_amd/csrc without its comments and white space."""
+    text = open(os.path.join(ROOT, "quarot_amd", "csrc", source)).read()
+    return hashlib.sha256(re.sub(r"/\*.*?\*/|//[^\n]*|\s+", "", text, flags=re.S).encode()).hexdigest()[:16]
+
+
 def traffic_from_profile(workload, kernel):
-    """(bytes per launch, source file) from the committed rocprofv3 summary of this workload, scaled by
-    the copy calibration; (None, None) when no summary carries the readings."""
+    """(bytes per launch, source file, whether the kernel's code is the code that was read) from the committed rocprofv3 summary of this
+    workload, scaled by the copy calibration; (None, None, None) when no summary carries the readings, None in the last place where the
+    summary does not say which code it read."""
     pdir = os.path.join(ROOT, "profiles")
     name = PROFILE_OF.get(workload)
     try:
         text = open(os.path.join(pdir, name)).read() if name else ""
         cal = open(os.path.join(pdir, "copy_calibration_256MiB.txt")).read()
     except OSError:
-        return None, None
+        return None, None, None
     sc = re.search(r"traffic_scale:\s*fetch=([\d.]+)\s+write=([\d.]+)", cal)
     if not sc:
-        return None, None
+        return None, None, None
     kib, seen = 0.0, set()                       # a dominant "kernel" of two launches (K-sliced decode) sums both
     for m in re.finditer(r"traffic_kib:\s*kernel=(\S+)\s+fetch=([\d.]+)\s+write=([\d.]+)", text):
         if m.group(1) in kernel and m.group(1) not in seen:
             seen.add(m.group(1))
             kib += float(m.group(2)) * float(sc.group(1)) + float(m.group(3)) * float(sc.group(2))
     if seen:
-        return round(kib * 1024), f"profiles/{name}"
-    return None, None
+        code = re.search(r"traffic_code:\s*file=(\S+)\s+sha256=([0-9a-f]+)", text)
+        return round(kib * 1024), f"profiles/{name}", code_digest(code[1]) == code[2] if code else None
+    return None, None, None
 
 
 def synth_x(m, k, seed=0, outliers=True, device="cpu"):
@@ -785,11 +795,12 @@ def main():
 
     wl, res, steps, repeats = measure(args.workload, True)
     roof = dict(res["roofline"])
-    traffic, source = traffic_from_profile(args.workload + ("_fp6" if args.fp6 else ""), roof["kernel"])
+    traffic, source, current = traffic_from_profile(args.workload + ("_fp6" if args.fp6 else ""), roof["kernel"])
     if traffic is not None and args.workload == "c3":
         traffic *= 4                                       # the step is four launches; the summary holds their average
     roof["traffic"] = traffic
     roof["traffic_source"] = source
+    roof["traffic_of_this_code"] = current
     if roof.get("bound") == "mfma" and roof["peak"] == INT8_MFMA_PEAK_TOPS:
         # what the int8 matrix instruction alone sustains on this box right now (register-only loop, operands with the
         # GEMM's bit statistics, ~60 ms of launches): the part's own ceiling for ANY int8 kernel; `frac` stays against `peak`
@@ -832,9 +843,9 @@ def main():
             torch.cuda.empty_cache()
             _, r, _, _ = measure(name, False)
             per[name] = brief(r)
-            t, s = traffic_from_profile(name, r["roofline"]["kernel"])
+            t, s, same = traffic_from_profile(name, r["roofline"]["kernel"])
             if t is not None:
-                per[name]["roofline"]["traffic"], per[name]["roofline"]["traffic_source"] = (4 * t if name in ("c3", "c3_fp6") else t), s
+                per[name]["roofline"].update(traffic=4 * t if name in ("c3", "c3_fp6") else t, traffic_source=s, traffic_of_this_code=same)
         out["per_config"] = per
         # the same table in a few numbers per workload: [step ms, dominant kernel ms, its roofline fraction, the step's]
         out["roofline"]["per_config"] = {name: [r["ms"], r["roofline"]["kernel_ms"], r["roofline"]["frac"], r.get("step_frac")]
