@@ -1161,24 +1161,28 @@ int ks_split(int64_t M, int64_t N, int64_t Kb) {
 
 // Which kernel takes an output of more than 64 tokens, by an estimate in microseconds (st = stages of 256 k, n = tiles on the
 // busiest of the CUs):
-//   64 x 64 tiles   3.9 + st 0.264 (n = 1), 4.6 + st 0.42 (n = 2; 0.50 heavy), 3.9 + n (0.75 + 0.21 st) beyond (0.60 for 0.75 at n = 3): three
-//                   workgroups share a CU; heavy = K > 8192 and weights over 36 MB: 0.23 for 0.21 from n = 5 on.  They are read
-//                   once per 64 tokens there and once per 128 or more by the larger tiles, from memory.
-//   96 x 64         5.1 + st 0.325 (n = 1; 0.37 heavy), 8.0 + st 0.69 (n = 2), 5.1 + n (2.0 + 0.335 st)
+//   64 x 64 tiles   3.9 + st 0.264 (n = 1; 0.30 heavy), 4.6 + st 0.42 (n = 2; 0.46 heavy), 3.9 + n (0.75 + 0.21 st) beyond (0.60 for 0.75 at n = 3):
+//                   three workgroups share a CU; heavy = K > 8192 and weights over 36 MB: 0.23 for 0.21 from n = 5 on, and 0.25 where K > 4096
+//                   and weights are over 96 MB: they are read once per 64 tokens there and once per 128 or more by the larger tiles, from
+//                   memory (111 x 28736 x 9024 63 us, 45 on 128 x 128 tiles; with 72 MB, which the last-level cache keeps, 27 / 31).
+//   96 x 64         5.1 + st 0.325 (n = 1; 0.37 heavy), 8.0 + st 0.69 (n = 2; 0.85 for one row of tiles, none of whose weights is shared), 5.1 + n (2.0 + 0.335 st)
 //   64 x 128        4.9 + st 0.40 (n = 1), 7.6 + st 0.90 (n = 2), 4.9 + n (2.4 + 0.453 st)
 //   128 x 128       5.5 + st 0.73 (n = 1; int32 6.2), 9.7 + st 1.50 (n = 2), 5.5 + n (3.6 + 0.755 st)
 //   128 / 192 / 256 x 256 (e2m3 kernels)   1.7 + n ({8.1, 6.8, 8.9} + {0.99, 1.56, 1.76} st (1 - {0.25, 0.18, 0.22} idle)), idle = share of
 //                   the rounds' places without a tile (the clock is higher then)
 //   256 and 128     whole rounds of 256-row tiles and the rest as 128-row ones in the same launch, where that rest is at most half a round
-// and what the output adds.  The small tiles put whole tiles of 16-byte pieces out as lines and anything else element by element, all the
-// waves of such a tile one after the other; the e2m3 kernels' stores drop what lies beyond the edge.  A last column of tiles that the
-// edge cuts: 2 / 3 / 3 / 5.8 us for the four small shapes (133 x 11112 x 1024 9.1 us on 64 x 64 tiles, 14.4 on 128 x 128, which
-// the estimate without it took), 0 for the large ones; rows of no whole pieces (N % 8): 3.5 / 4 / 4 / 6 and 0.8 us per million
-// elements, 3 / 5.5 / 7.5 for the large ones (5.5 for 256 and 128); int32 sums: 1.8 / 2.8 / 3.2 for the large ones, 6 more where N % 4.  Outputs of more than 100 MB
-// leave the last-level cache: 0.19 / 0.5 / 0.23 / 0.08 us per MB beyond for the small shapes, whose stores come in smaller pieces.
-// Fitted to 3600 shapes of 65 .. 8192 tokens x 64 .. 28672 weight rows at K = 64 .. 28672, three quarters of them of whole lines, with
-// every kernel forced, weights from memory and from cache, and to 108 of 4.2 million rows and more.  The choice costs 0.3 %
-// more than the best of all kernels (geometric mean over 1500 shapes; 0.2 % up to K = 1536; without the output's terms 1.6 and 3.2 %, 2 x at worst).
+// and what the output adds.  The small tiles put whole tiles of 16-byte pieces out as lines and anything else element by element; the
+// e2m3 kernels' stores drop what lies beyond the edge.  A last column of tiles that the edge cuts, by the columns left in it: 0.07 us each
+// up to 3.2, 3.3 (96 x 64), 0.045 up to 3.3, 0.085 up to 5.7 for the four small shapes (133 x 11112 x 1024 9.1 us on 64 x 64 tiles, 14.4 on
+// 128 x 128, which the estimate without it took), none for the large ones; rows of no whole pieces (N % 8): 3.5 / 4 / 4 / 6 and 0.8 us per
+// million elements, 3 / 5.5 / 7.5 for the large ones (5.5 for 256 and 128); rows that start within a line (N % 64): 0.20 / 0.35 / 0.40 us
+// per million elements for the large ones; int32 sums: 1.8 / 2.8 / 3.2 for the large ones, 6 more where N % 4.  Outputs of more than 100 MB leave the
+// last-level cache: 0.19 / 0.5 / 0.23 / 0.08 us per MB beyond for the small shapes, whose stores come in smaller pieces.
+// Fitted with every kernel forced, weights from memory and from cache, to 3600 shapes of 65 .. 8192 tokens x 64 .. 28672 weight rows at
+// K = 64 .. 28672, three quarters of them of whole lines, 1200 of N = 128 .. 28672 in steps of 8, 108 of 4.2 million rows and more, and 700
+// of few tiles and a long K with up to eight slices.  The choice costs 0.2 % more than the best of all kernels (geometric mean; 0.1 % up to
+// K = 1536, 0.3 % at N in steps of 8, 0.7 % where K may be sliced; without the output's terms and those of heavy weights 1.6, 3.2, 1.9 and
+// 1.1 %, 2 x at worst).
 // The small tiles are bound by the CUs' intake of operands, the large ones by instruction issue and power, so the small ones lead
 // while the large ones leave CUs idle: 333 x 4096 x 4096 11.2 us against 22, 777 x 4096 x 4096 17.7 (22), 512 x 8192 x 8192 32.1 (34).
 // Very few tiles and a long K: slices of K over several workgroups with int32 slabs in the caller's scratch and a second
@@ -1192,21 +1196,22 @@ MidPlan mid_plan(int64_t M, int64_t N, int64_t Kb, int64_t max_split, bool fp16)
     const double st = (double)((Kb + 127) / 128);
     auto tiles = [&](int64_t bm, int64_t bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
     auto loaded = [&](int64_t t) { return (double)((t + cus - 1) / cus); };
-    const bool heavy = Kb > 4096 && N * Kb > 36000000;
+    const bool heavy = Kb > 4096 && N * Kb > 36000000, stream = Kb > 2048 && N * Kb > 96000000;
     const bool odd = fp16 && N % 8 != 0;                    // rows of the output of no whole 16-byte pieces
     const double elements = (double)M * (double)N * 1e-6, megabytes = elements * (fp16 ? 2.0 : 4.0);
     const double far = megabytes > 100.0 ? megabytes - 100.0 : 0.0;
     // what the output adds on the small tiles: a last column that the edge cuts, rows of no whole pieces, what leaves the caches
-    auto put = [&](int64_t bn, double cut, double ragged, double beyond) {
-        return far * beyond + (odd ? ragged + 0.8 * elements : fp16 && N % bn != 0 ? cut : 0.0);
+    auto put = [&](int64_t bn, double column, double most, double ragged, double beyond) {
+        const double cut = fp16 ? column * (double)(N % bn) : 0.0;
+        return far * beyond + (odd ? ragged + 0.8 * elements : cut < most ? cut : most);
     };
     auto t64 = [&](int64_t t, double stages) {
         const double n = loaded(t);
-        if (n <= 2) return n == 1 ? 3.9 + 0.264 * stages : 4.6 + (heavy ? 0.50 : 0.42) * stages;
-        return 3.9 + n * ((n == 3 ? 0.60 : 0.75) + (n >= 5 && heavy ? 0.23 : 0.21) * stages);
+        if (n <= 2) return n == 1 ? 3.9 + (heavy ? 0.30 : 0.264) * stages : 4.6 + (heavy ? 0.46 : 0.42) * stages;
+        return 3.9 + n * ((n == 3 ? 0.60 : 0.75) + (stream ? 0.25 : n >= 5 && heavy ? 0.23 : 0.21) * stages);
     };
     MidPlan best{0, 1};
-    double t_best = t64(tiles(64, 64), st) + put(64, 2.0, 3.5, 0.19);
+    double t_best = t64(tiles(64, 64), st) + put(64, 0.07, 3.2, 3.5, 0.19);
     auto consider = [&](int kernel, int split, double t) {
         if (t < t_best) {
             t_best = t;
@@ -1214,14 +1219,14 @@ MidPlan mid_plan(int64_t M, int64_t N, int64_t Kb, int64_t max_split, bool fp16)
         }
     };
     const double n96 = loaded(tiles(96, 64));
-    consider(7, 1, put(64, 3.0, 4.0, 0.5) + (n96 == 1 ? 5.1 + (heavy ? 0.37 : 0.325) * st : n96 == 2 ? 8.0 + 0.69 * st : 5.1 + n96 * (2.0 + 0.335 * st)));
+    consider(7, 1, put(64, 0.4, 3.3, 4.0, 0.5) + (n96 == 1 ? 5.1 + (heavy ? 0.37 : 0.325) * st : n96 == 2 ? 8.0 + (M <= 96 ? 0.85 : 0.69) * st : 5.1 + n96 * (2.0 + 0.335 * st)));
     const double n128 = loaded(tiles(64, 128)), nsq = loaded(tiles(128, 128));
-    consider(1, 1, put(128, 3.0, 4.0, 0.23) + (n128 == 1 ? 4.9 + 0.40 * st : n128 == 2 ? 7.6 + 0.90 * st : 4.9 + n128 * (2.4 + 0.453 * st)));
-    consider(2, 1, put(128, 5.8, 6.0, 0.08) + (nsq == 1 ? (fp16 ? 5.5 : 6.2) + 0.73 * st : nsq == 2 ? 9.7 + 1.50 * st : 5.5 + nsq * (3.6 + 0.755 * st)));
+    consider(1, 1, put(128, 0.045, 3.3, 4.0, 0.23) + (n128 == 1 ? 4.9 + 0.40 * st : n128 == 2 ? 7.6 + 0.90 * st : 4.9 + n128 * (2.4 + 0.453 * st)));
+    consider(2, 1, put(128, 0.085, 5.7, 6.0, 0.08) + (nsq == 1 ? (fp16 ? 5.5 : 6.2) + 0.73 * st : nsq == 2 ? 9.7 + 1.50 * st : 5.5 + nsq * (3.6 + 0.755 * st)));
     const double fixed[3] = {8.1, 6.8, 8.9}, slope[3] = {0.99, 1.56, 1.76}, easier[3] = {0.25, 0.18, 0.22};
-    const double ragged[4] = {3.0, 5.5, 7.5, 5.5}, sums[4] = {1.8, 2.8, 3.2, 3.2};      // (the last: 256 and 128)
+    const double within[4] = {0.20, 0.35, 0.40, 0.40}, ragged[4] = {3.0, 5.5, 7.5, 5.5}, sums[4] = {1.8, 2.8, 3.2, 3.2};      // (the last: 256 and 128)
     auto round = [&](int i, double idle) { return fixed[i] + slope[i] * st * (1.0 - easier[i] * idle); };
-    auto put256 = [&](int i) { return odd ? ragged[i] : fp16 ? 0.0 : sums[i] + (N % 4 != 0 ? 6.0 : 0.0); };
+    auto put256 = [&](int i) { return odd ? ragged[i] : fp16 ? (N % 64 != 0 ? within[i] * elements : 0.0) : sums[i] + (N % 4 != 0 ? 6.0 : 0.0); };
     auto reach = [&](int64_t rows) { return qr_e2m3_reach(rows, N, fp16); };
     for (int i = 2; i >= 0; --i) {                          // (ties go to the taller tile)
         if (!reach(128 + 64 * i)) continue;
