@@ -230,10 +230,10 @@ int qr_linear_i4_f16_static(const void* A, const void* sA, const void* W, const 
                             void* stream);
 
 /*
- * Linear4bit.forward (quarot/nn/linear.py:42-56) for prefill shapes on the FP6 matrix path: the same
+ * Linear4bit.forward (quarot/nn/linear.py:42-56) for prefill shapes on 6-bit operands: the same
  * product and the same fp16 epilogue as qr_linear_i4_f16, bit for bit (every int4 code is a value of
- * FP6 E3M2, products and sums stay integers below 2^24, so the fp32 accumulators are exact), at a higher
- * matrix-instruction rate.  Both operands must first be converted to the 6-bit stage-major layout this
+ * FP6 E3M2, products and sums stay integers below 2^24, so the fp32 accumulators are exact).  qr_linear_i4_f16's long prompts
+ * use the same matrix instruction on the packed codes, without a conversion, and are faster.  Both operands must first be converted to the 6-bit stage-major layout this
  * kernel reads; the reference has no counterpart (its CUTLASS call takes the packed nibbles,
  * quarot/kernels/gemm.cu:16-41).
  *   qr_f6_bytes(rows, K): bytes of a converted operand (rows * K * 3 / 4; K % 64 == 0).

@@ -79,12 +79,13 @@ struct Origin {
 // for it inside the loop, or one that lets the epilogue's stores pass the first barrier, costs 6 % of every stage.)
 //
 // What bounds it (256 rows, 32768 x 4096 x 11008): a wave issues an instruction in about 5 cycles, and a sub-step has 20 matrix and 112
-// vector instructions, 8 LDS reads, 4 loads and some 20 others: 55 cycles of 2.05 GHz per accumulator tile and sub-step, where the
-// matrix unit alone would need 36; the clock is the power limit's (2.4 GHz without load).  Inside the loop that is 5.0e15 operations
-// per second (the int8 instruction with nothing else going on sustains 3.9-4.2e15); the whole launch, with about 6 us behind the loop of
-// every tile (3 us of arithmetic with one wave per SIMD, then the compute units write 33 MB at a time), 4.3e15: 690 us against
-// 870-890 of the int8 kernel with the same tiles; 32768 x 11008 x 4096 812 us (1010; 850 with a branch around every store),
-// 8192 x 5120 x 5120 124 (146), 1777 x 8192 x 28672 194 (244), 2048 x 4096 x 11008 53 (58-66).  Delaying the first workgroups by 0 .. 8 us, so
+// vector instructions, 8 LDS reads, 4 loads and some 20 others.  Counters: 61 cycles of 1.9 GHz per accumulator tile and sub-step over the
+// whole launch, 57 without the 6 us behind the loop of every tile (3 us of arithmetic with one wave per SIMD, then the compute units write
+// 33 MB at a time), where the matrix unit alone would need 36: it is busy for 0.60 of the launch, the vector unit for 0.52.  The clock is
+// the power limit's (2.4 GHz without load; 2.2 at K = 4096, where the matrix unit is busy for 0.51).  The whole launch is 4.15-4.3e15
+// operations per second, 7.1e15 being what the matrix instruction sustains on these operands with nothing else going on (the int8 one
+// 3.9-4.2e15): 690-712 us against 870-890 of the int8 kernel with the same tiles; 32768 x 11008 x 4096 812 us (1010; 850 with a branch around
+// every store), 8192 x 5120 x 5120 124 (146), 1777 x 8192 x 28672 195 (244), 2048 x 4096 x 11008 53-54 (58-66).  Delaying the first workgroups by 0 .. 8 us, so
 // that compute units do not write at once, changed nothing.
 template <bool DEQ, bool RAGGED, int BM, int KG, class Place>
 __device__ __forceinline__ void e2m3_tiles(

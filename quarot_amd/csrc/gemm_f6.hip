@@ -4,9 +4,11 @@
 // 8 = 1.0 * 8), every product is an integer of at most 64 and every partial sum an integer below 2^24
 // (K < 131072), so v_mfma_scale_f32_32x32x64_f8f6f4 with both operands as bf6 and unit scales returns
 // the int4 dot product exactly in fp32 -- at about 1.8 times the issue rate of the int8 instruction.
+// (gemm_e2m3.hip has since taken nibbles to E2M3 fields inside the loop, by an offset of 8, and is ahead of this kernel with its
+// conversion at every width: 32768 x 4096 x 11008 712 us against 804, 2048 x 4096 x 11008 54 / 62, 2048 x 8192 x 28672 222 / 236.)
 //
 // The price is the operand format: 6 bits per value, and no cheap way from packed nibbles to packed
-// 6-bit codes inside a GEMM loop.  Operands are therefore converted once (weights when they are
+// signed 6-bit codes inside a GEMM loop.  Operands are therefore converted once (weights when they are
 // loaded, activations by a pass behind the quantiser) into a layout made for this kernel:
 //   X6 / W6: [K / 64 stages][rows][48 bytes]   -- stage-major: the 64 values of a row and stage are 48
 //   contiguous bytes (two MFMA operands of 24 bytes: k 0..31 for lanes 0..31, k 32..63 for lanes 32..63),
