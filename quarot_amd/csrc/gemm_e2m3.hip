@@ -453,8 +453,9 @@ __device__ __forceinline__ void e2m3_tiles(
         slab_store(out, slab, wm * TM + ga(IM - 1) * 32, at.n0 + wn * 128 + gb(JO - 2) * 32, ln);
     } else {
     // int32 sums: four columns of a row per lane and store
+    const int m0 = __builtin_amdgcn_readfirstlane(at.m0);
     const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
-        (void*)(C + (int64_t)at.m0 * N), 0, (int)((u32)(M - at.m0 < BM ? M - at.m0 : BM) * (u32)N * 4u), 0x00020000);
+        (void*)(C + (int64_t)m0 * N), 0, (int)((u32)(M - m0 < BM ? M - m0 : BM) * (u32)N * 4u), 0x00020000);
 #pragma unroll
     for (int i = 0; i < IM; ++i) {
         const u32 row = (u32)(wm * TM + ga(i) * 32 + (ln & 31)) * (u32)N;
