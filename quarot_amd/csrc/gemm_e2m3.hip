@@ -316,7 +316,9 @@ __device__ __forceinline__ void e2m3_tiles(
             f32x16 none;
 #pragma unroll
             for (int v = 0; v < 16; ++v) none[v] = 0.f;
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(0.f, 0.f, none, 0, 0, 0);
+            float zero = 0.f;
+            asm volatile("" : "+v"(zero));                      // (or the compiler makes one tile of zeros and copies it)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(zero, zero, none, 0, 0, 0);
         }
     for (int ks = 0, seg = 0; ks < stages;) {
         const int end = seg + kSegment < stages ? seg + kSegment : stages;      // the accumulators are corrected here
@@ -439,7 +441,9 @@ __device__ __forceinline__ void e2m3_tiles(
                 f16x4 o[2][4];
 #pragma unroll
                 for (int jj = 0; jj < 2; ++jj) {
-                    asm volatile("" : "+a"(acc[i][jb + jj]));                   // (moved out of its registers here, not before)
+                    // (moved out of its registers here, not before; what the K-groups have added up is in vector registers already)
+                    if constexpr (KG == 1) asm volatile("" : "+a"(acc[i][jb + jj]));
+                    else asm volatile("" : "+v"(acc[i][jb + jj]));
 #pragma unroll
                     for (int gq = 0; gq < 4; ++gq)
                         o[jj][gq] = dequant4_f32x64(acc[i][jb + jj][gq * 4], acc[i][jb + jj][gq * 4 + 1], acc[i][jb + jj][gq * 4 + 2],
@@ -461,7 +465,8 @@ __device__ __forceinline__ void e2m3_tiles(
         const u32 row = (u32)(wm * TM + ga(i) * 32 + (ln & 31)) * (u32)N;
 #pragma unroll
         for (int j = 0; j < JO; ++j) {
-            asm volatile("" : "+a"(acc[i][j]));
+            if constexpr (KG == 1) asm volatile("" : "+a"(acc[i][j]));
+            else asm volatile("" : "+v"(acc[i][j]));
 #pragma unroll
             for (int gq = 0; gq < 4; ++gq) {
                 const int col = at.n0 + wn * 128 + gb(j) * 32 + gq * 8 + kh * 4;
