@@ -197,8 +197,12 @@ int qr_linear_i4_f16(const void* A, const void* sA, const void* W, const void* s
  *   workspace: device memory, 16-byte aligned, at least qr_workspace_bytes(M, N, K) bytes; NULL or a
  *   smaller size selects the single-launch path of qr_linear_i4_f16.  Results are identical bit for
  *   bit either way (integer partial sums).  Calls that share a workspace must not overlap.
+ *   qr_linear_spread_bytes: bytes with which it takes a long prompt in two launches that are faster than one, the operand of fewer
+ *   rows spread from 4 to 6 bits per code in the workspace first (three quarters of a byte per code of it; 0: no gain, any M, N, K).
+ *   It is optional: without it the single-launch kernels run, with the same results.
  */
 size_t qr_workspace_bytes(int64_t M, int64_t N, int64_t K);
+size_t qr_linear_spread_bytes(int64_t M, int64_t N, int64_t K);
 /* The kernel (and a second one that adds slices of K, if any) that qr_linear_i4_f16_ws launches for a shape with that much
  * workspace on the current device, as text for reports; NULL for a shape that it refuses.  *scratch_bytes (optional): how much
  * of the workspace they use; a workspace of that size selects the same kernels. */
@@ -270,7 +274,8 @@ int qr_linear_f6_f16(const void* A6, const void* sA, const void* W6, const void*
  *   sW fp16 [N], bias fp16 [N] or NULL -> y fp16 [M, N].
  *   workspace: device memory, 16-byte aligned, at least qr_quantized_linear_workspace_bytes(M, N, K)
  *   bytes (never 0 for M > 0), else QR_E_WORKSPACE.  Calls that share a workspace must not overlap.
- *   Of the qr_workspace_bytes(M, N, K) that it holds for slices of K, only what qr_linear_plan reports as used has to be there.
+ *   Of the qr_workspace_bytes(M, N, K) that it holds for slices of K, only what qr_linear_plan reports as used has to be there;
+ *   qr_linear_spread_bytes(M, N, K) in its place select the kernels that use those.
  */
 size_t qr_quantized_linear_workspace_bytes(int64_t M, int64_t N, int64_t K);
 int qr_quantized_linear_f16(const void* x, int64_t M, int64_t K, int had_K, const void* hadK, int mode,

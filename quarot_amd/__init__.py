@@ -311,11 +311,23 @@ def heads_hadamard_quantize(x, num_heads, clip_ratio=1.0, return_transformed=Fal
 
 @functools.lru_cache(maxsize=4096)
 def _workspace_bytes(M, N, K, device_index=None):
-    # what the library's plan uses of the scratch that it asks for.  (The plan depends on the CURRENT device's compute-unit
-    # count: callers make the device current first, and the device index is part of the cache key)
+    # what the library's plan uses of the scratch that it asks for, and what it would rather have to spread an operand.  (The plan
+    # depends on the CURRENT device's compute-unit count: callers make the device current first, and the device index is part of the
+    # cache key)
     used, L = ctypes.c_size_t(), _lib.lib()
     L.qr_linear_plan(M, N, K, L.qr_workspace_bytes(M, N, K), ctypes.byref(used))
-    return used.value
+    return used.value, L.qr_linear_spread_bytes(M, N, K)
+
+
+def _scratch(fixed, M, N, K, dev):
+    # fixed bytes and those of the product; a GPU too full for a spread operand does without
+    used, spread = _workspace_bytes(M, N, K, dev.index)
+    if spread:
+        try:
+            return torch.empty((fixed + spread,), dtype=torch.uint8, device=dev)
+        except torch.cuda.OutOfMemoryError:
+            pass
+    return torch.empty((fixed + used,), dtype=torch.uint8, device=dev)
 
 
 def linear_i4(x_q, scales_x, weight, weight_scales, bias=None):
@@ -337,12 +349,11 @@ def linear_i4(x_q, scales_x, weight, weight_scales, bias=None):
     y = torch.empty((M, N), dtype=torch.float16, device=dev)
     L = _lib.lib()
     with _lib.on_device(dev):
-        ws_bytes = _workspace_bytes(M, N, K, dev.index)
-        if ws_bytes:
-            # few output tiles: the library splits K across workgroups and needs int32 scratch for the sums
-            ws = torch.empty((ws_bytes,), dtype=torch.uint8, device=dev)
+        # few output tiles: the library splits K across workgroups and needs int32 scratch for the sums; many: it spreads an operand there
+        ws = _scratch(0, M, N, K, dev)
+        if ws.numel():
             _lib.check(L.qr_linear_i4_f16_ws(_ptr(a2), _ptr(sx), _ptr(weight), _ptr(sw), _ptr(bias), M, N, K, _ptr(y),
-                                             _ptr(ws), ws_bytes, _lib.stream_ptr(dev)))
+                                             _ptr(ws), ws.numel(), _lib.stream_ptr(dev)))
         else:
             _lib.check(L.qr_linear_i4_f16(_ptr(a2), _ptr(sx), _ptr(weight), _ptr(sw), _ptr(bias), M, N, K, _ptr(y),
                                           _lib.stream_ptr(dev)))
@@ -385,9 +396,9 @@ def linear_f6(x6, scales_x, weight6, weight_scales, bias=None):
 
 
 @functools.lru_cache(maxsize=4096)
-def _quantized_linear_workspace_bytes(M, N, K, device_index=None):
+def _quantized_linear_fixed_bytes(M, N, K, device_index=None):
     L = _lib.lib()                                                       # (per device, like _workspace_bytes)
-    return L.qr_quantized_linear_workspace_bytes(M, N, K) - L.qr_workspace_bytes(M, N, K) + _workspace_bytes(M, N, K, device_index)
+    return L.qr_quantized_linear_workspace_bytes(M, N, K) - L.qr_workspace_bytes(M, N, K)
 
 
 def quantized_linear(x, weight, weight_scales, bias=None, hadK=None, K=0, clip_ratio=1.0, force_fp32=False):
@@ -419,11 +430,10 @@ def quantized_linear(x, weight, weight_scales, bias=None, hadK=None, K=0, clip_r
     mode = _lib.QR_DTYPE_F32 if force_fp32 else _lib.QR_DTYPE_F16
     signs = _hadamard_sign_words(table, n, int(K)) if K else None
     with _lib.on_device(dev):
-        ws_bytes = _quantized_linear_workspace_bytes(M, N, n, dev.index)
-        ws = torch.empty((max(ws_bytes, 16),), dtype=torch.uint8, device=dev)
+        ws = _scratch(_quantized_linear_fixed_bytes(M, N, n, dev.index), M, N, n, dev)
         call = lambda table, md: _lib.lib().qr_quantized_linear_f16(
             _ptr(x2), M, n, int(K), _ptr(table), md, functional.hadamard.had_scale(n), float(clip_ratio), _ptr(weight),
-            _ptr(sw), _ptr(bias), N, _ptr(y), _ptr(ws), ws_bytes, _lib.stream_ptr(dev))
+            _ptr(sw), _ptr(bias), N, _ptr(y), _ptr(ws), ws.numel(), _lib.stream_ptr(dev))
         rc = _lib.QR_E_UNSUPPORTED
         if signs is not None:
             rc = call(signs, mode | _lib.QR_HADK_SIGNS)                  # (refused before anything is launched)

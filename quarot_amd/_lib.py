@@ -30,6 +30,7 @@ SIGNATURES = {
     "qr_linear_i4_f16": (_int, (_ptr, _ptr, _ptr, _ptr, _ptr, _i64, _i64, _i64, _ptr, _ptr)),
     "qr_linear_plan": (_c.c_char_p, (_i64, _i64, _i64, _c.c_size_t, _ptr)),
     "qr_workspace_bytes": (_c.c_size_t, (_i64, _i64, _i64)),
+    "qr_linear_spread_bytes": (_c.c_size_t, (_i64, _i64, _i64)),
     "qr_quantized_linear_workspace_bytes": (_c.c_size_t, (_i64, _i64, _i64)),
     "qr_quantized_linear_f16": (_int, (_ptr, _i64, _i64, _int, _ptr, _int, _f32, _f32, _ptr, _ptr, _ptr, _i64, _ptr, _ptr,
                                        _c.c_size_t, _ptr)),

@@ -15,7 +15,7 @@ CSRC = PKG / "csrc"
 LIB = PKG / "libquarot_hip.so"
 HOST = PKG / "_host.so"
 OBJ = PKG.parent / "build" / "obj"
-SOURCES = ("api.hip", "quant.hip", "gemm.hip", "gemm_mid.hip", "gemm_e2m3.hip", "gemm_f6.hip", "hadamard.hip", "kv.hip", "attn.hip", "calib.hip", "decode_fused.hip",
+SOURCES = ("api.hip", "quant.hip", "gemm.hip", "gemm_mid.hip", "gemm_e2m3.hip", "gemm_x6.hip", "gemm_f6.hip", "hadamard.hip", "kv.hip", "attn.hip", "calib.hip", "decode_fused.hip",
            "paged_f16.hip")
 FLAGS = ("--offload-arch=gfx950", "-O3", "-fPIC", "-std=c++17", "-fno-gpu-rdc",
          # every fp16/fp32 operation must round on its own (the reference's results are defined that

@@ -1190,6 +1190,7 @@ int ks_split(int64_t M, int64_t N, int64_t Kb) {
 struct MidPlan {
     int kernel;         // 0 .. 2: qr_internal_gemm_mid's shapes; 3 .. 6: qr_internal_gemm_e2m3's; 7: 96 x 64 tiles
     int split;
+    double us;
 };
 MidPlan mid_plan(int64_t M, int64_t N, int64_t Kb, int64_t max_split, bool fp16) {
     const int64_t cus = qr_device().cus;
@@ -1210,13 +1211,9 @@ MidPlan mid_plan(int64_t M, int64_t N, int64_t Kb, int64_t max_split, bool fp16)
         if (n <= 2) return n == 1 ? 3.9 + (heavy ? 0.30 : 0.264) * stages : 4.6 + (heavy ? 0.46 : 0.42) * stages;
         return 3.9 + n * ((n == 3 ? 0.60 : 0.75) + (stream ? 0.25 : n >= 5 && heavy ? 0.23 : 0.21) * stages);
     };
-    MidPlan best{0, 1};
-    double t_best = t64(tiles(64, 64), st) + put(64, 0.07, 3.2, 3.5, 0.19);
+    MidPlan best{0, 1, t64(tiles(64, 64), st) + put(64, 0.07, 3.2, 3.5, 0.19)};
     auto consider = [&](int kernel, int split, double t) {
-        if (t < t_best) {
-            t_best = t;
-            best = MidPlan{kernel, split};
-        }
+        if (t < best.us) best = MidPlan{kernel, split, t};
     };
     const double n96 = loaded(tiles(96, 64));
     consider(7, 1, put(64, 0.4, 3.3, 4.0, 0.5) + (n96 == 1 ? 5.1 + (heavy ? 0.37 : 0.325) * st : n96 == 2 ? 8.0 + (M <= 96 ? 0.85 : 0.69) * st : 5.1 + n96 * (2.0 + 0.335 * st)));
@@ -1244,31 +1241,66 @@ MidPlan mid_plan(int64_t M, int64_t N, int64_t Kb, int64_t max_split, bool fp16)
     return best;
 }
 
-// The kernel that takes a shape, with room for max_split slabs of the output, and the slices of K that it runs in.
-enum class Gemm { large, gemv, shared_tokens, decode, stream64, mid64, mid64x128, mid128, spk, sp192, sp256, sp256_tail, mid96 };
+// The same product with the operand of fewer rows spread in memory first (gemm_x6.hip), by tiles of 256 rows of the other operand and 32 nx of
+// that one, in microseconds: 5.8 + 0.307 per MB that is written, n times (0.26 + 0.675 nx) (1 - 0.23 idle) + (0.406 + 0.144 nx) st (1 - 0.285
+// idle), and 0.25 per million elements where rows of the output start within a line.  Fitted to 2200 shapes of 100 .. 32768 tokens x 512 .. 57344
+// weight rows, 1e9 .. 6e12 operations, all five nx forced (4.2 % rms; the nx taken costs 0.13 % over the best one).  It is ahead of
+// mid_plan's kernels on two thirds of them, from 3e11 operations on nearly always: 1.09 x over all, 1.14 x from there on; the choice between
+// the two costs 0.35 %.  It has to be 0.8 us ahead (nearer than that the estimates err by as much: 1297 x 4096 x 2240 17.2 us without, 18.6 with).
+// What it does not take: rows of the output that are no whole 16-byte pieces, a K of one stage, scratch beyond 512 MiB (a weight of 26000 x 26000).
+struct SpreadPlan {
+    int nx;             // 4 .. 8; 0: not this way
+    double us;
+};
+SpreadPlan spread_plan(int64_t M, int64_t N, int64_t Kb) {
+    SpreadPlan best{0, 0.0};
+    const int64_t rows = N <= M ? N : M, others = N <= M ? M : N, cus = qr_device().cus;
+    const int64_t bytes = (int64_t)qr_internal_x6_bytes(rows, Kb);
+    if (Kb <= 128 || N % 8 != 0 || bytes > (512LL << 20) || !qr_e2m3_reach(256, N, true)) return best;
+    const double st = (double)((Kb + 127) / 128), fixed = 5.8 + 0.307e-6 * (double)bytes + (N % 64 != 0 ? 0.25e-6 * (double)M * (double)N : 0.0);
+    for (int nx = 8; nx >= 4; --nx) {
+        const int64_t tiles = ((others + 255) / 256) * ((rows + 32 * nx - 1) / (32 * nx));
+        const double n = (double)((tiles + cus - 1) / cus), idle = 1.0 - (double)tiles / (n * (double)cus);
+        const double t = fixed + n * ((0.26 + 0.675 * nx) * (1.0 - 0.23 * idle) + (0.406 + 0.144 * nx) * st * (1.0 - 0.285 * idle));
+        if (best.nx == 0 || t < best.us) best = SpreadPlan{nx, t};
+    }
+    return best;
+}
+
+// The kernel that takes a shape, with so many bytes of scratch, and the slices of K that it runs in.  (pieces: the output is 16-byte aligned.)
+enum class Gemm { large, gemv, shared_tokens, decode, stream64, mid64, mid64x128, mid128, spk, sp192, sp256, sp256_tail, mid96, x6 };
 struct GemmPlan {
     Gemm kernel;
-    int split;
+    int split;          // (x6: nx)
+    size_t scratch;
 };
-GemmPlan gemm_plan(int64_t M, int64_t N, int64_t Kb, int64_t max_split, bool fp16) {
+GemmPlan gemm_plan(int64_t M, int64_t N, int64_t Kb, size_t scratch, bool fp16, bool pieces = true) {
     // An operand of 4 GiB or more: every specialised kernel below addresses its operands through 32-bit offsets;
     // the plain tiled kernel computes 64-bit row addresses and takes any shape (rows beyond M or N are clamped).
-    if (M * Kb >= (1LL << 32) || N * Kb >= (1LL << 32)) return GemmPlan{Gemm::large, 1};
+    if (M * Kb >= (1LL << 32) || N * Kb >= (1LL << 32)) return GemmPlan{Gemm::large, 1, 0};
+    const size_t slab = (size_t)M * (size_t)N * 4;
+    const int64_t max_split = scratch ? (int64_t)(scratch / slab) : 1;
+    auto sliced = [&](Gemm kernel, int split) { return GemmPlan{kernel, split, split > 1 ? slab * (size_t)split : 0}; };
     if (M > 64) {
         const MidPlan plan = mid_plan(M, N, Kb, max_split, fp16);
         constexpr Gemm kernels[] = {Gemm::mid64, Gemm::mid64x128, Gemm::mid128, Gemm::spk, Gemm::sp192, Gemm::sp256, Gemm::sp256_tail, Gemm::mid96};
-        return GemmPlan{kernels[plan.kernel], plan.split};
+        const size_t x6 = fp16 && pieces && scratch ? qr_internal_x6_bytes(N <= M ? N : M, Kb) : 0;
+        if (x6 && x6 <= scratch) {
+            const SpreadPlan spread = spread_plan(M, N, Kb);
+            if (spread.nx && spread.us + 0.8 < plan.us) return GemmPlan{Gemm::x6, spread.nx, x6};
+        }
+        return sliced(kernels[plan.kernel], plan.split);
     }
     // one to four tokens: the dot-product kernel -- except two to four tokens against a weight with enough rows for the
     // shared-token kernel, which is ahead there (57344 x 8192: 40.2 against 42.9 us)
     const bool xs = decode_xs_groups((int)N) != 0;
-    if (M == 1 || (M <= 4 && !xs)) return GemmPlan{Gemm::gemv, 1};
+    if (M == 1 || (M <= 4 && !xs)) return GemmPlan{Gemm::gemv, 1, 0};
     const DecodePlan plan = decode_plan(M, N, Kb, max_split);
-    if (plan.tiles) return GemmPlan{Gemm::stream64, plan.split};
+    if (plan.tiles) return sliced(Gemm::stream64, plan.split);
     // weight streaming: with enough groups of 32 rows to fill the CUs the kernel that shares the
     // tokens' codes through LDS (they are read once per workgroup); otherwise the barrier-free
     // kernel in which the waves of a workgroup split K over groups of 32 rows
-    return GemmPlan{xs ? Gemm::shared_tokens : Gemm::decode, 1};
+    return GemmPlan{xs ? Gemm::shared_tokens : Gemm::decode, 1, 0};
 }
 
 int gemm_dispatch(const void* A, const void* B, int64_t M, int64_t N, int64_t K, void* C, void* Y, const void* sA,
@@ -1280,9 +1312,10 @@ int gemm_dispatch(const void* A, const void* B, int64_t M, int64_t N, int64_t K,
     if (((uintptr_t)A & 15) || ((uintptr_t)B & 15)) return QR_E_ALIGN;
     if (Y ? ((uintptr_t)Y & 7) : ((uintptr_t)C & 15)) return QR_E_ALIGN;
     const int m = (int)M, n = (int)N, kb = (int)(K / 2);
-    // the slabs of a K split go to scratch from the caller; without it (or with too little) the single-launch kernels run
+    // the slabs of a K split and a spread operand go to scratch from the caller; without it (or with too little) the single-launch kernels run
     const bool scratch = Y && ws && ((uintptr_t)ws & 15) == 0;
-    const GemmPlan plan = gemm_plan(M, N, kb, scratch ? (int64_t)(ws_bytes / ((size_t)M * (size_t)N * 4)) : 1, Y != nullptr);
+    const GemmPlan plan = gemm_plan(M, N, kb, scratch ? ws_bytes : 0, Y != nullptr, ((uintptr_t)Y & 15) == 0);
+    if (plan.kernel == Gemm::x6) return qr_internal_gemm_x6(plan.split, A, B, m, n, kb, Y, sA, sB, bias, ws, st);
     const int mid = plan.kernel == Gemm::stream64 ? 3 : plan.kernel == Gemm::mid96 ? 4 : (int)plan.kernel - (int)Gemm::mid64;      // qr_internal_gemm_mid's shape
     if (plan.split > 1) {
         const int rc = qr_internal_gemm_mid(mid, A, B, m, n, kb, ws, nullptr, nullptr, nullptr, nullptr, st, plan.split);
@@ -1328,13 +1361,19 @@ extern "C" size_t qr_workspace_bytes(int64_t M, int64_t N, int64_t K) {
     return split > 1 ? (size_t)split * (size_t)M * (size_t)N * 4 : 0;
 }
 
+extern "C" size_t qr_linear_spread_bytes(int64_t M, int64_t N, int64_t K) {
+    if (M <= 64 || N <= 0 || K <= 0 || K % 64 != 0 || K > 131008 || M > 0x7fffffff || N > 0x7fffffff) return 0;
+    const size_t slabs = qr_workspace_bytes(M, N, K), x6 = qr_internal_x6_bytes(N <= M ? N : M, K / 2);
+    const GemmPlan plan = gemm_plan(M, N, K / 2, x6 > slabs ? x6 : slabs, true);
+    return plan.kernel == Gemm::x6 ? plan.scratch : 0;
+}
+
 extern "C" const char* qr_linear_plan(int64_t M, int64_t N, int64_t K, size_t workspace_bytes, size_t* scratch_bytes) {
     if (scratch_bytes) *scratch_bytes = 0;
     if (M <= 0 || N <= 0 || K <= 0 || K % 64 != 0 || K > 131008 || M > 0x7fffffff || N > 0x7fffffff) return nullptr;
-    const size_t slab = (size_t)M * (size_t)N * 4;
-    const GemmPlan plan = gemm_plan(M, N, K / 2, workspace_bytes ? (int64_t)(workspace_bytes / slab) : 1, true);
-    const bool slices = plan.split > 1;
-    if (slices && scratch_bytes) *scratch_bytes = slab * (size_t)plan.split;
+    const GemmPlan plan = gemm_plan(M, N, K / 2, workspace_bytes, true);
+    const bool slices = plan.scratch > 0;
+    if (scratch_bytes) *scratch_bytes = plan.scratch;
     switch (plan.kernel) {
         case Gemm::large: return "gemm_i4_kernel";
         case Gemm::gemv: return "gemv_i4_kernel";
@@ -1349,6 +1388,16 @@ extern "C" const char* qr_linear_plan(int64_t M, int64_t N, int64_t K, size_t wo
         case Gemm::sp192:
         case Gemm::sp256: return "gemm_sp256_kernel";
         case Gemm::sp256_tail: return "gemm_sp256_tail_kernel";
+        case Gemm::x6: {
+            static const char* const names[2][5] = {
+                {"spread_x6_kernel + gemm_x6_kernel<128,256> (x spread)", "spread_x6_kernel + gemm_x6_kernel<160,256> (x spread)",
+                 "spread_x6_kernel + gemm_x6_kernel<192,256> (x spread)", "spread_x6_kernel + gemm_x6_kernel<224,256> (x spread)",
+                 "spread_x6_kernel + gemm_x6_kernel<256,256> (x spread)"},
+                {"spread_x6_kernel + gemm_x6_kernel<256,128> (W spread)", "spread_x6_kernel + gemm_x6_kernel<256,160> (W spread)",
+                 "spread_x6_kernel + gemm_x6_kernel<256,192> (W spread)", "spread_x6_kernel + gemm_x6_kernel<256,224> (W spread)",
+                 "spread_x6_kernel + gemm_x6_kernel<256,256> (W spread)"}};
+            return names[N <= M][plan.split - 4];
+        }
     }
     return nullptr;
 }

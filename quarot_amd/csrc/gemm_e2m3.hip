@@ -10,41 +10,13 @@
 //
 // What it does without: converting signs (the sum of a row's codes costs less, see `ones`), and a second copy of either operand (the
 // format of gemm_f6.hip, 6 bits in memory, moves 1.5 times the bytes through L2 and LDS).
-#include <type_traits>
-#include <utility>
-#include "qr_common.h"
+#include "qr_e2m3.h"
 #include "qr_epilogue.h"
 
 namespace {
 
 typedef int i32x6 __attribute__((ext_vector_type(6)));
 typedef int i32x8 __attribute__((ext_vector_type(8)));
-
-template <int V>
-using IC = std::integral_constant<int, V>;
-template <class F, int... I>
-__device__ __forceinline__ void static_for_seq(F&& f, std::integer_sequence<int, I...>) {
-    (f(IC<I>()), ...);
-}
-// f(0), f(1) .. f(N - 1), the argument a constant of its type: the slots below are far beyond what the compiler unrolls
-template <int N, class F>
-__device__ __forceinline__ void static_for(F&& f) {
-    static_for_seq(f, std::make_integer_sequence<int, N>());
-}
-
-// Row and column of tile `unit` of a grid of tiles: columns of eight row tiles in turn, so that tiles in flight together
-// share rows of both operands in an XCD's L2.
-struct TilePlace {
-    int tm, tn;
-};
-__device__ __forceinline__ TilePlace tile_place(int unit, int tiles_m, int tiles_n) {
-    constexpr int GROUP_M = 8;
-    const int group_sz = GROUP_M * tiles_n;
-    const int g = unit / group_sz;
-    const int gm0 = g * GROUP_M;
-    const int gh = (tiles_m - gm0) < GROUP_M ? (tiles_m - gm0) : GROUP_M;
-    return TilePlace{gm0 + (unit - g * group_sz) % gh, (unit - g * group_sz) / gh};
-}
 
 // Stages (of 256 k) between two corrections of the accumulators by the row sums.  Between them a sum is at most 225 per k over 192 stages
 // on top of the corrected sum of everything before, 64 per k: (225 * 192 + 64 * (512 - 192)) * 256 = 16.3e6 < 2^24 for K up to 131072.
@@ -56,11 +28,6 @@ constexpr int e2m3_lds(int BM, int KG) {
     return KG == 1 ? 2 * (BM + 256) * 128 + 2 * (512 + BM) * 2 + (BM + 256) * 4 + 16384
                    : 3 * (BM + 256) * 128 + (512 + BM) * 2 + 2 * (BM + 256) * 4;
 }
-// First row of A and of B of a tile
-struct Origin {
-    int m0, n0;
-};
-
 // Four waves, ONE per SIMD, each with a wave tile of 128 (96) x 128: 16 (12) accumulator tiles, up to all 256 accumulation registers.
 //   KG = 1   waves 2 (M) x 2 (N), BM = 256 or 192, whole K per wave
 //   KG = 2   waves 2 (N) x 2 (K), BM = 128: the K-groups take alternate pairs of sub-steps and exchange half their accumulators at the end
@@ -182,21 +149,18 @@ __device__ __forceinline__ void e2m3_tiles(
         p.f[f] = *(const u32x4*)(lds + (base[u][base_of(f)] + buf_off) + dist_of(f));
     };
 
-    // Spreading: two words x, y (16 nibbles) -> 96 bits of sixteen 6-bit fields, in seven instructions.  Fields start at bits 0, 6, 12 ..
-    // of the 96, which are bits {0, 12, 24 | 6, 18, 30}, {4, 16, 28 | 10, 22, (30)} and {8, 20 | 2, 14, 26} of the three words: the first of each
-    // are where x has its nibbles 0, 3, 6 / 1, 4, 7 / 2, 5, the others where y rotated left by 2 has its.  Which k lands where is
-    // the same for both operands, and no sum depends on it.  Each word: (x & mask) ^ top bits of its eight nibbles' places, then
+    // Spreading (qr_e2m3.h), seven instructions per two words: y rotated by 2, then for each word (x & mask) ^ top bits of its eight nibbles' places, then
     // ^ (rotated y & mask), one v_bitop3_b32 each (one operand may be scalar: the masks of x are held in vector registers).
     u32 x0, x1, x2, y0, y1, y2, c0, c1, c2;
-    asm("v_mov_b32 %0, 0x0F00F00F" : "=v"(x0));
-    asm("v_mov_b32 %0, 0xF00F00F0" : "=v"(x1));
-    asm("v_mov_b32 %0, 0x00F00F00" : "=v"(x2));
-    asm("s_mov_b32 %0, 0xC03C03C0" : "=s"(y0));
-    asm("s_mov_b32 %0, 0x03C03C03" : "=s"(y1));
-    asm("s_mov_b32 %0, 0x3C03C03C" : "=s"(y2));
-    asm("s_mov_b32 %0, 0x08208208" : "=s"(c0));
-    asm("s_mov_b32 %0, 0x82082082" : "=s"(c1));
-    asm("s_mov_b32 %0, 0x20820820" : "=s"(c2));
+    asm("v_mov_b32 %0, %1" : "=v"(x0) : "n"(kSpreadX[0]));
+    asm("v_mov_b32 %0, %1" : "=v"(x1) : "n"(kSpreadX[1]));
+    asm("v_mov_b32 %0, %1" : "=v"(x2) : "n"(kSpreadX[2]));
+    asm("s_mov_b32 %0, %1" : "=s"(y0) : "n"(kSpreadY[0]));
+    asm("s_mov_b32 %0, %1" : "=s"(y1) : "n"(kSpreadY[1]));
+    asm("s_mov_b32 %0, %1" : "=s"(y2) : "n"(kSpreadY[2]));
+    asm("s_mov_b32 %0, %1" : "=s"(c0) : "n"(kSpreadFlip[0]));
+    asm("s_mov_b32 %0, %1" : "=s"(c1) : "n"(kSpreadFlip[1]));
+    asm("s_mov_b32 %0, %1" : "=s"(c2) : "n"(kSpreadFlip[2]));
     // the order in which a sub-step's fragments are spread (and read again)
     constexpr int order4[8] = {0, 2, 1, 3, 4, 6, 5, 7}, order3[7] = {0, 2, 1, 3, 5, 4, 6};
     auto frag_at = [&](int t) { return IM == 4 ? order4[t] : order3[t]; };
@@ -450,11 +414,11 @@ __device__ __forceinline__ void e2m3_tiles(
                                                     acc[i][jb + jj][gq * 4 + 3], sa, sbh[jj][gq], bih[jj][gq]);
                 }
                 if (jb + i > 0)
-                    slab_store(out, slab, wm * TM + ga(i > 0 ? i - 1 : IM - 1) * 32, at.n0 + wn * 128 + gb(i > 0 ? jb : jb - 2) * 32, ln);
+                    slab_store(out, slab, N, wm * TM + ga(i > 0 ? i - 1 : IM - 1) * 32, at.n0 + wn * 128 + gb(i > 0 ? jb : jb - 2) * 32, ln);
                 slab = slab_turn(region, o, ln);
             }
         }
-        slab_store(out, slab, wm * TM + ga(IM - 1) * 32, at.n0 + wn * 128 + gb(JO - 2) * 32, ln);
+        slab_store(out, slab, N, wm * TM + ga(IM - 1) * 32, at.n0 + wn * 128 + gb(JO - 2) * 32, ln);
     } else {
     // int32 sums: four columns of a row per lane and store
     const int m0 = __builtin_amdgcn_readfirstlane(at.m0);

@@ -319,14 +319,26 @@ bool weight_args(PyObject* w, PyObject* s, PyObject* b, int64_t half_k, int devi
     return out->N > 0 && out->s->numel() == out->N && (!out->b || out->b->numel() == out->N);
 }
 
-// What the library asks for as scratch of the product of a shape, and what its plan uses of it.
+// What the library asks for as scratch of the product of a shape, what its plan uses of it, and what it would rather have to spread an operand.
 struct Slabs {
-    size_t asked, used;
+    size_t asked, used, spread;
 };
 Slabs slab_bytes(int64_t M, int64_t N, int64_t K) {
-    Slabs s{qr_workspace_bytes(M, N, K), 0};
+    Slabs s{qr_workspace_bytes(M, N, K), 0, qr_linear_spread_bytes(M, N, K)};
     if (s.asked) qr_linear_plan(M, N, K, s.asked, &s.used);
     return s;
+}
+// `fixed` bytes and those of the product, at least 16; *bytes: how many.  A GPU too full for a spread operand does without.
+at::Tensor scratch(size_t fixed, const Slabs& s, int device, size_t* bytes) {
+    if (s.spread) {
+        try {
+            *bytes = fixed + s.spread;
+            return fresh({(int64_t)*bytes}, kByte, device);
+        } catch (const c10::OutOfMemoryError&) {
+        }
+    }
+    *bytes = fixed + s.used;
+    return *bytes ? fresh({(int64_t)(*bytes < 16 ? 16 : *bytes)}, kByte, device) : at::Tensor();
 }
 
 // linear(codes, scales, weight, weight_scales, bias or None) -> y
@@ -340,11 +352,12 @@ PyObject* linear(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
     if (sx->numel() != M || !weight_args(a[2], a[3], a[4], half_k, device, &w)) return none();
     c10::SmallVector<int64_t, 6> sizes(q->sizes().begin(), q->sizes().end());
     sizes.back() = w.N;
-    const size_t need = slab_bytes(M, w.N, half_k * 2).used;
-    at::Tensor y, ws;                                       // (ws: few output tiles, room for the slabs of a K split)
+    const Slabs slabs = slab_bytes(M, w.N, half_k * 2);
+    at::Tensor y, ws;
     const auto call = [&] {
+        size_t need;
         y = fresh(sizes, kHalf, device);
-        if (need) ws = fresh({(int64_t)need}, kByte, device);
+        ws = scratch(0, slabs, device, &need);
         return qr_linear_i4_f16_ws(q->data_ptr(), sx->data_ptr(), w.w->data_ptr(), w.s->data_ptr(), ptr(w.b), M, w.N, half_k * 2,
                                    y.data_ptr(), need ? ws.data_ptr() : nullptr, need, stream(device));
     };
@@ -368,11 +381,11 @@ PyObject* quantized_linear(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
     c10::SmallVector<int64_t, 6> sizes(r.x->sizes().begin(), r.x->sizes().end());
     sizes.back() = w.N;
     const Slabs slabs = slab_bytes(r.rows, w.N, r.n);
-    const size_t need = qr_quantized_linear_workspace_bytes(r.rows, w.N, r.n) - slabs.asked + slabs.used;
     at::Tensor y, ws;
     const auto call = [&] {
+        size_t need;
         y = fresh(sizes, kHalf, r.device);
-        ws = fresh({(int64_t)(need < 16 ? 16 : need)}, kByte, r.device);
+        ws = scratch(qr_quantized_linear_workspace_bytes(r.rows, w.N, r.n) - slabs.asked, slabs, r.device, &need);
         return qr_quantized_linear_f16(r.x->data_ptr(), r.rows, r.n, (int)K, ptr(table), (int)mode, (float)scale, (float)clip,
                                        w.w->data_ptr(), w.s->data_ptr(), ptr(w.b), w.N, y.data_ptr(), ws.data_ptr(), need,
                                        stream(r.device));

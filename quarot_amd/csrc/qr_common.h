@@ -124,7 +124,7 @@ int qr_internal_gemm_e2m3(int shape, const void* A, const void* B, int M, int N,
 
 // gemm_x6.hip: the same with the operand of fewer rows spread in memory first, into qr_internal_x6_bytes(min(M, N), Kb) of scratch
 size_t qr_internal_x6_bytes(int64_t rows, int64_t Kb);
-int qr_internal_gemm_x6(const void* A, const void* B, int M, int N, int Kb, void* Y, const void* sA, const void* sB, const void* bias,
+int qr_internal_gemm_x6(int nx, const void* A, const void* B, int M, int N, int Kb, void* Y, const void* sA, const void* sB, const void* bias,
                         void* scratch, hipStream_t st);
 static inline int qr_launch_status() {
     hipError_t e = hipGetLastError();

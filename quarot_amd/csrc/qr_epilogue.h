@@ -85,13 +85,13 @@ __device__ __forceinline__ SlabOut slab_out(f16* Y, int m0, int rows, int N, int
     return SlabOut{__builtin_amdgcn_make_buffer_rsrc((void*)(Y + (int64_t)m0 * N), 0, (int)((u32)rows * (u32)N * 2u), 0x00020000),
                    ((u32)(lane >> 3) * (u32)N + (u32)((lane & 7) * 8)) * 2u, N, (N & 7) == 0 && (((uintptr_t)Y) & 15) == 0, (N & 3) == 0};
 }
-// rows from `row` of the tile on, columns from col0 of the output on.  A caller that has looked at out.wide says so in WIDE (0 / 1), so that
+// rows from `row` of the tile on, columns from col0 of the output up to `end`.  A caller that has looked at out.wide says so in WIDE (0 / 1), so that
 // the code of whole pieces stands by itself.
 template <int WIDE = -1>
-__device__ __forceinline__ void slab_store(const SlabOut& out, const Slab& s, int row, int col0, int lane) {
+__device__ __forceinline__ void slab_store(const SlabOut& out, const Slab& s, int end, int row, int col0, int lane) {
     constexpr u32 GONE = 0xFFFFFF00u;           // beyond the range of every buffer here
     const u32 at = out.lane_at + ((u32)row * (u32)out.N + (u32)col0) * 2u, rows8 = (u32)out.N * 16u;
-    const int left = out.N - col0 - (lane & 7) * 8;         // columns from the piece on
+    const int left = end - col0 - (lane & 7) * 8;           // columns from the piece on
     // (nontemporal: the output is not read again by this launch, and written this way it disturbs the operands in L2 less --
     // measured 1-4 % off whole GEMM launches at 2048 and 32768 tokens)
     if (WIDE == 1 || (WIDE < 0 && out.wide)) {
@@ -155,6 +155,41 @@ __device__ __forceinline__ f16x4 dequant4_f32x64(float a0, float a1, float a2, f
     const f16x2 y01 = (s2 * f16x2{sb[0], sb[1]}) * q01 + f16x2{bi[0], bi[1]};
     const f16x2 y23 = (s2 * f16x2{sb[2], sb[3]}) * q23 + f16x2{bi[2], bi[3]};
     return f16x4{y01[0], y01[1], y23[0], y23[1]};
+}
+
+// A slab of two accumulator tiles, likewise.  One wave per SIMD has nobody to hide a chain of five dependent instructions behind: the 32
+// values go through each step together (in chains the slab took 1200 cycles, 8 per instruction).  No addition where there is no bias.
+__device__ __forceinline__ void dequant_slab_f32x64(const f32x16& a0, const f32x16& a1, f16 sa, const f16x4 (&sb)[2][4], const f16x4 (&bi)[2][4],
+                                                    bool with_bias, f16x4 (&o)[2][4]) {
+    const f16x2 s2 = {sa, sa}, x64 = {(f16)64.0f, (f16)64.0f};
+    float v[32];
+#pragma unroll
+    for (int k = 0; k < 32; ++k) {
+        v[k] = k < 16 ? a0[k] : a1[k - 16];
+        asm volatile("" : "+v"(v[k]));
+    }
+    f16x2 q[16], s[16];
+#pragma unroll
+    for (int k = 0; k < 16; ++k) q[k] = as_f16x2(cvt_f16x2(v[2 * k], v[2 * k + 1]));
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int k = 0; k < 16; ++k) {
+        const f16x4 b = sb[k >> 3][(k >> 1) & 3];
+        s[k] = s2 * ((k & 1) ? f16x2{b[2], b[3]} : f16x2{b[0], b[1]});
+        q[k] = q[k] * x64;
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int k = 0; k < 16; ++k) q[k] = s[k] * q[k];
+    if (with_bias) {
+#pragma unroll
+        for (int k = 0; k < 16; ++k) {
+            const f16x4 b = bi[k >> 3][(k >> 1) & 3];
+            q[k] = q[k] + ((k & 1) ? f16x2{b[2], b[3]} : f16x2{b[0], b[1]});
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < 8; ++k) o[k >> 2][k & 3] = f16x4{q[2 * k][0], q[2 * k][1], q[2 * k + 1][0], q[2 * k + 1][1]};
 }
 
 }  // namespace
