@@ -163,8 +163,9 @@ __device__ __forceinline__ void merge_states(const float* src, int splits, int d
 // ALIGNED: page_size is a multiple of 16, so the 16 positions of a wave step lie in one page.
 // NW: waves per workgroup (4, 8 or 16): a (sequence, head) gets NW * splits waves in all.
 // APPEND: the sequence's LAST position is the token of this step, and its key and value arrive as fp16 vectors
-// (knew, vnew: [batch, heads, 128]) instead of lying in the cache already: the first two waves of the (sequence, head)
-// quantise the key and the value (kv_quant_one_vector: the bits of the quantise-and-append kernel), write codes and
+// (knew, vnew: [batch, heads, 128]) instead of lying in the cache already: the last two waves of the (sequence, head), which
+// have no more of the cache to walk than the others and often less, quantise the key and the value (kv_quant_one_vector: the
+// bits of the quantise-and-append kernel) while their first loads are on the way, write codes and
 // parameters to the position's page slot, and leave the position's logit and its dequantised value in LDS as one more
 // softmax state for the merge; the walk over the cache stops one position short.  A decode step is then ONE launch
 // instead of append + attention.
@@ -180,7 +181,7 @@ __global__ __launch_bounds__(64 * NW, (NW == 16 ? 1 : NW == 8 ? 2 : 4)) void pag
     int q_had, u32* __restrict__ arrived, const u32x4* __restrict__ knew = nullptr, const u32x4* __restrict__ vnew = nullptr,
     int k_had = 0) {
     __shared__ f32x4 st4[NW * 33];                         // per wave: [m, d, -, -], 128 outputs; before that the query (256 bytes)
-    __shared__ u32x4 fresh[APPEND ? 2 * 16 : 1];           // APPEND: staging of the quantising waves, then their codes
+    __shared__ u32x4 fresh[APPEND ? 2 * 16 : 1];           // APPEND: staging of the quantising waves, then the key's codes
     __shared__ float newv[APPEND ? 128 + 2 : 1];           // APPEND: the new position's value and its [m, d]
     float* const st = (float*)st4;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -188,9 +189,10 @@ __global__ __launch_bounds__(64 * NW, (NW == 16 ? 1 : NW == 8 ? 2 : 4)) void pag
     const int bh = blockIdx.x / splits, sp = blockIdx.x - bh * splits;
     const int b = bh / c.num_heads, h = bh - b * c.num_heads;
     const u32 qword = ((const u32*)q)[(int64_t)bh * 64 + lane];          // dimensions 2 lane, 2 lane + 1
-    const bool appends = APPEND && sp == 0 && wave < 2;     // wave-uniform; wave 0: the key, wave 1: the value
+    const bool owns_new = APPEND && sp == splits - 1;       // uniform; of this workgroup's waves the last: the key, the last but one: the value
+    const bool appends = owns_new && wave >= NW - 2;
     u32x4 piece = {0, 0, 0, 0};
-    if (APPEND && appends) piece = (wave == 0 ? knew : vnew)[(int64_t)bh * 16 + (lane & 15)];
+    if (APPEND && appends) piece = (wave == NW - 1 ? knew : vnew)[(int64_t)bh * 16 + (lane & 15)];
     const int p0 = c.indptr[b], npages = c.indptr[b + 1] - p0;
     const int seq_all = npages > 0 ? (npages - 1) * c.page_size + c.last_page_offset[b] : 0;
     const int seq_len = APPEND ? seq_all - 1 : seq_all;     // positions read from the cache
@@ -223,10 +225,7 @@ __global__ __launch_bounds__(64 * NW, (NW == 16 ? 1 : NW == 8 ? 2 : 4)) void pag
     // ALIGNED: chunk g lies in page g / cpp at entry 16 (g % cpp); both advance without divisions
     const int cpp = ALIGNED ? c.page_size >> 4 : 1;
     const int it_step = stride / cpp, r_step = stride - it_step * cpp;
-    // APPEND: the wave that quantises the key leaves its first two chunks (one step's worth) to waves 2 and 3, which take
-    // one each after their own walk: its extra work would otherwise stand at the launch's end
-    const int g_first = sp * NW + wave;
-    int g = g_first + ((APPEND && appends && wave == 0) ? stride * AU : 0);
+    int g = sp * NW + wave;
     int it_u = g / cpp, r_u = g - it_u * cpp;
     // Two sets of AU positions per lane group: the loads of the next set are issued before the current
     // one is consumed, so their latency hides under the arithmetic.  Loads are unconditional (a position
@@ -289,7 +288,15 @@ __global__ __launch_bounds__(64 * NW, (NW == 16 ? 1 : NW == 8 ? 2 : 4)) void pag
         }
     };
     Step sa, sb;
-    if (!appends) issue(sa, g);                             // (the quantising waves: behind their quantiser, which needs the registers)
+    int new_page = -1, new_entry = 0;                       // the new token's place
+    if (appends) {
+        const int pos = seq_all - 1, it = pos / c.page_size;
+        new_entry = pos - it * c.page_size;
+        // (a scalar load: a vector load's wait would include the first step's, and the quantiser is to run under their latency)
+        const int32_t* const from = c.indices + p0 + __builtin_amdgcn_readfirstlane(it);
+        asm volatile("s_load_dword %0, %1, 0x0\n\ts_waitcnt lgkmcnt(0)" : "=&s"(new_page) : "s"(from) : "memory");
+    }
+    issue(sa, g);
     __builtin_amdgcn_sched_barrier(0);
 
     // The query, with the Hadamard over the head dimension (matmul_had_cuda on q, kv_cache.py:30-33,113) here instead of in
@@ -356,44 +363,29 @@ __global__ __launch_bounds__(64 * NW, (NW == 16 ? 1 : NW == 8 ? 2 : 4)) void pag
     };
 
     if (APPEND && appends) {
-        u32 W[8];
-        f16 sc, zp;
-        const int pos = seq_all - 1, it = pos / c.page_size, entry = pos - it * c.page_size;
-        const int64_t page = c.indices[p0 + it];
-        const bool page_ok = page >= 0 && page < c.num_pages;
-        const float hs = 0.08838834764831845f;                 // 1 / sqrt(128)
-        u32x4* const stage = fresh + wave * 16;
-        if (wave == 0 && k_had) kv_quant_one_vector<true>(piece, stage, hs, W, sc, zp);
-        else kv_quant_one_vector<false>(piece, stage, hs, W, sc, zp);
-        const u32 prm = pack_scale_zero(sc, zp);
-        const int hh = lane >> 5;
-        if ((lane & 31) == 0) {
-            const u32x4 c0 = {W[0], W[1], W[2], W[3]}, c1 = {W[4], W[5], W[6], W[7]};
-            stage[2 * hh] = c0;                                // the position's 64 code bytes, for its own turn below
-            stage[2 * hh + 1] = c1;
-            if (page_ok) {
-                const int64_t s = paged_slot(c, page, wave, h, entry);
-                u32x4* dst = (u32x4*)c.data + s * 4 + 2 * hh;
-                dst[0] = c0;
-                dst[1] = c1;
-                if (hh == 0) c.param[s] = prm;
-            }
+        const bool page_ok = new_page >= 0 && new_page < c.num_pages, key = wave == NW - 1;
+        u32x4* const stage = fresh + (key ? 16 : 0);
+        const OneVector r = kv_quant_one_vector(piece, stage, key && k_had, 0.08838834764831845f);      // 1 / sqrt(128)
+        const u32 prm = pack_scale_zero(r.sc, r.zp);
+        if (page_ok) {
+            const int64_t s = paged_slot(c, new_page, key ? 0 : 1, h, new_entry);
+            c.data[s * 64 + r.at] = (uint8_t)r.byte;
+            if (lane == 0) c.param[s] = prm;
         }
-        __builtin_amdgcn_wave_barrier();
-        if (wave == 0) {
+        if (key) {
+            ((uint8_t*)stage)[r.at] = (uint8_t)r.byte;
+            __builtin_amdgcn_wave_barrier();
             const float lg = logit(stage[c4], prm);
             if (lane == 0) {
                 newv[128] = page_ok ? lg : -__builtin_inff();
                 newv[129] = page_ok ? 1.f : 0.f;
             }
         } else {
-            const u32 byte = ((const uint8_t*)stage)[lane];
-            const float z = page_ok ? (float)zp : 0.f, s = page_ok ? (float)sc : 0.f;
-            newv[2 * lane] = (float)(byte & 15u) * s - z;
-            newv[2 * lane + 1] = (float)(byte >> 4) * s - z;
+            const float z = page_ok ? (float)r.zp : 0.f, s = page_ok ? (float)r.sc : 0.f;
+            newv[2 * r.at] = (float)(r.byte & 15u) * s - z;
+            newv[2 * r.at + 1] = (float)(r.byte >> 4) * s - z;
         }
         __builtin_amdgcn_sched_barrier(0);
-        issue(sa, g);
     }
 
     float m = -5e4f, d = 0.f, pz = 0.f, psum = 0.f, acc[32];
@@ -441,25 +433,23 @@ __global__ __launch_bounds__(64 * NW, (NW == 16 ? 1 : NW == 8 ? 2 : 4)) void pag
         }
     };
     const int gs = stride * AU;
+    // Of the waves on a SIMD the oldest is served first: at 32 x 4001 x 8 heads waves 0 .. 3 were through their walk 4.5 us before 4 .. 7,
+    // which then had the memory to themselves without the loads in flight that it takes to fill it.  With precedence for the later ones in half
+    // of the loop 3.5 us remain.  28.5 -> 28.0 us; 1 x 2048 x 32 heads 8.8 -> 8.4, where the later waves also start later.  (Precedence throughout
+    // turns the order round; by the turns that a wave and its partner have made, all end together and the launch is 2 us longer: in
+    // step, both wait for memory and then both compute.)
+    const bool late = NW > 4 && wave >= NW / 2;
     for (; g < chunks; g += 2 * gs) {
+        if (late) __builtin_amdgcn_s_setprio(1);
         issue(sb, g + gs);
         __builtin_amdgcn_sched_barrier(0);                 // the compiler would otherwise sink the loads below the arithmetic
         consume(sa);
         __builtin_amdgcn_sched_barrier(0);
+        if (late) __builtin_amdgcn_s_setprio(0);
         issue(sa, g + 2 * gs);
         __builtin_amdgcn_sched_barrier(0);
         if (g + gs < chunks) consume(sb);                  // (no loads inside: the branch does not disturb the wait counts)
         __builtin_amdgcn_sched_barrier(0);
-    }
-    if (APPEND && sp == 0 && (wave == 2 || wave == 3)) {
-        const int extra = wave == 3 ? stride : 0;                       // the first wave's first or second chunk
-        if (extra < chunks) {
-            it_u = extra / cpp;
-            r_u = extra - it_u * cpp;
-            issue(sb, extra);
-            sb.ok[1] = false;                                           // (the step's second chunk is not this wave's)
-            consume(sb);
-        }
     }
     // ---- merge.  Every lane first takes the remaining bias and the zero points out of its own sums -- sum p (scale code -
     // zero) remains --, so that no step of the merge rounds at the biased sums' magnitude.  (Taken out behind the merge, the
@@ -509,7 +499,7 @@ __global__ __launch_bounds__(64 * NW, (NW == 16 ? 1 : NW == 8 ? 2 : 4)) void pag
             M = __builtin_fmaxf(M, sm_[k]);
         }
         float nm = -__builtin_inff();
-        if (APPEND && sp == 0) {
+        if (owns_new) {
             nm = newv[128];
             M = __builtin_fmaxf(M, nm);
         }
@@ -520,7 +510,7 @@ __global__ __launch_bounds__(64 * NW, (NW == 16 ? 1 : NW == 8 ? 2 : 4)) void pag
             D = __builtin_fmaf(st[k * 132 + 1], w, D);
             O = __builtin_fmaf(st[k * 132 + 4 + dim], w, O);
         }
-        if (APPEND && sp == 0) {
+        if (owns_new) {
             const float w = __builtin_amdgcn_exp2f(nm - M) * newv[129];
             D += w;
             O = __builtin_fmaf(newv[dim], w, O);

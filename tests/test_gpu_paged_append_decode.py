@@ -68,6 +68,36 @@ def test_append_and_attention_in_one_launch(page_size, lens, heads, hadamard):
                                                     2, layer, heads, page_size, 128, B, 0, None, 0, None) == -5
 
 
+@pytest.mark.parametrize("hadamard", [True, False])
+def test_the_new_tokens_codes_come_from_every_lane_of_its_wave(hadamard):
+    """Keys and values that tell the positions of a vector apart (one value in turn at each of the 128), vectors of both zeros, of ranges around
+    the smallest normal scale and below, and of infinities and NaNs in one place each: pages as quantise-and-append stores them."""
+    rng = np.random.default_rng(3)
+    heads, B, page_size = 16, 24, 16
+    vecs = rng.standard_normal((B * heads, 128)).astype(F16)
+    for i in range(128):
+        vecs[i], vecs[i, i] = rng.standard_normal(128) * 0.05, 4.0 + i / 64
+        vecs[128 + i] = (rng.standard_normal(128) * 2.0 ** -(8 + i / 8)).astype(F16)
+    vecs[256:272] = np.where(rng.random((16, 128)) < 0.5, F16(0.0), F16(-0.0))
+    vecs[272:288, 0] = 0
+    vecs[272:288, 1:] = np.abs(vecs[272:288, 1:]) * F16(-1) ** (np.arange(16) % 2)[:, None].astype(F16)
+    for i, special in enumerate([np.inf, -np.inf, np.nan, 65504]):
+        for j in range(8):
+            vecs[288 + 8 * i + j, 17 * j + 5] = special
+    k = vecs.reshape(B, heads, 128)
+    v = vecs[::-1].copy().reshape(B, heads, 128)
+    lens = [int(n) for n in rng.integers(1, 70, B)]
+    data, param, indptr, indices, last = paged_case(rng, heads, page_size, lens, layers=1)
+    tabs, q = (gpu(indptr), gpu(indices), gpu(last)), gpu((rng.standard_normal((B, heads, 128)) * 2).astype(F16))
+    gd2, gp2 = gpu(data), gpu(param)
+    kv.quantize_append_kv_i4(gd2, gp2, *tabs, gpu(k), gpu(v), None, 0, hadamard=hadamard)
+    for hint in (0, max(lens), 2000):                        # workgroups of different sizes, split or not
+        gd1, gp1, out = gpu(data), gpu(param), torch.empty_like(q)
+        kv.batch_decode_i4(out, q, gd1, gp1, *tabs, 0, max_seq_len=hint, q_hadamard=True, append=(gpu(k), gpu(v), hadamard))
+        assert torch.equal(gd1, gd2), hint
+        assert torch.equal(gp1.view(torch.int16), gp2.view(torch.int16)), hint
+
+
 def test_cache_class_holds_the_token_for_the_attention_call_and_never_shows_a_stale_cache():
     """update() of a decode step hands the token to the attention call; reading the pages, asking for the tables or
     updating again before that call stores it first; a second call of the returned callable is plain attention."""
