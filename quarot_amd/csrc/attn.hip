@@ -177,24 +177,27 @@ __device__ __forceinline__ void merge_states(const float* src, int splits, int d
 // states remain.
 template <bool ALIGNED, int NW, bool APPEND = false>
 __global__ __launch_bounds__(64 * NW, (NW == 16 ? 1 : NW == 8 ? 2 : 4)) void paged_decode_i4_kernel(
-    const f16* __restrict__ q, PagedKV c, f16* __restrict__ o, float sm_scale_log2, int splits, float* __restrict__ part,
-    int q_had, u32* __restrict__ arrived, const u32x4* __restrict__ knew = nullptr, const u32x4* __restrict__ vnew = nullptr,
-    int k_had = 0) {
+    const f16* __restrict__ q, const int32_t* __restrict__ indptr, const int32_t* __restrict__ last_page_offset, const int32_t* __restrict__ indices,
+    const u32x4* __restrict__ knew, const u32x4* __restrict__ vnew, u32 heads_inverse, u32 page_inverse, u32 shifts, PagedKV c, f16* __restrict__ o,
+    float sm_scale_log2, float* __restrict__ part, int q_had, u32* __restrict__ arrived, int k_had) {
+    // (the arguments that the first loads wait for stand first: they arrive with the waves)
     __shared__ f32x4 st4[NW * 33];                         // per wave: [m, d, -, -], 128 outputs; before that the query (256 bytes)
     __shared__ u32x4 fresh[APPEND ? 2 * 16 : 1];           // APPEND: staging of the quantising waves, then the key's codes
     __shared__ float newv[APPEND ? 128 + 2 : 1];           // APPEND: the new position's value and its [m, d]
     float* const st = (float*)st4;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int slot = lane >> 2, c4 = lane & 3;
-    const int bh = blockIdx.x / splits, sp = blockIdx.x - bh * splits;
-    const int b = bh / c.num_heads, h = bh - b * c.num_heads;
+    const int splits = 1 << (shifts & 31), bh = blockIdx.x >> (shifts & 31), sp = blockIdx.x & (splits - 1);
+    const int b = (int)(__umulhi((u32)bh << 2, heads_inverse) >> (shifts >> 16)), h = bh - b * c.num_heads;
     const u32 qword = ((const u32*)q)[(int64_t)bh * 64 + lane];          // dimensions 2 lane, 2 lane + 1
     const bool owns_new = APPEND && sp == splits - 1;       // uniform; of this workgroup's waves the last: the key, the last but one: the value
     const bool appends = owns_new && wave >= NW - 2;
     u32x4 piece = {0, 0, 0, 0};
     if (APPEND && appends) piece = (wave == NW - 1 ? knew : vnew)[(int64_t)bh * 16 + (lane & 15)];
-    const int p0 = c.indptr[b], npages = c.indptr[b + 1] - p0;
-    const int seq_all = npages > 0 ? (npages - 1) * c.page_size + c.last_page_offset[b] : 0;
+    const int p0 = indptr[b], npages = indptr[b + 1] - p0;
+    int last = last_page_offset[b];
+    asm volatile("" : "+s"(last));                          // (requested along with the others, not behind the look at npages)
+    const int seq_all = npages > 0 ? (npages - 1) * c.page_size + last : 0;
     const int seq_len = APPEND ? seq_all - 1 : seq_all;     // positions read from the cache
     if (npages <= 0) {
         // A sequence without pages (uniform over the workgroups of the pair): nothing may be read -- its slice of kv_indices
@@ -224,9 +227,10 @@ __global__ __launch_bounds__(64 * NW, (NW == 16 ? 1 : NW == 8 ? 2 : 4)) void pag
     const int stride = NW * splits;                         // chunks between the steps of one wave
     // ALIGNED: chunk g lies in page g / cpp at entry 16 (g % cpp); both advance without divisions
     const int cpp = ALIGNED ? c.page_size >> 4 : 1;
-    const int it_step = stride / cpp, r_step = stride - it_step * cpp;
+    auto pages = [&](int n) { return ALIGNED ? (int)(__umulhi((u32)n << 2, page_inverse) >> (shifts >> 8 & 255)) : n; };       // n / cpp
+    const int it_step = pages(stride), r_step = stride - it_step * cpp;
     int g = sp * NW + wave;
-    int it_u = g / cpp, r_u = g - it_u * cpp;
+    int it_u = pages(g), r_u = g - it_u * cpp;
     // Two sets of AU positions per lane group: the loads of the next set are issued before the current
     // one is consumed, so their latency hides under the arithmetic.  Loads are unconditional (a position
     // beyond the sequence reads entry 0 of a valid page and is masked), which keeps the loop free of
@@ -259,7 +263,7 @@ __global__ __launch_bounds__(64 * NW, (NW == 16 ? 1 : NW == 8 ? 2 : 4)) void pag
                 entry[u] = pos - it * c.page_size;
             }
             t.ok[u] = pos < seq_len && it < npages;
-            pp[u] = c.indices + p0 + (it < npages ? it : 0);
+            pp[u] = indices + p0 + (it < npages ? it : 0);
             if (!ALIGNED) page[u] = *pp[u];
         }
         if (ALIGNED) {
@@ -290,10 +294,10 @@ __global__ __launch_bounds__(64 * NW, (NW == 16 ? 1 : NW == 8 ? 2 : 4)) void pag
     Step sa, sb;
     int new_page = -1, new_entry = 0;                       // the new token's place
     if (appends) {
-        const int pos = seq_all - 1, it = pos / c.page_size;
+        const int pos = seq_all - 1, it = ALIGNED && pos >= 0 ? pages(pos >> 4) : pos / c.page_size;
         new_entry = pos - it * c.page_size;
         // (a scalar load: a vector load's wait would include the first step's, and the quantiser is to run under their latency)
-        const int32_t* const from = c.indices + p0 + __builtin_amdgcn_readfirstlane(it);
+        const int32_t* const from = indices + p0 + __builtin_amdgcn_readfirstlane(it);
         asm volatile("s_load_dword %0, %1, 0x0\n\ts_waitcnt lgkmcnt(0)" : "=&s"(new_page) : "s"(from) : "memory");
     }
     issue(sa, g);
@@ -716,14 +720,22 @@ int batch_decode(void* o, const void* q, const void* kv_data, const void* kv_par
     const float sm = (float)(1.4426950408889634 / __builtin_sqrt((double)head_dim));
     const unsigned grid = (unsigned)(batch_size * num_heads * splits);
     hipStream_t st = (hipStream_t)stream;
+    // n / d as a multiplication: for n below 2^30, with s the least for which 2^s reaches d, floor(4 n ceil(2^(30 + s) / d) / 2^(32 + s))
+    auto log2_of = [](int64_t d) {
+        u32 s = 0;
+        while ((1ll << s) < d) ++s;
+        return s;
+    };
+    auto inverse = [](int64_t d, u32 s) { return (u32)(((1ull << (30 + s)) + (uint64_t)d - 1) / (uint64_t)d); };
+    const int64_t page_chunks = page_size % 16 == 0 ? page_size / 16 : 1;
+    const u32 heads_log2 = log2_of(num_heads), page_log2 = log2_of(page_chunks);
+    const u32 heads_inverse = inverse(num_heads, heads_log2), page_inverse = inverse(page_chunks, page_log2);
+    const u32 shifts = log2_of(splits) | page_log2 << 8 | heads_log2 << 16;
 #define QR_DECODE(AL, NWV)                                                                                              \
     do {                                                                                                                \
-        if (knew)                                                                                                       \
-            paged_decode_i4_kernel<AL, NWV, true><<<dim3(grid), dim3(64 * NWV), 0, st>>>(                               \
-                (const f16*)q, c, (f16*)o, sm, splits, part, q_had, arrived, (const u32x4*)knew, (const u32x4*)vnew, k_had); \
-        else                                                                                                            \
-            paged_decode_i4_kernel<AL, NWV><<<dim3(grid), dim3(64 * NWV), 0, st>>>((const f16*)q, c, (f16*)o, sm, splits, \
-                                                                                  part, q_had, arrived);               \
+        auto kern = knew ? paged_decode_i4_kernel<AL, NWV, true> : paged_decode_i4_kernel<AL, NWV, false>;              \
+        kern<<<dim3(grid), dim3(64 * NWV), 0, st>>>((const f16*)q, c.indptr, c.last_page_offset, c.indices, (const u32x4*)knew, \
+                                                    (const u32x4*)vnew, heads_inverse, page_inverse, shifts, c, (f16*)o, sm, part, q_had, arrived, k_had); \
     } while (0)
     if (page_size % 16 == 0) {
         if (plan.nw == 16) QR_DECODE(true, 16);
