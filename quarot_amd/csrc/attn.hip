@@ -228,9 +228,19 @@ __global__ __launch_bounds__(64 * NW, (NW == 16 ? 1 : NW == 8 ? 2 : 4)) void pag
     // ALIGNED: chunk g lies in page g / cpp at entry 16 (g % cpp); both advance without divisions
     const int cpp = ALIGNED ? c.page_size >> 4 : 1;
     auto pages = [&](int n) { return ALIGNED ? (int)(__umulhi((u32)n << 2, page_inverse) >> (shifts >> 8 & 255)) : n; };       // n / cpp
-    const int it_step = pages(stride), r_step = stride - it_step * cpp;
+    const int r_step = stride - pages(stride) * cpp;
     int g = sp * NW + wave;
-    int it_u = pages(g), r_u = g - it_u * cpp;
+    // ALIGNED: the page numbers of the wave's next 64 chunks, a lane each (-1: no such page), so that a step takes its own by
+    // a lane's number.  (A scalar load in every step, waited for where it stands:
+    // 3 x 8000 x 16 heads 16.9 us, now 15.9; 1 x 2048 x 32 8.4, now 8.0; 40 x 438 x 40 26.6, now 25.8.)
+    const int g_first = g;
+    int r_u = g - pages(g) * cpp, n_u = 0;                  // the chunk's place in its page, and its number among this wave's
+    auto fetch_pages = [&](int n) {
+        const int it = pages(g_first + (n + lane) * stride);
+        const int page = indices[p0 + (it < npages ? it : 0)];
+        return it < npages && page >= 0 && page < c.num_pages ? page : -1;
+    };
+    int page64 = ALIGNED ? fetch_pages(0) : 0;
     // Two sets of AU positions per lane group: the loads of the next set are issued before the current
     // one is consumed, so their latency hides under the arithmetic.  Loads are unconditional (a position
     // beyond the sequence reads entry 0 of a valid page and is masked), which keeps the loop free of
@@ -243,42 +253,33 @@ __global__ __launch_bounds__(64 * NW, (NW == 16 ? 1 : NW == 8 ? 2 : 4)) void pag
     auto issue = [&](Step& t, int g0) {
         int64_t page[AU];
         int entry[AU];
-        const int32_t* pp[AU];
-        // page numbers first (scalar loads when ALIGNED), then every vector load of the step
+        // page numbers first, then every vector load of the step
 #pragma unroll
         for (int u = 0; u < AU; ++u) {
             const int pos = (g0 + u * stride) * 16 + slot;
-            int it;
             if (ALIGNED) {
-                it = __builtin_amdgcn_readfirstlane(it_u);  // wave-uniform: the page number comes by a scalar load
+                page[u] = __builtin_amdgcn_readlane(page64, (n_u + u) & 63);        // (wave-uniform)
                 entry[u] = r_u * 16 + slot;
-                it_u += it_step;
                 r_u += r_step;
-                if (r_u >= cpp) {
-                    r_u -= cpp;
-                    ++it_u;
-                }
+                if (r_u >= cpp) r_u -= cpp;
+                t.ok[u] = pos < seq_len;
             } else {
-                it = pos / c.page_size;
+                const int it = pos / c.page_size;
                 entry[u] = pos - it * c.page_size;
+                t.ok[u] = pos < seq_len && it < npages;
+                page[u] = indices[p0 + (it < npages ? it : 0)];
             }
-            t.ok[u] = pos < seq_len && it < npages;
-            pp[u] = indices + p0 + (it < npages ? it : 0);
-            if (!ALIGNED) page[u] = *pp[u];
         }
         if (ALIGNED) {
-            // scalar loads, spelled out and waited for together: behind the scheduling barriers of the loop the compiler
-            // falls back to vector loads plus a wait for EVERY outstanding vector load, which would drain the pipeline
-            static_assert(AU == 2, "two page numbers per step");
-            int pg0, pg1;
-            asm volatile("s_load_dword %0, %2, 0x0\n\ts_load_dword %1, %3, 0x0\n\ts_waitcnt lgkmcnt(0)"
-                         : "=&s"(pg0), "=&s"(pg1) : "s"(pp[0]), "s"(pp[1]) : "memory");
-            page[0] = pg0;
-            page[1] = pg1;
+            n_u += AU;
+            if ((n_u & 63) == 0) {                          // (and waited for here, not at the next step)
+                page64 = fetch_pages(n_u);
+                asm volatile("" : "+v"(page64));
+            }
         }
 #pragma unroll
         for (int u = 0; u < AU; ++u) {
-            const bool page_ok = page[u] >= 0 && page[u] < c.num_pages;
+            const bool page_ok = page[u] >= 0 && (ALIGNED || page[u] < c.num_pages);
             t.ok[u] = t.ok[u] && page_ok;
             // the page part of the address is wave-uniform when ALIGNED (scalar base, 32-bit lane offsets)
             const int64_t kbase = (page_ok ? page[u] : 0) * page_slots + head_slots;
@@ -438,18 +439,16 @@ __global__ __launch_bounds__(64 * NW, (NW == 16 ? 1 : NW == 8 ? 2 : 4)) void pag
     };
     const int gs = stride * AU;
     // Of the waves on a SIMD the oldest is served first: at 32 x 4001 x 8 heads waves 0 .. 3 were through their walk 4.5 us before 4 .. 7,
-    // which then had the memory to themselves without the loads in flight that it takes to fill it.  With precedence for the later ones in half
-    // of the loop 3.5 us remain.  28.5 -> 28.0 us; 1 x 2048 x 32 heads 8.8 -> 8.4, where the later waves also start later.  (Precedence throughout
-    // turns the order round; by the turns that a wave and its partner have made, all end together and the launch is 2 us longer: in
-    // step, both wait for memory and then both compute.)
+    // which then had the memory to themselves without the loads in flight that it takes to fill it.  With precedence for the later ones, which
+    // also start later, 28.4 -> 27.8 us, 3 x 8000 x 16 heads 15.9 -> 15.6, 7 x 2500 x 16 13.1 -> 12.6.  (By the turns that a wave and
+    // its partner have made all end together, and the launch is 2 us longer: in step, both wait for memory and then both compute.)
     const bool late = NW > 4 && wave >= NW / 2;
+    if (late) __builtin_amdgcn_s_setprio(1);
     for (; g < chunks; g += 2 * gs) {
-        if (late) __builtin_amdgcn_s_setprio(1);
         issue(sb, g + gs);
         __builtin_amdgcn_sched_barrier(0);                 // the compiler would otherwise sink the loads below the arithmetic
         consume(sa);
         __builtin_amdgcn_sched_barrier(0);
-        if (late) __builtin_amdgcn_s_setprio(0);
         issue(sa, g + 2 * gs);
         __builtin_amdgcn_sched_barrier(0);
         if (g + gs < chunks) consume(sb);                  // (no loads inside: the branch does not disturb the wait counts)

@@ -98,6 +98,36 @@ def test_the_new_tokens_codes_come_from_every_lane_of_its_wave(hadamard):
         assert torch.equal(gp1.view(torch.int16), gp2.view(torch.int16)), hint
 
 
+@pytest.mark.parametrize("page_size", [16, 48, 128])
+def test_walks_of_more_chunks_than_a_wave_has_lanes(page_size):
+    """16 waves without a split: from 16384 positions on a wave walks 64 chunks of 16 and more, whose page numbers it fetches anew; pages of
+    one, three and eight chunks, one page number outside the pool among them (its positions do not count)."""
+    rng = np.random.default_rng(page_size)
+    heads, lens = 2, [16384, 16385, 18100, 40]
+    data, param, indptr, indices, last = paged_case(rng, heads, page_size, lens, layers=1)
+    q = (rng.standard_normal((len(lens), heads, 128)) * 2).astype(F16)
+    tabs = (gpu(indptr), gpu(indices), gpu(last))
+    k, v = synth_kv(rng, len(lens), heads), synth_kv(rng, len(lens), heads)
+    gd, gp = gpu(data), gpu(param)
+    one, two = torch.empty((len(lens), heads, 128), dtype=torch.float16, device="cuda:0"), torch.empty((len(lens), heads, 128), dtype=torch.float16, device="cuda:0")
+    kv.batch_decode_i4(one, gpu(q), gd, gp, *tabs, 0, q_hadamard=True, append=(gpu(k), gpu(v), True))
+    want = o.paged_batch_decode(o.kv_hadamard(q), gd.cpu().numpy(), gp.cpu().numpy(), indptr, indices, last, 0)
+    assert close(one.cpu().numpy(), want)
+    # without the middle page of the third sequence: the same as with its positions' keys infinitely far
+    gone = int(indptr[2] + (indptr[3] - indptr[2]) // 2)
+    holed = indices.copy()
+    holed[gone] = data.shape[0]
+    kv.batch_decode_i4(one, gpu(q), gd, gp, gpu(indptr), gpu(holed), gpu(last), 0, q_hadamard=True)
+    kv.batch_decode_i4(two, gpu(q), gd, gp, *tabs, 0, q_hadamard=True)
+    keep = [0, 1, 3]
+    assert torch.equal(one[keep], two[keep]) and not torch.equal(one[2], two[2])
+    dense = indices[indptr[2]:indptr[3]].tolist()
+    dense.remove(int(indices[gone]))
+    short = o.paged_batch_decode(o.kv_hadamard(q)[2:3], gd.cpu().numpy(), gp.cpu().numpy(), np.array([0, len(dense)], dtype=indptr.dtype),
+                                 np.array(dense, dtype=indices.dtype), last[2:3], 0)
+    assert close(one[2:3].cpu().numpy(), short)
+
+
 def test_cache_class_holds_the_token_for_the_attention_call_and_never_shows_a_stale_cache():
     """update() of a decode step hands the token to the attention call; reading the pages, asking for the tables or
     updating again before that call stores it first; a second call of the returned callable is plain attention."""
