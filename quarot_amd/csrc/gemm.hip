@@ -636,6 +636,24 @@ __global__ __launch_bounds__(768) void decode_xs_kernel(const uint8_t* __restric
             if (ks0 + q < stages) iteration(ks0 + q, regs[(q + 2) % RD]);
         return;
     }
+    // The outputs' scales and bias, read here, where a multiplying wave waits for the first stages anyway: behind the loop they
+    // were a memory latency at the end of every launch (7 tokens x 28672 x 8192 23.5 -> 22.6 us, 48 27.6 -> 26.5,
+    // 7 x 57344 x 8192 39.0 -> 38.0; in decode_i4_kernel, whose waves all stream, they stand in front of the stream and cost 2 %).
+    const int c0 = n0 + wave * 32;
+    f16x4 sb4[4], bi4[4];
+    f16 sa[MT];
+    if (DEQ && computes) {
+#pragma unroll
+        for (int gq = 0; gq < 4; ++gq)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int col = c0 + gq * 8 + h * 4 + e, cc = col < N ? col : N - 1;
+                sb4[gq][e] = sB[cc];
+                bi4[gq][e] = bias ? bias[cc] : (f16)0;
+            }
+#pragma unroll
+        for (int t = 0; t < MT; ++t) sa[t] = sA[t * 32 + r < M ? t * 32 + r : M - 1];
+    }
     __syncthreads();                                        // stages 0 and 1 visible
     if (computes) {
         read_w(xs_lds, 0, ops[0]);
@@ -664,29 +682,14 @@ __global__ __launch_bounds__(768) void decode_xs_kernel(const uint8_t* __restric
     }
 
     // ---- epilogue: lane l, register v -> weight row (v/4)*8 + (l/32)*4 + v%4 of the group, token l%32
-    auto finish = [&](const i32x16& a, int g, int t) {
-        const int c0 = n0 + g * 32;
+    auto finish = [&](const i32x16& a, int t) {
         const int row = t * 32 + r;
         const bool by_rows = DEQ && c0 + 32 <= N && (N & 7) == 0 && (((uintptr_t)Y) & 15) == 0 && t * 32 + 32 <= M;
-        f16x4 sb4[4], bi4[4];
-        if (DEQ) {
-#pragma unroll
-            for (int gq = 0; gq < 4; ++gq) {
-                const int col = c0 + gq * 8 + h * 4;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const int cc = col + e < N ? col + e : N - 1;
-                    sb4[gq][e] = sB[cc];
-                    bi4[gq][e] = bias ? bias[cc] : (f16)0;
-                }
-            }
-        }
         if (DEQ && by_rows) {
-            const f16 sa = sA[row];
             f16x4 o[1][4];
 #pragma unroll
             for (int gq = 0; gq < 4; ++gq)
-                o[0][gq] = dequant4(a[gq * 4], a[gq * 4 + 1], a[gq * 4 + 2], a[gq * 4 + 3], sa, sb4[gq], bi4[gq], bias != nullptr);
+                o[0][gq] = dequant4(a[gq * 4], a[gq * 4 + 1], a[gq * 4 + 2], a[gq * 4 + 3], sa[t], sb4[gq], bi4[gq], bias != nullptr);
             store_slab_rows<1>((u32x2*)(xs_lds + wave * 128), o, lane, Y + (int64_t)(t * 32) * N + c0, N);
             return;
         }
@@ -697,7 +700,7 @@ __global__ __launch_bounds__(768) void decode_xs_kernel(const uint8_t* __restric
             if (col >= N) continue;
             const bool whole = (col + 4 <= N) && ((N & 3) == 0);
             if (DEQ) {
-                const f16x4 o = dequant4(a[gq * 4], a[gq * 4 + 1], a[gq * 4 + 2], a[gq * 4 + 3], sA[row], sb4[gq], bi4[gq],
+                const f16x4 o = dequant4(a[gq * 4], a[gq * 4 + 1], a[gq * 4 + 2], a[gq * 4 + 3], sa[t], sb4[gq], bi4[gq],
                                          bias != nullptr);
                 f16* yp = Y + (int64_t)row * N + col;
                 if (whole) {
@@ -721,7 +724,7 @@ __global__ __launch_bounds__(768) void decode_xs_kernel(const uint8_t* __restric
     };
     if (!computes) return;
 #pragma unroll
-    for (int t = 0; t < MT; ++t) finish(acc[t], wave, t);
+    for (int t = 0; t < MT; ++t) finish(acc[t], t);
 }
 
 // ------------------------------------------------------------------------------------------------
