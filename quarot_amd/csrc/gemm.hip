@@ -484,7 +484,8 @@ __global__ __launch_bounds__(512) void decode_i4_kernel(const uint8_t* __restric
 // * Workgroup b starts its walk over K at stage b % stages and wraps around (integer sums do not depend
 //   on the order): with a row pitch that is a power of two, workgroups marching through K in step
 //   would all be reading the same few memory channels at any one time (measured 49 -> 41 us at
-//   57344 x 8192).
+//   57344 x 8192).  With such a pitch, stage b / 8: 7 tokens x 28672 x 8192 22.2 -> 21.9 us, 24 22.2 -> 21.6, 7 x 57344 x 8192 39.2 -> 38.2,
+//   16 x 28672 x 4096 13.0 -> 12.7; with others it is no better (32 x 27648 x 5120 16.2 -> 16.5).
 template <int MT, int R, int RD, bool DEQ>
 __global__ __launch_bounds__(768) void decode_xs_kernel(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B,
                                                         int M, int N, int Kb, int32_t* __restrict__ C,
@@ -522,7 +523,8 @@ __global__ __launch_bounds__(768) void decode_xs_kernel(const uint8_t* __restric
     }
     const int wdst0 = XPLANES + slot8(srow, piece);         // rows differ by multiples of 32: same swizzle
     const int xdst0 = slot16(srow, piece, 0);
-    const int s0 = blockIdx.x % stages;
+    // (consecutive workgroups are on different XCDs: the eight of a run start together, those of an XCD one stage after the other)
+    const int s0 = ((Kb & (Kb - 1)) == 0 ? blockIdx.x >> 3 : blockIdx.x) % stages;
     auto stage_of = [&](int st) {                           // absolute stage of this workgroup's st-th step
         const int a = (st < stages ? st : stages - 1) + s0;
         return a >= stages ? a - stages : a;
