@@ -417,7 +417,9 @@ int launch_mid(const void* A, const void* B, int M, int N, int Kb, void* C, void
 // tokens x 4096 x 4096): the loads are bound by rate, not by how many are in flight.  96 x 64 has a CU to itself as well (the
 // exchange is 96 KB) and four waves: four buffers 10.2, five 10.8 us at 333 x 4096 x 4096.  The STREAM form's come from memory:
 // with at most a workgroup per CU it takes five buffers, 64 KB in flight (48 x
-// 5120 x 13824 in two slices of K 17.8 -> 15.7 us), with more workgroups three (48 x 22016 x 4096 14.3 -> 13.5).
+// 5120 x 13824 in two slices of K 17.8 -> 15.7 us), with more workgroups three (48 x 22016 x 4096 14.3 -> 13.5).  Slices of K are short
+// walks, in which every further buffer delays the first stages of all: four (32 x 5120 x 13824 13.5 -> 13.1 us, 48 14.3 -> 14.0, 48 x 5120 x 20480
+// 17.6 -> 17.2; three 18.6, six 3 % and eight 7 % slower than five); whole walks are level or better with five (48 x 8192 x 8192 13.1, with four 13.4).
 __attribute__((visibility("hidden"))) int qr_internal_gemm_mid(int shape, const void* A, const void* B, int M, int N, int Kb,
                                                                void* C, void* Y, const void* sA, const void* sB,
                                                                const void* bias, hipStream_t st, int ksplit) {
@@ -427,6 +429,8 @@ __attribute__((visibility("hidden"))) int qr_internal_gemm_mid(int shape, const 
     if (shape == 4) return launch_mid<64, 64, 4, 4, false, 3>(A, B, M, N, Kb, C, Y, sA, sB, bias, st, ksplit);
     if (shape == 3) {
         if (M > 64) return QR_E_UNSUPPORTED;
+        if (ksplit > 1 && (int64_t)((N + 63) / 64) * ksplit <= qr_device().cus)
+            return launch_mid<64, 64, 4, 4, true>(A, B, M, N, Kb, C, Y, sA, sB, bias, st, ksplit);
         if ((int64_t)((N + 63) / 64) * ksplit <= qr_device().cus)
             return launch_mid<64, 64, 4, 5, true>(A, B, M, N, Kb, C, Y, sA, sB, bias, st, ksplit);
         return launch_mid<64, 64, 4, 3, true>(A, B, M, N, Kb, C, Y, sA, sB, bias, st, ksplit);
