@@ -189,10 +189,16 @@ __global__ __launch_bounds__(64 * (TM / 64) * (BN / 64) * WK) void gemm_mid_kern
 #pragma unroll
             for (int e = 0; e < 8; ++e) bi8[e] = (f16)-0.0f;
     }
-    for (int st = 0; st < NBUF && st < stages; ++st)
+    // (the buffers beyond three are asked for when the first stage has landed, which they would delay for all workgroups; the larger stages of
+    // 96-row tiles all at once: 333 x 4096 x 4096 three times 35.0 us behind two fronts, 35.3 this way)
+    constexpr int FIRST = IM == 3 ? NBUF : 3;
+    for (int st = 0; st < FIRST && st < stages; ++st)
 #pragma unroll
         for (int i = 0; i < NL; ++i) request1(st, st, i);
-    wait(stages - 1 < NBUF - 1 ? stages - 1 : NBUF - 1);
+    wait(stages - 1 < FIRST - 1 ? stages - 1 : FIRST - 1);
+    for (int st = FIRST; st < NBUF && st < stages; ++st)
+#pragma unroll
+        for (int i = 0; i < NL; ++i) request1(st, st, i);
     Ops ops[2];
     fill(0, 0, ops[0]);
     int buf = 0, s = 0;
@@ -413,8 +419,11 @@ int launch_mid(const void* A, const void* B, int M, int N, int Kb, void* C, void
 // shape: 0 = 64 x 64, 1 = 64 x 128, 2 = 128 x 128 tiles; 3 = 64 x 64 in the STREAM form (M <= 64); 4 = 96 x 64.  Three stage buffers of 16 KB
 // let three 64 x 64 workgroups share a CU.  A 64 x 128 or 128 x 128 one has a CU to itself: eight waves exchange 96 KB of
 // accumulators through LDS at the end, more than the 72 KB of its three stage buffers, and four buffers are 128 KB.
-// 64 x 128 with five and 64 x 64 with four buffers were no faster (11.8 against 11.2 us, 8.3 against 8.2 at 128 and 333
-// tokens x 4096 x 4096): the loads are bound by rate, not by how many are in flight.  96 x 64 has a CU to itself as well (the
+// One 64 x 64 workgroup to a CU at most and weights beyond 10 MB: four buffers.  Weights that come from memory, as a model's do layer by layer, have
+// more to wait for: 256 x 4096 x 11008 19.6 -> 17.1 us, 128 x 5120 x 5120 11.8 -> 10.8, 128 x 8192 x 8192 16.7 -> 14.9, 128 x 8192 x 28672
+// 47.7 -> 41.1; out of the last-level cache it is level (15.5 and 15.6, 9.2, 12.7).  (128 x 4096 x 4096 10.2 -> 9.1, but 8.1 -> 8.2 out of that cache, which
+// holds thirty of these.)  With two and three workgroups to a CU three buffers are ahead (512 x 5120 x 5120 18.2 us against 20.1), and
+// 64 x 128 with five was no faster (11.8 against 11.2 us at 128 x 4096 x 4096): the loads are bound by rate there.  96 x 64 has a CU to itself as well (the
 // exchange is 96 KB) and four waves: four buffers 10.2, five 10.8 us at 333 x 4096 x 4096.  The STREAM form's come from memory:
 // with at most a workgroup per CU it takes five buffers, 64 KB in flight (48 x
 // 5120 x 13824 in two slices of K 17.8 -> 15.7 us), with more workgroups three (48 x 22016 x 4096 14.3 -> 13.5).  Slices of K are short
@@ -424,7 +433,11 @@ __attribute__((visibility("hidden"))) int qr_internal_gemm_mid(int shape, const 
                                                                void* C, void* Y, const void* sA, const void* sB,
                                                                const void* bias, hipStream_t st, int ksplit) {
     if (ksplit > 1 && Y) return QR_E_UNSUPPORTED;           // partial sums exist only as int32
-    if (shape == 0) return launch_mid<64, 64, 4, 3>(A, B, M, N, Kb, C, Y, sA, sB, bias, st, ksplit);
+    if (shape == 0) {
+        if ((int64_t)((M + 63) / 64) * ((N + 63) / 64) * ksplit <= qr_device().cus && (int64_t)N * Kb > 10000000)
+            return launch_mid<64, 64, 4, 4>(A, B, M, N, Kb, C, Y, sA, sB, bias, st, ksplit);
+        return launch_mid<64, 64, 4, 3>(A, B, M, N, Kb, C, Y, sA, sB, bias, st, ksplit);
+    }
     if (shape == 1) return launch_mid<64, 128, 4, 3>(A, B, M, N, Kb, C, Y, sA, sB, bias, st, ksplit);
     if (shape == 4) return launch_mid<64, 64, 4, 4, false, 3>(A, B, M, N, Kb, C, Y, sA, sB, bias, st, ksplit);
     if (shape == 3) {
