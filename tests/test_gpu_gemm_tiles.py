@@ -117,6 +117,32 @@ def test_gemm_of_64_row_tiles_bit_exact(m, n, k, kind):
     _compare(m, n, k, kind)
 
 
+# (at most one 64 x 64 tile on a CU and weights on either side of 10 MB: four stage buffers or three; whole and ragged tiles, K that ends
+# inside a stage, walks of ten stages and of several hundred)
+@pytest.mark.parametrize("m,n,k", [(65, 8190, 2560), (128, 8192, 2432), (128, 8192, 2496), (127, 5121, 4160), (249, 4095, 11072), (70, 512, 65536)])
+@pytest.mark.parametrize("kind", ["random", "extreme"])
+def test_gemm_of_64_row_tiles_with_a_cu_each_bit_exact(m, n, k, kind):
+    assert _lib.lib().qr_linear_plan(m, n, k, 0, None) == b"gemm_mid_kernel<64,64>"
+    _compare(m, n, k, kind)
+
+
+# (slices of K; 70 rows: four buffers by the weights' size; up to 64 rows: four with at most one slice on a CU, or three)
+@pytest.mark.parametrize("m,n,k", [(70, 512, 65536), (193, 2500, 16448), (48, 5120, 13824), (23, 5100, 13888), (64, 4096, 11008), (48, 5120, 20480)])
+@pytest.mark.parametrize("kind", ["random", "extreme"])
+def test_gemm_of_64_row_tiles_in_slices_of_k_bit_exact(m, n, k, kind):
+    lib, used = _lib.lib(), ctypes.c_size_t()
+    assert lib.qr_linear_plan(m, n, k, lib.qr_workspace_bytes(m, n, k), ctypes.byref(used)) == b"gemm_mid_kernel<64,64> (K sliced) + dequant_slabs_kernel"
+    gen = torch.Generator(device="cuda").manual_seed(m + n + k)
+    a, b = _operand(m, k, kind, gen), _operand(n, k, kind, gen)
+    sa = (torch.rand(m, 1, device="cuda", generator=gen) * 0.1 + 0.01).half()
+    sb = (torch.rand(n, device="cuda", generator=gen) * 0.01 + 0.001).half()
+    ws = torch.full((used.value + 4096,), 0xA5, dtype=torch.uint8, device="cuda")
+    y = torch.full((m + 1, n), 7, dtype=torch.float16, device="cuda")
+    p = lambda t: ctypes.c_void_p(t.data_ptr())
+    assert lib.qr_linear_i4_f16_ws(p(a), p(sa), p(b), p(sb), None, m, n, k, p(y), p(ws), used.value, None) == 0
+    assert torch.equal(y[:m], (sa * sb) * _sums(a, b).float().half()) and bool((y[m] == 7).all()) and bool((ws[used.value:] == 0xA5).all())
+
+
 @pytest.mark.parametrize("m,n,k", [(333, 4096, 4096), (2048, 4096, 1088)])      # 96 x 64 tiles, 128 or more rows
 @pytest.mark.parametrize("shift", [1, 4])
 def test_scales_and_bias_may_start_anywhere(m, n, k, shift):
