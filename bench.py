@@ -131,8 +131,9 @@ def traffic_from_profile(workload, kernel):
         if m.group(1) in kernel and m.group(1) not in seen:
             seen.add(m.group(1))
             kib += float(m.group(2)) * float(sc.group(1)) + float(m.group(3)) * float(sc.group(2))
-    if seen:
-        code = re.search(r"traffic_code:\s*file=(\S+)\s+sha256=([0-9a-f]+)", text)
+            end = m.end()
+    if seen:                                     # (the code named next behind the readings)
+        code = re.compile(r"traffic_code:\s*file=(\S+)\s+sha256=([0-9a-f]+)").search(text, end)
         return round(kib * 1024), f"profiles/{name}", code_digest(code[1]) == code[2] if code else None
     return None, None, None
 
@@ -301,7 +302,7 @@ def gemm_kernel_name(m, n, k):
     """The library's own choice for a linear layer of this shape."""
     from quarot_amd import _lib
     L = _lib.lib()
-    return L.qr_linear_plan(m, n, k, L.qr_workspace_bytes(m, n, k), None).decode()
+    return L.qr_linear_plan(m, n, k, max(L.qr_workspace_bytes(m, n, k), L.qr_linear_spread_bytes(m, n, k)), None).decode()
 
 
 FRONT_KERNEL = {"had": "hadamard kernel + quantiser (fused)", "had32": "hadamard kernel in fp32 precision + quantiser (fused)",
@@ -310,9 +311,9 @@ FRONT_KERNEL = {"had": "hadamard kernel + quantiser (fused)", "had32": "hadamard
 
 
 def mfma_peak(kernel):
-    """Published rate of the matrix instruction that a GEMM kernel issues: the tiles of 128 and more rows x 256 columns multiply FP6
+    """Published rate of the matrix instruction that a GEMM kernel issues: the tiles with a side of 256 multiply FP6
     operands, the smaller ones int8."""
-    return FP6_MFMA_PEAK_TOPS if kernel.startswith(("gemm_sp", "gemm_f6")) else INT8_MFMA_PEAK_TOPS
+    return FP6_MFMA_PEAK_TOPS if kernel.startswith(("gemm_sp", "gemm_f6", "spread_x6")) else INT8_MFMA_PEAK_TOPS
 
 
 class LinearWorkload:
@@ -554,7 +555,7 @@ def run_layer(dev, steps, warmup, repeats, kernel_reps, fp6=False):
     roof = {"bound": "mfma", "achieved": round(ops / (gemm_total * 1e-3) / 1e12, 1), "peak": peak, "unit": "TOP/s"}
     roof["frac"] = round(roof["achieved"] / roof["peak"], 4)
     roof["kernel"] = ("gemm_f6_kernel (exact int4 GEMM on FP6 operands + dequant epilogue), four launches" if fp6
-                      else "gemm_sp256_kernel (int4 GEMM + dequant epilogue), four launches")
+                      else "spread_x6_kernel + gemm_x6_kernel (weights spread to six bits, int4 GEMM + dequant epilogue), four of each")
     roof["kernel_ms"] = round(gemm_total, 4)
     return {"ms": ms, "value": round(ops / (ms * 1e-3) / 1e12, 2), "unit": "TOPS", "timing": sp, "roofline": roof,
             "per_linear": per, "kernels_ms_sum": round(gemm_total + front_total, 4), "total_TOP": round(ops / 1e12, 2),
