@@ -192,3 +192,15 @@ def test_plan_counts_columns_left_in_a_cut_tile_and_weights_that_no_cache_holds(
     used = ctypes.c_size_t()
     lib.qr_linear_plan(100, 4096, 28672, lib.qr_workspace_bytes(100, 4096, 28672), ctypes.byref(used))
     assert used.value == 4 * 100 * 4096 * 4
+
+
+def test_plan_spreads_tokens_only_where_weights_from_memory_leave_a_lead(lib):
+    """Few tokens, spread, against wide weights, packed: the loop waits for weights that come from memory (measured with the tokens spread / in one
+    launch, in us: 36.1 / 30.6, 36.5 / 31.8, 50.5 / 45.8, 25.8 / 23.9, 35.5 / 29.8, 35.6 / 29.7, 43.3 / 38.2, 27.1 / 23.6, 61.9 / 59.5, 64.3 / 60.1);
+    with more tokens to a tile, and with the weights spread, the lead is there (29.6 / 33.1, 61.3 / 72.8, 30.7 / 35.4, 37.5 / 40.6, 123 / 140)."""
+    for m, n, k in ((160, 27648, 5120), (200, 27648, 5120), (256, 28672, 8192), (333, 12288, 4096), (333, 15360, 5120), (400, 13824, 5120),
+                    (512, 10240, 8192), (512, 11008, 4096), (65, 57344, 8192), (128, 57344, 8192)):
+        assert lib.qr_linear_spread_bytes(m, n, k) == 0, (m, n, k)
+    for m, n, k in ((333, 22016, 4096), (400, 28672, 8192), (700, 12288, 4096), (1024, 12288, 4096), (1024, 28672, 8192), (1777, 8192, 28672),
+                    (8191, 5120, 5120), (32768, 11008, 4096)):
+        assert lib.qr_linear_spread_bytes(m, n, k) > 0, (m, n, k)
