@@ -319,14 +319,37 @@ def _workspace_bytes(M, N, K, device_index=None):
     return used.value, L.qr_linear_spread_bytes(M, N, K)
 
 
+# devices that had no room for the scratch of a spread operand
+_SCRATCH_REFUSED = set()
+
+
+def _room_for(nbytes, dev):
+    # (as new memory, with 64 MiB to spare for what the allocator rounds up to)
+    if torch.cuda.is_current_stream_capturing():
+        return False
+    room, total = torch.cuda.mem_get_info(dev)
+    try:
+        room = min(room, torch.cuda.get_per_process_memory_fraction(dev) * total - torch.cuda.memory_reserved(dev))
+    except RuntimeError:                                                 # an allocator without these figures
+        pass
+    return room >= nbytes + (64 << 20)
+
+
 def _scratch(fixed, M, N, K, dev):
-    # fixed bytes and those of the product; a GPU too full for a spread operand does without
+    # fixed bytes and those of the product.  A GPU too full for a spread operand does without, whatever its allocator says so with; it is asked
+    # again only where there is room: a refusal makes torch's allocator wait for the GPU and give back every block that it keeps
     used, spread = _workspace_bytes(M, N, K, dev.index)
-    if spread:
+    if spread and (dev.index not in _SCRATCH_REFUSED or _room_for(fixed + spread, dev)):
         try:
-            return torch.empty((fixed + spread,), dtype=torch.uint8, device=dev)
-        except torch.cuda.OutOfMemoryError:
+            ws = torch.empty((fixed + spread,), dtype=torch.uint8, device=dev)
+            if ws.data_ptr():
+                _SCRATCH_REFUSED.discard(dev.index)
+                return ws
+        except torch.AcceleratorError:                                   # (of the device itself, not about room)
+            raise
+        except (RuntimeError, MemoryError):
             pass
+        _SCRATCH_REFUSED.add(dev.index)
     return torch.empty((fixed + used,), dtype=torch.uint8, device=dev)
 
 

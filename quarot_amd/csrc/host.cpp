@@ -10,13 +10,16 @@
 #include <Python.h>
 
 #include <ATen/ops/empty.h>
+#include <c10/hip/HIPCachingAllocator.h>
 #include <c10/hip/HIPFunctions.h>
+#include <c10/hip/HIPGraphsC10Utils.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/hip/HIPStream.h>
 #include <hip/hip_runtime_api.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
+#include <atomic>
 #include <stdexcept>
 #include <string>
 
@@ -328,13 +331,42 @@ Slabs slab_bytes(int64_t M, int64_t N, int64_t K) {
     if (s.asked) qr_linear_plan(M, N, K, s.asked, &s.used);
     return s;
 }
-// `fixed` bytes and those of the product, at least 16; *bytes: how many.  A GPU too full for a spread operand does without.
+// A refusal of memory is dear: torch's allocator waits for the GPU and gives back every block that it keeps before it raises, and what the program
+// allocates next is new memory.  So a device that had no room for the scratch of a spread operand, which is optional, is asked again only where
+// that would fit as new memory, with 64 MiB to spare for what the allocator rounds up to.
+std::atomic<bool> refused[64];
+bool room_for(size_t bytes, int device) {
+    if (c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None) return false;
+    auto* const allocator = c10::hip::HIPCachingAllocator::get();
+    const auto [free, total] = allocator->getMemoryInfo((c10::DeviceIndex)device);
+    size_t room = free;
+    try {
+        const double allowed = allocator->getMemoryFraction((c10::DeviceIndex)device) * (double)total;
+        const auto kept = allocator->getDeviceStats((c10::DeviceIndex)device).reserved_bytes[0].current;
+        const double left = allowed > (double)kept ? allowed - (double)kept : 0.0;
+        if (left < (double)room) room = (size_t)left;
+    } catch (const c10::Error&) {                           // an allocator without these figures
+    }
+    return room >= bytes + ((size_t)64 << 20);
+}
+// `fixed` bytes and those of the product, at least 16; *bytes: how many.  A GPU too full for a spread operand does without, whatever its
+// allocator says so with (torch's own raises OutOfMemoryError; errors of the device itself are not about room).
 at::Tensor scratch(size_t fixed, const Slabs& s, int device, size_t* bytes) {
     if (s.spread) {
-        try {
-            *bytes = fixed + s.spread;
-            return fresh({(int64_t)*bytes}, kByte, device);
-        } catch (const c10::OutOfMemoryError&) {
+        std::atomic<bool>& none_left = refused[device & 63];
+        *bytes = fixed + s.spread;
+        if (!none_left.load(std::memory_order_relaxed) || room_for(*bytes, device)) {
+            try {
+                at::Tensor ws = fresh({(int64_t)*bytes}, kByte, device);
+                if (ws.data_ptr()) {
+                    if (none_left.load(std::memory_order_relaxed)) none_left.store(false, std::memory_order_relaxed);
+                    return ws;
+                }
+            } catch (const c10::AcceleratorError&) {
+                throw;
+            } catch (const std::exception&) {
+            }
+            none_left.store(true, std::memory_order_relaxed);
         }
     }
     *bytes = fixed + s.used;

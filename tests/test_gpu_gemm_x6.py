@@ -122,6 +122,36 @@ def test_python_entry_points_with_and_without_room_for_it(general_route):
         general_route()
 
 
+def test_a_full_gpu_is_asked_for_the_scratch_once(general_route):
+    """A refusal costs the allocator's whole cache: of ten calls on a GPU without room one asks, and the first with room again has its scratch."""
+    m, n, k = 4096, 8192, 8192
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    q, w = _operand(m, k, "random", gen), _operand(n, k, "random", gen)
+    s, sw = (torch.rand(m, 1, device="cuda", generator=gen) * 0.1).half(), (torch.rand(n, 1, device="cuda", generator=gen) * 0.01).half()
+    need, total = _lib.lib().qr_linear_spread_bytes(m, n, k), torch.cuda.get_device_properties(0).total_memory
+    assert need > 20 << 20
+    want = quarot_amd.linear_i4(q, s, w, sw)
+    failed = lambda: sum(torch.cuda.memory_stats()[name] for name in ("num_alloc_retries", "num_ooms"))
+    for route in ("native", "general"):
+        quarot_amd.linear_i4(q, s, w, sw)                                         # (with room: whatever was refused before is forgotten)
+        torch.cuda.synchronize()
+        torch.cuda.empty_cache()
+        torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + 2 * m * n + 0.5 * need) / total)
+        before = failed()
+        try:
+            for _ in range(10):
+                assert torch.equal(quarot_amd.linear_i4(q, s, w, sw)[::64], want[::64]), route
+        finally:
+            torch.cuda.set_per_process_memory_fraction(1.0)
+        assert 1 <= failed() - before <= 2, route                                # (one request: its retry, and its failure)
+        torch.cuda.synchronize()
+        torch.cuda.reset_peak_memory_stats()
+        held = torch.cuda.memory_allocated()
+        assert torch.equal(quarot_amd.linear_i4(q, s, w, sw), want), route
+        assert torch.cuda.max_memory_allocated() - held >= 2 * m * n + need, route
+        general_route()
+
+
 def test_replays_of_a_captured_call():
     m, n, k = 4096, 8192, 4096
     gen = torch.Generator(device="cuda").manual_seed(4)

@@ -168,3 +168,46 @@ def test_package_works_without_the_native_host_route(monkeypatch):
     np.testing.assert_allclose(y.numpy(), o.rmsnorm(x.numpy(), 16, 1e-5), rtol=1e-3, atol=1e-3)
     with pytest.warns(UserWarning, match="_host.so"), pytest.raises(RuntimeError, match="GPU|CUDA|cuda"):
         quarot_amd.nn.Quantizer()(x)                                       # the general route's own error
+
+
+@pytest.mark.parametrize("error", [torch.OutOfMemoryError, MemoryError, RuntimeError, None])
+def test_scratch_that_was_refused_is_asked_for_again_only_where_there_is_room(monkeypatch, error):
+    """Whatever the allocator says no with (None: an address of zero); an error of the device itself is not taken for that."""
+    real, asked, free = torch.empty, [], [0]
+
+    class NoAddress:
+        def data_ptr(self):
+            return 0
+
+    def empty(size, **kw):
+        asked.append(size[0])
+        if size[0] < 1 << 20 or free[0] >= size[0]:
+            return real(size, dtype=torch.uint8)
+        if error is None:
+            return NoAddress()
+        raise error("no room")
+
+    dev = torch.device("cuda", 3)
+    monkeypatch.setattr(quarot_amd, "_workspace_bytes", lambda *a: (64, 1 << 20))
+    monkeypatch.setattr(quarot_amd, "_SCRATCH_REFUSED", set())
+    monkeypatch.setattr(torch, "empty", empty)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    monkeypatch.setattr(torch.cuda, "mem_get_info", lambda d: (free[0], 1 << 40))
+    monkeypatch.setattr(torch.cuda, "get_per_process_memory_fraction", lambda d: 0.5)
+    monkeypatch.setattr(torch.cuda, "memory_reserved", lambda d: 1 << 20)
+    for _ in range(3):
+        assert quarot_amd._scratch(16, 1, 1, 1, dev).numel() == 16 + 64
+    assert asked == [16 + (1 << 20), 80, 80, 80]
+    free[0] = 1 << 30
+    monkeypatch.setattr(torch.cuda, "memory_reserved", lambda d: 1 << 39)         # (the process has had what it is allowed)
+    assert quarot_amd._scratch(16, 1, 1, 1, dev).numel() == 80
+    monkeypatch.setattr(torch.cuda, "memory_reserved", lambda d: 1 << 20)
+    for _ in range(2):
+        assert quarot_amd._scratch(16, 1, 1, 1, dev).numel() == 16 + (1 << 20)
+    assert not quarot_amd._SCRATCH_REFUSED
+
+    def broken(size, **kw):
+        raise torch.AcceleratorError("device")
+    monkeypatch.setattr(torch, "empty", broken)
+    with pytest.raises(torch.AcceleratorError):
+        quarot_amd._scratch(16, 1, 1, 1, dev)
