@@ -251,12 +251,19 @@ struct SeqPlace {
 constexpr int KM_SEQS = 1024;                                      // sequences whose places fit the LDS table
 __device__ u32x4 kv_nowhere[8];                                    // what lanes without a place store to
 
+// (What a launch needs of the paged cache leads its arguments: behind a structure the compiler has none preloaded.  Every address waits for the
+// structure's load here, which the preload only puts off: 2 x 257 tokens x 8 heads 5.87 us, 5.97 with it, 4 x 244 x 16 6.45 / 6.61; the other forms gain by it.)
+template <bool PAGED>
+using Lead = std::conditional_t<PAGED, PagedDst, int>;
+
 template <bool QUANT, bool PAGED = false, bool TABLE = true>
-__global__ __launch_bounds__(64 * KM_WAVES, 2) void kv_had128_kernel(const u32x4* __restrict__ x, int64_t vectors,
+__global__ __launch_bounds__(64 * KM_WAVES, 2) void kv_had128_kernel(Lead<PAGED> lead, const u32x4* __restrict__ x, int64_t vectors,
                                                                      float hscale, u32x4* __restrict__ q,
                                                                      f16* __restrict__ scale, f16* __restrict__ zero,
-                                                                     u32x4* __restrict__ y, PagedDst pd,
+                                                                     u32x4* __restrict__ y,
                                                                      const u32x4* __restrict__ x2, int plain_mask, int log2t) {
+    PagedDst pd{};
+    if constexpr (PAGED) pd = lead;
     __shared__ u32x4 km_lds[KM_WAVES * 512];                       // 8 KB per wave
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int v = lane & 31, h = lane >> 5;
@@ -626,8 +633,10 @@ int launch_had128(const void* x, int64_t vectors, float hscale, void* q, void* s
     // nine blocks 12 x 1500 takes 78.6 us instead of 76.7, with four of three 2 x 7847 x 8 heads 27.3 instead of 20.8).
     const int64_t turns = want / (20 * cap), rounds = !PAGED || turns < 1 ? 1 : turns < 8 ? turns : 8;
     const unsigned grid = (unsigned)(want < cap * rounds ? want : cap * rounds);
-    kern<<<dim3(grid), dim3(64 * KM_WAVES), lds, st>>>((const u32x4*)x, vectors, hscale, (u32x4*)q, (f16*)scale, (f16*)zero,
-                                                      (u32x4*)y, pd, (const u32x4*)x2, plain_mask, log2t);
+    Lead<PAGED> lead{};
+    if constexpr (PAGED) lead = pd;
+    kern<<<dim3(grid), dim3(64 * KM_WAVES), lds, st>>>(lead, (const u32x4*)x, vectors, hscale, (u32x4*)q, (f16*)scale, (f16*)zero,
+                                                      (u32x4*)y, (const u32x4*)x2, plain_mask, log2t);
     return qr_launch_status();
 }
 
