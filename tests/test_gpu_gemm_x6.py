@@ -122,6 +122,30 @@ def test_python_entry_points_with_and_without_room_for_it(general_route):
         general_route()
 
 
+def test_scratch_of_a_shape_after_many_others():
+    """The native route keeps the sizes of a thread's last shapes: more of them than it keeps, and the first again."""
+    m, n, k = 4096, 8192, 4096
+    gen = torch.Generator(device="cuda").manual_seed(6)
+    q, w = _operand(m, k, "random", gen), _operand(n, k, "random", gen)
+    s, sw = (torch.rand(m, 1, device="cuda", generator=gen) * 0.1).half(), (torch.rand(n, 1, device="cuda", generator=gen) * 0.01).half()
+    need = _lib.lib().qr_linear_spread_bytes(m, n, k)
+    want = (s * sw.view(-1)) * _sums(q, w).float().half()
+
+    def check():
+        torch.cuda.synchronize()
+        torch.cuda.reset_peak_memory_stats()
+        held = torch.cuda.memory_allocated()
+        y = quarot_amd._host.linear(q, s, w, sw, None)
+        assert torch.cuda.max_memory_allocated() - held >= 2 * m * n + need > 2 * m * n and torch.equal(y, want)
+
+    check()
+    for rows in range(1, 300, 2):                            # (with slices of K and without, on either side of the fused tokens)
+        y = quarot_amd._host.linear(q[:rows], s[:rows], w[:1024], sw[:1024], None)
+        assert torch.equal(y, want[:rows, :1024]), rows
+        if rows % 50 == 1:
+            check()
+
+
 def test_a_full_gpu_is_asked_for_the_scratch_once(general_route):
     """A refusal costs the allocator's whole cache: of ten calls on a GPU without room one asks, and the first with room again has its scratch."""
     m, n, k = 4096, 8192, 8192
