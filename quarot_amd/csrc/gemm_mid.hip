@@ -189,14 +189,16 @@ __global__ __launch_bounds__(64 * (TM / 64) * (BN / 64) * WK) void gemm_mid_kern
 #pragma unroll
             for (int e = 0; e < 8; ++e) bi8[e] = (f16)-0.0f;
     }
-    // (the buffers beyond three are asked for when the first stage has landed, which they would delay for all workgroups; the larger stages of
-    // 96-row tiles all at once: 333 x 4096 x 4096 three times 35.0 us behind two fronts, 35.3 this way)
-    constexpr int FIRST = IM == 3 ? NBUF : 3;
-    for (int st = 0; st < FIRST && st < stages; ++st)
+    // (the buffers beyond three are asked for when the first stage has landed, which they would delay for all workgroups: 64 x 64 tiles with four, see
+    // below, 128 x 128 tiles 0.8 % faster over 26 shapes, 64 tokens x 11008 x 4096 9.56 -> 9.40 us.  All at once where little is delayed or the walk
+    // is short: the larger stages of 96-row tiles, 333 x 4096 x 4096 three times 35.0 us behind two fronts, 35.3 the other way; few rows of x, 8 x
+    // 12288 x 4096 8.52, 8.62; slices of K, 24 x 1000 x 12288 9.53, 9.65)
+    const int first = IM == 3 || (STREAM && (ksplit > 1 || M <= 16)) ? NBUF : 3;
+    for (int st = 0; st < first && st < stages; ++st)
 #pragma unroll
         for (int i = 0; i < NL; ++i) request1(st, st, i);
-    wait(stages - 1 < FIRST - 1 ? stages - 1 : FIRST - 1);
-    for (int st = FIRST; st < NBUF && st < stages; ++st)
+    wait(stages - 1 < first - 1 ? stages - 1 : first - 1);
+    for (int st = first; st < NBUF && st < stages; ++st)
 #pragma unroll
         for (int i = 0; i < NL; ++i) request1(st, st, i);
     Ops ops[2];

@@ -126,6 +126,15 @@ def test_gemm_of_64_row_tiles_with_a_cu_each_bit_exact(m, n, k, kind):
     _compare(m, n, k, kind)
 
 
+# (up to 64 rows, K whole: 16 rows ask for all stage buffers at once and 17 for the later ones behind the first stage; five buffers with a CU each, or
+# three; ragged last tiles and stages)
+@pytest.mark.parametrize("m,n,k", [(8, 12288, 4096), (16, 12280, 4160), (17, 12280, 4160), (17, 12288, 4096), (16, 22009, 4096), (64, 15361, 5120)])
+@pytest.mark.parametrize("kind", ["random", "extreme"])
+def test_gemm_of_64_row_tiles_of_one_row_bit_exact(m, n, k, kind):
+    assert _lib.lib().qr_linear_plan(m, n, k, 0, None) == b"gemm_mid_kernel<64,64>"
+    _compare(m, n, k, kind)
+
+
 # (slices of K; 70 rows: four buffers by the weights' size; up to 64 rows: four with at most one slice on a CU, or three)
 @pytest.mark.parametrize("m,n,k", [(70, 512, 65536), (193, 2500, 16448), (48, 5120, 13824), (23, 5100, 13888), (64, 4096, 11008), (48, 5120, 20480)])
 @pytest.mark.parametrize("kind", ["random", "extreme"])
