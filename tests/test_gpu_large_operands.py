@@ -50,3 +50,23 @@ def test_linear_with_an_operand_of_four_gib_and_more(m, n, k):
     assert int(c[0, 0]) == 64 * k and int(c[m - 1, n - 1]) == -56 * k
     ref = o.int4_matmul(a[rows].cpu().numpy(), lin.weight[cols].cpu().numpy())
     assert np.array_equal(c[rows][:, cols].cpu().numpy(), ref)
+
+
+@pytest.mark.parametrize("m,n,k", [(60000, 1024, 131008), (1024, 60000, 131008)])        # activations, weights of 3.9 GB
+def test_linear_with_an_operand_past_two_gib_and_the_other_one_spread(m, n, k):
+    """Offsets from 2^31 on in the packed operand of the GEMM whose other operand is spread to six bits first."""
+    from quarot_amd import _lib
+    lib = _lib.lib()
+    need = lib.qr_linear_spread_bytes(m, n, k)
+    assert b"gemm_x6" in lib.qr_linear_plan(m, n, k, need, None) and 1 << 31 < max(m, n) * (k // 2) < 1 << 32
+    dev = torch.device("cuda:0")
+    g = torch.Generator(device=dev).manual_seed(m)
+    a, w = [torch.randint(0, 256, (r, k // 2), dtype=torch.uint8, device=dev, generator=g) for r in (m, n)]
+    sa, sw = [(torch.rand(r, 1, device=dev, generator=g) * 0.1 + 0.01).half() for r in (m, n)]
+    a[m - 1].fill_(0x88)
+    w[n - 1].fill_(0x77)
+    y = quarot_amd.linear_i4(a, sa, w, sw)
+    rng, past = np.random.default_rng(m), (1 << 31) // (k // 2)                         # the row that holds byte 2^31
+    rows, cols = [sorted(set([0, r - 1] + [v for v in (past - 1, past, past + 1) if v < r] + [int(v) for v in rng.integers(0, r, 5)])) for r in (m, n)]
+    want = o.linear4bit(a[rows].cpu().numpy(), sa.view(-1)[rows].cpu().numpy(), w[cols].cpu().numpy(), sw.view(-1)[cols].cpu().numpy())
+    assert np.array_equal(bits(y[rows][:, cols].cpu().numpy()), bits(want))
