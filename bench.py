@@ -533,6 +533,8 @@ def run_layer(dev, steps, warmup, repeats, kernel_reps, fp6=False):
     ms = sp["median_ms"]
     per, gemm_total, front_total = {}, 0.0, 0.0
     peak = FP6_MFMA_PEAK_TOPS
+    plans = [gemm_kernel_name(m, n, k) for _, k, n, _, _ in parts]
+    launches = 12 if fp6 else sum(2 + plan.count(" + ") for plan in plans)      # (a front and a product, which may be two)
     for (name, k, n, kind, _), (x, front, lin) in zip(parts, mods):
         p = front(x)
         f_ms = kernel_ms(lambda: front(x), kernel_reps)
@@ -555,13 +557,13 @@ def run_layer(dev, steps, warmup, repeats, kernel_reps, fp6=False):
     roof = {"bound": "mfma", "achieved": round(ops / (gemm_total * 1e-3) / 1e12, 1), "peak": peak, "unit": "TOP/s"}
     roof["frac"] = round(roof["achieved"] / roof["peak"], 4)
     roof["kernel"] = ("gemm_f6_kernel (exact int4 GEMM on FP6 operands + dequant epilogue), four launches" if fp6
-                      else "spread_x6_kernel + gemm_x6_kernel (weights spread to six bits, int4 GEMM + dequant epilogue), four of each")
+                      else ", ".join(f"{plans.count(plan)} x {plan}" for plan in dict.fromkeys(plans)) + " (int4 GEMM + dequant epilogue)")
     roof["kernel_ms"] = round(gemm_total, 4)
     return {"ms": ms, "value": round(ops / (ms * 1e-3) / 1e12, 2), "unit": "TOPS", "timing": sp, "roofline": roof,
             "per_linear": per, "kernels_ms_sum": round(gemm_total + front_total, 4), "total_TOP": round(ops / 1e12, 2),
             "step_frac": round(ops / (ms * 1e-3) / 1e12 / peak, 4),
             "workload": "c3: Llama-2-7B decoder-layer linear set at M=32768 (qkv 4096->12288, o 4096->4096, gate_up 4096->22016, "
-                        "down 11008->4096 with online Hadamard), W4A4, one step = " + ("12 launches (fronts, conversions to 6-bit operands, GEMMs)" if fp6 else "8 launches")}
+                        "down 11008->4096 with online Hadamard), W4A4, one step = " + f"{launches} launches" + (" (fronts, conversions to 6-bit operands, GEMMs)" if fp6 else " (fronts, operands spread to 6 bits, GEMMs)" if launches > 8 else "")}
 
 
 def run_kv(dev, steps, warmup, repeats, kernel_reps, cpu_baseline):
