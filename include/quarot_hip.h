@@ -198,8 +198,8 @@ int qr_linear_i4_f16(const void* A, const void* sA, const void* W, const void* s
  *   smaller size selects the single-launch path of qr_linear_i4_f16.  Results are identical bit for
  *   bit either way (integer partial sums).  Calls that share a workspace must not overlap.
  *   qr_linear_spread_bytes: bytes with which it takes a long prompt in two launches that are faster than one, the operand of fewer
- *   rows spread from 4 to 6 bits per code in the workspace first (three quarters of a byte per code of it; 0: no gain, any M, N, K).
- *   It is optional: without it the single-launch kernels run, with the same results.
+ *   rows spread from 4 to 6 bits per code in the workspace first (three quarters of a byte per code of it, at most 512 MiB; 0: no gain, any M, N, K).
+ *   It is optional: without it the single-launch kernels run, with the same results.  A graph that captures such a call keeps the workspace.
  */
 size_t qr_workspace_bytes(int64_t M, int64_t N, int64_t K);
 size_t qr_linear_spread_bytes(int64_t M, int64_t N, int64_t K);
@@ -237,7 +237,7 @@ int qr_linear_i4_f16_static(const void* A, const void* sA, const void* W, const 
  * Linear4bit.forward (quarot/nn/linear.py:42-56) for prefill shapes on 6-bit operands: the same
  * product and the same fp16 epilogue as qr_linear_i4_f16, bit for bit (every int4 code is a value of
  * FP6 E3M2, products and sums stay integers below 2^24, so the fp32 accumulators are exact).  qr_linear_i4_f16's long prompts
- * use the same matrix instruction on the packed codes, without a conversion, and are faster.  Both operands must first be converted to the 6-bit stage-major layout this
+ * use the same matrix instruction on the packed codes, at most one of the operands converted for the call, and are faster.  Both operands must first be converted to the 6-bit stage-major layout this
  * kernel reads; the reference has no counterpart (its CUTLASS call takes the packed nibbles,
  * quarot/kernels/gemm.cu:16-41).
  *   qr_f6_bytes(rows, K): bytes of a converted operand (rows * K * 3 / 4; K % 64 == 0).
@@ -392,10 +392,10 @@ int qr_batch_decode_qhad_i4(void* o, const void* q, const void* kv_data, const v
  * append_indptr NULL) followed by qr_batch_decode_i4 / qr_batch_decode_qhad_i4 -- what
  * MultiLayerPagedKVCache4Bit.update and the callable it returns do for a decode step
  * (quarot/transformers/kv_cache.py:104-129,224-251).  The page tables already count the new token (it is the
- * LAST position of its sequence, as for qr_kv_quant_append_f16_i4); the first two waves of every (sequence, head)
+ * LAST position of its sequence, as for qr_kv_quant_append_f16_i4); the last two waves of every (sequence, head)
  * quantise the token's key (through H_128 when k_had_mode = 1) and value with the arithmetic of that entry
- * point -- the same codes, scales and zeros, written to the same page slots -- while the other waves walk the
- * cached positions.
+ * point -- the same codes, scales and zeros, written to the same page slots -- while their first loads of the
+ * cached positions are on the way, and the other waves walk those.
  *   k, v fp16 [batch_size, num_heads, 128] (16-byte aligned); q_had_mode 0 / 1 as the two entry points above, optionally
  *   | QR_DECODE_COUNTERS_ZERO (then also a split along the sequence is one launch);
  *   everything else as qr_batch_decode_i4.  A sequence whose page list is empty is skipped by the append and

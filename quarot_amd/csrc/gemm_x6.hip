@@ -372,11 +372,11 @@ __device__ __forceinline__ void x6_tiles(const uint8_t* __restrict__ U, const ui
                 f16x4 o[2][4];
                 dequant_slab_f32x64(a0, a1, sa[i], sbh, bih, bias != nullptr, o);
                 if (jb + i > 0)
-                    slab_store<1>(out, slab, limit, m1 + (i > 0 ? i - 1 : IB - 1) * 32, at.n0 + n1 + (i > 0 ? jb : jb - 2) * 32, ln);
+                    slab_store<true>(out, slab, limit, m1 + (i > 0 ? i - 1 : IB - 1) * 32, at.n0 + n1 + (i > 0 ? jb : jb - 2) * 32, ln);
                 slab = slab_turn(region, o, ln);
             }
         }
-        slab_store<1>(out, slab, limit, m1 + (IB - 1) * 32, at.n0 + n1 + (JB - 1) / 2 * 64, ln);
+        slab_store<true>(out, slab, limit, m1 + (IB - 1) * 32, at.n0 + n1 + (JB - 1) / 2 * 64, ln);
         if (last) return;
         // the next tile's scales into the other half of their place (a slower wave may still read this tile's)
         scales = scales == (f16*)(lds + kAtX + 3 * kUnitX) ? scales + kScales : (f16*)(lds + kAtX + 3 * kUnitX);

@@ -85,16 +85,16 @@ __device__ __forceinline__ SlabOut slab_out(f16* Y, int m0, int rows, int N, int
     return SlabOut{__builtin_amdgcn_make_buffer_rsrc((void*)(Y + (int64_t)m0 * N), 0, (int)((u32)rows * (u32)N * 2u), 0x00020000),
                    ((u32)(lane >> 3) * (u32)N + (u32)((lane & 7) * 8)) * 2u, N, (N & 7) == 0 && (((uintptr_t)Y) & 15) == 0, (N & 3) == 0};
 }
-// rows from `row` of the tile on, columns from col0 of the output up to `end`.  A caller that has looked at out.wide says so in WIDE (0 / 1), so that
-// the code of whole pieces stands by itself.
-template <int WIDE = -1>
+// rows from `row` of the tile on, columns from col0 of the output up to `end`.  A caller whose outputs are all wide says so in WIDE, and has the code
+// of whole pieces alone.
+template <bool WIDE = false>
 __device__ __forceinline__ void slab_store(const SlabOut& out, const Slab& s, int end, int row, int col0, int lane) {
     constexpr u32 GONE = 0xFFFFFF00u;           // beyond the range of every buffer here
     const u32 at = out.lane_at + ((u32)row * (u32)out.N + (u32)col0) * 2u, rows8 = (u32)out.N * 16u;
     const int left = end - col0 - (lane & 7) * 8;           // columns from the piece on
     // (nontemporal: the output is not read again by this launch, and written this way it disturbs the operands in L2 less --
     // measured 1-4 % off whole GEMM launches at 2048 and 32768 tokens)
-    if (WIDE == 1 || (WIDE < 0 && out.wide)) {
+    if (WIDE || out.wide) {
         const u32 off = left > 0 ? at : GONE, step = left > 0 ? rows8 : 0u;
 #pragma unroll
         for (int p = 0; p < 4; ++p) __builtin_amdgcn_raw_buffer_store_b128(s.v[p], out.rsrc, off + step * (u32)p, 0, 2);
