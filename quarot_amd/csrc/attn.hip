@@ -655,8 +655,9 @@ extern "C" int qr_kv_append_i4(void* kv_data, void* kv_param, const void* kv_ind
 
 namespace {
 // Waves of a workgroup and workgroups of a (sequence, head), by an estimate in microseconds fitted to a sweep of 1 .. 40
-// sequences x 89 .. 16000 positions x 8 .. 64 heads with every plan forced (within 20 % of them, the chosen plan within
-// 5 % of the best one measured):
+// sequences x 89 .. 16000 positions x 8 .. 64 heads with every plan forced, when a workgroup's fixed path was longer than it is now (2099 cases of
+// the present kernel: the chosen plan costs 1.1 % more than the best, 4 % in one of ten, 26 % at worst, where few heads are split sixteen times
+// and eight are better):
 //   3.3 for the launch and its first loads, 2.7 / 3.4 / 5.0 per workgroup of 4 / 8 / 16 waves on the busiest CU (query,
 //   merge), 1.8 when the states of several workgroups are merged (+ 0.3 for every eight of them), and the walk: 0.37 per
 //   chunk of 16 positions for one wave, but no faster than 0.069 per chunk for a CU (its vector units dequantise; 0.093

@@ -1109,6 +1109,9 @@ __global__ __launch_bounds__(256) void dequant_slabs_kernel(const int32_t* __res
 // 13824 17.6 / 13.3, 48 x 4096 x 11008 14.9 / 12.0, 25 x 12288 x 8192 17.0 / 14.3; 32 x 4096 x 4096 stays (6.1 against 8.3).  Below eight tokens
 // the two are within 5 % of each other where the tiles lead at all.  Slices only where three or more fit, or where two save 4 us
 // (40 tokens and K = 16384 on): the scratch that callers are asked for grows with them.
+// (The fit is older than the slices' four stage buffers.  4843 shapes of 8 .. 64 tokens with weights from memory: the choice costs 1.1 % more than the best, of
+// which 0.3 is the readings' spread; 24 % and more in one of a hundred, wide weights with a short K: 35 x 21824 x 1536 in 15.8 us on the barrier-free
+// kernel, 9.0 on tiles.)
 struct DecodePlan {
     bool tiles;
     int split;
@@ -1188,6 +1191,9 @@ int ks_split(int64_t M, int64_t N, int64_t Kb) {
 // of few tiles and a long K with up to eight slices.  The choice costs 0.2 % more than the best of all kernels (geometric mean; 0.1 % up to
 // K = 1536, 0.3 % at N in steps of 8, 0.7 % where K may be sliced; without the output's terms and those of heavy weights 1.6, 3.2, 1.9 and
 // 1.1 %, 2 x at worst).
+// The fit is older than the fourth stage buffer of 64 x 64 tiles with a CU each, which take up to 14 % less from memory than it says.  Of the present
+// kernels, 814 shapes of 65 .. 1500 tokens with weights from memory: the choice, spread operands among them, costs 1.2 % more than the best (the readings'
+// own spread is 0.5 of it), 3 % or more in one of ten, 23 % at worst (268 x 8232 x 8768, on 64 x 64 tiles instead of 128 x 128).
 // The small tiles are bound by the CUs' intake of operands, the large ones by instruction issue and power, so the small ones lead
 // while the large ones leave CUs idle: 333 x 4096 x 4096 11.2 us against 22, 777 x 4096 x 4096 17.7 (22), 512 x 8192 x 8192 32.1 (34).
 // Very few tiles and a long K: slices of K over several workgroups with int32 slabs in the caller's scratch and a second

@@ -424,7 +424,7 @@ int launch_mid(const void* A, const void* B, int M, int N, int Kb, void* C, void
 // One 64 x 64 workgroup to a CU at most and weights beyond 10 MB: four buffers.  Weights that come from memory, as a model's do layer by layer, have
 // more to wait for: 256 x 4096 x 11008 19.6 -> 17.1 us, 128 x 5120 x 5120 11.8 -> 10.8, 128 x 8192 x 8192 16.7 -> 14.9, 128 x 8192 x 28672
 // 47.7 -> 41.1; out of the last-level cache it is level (15.5 and 15.6, 9.2, 12.7).  (128 x 4096 x 4096 10.2 -> 9.1, but 8.1 -> 8.2 out of that cache, which
-// holds thirty of these.)  With two and three workgroups to a CU three buffers are ahead (512 x 5120 x 5120 18.2 us against 20.1), and
+// holds thirty of these.  The line is not a capacity: below it a loop over few layers loses 1 %, and a model of many would gain there too.)  With two and three workgroups to a CU three buffers are ahead (512 x 5120 x 5120 18.2 us against 20.1), and
 // 64 x 128 with five was no faster (11.8 against 11.2 us at 128 x 4096 x 4096): the loads are bound by rate there.  96 x 64 has a CU to itself as well (the
 // exchange is 96 KB) and four waves: four buffers 10.2, five 10.8 us at 333 x 4096 x 4096.  The STREAM form's come from memory:
 // with at most a workgroup per CU it takes five buffers, 64 KB in flight (48 x
