@@ -160,6 +160,8 @@ def test_a_full_gpu_is_asked_for_the_scratch_once(general_route):
         quarot_amd.linear_i4(q, s, w, sw)                                         # (with room: whatever was refused before is forgotten)
         torch.cuda.synchronize()
         torch.cuda.empty_cache()
+        holes = [torch.empty(b["size"], dtype=torch.uint8, device="cuda") for segment in torch.cuda.memory_snapshot() for b in segment["blocks"]
+                 if b["state"] == "inactive" and b["size"] >= 1 << 20]            # (what is free in memory that others keep)
         torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + 2 * m * n + 0.5 * need) / total)
         before = failed()
         try:
@@ -167,6 +169,7 @@ def test_a_full_gpu_is_asked_for_the_scratch_once(general_route):
                 assert torch.equal(quarot_amd.linear_i4(q, s, w, sw)[::64], want[::64]), route
         finally:
             torch.cuda.set_per_process_memory_fraction(1.0)
+        del holes
         assert 1 <= failed() - before <= 2, route                                # (one request: its retry, and its failure)
         torch.cuda.synchronize()
         torch.cuda.reset_peak_memory_stats()
