@@ -178,8 +178,8 @@ __device__ __forceinline__ void merge_states(const float* src, int splits, int d
 template <bool ALIGNED, int NW, bool APPEND = false>
 __global__ __launch_bounds__(64 * NW, (NW == 16 ? 1 : NW == 8 ? 2 : 4)) void paged_decode_i4_kernel(
     const f16* __restrict__ q, uint64_t indptr_at, uint64_t last_page_offset_at, uint64_t indices_at,
-    const u32x4* __restrict__ knew, const u32x4* __restrict__ vnew, u32 heads_inverse, u32 page_inverse, u32 bits, PagedKV c, f16* __restrict__ o,
-    float* __restrict__ part, u32* __restrict__ arrived) {
+    const u32x4* __restrict__ knew, const u32x4* __restrict__ vnew, u32 heads_inverse, u32 page_inverse, u32 shifts, PagedKV c, f16* __restrict__ o,
+    float sm_scale_log2, float* __restrict__ part, int had, u32* __restrict__ arrived) {
     // (the arguments that the first loads wait for stand first: they arrive with the waves.  The page tables' addresses come as numbers: for
     // every argument that is a pointer the launch looks its allocation up, 0.06 us each on the host, which bounds the smallest steps)
     using Ints = const __attribute__((address_space(1))) int32_t*;
@@ -190,11 +190,9 @@ __global__ __launch_bounds__(64 * NW, (NW == 16 ? 1 : NW == 8 ? 2 : 4)) void pag
     float* const st = (float*)st4;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int slot = lane >> 2, c4 = lane & 3;
-    // bits: log2 of the splits | shift of the page division << 8 | of the division by the heads << 16 | transform the query << 24 | the key << 25
-    const int splits = 1 << (bits & 31), bh = blockIdx.x >> (bits & 31), sp = blockIdx.x & (splits - 1);
-    const int b = (int)(__umulhi((u32)bh << 2, heads_inverse) >> (bits >> 16 & 255)), h = bh - b * c.num_heads;
-    const bool q_had = (bits >> 24 & 1) != 0, k_had = (bits >> 25 & 1) != 0;
-    constexpr float sm_scale_log2 = (float)(1.4426950408889634 / 11.313708498984761);      // log2(e) / sqrt(128)
+    const int q_had = had & 1, k_had = had >> 1;            // whether the query and the new key are transformed
+    const int splits = 1 << (shifts & 31), bh = blockIdx.x >> (shifts & 31), sp = blockIdx.x & (splits - 1);
+    const int b = (int)(__umulhi((u32)bh << 2, heads_inverse) >> (shifts >> 16)), h = bh - b * c.num_heads;
     const u32 qword = ((const u32*)q)[(int64_t)bh * 64 + lane];          // dimensions 2 lane, 2 lane + 1
     const bool owns_new = APPEND && sp == splits - 1;       // uniform; of this workgroup's waves the last: the key, the last but one: the value
     const bool appends = owns_new && wave >= NW - 2;
@@ -233,7 +231,7 @@ __global__ __launch_bounds__(64 * NW, (NW == 16 ? 1 : NW == 8 ? 2 : 4)) void pag
     const int stride = NW * splits;                         // chunks between the steps of one wave
     // ALIGNED: chunk g lies in page g / cpp at entry 16 (g % cpp); both advance without divisions
     const int cpp = ALIGNED ? c.page_size >> 4 : 1;
-    auto pages = [&](int n) { return ALIGNED ? (int)(__umulhi((u32)n << 2, page_inverse) >> (bits >> 8 & 255)) : n; };       // n / cpp
+    auto pages = [&](int n) { return ALIGNED ? (int)(__umulhi((u32)n << 2, page_inverse) >> (shifts >> 8 & 255)) : n; };       // n / cpp
     const int r_step = stride - pages(stride) * cpp;
     int g = sp * NW + wave;
     // ALIGNED: the page numbers of the wave's next 64 chunks, a lane each (-1: no such page), so that a step takes its own by
@@ -723,6 +721,7 @@ int batch_decode(void* o, const void* q, const void* kv_data, const void* kv_par
         splits = 1;                                        // no room for partial states: one workgroup per (sequence, head)
     float* const part = splits > 1 ? (float*)((char*)workspace + counters) : nullptr;
     u32* const arrived = splits > 1 && counters_zero ? (u32*)workspace : nullptr;
+    const float sm = (float)(1.4426950408889634 / __builtin_sqrt((double)head_dim));
     const unsigned grid = (unsigned)(batch_size * num_heads * splits);
     hipStream_t st = (hipStream_t)stream;
     // n / d as a multiplication: for n below 2^30, with s the least for which 2^s reaches d, floor(4 n ceil(2^(30 + s) / d) / 2^(32 + s))
@@ -731,12 +730,12 @@ int batch_decode(void* o, const void* q, const void* kv_data, const void* kv_par
     const int64_t page_chunks = page_size % 16 == 0 ? page_size / 16 : 1;
     const u32 heads_log2 = log2_of(num_heads), page_log2 = log2_of(page_chunks);
     const u32 heads_inverse = inverse(num_heads, heads_log2), page_inverse = inverse(page_chunks, page_log2);
-    const u32 bits = log2_of(splits) | page_log2 << 8 | heads_log2 << 16 | (u32)(q_had != 0) << 24 | (u32)(k_had != 0) << 25;
+    const u32 shifts = log2_of(splits) | page_log2 << 8 | heads_log2 << 16;
 #define QR_DECODE(AL, NWV)                                                                                              \
     do {                                                                                                                \
         auto kern = knew ? paged_decode_i4_kernel<AL, NWV, true> : paged_decode_i4_kernel<AL, NWV, false>;              \
         kern<<<dim3(grid), dim3(64 * NWV), 0, st>>>((const f16*)q, (uint64_t)c.indptr, (uint64_t)c.last_page_offset, (uint64_t)c.indices, \
-                                                    (const u32x4*)knew, (const u32x4*)vnew, heads_inverse, page_inverse, bits, c, (f16*)o, part, arrived); \
+                                                    (const u32x4*)knew, (const u32x4*)vnew, heads_inverse, page_inverse, shifts, c, (f16*)o, sm, part, (q_had ? 1 : 0) | (k_had ? 2 : 0), arrived); \
     } while (0)
     if (page_size % 16 == 0) {
         if (plan.nw == 16) QR_DECODE(true, 16);
