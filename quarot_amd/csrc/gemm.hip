@@ -1255,14 +1255,16 @@ MidPlan mid_plan(int64_t M, int64_t N, int64_t Kb, int64_t max_split, bool fp16)
 // The same product with the operand of fewer rows spread in memory first (gemm_x6.hip), by tiles of 256 rows of the other operand and 32 nx of
 // that one, in microseconds: 5.8 + 0.307 per MB that is written, n times (0.26 + 0.675 nx) (1 - 0.23 idle) + st times a stage of (0.406 + 0.144 nx)
 // (1 - 0.285 idle), and 0.25 per million elements where rows of the output start within a line.  Where x is spread and the weights stay packed, they
-// come from memory: a stage takes 1.15 at least (with two stage buffers each is asked for one stage ahead), all of them what their bytes take at 5 TB/s.
-// Without these limits, which the last-level cache hides, prompts of 65 .. 550 tokens against wide weights took this way: 400 tokens x 13824 x 5120
-// 35.6 us, 29.7 without, 200 x 27648 x 5120 36.5 / 31.8, 512 x 11008 x 4096 27.1 / 23.6, 100 x 57344 x 8192 63.7 / 60.0.
+// come from memory: a stage takes 1.15 at least (with two stage buffers each is asked for one stage ahead; 1.05 where a CU has several tiles, whose
+// first stages come under the tile before), all of them what their bytes take at 5 TB/s.  Without these limits, which the last-level cache hides,
+// prompts of 65 .. 550 tokens against wide weights took this way: 400 tokens x 13824 x 5120 35.6 us, 29.7 without, 200 x 27648 x 5120 36.5 / 31.8,
+// 512 x 11008 x 4096 27.1 / 23.6, 100 x 57344 x 8192 63.7 / 60.0 (out of that cache they lose 4 % by the limits).
 // The terms are fitted to 2200 shapes of 100 .. 32768 tokens x 512 .. 57344 weight rows, 1e9 .. 6e12 operations, all five nx forced; the limits and
-// the lead of 2.5 us that it must have over mid_plan's kernels to 4845 more of 65 .. 32768 tokens, every kernel forced, weights from memory and from
-// cache.  From memory the choice is 1.045 x as fast as without these kernels (1.047 with the best of all; 1.033 without the limits and 0.8 us of
-// lead, when a fifth of the shapes that took them were slower, by up to 28 %) and 6 % slower than without at worst; from cache 1.065 x (1.070, 1.068)
-// and 5 %.  Nearly half of the shapes take them, nine in ten from 3e11 operations on.
+// the lead of 1.2 us that it must have over mid_plan's kernels to 8693 more of 65 .. 32768 tokens, every nx forced, weights from memory and from cache, codes
+// uniform and as quantisers leave them (Gaussian: with few bits toggling, these kernels' clock is higher).  With the latter, from memory the choice
+// is 1.073 x as fast as without these kernels (1.076 with the best of all; 1.062 without the limits, when a seventh of the shapes that took them
+// were 3 % and more slower, by up to 25 %; now a hundredth, 14 % at worst), from cache 1.103 x (1.109, 1.106).  With uniform codes 1.044 and 1.066 x.
+// About half of the shapes take them, nine in ten from 3e11 operations on.
 // What it does not take: rows of the output that are no whole 16-byte pieces, a K of one stage, scratch beyond 512 MiB (a weight of 26000 x 26000).
 struct SpreadPlan {
     int nx;             // 4 .. 8; 0: not this way
@@ -1279,7 +1281,8 @@ SpreadPlan spread_plan(int64_t M, int64_t N, int64_t Kb) {
         const int64_t tiles = ((others + 255) / 256) * ((rows + 32 * nx - 1) / (32 * nx));
         const double n = (double)((tiles + cus - 1) / cus), idle = 1.0 - (double)tiles / (n * (double)cus);
         const double stage = (0.406 + 0.144 * nx) * (1.0 - 0.285 * idle);
-        double walk = n * st * (N > M && stage < 1.15 ? 1.15 : stage);
+        const double least = N <= M ? 0.0 : n > 1.0 ? 1.05 : 1.15;
+        double walk = n * st * (stage < least ? least : stage);
         if (N > M && walk < bytes_us) walk = bytes_us;
         const double t = fixed + n * (0.26 + 0.675 * nx) * (1.0 - 0.23 * idle) + walk;
         if (best.nx == 0 || t < best.us) best = SpreadPlan{nx, t};
@@ -1307,7 +1310,7 @@ GemmPlan gemm_plan(int64_t M, int64_t N, int64_t Kb, size_t scratch, bool fp16, 
         const size_t x6 = fp16 && pieces && scratch ? qr_internal_x6_bytes(N <= M ? N : M, Kb) : 0;
         if (x6 && x6 <= scratch) {
             const SpreadPlan spread = spread_plan(M, N, Kb);
-            if (spread.nx && spread.us + 2.5 < plan.us) return GemmPlan{Gemm::x6, spread.nx, x6};
+            if (spread.nx && spread.us + 1.2 < plan.us) return GemmPlan{Gemm::x6, spread.nx, x6};
         }
         return sliced(kernels[plan.kernel], plan.split);
     }

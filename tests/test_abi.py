@@ -202,5 +202,5 @@ def test_plan_spreads_tokens_only_where_weights_from_memory_leave_a_lead(lib):
                     (512, 10240, 8192), (512, 11008, 4096), (65, 57344, 8192), (128, 57344, 8192)):
         assert lib.qr_linear_spread_bytes(m, n, k) == 0, (m, n, k)
     for m, n, k in ((333, 22016, 4096), (400, 28672, 8192), (700, 12288, 4096), (1024, 12288, 4096), (1024, 28672, 8192), (1777, 8192, 28672),
-                    (8191, 5120, 5120), (32768, 11008, 4096)):
+                    (8191, 5120, 5120), (32768, 11008, 4096), (2048, 5120, 5120), (2048, 8192, 8192)):
         assert lib.qr_linear_spread_bytes(m, n, k) > 0, (m, n, k)
